@@ -1,0 +1,608 @@
+"""Workloads that stand for what a GRPO program has this framework do: rollouts through `Sampler`, per-token
+log-probabilities through `compute_per_token_logps`, and the loss terms behind them.
+
+A case is a dict of plain values.  kind "rollout": `prompt` columns of left-padded prompts, `gen` new tokens;
+kind "logps": `prompt` + `gen` columns scored in one pass, packed or not; kind "loss": ratio, KL and aggregate over
+[batch, gen].  The models are the configurations of this repository with fewer layers (every layer of a kind
+does the same work; `layers` 0 is the configuration's own number).
+
+Weights are random.  So that a token does not hang on the last bit of a sum, as it would between the nearly equal logits of a
+random head, the head's row of token t + 1 is aligned with the embedding of t (tied heads: of t with itself), at a
+scale that gives the preferred token a probability of 0.05 to 0.7, as a trained model's tokens have; what the layers
+write into the residual stream is about as large as the embedding in it.
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+DEV = "cuda"
+PAD, EOS = 0, 1
+
+MODELS = {   # name: (function of tunix_amd.config, its arguments)
+    "tiny_qwen3": ("tiny_qwen3", {}),
+    "gemma3_1b": ("gemma3_1b", {}),
+    "llama31_8b": ("llama31_8b", {}),
+    "qwen3_30b_a3b": ("qwen3_30b_a3b", {}),
+    "nunezen": ("nunezen_shape", dict(width=2048, heads=16, kv_heads=4, ff=8192)),
+    "kezolix": ("kezolix_shape", dict(width=2048, heads=16, kv_heads=4, ff=8192, experts=64, top=8, expert_ff=768)),
+}
+STACKS = ("nunezen", "kezolix")
+LAYERS = {"tiny_qwen3": 0, "gemma3_1b": 0, "llama31_8b": 8, "qwen3_30b_a3b": 4, "nunezen": 4, "kezolix": 6}
+LOGIT = {"tiny_qwen3": 11.0, "llama31_8b": 16.0, "qwen3_30b_a3b": 12.0, "kezolix": 14.0}   # untied heads: logit of the preferred token before the layers' share
+
+
+def case(name, kind, model="", **kw):
+  out = dict(name=name, kind=kind, model=model, layers=LAYERS.get(model, 0), batch=1, prompt=0, gen=0, sampling="greedy",
+             packed=False, entropy=False, quantized_head=False, dtype="bf16")
+  out.update(kw)
+  return out
+
+
+def listed():
+  return [
+      # one conversation on the small test model: launches and host work alone
+      case("tiny_rollout_1", "rollout", "tiny_qwen3", batch=1, prompt=16, gen=32),
+      # a batch of a small model with the recipe's top-k draw over a large vocabulary
+      case("gemma_rollout_64", "rollout", "gemma3_1b", batch=64, prompt=256, gen=32, sampling="topk"),
+      # a few prompts of odd length and a long context, as in interactive use and evaluation
+      case("llama_rollout_3_long", "rollout", "llama31_8b", batch=3, prompt=2900, gen=40),
+      # one GRPO group of 16
+      case("llama_rollout_16", "rollout", "llama31_8b", batch=16, prompt=128, gen=64),
+      # the headline batch, 16 prompts x 8 completions
+      case("llama_rollout_128", "rollout", "llama31_8b", batch=128, prompt=256, gen=96),
+      # routed experts in int4
+      case("moe_rollout_64", "rollout", "qwen3_30b_a3b", batch=64, prompt=128, gen=32),
+      # a decoder given layer by layer with dense weights: attention and linear recurrences
+      case("nunezen_rollout_32", "rollout", "nunezen", batch=32, prompt=256, gen=48),
+      # the rollout batch scored again for the ratio, in packed rows, with entropies
+      case("llama_logps_packed", "logps", "llama31_8b", batch=13, gen=1024, packed=True, entropy=True),
+      # long reasoning traces through a quantised head with its own adapter
+      case("llama_logps_long", "logps", "llama31_8b", batch=2, prompt=1021, gen=5123, quantized_head=True),
+      # routed experts over many rows, odd lengths
+      case("moe_logps", "logps", "qwen3_30b_a3b", batch=7, prompt=211, gen=812),
+      # dense experts, gated recurrences, chunked attention
+      case("kezolix_logps", "logps", "kezolix", batch=8, prompt=256, gen=768),
+      # the loss terms of one small batch
+      case("loss_8", "loss", batch=8, gen=64),
+  ]
+
+
+def draw(rng):
+  def log(lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+  kind = rng.choice(["rollout", "rollout", "rollout", "logps", "logps", "loss"])
+  if kind == "loss":
+    return {k: v for k, v in case("", kind, batch=log(2, 256), gen=log(5, 4000)).items() if k != "name"}
+  model = rng.choice(["tiny_qwen3", "gemma3_1b", "llama31_8b", "llama31_8b", "llama31_8b", "qwen3_30b_a3b", "nunezen", "kezolix"])
+  kw = {}
+  if kind == "rollout":
+    batch = log(1, 128)
+    prompt = log(8, min(3000, 24000 // batch))
+    kw.update(batch=batch, prompt=prompt, gen=log(9, 48), sampling="topk" if model == "gemma3_1b" and rng.random() < 0.5 else "greedy")
+  else:
+    total = log(64, 6000)
+    prompt = rng.randrange(16, total // 2)
+    kw.update(batch=log(1, max(1.01, 10000 / total)), prompt=prompt, gen=total - prompt, entropy=rng.random() < 0.5)
+    if model not in STACKS and rng.random() < 0.3:
+      kw.update(packed=True, gen=total, prompt=0)
+    if model == "llama31_8b":
+      kw.update(quantized_head=rng.random() < 0.5)
+  if model in STACKS and rng.random() < 0.25:
+    kw["batch"] = max(1, kw["batch"] // 4)
+    kw["dtype"] = "fp32"
+  return {k: v for k, v in case("", kind, model, **kw).items() if k != "name"}
+
+
+# ---- inputs ------------------------------------------------------------------------------------
+def config_of(c):
+  from tunix_amd import config
+  name, kw = MODELS[c["model"]]
+  kw = dict(kw)
+  if c["model"] in STACKS:
+    kw["layers"] = c["layers"]
+  elif c["layers"]:
+    kw["num_layers"] = c["layers"]
+  if c["quantized_head"]:
+    kw.update(quantize_head=True, head_lora=True)
+  return getattr(config, name)(**kw)
+
+
+def generator(seed, n=0):
+  g = torch.Generator(device=DEV)
+  g.manual_seed(seed * 16 + n)
+  return g
+
+
+def qlora_weights(cfg, seed, head_logit):
+  """Flat parameter names (2-D kernels [in, out]) -> bf16 tensors."""
+  g, bf = generator(seed), torch.bfloat16
+  D, F, V, n = cfg.embed_dim, cfg.hidden_dim, cfg.vocab_size, cfg.num_layers
+  gemma = cfg.family == "gemma3"
+
+  def normal(*shape, s=0.02):
+    return (torch.randn(*shape, generator=g, device=DEV) * s).to(bf)
+
+  def norm(size, mean=0.0):
+    return (torch.randn(size, generator=g, device=DEV) * 0.05 + (mean if gemma else mean + 1.0)).to(bf)
+
+  out_s = 0.02 * (2 * n) ** -0.5 if not gemma else 0.02      # what writes into the residual stream
+  w = {"embed": normal(V, D, s=D ** -0.5 if gemma else 1.0), "final_norm": norm(D, -0.6 if gemma else 0.0)}
+  if not cfg.tied_embedding:
+    w["lm_head"] = (torch.roll(w["embed"], 1, 0).float() * (head_logit / D)).to(bf).T
+  for i in range(n):
+    p = f"l{i}."
+    w[p + "attn_norm"], w[p + "mlp_norm"] = norm(D), norm(D)
+    if cfg.family != "llama3":
+      w[p + "q_norm"], w[p + "k_norm"] = norm(cfg.head_dim), norm(cfg.head_dim)
+    if gemma:
+      w[p + "post_attn_norm"], w[p + "post_ffw_norm"] = norm(D, -0.9), norm(D, -0.9)
+    w[p + "wq"], w[p + "wk"], w[p + "wv"] = normal(D, cfg.q_dim), normal(D, cfg.kv_dim), normal(D, cfg.kv_dim)
+    w[p + "wo"] = normal(cfg.q_dim, D, s=out_s)
+    if cfg.num_experts:
+      E = cfg.num_experts
+      w[p + "router"] = normal(D, E)
+      w[p + "e_gate"], w[p + "e_up"], w[p + "e_down"] = normal(E, D, F), normal(E, D, F), normal(E, F, D, s=0.05)
+    else:
+      w[p + "w_gate"], w[p + "w_up"], w[p + "w_down"] = normal(D, F), normal(D, F), normal(F, D, s=out_s)
+  for name in cfg.lora_names():
+    K, N = w[name].shape
+    w[name + ".lora_a"], w[name + ".lora_b"] = normal(K, cfg.lora_rank), normal(cfg.lora_rank, N, s=0.01)
+  return w
+
+
+def stack_weights(cfg, seed, head_logit):
+  """File names (linears [out, in]) -> bf16 tensors."""
+  g, D = generator(seed), cfg.embed_dim
+  out = {}
+  for name, shape in cfg.weight_shapes().items():
+    if name == "head":
+      continue
+    t = torch.randn(*shape, generator=g, device=DEV)
+    if name in ("embed", "mix.sink") or name.endswith("mix.sink"):
+      pass
+    elif name == "pos":
+      t = 0.3 * t
+    elif name == "loop.in":
+      t = 0.2 * t * shape[1] ** -0.5 + torch.cat([0.8 * torch.eye(D, device=DEV), 0.2 * torch.eye(D, device=DEV)], 1)
+    elif name.endswith(".lower"):
+      t = torch.sigmoid(t)
+    elif name.endswith(".dwa"):
+      t = 0.05 * t
+      t[-1] += 1.0
+    elif name.endswith("mlp.correction"):
+      t = (0.1 / shape[0]) * t
+    elif name.endswith("mlp.act"):
+      t = 0.3 * t
+    elif name == "final.norm" and cfg.tied_head:
+      t = torch.full_like(t, 2.0 ** -8 - cfg.norm_offset)    # (a logit of 8 for a tied row of width 2048)
+    elif name.endswith(("norm1b", "norm2b")):
+      t = 0.05 * t + (0.3 - cfg.norm_offset)
+    elif name.endswith("mix.norm"):
+      t = 1.0 + 0.05 * t
+    elif "norm" in name:
+      t = 0.05 * t + (1.0 - cfg.norm_offset)
+    elif len(shape) == 1:
+      t = 0.1 * t
+    else:
+      t = t * shape[1] ** -0.5
+    out[name] = t.to(torch.bfloat16)
+  if not cfg.tied_head:
+    out["head"] = (torch.roll(out["embed"], 1, 0).float() * (head_logit / D)).to(torch.bfloat16)
+  return out
+
+
+def weights_of(c, cfg, seed):
+  make = stack_weights if c["model"] in STACKS else qlora_weights
+  return make(cfg, seed, LOGIT.get(c["model"], 0.0))
+
+
+def tied(cfg):
+  return cfg.tied_head if hasattr(cfg, "tied_head") else cfg.tied_embedding
+
+
+def continuation(cfg, first, n):
+  """The preferred tokens behind `first` [B]."""
+  step = 0 if tied(cfg) else 1
+  return first[:, None] + step * (1 + np.arange(n))[None, :]
+
+
+def prompts_of(c, cfg, seed):
+  """[B, prompt] ids, left-padded to ragged lengths."""
+  rng = np.random.default_rng(seed + 1)
+  B, P = c["batch"], c["prompt"]
+  ids = rng.integers(2, cfg.vocab_size - c["gen"] - 2, size=(B, P))
+  for b, pads in enumerate(rng.integers(0, max(P // 4, 1), size=B)):
+    if b:
+      ids[b, :pads] = PAD
+  return ids.astype(np.int32)
+
+
+def scored_ids(c, cfg, seed):
+  """(prompt ids, completion ids, segment ids or None, positions or None) of a "logps" case."""
+  rng = np.random.default_rng(seed + 2)
+  B, T = c["batch"], c["gen"]
+  if not c["packed"]:
+    prompt = prompts_of(c, cfg, seed)
+    done = continuation(cfg, prompt[:, -1].astype(np.int64), T).astype(np.int32)
+    if c["model"] not in STACKS:     # completions that ended early are padded behind
+      for b, n in enumerate(rng.integers(0, T // 4 + 1, size=B)):
+        if b and n:
+          done[b, T - n:] = PAD
+    return prompt, done, None, None
+  ids, seg, pos = (np.zeros((B, T), np.int32) for _ in range(3))
+  for b in range(B):
+    at, k = 0, 1
+    while at < T:
+      n = min(T - at, int(rng.integers(max(T // 8, 2), max(T // 2, 3))))
+      half = max(1, n // 3)
+      one = rng.integers(2, cfg.vocab_size - T - 2, size=half)
+      ids[b, at:at + n] = np.concatenate([one, continuation(cfg, one[-1:], n - half)[0]])
+      seg[b, at:at + n], pos[b, at:at + n] = k, np.arange(n)
+      at, k = at + n, k + 1
+  return np.zeros((B, 0), np.int32), ids, seg, pos
+
+
+def loss_inputs(c, seed):
+  g, B, T = generator(seed), c["batch"], c["gen"]
+  r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+  old = -2.0 * r(B, T).abs()
+  lengths = torch.randint(1, T + 1, (B, 1), generator=g, device=DEV)
+  return dict(old=old, logp=old + 0.1 * r(B, T), ref=old + 0.1 * r(B, T), adv=r(B),
+              mask=(torch.arange(T, device=DEV)[None, :] < lengths).to(torch.float32))
+
+
+def prepare(c, seed):
+  if c["kind"] == "loss":
+    return dict(case=c, **loss_inputs(c, seed))
+  from tunix_amd.generate.sampler import CacheConfig, Sampler
+  from tunix_amd.generate.utils import IdTokenizer
+  from tunix_amd.model import QLoRAModel
+  from tunix_amd.stack_model import StackModel
+  cfg = config_of(c)
+  w = weights_of(c, cfg, seed)
+  if c["model"] in STACKS:
+    model = StackModel(cfg, w, DEV, torch.float32 if c["dtype"] == "fp32" else torch.bfloat16)
+  else:
+    model = QLoRAModel(cfg, w, DEV)
+  if c["kind"] == "rollout":
+    sampler = Sampler(model, IdTokenizer(cfg.vocab_size, PAD, EOS), CacheConfig(c["prompt"] + c["gen"]))
+    ids = prompts_of(c, cfg, seed)
+    return dict(case=c, sampler=sampler, prompts=[r[int(np.argmax(r != PAD)):].tolist() for r in ids], seed=seed)
+  to = lambda a: None if a is None else torch.from_numpy(a).to(DEV)
+  prompt, done, seg, pos = map(to, scored_ids(c, cfg, seed))
+  return dict(case=c, model=model, prompt=prompt, completion=done, segment_ids=seg, segment_positions=pos)
+
+
+# ---- one pass ------------------------------------------------------------------------------------
+RECIPE = dict(temperature=0.9, top_p=1.0, top_k=50)
+BETA, EPSILON = 0.04, 0.2
+
+
+def run(state):
+  c = state["case"]
+  if c["kind"] == "rollout":
+    kw = dict(RECIPE, seed=state["seed"]) if c["sampling"] == "topk" else {}
+    out = state["sampler"](state["prompts"], c["gen"], max_prompt_length=c["prompt"], return_logprobs=True, pad_output=True, **kw)
+    return {"tokens": np.stack(out.tokens), "logprobs": np.asarray(out.logprobs, dtype=np.float32)}
+  if c["kind"] == "logps":
+    from tunix_amd.rl.common import compute_per_token_logps
+    got = compute_per_token_logps(state["model"], state["prompt"], state["completion"], PAD, return_entropy=c["entropy"],
+                                  segment_ids=state["segment_ids"], segment_positions=state["segment_positions"])
+    return dict(zip(("logps", "entropy"), got if c["entropy"] else (got,)))
+  from tunix_amd.rl.common import aggregate_loss, compute_kl_divergence, grpo_clipped_ratio
+  ratio, loss, clipped = grpo_clipped_ratio(state["logp"], state["old"], state["adv"], EPSILON)
+  kl = compute_kl_divergence(state["logp"], state["ref"])
+  total = aggregate_loss(loss + BETA * kl, state["mask"], "sequence-mean-token-mean").compute()
+  return {"ratio": ratio, "loss": loss, "clipped": clipped, "kl": kl, "total": total}
+
+
+# ---- what a pass cannot do without ----------------------------------------------------------------
+def sizes(c, cfg):
+  """(weights every token passes, weights of one expert x layers, experts, experts per token, bytes per weight, KV or
+  latent numbers of one token, score and value multiplications per (query, key), recurrent state numbers, head weights)."""
+  if c["model"] in STACKS:
+    shapes, runs = cfg.weight_shapes(), [i for i, _ in cfg.layer_runs]
+    dense = expert = kv = pair = state = 0
+    for name, s in shapes.items():
+      if name in ("embed", "head", "pos") or len(s) < 2:
+        continue
+      times = runs.count(int(name.split(".")[0][1:])) if name[0] == "l" and name[1].isdigit() else cfg.loop.times
+      n = s[0] * s[1] * times
+      if ".mlp.e" in name:
+        expert += n
+      else:
+        dense += n
+    moe = next((ly.mlp for ly in cfg.layers if hasattr(ly.mlp, "experts")), None)
+    for i in runs:
+      m = cfg.layers[i].mixer
+      if hasattr(m, "kv_heads"):
+        kv += m.kv_heads * (m.dim + m.vdim)
+        pair += m.heads * (m.dim + m.vdim)
+      else:
+        state += m.heads * m.dim * m.vdim
+    E, k = (moe.experts, moe.top) if moe else (1, 1)
+    return dense, expert / E, E, k, 4.0 if c["dtype"] == "fp32" else 2.0, kv, pair, state, cfg.vocab_size * cfg.embed_dim
+  D, n, E = cfg.embed_dim, cfg.num_layers, max(cfg.num_experts, 1)
+  dense, mlp = n * 2 * D * (cfg.q_dim + cfg.kv_dim), n * 3 * D * cfg.hidden_dim
+  if not cfg.num_experts:
+    dense, mlp = dense + mlp, 0
+  return (dense, mlp, E, max(cfg.num_experts_per_tok, 1), 0.5 + 2.0 / cfg.group, 2 * cfg.kv_dim * n, 2 * cfg.q_dim * n, 0, cfg.vocab_size * D)
+
+
+def work(c):
+  B, P, T = c["batch"], c["prompt"], c["gen"]
+  if c["kind"] == "loss":
+    return {"bytes": 4.0 * B * T * 9, "flops": 30.0 * B * T}
+  cfg = config_of(c)
+  dense, expert, E, k, per, kv, pair, state, head = sizes(c, cfg)
+  kv_b = 4.0 if c["dtype"] == "fp32" else 2.0
+  head_b = per if c["quantized_head"] else kv_b
+  one = lambda rows: per * (dense + expert * min(E, rows * k))          # weights read by a pass over `rows` tokens
+  row_flops = 2.0 * (dense + expert * k)
+  causal = lambda n: n * (n + 1) / 2
+  if c["kind"] == "logps":
+    n = P + T
+    rows = B * n
+    return {"bytes": one(rows) + head_b * head + 4.0 * rows + 4.0 * B * T,
+            "flops": rows * row_flops + 2.0 * B * pair * causal(n) * (0.5 if c["packed"] else 1.0) + 2.0 * B * T * head + 4.0 * rows * state}
+  steps = T - 1
+  ctx = steps * P + causal(steps)
+  return {"bytes": one(B * P) + steps * one(B) + T * head_b * head + B * ctx * kv * kv_b + 8.0 * steps * B * state + 8.0 * B * (P + T),
+          "flops": B * (P + steps) * row_flops + 2.0 * B * pair * (causal(P) + ctx) + 2.0 * B * T * head + 4.0 * B * (P + steps) * state}
+
+
+def tolerance(c):
+  """About four times what the passes are off 64 bits.  bf16: two roundings of the residual stream per sublayer move a log-probability
+  of -1 to -3 by about 0.01 (0.0025 of it over the Llama layers, up to 0.017 over the 26 Gemma layers, routed experts with close
+  calls and depth averages), single ones by some times as much.  The top-k draw may turn on a close call, after which a row goes
+  its own way.  fp32: the order of sums (the KL is a difference of numbers near one)."""
+  if c["kind"] == "loss":
+    return {"rel": 1e-5, "max": 1e-4}
+  if c["dtype"] == "fp32":
+    return {"rel": 3e-5, "max": 2e-4}
+  if c["sampling"] == "topk":
+    return {"rel": 0.03, "max": 0.9, "differ": 0.01}
+  return {"rel": 0.01, "max": 0.08} if c["model"] == "llama31_8b" else {"rel": 0.03, "max": 0.2}
+
+
+# ---- the same in 64 bits ---------------------------------------------------------------------------
+NF4 = (-1.0, -0.6961928, -0.52507305, -0.39491749, -0.28444138, -0.18477343, -0.09105004, 0.0,
+       0.0795803, 0.1609302, 0.2461123, 0.33791524, 0.44070983, 0.562617, 0.72295684, 1.0)
+F64 = torch.float64
+
+
+def dequantized(w, cfg):
+  """The values that group-quantised weights [K, N] stand for: level x scale of every `group` inputs, as bf16."""
+  K, N = w.shape
+  x = w.float().view(K // cfg.group, cfg.group, N)
+  top = x.abs().amax(1, keepdim=True)
+  nf4 = cfg.qtype == 1
+  scale = (top if nf4 else top / cfg.int4_bound).bfloat16().float()
+  x = x / torch.where(scale == 0, torch.ones_like(scale), scale)
+  if nf4:
+    lv = torch.tensor(NF4, dtype=torch.float32, device=w.device)
+    level = lv.bfloat16().float()[torch.searchsorted(0.5 * (lv[:-1] + lv[1:]), x.contiguous())]
+  else:
+    level = x.round().clamp(-8, 7)
+  return (level * scale).bfloat16().view(K, N).to(F64)
+
+
+def rms(x, eps, w=None):
+  y = x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)
+  return y if w is None else y * w
+
+
+def rotated(x, pos, dims, base):
+  """x [B, T, H, d]: the first `dims` of d rotated in pairs (i, i + dims / 2)."""
+  half = dims // 2
+  a = pos[:, :, None, None].to(F64) * base ** (-2.0 * torch.arange(half, device=x.device, dtype=F64) / dims)
+  u, v, s, co = x[..., :half], x[..., half:dims], torch.sin(a), torch.cos(a)
+  return torch.cat([u * co - v * s, v * co + u * s, x[..., dims:]], -1)
+
+
+def attended(q, k, v, scale, mask, sink=None, slopes=None):
+  """q [B, T, H, d], k / v [B, T, G, .], mask [B, T, T] of the keys a query sees."""
+  B, T, H, _ = q.shape
+  G = k.shape[2]
+  out = torch.empty(B, T, H, v.shape[-1], dtype=F64, device=q.device)
+  away = (torch.arange(T, device=q.device)[:, None] - torch.arange(T, device=q.device)[None, :]).to(F64)
+  for b in range(B):
+    for h in range(H):
+      g = h // (H // G)
+      s = (q[b, :, h].contiguous() @ k[b, :, g].T.contiguous()) * scale
+      if slopes is not None:
+        s = s - slopes[h] * away
+      s = s.masked_fill(~mask[b], -1e30)
+      top = s.amax(-1, keepdim=True)
+      if sink is not None:
+        top = torch.maximum(top, sink[h])
+      e = torch.exp(s - top)
+      den = e.sum(-1, keepdim=True) + (0.0 if sink is None else torch.exp(sink[h] - top))
+      out[b, :, h] = (e / den) @ v[b, :, g].contiguous()
+  return out
+
+
+def qlora_hidden(c, cfg, w, ids, pos, mask):
+  gemma, B, T = cfg.family == "gemma3", *ids.shape
+  norm = lambda x, n, eps=cfg.norm_eps: rms(x, eps, w[n].to(F64) + (1.0 if gemma else 0.0))
+
+  def linear(x, n):
+    y = x @ dequantized(w[n], cfg)
+    if n + ".lora_a" in w:
+      y = y + (x @ w[n + ".lora_a"].to(F64)) @ w[n + ".lora_b"].to(F64) * (cfg.lora_alpha / cfg.lora_rank)
+    return y
+
+  def gated(g, u):
+    return (torch.nn.functional.gelu(g, approximate="tanh") if gemma else g * torch.sigmoid(g)) * u
+
+  def experts(x, p):
+    flat = x.reshape(-1, x.shape[-1])
+    prob = torch.softmax(flat @ w[p + "router"].to(F64), -1)
+    top, at = prob.topk(cfg.num_experts_per_tok, -1)
+    top, out = top / top.sum(-1, keepdim=True), torch.zeros_like(flat)
+    for e in range(cfg.num_experts):
+      row, j = torch.nonzero(at == e, as_tuple=True)
+      h = flat[row]
+      y = gated(h @ dequantized(w[p + "e_gate"][e], cfg), h @ dequantized(w[p + "e_up"][e], cfg)) @ dequantized(w[p + "e_down"][e], cfg)
+      out.index_add_(0, row, y * top[row, j, None])
+    return out.view_as(x)
+
+  x = w["embed"][ids].to(F64) * (math.sqrt(cfg.embed_dim) if gemma else 1.0)
+  cols = torch.arange(T, device=ids.device)
+  for i in range(cfg.num_layers):
+    p, (base, _) = f"l{i}.", cfg.rope_params(i)
+    h = norm(x, p + "attn_norm")
+    q, k, v = (linear(h, p + n).view(B, T, -1, cfg.head_dim) for n in ("wq", "wk", "wv"))
+    if cfg.family != "llama3":
+      q, k = norm(q, p + "q_norm"), norm(k, p + "k_norm")
+    q, k = rotated(q, pos, cfg.head_dim, base), rotated(k, pos, cfg.head_dim, base)
+    seen = mask & (cols[None, :] > cols[:, None] - cfg.sliding_window) if cfg.is_local_layer(i) else mask
+    y = linear(attended(q, k, v, cfg.head_dim ** -0.5, seen).reshape(B, T, -1), p + "wo")
+    x = x + (norm(y, p + "post_attn_norm") if gemma else y)
+    h = norm(x, p + "mlp_norm")
+    y = experts(h, p) if cfg.num_experts else linear(gated(linear(h, p + "w_gate"), linear(h, p + "w_up")), p + "w_down")
+    x = x + (norm(y, p + "post_ffw_norm") if gemma else y)
+  x = norm(x, "final_norm")
+  if tied(cfg):
+    return x, w["embed"].to(F64).T
+  if not cfg.quantize_head:
+    return x, w["lm_head"].to(F64)
+  return x, dequantized(w["lm_head"], cfg) + w["lm_head.lora_a"].to(F64) @ w["lm_head.lora_b"].to(F64) * (cfg.lora_alpha / cfg.lora_rank)
+
+
+def stack_hidden(c, cfg, w, ids, start, mask):
+  """Nunezen and Kezolix decoders; `start` [B]: the column of a row's first token."""
+  w = {n: t.to(F64) if len(t.shape) == 1 or n.endswith(".dwa") else t for n, t in w.items()}
+  B, T = ids.shape
+  cols = torch.arange(T, device=ids.device)
+  pos = (cols[None, :] - start[:, None]).clamp(min=0)
+  real = (cols[None, :] >= start[:, None]).to(F64)[:, :, None, None]
+  eps = cfg.norm_eps
+  linear = lambda x, n: x @ w[n].to(F64).T
+  silu = lambda z: z * torch.sigmoid(z)
+
+  def norm(x, n):
+    return rms(x - x.mean(-1, keepdim=True) if cfg.center_norm else x, eps, w[n] + cfg.norm_offset)
+
+  def attention(h, m, p, kept, i):
+    heads = lambda n, k, d: linear(h, p + n).view(B, T, k, d)
+    if m.row_norm:
+      q = rms(linear(h, p + "q"), eps, w[p + "q.norm"]).view(B, T, m.heads, m.dim)
+      if m.kv_from is None:
+        kept[i] = rms(linear(h, p + "k"), eps, w[p + "k.norm"]).view(B, T, m.kv_heads, m.dim), heads("v", m.kv_heads, m.vdim)
+      k, v = kept[i if m.kv_from is None else m.kv_from]
+    else:
+      q = rotated(heads("q", m.heads, m.dim), pos, m.rot_dims, m.rot_base)
+      k, v = rotated(heads("k", m.kv_heads, m.dim), pos, m.rot_dims, m.rot_base), heads("v", m.kv_heads, m.vdim)
+    seen = mask & (pos[:, :, None] // m.chunk == pos[:, None, :] // m.chunk) if m.chunk else mask
+    o = attended(q, k, v, m.scale, seen, w[p + "sink"] if m.sink else None, m.slopes or None)
+    return linear(o.reshape(B, T, -1), p + "o")
+
+  def lightning(h, m, p):
+    q, k, v = (silu(linear(h, p + n)).view(B, T, m.heads, -1) for n in "qkv")
+    k, o = k * real, torch.empty_like(v)
+    away = (cols[:, None] - cols[None, :]).to(F64)
+    for b in range(B):
+      for n in range(m.heads):
+        fade = torch.where(away >= 0, m.decay[n] ** away.clamp(min=0), torch.zeros_like(away))
+        o[b, :, n] = ((q[b, :, n].contiguous() @ k[b, :, n].T.contiguous()) * fade) @ v[b, :, n].contiguous()
+    return linear(rms(o.reshape(B, T, -1), eps, w[p + "norm"]) * torch.sigmoid(linear(h, p + "g")), p + "o")
+
+  def recurrence(h, m, p):
+    q = silu(linear(h, p + "q")).view(B, T, m.heads, m.dim)
+    low = w[p + "lower"]
+    f = (low + (1.0 - low) * torch.sigmoid(linear(h, p + "f") + w[p + "f.b"])).view(B, T, m.heads, m.dim)
+    v, o = linear(h, p + "v").view(B, T, m.heads, m.vdim), []
+    s = torch.zeros(B, m.heads, m.dim, m.vdim, dtype=F64, device=ids.device)
+    add = (1.0 - f) * real
+    for t in range(T):
+      s = f[:, t, :, :, None] * s + add[:, t, :, :, None] * v[:, t, :, None, :]
+      o.append((q[:, t, :, :, None] * s).sum(2))
+    return linear(rms(torch.stack(o, 1), eps, w[p + "norm"]).reshape(B, T, -1), p + "o")
+
+  def feed_forward(h, mlp, p):
+    if hasattr(mlp, "experts"):
+      flat = h.reshape(-1, h.shape[-1])
+      square = lambda x, n: linear(linear(x, n + ".up").clamp(min=0.0) ** 2, n + ".down")
+      score = torch.softmax(linear(flat, p + "router"), -1)
+      at = (score + w[p + "correction"]).topk(mlp.top, -1).indices
+      share = torch.gather(score, 1, at)
+      share = share / (share.sum(-1, keepdim=True) + 1e-20) * mlp.scale
+      out = torch.sigmoid(linear(flat, p + "shared.sg")) * square(flat, p + "shared")
+      for e in range(mlp.experts):
+        row, j = torch.nonzero(at == e, as_tuple=True)
+        out.index_add_(0, row, square(flat[row], f"{p}e{e}") * share[row, j, None])
+      return out.view_as(h)
+    z = linear(h, p + "up")
+    if p + "act" in w:
+      a = w[p + "act"]
+      return linear(a[0] * rms(z, eps) + a[1] * rms(z * z, eps) + a[2] * rms(z * z * z, eps) + a[3], p + "down")
+    return linear(torch.nn.functional.gelu(linear(h, p + "gate"), approximate="tanh") * z, p + "down")
+
+  x = x0 = w["embed"][ids].to(F64) + (w["pos"][pos].to(F64) if cfg.max_positions else 0.0)
+  rows, kept = [x], {}
+  for i, begins in cfg.layer_runs:
+    p, ly = f"l{i}.", cfg.layers[i]
+    if begins:
+      x = linear(torch.cat([x, x0], -1), "loop.in")
+    h, m = norm(x, p + "norm1"), ly.mixer
+    y = attention(h, m, p + "mix.", kept, i) if hasattr(m, "kv_heads") else lightning(h, m, p + "mix.") if hasattr(m, "decay") else recurrence(h, m, p + "mix.")
+    x = x + cfg.residual_mult * norm(y, p + "norm1b")
+    if ly.mlp is not None:
+      x = x + cfg.residual_mult * norm(feed_forward(norm(x, p + "norm2"), ly.mlp, p + "mlp."), p + "norm2b")
+    if cfg.depth_average:
+      rows.append(x)
+      x = sum(a * r for a, r in zip(w[p + "dwa"], rows))
+  return norm(x, "final.norm"), (w["embed"] if tied(cfg) else w["head"]).to(F64).T
+
+
+def exact(c, seed):
+  if c["kind"] == "loss":
+    s = {k: v.to(F64) for k, v in loss_inputs(c, seed).items()}
+    ratio, adv = torch.exp(s["logp"] - s["old"]), s["adv"][:, None]
+    loss = torch.maximum(-adv * ratio, -adv * ratio.clamp(1 - EPSILON, 1 + EPSILON))
+    d = s["ref"] - s["logp"]
+    kl = torch.exp(d) - d - 1.0
+    total = (((loss + BETA * kl) * s["mask"]).sum(1) / s["mask"].sum(1).clamp(min=1.0)).sum() / (s["mask"].sum(1) > 0).sum().clamp(min=1)
+    return {"ratio": ratio, "loss": loss, "clipped": None, "kl": kl, "total": total}
+  if c["sampling"] == "topk":     # which tokens the draws give is not known here
+    return None
+  cfg = config_of(c)
+  w = weights_of(c, cfg, seed)
+  rollout = c["kind"] == "rollout"
+  if rollout:
+    prompt, seg, pos = prompts_of(c, cfg, seed), None, None
+    done = continuation(cfg, prompt[:, -1].astype(np.int64), c["gen"])
+  else:
+    prompt, done, seg, pos = scored_ids(c, cfg, seed)
+  ids = torch.from_numpy(np.concatenate([prompt, done], 1).astype(np.int64)).to(DEV)
+  B, n = ids.shape
+  T = n - 1 if c["packed"] else c["gen"]
+  mask = torch.ones(n, n, dtype=torch.bool, device=DEV).tril()[None].expand(B, n, n)
+  if c["packed"]:
+    seg, pos = torch.from_numpy(seg).to(DEV), torch.from_numpy(pos).to(DEV)
+    mask = mask & (seg[:, :, None] == seg[:, None, :])
+  else:
+    mask = mask & (ids != PAD)[:, None, :]
+    run_ = torch.cumsum((ids != PAD).to(torch.int64), 1)
+    pos = run_ - (run_ >= 1).to(torch.int64)
+  if c["model"] in STACKS:
+    x, head = stack_hidden(c, cfg, w, ids, torch.cumprod((ids == PAD).to(torch.int64), 1).sum(1), mask)
+  else:
+    x, head = qlora_hidden(c, cfg, w, ids, pos, mask)
+  x, target = x[:, n - T - 1:n - 1].reshape(B * T, -1), ids[:, n - T:].reshape(-1)
+  lp, ent = torch.empty(B * T, dtype=F64, device=DEV), torch.empty(B * T, dtype=F64, device=DEV)
+  for r in range(0, B * T, 512):
+    z = torch.log_softmax(x[r:r + 512] @ head, -1)
+    lp[r:r + 512] = torch.gather(z, 1, target[r:r + 512, None])[:, 0]
+    ent[r:r + 512] = -(z.exp() * z).sum(-1)
+  lp, ent = lp.view(B, T), ent.view(B, T)
+  if rollout:
+    return {"tokens": None, "logprobs": lp}
+  if c["packed"]:
+    lp, ent = (torch.cat([torch.zeros(B, 1, dtype=F64, device=DEV), v], 1) for v in (lp, ent))
+  return {"logps": lp, "entropy": ent} if c["entropy"] else {"logps": lp}
