@@ -171,7 +171,7 @@ def many_rows_breakdown(model, rows, iters):
   tot_flops = sum(2.0 * rows * ly[k].K * ly[k].N for k in out)
   tot_s = sum(v["us"] for v in out.values()) * 1e-6
   tf = tot_flops / tot_s / 1e12
-  return {"kernel": "qgemm_wide_kernel", "rows": rows, "bound": "mfma", "achieved": round(tf, 1),
+  return {"kernel": "qgemm_pre_kernel", "rows": rows, "bound": "mfma", "achieved": round(tf, 1),
           "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(tf / MFMA_BF16_PEAK_TFLOPS, 4),
           "linears": out}
 
@@ -267,7 +267,7 @@ def write_traffic_profile(fetch_csv, write_csv):
 # The same for the many-row kernel on the standalone log-probability pass (one launch = 16384 rows
 # x 128256 columns): counter runs of `bench.py --fused-logps`.
 FUSED_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "qgemm_wide_kernel_fused_logps_131072rows.json")
-FUSED_KERNEL_SOURCES = ("csrc/qgemm_wide.h", "csrc/gemm_tile.h", "csrc/common.h", "csrc/qlinear.hip",
+FUSED_KERNEL_SOURCES = ("csrc/qgemm_pre.h", "csrc/wide_out.h", "csrc/gemm_tile.h", "csrc/common.h", "csrc/qlinear.hip",
                         "csrc/lmhead.hip")
 
 
@@ -294,15 +294,15 @@ def fused_measured_traffic():
 def write_fused_traffic_profile(fetch_csv, write_csv):
   """Rebuilds the tracked traffic record of the log-probability pass from two `rocprofv3 --pmc`
   runs of `bench.py --fused-logps` (FETCH_SIZE in one, WRITE_SIZE in the other; KiB per dispatch of
-  qgemm_wide_kernel).  FETCH_SIZE is scaled with the factor the decode GEMM's record holds for
+  qgemm_pre_kernel).  FETCH_SIZE is scaled with the factor the decode GEMM's record holds for
   buffer loads (its 1 GiB yardstick reads)."""
   import csv
 
   def mean(path, counter):
     v = [float(r["Counter_Value"]) for r in csv.DictReader(open(path))
-         if r["Counter_Name"] == counter and "qgemm_wide_kernel" in r["Kernel_Name"]]
+         if r["Counter_Name"] == counter and "qgemm_pre_kernel" in r["Kernel_Name"]]
     if not v:
-      raise SystemExit(f"no qgemm_wide_kernel dispatches with {counter} in {path}")
+      raise SystemExit(f"no qgemm_pre_kernel dispatches with {counter} in {path}")
     return sum(v) / len(v), len(v)
 
   with open(TRAFFIC_PROFILE) as f:
@@ -311,7 +311,7 @@ def write_fused_traffic_profile(fetch_csv, write_csv):
   wk, nw = mean(write_csv, "WRITE_SIZE")
   rows, D, V, r = 16384, 4096, 128256, 64
   rec = {
-      "kernel": "qgemm_wide_kernel (head-statistics epilogue)",
+      "kernel": "qgemm_pre_kernel (head-statistics form)",
       "workload": "one launch of the standalone log-probability pass: 16384 rows x 4096 -> 128256, int4 g128 + LoRA r64, "
                   "the head read from its expanded bf16 copy",
       "kernel_source_sha256_16": source_hash(FUSED_KERNEL_SOURCES),
@@ -520,7 +520,7 @@ def fused_logps_workload(rows, chunk, iters, expanded=True):
       "config": {"workload": "standalone fused lm_head -> log-softmax -> gather -> GRPO ratio", "rows": rows,
                  "rows_per_launch": chunk,
                  "head_operand": "expanded bf16 copy of the int4 head" if expanded else "int4 codes converted in the loop"},
-      "roofline": {"kernel": "qgemm_wide_kernel (statistics epilogue)", "bound": "mfma",
+      "roofline": {"kernel": "qgemm_pre_kernel (head-statistics form)", "bound": "mfma",
                    "achieved": round(flops / (ms * 1e-3) / 1e12, 1), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                    "frac": round(flops / (ms * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4),
                    # HBM bytes of one 16384-row launch, from the tracked counter record

@@ -1724,3 +1724,93 @@ def test_mul_epilogue_fuses_next_adapter_projection(gpu, M, F, r):
   t2 = torch.zeros(M, r, dtype=torch.bfloat16, device=gpu)
   ops.lora_down(y1, a_t, t2)
   assert (t[:, :r].float() - t2.float()).abs().max().item() <= 2.0 ** -7 * max(1e-3, t2.float().abs().max().item())
+
+
+# (the second half of the shapes runs 256-row tiles, the first 128-row ones: what fills the device better)
+PRE_SHAPES = [(65, 128, 16), (128, 256, 272), (129, 384, 48), (255, 128, 528), (769, 2048, 16304), (1024, 2048, 16384), (1023, 2176, 16144)]
+
+
+@pytest.mark.parametrize("M,K,N", PRE_SHAPES)
+def test_many_rows_from_the_expanded_copy(gpu, M, K, N):
+  """Every form of the tile that qgemm_pre.h stores, at the edges of its row and column tiles, against 64-bit sums: fp32 results
+  within the worst case of K roundings, bf16 ones within half an ulp more."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  g = torch.Generator(device=gpu).manual_seed(M)
+  x = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+  w = (torch.randn(N, K, generator=g, device=gpu) * K ** -0.5).bfloat16()
+  want = x.double() @ w.double().T
+  err = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+
+  def run(wt, epilogue, n, dtype):
+    y = torch.full((M + 1, n), 7.0, dtype=dtype, device=gpu)
+    d = L.DenseDesc()
+    d.M, d.K, d.N, d.dtype, d.batch, d.split_k = M, K, N, ops.DTYPES[torch.bfloat16], 1, 1
+    d.x, d.ldx, d.w, d.epilogue, d.y, d.ldy = x.data_ptr(), K, ops.dense_expand(wt).data_ptr(), epilogue, y.data_ptr(), n
+    ops.dense_linear(d)
+    torch.cuda.synchronize()
+    assert (y[M] == 7.0).all()      # nothing behind the last row
+    return y[:M].double()
+
+  for epilogue, ref, e, dtype in ((L.TNX_EPI_F32, want, err, torch.float32), (L.TNX_EPI_STORE, want, err, torch.bfloat16),
+                                  (L.TNX_EPI_RELU2, want.clamp(min=0) ** 2, 2.1 * err * want.abs() + err ** 2, torch.bfloat16)):
+    rounding = 0.0 if dtype == torch.float32 else 2.0 ** -8
+    assert ((run(w, epilogue, N, dtype) - ref).abs() <= rounding * ref.abs() + e + 1e-30).all(), epilogue
+  if N % 32:
+    return
+  half = N // 2
+  paired = w.view(2, N // 32, 16, K).transpose(0, 1).reshape(N, K).contiguous()
+  gate, up = want[:, :half], want[:, half:]
+  for epilogue, act in ((L.TNX_EPI_SILU_MUL, torch.nn.functional.silu(gate)), (L.TNX_EPI_GELU_MUL, torch.nn.functional.gelu(gate, approximate="tanh"))):
+    got = run(paired, epilogue, half, torch.bfloat16)
+    assert ((got - act * up).norm() / (act * up).norm()) < 2.0 ** -8, epilogue
+
+
+@pytest.mark.parametrize("M,K,widths", [(600, 256, (3968, 4112, 16)), (1000, 2048, (8176, 4096, 4112))])
+@pytest.mark.parametrize("rank", [32, 64])
+@pytest.mark.parametrize("scale", [1.0, 0.25, 0.75])
+def test_many_rows_adapter(gpu, M, K, widths, rank, scale):
+  """The adapter behind the last k of 128- and 256-row tiles: scales that go into B (powers of two) and others, segments that begin
+  inside a work-group's columns; against 64-bit sums of the same t."""
+  from tunix_amd import ops
+  N = sum(widths)
+  g = torch.Generator(device=gpu).manual_seed(rank)
+  r = lambda *s: torch.randn(*s, generator=g, device=gpu)
+  x, w, t, b = r(M, K).bfloat16(), (r(K, N) * 0.02).bfloat16(), r(M, 3 * rank).bfloat16(), (r(N, rank) * 0.1).bfloat16()
+  codes, scales = ops.quantize_pack(w, 64, Q.NF4)
+  wd = ops.qw_dequant(codes, scales, K, N, 64, Q.NF4).double()
+  ends = [int(v) for v in np.cumsum(widths)]
+  want, size = x.double() @ wd, x.double().abs() @ wd.abs()
+  for i, (a0, a1) in enumerate(zip([0] + ends[:-1], ends)):
+    ti, bi = t[:, i * rank:(i + 1) * rank].double(), b[a0:a1].double().T
+    want[:, a0:a1] += scale * (ti @ bi)
+    size[:, a0:a1] += scale * (ti.abs() @ bi.abs())
+  y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=gpu)
+  ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=Q.NF4, x=x, codes=codes, scales=scales, y=y, lora_rank=rank, lora_nseg=3,
+                                    lora_seg_end=ends, lora_seg_toff=[0, rank, 2 * rank], t=t, t_ld=3 * rank, lora_b=b, lora_scale=scale,
+                                    w_expanded=ops.qw_expand(codes, scales, K, N, 64, Q.NF4)))
+  assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (K + rank) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("K,counts", [(128, (70, 0, 129, 40)), (4096, (1300, 1255))])
+def test_many_rows_experts_from_expanded_copies(gpu, K, counts):
+  """Row blocks of 128 and of 256 routes: experts without rows, blocks that end inside a tile."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  E, N, n = len(counts), 272, sum(counts)
+  g = torch.Generator(device=gpu).manual_seed(n)
+  x = torch.randn(n, K, generator=g, device=gpu).bfloat16()
+  w = (torch.randn(E, N, K, generator=g, device=gpu) * K ** -0.5).bfloat16()
+  bank = torch.stack([ops.dense_expand(e) for e in w])
+  route = torch.randperm(n, generator=torch.Generator().manual_seed(1)).to(torch.int32).to(gpu)
+  offsets = torch.tensor([0] + [int(v) for v in np.cumsum(counts)], dtype=torch.int32, device=gpu)
+  y = torch.full((n, N), float("nan"), dtype=torch.bfloat16, device=gpu)
+  d = L.DenseDesc()
+  d.M, d.K, d.N, d.dtype, d.batch, d.split_k = n, K, N, ops.DTYPES[torch.bfloat16], 1, 1
+  d.x, d.ldx, d.w, d.w_stride, d.epilogue, d.y, d.ldy = x.data_ptr(), K, bank.data_ptr(), bank[0].numel(), L.TNX_EPI_STORE, y.data_ptr(), N
+  d.n_experts, d.x_div, d.offsets, d.sorted_route = E, 1, offsets.data_ptr(), route.data_ptr()
+  ops.dense_linear(d)
+  for e, (a0, a1) in enumerate(zip(offsets.tolist()[:-1], offsets.tolist()[1:])):
+    xe, we = x[route[a0:a1].long()].double(), w[e].double()
+    want = xe @ we.T
+    assert ((y[route[a0:a1].long()].double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()

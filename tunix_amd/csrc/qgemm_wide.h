@@ -22,15 +22,14 @@
 // ids go to consecutive XCDs): the eight row blocks an XCD works on at a time want the same
 // column tile's weights, which its L2 then holds for all of them.
 //
-// From the expanded copy of the weights (kWidePre) a wave needs half the register file, and
-// two work-groups share a compute unit, two waves a SIMD.
+// Weights that a model keeps converted take qgemm_pre.h instead.
 //
-// Included by qlinear.hip after qgemm128.h.
+// Included by qlinear.hip after qgemm128.h and wide_out.h.
 #pragma once
 
 namespace {
 
-constexpr int kWideRows = 128, kWideCols = 256;
+constexpr int kWideRows = 128;
 // LDS: two activation tiles of 128 rows x 128 k (256-byte rows, 16-byte chunks XOR-swizzled by
 // row) at 0 and 32 KB, the table behind them.
 constexpr uint32_t kWideTileBytes = kWideRows * KTILE * 2, kWideLutBase = 2 * kWideTileBytes;
@@ -49,29 +48,14 @@ __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
 // (expert, row block) is found from the expert offsets by a running sum; activation rows are
 // gathered through sorted_route (row = route / x_div), output rows are routes.  No adapter, no
 // lm_head statistics in this mode.
-// MODE: where the bf16 weight fragments come from.  kWideTable: codes through the LDS table;
-// kWideInt4: integer codes converted without the table (Int4Magic in common.h); kWidePre: a copy
-// of the weights that was converted once, bf16(bf16(level) * scale), and laid out as the
-// fragments themselves (tnx_qw_expand: [column tile][k-tile][wave][column group][slab][lane] x
-// 16 bytes), so that a lane's fragment of a slab is one 16-byte load and the loop has neither
-// conversion instructions nor look-ups.  The frozen base weights of a model fit HBM a second time
-// in that form; rows in the hundreds of thousands per weight byte make its four times larger
-// stream irrelevant.  Same MFMA sequence on the same operand bits: results are bit-identical.
-constexpr int kWideTable = 0, kWideInt4 = 1, kWidePre = 2;
-// kWidePre keeps so little besides its accumulators in registers that two of its waves fit one
-// SIMD (128 accumulator registers + 128 others each) and two of its work-groups one compute unit
-// (68 KB of LDS each: the two activation tiles, later the output stage): each covers the other's
-// barriers, first loads and epilogue.
-constexpr int kWidePreStages = 6;   // slabs of weight fragments in flight per wave
-constexpr size_t kWidePreSmemBytes = 68 * 1024;
-static_assert(kWidePreSmemBytes >= 2 * kWideTileBytes && kWidePreSmemBytes >= kWideRows * (kWideCols + 8) * 2,
-              "the activation tiles and the output stage fit");
-static_assert(24 % kWidePreStages == 0, "a stage keeps its slot over the three unrolled k-tiles");
+// MODE: how codes become bf16 weight fragments.  kWideTable: through the LDS table; kWideInt4: integer codes
+// converted without the table (Int4Magic in common.h).
+constexpr int kWideTable = 0, kWideInt4 = 1;
 template <int SPT, bool GROUPED = false, int MODE = kWideTable>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(MODE == kWidePre ? 2 : 1, MODE == kWidePre ? 2 : 1)))
+__attribute__((amdgpu_waves_per_eu(1, 1)))
 void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
-  constexpr bool INT4 = MODE == kWideInt4, PRE = MODE == kWidePre;
+  constexpr bool INT4 = MODE == kWideInt4;
   constexpr int RT = 4, CG = 2, PF = 3, AP = 8;   // 32-row tiles, 32-column groups per wave
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -143,8 +127,8 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
   const u32x4 rx = GROUPED ? raw_rsrc(a.x, (uint64_t)(a.M / a.x_div) * a.K * 2)
                            : raw_rsrc(a.x + m0 * a.K, (uint64_t)rows_here * a.K * 2);
   const uint64_t ntk = (uint64_t)ntiles * ktiles;
-  const rsrc_t rc = make_rsrc(a.codes + (GROUPED && !PRE ? (int64_t)expert * a.codes_stride : 0), ntk * 1024);
-  const rsrc_t rs = make_rsrc(a.scales + (GROUPED && !PRE ? (int64_t)expert * a.scales_stride : 0), ntk * 16 * SPT * 2 + 16);
+  const rsrc_t rc = make_rsrc(a.codes + (GROUPED ? (int64_t)expert * a.codes_stride : 0), ntk * 1024);
+  const rsrc_t rs = make_rsrc(a.scales + (GROUPED ? (int64_t)expert * a.scales_stride : 0), ntk * 16 * SPT * 2 + 16);
   // Lane l: column l % 32 of a group = column (l % 16) of packed tile 2 cg + (l % 32) / 16.  A
   // packed tile holds, at chunk 16 q + c, the k-groups 8 q + 32 j (dword j) of its column c;
   // slab u of the MFMA wants k-group 2 u + l / 32 from this lane: chunk q = l / 32 gives the
@@ -204,19 +188,6 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
   };
   u32x4 xf[2][RT];           // activation fragments of the current / next slab
   u32x4 wf[2][CG];           // weight fragments of the current / next slab
-  // PRE: the fragments of the next kWidePreStages slabs, loaded as they are; stage = slab % stages
-  u32x4 wr[PRE ? kWidePreStages : 1][CG];
-  const rsrc_t re = make_rsrc(PRE ? (const void*)(a.w_pre + (GROUPED ? (int64_t)expert * tiles_n * ktiles * 32768 : 0)) : (const void*)a.x,
-                              PRE ? (uint64_t)tiles_n * (uint64_t)ktiles * 65536u : 0u);
-  uint32_t evoff[CG];
-#pragma unroll
-  for (int cg = 0; cg < CG; ++cg) evoff[cg] = (uint32_t)(((wn * CG + cg) * 8 * 64 + lane) * 16);
-  // slab `sl` (counted from this work-group's first k-tile) of column group cg -> its stage
-  auto load_pre = [&](int sl, int u, int cg) {
-    const int kt_ = min(sl >> 3, ktiles - 1);
-    wr[PRE ? sl % kWidePreStages : 0][cg] =
-        __builtin_amdgcn_raw_buffer_load_b128(re, evoff[cg] + (uint32_t)u * 1024u, (ntile * ktiles + kt_) * 65536, 0);
-  };
   // f16 level pairs of the slab after the next (table path: entry b = the pair of byte b, looked
   // up into the place of the entry just consumed; INT4: entries as described above, the slab's
   // parity picks the set, since a set is read until its slab has been converted)
@@ -365,18 +336,6 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int cg = i >> 2, rt = i & 3;
-      if constexpr (PRE) {
-        // the fragment as loaded; once a column group's four MFMAs have read it, its stage takes
-        // the same group's fragment of the slab kWidePreStages further on
-        constexpr int SL = D * 8 + U;
-        acc[rt][cg] = mfma32(wr[SL % kWidePreStages][cg], xf[CUR][rt], acc[rt][cg]);
-        if (rt == 3) {
-          const int sl = kt * 8 + U + kWidePreStages;   // (kt counts from this work-group's first k-tile: no k split here)
-          const int kt_ = min(sl >> 3, ktiles - 1);
-          wr[SL % kWidePreStages][cg] = __builtin_amdgcn_raw_buffer_load_b128(
-              re, evoff[cg] + (uint32_t)((U + kWidePreStages) & 7) * 1024u, (ntile * ktiles + kt_) * 65536, 0);
-        }
-      } else {
       acc[rt][cg] = mfma32(wf[CUR][cg], xf[CUR][rt], acc[rt][cg]);
       {
         // the pack of the pair before this one (a slot behind its products: packed in the same
@@ -387,15 +346,14 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
         pair_products(lp[INT4 ? (UC & 1) : 0][cg], rt, DC, cg, SPT == 2 ? (UC >> 2) : (UC >> 1), cf0, cf1);
         lp[INT4 ? (UL & 1) : 0][cg][rt] = level_entry(ring_c[DL][cg][UL & 1][UL >> 1], rt);
       }
-      }
       if ((i & 1) == 0) xf[NXT][i >> 1] = lds_ld128(xaddr[UC] + (uint32_t)((i >> 1) * 32 * 256));
       if (i == 7) xaddr[UC] ^= kWideTileBytes;
       if (LD) dma16(dma_buf + dma_wave + (uint32_t)i * 4096u, xr, xoff(i, xo, xst), xs);
-      if (LW && !PRE) {
+      if (LW) {
         if (i < 4) ring_c[D][i >> 1][i & 1] = __builtin_amdgcn_raw_buffer_load_b128(rc, coff[i >> 1] + (uint32_t)(i & 1) * 512u, wkt * 1024, 0);
         else if (i < 6) load_scale(Dc, i - 4, wkt);
       }
-      if (EX && !PRE && i < CG * SPT) {
+      if (EX && i < CG * SPT) {
         const uint32_t w = ring_s[DN][i / SPT][(i % SPT) >> 1];
         set_scale(DN, i / SPT, i % SPT, next_active ? (((i % SPT) & 1) ? bfhi(w) : bflo(w)) : 0.f);
       }
@@ -414,9 +372,8 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
     slab(ic<5>{}, Dc, kt, next_active);
     slab(ic<6>{}, Dc, kt, next_active);
     // the next tile's activations, requested by slab 7 of the tile before, have landed in LDS:
-    // the only younger loads are the six weight / scale loads slab 6 has just issued (PRE: the
-    // second fragment load of that slab 7 and the two of each slab since, fifteen)
-    tnx_wait_vm(PRE ? 14 : 6);
+    // the only younger loads are the six weight / scale loads slab 6 has just issued
+    tnx_wait_vm(6);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
     slab(ic<7>{}, Dc, kt, next_active);
@@ -427,14 +384,7 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
   // in the steady state of the loop, so the counted waits of the loop body never have to fall
   // back to "everything outstanding" for the sake of the path that enters from here)
   load_a(0, 0u);
-  if constexpr (PRE) {
-#pragma unroll
-    for (int sl = 0; sl < kWidePreStages; ++sl)
-#pragma unroll
-      for (int cg = 0; cg < CG; ++cg) load_pre(sl, sl & 7, cg);
-  } else {
-    load_w(ic<0>{}, 0);
-  }
+  load_w(ic<0>{}, 0);
   if constexpr (MODE == kWideTable) {  // table entry e = f16 pair (level[e & 15], level[e >> 4]), 64 copies rotated over the banks
     uint32_t* lut = reinterpret_cast<uint32_t*>(smem + kWideLutBase);
     const h16x2 h = {(_Float16)lvl0, (_Float16)lvl1};
@@ -443,12 +393,9 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
     for (int c = 0; c < 64; ++c) lut[tid * 64 + ((c + lane) & 63)] = v;
   }
   load_a(1, kWideTileBytes);
-  if constexpr (!PRE) {
-    load_w(ic<1>{}, 1);
-    load_w(ic<2>{}, 2);
-  }
-  // the adapter's B^T fragments: up front, or (two work-groups per unit: no registers to park
-  // them in) behind the loop, where the other work-group covers their round trip
+  load_w(ic<1>{}, 1);
+  load_w(ic<2>{}, 2);
+  // the adapter's B^T fragments, up front
   auto load_adapter_b = [&]() {
     const rsrc_t rb = make_rsrc(a.lora_b, (uint64_t)a.N * a.lora_rank * 2);
 #pragma unroll
@@ -459,36 +406,30 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
           lbv[cg][u] = buf_load128(rb, (((uint32_t)(ntile0 + 2 * cg) * 16u + (uint32_t)l32) * (uint32_t)a.lora_rank +
                                         (uint32_t)(u * 16 + lh * 8)) * 2u);
   };
-  constexpr bool LATE_B = PRE;
-  if (lora && !LATE_B) load_adapter_b();
-  if constexpr (!PRE) expand_scales(ic<0>{}, true);
+  if (lora) load_adapter_b();
+  expand_scales(ic<0>{}, true);
   // the first tile is in LDS: its eight loads are the oldest, and at least 26 follow them (three
   // ring stages of six, the second tile's eight); vmcnt(20) also covers the first ring stage
-  // (PRE: 24 fragment loads and the second tile's eight follow them)
-  tnx_wait_vm(PRE ? 2 * kWidePreStages + 8 : 20);
+  tnx_wait_vm(20);
   __syncthreads();
   // slab 0: table entries, conversion, fragments; then the table entries of slab 1
-  if constexpr (!PRE) {
 #pragma unroll
-    for (int cg = 0; cg < CG; ++cg)
+  for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) lp[0][cg][b] = level_entry(ring_c[0][cg][0][0], b);
-  }
+    for (int b = 0; b < 4; ++b) lp[0][cg][b] = level_entry(ring_c[0][cg][0][0], b);
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) xf[0][rt] = lds_ld128((xaddr[0] ^ kWideTileBytes) + (uint32_t)(rt * 32 * 256));
-  if constexpr (!PRE) {
 #pragma unroll
-    for (int cg = 0; cg < CG; ++cg)
+  for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        pair_products(lp[0][cg], b, 0, cg, 0, cf0, cf1);
-        if (cg < CG - 1 || b < 3) wf[0][cg][b] = cvt_pk_bf16(cf0, cf1);   // the last pair: slot 0 of the loop
-      }
+    for (int b = 0; b < 4; ++b) {
+      pair_products(lp[0][cg], b, 0, cg, 0, cf0, cf1);
+      if (cg < CG - 1 || b < 3) wf[0][cg][b] = cvt_pk_bf16(cf0, cf1);   // the last pair: slot 0 of the loop
+    }
 #pragma unroll
-    for (int cg = 0; cg < CG; ++cg)
+  for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) lp[INT4 ? 1 : 0][cg][b] = level_entry(ring_c[0][cg][1][0], b);
-  }
+    for (int b = 0; b < 4; ++b) lp[INT4 ? 1 : 0][cg][b] = level_entry(ring_c[0][cg][1][0], b);
   // whole turns of the ring without a branch inside (a conditional tile would make the waits
   // of the tile after it assume that its loads never happened), then the one or two tiles left
   int kt = 0;
@@ -503,10 +444,10 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
   }
 
   if (lora) {
-    if constexpr (LATE_B) load_adapter_b();
     // The t block is k-tile number ktiles: it sits in tile buffer ktiles % 2.  The
     // two 16-column halves of a group may belong to different adapters (always so for a
     // gate | up pair): one pass per half then, the other half's lanes contributing zeros.
+    const bool in_place = lora_in_place(a.lora_scale);   // (as qgemm_pre.h: the same sums in the same order)
 #pragma unroll
     for (int cg = 0; cg < CG; ++cg) {
       const bool same = toff[2 * cg] == toff[2 * cg + 1];
@@ -514,7 +455,13 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) part[rt][i] = 0.f;
+        for (int i = 0; i < 16; ++i) part[rt][i] = in_place ? acc[rt][cg][i] : 0.f;
+      if (in_place) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) lbv[cg][u][q] = pack2bf(bflo(lbv[cg][u][q]) * a.lora_scale, bfhi(lbv[cg][u][q]) * a.lora_scale);
+      }
       for (int p = 0; p < (same ? 1 : 2); ++p) {
         const uint32_t half = toff[2 * cg + p] == toff_a ? 0u : 8u;   // first 16-byte chunk of the segment's 64 columns
         const uint32_t base = (uint32_t)(ktiles & 1) * kWideTileBytes + (uint32_t)l32 * 256u;
@@ -533,7 +480,7 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[rt][cg][i] += a.lora_scale * part[rt][i];
+        for (int i = 0; i < 16; ++i) acc[rt][cg][i] = in_place ? part[rt][i] : acc[rt][cg][i] + a.lora_scale * part[rt][i];
     }
   }
   tnx_wait_vm(0);   // no load into LDS is still on its way
@@ -542,48 +489,7 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
   // The bf16 tile goes through LDS (row stride cols + 8 elements) and leaves as 16-byte chunks
   // of whole rows.  A lane holds, for row rt * 32 + l % 32 and group cg, the columns
   // 8 b + 4 (l / 32) + e of the group in register 4 b + e.
-  const bool mul = a.epilogue == TNX_EPI_SILU_MUL || a.epilogue == TNX_EPI_GELU_MUL || a.epilogue == kEpiGeluMulF32 || a.epilogue == kEpiSiluMulF32;
-  if constexpr (PRE) {
-    if (a.epilogue == TNX_EPI_F32) {   // fp32 results leave from the accumulators, 16 bytes per lane
-      float* y = reinterpret_cast<float*>(a.y);
-#pragma unroll
-      for (int cg = 0; cg < CG; ++cg)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const int64_t col = (int64_t)ntile * kWideCols + wn * 64 + cg * 32 + 8 * b + 4 * lh;
-            float* o = y + (m0 + rt * 32 + l32) * a.ldy + col;
-            if (rt * 32 + l32 >= rows_here) continue;
-            if (col + 4 <= a.N && (a.ldy & 3) == 0) {
-              *reinterpret_cast<f32x4*>(o) = f32x4{acc[rt][cg][4 * b], acc[rt][cg][4 * b + 1], acc[rt][cg][4 * b + 2], acc[rt][cg][4 * b + 3]};
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                if (col + e < a.N) o[e] = acc[rt][cg][4 * b + e];
-            }
-          }
-      return;
-    }
-  }
-  if constexpr (PRE) {
-    if (a.epilogue == TNX_EPI_RELU2) {
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int cg = 0; cg < CG; ++cg)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[rt][cg][i] = fmaxf(acc[rt][cg][i], 0.f) * fmaxf(acc[rt][cg][i], 0.f);
-    }
-    if (h.part != nullptr && h.softcap > 0.f) {
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int cg = 0; cg < CG; ++cg)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[rt][cg][i] = soft_cap_fast(acc[rt][cg][i], h.softcap);
-    }
-  }
+  const bool mul = a.epilogue == TNX_EPI_SILU_MUL || a.epilogue == TNX_EPI_GELU_MUL;
   const int cols = mul ? kWideCols / 2 : kWideCols;      // output columns of the work-group
   const int sld = cols + 8;
   const uint32_t stage = 0;   // 128 rows x (256 + 8) columns: over both tiles and into the table, all dead now
@@ -598,17 +504,6 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
           float v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            if (PRE && a.epilogue == kEpiSiluMulF32) {
-              const float z = acc[rt][cg][4 * b + e];
-              v[e] = z / (1.0f + expf(-z)) * acc[rt][cg][4 * (b + 2) + e];
-              continue;
-            }
-            if (PRE && a.epilogue == kEpiGeluMulF32) {
-              const float z = acc[rt][cg][4 * b + e];
-              v[e] = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))) *
-                     acc[rt][cg][4 * (b + 2) + e];
-              continue;
-            }
             const float g = rbf(acc[rt][cg][4 * b + e]);
             const float u = rbf(acc[rt][cg][4 * (b + 2) + e]);
             const float act = a.epilogue == TNX_EPI_SILU_MUL ? silu_bf16(g) : gelu_tanh_bf16(g);
@@ -632,179 +527,9 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
         }
   }
   __syncthreads();
-  if (h.part != nullptr && h.logits_out != nullptr) {
-    // the raw logits (no temperature) as fp32: a wave writes one row of the tile at a time, a
-    // lane four columns (1 KB per row, whole lines)
-    const int64_t c0 = (int64_t)ntile * kWideCols + lane * 4;
-    for (int row = wn; row < rows_here; row += 4) {
-      const u32x2 v = *reinterpret_cast<const __attribute__((address_space(3))) u32x2*>(
-          static_cast<uintptr_t>(stage + (uint32_t)((row * sld + lane * 4) * 2)));
-      float* o = h.logits_out + (m0 + row) * a.N + c0;
-      if (c0 + 4 <= a.N) {
-        *reinterpret_cast<f32x4*>(o) = f32x4{bflo(v[0]), bfhi(v[0]), bflo(v[1]), bfhi(v[1])};
-      } else {
-        const float x[4] = {bflo(v[0]), bfhi(v[0]), bflo(v[1]), bfhi(v[1])};
-        for (int e = 0; e < 4; ++e)
-          if (c0 + e < a.N) o[e] = x[e];
-      }
-    }
-  }
-  if (h.part != nullptr) {
-    // lm_head: thread (row, half) reduces the row's 128 staged logits of column block
-    // 2 * ntile + half to (max, first arg-max, sum of exp(l - max), logit of the row's target)
-    const int row = tid & 127, half = tid >> 7;
-    const int64_t pb = (int64_t)ntile * 2 + half;
-    if (row >= rows_here || pb >= h.nvb) return;
-    const int64_t grow = m0 + row, c0 = pb * 128;
-    const int tg = h.targets ? h.targets[grow] : -1;
-    const uint32_t base = stage + (uint32_t)((row * sld + half * 128) * 2);
-    const float ninf = -__builtin_inff();
-    float mx = ninf, tgt = ninf, se = 0.f, we = 0.f;
-    int idx = (int)c0;
-    // The logits are divided by the temperature in fp32, as the reference does.  At temperature 1
-    // the division is the identity and is left out: an IEEE division is a dozen instructions, and
-    // at two per element it was a seventh of this kernel's time on the log-probability pass.
-    auto reduce = [&](auto unit_c) {
-      constexpr bool unit = decltype(unit_c)::value;
-#pragma unroll 4
-      for (int ch = 0; ch < 16; ++ch) {
-        const u32x4 v = lds_ld128(base + (uint32_t)(ch * 16));
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int64_t col = c0 + ch * 8 + q;
-          const float raw = (q & 1) ? bfhi(v[q >> 1]) : bflo(v[q >> 1]);
-          const float l = col < a.N ? (unit ? raw : __fdiv_rn(raw, h.temperature)) : ninf;
-          if (l > mx) {   // columns ascend: the first maximal index stays
-            mx = l;
-            idx = (int)col;
-          }
-          if ((int)col == tg) tgt = l;
-        }
-      }
-      if (mx != ninf) {
-#pragma unroll 4
-        for (int ch = 0; ch < 16; ++ch) {
-          const u32x4 v = lds_ld128(base + (uint32_t)(ch * 16));
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const int64_t col = c0 + ch * 8 + q;
-            const float raw = (q & 1) ? bfhi(v[q >> 1]) : bflo(v[q >> 1]);
-            if (col < a.N) {
-              const float l = unit ? raw : __fdiv_rn(raw, h.temperature);
-              const float e = __expf(l - mx);
-              se += e;
-              we += e * l;
-            }
-          }
-        }
-      }
-    };
-    // A block that lies wholly inside the vocabulary, no entropy term asked for (every block of a
-    // log-probability pass over a head whose width is a multiple of 128): the same arithmetic in
-    // the same order without the per-element column tests, and the target's logit is read from its
-    // place in the staged row instead of being compared for 128 times.
-    auto reduce_full = [&](auto unit_c) {
-      constexpr bool unit = decltype(unit_c)::value;
-      const int c0i = (int)c0;
-      if (tg >= c0i && tg < c0i + 128) {
-        const uint32_t w = lds_ld32(base + (uint32_t)((tg - c0i) >> 1) * 4u);
-        const float raw = ((tg - c0i) & 1) ? bfhi(w) : bflo(w);
-        tgt = unit ? raw : __fdiv_rn(raw, h.temperature);
-      }
-#pragma unroll 4
-      for (int ch = 0; ch < 16; ++ch) {
-        const u32x4 v = lds_ld128(base + (uint32_t)(ch * 16));
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const float raw = (q & 1) ? bfhi(v[q >> 1]) : bflo(v[q >> 1]);
-          const float l = unit ? raw : __fdiv_rn(raw, h.temperature);
-          if (l > mx) {
-            mx = l;
-            idx = c0i + ch * 8 + q;
-          }
-        }
-      }
-      if (mx != ninf) {
-#pragma unroll 4
-        for (int ch = 0; ch < 16; ++ch) {
-          const u32x4 v = lds_ld128(base + (uint32_t)(ch * 16));
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const float raw = (q & 1) ? bfhi(v[q >> 1]) : bflo(v[q >> 1]);
-            const float l = unit ? raw : __fdiv_rn(raw, h.temperature);
-            se += __expf(l - mx);
-          }
-        }
-      }
-    };
-    // The whole-vocabulary draw: the statistics of the general form and, per column, the logit
-    // plus the Gumbel noise of element row * N + col of rows_total * N; the block's best (first
-    // among equals: columns ascend), its id and its logit go to part_draw.
-    if (h.part_draw != nullptr) {
-      uint32_t ks0 = 0u, ks1 = (uint32_t)(*h.step_ptr);
-      threefry2x32(h.key0, h.key1, ks0, ks1);   // fold_in(key, step)
-      const uint64_t total = (uint64_t)h.rows_total * (uint64_t)a.N;
-      float gv = ninf, gl = ninf;
-      int gi = 0x7fffffff;
-      for (int ch = 0; ch < 16; ++ch) {
-        const u32x4 v = lds_ld128(base + (uint32_t)(ch * 16));
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int64_t col = c0 + ch * 8 + q;
-          if (col < a.N) {
-            const float raw = (q & 1) ? bfhi(v[q >> 1]) : bflo(v[q >> 1]);
-            const float l = __fdiv_rn(raw, h.temperature);
-            const float n = l + gumbel_from_bits(random_bits(ks0, ks1, (uint64_t)grow * (uint64_t)a.N + (uint64_t)col,
-                                                             total, h.variant));
-            if (n > gv) {
-              gv = n;
-              gi = (int)col;
-              gl = l;
-            }
-          }
-        }
-      }
-      float* q3 = h.part_draw + (grow * h.nvb + pb) * 3;
-      q3[0] = gv;
-      q3[1] = __int_as_float(gi);
-      q3[2] = gl;
-    }
-    const bool plain = c0 + 128 <= a.N && h.part_ent == nullptr;
-    if (h.temperature == 1.0f) {
-      if (plain) reduce_full(std::true_type{});
-      else reduce(std::true_type{});
-    } else {
-      if (plain) reduce_full(std::false_type{});
-      else reduce(std::false_type{});
-    }
-    float* p = h.part + (grow * h.nvb + pb) * 4;
-    p[0] = mx;
-    p[1] = __int_as_float(idx);
-    p[2] = se;
-    p[3] = tgt;
-    if (h.part_ent) h.part_ent[grow * h.nvb + pb] = we;
-    return;
-  }
-  {
-    const int64_t width = mul ? a.N / 2 : a.N, ldy = a.ldy > 0 ? a.ldy : width;
-    const int64_t col0 = (int64_t)ntile * cols;
-    const int chunks = cols / 8;                       // 16-byte chunks per row: 16 | 32
-    const int ch = tid % chunks, r0 = tid / chunks, rstep = 256 / chunks;
-    uint16_t* y = reinterpret_cast<uint16_t*>(a.y);
-    const bool col_ok = col0 + ch * 8 + 8 <= width;
-    for (int row = r0; row < kWideRows; row += rstep) {
-      if (row >= rows_here || !col_ok) continue;
-      u32x4 v = lds_ld128(stage + (uint32_t)((row * sld + ch * 8) * 2));
-      const int64_t orow = GROUPED ? (int64_t)a.sorted_route[m0 + row] : m0 + row;
-      const int64_t o = orow * ldy + col0 + ch * 8;
-      if (a.epilogue == TNX_EPI_RESIDUAL) {
-        const u32x4 res = *reinterpret_cast<const u32x4*>(a.residual + o);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = pack2bf(bflo(v[q]) + bflo(res[q]), bfhi(v[q]) + bfhi(res[q]));
-      }
-      *reinterpret_cast<u32x4*>(y + o) = v;
-    }
-  }
+  if (mul) wide_tile_out<kWideRows, GROUPED, false, true>(a, h, ntile, m0, rows_here);
+  else if (!GROUPED && h.part != nullptr) wide_tile_out<kWideRows, GROUPED, true, false>(a, h, ntile, m0, rows_here);
+  else wide_tile_out<kWideRows, GROUPED, false, false>(a, h, ntile, m0, rows_here);
 }
 
 }  // namespace

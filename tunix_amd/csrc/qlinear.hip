@@ -47,7 +47,7 @@ struct QLArgs {
 // gate | up with the activation and the product in fp32 and one rounding (dense-weight decoders;
 // many-row kernel only)
 constexpr int kEpiGeluMulF32 = 16, kEpiSiluMulF32 = 17;
-// Second argument of the 128 x 256 kernel: with `part` set it reduces its tile to lm_head
+// Second argument of the many-row kernels: with `part` set they reduce their tile to lm_head
 // statistics instead of storing it.
 struct WideHead {
   float* part;               // [M, nvb, 4]: max, first arg-max, sum of exp, target logit
@@ -67,8 +67,9 @@ struct WideHead {
 };
 
 __device__ __forceinline__ float silu_bf16(float g) {
-  // jax.nn.silu = x * sigmoid(x) as two bf16 HLO ops.
-  float s = rbf(1.0f / (1.0f + __expf(-g)));
+  // jax.nn.silu = x * sigmoid(x) as two bf16 HLO ops.  (The hardware reciprocal, one ulp of fp32 in front of a rounding
+  // to eight bits: an IEEE division is ten instructions more per element.)
+  float s = rbf(__builtin_amdgcn_rcpf(1.0f + __expf(-g)));
   return rbf(g * s);
 }
 __device__ __forceinline__ float gelu_tanh_bf16(float g) {
@@ -184,7 +185,9 @@ __global__ __launch_bounds__(256) void moe_gmm_kernel(const QLArgs a) {
 
 }  // namespace
 #include "qgemm128.h"
+#include "wide_out.h"
 #include "qgemm_wide.h"
+#include "qgemm_pre.h"
 #include "moe_gmm16.h"
 namespace {
 
@@ -698,7 +701,7 @@ int raise_lds_limit(Kern kern, size_t bytes) {
   return TNX_OK;
 }
 
-// qgemm128_kernel and qgemm_wide_kernel address LDS absolutely (their table sits at LDS address 0),
+// qgemm128_kernel, qgemm_wide_kernel and qgemm_pre_kernel address LDS absolutely (their table sits at LDS address 0),
 // which holds as long as they have no static LDS: checked here, once per instantiation, before the
 // first launch.
 template <class Kern>
@@ -740,7 +743,7 @@ template <int SPT, int MODE>
 int launch_qgemm_wide_as(hipStream_t st, const QLArgs& a, const WideHead& h) {
   static std::once_flag once;
   static int attr_rc = TNX_OK;
-  constexpr size_t kSmem = MODE == kWidePre ? kWidePreSmemBytes : kWideSmemBytes;
+  constexpr size_t kSmem = kWideSmemBytes;
   std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_wide_kernel<SPT, false, MODE>, kSmem); });
   if (attr_rc) return attr_rc;
   const unsigned wgs = (unsigned)(cdiv(a.M, kWideRows) * cdiv(a.N, kWideCols));
@@ -749,12 +752,79 @@ int launch_qgemm_wide_as(hipStream_t st, const QLArgs& a, const WideHead& h) {
   return TNX_OK;
 }
 
+constexpr WideHead kNoHead{nullptr, nullptr, nullptr, 0, 1.0f, nullptr};
+
+template <int RT, bool GROUPED, int KIND, int LORA>
+int launch_qgemm_pre_as(hipStream_t st, const QLArgs& a, const WideHead& h) {
+  static std::once_flag once;
+  static int attr_rc = TNX_OK;
+  constexpr size_t kSmem = pre_smem_bytes<RT>();
+  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_pre_kernel<RT, GROUPED, KIND, LORA>, kSmem); });
+  if (attr_rc) return attr_rc;
+  // grouped: an upper bound of the row blocks, sum over the experts of ceil(rows / ROWS) <= n_routes / ROWS + E (work-groups
+  // past the last block exit at once)
+  const int64_t blocks = GROUPED ? a.M / (16 * RT) + a.n_experts : cdiv(a.M, 16 * RT);
+  hipLaunchKernelGGL((qgemm_pre_kernel<RT, GROUPED, KIND, LORA>), dim3((unsigned)(blocks * cdiv(a.N, kWideCols))), dim3(256), kSmem, st, a, h);
+  TNX_CHECK_LAUNCH("qgemm_pre");
+  return TNX_OK;
+}
+
+template <int RT, int KIND>
+int launch_qgemm_pre_lora(hipStream_t st, const QLArgs& a, const WideHead& h) {
+  if (a.lora_rank <= 0) return launch_qgemm_pre_as<RT, false, KIND, 0>(st, a, h);
+  return lora_in_place(a.lora_scale) ? launch_qgemm_pre_as<RT, false, KIND, kLoraInPlace>(st, a, h)
+                                     : launch_qgemm_pre_as<RT, false, KIND, kLoraScaled>(st, a, h);
+}
+
+template <int RT>
+int launch_qgemm_pre_rt(hipStream_t st, const QLArgs& a, const WideHead& h) {
+  if (h.part) return launch_qgemm_pre_lora<RT, kPreHead>(st, a, h);
+  switch (a.epilogue) {
+    case TNX_EPI_STORE: case TNX_EPI_RESIDUAL: return launch_qgemm_pre_lora<RT, kPreStore>(st, a, h);
+    case TNX_EPI_SILU_MUL: return launch_qgemm_pre_lora<RT, kPreSilu>(st, a, h);
+    case TNX_EPI_GELU_MUL: return launch_qgemm_pre_lora<RT, kPreGelu>(st, a, h);
+    default: break;
+  }
+  TNX_REQUIRE(a.lora_rank <= 0, "many-row linear: epilogue %d takes no adapter", a.epilogue);
+  switch (a.epilogue) {
+    case TNX_EPI_F32: return launch_qgemm_pre_as<RT, false, kPreF32, 0>(st, a, h);
+    case TNX_EPI_RELU2: return launch_qgemm_pre_as<RT, false, kPreRelu2, 0>(st, a, h);
+    case kEpiSiluMulF32: return launch_qgemm_pre_as<RT, false, kPreSiluF32, 0>(st, a, h);
+    case kEpiGeluMulF32: return launch_qgemm_pre_as<RT, false, kPreGeluF32, 0>(st, a, h);
+    default: break;
+  }
+  TNX_REQUIRE(false, "many-row linear: bad epilogue %d", a.epilogue);
+}
+
+// Row tiles of a call: 256 rows run one work-group per compute unit at 1.45 PFLOP/s with about 150 k's worth of time
+// between two tiles, 128 rows two per unit (each covers the other's) at 8 % less.  What decides is mostly how full the last round
+// is: us at 256 | 128 rows, 16384 x 14336 -> 4096: 1310 | 1431, 2048 x 4096 -> 28672: 377 | 366 (3.5 rounds), 8704 x 4096 ->
+// 4096: 261 | 222 (2.1 rounds), 16384 x 1152 -> 13824: 453 | 414, 8192 x 2048 -> 16384: 448 | 477.
+int launch_qgemm_pre(hipStream_t st, const QLArgs& a, const WideHead& h) {
+  const int64_t tn = cdiv(a.N, kWideCols);
+  const double tall = (double)cdiv(cdiv(a.M, 256) * tn, 256) * (double)(a.K + 150);
+  const double low = 0.5 * (double)cdiv(cdiv(a.M, 128) * tn, 256) * 1.09 * (double)a.K;
+  return tall < low ? launch_qgemm_pre_rt<16>(st, a, h) : launch_qgemm_pre_rt<8>(st, a, h);
+}
+
+template <int RT>
+int launch_qgemm_pre_grouped_rt(hipStream_t st, const QLArgs& a) {
+  switch (a.epilogue) {
+    case TNX_EPI_STORE: return launch_qgemm_pre_as<RT, true, kPreStore, 0>(st, a, kNoHead);
+    case TNX_EPI_RELU2: return launch_qgemm_pre_as<RT, true, kPreRelu2, 0>(st, a, kNoHead);
+    case kEpiSiluMulF32: return launch_qgemm_pre_as<RT, true, kPreSiluF32, 0>(st, a, kNoHead);
+    case kEpiGeluMulF32: return launch_qgemm_pre_as<RT, true, kPreGeluF32, 0>(st, a, kNoHead);
+    default: break;
+  }
+  TNX_REQUIRE(false, "experts over many rows: bad epilogue %d", a.epilogue);
+}
+
 template <int SPT>
-int launch_qgemm_wide(hipStream_t st, const QLArgs& a, const WideHead& h = WideHead{nullptr, nullptr, nullptr, 0, 1.0f, nullptr}) {
+int launch_qgemm_wide(hipStream_t st, const QLArgs& a, const WideHead& h = kNoHead) {
   // the converted copy when the caller keeps one (its block offsets are 32-bit); else integer
   // codes take the instantiation that converts them without the table
   if (a.w_pre && cdiv(a.N, kWideCols) * (a.K / KTILE) * 65536 < (int64_t)1 << 31)
-    return launch_qgemm_wide_as<2, kWidePre>(st, a, h);
+    return launch_qgemm_pre(st, a, h);
   TNX_REQUIRE(a.codes && a.scales, "quantised GEMM: no packed weights and no usable expanded copy");
   return a.qtype == TNX_Q_INT4 ? launch_qgemm_wide_as<SPT, kWideInt4>(st, a, h)
                                : launch_qgemm_wide_as<SPT, kWideTable>(st, a, h);
@@ -766,13 +836,12 @@ template <int SPT, int MODE>
 int launch_qgemm_wide_grouped_as(hipStream_t st, const QLArgs& a) {
   static std::once_flag once;
   static int attr_rc = TNX_OK;
-  constexpr size_t kSmem = MODE == kWidePre ? kWidePreSmemBytes : kWideSmemBytes;
+  constexpr size_t kSmem = kWideSmemBytes;
   std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_wide_kernel<SPT, true, MODE>, kSmem); });
   if (attr_rc) return attr_rc;
   const int64_t blocks = a.M / kWideRows + a.n_experts;
   const unsigned wgs = (unsigned)(blocks * cdiv(a.N, kWideCols));
-  hipLaunchKernelGGL((qgemm_wide_kernel<SPT, true, MODE>), dim3(wgs), dim3(256), kSmem, st, a,
-                     WideHead{nullptr, nullptr, nullptr, 0, 1.0f, nullptr});
+  hipLaunchKernelGGL((qgemm_wide_kernel<SPT, true, MODE>), dim3(wgs), dim3(256), kSmem, st, a, kNoHead);
   TNX_CHECK_LAUNCH("qgemm_wide_grouped");
   return TNX_OK;
 }
@@ -782,7 +851,7 @@ int launch_qgemm_wide_grouped(hipStream_t st, const QLArgs& a) {
   return a.qtype == TNX_Q_INT4 ? launch_qgemm_wide_grouped_as<SPT, kWideInt4>(st, a) : launch_qgemm_wide_grouped_as<SPT, kWideTable>(st, a);
 }
 
-// Shapes the 128 x 256 kernel takes: enough rows to fill the device with its tiles, no k split,
+// Shapes the many-row kernels take: enough rows to fill the device with its tiles, no k split,
 // a bf16 output whose rows can be written in 16-byte chunks, and an adapter (if any) of rank
 // <= 64 none of whose 256-column windows touches more than two segments.
 bool wide_shape(const QLArgs& a, int64_t min_rows = 512) {
@@ -963,7 +1032,7 @@ extern "C" int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* d) {
   return s2 ? launch_qgemm128<2, 2, 8>(st, a) : launch_qgemm128<2, 4, 8>(st, a);
 }
 
-// The quantised lm_head over many rows on the 128 x 256 kernel: per 128-column block statistics
+// The lm_head over many rows on the many-row kernels: per 128-column block statistics
 // in the layout lmhead_kernel writes, so the same finishing kernel merges them.  Returns 1 when
 // the shape is not one the kernel takes (the caller then uses its own kernel), 0 when launched.
 int tnx_internal_wide_head(hipStream_t st, const tnx_lmhead_desc* d, float temperature, int64_t nvb,
@@ -1007,7 +1076,7 @@ int tnx_internal_wide_head(hipStream_t st, const tnx_lmhead_desc* d, float tempe
 static int once_rounded(int epilogue) {
   return epilogue == TNX_EPI_GELU_MUL ? kEpiGeluMulF32 : epilogue == TNX_EPI_SILU_MUL ? kEpiSiluMulF32 : epilogue;
 }
-// A dense linear over many rows on the 128 x 256 kernel, from its fragment-order weights
+// A dense linear over many rows (qgemm_pre.h), from its fragment-order weights
 // (tnx_dense_expand).  The caller has checked the shapes.
 int tnx_internal_wide_dense(hipStream_t st, int64_t M, int64_t K, int64_t N, const uint16_t* x, const uint16_t* w,
                             int epilogue, void* y, int64_t ldy) {
@@ -1029,7 +1098,10 @@ int tnx_internal_wide_dense_grouped(hipStream_t st, int64_t n_routes, int64_t K,
   a.epilogue = once_rounded(epilogue);
   a.y = y; a.ldy = ldy; a.split_k = 1; a.ktiles_per_split = (int)(K / KTILE);
   a.n_experts = n_experts; a.offsets = offsets; a.sorted_route = sorted_route;
-  return launch_qgemm_wide_grouped_as<2, kWidePre>(st, a);
+  // as launch_qgemm_pre, with half a row block per expert left empty on average
+  const double avg = (double)n_routes / (double)n_experts;
+  const bool tall = (avg + 128.0) * (double)(K + 150) < (avg + 64.0) * 1.09 * (double)K;
+  return tall ? launch_qgemm_pre_grouped_rt<16>(st, a) : launch_qgemm_pre_grouped_rt<8>(st, a);
 }
 
 extern "C" int tnx_splitk_finish(void* stream, const tnx_qlinear_desc* d) {
