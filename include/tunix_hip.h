@@ -79,9 +79,10 @@ const char* tnx_last_error(void);
  * tnx_parallel_step, tnx_conv_kvwrite, tnx_mixed_attn, tnx_memory and tnx_soft_cap; 6.0 adds learned positions to
  * tnx_embed_rows, centred norms, a factor, an extra row and the depth average to tnx_residual_norm_desc, slopes and
  * chunks to tnx_sink_attn_desc, an ungated form and shared weights to tnx_gated_norm_desc, TNX_EPI_RELU2, and
- * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores. */
+ * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
+ * tnx_moe_gmm_expanded and tnx_qw_expand_bank. */
 #define TNX_ABI_VERSION_MAJOR 6
-#define TNX_ABI_VERSION_MINOR 0
+#define TNX_ABI_VERSION_MINOR 1
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
 int tnx_version(void);
 
@@ -134,6 +135,10 @@ int tnx_qw_dequant(void* stream, const uint32_t* codes, const uint16_t* scales, 
 size_t tnx_qw_expanded_bytes(int64_t K, int64_t N);
 int tnx_qw_expand(void* stream, const uint32_t* codes, const uint16_t* scales, int64_t K, int64_t N,
                   int group, int qtype, uint16_t* w_expanded /* 16-byte aligned */);
+/* The same for E weights of one shape behind each other (an expert bank: codes and scales tnx_qw_sizes apart, copies
+ * tnx_qw_expanded_bytes apart). */
+int tnx_qw_expand_bank(void* stream, const uint32_t* codes, const uint16_t* scales, int64_t E, int64_t K, int64_t N,
+                       int group, int qtype, uint16_t* w_expanded);
 /* The same layout from a dense bf16 matrix w[N][K] (an unquantised or tied lm_head, [V][D]): a
  * log-probability pass over 512 rows or more then runs the head on the many-row kernel
  * (tnx_lmhead_desc.w_expanded next to w_bf16) instead of the 128 x 128 one. */
@@ -475,6 +480,9 @@ typedef struct tnx_moe_gmm_desc {
   uint16_t* y;               /* bf16 [n_routes, N or N/2], indexed by route                  */
 } tnx_moe_gmm_desc;
 int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* h_desc);
+/* The same with a second copy of the weights: every expert's tnx_qw_expand output, behind each other
+ * (tnx_qw_expanded_bytes(K, N) apart).  Calls with enough rows per expert read the copy, others the codes. */
+int tnx_moe_gmm_expanded(void* stream, const tnx_moe_gmm_desc* h_desc, const uint16_t* w_expanded);
 /* out[m,:] = bf16( sum_j f32(topk_w[m,j]) * f32(y[m*k+j,:]) )  (qwen3/model.py:827-832). */
 int tnx_moe_combine(void* stream, const uint16_t* y, const uint16_t* topk_w, int64_t M, int k,
                     int64_t D, const uint16_t* residual, uint16_t* out);

@@ -1814,3 +1814,34 @@ def test_many_rows_experts_from_expanded_copies(gpu, K, counts):
     xe, we = x[route[a0:a1].long()].double(), w[e].double()
     want = xe @ we.T
     assert ((y[route[a0:a1].long()].double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()
+
+
+@pytest.mark.parametrize("M,counts_scale", [(36, 1), (320, 1), (333, 2)])
+@pytest.mark.parametrize("qtype", [Q.INT4, Q.NF4])
+def test_moe_from_the_experts_copies(gpu, M, counts_scale, qtype):
+  """Experts read from their converted copies give the bits that they give from the codes, on both sides of the line between
+  the two, with experts of very different sizes."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  E, k, K, N, group = 4, 2, 256, 512, 64
+  g = torch.Generator(device=gpu).manual_seed(M)
+  w = (torch.randn(E, K, N, generator=g, device=gpu) * 0.05).bfloat16()
+  packed = [ops.quantize_pack(e, group, qtype, True) for e in w]
+  codes, scales = (torch.cat([p[i] for p in packed]) for i in (0, 1))
+  bank = ops.qw_expand_bank(codes, scales, E, K, N, group, qtype)
+  assert torch.equal(bank[2], ops.qw_expand(*packed[2], K, N, group, qtype))
+  ids = torch.stack([(torch.arange(M, device=gpu) // counts_scale) % 3, torch.full((M,), 3, device=gpu)], 1).to(torch.int32)
+  counts, offsets = torch.empty(E, dtype=torch.int32, device=gpu), torch.empty(E + 1, dtype=torch.int32, device=gpu)
+  route = torch.empty(M * k, dtype=torch.int32, device=gpu)
+  ops.moe_sort_routes(ids, E, counts, offsets, route)
+  x = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+  got = []
+  for copies in (None, bank):
+    y = torch.full((M * k, N // 2), float("nan"), dtype=torch.bfloat16, device=gpu)
+    d = L.MoeGmmDesc()
+    d.n_routes, d.E, d.k, d.K, d.N, d.group, d.qtype, d.x, d.x_div = M * k, E, k, K, N, group, qtype, x.data_ptr(), k
+    d.codes, d.scales, d.offsets, d.sorted_route = codes.data_ptr(), scales.data_ptr(), offsets.data_ptr(), route.data_ptr()
+    d.epilogue, d.y = L.TNX_EPI_SILU_MUL, y.data_ptr()
+    ops.moe_gmm(d, copies)
+    got.append(y)
+  assert got[0].isfinite().all() and torch.equal(got[0], got[1])

@@ -480,8 +480,13 @@ __global__ void qw_dequant_kernel(const uint32_t* codes, const uint16_t* scales,
 // bf16(bf16(level) * scale) of packed column 64 wave + 32 group + lane % 32 of the tile at
 // k = 128 kt + 16 slab + 8 (lane / 32) .. + 7: the A fragment of one 32x32x16 MFMA.  Columns past N
 // are zeros.  One thread per 16 bytes.
+// blockIdx.z: one of several weights behind each other (experts), at the strides given in elements.
 __global__ __launch_bounds__(256) void qw_expand_kernel(const uint32_t* codes, const uint16_t* scales, int64_t K,
-                                                         int64_t N, int group, int qtype, u32x4* out) {
+                                                         int64_t N, int group, int qtype, u32x4* out, int64_t codes_stride,
+                                                         int64_t scales_stride, int64_t out_stride) {
+  codes += blockIdx.z * codes_stride;
+  scales += blockIdx.z * scales_stride;
+  out += blockIdx.z * out_stride;
   const int ntile = blockIdx.x, kt = blockIdx.y, ktiles = (int)(K / KTILE);
   const int wn = threadIdx.x >> 6, lane = threadIdx.x & 63, l32 = lane & 31, lh = lane >> 5;
   const int spt = scales_per_tile(group);
@@ -812,12 +817,24 @@ int launch_qgemm_pre_grouped_rt(hipStream_t st, const QLArgs& a) {
   switch (a.epilogue) {
     case TNX_EPI_STORE: return launch_qgemm_pre_as<RT, true, kPreStore, 0>(st, a, kNoHead);
     case TNX_EPI_RELU2: return launch_qgemm_pre_as<RT, true, kPreRelu2, 0>(st, a, kNoHead);
+    case TNX_EPI_SILU_MUL: return launch_qgemm_pre_as<RT, true, kPreSilu, 0>(st, a, kNoHead);
     case kEpiSiluMulF32: return launch_qgemm_pre_as<RT, true, kPreSiluF32, 0>(st, a, kNoHead);
     case kEpiGeluMulF32: return launch_qgemm_pre_as<RT, true, kPreGeluF32, 0>(st, a, kNoHead);
     default: break;
   }
   TNX_REQUIRE(false, "experts over many rows: bad epilogue %d", a.epilogue);
 }
+
+int launch_qgemm_pre_grouped(hipStream_t st, const QLArgs& a) {
+  // as launch_qgemm_pre, with half a row block per expert left empty on average
+  const double avg = (double)a.M / (double)a.n_experts;
+  const bool tall = (avg + 128.0) * (double)(a.K + 150) < (avg + 64.0) * 1.09 * (double)a.K;
+  return tall ? launch_qgemm_pre_grouped_rt<16>(st, a) : launch_qgemm_pre_grouped_rt<8>(st, a);
+}
+// Rows per expert from which the experts' converted copies beat the codes (four times the bytes, no conversion in the loop):
+// Qwen3-30B-A3B shape, gate|up + down, us from codes | copies: 96 rows 125 + 97 | 152 + 100, 128: 193 + 120 | 191 + 121, 192: 254 +
+// 179 | 205 + 144, 447: 518 + 346 | 363 + 261, 1024: 1000 + 727 | 721 + 502.
+constexpr int64_t kMoeExpandedRows = 144;
 
 template <int SPT>
 int launch_qgemm_wide(hipStream_t st, const QLArgs& a, const WideHead& h = kNoHead) {
@@ -988,19 +1005,25 @@ extern "C" size_t tnx_qw_expanded_bytes(int64_t K, int64_t N) {
   return (size_t)(cdiv(N, kWideCols) * (K / KTILE)) * 65536u;
 }
 
-extern "C" int tnx_qw_expand(void* stream, const uint32_t* codes, const uint16_t* scales, int64_t K, int64_t N,
-                             int group, int qtype, uint16_t* w_expanded) {
-  int rc = tnx_qw_sizes(K, N, group, nullptr, nullptr);
+extern "C" int tnx_qw_expand_bank(void* stream, const uint32_t* codes, const uint16_t* scales, int64_t E, int64_t K, int64_t N,
+                                  int group, int qtype, uint16_t* w_expanded) {
+  size_t cb = 0, sb = 0;
+  int rc = tnx_qw_sizes(K, N, group, &cb, &sb);
   if (rc) return rc;
   TNX_REQUIRE(codes && scales && w_expanded, "qw_expand: null pointer");
   TNX_REQUIRE(qtype == TNX_Q_INT4 || qtype == TNX_Q_NF4, "qw_expand: bad qtype %d", qtype);
   TNX_REQUIRE(((uintptr_t)w_expanded & 15) == 0, "qw_expand: the output must be 16-byte aligned");
-  TNX_REQUIRE(K / KTILE <= 65535, "qw_expand: K=%lld too large", (long long)K);
-  dim3 grid((unsigned)cdiv(N, kWideCols), (unsigned)(K / KTILE));
+  TNX_REQUIRE(K / KTILE <= 65535 && E > 0 && E <= 65535, "qw_expand: K=%lld or %lld weights too many", (long long)K, (long long)E);
+  dim3 grid((unsigned)cdiv(N, kWideCols), (unsigned)(K / KTILE), (unsigned)E);
   hipLaunchKernelGGL(qw_expand_kernel, grid, dim3(256), 0, as_stream(stream), codes, scales, K, N, group, qtype,
-                     reinterpret_cast<u32x4*>(w_expanded));
+                     reinterpret_cast<u32x4*>(w_expanded), (int64_t)(cb / 4), (int64_t)(sb / 2), (int64_t)(tnx_qw_expanded_bytes(K, N) / 16));
   TNX_CHECK_LAUNCH("qw_expand");
   return TNX_OK;
+}
+
+extern "C" int tnx_qw_expand(void* stream, const uint32_t* codes, const uint16_t* scales, int64_t K, int64_t N,
+                             int group, int qtype, uint16_t* w_expanded) {
+  return tnx_qw_expand_bank(stream, codes, scales, 1, K, N, group, qtype, w_expanded);
 }
 
 extern "C" int tnx_dense_expand(void* stream, const uint16_t* w_bf16, int64_t K, int64_t N, uint16_t* w_expanded) {
@@ -1098,10 +1121,7 @@ int tnx_internal_wide_dense_grouped(hipStream_t st, int64_t n_routes, int64_t K,
   a.epilogue = once_rounded(epilogue);
   a.y = y; a.ldy = ldy; a.split_k = 1; a.ktiles_per_split = (int)(K / KTILE);
   a.n_experts = n_experts; a.offsets = offsets; a.sorted_route = sorted_route;
-  // as launch_qgemm_pre, with half a row block per expert left empty on average
-  const double avg = (double)n_routes / (double)n_experts;
-  const bool tall = (avg + 128.0) * (double)(K + 150) < (avg + 64.0) * 1.09 * (double)K;
-  return tall ? launch_qgemm_pre_grouped_rt<16>(st, a) : launch_qgemm_pre_grouped_rt<8>(st, a);
+  return launch_qgemm_pre_grouped(st, a);
 }
 
 extern "C" int tnx_splitk_finish(void* stream, const tnx_qlinear_desc* d) {
@@ -1220,7 +1240,7 @@ extern "C" int tnx_lora_down(void* stream, const uint16_t* x, int64_t M, int64_t
   return TNX_OK;
 }
 
-extern "C" int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* d) {
+static int moe_gmm(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_expanded) {
   TNX_REQUIRE(d, "moe_gmm: null descriptor");
   TNX_REQUIRE(d->n_routes > 0 && d->E > 0 && d->k > 0, "moe_gmm: bad shape");
   size_t cb = 0, sb = 0;
@@ -1257,7 +1277,14 @@ extern "C" int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* d) {
   const bool mul = d->epilogue == TNX_EPI_SILU_MUL;
   if (avg_rows > 24 && d->N % kWideCols == 0 && (mul ? d->N / 2 : d->N) % 8 == 0 && ((uintptr_t)d->y & 15) == 0 &&
       (uint64_t)(d->n_routes / d->x_div) * (uint64_t)d->K * 2 < 0xfffff000ull && d->n_routes % d->x_div == 0)
+  {
+    // from the experts' converted copies where those are worth four times the bytes
+    if (w_expanded && avg_rows >= kMoeExpandedRows && cdiv(d->N, kWideCols) * (d->K / KTILE) * 65536 < (int64_t)1 << 31) {
+      a.w_pre = w_expanded;
+      return launch_qgemm_pre_grouped(st, a);
+    }
     return scales_per_tile(d->group) == 2 ? launch_qgemm_wide_grouped<2>(st, a) : launch_qgemm_wide_grouped<4>(st, a);
+  }
   // Up to about 12 rows per expert the streaming kernel (16-row blocks, an expert with more
   // rows streams its weights once per block) beats the 32-row tiles: 87 + 48 against 96 + 56 us
   // at 10 rows per expert, 90 + 49 against 96 + 58 us at 12, 112 + 54 against 98 + 60 us at 16.
@@ -1268,6 +1295,13 @@ extern "C" int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* d) {
   if (max_rows <= 16 || avg_rows <= 8) return launch_moe<1, 2>(st, a, d->E, max_rows);
   if (max_rows <= 32 || avg_rows <= 24) return launch_moe<2, 2>(st, a, d->E, max_rows);
   return launch_moe<4, 2>(st, a, d->E, max_rows);
+}
+
+extern "C" int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* d) { return moe_gmm(stream, d, nullptr); }
+
+extern "C" int tnx_moe_gmm_expanded(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_expanded) {
+  TNX_REQUIRE(w_expanded && ((uintptr_t)w_expanded & 15) == 0, "moe_gmm_expanded: the copies must be there and 16-byte aligned");
+  return moe_gmm(stream, d, w_expanded);
 }
 
 #ifdef TNX_TIMING

@@ -170,6 +170,7 @@ class ExpertBank:
     self.dn_codes = torch.empty(E * cb2 // 4, dtype=torch.int32, device=device)
     self.dn_scales = torch.empty(E * sb2 // 2, dtype=torch.bfloat16, device=device)
     self.router_t = torch.empty(E, self.D, dtype=torch.bfloat16, device=device)
+    self.gu_expanded = self.dn_expanded = None   # optional second copy for calls with many rows (`expand`)
     self.load_base(weights)
 
   def check_base(self, weights: dict):
@@ -200,6 +201,23 @@ class ExpertBank:
       self.dn_codes[e * cb2 // 4:(e + 1) * cb2 // 4].copy_(c)
       self.dn_scales[e * sb2 // 2:(e + 1) * sb2 // 2].copy_(s)
     self.router_t.copy_(weights[prefix + "router"].to(device, torch.bfloat16).t())
+    if self.gu_expanded is not None:
+      self._fill_expanded()
+
+  def expanded_bytes(self) -> int:
+    size = L.lib().tnx_qw_expanded_bytes
+    return self.E * (int(size(self.D, 2 * self.F)) + int(size(self.F, self.D)))
+
+  def expand(self):
+    """The same second copy as `FusedLinear.expand`, of every expert: calls with some hundred rows per expert are bound
+    by the conversion of codes in their loop."""
+    if self.gu_expanded is None:
+      self._fill_expanded()
+
+  def _fill_expanded(self):
+    cfg = self.cfg
+    self.gu_expanded = ops.qw_expand_bank(self.gu_codes, self.gu_scales, self.E, self.D, 2 * self.F, cfg.group, cfg.qtype, self.gu_expanded)
+    self.dn_expanded = ops.qw_expand_bank(self.dn_codes, self.dn_scales, self.E, self.F, self.D, cfg.group, cfg.qtype, self.dn_expanded)
 
 
 class QLoRAModel:
@@ -207,8 +225,8 @@ class QLoRAModel:
 
   def __init__(self, cfg: ModelConfig, weights: dict, device="cuda", expand_many_rows: bool | None = None):
     """expand_many_rows: keep the converted second copy of every dense quantised linear
-    (`FusedLinear.expand`) for the calls with many rows.  None (default): when the copies take
-    less than a quarter of the device memory that is free once the model is built."""
+    (`FusedLinear.expand`) and of the experts for the calls with many rows.  None (default): when the copies take
+    less than a quarter of the device memory that is free once the model is built (experts: together with the others)."""
     L.lib()  # fail loudly when the HIP library is missing
     self.cfg = cfg
     self.device = torch.device(device)
@@ -252,9 +270,16 @@ class QLoRAModel:
       head_need = int(L.lib().tnx_qw_expanded_bytes(cfg.embed_dim, cfg.vocab_size))
       if head_need >= (1 << 31):
         head_need = 0
+    banks = [ly["experts"] for ly in self.layers if "experts" in ly]
+    expand_experts = expand_many_rows
     if expand_many_rows is None:
       need = head_need + sum(f.expanded_bytes() for f in self._linears() if f.wants_expansion())
-      expand_many_rows = need <= torch.cuda.mem_get_info(dev)[0] // 4
+      room = torch.cuda.mem_get_info(dev)[0] // 4
+      expand_many_rows = need <= room
+      expand_experts = need + sum(bank.expanded_bytes() for bank in banks) <= room
+    if expand_experts:
+      for bank in banks:
+        bank.expand()
     if expand_many_rows:
       for f in self._linears():
         f.expand()
@@ -726,7 +751,7 @@ class Runner(HeadRunner):
     d.codes, d.scales = ex.gu_codes.data_ptr(), ex.gu_scales.data_ptr()
     d.offsets, d.sorted_route = self.offsets.data_ptr(), self.sorted_route.data_ptr()
     d.epilogue, d.y = L.TNX_EPI_SILU_MUL, self.act.data_ptr()
-    ops.moe_gmm(d)
+    ops.moe_gmm(d, ex.gu_expanded)
     d2 = L.MoeGmmDesc()
     d2.n_routes, d2.E, d2.k, d2.K, d2.N = M * k, E, k, ex.F, ex.D
     d2.group, d2.qtype = cfg.group, cfg.qtype
@@ -734,7 +759,7 @@ class Runner(HeadRunner):
     d2.codes, d2.scales = ex.dn_codes.data_ptr(), ex.dn_scales.data_ptr()
     d2.offsets, d2.sorted_route = self.offsets.data_ptr(), self.sorted_route.data_ptr()
     d2.epilogue, d2.y = L.TNX_EPI_STORE, self.y_route.data_ptr()
-    ops.moe_gmm(d2)
+    ops.moe_gmm(d2, ex.dn_expanded)
     if cfg.embed_dim % 8 == 0:   # the next norm adds the weighted combine to the residual stream
       return _MOE_PENDING
     ops.moe_combine(self.y_route, self.topk_w, M, k, cfg.embed_dim, self.h, self.h)

@@ -91,6 +91,17 @@ def qw_expand(codes, scales, K, N, group, qtype):
   return out
 
 
+def qw_expand_bank(codes, scales, E, K, N, group, qtype, out=None):
+  """The copies of E weights of one shape, [E, ...]; out: where they go."""
+  n = int(L.lib().tnx_qw_expanded_bytes(K, N)) // 2
+  if out is None:
+    out = torch.empty(E, n, dtype=torch.bfloat16, device=codes.device)
+  elif tuple(out.shape) != (E, n) or out.dtype != torch.bfloat16:
+    raise ValueError(f"qw_expand_bank: the copies are bfloat16 {(E, n)}")
+  L.check(L.lib().tnx_qw_expand_bank(_stream(), _ptr(codes), _ptr(scales), E, K, N, group, qtype, _ptr(out)), "tnx_qw_expand_bank")
+  return out
+
+
 def dense_expand(w):
   """The same copy for a dense bf16 matrix w [N, K] (an unquantised or tied lm_head [V, D])."""
   import torch
@@ -242,8 +253,12 @@ def moe_sort_routes(topk_id, E, counts, offsets, sorted_route):
                                       _ptr(offsets), _ptr(sorted_route)), "tnx_moe_sort_routes")
 
 
-def moe_gmm(desc: L.MoeGmmDesc):
-  L.check(L.lib().tnx_moe_int4_gmm(_stream(), C.byref(desc)), "tnx_moe_int4_gmm")
+def moe_gmm(desc: L.MoeGmmDesc, w_expanded=None):
+  """w_expanded: the experts' converted copies (`qw_expand`), [E, ...] behind each other."""
+  if w_expanded is None:
+    L.check(L.lib().tnx_moe_int4_gmm(_stream(), C.byref(desc)), "tnx_moe_int4_gmm")
+  else:
+    L.check(L.lib().tnx_moe_gmm_expanded(_stream(), C.byref(desc), _ptr(w_expanded)), "tnx_moe_gmm_expanded")
 
 
 def moe_combine(y, topk_w, M, k, D, residual, out):
