@@ -36,8 +36,13 @@ constexpr size_t pre_smem_bytes() {
   return std::max<size_t>(4 * pre_step_bytes<RT>(), 16 * RT * (kWideCols + 8) * 2);
 }
 
+// (operands that loads have written: the wait for those is all it needs)
 __device__ __forceinline__ void mfma16_acc(u32x4 a, u32x4 b, f32x4& c) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+// the same for operands that vector instructions may just have written: the wait states in front of it
+__device__ __forceinline__ void mfma16_acc_wait(u32x4 a, u32x4 b, f32x4& c) {
+  asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 // keeps a value that was changed outside the loop in accumulator registers: the whole tile does not fit the others
 __device__ __forceinline__ void pin_acc(f32x4& c) { asm volatile("" : "+a"(c)); }
@@ -347,16 +352,13 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
         for (int j = 0; j < 2; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) lbv[ct][j][q] = pack2bf(bflo(lbv[ct][j][q]) * a.lora_scale, bfhi(lbv[ct][j][q]) * a.lora_scale);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_nop 3");   // (vector writes in front of an MFMA in assembly)
-      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         if (rt + 1 < RT) load_t(rt + 1);
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) mfma16_acc(lbv[ct][0], tf[rt & 1][ct][0], acc[rt][ct]);
+        for (int ct = 0; ct < CT; ++ct) mfma16_acc_wait(lbv[ct][0], tf[rt & 1][ct][0], acc[rt][ct]);
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) mfma16_acc(lbv[ct][1], tf[rt & 1][ct][1], acc[rt][ct]);
+        for (int ct = 0; ct < CT; ++ct) mfma16_acc_wait(lbv[ct][1], tf[rt & 1][ct][1], acc[rt][ct]);
         __builtin_amdgcn_sched_barrier(0);   // (all tiles' fragments at once do not fit the registers)
       }
       settle();
