@@ -629,6 +629,56 @@ def test_gqa_attention_through_lds_equals_the_per_wave_form(gpu, B, T, S, Hq, Hk
     assert diff.max().item() <= 2.0 ** -6 * max(1.0, ref.abs().max().item()), diff.max().item()
 
 
+@pytest.mark.parametrize("B,T,S,Hq,Hkv,col,window,seg,scale", [
+    (2, 61, 61, 8, 2, 0, 0, False, None),        # fewest tiles of the work-group form, odd rows of ids and slots
+    (3, 131, 333, 6, 2, 77, 0, False, 1.0),      # three query heads in lanes of four, queries from column 77, no scaling
+    (1, 1023, 1023, 4, 4, 0, 0, True, None),     # a packed batch of several segments, one head per kv head
+    (2, 259, 263, 8, 1, 3, 40, False, None),     # a window inside two key blocks
+    (1, 65, 70, 32, 2, 5, 0, True, 0.125),       # sixteen heads per kv head: one position per tile
+])
+def test_gqa_attention_many_positions_equals_few(gpu, B, T, S, Hq, Hkv, col, window, seg, scale):
+  """head_dim 128: all positions in one call (keys and values through LDS) against calls of a few
+  positions each (every wave loads its own), bit for bit: the same blocks in the same order with the
+  same arithmetic."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  dh, pad = 128, 0
+  g = torch.Generator().manual_seed(90 + T)
+  if seg:
+    ids = torch.sort(torch.randint(1, 5, (B, S), generator=g, dtype=torch.int32), dim=1).values
+  else:
+    ids = torch.randint(1, 100, (B, S), generator=g, dtype=torch.int32)
+    ids[0, :5] = pad
+    ids[B - 1, 9] = pad
+  q = bf(rnd((B, T, Hq * dh), 91)).to(gpu)
+  kc, vc = bf(rnd((B, Hkv, S, dh), 92)).to(gpu), bf(rnd((B, Hkv, S, dh), 93)).to(gpu)
+  ids = ids.to(gpu).contiguous()
+
+  def attn(t0, n):
+    qs = q[:, t0:t0 + n].contiguous()
+    out = torch.full((B, n, Hq * dh), 7.0, dtype=torch.bfloat16, device=gpu)
+    colp = torch.tensor([col + t0], dtype=torch.int32, device=gpu)
+    d = L.AttnDesc()
+    d.B, d.T, d.S, d.Hq, d.Hkv, d.dh = B, n, S, Hq, Hkv, dh
+    d.scale, d.window, d.pad_id = dh ** -0.5 if scale is None else scale, window, pad
+    d.q, d.kcache, d.vcache, d.out = qs.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr()
+    if seg:
+      d.segment_ids = ids.data_ptr()
+    else:
+      d.tokens = ids.data_ptr()
+    d.tok_ld, d.col_ptr, d.kv_chunk = S, colp.data_ptr(), 0
+    ops.gqa_attn(d)
+    torch.cuda.synchronize()
+    return out
+
+  whole = attn(0, T)
+  G = Hq // Hkv
+  few = 3 * max(1, 16 // (1 << (G - 1).bit_length()))       # three tiles of queries
+  parts = torch.cat([attn(t0, min(few, T - t0)) for t0 in range(0, T, few)], dim=1)
+  assert torch.isfinite(whole.float()).all()
+  assert torch.equal(whole.view(torch.int16), parts.view(torch.int16))
+
+
 @pytest.mark.parametrize("M,D,V,dense", [(8, 512, 32000, True), (128, 512, 4096, True),
                                          (130, 256, 1040, True),   # two row blocks, partial last column block
                                          (50, 256, 1040, False), (130, 256, 4096, False)])

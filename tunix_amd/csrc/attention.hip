@@ -764,23 +764,44 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 // takes 4 x QW consecutive query tiles of one (row, kv head), and every 32-key block is requested
 // once per work-group straight into LDS (16 bytes per lane, key rows with their 16-byte chunks
 // XOR-swizzled by row so that the fragment reads of 16 rows hit 16 bank groups; value rows as they
-// are; the block's 32 token / segment ids next to them), two blocks in flight.  A wave reads its
-// fragments from there instead of drawing them through its own loads in the MFMA operand layout,
-// which the memory path serves a few lanes at a time, and two such work-groups per compute unit
-// (227 registers per lane, 68 KB of LDS) put the softmax arithmetic of one wave under the MFMAs of
-// another.  Two query tiles per wave: with three the kernel spills.  Every wave computes exactly
-// the blocks attn_tiles_kernel would give it, in the same order with the same arithmetic: outputs
-// are bit-identical.
+// are; the block's 32 token / segment ids next to them, by the dword: rows of ids need no alignment),
+// three blocks in flight.  Every wave computes exactly the blocks attn_tiles_kernel would give it, in the same order
+// with the same arithmetic: outputs are bit-identical.
+//
+// What bounds it is vector work: per score 11 lane-instructions (two roundings to bf16 with a scale between them, maximum, exponential,
+// sum, rounding of P) against half a clock of matrix pipe.  So the tiles of a wave run through one straight line of code, whose
+// chains hide each other's latency, with two such work-groups per compute unit; values are rounded in pairs; maxima cross the
+// lanes in registers (permlane swaps) instead of through LDS; and O is kept transposed (P.V formed as V^T . P^T: the same operand
+// registers with the operands exchanged), so that a query's rescaling factor is already in the lanes that need it.
+// 32 heads of 128 over 8 kv heads, us: 2 x 6144 positions 1369 -> 1110 (451 -> 557 TFLOP/s), 13 x 1024 packed 395 -> 306; rows of ids
+// off 16-byte alignment, which took attn_tiles_kernel, 7 x 1023 over 4 kv heads: 363 -> 167.
 typedef uint32_t __attribute__((address_space(3))) lds_word_t;
 typedef u32x4 __attribute__((address_space(3))) lds_vec_t;
 __device__ __forceinline__ u32x4 attn_lds128(uint32_t addr) {
   return *reinterpret_cast<const lds_vec_t*>(static_cast<uintptr_t>(addr));
 }
-constexpr uint32_t kWgStageBytes = 8192 + 8192 + 1024;   // 32 keys x 256 B, 32 values x 256 B, ids
-// blocks in LDS: one computed, three in flight (three / six measured 3 % / 50 % slower: with six a
-// compute unit holds one work-group instead of two)
+// four bytes per lane straight into LDS, at `lds` + 4 * lane (as dma16 of gemm_tile.h)
+__device__ __forceinline__ void dma4(uint32_t lds, const u32x4& r, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(r) : "memory", "m0");
+}
+// f over the four lanes lm + 16 {0, 1, 2, 3} that share a query, in all of them
+template <class F>
+__device__ __forceinline__ float across_quarters(float x, F f) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+// c += a . b with the accumulator in place (the compiler's form copies O at every branch of the loop).  The wait states between a
+// vector write of an operand and the MFMA that reads it stand inside, under the MFMA before; what reads c next has to lie 18
+// instructions behind.
+__device__ __forceinline__ void mfma16_tied(u32x4 a, u32x4 b, f32x4& c) {
+  asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+constexpr uint32_t kWgStageBytes = 8192 + 8192 + 256;   // 32 keys x 256 B, 32 values x 256 B, ids
+// blocks in LDS: one computed, three in flight
 constexpr int kWgStages = 4;
-template <int QW>
+template <int QW, bool SCALED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_wg_kernel(const AttnArgs a) {
   constexpr int DH = 128, KS = 4;
   extern __shared__ __align__(16) unsigned char smem_a[];
@@ -824,6 +845,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int kb0 = k_lo & ~31, kb_last = k_hi & ~31;
   const bool any = wave_live && kb0 <= k_hi;
 
+  // O^T: lane (query lm, quarter lq) holds dimensions 32 lq + 8 i + jj in O[w][jj][i]
   f32x4 O[QW][8];
   float m_run[QW], l_run[QW];
 #pragma unroll
@@ -844,22 +866,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int32_t id_q = tok[min((int64_t)c_n[w], a.tok_ld - 1)];
     id_ref[w] = a.seg_mode ? id_q : a.pad_id;
   }
-  // A block that lies wholly inside every query's range of a tile, with no id to mask, takes the
-  // same arithmetic without the per-key tests: the bounds of that, uniform over the wave.
-  // (Packed batches compare ids per query and always take the general form.)
-  int lo_max[QW], hi_min[QW];
+  // A block that lies wholly inside every query's range of all tiles, with no id to mask, takes the
+  // same arithmetic without the per-key tests: the bounds of that, uniform over the wave.  In a packed batch the
+  // ids that allow it are those of one segment that all queries of the wave belong to.
+  int lo_max = -0x7fffffff, hi_min = 0x7fffffff;
+  bool full = true;
+  const int32_t one_id = __builtin_amdgcn_readfirstlane(id_ref[0]);
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
-    int lo = max(k_lo, lo_n[w]), hi = min(k_hi, c_n[w]);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      lo = max(lo, __shfl_xor(lo, o, 64));
-      hi = min(hi, __shfl_xor(hi, o, 64));
-    }
-    const bool full = __builtin_amdgcn_ballot_w64(qvalid[w]) == ~0ull && !id_equal;
-    lo_max[w] = __builtin_amdgcn_readfirstlane(full ? lo : 0x7fffffff);
-    hi_min[w] = __builtin_amdgcn_readfirstlane(hi);
+    lo_max = max(lo_max, max(k_lo, lo_n[w]));
+    hi_min = min(hi_min, min(k_hi, c_n[w]));
+    full = full && __builtin_amdgcn_ballot_w64(qvalid[w] && id_ref[w] == one_id) == ~0ull;
   }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo_max = max(lo_max, __shfl_xor(lo_max, o, 64));
+    hi_min = min(hi_min, __shfl_xor(hi_min, o, 64));
+  }
+  lo_max = __builtin_amdgcn_readfirstlane(full ? lo_max : 0x7fffffff);
+  hi_min = __builtin_amdgcn_readfirstlane(hi_min);
   const uint32_t slab_bytes = (uint32_t)a.S * DH * 2u;
   const u32x4 rk = raw_rsrc(kbase, slab_bytes), rv = raw_rsrc(vbase, slab_bytes);
   const u32x4 rtok = raw_rsrc(tok, (uint64_t)min(a.S, a.tok_ld) * 4);
@@ -876,98 +901,102 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       dma16(base + (uint32_t)c * 4096u, rk, kb_bytes + (uint32_t)c * 4096u + kreq, 0);
       dma16(base + 8192u + (uint32_t)c * 4096u, rv, kb_bytes + (uint32_t)c * 4096u + vreq, 0);
     }
-    // ids kb .. kb + 255 (the block's 32 and whatever follows them; past the row: zeros)
-    dma16(lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes + 16384u, rtok, (uint32_t)(kb0_wg + 32 * i + 4 * lane) * 4u, 0);
+    // ids kb .. kb + 63 (the block's 32 and whatever follows them; past the row: zeros)
+    dma4(lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes + 16384u, rtok, (uint32_t)(kb0_wg + 32 * i + lane) * 4u);
   };
+  // this lane's places in a stage: key row lm (+ 16 tt), chunk 4 j + lq; value rows 4 lq + s (+ 16), chunk lm; ids 4 lq
+  uint32_t kat[KS];
+#pragma unroll
+  for (int j = 0; j < KS; ++j) kat[j] = (uint32_t)(lm * 256) + (((uint32_t)(j * 4 + lq) ^ (uint32_t)lm) * 16u);
+  const uint32_t vat = 8192u + (uint32_t)(lq * 1024 + lm * 16), iat = 16384u + (uint32_t)(lq * 16);
   auto compute_block = [&](int kb, uint32_t base) {
     u32x4 kf[2][KS], vf[8];
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
+    for (int j = 0; j < KS; ++j) {
+      const uint32_t at = base + kat[j];
 #pragma unroll
-      for (int j = 0; j < KS; ++j)
-        kf[tt][j] = attn_lds128(base + (uint32_t)((tt * 16 + lm) * 256) + (((uint32_t)(j * 4 + lq) ^ (uint32_t)lm) * 16u));
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-      vf[s] = attn_lds128(base + 8192u + (uint32_t)((s < 4 ? 4 * lq + s : 12 + 4 * lq + s) * 256) + (uint32_t)lm * 16u);
-    const u32x4 t0 = attn_lds128(base + 16384u + (uint32_t)(4 * lq) * 4u);
-    const u32x4 t1 = attn_lds128(base + 16384u + (uint32_t)(16 + 4 * lq) * 4u);
-    int tk[8];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      tk[s] = (int)t0[s];
-      tk[4 + s] = (int)t1[s];
+      for (int tt = 0; tt < 2; ++tt) kf[tt][j] = attn_lds128(at + (uint32_t)(tt * 4096));
     }
-    // (pad mode: a key counts when its id differs from pad_id, the same test for every tile)
-    bool idok[8];
+    const uint32_t va = base + vat, ia = base + iat;
+    const u32x4 t0 = attn_lds128(ia), t1 = attn_lds128(ia + 64u);
 #pragma unroll
-    for (int s = 0; s < 8; ++s) idok[s] = (tk[s] == a.pad_id) == id_equal;
-    const bool ids_all = !id_equal && __builtin_amdgcn_ballot_w64(idok[0] && idok[1] && idok[2] && idok[3] && idok[4] &&
-                                                                  idok[5] && idok[6] && idok[7]) == ~0ull;
+    for (int s = 0; s < 8; ++s) vf[s] = attn_lds128(va + (uint32_t)((s < 4 ? s : 12 + s) * 256));
+    // (pad mode: a key counts when its id differs from pad_id; packed: when it is the query's)
+    bool ids = true;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) ids = ids & (((int)t0[s] == one_id) == id_equal) & (((int)t1[s] == one_id) == id_equal);
+    const bool inside = kb >= lo_max && kb + 31 <= hi_min && __builtin_amdgcn_ballot_w64(ids) == ~0ull;
+    f32x4 st[QW][2];
+#pragma unroll
+    for (int w = 0; w < QW; ++w)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) st[w][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < KS; ++j)
+#pragma unroll
+      for (int w = 0; w < QW; ++w)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) st[w][tt] = mfma16(kf[tt][j], qf[w][j], st[w][tt]);
+    float sv[QW][8], alpha[QW];
+#pragma unroll
+    for (int w = 0; w < QW; ++w)
+#pragma unroll
+      for (int s = 0; s < 8; s += 2) {
+        uint32_t u = cvt_pk_bf16(st[w][s >> 2][s & 3], st[w][s >> 2][(s & 3) + 1]);
+        if constexpr (SCALED) u = cvt_pk_bf16(bflo(u) * a.scale_bf, bfhi(u) * a.scale_bf);
+        sv[w][s] = bflo(u);
+        sv[w][s + 1] = bfhi(u);
+      }
+    if (!inside) {
+      asm volatile("");   // (a branch, not selects in every block)
+#pragma unroll
+      for (int w = 0; w < QW; ++w)
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          const int key = kb + (s < 4 ? 4 * lq + s : 16 + 4 * lq + (s - 4));
+          const int id = s < 4 ? (int)t0[s & 3] : (int)t1[s & 3];
+          const bool ok = qvalid[w] & (key >= max(k_lo, lo_n[w])) & (key <= min(k_hi, c_n[w])) & ((id == id_ref[w]) == id_equal);
+          sv[w][s] = ok ? sv[w][s] : -__builtin_inff();
+        }
+    }
+    bool moved = false;
     u32x4 pa[QW];
-    auto tile_step = [&](int w, auto inside_c) {
-      constexpr bool INSIDE = decltype(inside_c)::value;
-      bool kvalid[8];
 #pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const int key = kb + (s < 4 ? 4 * lq + s : 16 + 4 * lq + (s - 4));
-        kvalid[s] = INSIDE || (qvalid[w] && key >= max(k_lo, lo_n[w]) && key <= min(k_hi, c_n[w]) &&
-                               ((tk[s] == id_ref[w]) == id_equal));
-      }
-      f32x4 st[2];
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        st[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < KS; ++j) st[tt] = mfma16(kf[tt][j], qf[w][j], st[tt]);
-      }
-      float sv[8];
-      float bmax = kNegBig;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        float x = rbf(st[s >> 2][s & 3]);
-        if (a.scale_bf != 0.f) x = rbf(x * a.scale_bf);
-        sv[s] = x;
-        if (kvalid[s]) bmax = fmaxf(bmax, x);
-      }
-      bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
-      bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
-      const float m_new = fmaxf(m_run[w], bmax);
-      const float alpha = __expf(m_run[w] - m_new);
+    for (int w = 0; w < QW; ++w) {
+      const float lo = fmaxf(fmaxf(fmaxf(sv[w][0], sv[w][1]), sv[w][2]), sv[w][3]);
+      const float hi = fmaxf(fmaxf(fmaxf(sv[w][4], sv[w][5]), sv[w][6]), sv[w][7]);
+      const float m_new = fmaxf(m_run[w], across_quarters(fmaxf(lo, hi), [](float x, float y) { return fmaxf(x, y); }));
+      alpha[w] = __expf(m_run[w] - m_new);
+      moved = moved || alpha[w] != 1.0f;
       m_run[w] = m_new;
       float p[8], psum = 0.f;
 #pragma unroll
       for (int s = 0; s < 8; ++s) {
-        p[s] = kvalid[s] ? __expf(sv[s] - m_new) : 0.f;
+        p[s] = __expf(sv[w][s] - m_new);   // (a masked key: exp(-inf) = 0)
         psum += p[s];
       }
-      l_run[w] = l_run[w] * alpha + psum;
-      pa[w][0] = pack2bf(p[0], p[1]);
-      pa[w][1] = pack2bf(p[2], p[3]);
-      pa[w][2] = pack2bf(p[4], p[5]);
-      pa[w][3] = pack2bf(p[6], p[7]);
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-        float ar[4];
+      l_run[w] = l_run[w] * alpha[w] + psum;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ar[i] = __shfl(alpha, 4 * lq + i, 64);
+      for (int e = 0; e < 4; ++e) pa[w][e] = cvt_pk_bf16(p[2 * e], p[2 * e + 1]);
+    }
+    // the running maximum settles after a few blocks: rescale O only when some column moved
+    if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+#pragma unroll
+      for (int w = 0; w < QW; ++w)
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) O[w][jj][i] *= ar[i];
-      }
-    };
-#pragma unroll
-    for (int w = 0; w < QW; ++w) {
-      if (ids_all && kb >= lo_max[w] && kb + 31 <= hi_min[w]) tile_step(w, std::true_type{});
-      else tile_step(w, std::false_type{});
+          for (int i = 0; i < 4; ++i) O[w][jj][i] *= alpha[w];
     }
+    // a value fragment is transposed once for all tiles
 #pragma unroll
     for (int jj = 0; jj < 8; ++jj) {
       const uint32_t sel = (jj & 1) ? 0x07060302u : 0x05040100u;
-      u32x4 bfrag;
+      u32x4 vt;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bfrag[r] = __builtin_amdgcn_perm(vf[2 * r + 1][jj >> 1], vf[2 * r][jj >> 1], sel);
+      for (int r = 0; r < 4; ++r) vt[r] = __builtin_amdgcn_perm(vf[2 * r + 1][jj >> 1], vf[2 * r][jj >> 1], sel);
 #pragma unroll
-      for (int w = 0; w < QW; ++w) O[w][jj] = mfma16(pa[w], bfrag, O[w][jj]);
+      for (int w = 0; w < QW; ++w) mfma16_tied(vt, pa[w], O[w][jj]);
     }
   };
 #pragma unroll
@@ -983,23 +1012,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int kb = kb0_wg + 32 * i;
     if (any && kb >= kb0 && kb <= kb_last) compute_block(kb, lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes);
   }
+  asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+  for (int w = 0; w < QW; ++w)
+#pragma unroll
+    for (int jj = 0; jj < 8; ++jj) asm volatile("" : "+v"(O[w][jj]));
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
-    float lr = l_run[w];
-    lr += __shfl_xor(lr, 16, 64);
-    lr += __shfl_xor(lr, 32, 64);
+    const float l = across_quarters(l_run[w], [](float x, float y) { return x + y; });
+    const int ti = (qt0 + w) * PT + (lm >> a.gp_shift);
+    if (!qvalid[w]) continue;
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    uint16_t* o = a.out + ((b * a.T + ti) * a.Hq + hkv * a.G + g) * DH + 32 * lq;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int n = 4 * lq + i;
-      const float l = __shfl(lr, n, 64);
-      const int gi = n & (a.Gp - 1), ti = (qt0 + w) * PT + (n >> a.gp_shift);
-      if (!(gi < a.G && ti < a.T)) continue;
-      const float inv = l > 0.f ? 1.0f / l : 0.f;
-      uint16_t* o = a.out + ((b * a.T + ti) * a.Hq + hkv * a.G + gi) * DH;
       u32x4 wv;
 #pragma unroll
       for (int r = 0; r < 4; ++r) wv[r] = pack2bf(O[w][2 * r][i] * inv, O[w][2 * r + 1][i] * inv);
-      *reinterpret_cast<u32x4*>(o + 8 * lm) = wv;
+      *reinterpret_cast<u32x4*>(o + 8 * i) = wv;
     }
   }
 }
@@ -1115,20 +1145,24 @@ extern "C" int tnx_gqa_attn(void* stream, const tnx_attn_desc* d) {
   // many query positions at head_dim 128, no key split, no fused rotation: keys and values through
   // LDS, eight query tiles per work-group
   constexpr int kWgTilesPerWave = 2;
-  if (!a.rope_sin && a.n_chunks == 1 && d->dh == 128 && tv && QT >= 2 * 4 * kWgTilesPerWave &&
+  if (!a.rope_sin && a.n_chunks == 1 && d->dh == 128 && QT >= 2 * 4 * kWgTilesPerWave &&
       (uint64_t)d->S * 256u < (1ull << 32) && d->B * cdiv(QT, 4 * kWgTilesPerWave) <= 65535) {
     a.QTG = (unsigned)cdiv(QT, 4 * kWgTilesPerWave);
-    dim3 wgrid(1u, (unsigned)d->Hkv, (unsigned)(d->B * a.QTG));
-    static std::once_flag wg_once;
-    static hipError_t wg_rc = hipSuccess;
-    std::call_once(wg_once, [] {
-      wg_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_wg_kernel<kWgTilesPerWave>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kWgStages * kWgStageBytes));
-    });
-    TNX_REQUIRE(wg_rc == hipSuccess, "attn: cannot raise the dynamic LDS limit");
-    hipLaunchKernelGGL((attn_wg_kernel<kWgTilesPerWave>), wgrid, dim3(256), kWgStages * kWgStageBytes, st, a);
-    TNX_CHECK_LAUNCH("gqa_attn (work-group tiles)");
-    return TNX_OK;
+    auto launch = [&](auto scaled_c) -> int {
+      constexpr bool SCALED = decltype(scaled_c)::value;
+      static std::once_flag wg_once;
+      static hipError_t wg_rc = hipSuccess;
+      std::call_once(wg_once, [] {
+        wg_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_wg_kernel<kWgTilesPerWave, SCALED>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kWgStages * kWgStageBytes));
+      });
+      TNX_REQUIRE(wg_rc == hipSuccess, "attn: cannot raise the dynamic LDS limit");
+      hipLaunchKernelGGL((attn_wg_kernel<kWgTilesPerWave, SCALED>), dim3(1u, (unsigned)d->Hkv, (unsigned)(d->B * a.QTG)), dim3(256),
+                         kWgStages * kWgStageBytes, st, a);
+      TNX_CHECK_LAUNCH("gqa_attn (work-group tiles)");
+      return TNX_OK;
+    };
+    return a.scale_bf != 0.f ? launch(std::true_type{}) : launch(std::false_type{});
   }
   // many query positions, no key split, no fused rotation: two query tiles per wave
   constexpr int kTilesPerWave = 2;
