@@ -195,6 +195,32 @@ def test_qlinear_lora_matches_oracle(gpu, M, K, N, group, qtype, r, split):
   assert_bf16_close(y, ref, what="qlinear")
 
 
+@pytest.mark.parametrize("M,K,N,split", [
+    (128, 4096, 1024, 1),       # 32 k-tiles: two behind the whole turns of the weight ring
+    (128, 4096, 1024, 4),       # eight of each split: two
+    (100, 1280, 512, 1),        # ten: one
+    (600, 640, 24576, 1),       # many rows, from the codes: five, two behind the turn
+])
+def test_qlinear_lora_repeats_bit_for_bit(gpu, M, K, N, split):
+  """The k-tiles behind the last whole turn of the weight ring request no weights, so nothing younger than
+  the activations is in flight there: their wait covers all of it.  (One that left as many loads out as in
+  the turns multiplied rows of the adapter's block that had not landed, now and then.)"""
+  from tunix_amd import ops
+  x, t = bf(rnd((M, K), 61)).to(gpu), bf(rnd((M, 64), 62)).to(gpu)
+  c, s = ops.quantize_pack(bf(rnd((K, N), 63, 0.02)).to(gpu), 64, Q.NF4)
+  lb = bf(rnd((N, 64), 64, 0.1)).to(gpu)
+  outs = []
+  for _ in range(40):
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+    ws = torch.empty(split * M * N, dtype=torch.float32, device=gpu) if split > 1 else None
+    ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=Q.NF4, x=x, codes=c, scales=s, y=y, split_k=split,
+                                      ws=ws, lora_rank=64, lora_nseg=1, lora_seg_end=[N], lora_seg_toff=[0], t=t, t_ld=64,
+                                      lora_b=lb, lora_scale=2.0))
+    outs.append(y)
+    torch.cuda.synchronize()
+  assert all(torch.equal(outs[0], o) for o in outs[1:])
+
+
 @pytest.mark.parametrize("M,K,N,group,qtype,r,seg_widths,epi", [
     (1100, 256, 7424, 64, Q.NF4, 64, None, "store"),             # ragged rows, one adapter
     (640, 384, 13312, 128, Q.INT4, 16, [8192, 2560, 2560], "store"),  # three adapter segments, 3 k-tiles

@@ -406,12 +406,14 @@ void qgemm128_kernel(const QLArgs a) {
   // The one barrier of the k-tile sits between the steps: every wave has finished reading this
   // tile, and the next tile, requested by the second step of the tile before, has landed in LDS
   // (the only younger loads are the 2 NT weight / scale loads the first step has just issued).
-  auto tile = [&](auto Dc, int kt) {
+  // REST (the tiles behind the loop): nobody reads the weights requested there, so the compiler drops the requests, and the
+  // activations are the youngest loads: everything is waited for.
+  auto tile = [&](auto Dc, int kt, auto RESTc) {
     constexpr int d = decltype(Dc)::value, dn = (d + 1) % PF;
     const bool next_active = kt + 1 < kt_end;
     __builtin_amdgcn_sched_barrier(0);
     kstep(ic<0>{}, Dc, ic<1>{}, ic<dn>{}, ic<0>{}, a_cur1, ic<1>{}, ic<1>{}, ic<0>{}, ic<dn>{}, kt + 2, next_active);
-    tnx_wait_vm(2 * NT);
+    tnx_wait_vm(decltype(RESTc)::value ? 0 : 2 * NT);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
     kstep(ic<1>{}, ic<dn>{}, ic<0>{}, ic<dn>{}, ic<1>{}, a_nxt0, ic<0>{}, ic<0>{}, ic<1>{}, ic<-1>{}, kt + 2, false);
@@ -468,13 +470,13 @@ void qgemm128_kernel(const QLArgs a) {
     // the one or two tiles left
     int kt = kt_begin;
     for (; kt + PF <= kt_end; kt += PF) {
-      tile(ic<0>{}, kt);
-      tile(ic<1>{}, kt + 1);
-      tile(ic<2>{}, kt + 2);
+      tile(ic<0>{}, kt, ic<0>{});
+      tile(ic<1>{}, kt + 1, ic<0>{});
+      tile(ic<2>{}, kt + 2, ic<0>{});
     }
     if (kt < kt_end) {
-      tile(ic<0>{}, kt);
-      if (kt + 1 < kt_end) tile(ic<1>{}, kt + 1);
+      tile(ic<0>{}, kt, ic<1>{});
+      if (kt + 1 < kt_end) tile(ic<1>{}, kt + 1, ic<1>{});
     }
   }
   TNX_STAMP(3);

@@ -361,7 +361,9 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto tile = [&](auto Dc, int kt) {
+  // REST (the tiles behind the loop): nobody reads the weights requested there, so the compiler drops the requests, and the
+  // activations are the youngest loads: everything is waited for.
+  auto tile = [&](auto Dc, int kt, auto RESTc) {
     const bool next_active = kt + 1 < ktiles;
     __builtin_amdgcn_sched_barrier(0);
     slab(ic<0>{}, Dc, kt, next_active);
@@ -373,7 +375,7 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
     slab(ic<6>{}, Dc, kt, next_active);
     // the next tile's activations, requested by slab 7 of the tile before, have landed in LDS:
     // the only younger loads are the six weight / scale loads slab 6 has just issued
-    tnx_wait_vm(6);
+    tnx_wait_vm(decltype(RESTc)::value ? 0 : 6);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
     slab(ic<7>{}, Dc, kt, next_active);
@@ -434,13 +436,13 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
   // of the tile after it assume that its loads never happened), then the one or two tiles left
   int kt = 0;
   for (; kt + PF <= ktiles; kt += PF) {
-    tile(ic<0>{}, kt);
-    tile(ic<1>{}, kt + 1);
-    tile(ic<2>{}, kt + 2);
+    tile(ic<0>{}, kt, ic<0>{});
+    tile(ic<1>{}, kt + 1, ic<0>{});
+    tile(ic<2>{}, kt + 2, ic<0>{});
   }
   if (kt < ktiles) {
-    tile(ic<0>{}, kt);
-    if (kt + 1 < ktiles) tile(ic<1>{}, kt + 1);
+    tile(ic<0>{}, kt, ic<1>{});
+    if (kt + 1 < ktiles) tile(ic<1>{}, kt + 1, ic<1>{});
   }
 
   if (lora) {
