@@ -705,6 +705,42 @@ def test_gqa_attention_many_positions_equals_few(gpu, B, T, S, Hq, Hkv, col, win
   assert torch.equal(whole.view(torch.int16), parts.view(torch.int16))
 
 
+@pytest.mark.parametrize("M,D,V,temperature", [(1, 128, 65536, 1.0), (17, 384, 65552, 0.7), (64, 256, 66000, 1.0),
+                                               (65, 256, 65536, 1.0)])
+def test_dense_head_over_few_rows_equals_many(gpu, M, D, V, temperature):
+  """A dense head's copy over at most 64 rows takes a tile of 64 rows: every statistic is bit for bit that
+  of the same rows inside a call of 200 (the sums run over the same k in the same order)."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  w = bf(rnd((V, D), 101, 0.05)).to(gpu)
+  we = ops.dense_expand(w)
+  x = bf(rnd((200, D), 102)).to(gpu)
+  targets = torch.randint(0, V, (200,), generator=torch.Generator().manual_seed(103), dtype=torch.int32).to(gpu)
+
+  def run(n):
+    d = L.LmHeadDesc()
+    nvb = (V + 127) // 128
+    part = torch.full((n, nvb, 4), float("nan"), device=gpu)
+    out = [torch.empty(n, dtype=t, device=gpu) for t in (torch.int32, torch.float32, torch.float32, torch.float32)]
+    d.M, d.D, d.V, d.x, d.w_bf16, d.w_expanded = n, D, V, x.data_ptr(), w.data_ptr(), we.data_ptr()
+    d.targets, d.part, d.temperature = targets.data_ptr(), part.data_ptr(), temperature
+    d.best_id, d.best_logp, d.target_logp, d.lse = (o.data_ptr() for o in out)
+    ops.lmhead(d)
+    torch.cuda.synchronize()
+    return out, part
+
+  (few, fp), (many, mp) = run(M), run(200)
+  assert torch.isfinite(few[3]).all()
+  for a, b in zip(few, many):
+    assert torch.equal(a, b[:M])
+  assert torch.equal(fp.view(torch.int32), mp[:M].view(torch.int32))
+  ref = torch.log_softmax((x[:M].float().cpu() @ w.float().cpu().T).bfloat16().float() / temperature, -1)
+  got = few[2].cpu()
+  want = ref.gather(1, targets[:M].long().cpu()[:, None])[:, 0]
+  # (a logit may round to the neighbouring bf16 value: one ulp of the largest, scaled by the temperature)
+  assert (got - want).abs().max() <= 2.0 ** -7 * ref.abs().max() / temperature
+
+
 @pytest.mark.parametrize("M,D,V,dense", [(8, 512, 32000, True), (128, 512, 4096, True),
                                          (130, 256, 1040, True),   # two row blocks, partial last column block
                                          (50, 256, 1040, False), (130, 256, 4096, False)])

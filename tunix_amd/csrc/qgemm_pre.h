@@ -9,6 +9,9 @@
 //     compiler's form gives source and destination registers of their own and spent 720 register copies per k-tile.
 //   * RT = 16 (one work-group per compute unit, 256 accumulators): a wave's weights serve 256 rows, half the bytes from L2
 //     per row of RT = 8 (two work-groups per unit), which is there for calls with too few tiles to fill the device.
+//   * RT = 4 (three work-groups per unit) is for an lm_head over at most 64 rows, which is bound by the stream of its weights: they
+//     are read once, with the non-temporal policy, and a row tile's MFMAs stay below that.  128256 x 4096 at 16 rows 203 -> 172 us
+//     (1.05 GB: 6.1 TB/s with the finishing launch), 262144 x 1152 at 64 rows 143 -> 109 us, 151936 x 2048 at 64 rows 150 -> 120 us.
 //   * activations go from memory straight into LDS, in steps of 64 k (rows of 128 bytes, 16-byte chunks swizzled by row)
 //     through four buffers, two steps ahead of their use and spread evenly over the loop: a burst of such loads would
 //     stand between a weight fragment and the compiler's wait for it, which does not count them.
@@ -71,7 +74,7 @@ constexpr int kLoraInPlace = 1, kLoraScaled = 2;
 
 template <int RT, bool GROUPED, int KIND, int LORA>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(RT == 16 ? 1 : 2, RT == 16 ? 1 : 2)))
+__attribute__((amdgpu_waves_per_eu(RT == 16 ? 1 : RT == 8 ? 2 : 3, RT == 16 ? 1 : RT == 8 ? 2 : 3)))
 void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   constexpr int ROWS = 16 * RT, CT = 4, S = kPreStages, PASSES = RT / 2, HALF = RT / 4;   // PASSES: LDS loads of a step per thread
   constexpr uint32_t SB = pre_step_bytes<RT>();
@@ -254,7 +257,8 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   auto load_w = [&](auto Qc, int ct, int kt) {   // slab Q (0..3) of k-tile kt
     constexpr int Q = decltype(Qc)::value;
     wr[Q % S][ct] = __builtin_amdgcn_raw_buffer_load_b128(re, evoff + (uint32_t)(ct & 1) * 256u,
-                                                         (wt0 + min(kt, ktiles - 1)) * 65536 + (ct >> 1) * 8192 + Q * 2048, 0);
+                                                         (wt0 + min(kt, ktiles - 1)) * 65536 + (ct >> 1) * 8192 + Q * 2048,
+                                                         RT == 4 ? kStreamOnce : 0);
   };
   // One slab (32 k) of k-tile kt: RT x 4 MFMAs, and with them the fragments of the next slab, the weights of the slab three
   // further on into the stage that the slab before has finished with, and half a step of activations for the buffer
