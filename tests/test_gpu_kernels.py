@@ -195,6 +195,65 @@ def test_qlinear_lora_matches_oracle(gpu, M, K, N, group, qtype, r, split):
   assert_bf16_close(y, ref, what="qlinear")
 
 
+@pytest.mark.parametrize("M,K,N,split,group,qtype,rank,nseg,epi", [
+    (1, 512, 128, 1, 64, Q.NF4, 64, 1, "store"),          # four k-tiles: the four-way form's first, half a turn
+    (3, 640, 208, 1, 32, Q.NF4, 32, 1, "residual"),       # a last column block of five tiles, four scales per k-tile
+    (8, 1408, 512, 3, 64, Q.INT4, 64, 3, "store"),        # eleven k-tiles in splits of 4, 4, 3; three adapter segments
+    (5, 1152, 768, 1, 128, Q.NF4, 64, -1, "silu"),        # nine k-tiles, gate | up with the next adapter's planes
+    (9, 1536, 256, 1, 64, Q.NF4, 0, 1, "f32"),            # twelve k-tiles: the two-way form's first
+    (16, 1664, 384, 1, 64, Q.INT4, 96, 1, "store"),       # thirteen; an adapter of more than 64 ranks
+    (12, 4096, 320, 2, 256, Q.NF4, 64, -1, "gelu"),       # sixteen per split
+    (16, 2304, 640, 1, 64, Q.NF4, 64, -1, "silu"),        # eighteen
+])
+def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank, nseg, epi):
+  """At most 16 rows (activations straight from memory, sums of the k slices at the end) against the same rows
+  in a call of 24 (activations through LDS).  Same products; a column's fp32 sum of K terms in another order, so a
+  rounded result may be the neighbouring bf16 value."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  mul = epi in ("silu", "gelu")
+  x, t, res = bf(rnd((24, K), 111)).to(gpu), bf(rnd((24, 320), 112)).to(gpu), bf(rnd((24, N), 113)).to(gpu)
+  c, s = ops.quantize_pack(bf(rnd((K, N), 114, 0.03)).to(gpu), group, qtype, mul)
+  lb = bf(rnd((N, max(rank, 32)), 115, 0.1)).to(gpu)
+  ends = [N] if nseg < 2 else [N // 2, N * 3 // 4 // 16 * 16, N][:nseg]
+  nxt = bf(rnd((64, N // 2), 116, 0.05)).to(gpu)
+
+  def run(n):
+    y = torch.full((n, N // 2 if mul else N), 7.0, dtype=torch.float32 if epi == "f32" else torch.bfloat16, device=gpu)
+    ws = torch.full((split * n * N,), float("nan"), device=gpu) if split > 1 else None
+    kw = dict(lora_rank=rank, lora_nseg=nseg, lora_seg_end=ends, lora_seg_toff=[i * 64 for i in range(len(ends))], t=t,
+              t_ld=320, lora_b=lb, lora_scale=1.5) if rank else {}
+    planes = None
+    if mul and split == 1:
+      planes = torch.full(((N + 127) // 128 * 8192,), float("nan"), device=gpu)
+      kw.update(next_a_t=nxt, next_rank=64, next_tpart=planes)
+    d = ops.make_qlinear_desc(M=n, K=K, N=N, group=group, qtype=qtype, x=x, codes=c, scales=s, y=y, split_k=split, ws=ws,
+                              epilogue={"store": L.TNX_EPI_STORE, "residual": L.TNX_EPI_RESIDUAL, "f32": L.TNX_EPI_F32,
+                                        "silu": L.TNX_EPI_SILU_MUL, "gelu": L.TNX_EPI_GELU_MUL}[epi],
+                              residual=res if epi == "residual" else None, **kw)
+    ops.qlinear(d)
+    tn = None
+    if planes is not None:
+      tn = torch.zeros(n, 64, dtype=torch.bfloat16, device=gpu)
+      ops.lora_reduce(planes, n, (N + 127) // 128, 64, tn)
+    torch.cuda.synchronize()
+    return y, tn
+
+  (few, tf), (many, tm) = run(M), run(24)
+  # (magnitude of a result's terms: gated products and sums with a residual are rounded more than once)
+  ulps = 3 if mul else 1
+  if epi == "f32":
+    # |sum error| <= 2 K eps * sum |terms|: K terms of about 0.03 in random signs
+    assert (few - many[:M]).abs().max().item() <= 2 * K * 2.0 ** -24 * K * 0.03
+  else:
+    mag = None if epi != "residual" else torch.maximum(many[:M].float().abs(), res[:M].float().abs())
+    assert_bf16_close(few, many[:M], min_equal=0.95, what=epi, mag=mag, ulps=ulps)
+  if tf is not None:
+    assert torch.isfinite(tf.float()).all()
+    # t of the next adapter: products of activations that may differ by an ulp each
+    assert (tf.float() - tm[:M].float()).abs().max().item() <= 2.0 ** -6 * tm.float().abs().max().item()
+
+
 @pytest.mark.parametrize("M,K,N,split", [
     (128, 4096, 1024, 1),       # 32 k-tiles: two behind the whole turns of the weight ring
     (128, 4096, 1024, 4),       # eight of each split: two

@@ -78,15 +78,7 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs 
   for (int i = tid; i <= E; i += kMoeWaves * 64) offs[i] = a.offsets[i];
   for (int i = tid; i < n_routes; i += kMoeWaves * 64) routes[i] = a.sorted_route[i];
   static_assert(kMoeWaves == 8, "the table is written by 512 threads");
-  if constexpr (!INT4) {  // table entry e = f16 pair (level[e & 15], level[e >> 4]), 64 copies rotated over the banks
-    const float lvl0 = rbf(code_level_imm(a.qtype, tid & 15)), lvl1 = rbf(code_level_imm(a.qtype, (tid >> 4) & 15));
-    uint32_t* lut = reinterpret_cast<uint32_t*>(smem);
-    const h16x2 h = {(_Float16)lvl0, (_Float16)lvl1};
-    const uint32_t v = __builtin_bit_cast(uint32_t, h);
-    const int e = tid & 255, c0 = (tid >> 8) * 32;
-#pragma unroll
-    for (int c = 0; c < 32; ++c) lut[e * 64 + ((c0 + c + lane) & 63)] = v;
-  }
+  if constexpr (!INT4) fill_level_table<512>(0u, tid);
   __syncthreads();
   if (wv == 0) {  // non-empty (expert, row block) pairs in expert order: a running sum over the experts
     int carry = 0;

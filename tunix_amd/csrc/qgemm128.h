@@ -36,6 +36,7 @@ constexpr int kBigLutBytes = 256 * 256;
 // column tile) behind it
 constexpr uint32_t kBigLutBase = 0x10000, kBigAdapterBase = kBigLutBase + kBigLutBytes;
 constexpr size_t big_abytes(int mt) { return (size_t)(mt < 2 ? 32 : 16 * mt) * KTILE * 2; }
+static_assert(8 * 16 * 36 * 4 <= 2 * (int)big_abytes(4), "the plane transposition fits the activation buffers");
 constexpr size_t big_smem_bytes(int nt, int mt) { return kBigAdapterBase + 4 * (size_t)nt * 2048; }
 static_assert(2 * big_abytes(8) <= kBigLutBase, "the activation tiles end where the table starts");
 
@@ -65,6 +66,143 @@ __device__ unsigned long long tnx_stamps[8];
 #else
 #define TNX_STAMP(i) do {} while (0)
 #endif
+
+// The table of the code book: entry e at base + 256 e = the f16 pair (level[e & 15], level[e >> 4]), 64 copies.  16 bytes per lane and store, one
+// entry per 16 lanes; a pass of the work-group covers THREADS / 16 entries, so the lower level is the thread's own throughout and the
+// upper one uniform per wave, from literals: nothing here waits on memory.  (Against a row per thread in 4-byte stores:
+// a decode linear takes 0.2-0.3 us less, 4096 -> 4096 over 64 rows 9.1 -> 9.0, 1152 -> 13824 11.7 -> 11.3.)
+template <int THREADS>
+__device__ __forceinline__ void fill_level_table(uint32_t base, int tid) {
+  static_assert(THREADS % 256 == 0, "whole rows of upper levels per pass");
+  constexpr int RPP = THREADS / 256;   // upper levels per pass
+  const uint32_t lo = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)rbf(code_level_imm(TNX_Q_NF4, (tid >> 4) & 15)));
+  const int r = __builtin_amdgcn_readfirstlane(tid >> 8);
+#pragma unroll
+  for (int c = 0; c < 16 / RPP; ++c) {
+    uint32_t hi = 0;
+#pragma unroll
+    for (int i = 0; i < RPP; ++i) {
+      const uint32_t h = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)rbf(code_level_imm(TNX_Q_NF4, c * RPP + i))) << 16;
+      hi = i == 0 || r == i ? h : hi;
+    }
+    const uint32_t v = lo | hi;
+    lds_st128(base + (uint32_t)(c * THREADS + tid) * 16u, u32x4{v, v, v, v});
+  }
+}
+
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+constexpr uint32_t kRowsActBytes = 72 * 2;            // per row of the activation staging
+constexpr uint32_t kRowsScratchBytes = 8 * 16 * 36 * 4;
+// The end of a work-group of eight waves over 16 * MT rows x 128 columns: wave wv holds in `out` the sums of row tiles
+// (wv / 4) * HM ... and column tiles 2 (wv % 4), + 1 (with one row tile waves 0-3 hold all of it).  act_lds: 16 MT rows of
+// kRowsActBytes; scr_lds (SCRATCH): kRowsScratchBytes; both idle for every wave by now.
+template <int MT, int NT, bool SCRATCH>
+__device__ __forceinline__ void quant_rows_out(const QLArgs& a, f32x4 (&out)[(MT + 1) / 2][NT], int64_t m0, int64_t ntile0, int wv,
+                                               uint32_t act_lds, uint32_t scr_lds) {
+  constexpr int HM = (MT + 1) / 2, ROWS = 16 * MT;
+  const int tid = threadIdx.x, lane = tid & 63, lm = lane & 15, lq = lane >> 4, wn = wv & 3, kh = wv >> 2;
+  const bool has_rows = MT > 1 || kh == 0;
+  const int64_t m0w = m0 + kh * (HM * 16), ntiles = a.N / 16;
+  const bool mul = a.epilogue == TNX_EPI_SILU_MUL || a.epilogue == TNX_EPI_GELU_MUL;
+  if (NT == 2 && mul && a.split_k <= 1) {
+    // act = f(gate) * up goes through LDS (the activation buffer the adapter block is not in):
+    // rows leave the work-group as 128-byte runs instead of 2-byte scatters, and, when asked,
+    // the tile is multiplied with the NEXT linear's adapter A (its LoRA down-projection, whose
+    // K axis is this kernel's output axis), one fp32 fragment plane per work-group.
+    constexpr int ACT_LD = 72;  // 64 act columns + 8 pad (bf16 elements)
+    const int64_t ldy = a.N / 2;
+    const int64_t wgcol0 = (int64_t)blockIdx.y * 64;      // first act column of the work-group
+    const bool fuse_next = a.next_tpart != nullptr;
+    u32x4 bn[4][2];
+    if (fuse_next) {
+      const rsrc_t rn = make_rsrc(a.next_a_t, (uint64_t)a.next_rank * ldy * 2);
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int64_t k = wgcol0 + j * 32 + lq * 8;
+          const bool ok = n * 16 < a.next_rank && k + 8 <= ldy;
+          bn[n][j] = buf_load128(rn, ok ? (uint32_t)(((int64_t)(n * 16 + lm) * ldy + k) * 2) : 0xfffffff0u);
+        }
+    }
+    if (has_rows) {
+#pragma unroll
+      for (int mt = 0; mt < HM; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float g = rbf(out[mt][0][i]);
+          const float u = rbf(out[mt][1][i]);
+          const float act = a.epilogue == TNX_EPI_SILU_MUL ? silu_bf16(g) : gelu_tanh_bf16(g);
+          *reinterpret_cast<lds_u16*>(static_cast<uintptr_t>(act_lds + (uint32_t)(((kh * (HM * 16) + mt * 16 + lq * 4 + i) * ACT_LD + wn * 16 + lm) * 2))) =
+              f2bf(rbf(act) * u);
+        }
+    }
+    __syncthreads();
+    uint16_t* y = reinterpret_cast<uint16_t*>(a.y);
+#pragma unroll
+    for (int c = 0; c < (ROWS * 8 + 511) / 512; ++c) {
+      const int idx = tid + 512 * c, row = idx >> 3, ch = idx & 7;
+      if (row >= ROWS) break;
+      const u32x4 v = lds_ld128(act_lds + (uint32_t)((row * ACT_LD + ch * 8) * 2));
+      if (m0 + row < a.M && wgcol0 + ch * 8 + 8 <= ldy)
+        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(y + (m0 + row) * ldy + wgcol0 + ch * 8));
+    }
+    if (fuse_next && wv < MT) {   // one row tile per wave; fewer rows leave plane slots unwritten
+      float* plane = a.next_tpart + ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * 8192;
+      {
+        const int mt = wv;
+        u32x4 af2[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          af2[j] = lds_ld128(act_lds + (uint32_t)(((mt * 16 + lm) * ACT_LD + j * 32 + lq * 8) * 2));
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+          f32x4 pacc = f32x4{0.f, 0.f, 0.f, 0.f};
+          pacc = mfma16(af2[0], bn[n][0], pacc);
+          pacc = mfma16(af2[1], bn[n][1], pacc);
+          __builtin_nontemporal_store(pacc, reinterpret_cast<f32x4*>(plane + ((mt * 4 + n) * 64 + lane) * 4));
+        }
+      }
+    }
+  } else if (NT == 2 && SCRATCH && a.split_k > 1 && has_rows && ntile0 + NT <= ntiles &&
+             (uint64_t)a.M * (uint64_t)a.N * 4 < (1ull << 32)) {
+    // fp32 partial plane of this k split.  A lane's accumulators are four rows of one column;
+    // stored as they are, a wave would issue 32 four-byte stores of 64-byte runs.  Each 16 x 32
+    // row tile goes through a wave-private corner of LDS instead and leaves as two 16-byte stores per lane, 128-byte
+    // runs (rows past M fall outside the plane's buffer and are dropped).  The planes are written
+    // once and read once, by another kernel on other XCDs: stored with the non-temporal policy
+    // (decode step 6.51 -> 6.42 ms; the same policy on the outputs of the norm and of attention,
+    // which many work-groups re-read, measured neutral and is not used there).
+    constexpr int T_LD = 36;   // floats per LDS row: 32 + 4, conflict-free for both passes
+    const uint32_t scr = scr_lds + (uint32_t)wv * (16u * T_LD * 4u);
+    const rsrc_t rp = make_rsrc(a.ws + (int64_t)blockIdx.z * a.M * a.N, (uint64_t)a.M * a.N * 4);
+    const uint32_t col0 = (uint32_t)ntile0 * 16u;
+#pragma unroll
+    for (int mt = 0; mt < HM; ++mt) {
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = out[mt][nt][i];   // (a bit cast applied to the vector element itself reads element 0)
+          *reinterpret_cast<lds_u32*>(static_cast<uintptr_t>(scr + (uint32_t)(((lq * 4 + i) * T_LD + nt * 16 + lm) * 4))) =
+              __float_as_uint(v);
+        }
+      // (the reads below are of another type than the writes above: keep the compiler from
+      // moving them across; LDS itself executes a wave's accesses in order)
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int r = (lane >> 3) + 8 * j, c4 = (lane & 7) * 4;
+        const u32x4 v = lds_ld128(scr + (uint32_t)((r * T_LD + c4) * 4));
+        const uint32_t off = ((uint32_t)(m0w + mt * 16 + r) * (uint32_t)a.N + col0 + (uint32_t)c4) * 4u;
+        __builtin_amdgcn_raw_buffer_store_b128(v, rp, off, 0, kStreamOnce);
+      }
+      asm volatile("" ::: "memory");
+    }
+  } else {
+    if (has_rows) store_tile<HM, NT>(a, m0w, a.M, ntile0, ntiles, out, [](int64_t r) { return r; });
+  }
+}
 
 // 512 threads: waves 0-3 and 4-7 share the four column groups and split every k-tile between
 // them (k-steps 0,1 | 2,3), which puts two waves on each SIMD at 256 registers each.
@@ -97,9 +235,6 @@ void qgemm128_kernel(const QLArgs a) {
   asm volatile("" ::"s"(a.t_ld), "s"(a.t), "s"(a.lora_b), "s"(a.lora_scale), "s"(a.epilogue), "s"(a.y),
                "s"(a.split_k), "s"(a.ws), "s"(a.ktiles_per_split), "s"(a.next_a_t), "s"(a.next_rank),
                "s"(a.next_tpart));
-  // the two code-book levels of this thread's table entry, from literals: nothing at the start
-  // of the kernel waits on memory except the loads of the first tiles
-  const float lvl0 = rbf(code_level_imm(a.qtype, tid & 15)), lvl1 = rbf(code_level_imm(a.qtype, (tid >> 4) & 15));
   const uint32_t lane_off = (uint32_t)lane * 4u | kBigLutBase;   // byte 2 = 1: the table's base
   Int4Magic magic;
   if constexpr (INT4) magic.pin<true>();
@@ -429,14 +564,7 @@ void qgemm128_kernel(const QLArgs a) {
     // to "everything outstanding" for the sake of the path that enters from here.
     TNX_STAMP(7);
     if constexpr (!INT4) {
-       // table entry e = f16 pair (level[e & 15], level[e >> 4]); copies rotated over banks,
-       // half of them per thread; built while the first loads are in flight
-      uint32_t* lut = reinterpret_cast<uint32_t*>(smem + kBigLutBase);
-      const h16x2 h = {(_Float16)lvl0, (_Float16)lvl1};
-      const uint32_t v = __builtin_bit_cast(uint32_t, h);
-      const int e = tid & 255, c0 = (tid >> 8) * 32;
-#pragma unroll
-      for (int c = 0; c < 32; ++c) lut[e * 64 + ((c0 + c + lane) & 63)] = v;
+      fill_level_table<512>(kBigLutBase, tid);   // while the first loads are in flight
     }
     // The rest of the first loads go out behind the table: what the first k-tile needs (its
     // activations and weights, requested above by every wave) is then at the head of the unit's
@@ -558,108 +686,7 @@ void qgemm128_kernel(const QLArgs a) {
     tile_lora<HM, NT>(s, m0w, ntile0, toff, out);
   }
   TNX_STAMP(4);
-  const bool mul = a.epilogue == TNX_EPI_SILU_MUL || a.epilogue == TNX_EPI_GELU_MUL;
-  if (NT == 2 && mul && a.split_k <= 1) {
-    // act = f(gate) * up goes through LDS (the activation buffer the adapter block is not in):
-    // rows leave the work-group as 128-byte runs instead of 2-byte scatters, and, when asked,
-    // the tile is multiplied with the NEXT linear's adapter A (its LoRA down-projection, whose
-    // K axis is this kernel's output axis), one fp32 fragment plane per work-group.
-    constexpr int ACT_LD = 72;  // 64 act columns + 8 pad (bf16 elements)
-    const uint32_t act_lds = t_buf ^ ABYTES;
-    const int64_t ldy = a.N / 2;
-    const int64_t wgcol0 = (int64_t)blockIdx.y * 64;      // first act column of the work-group
-    const bool fuse_next = a.next_tpart != nullptr;
-    u32x4 bn[4][2];
-    if (fuse_next) {
-      const rsrc_t rn = make_rsrc(a.next_a_t, (uint64_t)a.next_rank * ldy * 2);
-#pragma unroll
-      for (int n = 0; n < 4; ++n)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int64_t k = wgcol0 + j * 32 + lq * 8;
-          const bool ok = n * 16 < a.next_rank && k + 8 <= ldy;
-          bn[n][j] = buf_load128(rn, ok ? (uint32_t)(((int64_t)(n * 16 + lm) * ldy + k) * 2) : 0xfffffff0u);
-        }
-    }
-    uint16_t* act_s = reinterpret_cast<uint16_t*>(smem + act_lds);
-    if (has_rows) {
-#pragma unroll
-      for (int mt = 0; mt < HM; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float g = rbf(out[mt][0][i]);
-          const float u = rbf(out[mt][1][i]);
-          const float act = a.epilogue == TNX_EPI_SILU_MUL ? silu_bf16(g) : gelu_tanh_bf16(g);
-          act_s[(kh * (HM * 16) + mt * 16 + lq * 4 + i) * ACT_LD + wn * 16 + lm] = f2bf(rbf(act) * u);
-        }
-    }
-    __syncthreads();
-    uint16_t* y = reinterpret_cast<uint16_t*>(a.y);
-#pragma unroll
-    for (int c = 0; c < (ROWS * 8 + 511) / 512; ++c) {
-      const int idx = tid + 512 * c, row = idx >> 3, ch = idx & 7;
-      if (row >= ROWS) break;
-      const u32x4 v = lds_ld128(act_lds + (uint32_t)((row * ACT_LD + ch * 8) * 2));
-      if (m0 + row < a.M && wgcol0 + ch * 8 + 8 <= ldy)
-        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(y + (m0 + row) * ldy + wgcol0 + ch * 8));
-    }
-    if (fuse_next && wv < MT) {   // one row tile per wave; fewer rows leave plane slots unwritten
-      float* plane = a.next_tpart + ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * 8192;
-      {
-        const int mt = wv;
-        u32x4 af2[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          af2[j] = lds_ld128(act_lds + (uint32_t)(((mt * 16 + lm) * ACT_LD + j * 32 + lq * 8) * 2));
-#pragma unroll
-        for (int n = 0; n < 4; ++n) {
-          f32x4 pacc = f32x4{0.f, 0.f, 0.f, 0.f};
-          pacc = mfma16(af2[0], bn[n][0], pacc);
-          pacc = mfma16(af2[1], bn[n][1], pacc);
-          __builtin_nontemporal_store(pacc, reinterpret_cast<f32x4*>(plane + ((mt * 4 + n) * 64 + lane) * 4));
-        }
-      }
-    }
-  } else if (NT == 2 && MT >= 4 && a.split_k > 1 && has_rows && ntile0 + NT <= ntiles &&
-             (uint64_t)a.M * (uint64_t)a.N * 4 < (1ull << 32)) {
-    // fp32 partial plane of this k split.  A lane's accumulators are four rows of one column;
-    // stored as they are, a wave would issue 32 four-byte stores of 64-byte runs.  Each 16 x 32
-    // row tile goes through a wave-private corner of the activation buffers instead (idle since
-    // the barriers of the exchange above) and leaves as two 16-byte stores per lane, 128-byte
-    // runs (rows past M fall outside the plane's buffer and are dropped).  The planes are written
-    // once and read once, by another kernel on other XCDs: stored with the non-temporal policy
-    // (decode step 6.51 -> 6.42 ms; the same policy on the outputs of the norm and of attention,
-    // which many work-groups re-read, measured neutral and is not used there).
-    constexpr int T_LD = 36;   // floats per LDS row: 32 + 4, conflict-free for both passes
-    const uint32_t scr = (uint32_t)wv * (16u * T_LD * 4u);
-    static_assert(MT < 4 || 8 * 16 * T_LD * 4 <= 2 * (int)ABYTES, "transposition scratch fits the activation buffers");
-    const rsrc_t rp = make_rsrc(a.ws + (int64_t)blockIdx.z * a.M * a.N, (uint64_t)a.M * a.N * 4);
-    const uint32_t col0 = (uint32_t)ntile0 * 16u;
-#pragma unroll
-    for (int mt = 0; mt < HM; ++mt) {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float v = out[mt][nt][i];   // (a bit cast applied to the vector element itself reads element 0)
-          *reinterpret_cast<lds_u32*>(static_cast<uintptr_t>(scr + (uint32_t)(((lq * 4 + i) * T_LD + nt * 16 + lm) * 4))) =
-              __float_as_uint(v);
-        }
-      // (the reads below are of another type than the writes above: keep the compiler from
-      // moving them across; LDS itself executes a wave's accesses in order)
-      asm volatile("" ::: "memory");
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int r = (lane >> 3) + 8 * j, c4 = (lane & 7) * 4;
-        const u32x4 v = lds_ld128(scr + (uint32_t)((r * T_LD + c4) * 4));
-        const uint32_t off = ((uint32_t)(m0w + mt * 16 + r) * (uint32_t)a.N + col0 + (uint32_t)c4) * 4u;
-        __builtin_amdgcn_raw_buffer_store_b128(v, rp, off, 0, kStreamOnce);
-      }
-      asm volatile("" ::: "memory");
-    }
-  } else {
-    if (has_rows) store_tile<HM, NT>(a, m0w, a.M, ntile0, ntiles, out, [](int64_t r) { return r; });
-  }
+  quant_rows_out<MT, NT, (MT >= 4)>(a, out, m0, ntile0, wv, t_buf ^ ABYTES, 0u);
   TNX_STAMP(5);
 }
 

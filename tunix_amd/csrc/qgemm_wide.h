@@ -68,7 +68,6 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
                "s"(a.lora_seg_toff[2]), "s"(a.lora_seg_toff[3]));
   asm volatile("" ::"s"(a.t_ld), "s"(a.t), "s"(a.lora_b), "s"(a.lora_scale), "s"(a.epilogue), "s"(a.y),
                "s"(a.residual));
-  const float lvl0 = rbf(code_level_imm(a.qtype, tid & 15)), lvl1 = rbf(code_level_imm(a.qtype, (tid >> 4) & 15));
   const uint32_t lane_off = (uint32_t)lane * 4u | kWideLutBase;   // byte 2 = 1: the table's base
 
   // work-group id -> (row block, column tile): groups of 64 row blocks, the column tile moves
@@ -387,13 +386,7 @@ void qgemm_wide_kernel(const QLArgs a, const WideHead h) {
   // back to "everything outstanding" for the sake of the path that enters from here)
   load_a(0, 0u);
   load_w(ic<0>{}, 0);
-  if constexpr (MODE == kWideTable) {  // table entry e = f16 pair (level[e & 15], level[e >> 4]), 64 copies rotated over the banks
-    uint32_t* lut = reinterpret_cast<uint32_t*>(smem + kWideLutBase);
-    const h16x2 h = {(_Float16)lvl0, (_Float16)lvl1};
-    const uint32_t v = __builtin_bit_cast(uint32_t, h);
-#pragma unroll
-    for (int c = 0; c < 64; ++c) lut[tid * 64 + ((c + lane) & 63)] = v;
-  }
+  if constexpr (MODE == kWideTable) fill_level_table<256>(kWideLutBase, tid);
   load_a(1, kWideTileBytes);
   load_w(ic<1>{}, 1);
   load_w(ic<2>{}, 2);

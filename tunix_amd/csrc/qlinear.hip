@@ -185,6 +185,7 @@ __global__ __launch_bounds__(256) void moe_gmm_kernel(const QLArgs a) {
 
 }  // namespace
 #include "qgemm128.h"
+#include "qgemm_few.h"
 #include "wide_out.h"
 #include "qgemm_wide.h"
 #include "qgemm_pre.h"
@@ -744,6 +745,22 @@ int launch_qgemm128(hipStream_t st, const QLArgs& a) {
   return a.qtype == TNX_Q_INT4 ? launch_qgemm128_as<NT, SPT, MT, true>(st, a) : launch_qgemm128_as<NT, SPT, MT, false>(st, a);
 }
 
+template <int SPT, bool INT4, int CW>
+int launch_qgemm_few_as(hipStream_t st, const QLArgs& a) {
+  static std::once_flag once;
+  static int attr_rc = TNX_OK;
+  constexpr size_t kSmem = few_smem_bytes(INT4, CW);
+  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, CW>, kSmem); });
+  if (attr_rc) return attr_rc;
+  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, CW>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kSmem, st, a);
+  TNX_CHECK_LAUNCH("qgemm_few");
+  return TNX_OK;
+}
+template <int SPT, int CW>
+int launch_qgemm_few(hipStream_t st, const QLArgs& a) {
+  return a.qtype == TNX_Q_INT4 ? launch_qgemm_few_as<SPT, true, CW>(st, a) : launch_qgemm_few_as<SPT, false, CW>(st, a);
+}
+
 template <int SPT, int MODE>
 int launch_qgemm_wide_as(hipStream_t st, const QLArgs& a, const WideHead& h) {
   static std::once_flag once;
@@ -1051,6 +1068,9 @@ extern "C" int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* d) {
   // in register copies that cost more than the halved LDS traffic gains.
   const bool s2 = scales_per_tile(a.group) == 2;
   if (wide_shape(a)) return s2 ? launch_qgemm_wide<2>(st, a) : launch_qgemm_wide<4>(st, a);
+  // few rows: activations from memory instead of through LDS (both sides of the lines: qgemm_few.h)
+  if (a.M <= 8 && a.ktiles_per_split >= 4) return s2 ? launch_qgemm_few<2, 4>(st, a) : launch_qgemm_few<4, 4>(st, a);
+  if (a.M <= 16 && a.ktiles_per_split >= 12) return s2 ? launch_qgemm_few<2, 2>(st, a) : launch_qgemm_few<4, 2>(st, a);
   if (a.M <= 16) return s2 ? launch_qgemm128<2, 2, 1>(st, a) : launch_qgemm128<2, 4, 1>(st, a);
   if (a.M <= 32) return s2 ? launch_qgemm128<2, 2, 2>(st, a) : launch_qgemm128<2, 4, 2>(st, a);
   if (a.M <= 64) return s2 ? launch_qgemm128<2, 2, 4>(st, a) : launch_qgemm128<2, 4, 4>(st, a);
