@@ -1816,6 +1816,46 @@ def test_rope_row_kernel_equals_the_per_head_kernel(gpu, family, dh, Hq, Hkv):
     assert torch.equal(x, y), (name, int((diff > 0).sum()), diff.max().item(), torch.nonzero(diff > 0)[:4].tolist())
   assert one[0].float().abs().max() > 0.1 and one[1][:, :, col: col + T].float().abs().max() > 0.5
 
+@pytest.mark.parametrize("family,norm,Hq,Hkv,dh", [("qwen3", "qwen3", 32, 4, 128), ("gemma3", "gemma3", 4, 1, 256), ("llama3", "llama3", 3, 1, 16),
+                                                   ("qwen3", "gemma3", 5, 2, 64), ("llama3", "qwen3", 2, 1, 512)])
+def test_normed_heads_over_many_rows_equal_the_per_head_kernel(gpu, family, norm, Hq, Hkv, dh):
+  """512 rows in one call (a head's squares summed over its own lanes) against 128 per call (over a work-group):
+  the fp32 sum runs in another order, so a rounded result may be the neighbouring bf16 value; columns that
+  wrap around the cache included."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  from tunix_amd.model import _NORM, _ROPE, rope_timescale
+  B, T, S, col = 4, 128, 132, 9
+  qkv = bf(rnd((B, T, (Hq + 2 * Hkv) * dh), 121)).to(gpu)
+  pos = torch.randint(0, 2000, (B, col + T), generator=torch.Generator().manual_seed(122), dtype=torch.int32).to(gpu)
+  ts = torch.from_numpy(rope_timescale(dh, 1e6)).to(gpu)
+  wq, wk = bf(rnd((dh,), 123)).to(gpu), bf(rnd((dh,), 124)).to(gpu)
+  colp = torch.tensor([col], dtype=torch.int32, device=gpu)
+
+  def run(rows):
+    q = torch.zeros(B, T, Hq * dh, dtype=torch.bfloat16, device=gpu)
+    kc = torch.zeros(B, Hkv, S, dh, dtype=torch.bfloat16, device=gpu)
+    vc = torch.zeros_like(kc)
+    for b0 in range(0, B, rows):
+      d = L.RopeDesc()
+      d.B, d.T, d.S, d.Hq, d.Hkv, d.dh = rows, T, S, Hq, Hkv, dh
+      d.rope_flavor, d.rope_scale, d.timescale = _ROPE[family], 8.0 if family == "gemma3" else 1.0, ts.data_ptr()
+      d.qk_norm, d.norm_eps, d.q_norm_w, d.k_norm_w = _NORM[norm], 1e-6, wq.data_ptr(), wk.data_ptr()
+      d.q_prescale = 0.25 if family == "gemma3" else 0.0
+      d.qkv, d.positions, d.pos_ld, d.col_ptr = qkv[b0:].data_ptr(), pos[b0:].data_ptr(), pos.shape[1], colp.data_ptr()
+      d.q_out, d.kcache, d.vcache = q[b0:].data_ptr(), kc[b0:].data_ptr(), vc[b0:].data_ptr()
+      ops.rope_kvwrite(d)
+    torch.cuda.synchronize()
+    return q, kc, vc
+
+  one, four = run(B), run(1)
+  # a rotated element is x1 cos - x2 sin of normed elements that may each be one ulp off: ulps of the larger operand
+  mag = float(max(one[0].abs().max(), one[1].abs().max()))
+  for what, x, y in zip(("q", "k cache"), one, four):
+    assert_bf16_close(x, y, min_equal=0.98, what=what, atol=2 * mag * 2.0 ** -7)
+  assert torch.equal(one[2], four[2])
+
+
 
 @pytest.mark.parametrize("family", ["llama3", "qwen3"])
 def test_rope_from_splitk_planes_equals_finish_then_rope(gpu, family):

@@ -352,149 +352,213 @@ struct RopeArgs {
   int split_k;
 };
 
-// grid (B*T, Hq + 2*Hkv); max(64, dh/2) threads: thread i < dh/2 owns elements i and i + dh/2
-// of one head; the other threads only take part in the reductions.
-__global__ void rope_kernel(const RopeArgs a) {
-  __shared__ float red[4];
-  const int64_t row = blockIdx.x;
-  const int64_t b = row / a.T, t = row % a.T;
-  const int head = blockIdx.y;
-  const int half = a.dh / 2, i = threadIdx.x;
-  const bool live = i < half;
-  const int col = *a.col_ptr;
-  const int ld = (a.Hq + 2 * a.Hkv) * a.dh;
-  const int64_t src_off = row * ld + (int64_t)head * a.dh;
-  // element e of this head: from the finished linear output, or as the linear's own finishing
-  // pass would produce it, bf16(sum of the split-k planes in split order)
-  auto src_at = [&](int e) -> float {
-    if (a.ws == nullptr) return bf2f(a.qkv[src_off + e]);
-    const int64_t plane = a.B * a.T * (int64_t)ld;
-    float v = 0.f;
-    for (int z0 = 0; z0 < a.split_k; z0 += 8) {  // eight planes' loads in flight; sum in split order
-      float p[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) p[u] = a.ws[(int64_t)min(z0 + u, a.split_k - 1) * plane + src_off + e];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (z0 + u < a.split_k) v += p[u];
-    }
-    return rbf(v);
-  };
-  const int slot = (int)((col + t) % a.S);
-  if (head >= a.Hq + a.Hkv) {  // V: plain copy into the cache slot
-    const int hk = head - a.Hq - a.Hkv;
-    uint16_t* dst = a.vcache + (((b * a.Hkv + hk) * a.S) + slot) * a.dh;
-    if (live) {
-      dst[i] = f2bf(src_at(i));
-      dst[i + half] = f2bf(src_at(i + half));
-    }
-    return;
-  }
-  const bool is_q = head < a.Hq;
-  float x1 = live ? src_at(i) : 0.f, x2 = live ? src_at(i + half) : 0.f;
-  if (a.qk_norm >= 0) {
-    const float ss = block_sum(sq_term(x1, a.qk_norm) + sq_term(x2, a.qk_norm), red);
-    const float ms = finish_ms(ss, (float)a.dh, a.qk_norm);
-    const uint16_t* w = is_q ? a.q_norm_w : a.k_norm_w;
-    if (live) {
-      x1 = norm_elem(x1, bf2f(w[i]), ms, a.norm_eps, a.qk_norm);
-      x2 = norm_elem(x2, bf2f(w[i + half]), ms, a.norm_eps, a.qk_norm);
-    }
-  }
-  if (!live) return;
-  const float pos = (float)a.positions[b * a.pos_ld + col + t];
-  float ang = __fdiv_rn(pos, a.timescale[i]);
-  if (a.rope_flavor == TNX_ROPE_GEMMA3) ang = __fdiv_rn(ang, a.rope_scale);
-  float sn = sinf(ang), cs = cosf(ang);
-  float o1, o2;
+// The rotated pair (x1, x2) of a q or k head, as bf16 values.
+__device__ __forceinline__ void rotate_pair(const RopeArgs& a, bool is_q, float x1, float x2, float sn, float cs, float& o1, float& o2) {
   if (a.rope_flavor == TNX_ROPE_QWEN3) {
-    sn = rbf(sn);
-    cs = rbf(cs);
     o1 = rbf(rbf(x1 * cs) - rbf(x2 * sn));
     o2 = rbf(rbf(x2 * cs) + rbf(x1 * sn));
   } else {
-    // fp32 products and sum, one rounding at the end (no fused multiply-add)
-    o1 = rbf(__fsub_rn(__fmul_rn(x1, cs), __fmul_rn(x2, sn)));
-    o2 = rbf(__fadd_rn(__fmul_rn(x2, cs), __fmul_rn(x1, sn)));
+    // fp32, one rounding to bf16 at the end; written as the fused forms the compiler makes of such a sum, so that every kernel takes the
+    // same one
+    o1 = rbf(__builtin_fmaf(x1, cs, -(x2 * sn)));
+    o2 = rbf(__builtin_fmaf(x2, cs, x1 * sn));
   }
-  if (is_q) {
-    if (a.q_prescale_bf != 0.f) {
-      o1 = rbf(o1 * a.q_prescale_bf);
-      o2 = rbf(o2 * a.q_prescale_bf);
-    }
-    uint16_t* dst = a.q_out + (row * a.Hq + head) * a.dh;
-    dst[i] = f2bf(o1);
-    dst[i + half] = f2bf(o2);
-  } else {
-    const int hk = head - a.Hq;
-    uint16_t* dst = a.kcache + (((b * a.Hkv + hk) * a.S) + slot) * a.dh;
-    dst[i] = f2bf(o1);
-    dst[i + half] = f2bf(o2);
+  if (is_q && a.q_prescale_bf != 0.f) {
+    o1 = rbf(o1 * a.q_prescale_bf);
+    o2 = rbf(o2 * a.q_prescale_bf);
   }
 }
+// sine and cosine of one (position, pair), rounded where the flavor rounds them
+__device__ __forceinline__ void rope_angle(const RopeArgs& a, float pos, float timescale, float& sn, float& cs) {
+  float ang = __fdiv_rn(pos, timescale);
+  if (a.rope_flavor == TNX_ROPE_GEMMA3) ang = __fdiv_rn(ang, a.rope_scale);
+  sn = sinf(ang);
+  cs = cosf(ang);
+  if (a.rope_flavor == TNX_ROPE_QWEN3) {
+    sn = rbf(sn);
+    cs = rbf(cs);
+  }
+}
+// cache slot of the token at column c (the cache is a ring; a division only where it wraps)
+__device__ __forceinline__ int64_t ring_slot(int64_t c, int64_t S) { return c < S ? c : c % S; }
 
-// Many rows, no q / k norm (a Llama prefill or whole-sequence pass): one work-group per token row,
-// 16-byte accesses, and the sine / cosine of a (row, i) computed once for all heads instead of
-// once per head.  Thread (ch, h0) owns the eight pairs i = 8 ch .. + 7 of heads h0, h0 + hstep, ...;
-// the arithmetic per element is rope_kernel's, so the outputs are bit-identical.
+// grid (B*T, Hq + 2*Hkv); max(64, dh/2) threads: thread i < dh/2 owns elements i and i + dh/2
+// of one head; the other threads only take part in the reductions.
+// A decode step's launch is a chain of round trips to memory, so everything that needs no other load is asked for at
+// once, ahead of the first wait, and the angle is computed while the planes arrive.  64 rows of 4 + 2 heads of 256 from eight planes, us
+// per launch 4.5 -> 3.7 alone; 32 + 8 heads of 128 from six 5.2 -> 4.2.
+template <bool PLANES>
+__global__ void rope_kernel(const RopeArgs a) {
+  __shared__ float red[4];
+  const uint32_t row = blockIdx.x;
+  const uint32_t b = row / (uint32_t)a.T, t = row - b * (uint32_t)a.T;
+  const int head = blockIdx.y;
+  const int half = a.dh / 2, i = threadIdx.x, il = min(i, half - 1);
+  const bool live = i < half, is_v = head >= a.Hq + a.Hkv, is_q = head < a.Hq, normed = a.qk_norm >= 0 && !is_v;
+  const int col = *a.col_ptr;
+  const int ld = (a.Hq + 2 * a.Hkv) * a.dh;
+  const int64_t src_off = (int64_t)row * ld + (int64_t)head * a.dh + il;
+  // elements i and i + half of this head: from the finished linear output, or as the linear's own finishing
+  // pass would produce them, bf16(sum of the split-k planes in split order)
+  float x1, x2;
+  float p1[8], p2[8];
+  uint16_t h1 = 0, h2 = 0;
+  const int64_t plane = a.B * a.T * (int64_t)ld;
+  if constexpr (PLANES) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float* p = a.ws + (int64_t)min(u, a.split_k - 1) * plane + src_off;
+      p1[u] = p[0];
+      p2[u] = p[half];
+    }
+  } else {
+    h1 = a.qkv[src_off];
+    h2 = a.qkv[src_off + half];
+  }
+  const uint16_t* wn = is_q ? a.q_norm_w : a.k_norm_w;
+  const float ts = a.timescale[il];
+  uint16_t w1 = 0, w2 = 0;
+  if (normed) {
+    w1 = wn[il];
+    w2 = wn[il + half];
+  }
+  const float pos = (float)a.positions[b * a.pos_ld + col + t];
+  float sn = 0.f, cs = 0.f;
+  if (!is_v) rope_angle(a, pos, ts, sn, cs);
+  if constexpr (PLANES) {
+    x1 = 0.f;
+    x2 = 0.f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (u < a.split_k) {
+        x1 += p1[u];
+        x2 += p2[u];
+      }
+    for (int z0 = 8; z0 < a.split_k; z0 += 8) {   // eight planes' loads in flight; sum in split order
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float* p = a.ws + (int64_t)min(z0 + u, a.split_k - 1) * plane + src_off;
+        p1[u] = p[0];
+        p2[u] = p[half];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (z0 + u < a.split_k) {
+          x1 += p1[u];
+          x2 += p2[u];
+        }
+    }
+    x1 = rbf(x1);
+    x2 = rbf(x2);
+  } else {
+    x1 = bf2f(h1);
+    x2 = bf2f(h2);
+  }
+  const int64_t slot = ring_slot((int64_t)col + t, a.S);
+  uint16_t* dst;
+  if (is_v) {   // V: plain copy into the cache slot
+    dst = a.vcache + ((((int64_t)b * a.Hkv + (head - a.Hq - a.Hkv)) * a.S) + slot) * a.dh;
+  } else {
+    if (normed) {
+      const float ss = block_sum(live ? sq_term(x1, a.qk_norm) + sq_term(x2, a.qk_norm) : 0.f, red);
+      const float ms = finish_ms(ss, (float)a.dh, a.qk_norm);
+      x1 = norm_elem(x1, bf2f(w1), ms, a.norm_eps, a.qk_norm);
+      x2 = norm_elem(x2, bf2f(w2), ms, a.norm_eps, a.qk_norm);
+    }
+    float o1, o2;
+    rotate_pair(a, is_q, x1, x2, sn, cs, o1, o2);
+    x1 = o1;
+    x2 = o2;
+    dst = is_q ? a.q_out + ((int64_t)row * a.Hq + head) * a.dh
+               : a.kcache + ((((int64_t)b * a.Hkv + (head - a.Hq)) * a.S) + slot) * a.dh;
+  }
+  if (!live) return;
+  dst[i] = f2bf(x1);
+  dst[i + half] = f2bf(x2);
+}
+
+// Many rows (a prefill or whole-sequence pass): one work-group per token row, 16-byte accesses; the sines and cosines of the
+// row's pairs are computed once, a pair per thread, and shared through LDS.  Thread (ch, h0) owns the eight pairs i = 8 ch .. + 7 of
+// heads h0, h0 + hstep, ...; a head's sum of squares (NORM) is formed over its dh / 16 neighbouring lanes.  Bound by
+// memory: qkv in, q and the cache slots out.  us: 7 x 1023 rows of 32 + 2 x 4 normed heads of 128 136 -> 49 (146 MB; before in rope_kernel, a
+// work-group per head), 2 x 6144 rows of 32 + 2 x 8 heads of 128 83 -> 49 (302 MB: 6.2 TB/s; before, sines by every thread for itself).
+template <bool NORM>
 __global__ __launch_bounds__(256) void rope_rows_kernel(const RopeArgs a) {
-  const int64_t row = blockIdx.x;
-  const int64_t b = row / a.T, t = row % a.T;
+  __shared__ float trig[2][256];   // [sine, cosine][pair]: head_dim at most 512
+  const uint32_t row = blockIdx.x;
+  const uint32_t b = row / (uint32_t)a.T, t = row - b * (uint32_t)a.T;
   const int half = a.dh / 2, CH = half / 8, heads = a.Hq + 2 * a.Hkv;
   const int ch = threadIdx.x % CH, h0 = threadIdx.x / CH, hstep = 256 / CH;
   const int col = *a.col_ptr;
   const int ld = heads * a.dh;
-  const int slot = (int)((col + t) % a.S);
+  const int64_t slot = ring_slot((int64_t)col + t, a.S);
   const int i0 = ch * 8;
-  const float pos = (float)a.positions[b * a.pos_ld + col + t];
-  float sn[8], cs[8];
+  u32x4 wq[2], wk[2];
+  if constexpr (NORM) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    float ang = __fdiv_rn(pos, a.timescale[i0 + e]);
-    if (a.rope_flavor == TNX_ROPE_GEMMA3) ang = __fdiv_rn(ang, a.rope_scale);
-    sn[e] = sinf(ang);
-    cs[e] = cosf(ang);
-    if (a.rope_flavor == TNX_ROPE_QWEN3) {
-      sn[e] = rbf(sn[e]);
-      cs[e] = rbf(cs[e]);
+    for (int p = 0; p < 2; ++p) {
+      wq[p] = *reinterpret_cast<const u32x4*>(a.q_norm_w + i0 + p * half);
+      wk[p] = *reinterpret_cast<const u32x4*>(a.k_norm_w + i0 + p * half);
     }
   }
-  for (int head = h0; head < heads; head += hstep) {
-    const uint16_t* src = a.qkv + row * ld + (int64_t)head * a.dh + i0;
+  if ((int)threadIdx.x < half) {
+    const float pos = (float)a.positions[b * a.pos_ld + col + t];
+    float sn, cs;
+    rope_angle(a, pos, a.timescale[threadIdx.x], sn, cs);
+    trig[0][threadIdx.x] = sn;
+    trig[1][threadIdx.x] = cs;
+  }
+  __syncthreads();
+  f32x4 sn[2], cs[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    sn[p] = *reinterpret_cast<const f32x4*>(&trig[0][i0 + 4 * p]);
+    cs[p] = *reinterpret_cast<const f32x4*>(&trig[1][i0 + 4 * p]);
+  }
+  for (int head = h0; head < heads; head += hstep) {   // (the lanes of a head stay together: heads differ by whole groups)
+    const uint16_t* src = a.qkv + (int64_t)row * ld + (int64_t)head * a.dh + i0;
     const u32x4 v1 = *reinterpret_cast<const u32x4*>(src), v2 = *reinterpret_cast<const u32x4*>(src + half);
     uint16_t* dst;
     if (head >= a.Hq + a.Hkv) {   // V: plain copy into the cache slot
-      dst = a.vcache + (((b * a.Hkv + (head - a.Hq - a.Hkv)) * a.S) + slot) * a.dh + i0;
+      dst = a.vcache + ((((int64_t)b * a.Hkv + (head - a.Hq - a.Hkv)) * a.S) + slot) * a.dh + i0;
       *reinterpret_cast<u32x4*>(dst) = v1;
       *reinterpret_cast<u32x4*>(dst + half) = v2;
       continue;
     }
     const bool is_q = head < a.Hq;
+    float x1[8], x2[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      x1[e] = (e & 1) ? bfhi(v1[e >> 1]) : bflo(v1[e >> 1]);
+      x2[e] = (e & 1) ? bfhi(v2[e >> 1]) : bflo(v2[e >> 1]);
+    }
+    if constexpr (NORM) {
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += sq_term(x1[e], a.qk_norm) + sq_term(x2[e], a.qk_norm);
+      for (int o = CH / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      const float ms = finish_ms(ss, (float)a.dh, a.qk_norm);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t w1 = is_q ? wq[0][e >> 1] : wk[0][e >> 1], w2 = is_q ? wq[1][e >> 1] : wk[1][e >> 1];
+        x1[e] = norm_elem(x1[e], (e & 1) ? bfhi(w1) : bflo(w1), ms, a.norm_eps, a.qk_norm);
+        x2[e] = norm_elem(x2[e], (e & 1) ? bfhi(w2) : bflo(w2), ms, a.norm_eps, a.qk_norm);
+      }
+    }
     u32x4 o1v, o2v;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float o1[2], o2[2];
 #pragma unroll
-      for (int hsel = 0; hsel < 2; ++hsel) {
-        const int e = 2 * r + hsel;
-        const float x1 = hsel ? bfhi(v1[r]) : bflo(v1[r]), x2 = hsel ? bfhi(v2[r]) : bflo(v2[r]);
-        if (a.rope_flavor == TNX_ROPE_QWEN3) {
-          o1[hsel] = rbf(rbf(x1 * cs[e]) - rbf(x2 * sn[e]));
-          o2[hsel] = rbf(rbf(x2 * cs[e]) + rbf(x1 * sn[e]));
-        } else {
-          o1[hsel] = rbf(__fsub_rn(__fmul_rn(x1, cs[e]), __fmul_rn(x2, sn[e])));
-          o2[hsel] = rbf(__fadd_rn(__fmul_rn(x2, cs[e]), __fmul_rn(x1, sn[e])));
-        }
-        if (is_q && a.q_prescale_bf != 0.f) {
-          o1[hsel] = rbf(o1[hsel] * a.q_prescale_bf);
-          o2[hsel] = rbf(o2[hsel] * a.q_prescale_bf);
-        }
+      for (int k = 0; k < 2; ++k) {
+        const int e = 2 * r + k;
+        rotate_pair(a, is_q, x1[e], x2[e], sn[e >> 2][e & 3], cs[e >> 2][e & 3], o1[k], o2[k]);
       }
       o1v[r] = pack2bf(o1[0], o1[1]);
       o2v[r] = pack2bf(o2[0], o2[1]);
     }
-    if (is_q) dst = a.q_out + (row * a.Hq + head) * a.dh + i0;
-    else dst = a.kcache + (((b * a.Hkv + (head - a.Hq)) * a.S) + slot) * a.dh + i0;
+    if (is_q) dst = a.q_out + ((int64_t)row * a.Hq + head) * a.dh + i0;
+    else dst = a.kcache + ((((int64_t)b * a.Hkv + (head - a.Hq)) * a.S) + slot) * a.dh + i0;
     *reinterpret_cast<u32x4*>(dst) = o1v;
     *reinterpret_cast<u32x4*>(dst + half) = o2v;
   }
@@ -628,17 +692,22 @@ extern "C" int tnx_qknorm_rope_kvwrite(void* stream, const tnx_rope_desc* d) {
   a.qkv = d->qkv; a.positions = d->positions; a.pos_ld = d->pos_ld; a.col_ptr = d->col_ptr;
   a.timescale = d->timescale; a.q_out = d->q_out; a.kcache = d->kcache; a.vcache = d->vcache;
   a.ws = d->qkv_ws; a.split_k = d->split_k;
-  // many rows of a model without q / k norm, from the finished linear output: the row kernel
+  // many rows, from the finished linear output: the row kernel.  Its thread groups are a head's dh / 16 lanes, whole ones in a
+  // work-group and, where they add up a head's squares, inside a wave and a power of two.
   const int chunks = d->dh / 16;
-  const bool aligned = (((uintptr_t)d->qkv | (uintptr_t)d->q_out | (uintptr_t)d->kcache | (uintptr_t)d->vcache) & 15) == 0;
-  if (d->qk_norm < 0 && !d->qkv_ws && d->B * d->T >= 256 && d->dh % 16 == 0 && chunks <= 256 && 256 % chunks == 0 &&
-      aligned) {
-    hipLaunchKernelGGL(rope_rows_kernel, dim3((unsigned)(d->B * d->T)), dim3(256), 0, as_stream(stream), a);
+  const bool norm = d->qk_norm >= 0;
+  const bool aligned = (((uintptr_t)d->qkv | (uintptr_t)d->q_out | (uintptr_t)d->kcache | (uintptr_t)d->vcache) & 15) == 0 &&
+                       (!norm || (((uintptr_t)d->q_norm_w | (uintptr_t)d->k_norm_w) & 15) == 0);
+  TNX_REQUIRE(d->B * d->T < (int64_t)1 << 31, "rope: too many rows");
+  if (!d->qkv_ws && d->B * d->T >= 256 && d->dh % 16 == 0 && 256 % chunks == 0 && aligned) {
+    if (norm) hipLaunchKernelGGL(rope_rows_kernel<true>, dim3((unsigned)(d->B * d->T)), dim3(256), 0, as_stream(stream), a);
+    else hipLaunchKernelGGL(rope_rows_kernel<false>, dim3((unsigned)(d->B * d->T)), dim3(256), 0, as_stream(stream), a);
     TNX_CHECK_LAUNCH("qknorm_rope_kvwrite (rows)");
     return TNX_OK;
   }
-  dim3 grid((unsigned)(d->B * d->T), (unsigned)(d->Hq + 2 * d->Hkv));
-  hipLaunchKernelGGL(rope_kernel, grid, dim3(d->dh / 2 < 64 ? 64 : d->dh / 2), 0, as_stream(stream), a);
+  dim3 grid((unsigned)(d->B * d->T), (unsigned)(d->Hq + 2 * d->Hkv)), block(d->dh / 2 < 64 ? 64 : d->dh / 2);
+  if (d->qkv_ws) hipLaunchKernelGGL(rope_kernel<true>, grid, block, 0, as_stream(stream), a);
+  else hipLaunchKernelGGL(rope_kernel<false>, grid, block, 0, as_stream(stream), a);
   TNX_CHECK_LAUNCH("qknorm_rope_kvwrite");
   return TNX_OK;
 }
