@@ -99,6 +99,21 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, con
   const int nchunks = (int)(D / 8);
   float h[MAXC][8];
   float ss = 0.f;
+  // The norm weights and the post-norm residual do not depend on the row: they are asked for ahead of its planes (a launch is a
+  // few round trips to memory long, and one that starts behind the sums adds a whole one: 16 rows of 4096 from
+  // eight planes 6.2 -> 5.7 us), or, for rows of more than 4096,
+  // whose registers do not hold them that long, before the reduction.
+  u32x4 wpre[MAXC], rpost[MAXC], w2pre[MAXC];
+  auto fetch_weights = [&]() {
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {
+      const int64_t at = (int64_t)min(c * 256 + (int)threadIdx.x, nchunks - 1) * 8;
+      wpre[c] = *reinterpret_cast<const u32x4*>(w + at);
+      if (w2) w2pre[c] = *reinterpret_cast<const u32x4*>(w2 + at);
+      if (res_post && res_post != h_out) rpost[c] = *reinterpret_cast<const u32x4*>(res_post + row * D + at);
+    }
+  };
+  if constexpr (MAXC <= 2) fetch_weights();
   // Chunks are taken two at a time with every load of the pair issued before the first sum (up
   // to eight planes per chunk at once, further planes in groups of eight): the kernel is a few
   // dependent memory round trips long, and each group of loads that waits for the previous sum
@@ -218,17 +233,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, con
       }
     }
   }
-  // the norm weights and the post-norm residual do not depend on the row statistics: fetch them
-  // before the reduction instead of behind it
-  u32x4 wpre[MAXC], rpost[MAXC];
-#pragma unroll
-  for (int c = 0; c < MAXC; ++c) {
-    const int ch = c * 256 + threadIdx.x;
-    if (ch < nchunks) {
-      wpre[c] = *reinterpret_cast<const u32x4*>(w + (int64_t)ch * 8);
-      if (res_post && res_post != h_out) rpost[c] = *reinterpret_cast<const u32x4*>(res_post + row * D + (int64_t)ch * 8);
-    }
-  }
+  if constexpr (MAXC > 2) fetch_weights();
   ss = block_sum(ss, red);
   const float ms = finish_ms(ss, (float)D, FLAVOR);
   float ss2 = 0.f;
@@ -271,7 +276,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, con
     const int ch = c * 256 + threadIdx.x;
     if (ch < nchunks) {
       float wv[8];
-      unpack8(*reinterpret_cast<const u32x4*>(w2 + (int64_t)ch * 8), wv);
+      unpack8(w2pre[c], wv);
       u32x4 q;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
