@@ -765,9 +765,9 @@ def test_gqa_attention_many_positions_equals_few(gpu, B, T, S, Hq, Hkv, col, win
 
 
 @pytest.mark.parametrize("M,D,V,temperature", [(1, 128, 65536, 1.0), (17, 384, 65552, 0.7), (64, 256, 66000, 1.0),
-                                               (65, 256, 65536, 1.0)])
+                                               (65, 256, 65536, 1.0), (128, 128, 65600, 1.0)])
 def test_dense_head_over_few_rows_equals_many(gpu, M, D, V, temperature):
-  """A dense head's copy over at most 64 rows takes a tile of 64 rows: every statistic is bit for bit that
+  """A dense head's copy over at most 64 rows takes a tile of 64 rows (up to 128: one of 128): every statistic is bit for bit that
   of the same rows inside a call of 200 (the sums run over the same k in the same order)."""
   from tunix_amd import _lib as L
   from tunix_amd import ops

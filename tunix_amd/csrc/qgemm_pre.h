@@ -9,8 +9,8 @@
 //     compiler's form gives source and destination registers of their own and spent 720 register copies per k-tile.
 //   * RT = 16 (one work-group per compute unit, 256 accumulators): a wave's weights serve 256 rows, half the bytes from L2
 //     per row of RT = 8 (two work-groups per unit), which is there for calls with too few tiles to fill the device.
-//   * RT = 4 (three work-groups per unit) is for an lm_head over at most 64 rows, which is bound by the stream of its weights: they
-//     are read once, with the non-temporal policy, and a row tile's MFMAs stay below that.  128256 x 4096 at 16 rows 203 -> 172 us
+//   * RT = 4 (three work-groups per unit) is for an lm_head over at most 64 rows, which is bound by the stream of its weights: the
+//     MFMAs of 64 rows stay below that.  128256 x 4096 at 16 rows 203 -> 172 us
 //     (1.05 GB: 6.1 TB/s with the finishing launch), 262144 x 1152 at 64 rows 143 -> 109 us, 151936 x 2048 at 64 rows 150 -> 120 us.
 //   * activations go from memory straight into LDS, in steps of 64 k (rows of 128 bytes, 16-byte chunks swizzled by row)
 //     through four buffers, two steps ahead of their use and spread evenly over the loop: a burst of such loads would
@@ -65,7 +65,11 @@ __device__ __forceinline__ int xcd_tile(int id, int tiles) {
 }
 // KIND, LORA: what happens to the finished tile, an instance each: with the forms as branches of one kernel the code between the
 // loops of two tiles took 5 us longer.
-enum PreKind { kPreStore, kPreF32, kPreRelu2, kPreSilu, kPreGelu, kPreSiluF32, kPreGeluF32, kPreHead };
+enum PreKind { kPreStore, kPreF32, kPreRelu2, kPreSilu, kPreGelu, kPreSiluF32, kPreGeluF32, kPreHead, kPreHeadOnce };
+// kPreHeadOnce: a head whose rows are one block: nobody else reads its weights, which are loaded with the non-temporal policy.  us with |
+// without it, 128256 x 4096 over 128 rows 181 | 197, 262144 x 1152 123 | 136; with a second block of rows the weights come from L2 and the
+// policy loses: 151936 x 2048 over 256 rows 194 | 183.
+constexpr bool pre_head(int kind) { return kind == kPreHead || kind == kPreHeadOnce; }
 constexpr bool pre_mul(int kind) { return kind == kPreSilu || kind == kPreGelu || kind == kPreSiluF32 || kind == kPreGeluF32; }
 
 // LORA: 0 no adapter, kLoraInPlace: its scale is a power of two near one (1 where alpha is the rank): B times the scale is exact, and
@@ -258,7 +262,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
     constexpr int Q = decltype(Qc)::value;
     wr[Q % S][ct] = __builtin_amdgcn_raw_buffer_load_b128(re, evoff + (uint32_t)(ct & 1) * 256u,
                                                          (wt0 + min(kt, ktiles - 1)) * 65536 + (ct >> 1) * 8192 + Q * 2048,
-                                                         RT == 4 ? kStreamOnce : 0);
+                                                         KIND == kPreHeadOnce ? kStreamOnce : 0);
   };
   // One slab (32 k) of k-tile kt: RT x 4 MFMAs, and with them the fragments of the next slab, the weights of the slab three
   // further on into the stage that the slab before has finished with, and half a step of activations for the buffer
@@ -441,7 +445,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
     };
     if constexpr (KIND == kPreRelu2) {
       stage_tile([](float v) { return fmaxf(v, 0.f) * fmaxf(v, 0.f); });
-    } else if constexpr (KIND == kPreHead && LORA == 0) {   // (the soft cap comes with dense heads only)
+    } else if constexpr (pre_head(KIND) && LORA == 0) {   // (the soft cap comes with dense heads only)
       if (h.softcap > 0.f) stage_tile([&](float v) { return soft_cap_fast(v, h.softcap); });
       else stage_tile([](float v) { return v; });
     } else {
@@ -449,7 +453,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
     }
   }
   __syncthreads();
-  wide_tile_out<ROWS, GROUPED, KIND == kPreHead, mul>(a, h, ntile, m0, rows_here);
+  wide_tile_out<ROWS, GROUPED, pre_head(KIND), mul>(a, h, ntile, m0, rows_here);
 }
 
 }  // namespace

@@ -823,8 +823,9 @@ int launch_qgemm_pre_rt(hipStream_t st, const QLArgs& a, const WideHead& h) {
 // is: us at 256 | 128 rows, 16384 x 14336 -> 4096: 1310 | 1431, 2048 x 4096 -> 28672: 377 | 366 (3.5 rounds), 8704 x 4096 ->
 // 4096: 261 | 222 (2.1 rounds), 16384 x 1152 -> 13824: 453 | 414, 8192 x 2048 -> 16384: 448 | 477.
 int launch_qgemm_pre(hipStream_t st, const QLArgs& a, const WideHead& h) {
-  // (a head over one block of 64 rows: the weights are streamed once either way; over 65 to 128 rows two such blocks would read them twice)
-  if (h.part && a.M <= 64 && a.lora_rank <= 0) return launch_qgemm_pre_as<4, false, kPreHead, 0>(st, a, h);
+  // (a head over one block of rows: two blocks of 64 would read the weights twice, 128 rows 251 us against 197)
+  if (h.part && a.M <= 128 && a.lora_rank <= 0)
+    return a.M <= 64 ? launch_qgemm_pre_as<4, false, kPreHeadOnce, 0>(st, a, h) : launch_qgemm_pre_as<8, false, kPreHeadOnce, 0>(st, a, h);
   const int64_t tn = cdiv(a.N, kWideCols);
   const double tall = (double)cdiv(cdiv(a.M, 256) * tn, 256) * (double)(a.K + 150);
   const double low = 0.5 * (double)cdiv(cdiv(a.M, 128) * tn, 256) * 1.09 * (double)a.K;
