@@ -74,6 +74,15 @@ __device__ __forceinline__ float code_level_imm(int qtype, int code) {
   return qtype == TNX_Q_NF4 ? nf4 : (float)(code - 8);
 }
 
+// gelu, tanh form, for a result that is rounded to bf16: 0.5 z (1 + tanh(w)) = z / (1 + exp(-2 w)), w = k0 (z + k1 z^3), with the hardware's
+// exponential and reciprocal.  Against 64 bits over z = -12 .. 12: relative error 1e-6 where 0.5 z (1 + tanhf(w)), whose sum cancels for
+// negative z, has 5e-4; the rounded result is the nearest bf16 value for 99.9 % of all z against 95.7 %.  A tanhf is some forty
+// instructions: 16384 rows x 1152 -> 13824 gated with an adapter 522 -> 459 us.
+__device__ __forceinline__ float gelu_tanh_fast(float z) {
+  const float c0 = -2.0f * 1.4426950408889634f * 0.7978845608028654f, c1 = c0 * 0.044715f;
+  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * __builtin_fmaf(z * z, c1, c0)));
+}
+
 // Scales stored per (k-tile of 128, column): S = max(2, 128 / group) slots of 128 / S k each
 // (a group of 128 or more repeats its scale), so that a lane's scales are one aligned 4- or 8-byte word.
 __host__ __device__ inline int scales_per_tile(int group) { return group >= 64 ? 2 : 128 / group; }

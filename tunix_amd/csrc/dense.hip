@@ -210,7 +210,7 @@ void dense_rows_kernel(const DenseArgs a) {
       if (col >= a.N / 2) continue;
       float v[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = (silu ? silu_f32(g[e]) : gelu_tanh_f32(g[e])) * u[e];
+      for (int e = 0; e < 4; ++e) v[e] = (silu ? silu_f32(g[e]) : gelu_tanh_fast(g[e])) * u[e];   // (rounded to bf16 below)
       const u32x2 pk = {pack2bf(v[0], v[1]), pack2bf(v[2], v[3])};
       uint16_t* y = reinterpret_cast<uint16_t*>(a.y);
       *reinterpret_cast<u32x2*>(y + (a.y_frag ? frag_index(row, col, a.ldy) : row * a.ldy + col)) = pk;

@@ -424,7 +424,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
       if constexpr (KIND == kPreSilu) return rbf(silu_bf16(rbf(z))) * rbf(u);
       else if constexpr (KIND == kPreGelu) return rbf(gelu_tanh_bf16(rbf(z))) * rbf(u);
       else if constexpr (KIND == kPreSiluF32) return z / (1.0f + expf(-z)) * u;
-      else return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))) * u;
+      else return gelu_tanh_fast(z) * u;
     };
 #pragma unroll
     for (int c = 0; c < CT / 2; ++c)

@@ -72,11 +72,7 @@ __device__ __forceinline__ float silu_bf16(float g) {
   float s = rbf(__builtin_amdgcn_rcpf(1.0f + __expf(-g)));
   return rbf(g * s);
 }
-__device__ __forceinline__ float gelu_tanh_bf16(float g) {
-  const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-  float inner = k0 * (g + k1 * g * g * g);
-  return rbf(0.5f * g * (1.0f + tanhf(inner)));
-}
+__device__ __forceinline__ float gelu_tanh_bf16(float g) { return rbf(gelu_tanh_fast(g)); }
 
 // Epilogue shared by the plain and the grouped kernel.  `out_row(r)` maps a tile row to the
 // output row (identity, or the route id in grouped mode).
