@@ -793,8 +793,8 @@ __device__ __forceinline__ float across_quarters(float x, F f) {
   return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 // c += a . b with the accumulator in place (the compiler's form copies O at every branch of the loop).  The wait states between a
-// vector write of an operand and the MFMA that reads it stand inside, under the MFMA before; what reads c next has to lie 18
-// instructions behind.
+// vector write of an operand and the MFMA that reads it stand inside, under the MFMA before; what reads c next has to lie eight
+// instruction slots behind (the compiler does not know that this is an MFMA: tests/test_mfma_wait_states.py checks the built code).
 __device__ __forceinline__ void mfma16_tied(u32x4 a, u32x4 b, f32x4& c) {
   asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
 }

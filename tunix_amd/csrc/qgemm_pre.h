@@ -39,11 +39,13 @@ constexpr size_t pre_smem_bytes() {
   return std::max<size_t>(4 * pre_step_bytes<RT>(), 16 * RT * (kWideCols + 8) * 2);
 }
 
-// (operands that loads have written: the wait for those is all it needs)
+// (operands that loads have written: the wait for those is all it needs.  The compiler does not know that this is an MFMA and inserts no wait
+// states between a copy of an operand and its use: that the built code has no such copy is checked in its listing,
+// tests/test_mfma_wait_states.py)
 __device__ __forceinline__ void mfma16_acc(u32x4 a, u32x4 b, f32x4& c) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
-// the same for operands that vector instructions may just have written: the wait states in front of it
+// the same for operands that vector instructions may just have written: the two wait states in front of it
 __device__ __forceinline__ void mfma16_acc_wait(u32x4 a, u32x4 b, f32x4& c) {
   asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
@@ -275,7 +277,10 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
         const int ct = (rt & 1) ? 3 - j : j;
-        mfma16_acc(wr[U % S][ct], xf[rt], acc[rt][ct]);
+        // (three waves per unit leave the weights of some slabs in accumulator registers, from which the compiler copies them right in front of
+        // their use; the stream of the weights, which bounds this form, hides the wait states)
+        if constexpr (RT == 4) mfma16_acc_wait(wr[U % S][ct], xf[rt], acc[rt][ct]);
+        else mfma16_acc(wr[U % S][ct], xf[rt], acc[rt][ct]);
         if (j == 1 && rt % HALF == HALF - 1) load_w(ic<UL>{}, rt / HALF, kt + ((U + 3) >> 2));
         if (j == 2 && (rt & 3) == 1) dma(src, ((U & 1) ? 0 : HALF) + (rt >> 2), dbuf);
         if (j == 3) xf[rt] = lds_ld128(xaddr[UN & 1] + (uint32_t)(rt * 2048) + ((UN >> 1) ? SB : 0u));
