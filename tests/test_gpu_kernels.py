@@ -254,6 +254,42 @@ def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank,
     assert (tf.float() - tm[:M].float()).abs().max().item() <= 2.0 ** -6 * tm.float().abs().max().item()
 
 
+@pytest.mark.parametrize("rows,copy,split", [(65536, False, 1), (65536, True, 1), (100, False, 1), (100, False, 2), (16, False, 1)])
+def test_silu_of_every_gate(gpu, rows, copy, split):
+  """Gates of every finite bf16 value (weights that pick one element of x), among them those whose sigmoid is not a normal fp32
+  number any more: x * sigmoid(x) with both factors' roundings, no result lost to zero before the exponential overflows."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  K, N = 512, 32
+  w = torch.zeros(K, N)
+  w[0, :N // 2] = 1.0
+  w[1, N // 2:] = 1.0
+  codes, scales = ops.quantize_pack(bf(w).to(gpu), 64, Q.NF4, True)
+  gates = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+  gates = gates[torch.isfinite(gates.float())]
+  if rows < 65536:                       # (the whole range in one large call, its ends and the far tail in small ones)
+    gates = torch.cat([gates[gates.float().abs() < 1e-30][:rows // 4], bf(torch.linspace(-92, -80, rows // 2)), gates[-(rows // 4):]])
+  g = gates.double()
+  x = torch.zeros(len(gates), K, dtype=torch.bfloat16)
+  x[:, 0], x[:, 1] = gates, 1.0
+  x = x.to(gpu)
+  M = len(gates)
+  y = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=gpu)
+  ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=Q.NF4, x=x, codes=codes, scales=scales, y=y, epilogue=L.TNX_EPI_SILU_MUL,
+                                    split_k=split, ws=torch.empty(split * M * N, device=gpu) if split > 1 else None,
+                                    w_expanded=ops.qw_expand(codes, scales, K, N, 64, Q.NF4) if copy else None))
+  torch.cuda.synchronize()
+  got = y.double().cpu()
+  assert (got == got[:, :1]).all()
+  want = g * torch.sigmoid(g)
+  # one ulp (2^-8 and 2^-8 of the two roundings, the exponential's error may move the first by one), the spacing of bf16 sigmoids
+  # below the normal range, and exp(-g) overflows from -88.72 on
+  bound = 2.0 ** -7 * 1.01 * want.abs() + g.abs() * 2.0 ** -133 + 2.0 ** -133
+  bound = torch.where(g < -88.7, want.abs() + 2.0 ** -133, bound)
+  bad = (got[:, 0] - want).abs() > bound
+  assert not bad.any(), [(float(a), float(b), float(c)) for a, b, c in zip(g[bad], got[bad, 0], want[bad])][:5]
+
+
 @pytest.mark.parametrize("M,K,N,split", [
     (128, 4096, 1024, 1),       # 32 k-tiles: two behind the whole turns of the weight ring
     (128, 4096, 1024, 4),       # eight of each split: two

@@ -67,9 +67,11 @@ struct WideHead {
 };
 
 __device__ __forceinline__ float silu_bf16(float g) {
-  // jax.nn.silu = x * sigmoid(x) as two bf16 HLO ops.  (The hardware reciprocal, one ulp of fp32 in front of a rounding
-  // to eight bits: an IEEE division is ten instructions more per element.)
-  float s = rbf(__builtin_amdgcn_rcpf(1.0f + __expf(-g)));
+  // jax.nn.silu = x * sigmoid(x) as two bf16 HLO ops.  g is a bf16 value, so the rounded sigmoid is one of 65536 results, and the hardware
+  // reciprocal gives each of them as an IEEE division does (compared over all of them), as long as it sees a normal number:
+  // hence the scaling, without which sigmoids below 2^-126 were lost to zero.  The division takes ten instructions more per element:
+  // 16384 x 4096 -> 28672 from the copy 2780 us against 2735, 1152 -> 13824 467 against 451.
+  float s = rbf(__builtin_amdgcn_rcpf((1.0f + __expf(-g)) * 0x1p-32f) * 0x1p-32f);
   return rbf(g * s);
 }
 __device__ __forceinline__ float gelu_tanh_bf16(float g) { return rbf(gelu_tanh_fast(g)); }
