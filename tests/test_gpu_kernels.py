@@ -196,14 +196,16 @@ def test_qlinear_lora_matches_oracle(gpu, M, K, N, group, qtype, r, split):
 
 
 @pytest.mark.parametrize("M,K,N,split,group,qtype,rank,nseg,epi", [
-    (1, 512, 128, 1, 64, Q.NF4, 64, 1, "store"),          # four k-tiles: the four-way form's first, half a turn
-    (3, 640, 208, 1, 32, Q.NF4, 32, 1, "residual"),       # a last column block of five tiles, four scales per k-tile
-    (8, 1408, 512, 3, 64, Q.INT4, 64, 3, "store"),        # eleven k-tiles in splits of 4, 4, 3; three adapter segments
-    (5, 1152, 768, 1, 128, Q.NF4, 64, -1, "silu"),        # nine k-tiles, gate | up with the next adapter's planes
-    (9, 1536, 256, 1, 64, Q.NF4, 0, 1, "f32"),            # twelve k-tiles: the two-way form's first
-    (16, 1664, 384, 1, 64, Q.INT4, 96, 1, "store"),       # thirteen; an adapter of more than 64 ranks
+    (1, 512, 128, 1, 64, Q.INT4, 64, 1, "store"),         # one row of int4: four k-tiles, half a turn of the four-way form
+    (3, 1280, 208, 1, 32, Q.NF4, 32, 1, "residual"),      # a last column block of five tiles, four scales per k-tile
+    (8, 3584, 512, 3, 64, Q.INT4, 64, 3, "store"),        # 28 k-tiles in splits of 10, 10, 8; three adapter segments
+    (4, 1792, 512, 2, 64, Q.NF4, 64, 1, "residual"),      # seven per split: two turns less one
+    (5, 2176, 768, 1, 128, Q.NF4, 64, -1, "silu"),        # 17 k-tiles, gate | up with the next adapter's planes
+    (7, 1024, 25600, 1, 64, Q.INT4, 64, -1, "gelu"),      # eight k-tiles, work-groups for most of the device
+    (9, 2048, 12288, 1, 64, Q.NF4, 0, 1, "f32"),          # 16 k-tiles: the two-way form's first
+    (16, 3712, 384, 2, 64, Q.INT4, 96, 1, "store"),       # 15 and 14; an adapter of more than 64 ranks
     (12, 4096, 320, 2, 256, Q.NF4, 64, -1, "gelu"),       # sixteen per split
-    (16, 2304, 640, 1, 64, Q.NF4, 64, -1, "silu"),        # eighteen
+    (16, 2304, 8192, 1, 64, Q.NF4, 64, -1, "silu"),       # eighteen
 ])
 def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank, nseg, epi):
   """At most 16 rows (activations straight from memory, sums of the k slices at the end) against the same rows

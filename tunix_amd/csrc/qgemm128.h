@@ -92,10 +92,9 @@ __device__ __forceinline__ void fill_level_table(uint32_t base, int tid) {
 
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 constexpr uint32_t kRowsActBytes = 72 * 2;            // per row of the activation staging
-constexpr uint32_t kRowsScratchBytes = 8 * 16 * 36 * 4;
 // The end of a work-group of eight waves over 16 * MT rows x 128 columns: wave wv holds in `out` the sums of row tiles
 // (wv / 4) * HM ... and column tiles 2 (wv % 4), + 1 (with one row tile waves 0-3 hold all of it).  act_lds: 16 MT rows of
-// kRowsActBytes; scr_lds (SCRATCH): kRowsScratchBytes; both idle for every wave by now.
+// kRowsActBytes; scr_lds (SCRATCH): 16 x 36 floats per wave; both idle for every wave by now.
 template <int MT, int NT, bool SCRATCH>
 __device__ __forceinline__ void quant_rows_out(const QLArgs& a, f32x4 (&out)[(MT + 1) / 2][NT], int64_t m0, int64_t ntile0, int wv,
                                                uint32_t act_lds, uint32_t scr_lds) {

@@ -8,13 +8,10 @@
 // at the end.  qgemm128_kernel shares the activations through LDS behind one barrier per k-tile: 24 KB per compute unit in flight and
 // its waves in step; here it is 64 to 96 KB, and every wave runs on as its own data arrives.
 // CW = 4: fewer sums to exchange, activations read four times over: for up to 8 rows.  CW = 2: twice over, for up to 16 rows and many
-// k-tiles.  With few k-tiles there is nothing to stream and the shared activations are the faster ones.  us, shared | CW = 4 | CW = 2
-// (4096 -> 6144 in 5 splits, 4096 -> 4096 in 8, 4096 -> 28672 gated, 14336 -> 4096 in 8; NF4, adapters of rank 64):
-//    3 rows   9.2 | 8.4 | 8.9    7.5 | 7.0 | 7.5    23.4 | 18.5 | 18.8    14.1 | 11.8 | 12.0
-//    8 rows   9.2 | 8.7          7.7 | 7.5          23.8 | 19.5           13.5 | 12.0
-//   16 rows   9.1 | 9.6 | 9.6    7.7 | 8.1 | 8.0    23.9 | 23.4 | 20.6    13.6 | 13.8 | 13.1
-// One or two k-tiles: 1152 -> 1536 in 8 splits, 8 rows 5.6 | 6.0.  CW = 1 pays a microsecond for the exchange of 64 KB; at 32 rows the
-// shared form wins everywhere.
+// k-tiles.  CW = 1 pays a microsecond for the exchange of 64 KB; at 32 rows the shared form wins everywhere.  Which calls come here:
+// few_shape in qlinear.hip.  The planes of a split are stored as they lie in the accumulators and without the non-temporal policy:
+// with it the pass that sums them waits longer than this one gains (14336 -> 4096 in 8 splits, 8 rows, with that pass: 16.1 us
+// against 17.0, 4096 -> 4096 in 8: 11.6 against 12.5).
 //
 // Included by qlinear.hip after qgemm128.h.
 #pragma once
@@ -25,8 +22,7 @@ constexpr uint32_t few_out_base(bool int4, int cw) {
   return int4 ? 65536u / (uint32_t)cw : kBigLutBase + (uint32_t)kBigLutBytes;
 }
 constexpr size_t few_smem_bytes(bool int4, int cw) {
-  static_assert(16 * kRowsActBytes <= kRowsScratchBytes, "one stage for either output");
-  return few_out_base(int4, cw) + kRowsScratchBytes;
+  return few_out_base(int4, cw) + 16 * kRowsActBytes;
 }
 
 template <int SPT, bool INT4, int CW>
@@ -238,7 +234,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     s.lora_scale = a.lora_scale;
     tile_lora<1, NT>(s, 0, ntile0, toff, out);
   }
-  quant_rows_out<1, NT, true>(a, out, 0, ntile0, wv, few_out_base(INT4, CW), few_out_base(INT4, CW));
+  quant_rows_out<1, NT, false>(a, out, 0, ntile0, wv, few_out_base(INT4, CW), 0u);
 }
 
 }  // namespace
