@@ -80,9 +80,9 @@ const char* tnx_last_error(void);
  * tnx_embed_rows, centred norms, a factor, an extra row and the depth average to tnx_residual_norm_desc, slopes and
  * chunks to tnx_sink_attn_desc, an ungated form and shared weights to tnx_gated_norm_desc, TNX_EPI_RELU2, and
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
- * tnx_moe_gmm_expanded and tnx_qw_expand_bank. */
+ * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows. */
 #define TNX_ABI_VERSION_MAJOR 6
-#define TNX_ABI_VERSION_MINOR 1
+#define TNX_ABI_VERSION_MINOR 2
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
 int tnx_version(void);
 
@@ -483,6 +483,9 @@ int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* h_desc);
 /* The same with a second copy of the weights: every expert's tnx_qw_expand output, behind each other
  * (tnx_qw_expanded_bytes(K, N) apart).  Calls with enough rows per expert read the copy, others the codes. */
 int tnx_moe_gmm_expanded(void* stream, const tnx_moe_gmm_desc* h_desc, const uint16_t* w_expanded);
+/* Rows per expert (n_routes / E) from which tnx_moe_gmm_expanded reads the copies of weights [K, N]; 0: it never does, and a
+ * caller has no use for them. */
+int64_t tnx_moe_expanded_rows(int64_t K, int64_t N, int qtype);
 /* out[m,:] = bf16( sum_j f32(topk_w[m,j]) * f32(y[m*k+j,:]) )  (qwen3/model.py:827-832). */
 int tnx_moe_combine(void* stream, const uint16_t* y, const uint16_t* topk_w, int64_t M, int k,
                     int64_t D, const uint16_t* residual, uint16_t* out);

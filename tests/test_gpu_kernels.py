@@ -2094,3 +2094,30 @@ def test_moe_from_the_experts_copies(gpu, M, counts_scale, qtype):
     ops.moe_gmm(d, copies)
     got.append(y)
   assert got[0].isfinite().all() and torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("qtype,K,N,rows", [(Q.INT4, 1024, 256, 144), (Q.INT4, 2048, 256, 176), (Q.INT4, 4096, 256, 304), (Q.INT4, 8320, 256, 0),
+                                            (Q.NF4, 1152, 512, 144), (Q.NF4, 4096, 256, 176), (Q.NF4, 8320, 256, 242), (Q.NF4, 1024, 384, 0)])
+def test_experts_copies_are_read_from_the_rows_on_that_pay(gpu, qtype, K, N, rows):
+  """Copies that hold NaN show which calls read them: those with tnx_moe_expanded_rows rows per expert or more, and none where it
+  says 0 (a contraction too long for int4, a width the many-row kernel does not take)."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  assert L.lib().tnx_moe_expanded_rows(K, N, qtype) == rows
+  E, group = 2, 64
+  g = torch.Generator(device=gpu).manual_seed(K)
+  packed = ops.quantize_pack((torch.randn(K, N, generator=g, device=gpu) * 0.05).bfloat16(), group, qtype)
+  codes, scales = (torch.cat([p, p]) for p in packed)
+  bank = torch.full((E, L.lib().tnx_qw_expanded_bytes(K, N) // 2), float("nan"), dtype=torch.bfloat16, device=gpu)
+  for avg in ((rows - 1, rows) if rows else (1024,)):
+    n = E * avg
+    x = torch.randn(n, K, generator=g, device=gpu).bfloat16()
+    offsets = torch.tensor([0, avg, n], dtype=torch.int32, device=gpu)
+    route = torch.arange(n, dtype=torch.int32, device=gpu)
+    y = torch.zeros(n, N, dtype=torch.bfloat16, device=gpu)
+    d = L.MoeGmmDesc()
+    d.n_routes, d.E, d.k, d.K, d.N, d.group, d.qtype, d.x, d.x_div = n, E, 1, K, N, group, qtype, x.data_ptr(), 1
+    d.codes, d.scales, d.offsets, d.sorted_route = codes.data_ptr(), scales.data_ptr(), offsets.data_ptr(), route.data_ptr()
+    d.epilogue, d.y = L.TNX_EPI_STORE, y.data_ptr()
+    ops.moe_gmm(d, bank)
+    assert bool(torch.isnan(y).all()) == (avg == rows) and bool(torch.isnan(y).any()) == (avg == rows), avg

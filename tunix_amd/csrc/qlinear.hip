@@ -874,10 +874,21 @@ int launch_qgemm_pre_grouped(hipStream_t st, const QLArgs& a) {
   const bool tall = (avg + 128.0) * (double)(a.K + 150) < (avg + 64.0) * 1.09 * (double)a.K;
   return tall ? launch_qgemm_pre_grouped_rt<16>(st, a) : launch_qgemm_pre_grouped_rt<8>(st, a);
 }
-// Rows per expert from which the experts' converted copies beat the codes (four times the bytes, no conversion in the loop):
-// Qwen3-30B-A3B shape, gate|up + down, us from codes | copies: 96 rows 125 + 97 | 152 + 100, 128: 193 + 120 | 191 + 121, 192: 254 +
-// 179 | 205 + 144, 447: 518 + 346 | 363 + 261, 1024: 1000 + 727 | 721 + 502.
-constexpr int64_t kMoeExpandedRows = 144;
+// Rows per expert from which the experts' converted copies beat the codes (four times the bytes, no conversion in the loop); 0: never.
+// The longer the contraction, the better the conversion hides under the MFMAs and the more the bytes of the copy cost, which few rows do
+// not repay; nf4, whose conversion goes through LDS, gains more than int4.  us from codes | copies at rows per expert (8 to 128
+// experts of random loads):
+//           K     int4                                                nf4
+//           768   144: 144 | 136   512: 380 | 275                     144: 155 | 133   512: 394 | 275    (128 experts, N = 2048)
+//           2048  144: 135 | 138   180: 144 | 136   512: 322 | 257    144: 147 | 133   512: 358 | 259    (64, N = 2048)
+//           4096  144: 693 | 967   256: 927 | 907   320: 1110 | 1040  180: 797 | 738   256: 1026 | 924   (128, N = 3072)
+//           6400  256: 250 | 281   448: 367 | 351                     180: 203 | 206   256: 283 | 281    (16, N = 4096)
+//           14336 256: 327 | 389   512: 509 | 558   1024: 900 | 930   256: 358 | 389   384: 409 | 396    (8, N = 4096)
+int64_t moe_expanded_rows(int64_t K, int64_t N, int qtype) {
+  if (N % kWideCols != 0 || cdiv(N, kWideCols) * (K / KTILE) * 65536 >= (int64_t)1 << 31) return 0;   // (32-bit offsets inside an expert's copy)
+  if (qtype != TNX_Q_INT4) return 144 + std::max<int64_t>(0, K - 2048) / 64;
+  return K <= 1024 ? 144 : K <= 8192 ? 176 + std::max<int64_t>(0, K - 2048) / 16 : 0;
+}
 
 template <int SPT>
 int launch_qgemm_wide(hipStream_t st, const QLArgs& a, const WideHead& h = kNoHead) {
@@ -1326,7 +1337,8 @@ static int moe_gmm(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_ex
       (uint64_t)(d->n_routes / d->x_div) * (uint64_t)d->K * 2 < 0xfffff000ull && d->n_routes % d->x_div == 0)
   {
     // from the experts' converted copies where those are worth four times the bytes
-    if (w_expanded && avg_rows >= kMoeExpandedRows && cdiv(d->N, kWideCols) * (d->K / KTILE) * 65536 < (int64_t)1 << 31) {
+    const int64_t from = moe_expanded_rows(d->K, d->N, d->qtype);
+    if (w_expanded && from > 0 && avg_rows >= from) {
       a.w_pre = w_expanded;
       return launch_qgemm_pre_grouped(st, a);
     }
@@ -1345,6 +1357,10 @@ static int moe_gmm(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_ex
 }
 
 extern "C" int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* d) { return moe_gmm(stream, d, nullptr); }
+
+extern "C" int64_t tnx_moe_expanded_rows(int64_t K, int64_t N, int qtype) {
+  return K > 0 && N > 0 && K % KTILE == 0 ? moe_expanded_rows(K, N, qtype) : 0;
+}
 
 extern "C" int tnx_moe_gmm_expanded(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_expanded) {
   TNX_REQUIRE(w_expanded && ((uintptr_t)w_expanded & 15) == 0, "moe_gmm_expanded: the copies must be there and 16-byte aligned");
