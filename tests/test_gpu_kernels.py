@@ -2121,3 +2121,30 @@ def test_experts_copies_are_read_from_the_rows_on_that_pay(gpu, qtype, K, N, row
     d.epilogue, d.y = L.TNX_EPI_STORE, y.data_ptr()
     ops.moe_gmm(d, bank)
     assert bool(torch.isnan(y).all()) == (avg == rows) and bool(torch.isnan(y).any()) == (avg == rows), avg
+
+
+@pytest.mark.parametrize("D,F,wanted", [(384, 256, (True, False)), (384, 384, (True, False)), (128, 384, (True, False)), (256, 256, (True, True))])
+def test_expert_bank_copies_what_calls_read(gpu, D, F, wanted):
+  """A bank copies, counts and refreshes the weights whose copy some call reads, and no others."""
+  import types
+
+  from tunix_amd import ops
+  from tunix_amd.model import ExpertBank
+  cfg = types.SimpleNamespace(group=64, qtype=Q.INT4, int4_bound=7.0)
+  E = 3
+
+  def weights(seed):
+    return {"p.e_gate": rnd((E, D, F), seed), "p.e_up": rnd((E, D, F), seed + 1), "p.e_down": rnd((E, F, D), seed + 2),
+            "p.router": rnd((D, E), seed + 3)}
+  bank = ExpertBank(cfg, weights(1), "p.", gpu)
+  assert bank.wants_expansion() == wanted
+  bank.expand()
+  for seed in (1, 11):
+    if seed > 1:
+      bank.load_base(weights(seed))
+    for copy, want, codes, scales, K, N in ((bank.gu_expanded, wanted[0], bank.gu_codes, bank.gu_scales, D, 2 * F),
+                                            (bank.dn_expanded, wanted[1], bank.dn_codes, bank.dn_scales, F, D)):
+      assert (copy is not None) == want
+      if want:
+        assert torch.equal(copy, ops.qw_expand_bank(codes, scales, E, K, N, 64, Q.INT4))
+  assert bank.expanded_bytes() == 2 * sum(c.numel() for c in (bank.gu_expanded, bank.dn_expanded) if c is not None)

@@ -201,23 +201,31 @@ class ExpertBank:
       self.dn_codes[e * cb2 // 4:(e + 1) * cb2 // 4].copy_(c)
       self.dn_scales[e * sb2 // 2:(e + 1) * sb2 // 2].copy_(s)
     self.router_t.copy_(weights[prefix + "router"].to(device, torch.bfloat16).t())
-    if self.gu_expanded is not None:
+    if self.gu_expanded is not None or self.dn_expanded is not None:
       self._fill_expanded()
 
+  def wants_expansion(self) -> tuple[bool, bool]:
+    """Whether any call reads a copy of gate|up and of down: not of a width or a contraction that the many-row kernel leaves to
+    the codes."""
+    rows, qtype = L.lib().tnx_moe_expanded_rows, self.cfg.qtype
+    return rows(self.D, 2 * self.F, qtype) > 0, rows(self.F, self.D, qtype) > 0
+
   def expanded_bytes(self) -> int:
-    size = L.lib().tnx_qw_expanded_bytes
-    return self.E * (int(size(self.D, 2 * self.F)) + int(size(self.F, self.D)))
+    size, (gu, dn) = L.lib().tnx_qw_expanded_bytes, self.wants_expansion()
+    return self.E * ((int(size(self.D, 2 * self.F)) if gu else 0) + (int(size(self.F, self.D)) if dn else 0))
 
   def expand(self):
     """The same second copy as `FusedLinear.expand`, of every expert: calls with some hundred rows per expert are bound
     by the conversion of codes in their loop."""
-    if self.gu_expanded is None:
+    if self.gu_expanded is None and self.dn_expanded is None:
       self._fill_expanded()
 
   def _fill_expanded(self):
-    cfg = self.cfg
-    self.gu_expanded = ops.qw_expand_bank(self.gu_codes, self.gu_scales, self.E, self.D, 2 * self.F, cfg.group, cfg.qtype, self.gu_expanded)
-    self.dn_expanded = ops.qw_expand_bank(self.dn_codes, self.dn_scales, self.E, self.F, self.D, cfg.group, cfg.qtype, self.dn_expanded)
+    cfg, (gu, dn) = self.cfg, self.wants_expansion()
+    if gu:
+      self.gu_expanded = ops.qw_expand_bank(self.gu_codes, self.gu_scales, self.E, self.D, 2 * self.F, cfg.group, cfg.qtype, self.gu_expanded)
+    if dn:
+      self.dn_expanded = ops.qw_expand_bank(self.dn_codes, self.dn_scales, self.E, self.F, self.D, cfg.group, cfg.qtype, self.dn_expanded)
 
 
 class QLoRAModel:
