@@ -2034,11 +2034,15 @@ def test_many_rows_adapter(gpu, M, K, widths, rank, scale):
     ti, bi = t[:, i * rank:(i + 1) * rank].double(), b[a0:a1].double().T
     want[:, a0:a1] += scale * (ti @ bi)
     size[:, a0:a1] += scale * (ti.abs() @ bi.abs())
-  y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=gpu)
-  ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=Q.NF4, x=x, codes=codes, scales=scales, y=y, lora_rank=rank, lora_nseg=3,
-                                    lora_seg_end=ends, lora_seg_toff=[0, rank, 2 * rank], t=t, t_ld=3 * rank, lora_b=b, lora_scale=scale,
-                                    w_expanded=ops.qw_expand(codes, scales, K, N, 64, Q.NF4)))
-  assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (K + rank) * 2.0 ** -24 * size).all()
+  got = []
+  for copy in (ops.qw_expand(codes, scales, K, N, 64, Q.NF4), None):
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=gpu)
+    ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=Q.NF4, x=x, codes=codes, scales=scales, y=y, lora_rank=rank, lora_nseg=3,
+                                      lora_seg_end=ends, lora_seg_toff=[0, rank, 2 * rank], t=t, t_ld=3 * rank, lora_b=b, lora_scale=scale,
+                                      w_expanded=copy))
+    assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (K + rank) * 2.0 ** -24 * size).all()
+    got.append(y)
+  assert torch.equal(got[0], got[1])   # from the copy and from the codes: the same sums
 
 
 @pytest.mark.parametrize("K,counts", [(128, (70, 0, 129, 40)), (4096, (1300, 1255))])
