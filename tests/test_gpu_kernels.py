@@ -2045,12 +2045,13 @@ def test_many_rows_adapter(gpu, M, K, widths, rank, scale):
   assert torch.equal(got[0], got[1])   # from the copy and from the codes: the same sums
 
 
-@pytest.mark.parametrize("K,counts", [(128, (70, 0, 129, 40)), (4096, (1300, 1255))])
-def test_many_rows_experts_from_expanded_copies(gpu, K, counts):
-  """Row blocks of 128 and of 256 routes: experts without rows, blocks that end inside a tile."""
+@pytest.mark.parametrize("K,N,counts", [(128, 272, (70, 0, 129, 40)), (4096, 272, (1300, 1255)), (4096, 3344, (1300, 1255)), (128, 528, (2200, 0, 1030, 8))])
+def test_many_rows_experts_from_expanded_copies(gpu, K, N, counts):
+  """Row blocks of 128 and (4096 -> 3344) of 256 routes: experts without rows, blocks that end inside a tile, experts of several groups of
+  1024 rows."""
   from tunix_amd import _lib as L
   from tunix_amd import ops
-  E, N, n = len(counts), 272, sum(counts)
+  E, n = len(counts), sum(counts)
   g = torch.Generator(device=gpu).manual_seed(n)
   x = torch.randn(n, K, generator=g, device=gpu).bfloat16()
   w = (torch.randn(E, N, K, generator=g, device=gpu) * K ** -0.5).bfloat16()
@@ -2069,14 +2070,14 @@ def test_many_rows_experts_from_expanded_copies(gpu, K, counts):
     assert ((y[route[a0:a1].long()].double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()
 
 
-@pytest.mark.parametrize("M,counts_scale", [(36, 1), (320, 1), (333, 2)])
+@pytest.mark.parametrize("M,counts_scale,K,N", [(36, 1, 256, 512), (320, 1, 256, 512), (333, 2, 256, 512), (2601, 1, 4096, 2048)])
 @pytest.mark.parametrize("qtype", [Q.INT4, Q.NF4])
-def test_moe_from_the_experts_copies(gpu, M, counts_scale, qtype):
+def test_moe_from_the_experts_copies(gpu, M, counts_scale, K, N, qtype):
   """Experts read from their converted copies give the bits that they give from the codes, on both sides of the line between
-  the two, with experts of very different sizes."""
+  the two, with experts of very different sizes, in tiles of 128 and (2601 rows) of 256 rows."""
   from tunix_amd import _lib as L
   from tunix_amd import ops
-  E, k, K, N, group = 4, 2, 256, 512, 64
+  E, k, group = 4, 2, 64
   g = torch.Generator(device=gpu).manual_seed(M)
   w = (torch.randn(E, K, N, generator=g, device=gpu) * 0.05).bfloat16()
   packed = [ops.quantize_pack(e, group, qtype, True) for e in w]

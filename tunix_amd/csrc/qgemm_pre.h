@@ -90,8 +90,19 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   const int lm = lane & 15, lq = lane >> 4;
   const int tiles_m = (int)((a.M + ROWS - 1) / ROWS), tiles_n = (int)((a.N + kWideCols - 1) / kWideCols);
   int mtile, ntile, expert = 0, m_end = 0;
+  // tile number `tile` of row blocks x column tiles: in groups of 1024 rows, inside a group column tile by column tile, so that an XCD works on
+  // about 1024 rows x 8 column tiles at a time (2048 or 4096 rows: the same at 16 row tiles, 3 to 20 % slower at 8).  An expert of many rows the
+  // same: with all its row blocks per column tile, 8 experts of 8000 rows x 4096 -> 4096 took 2340 us against 1710 (256-row tiles), 2395 against
+  // 1760 (128).
+  auto tile_in = [&](int tile, int row_blocks) {
+    constexpr int GR = 1024 / ROWS;
+    const int per_group = GR * tiles_n, g = tile / per_group, r = tile % per_group;
+    const int gm = min(GR, row_blocks - g * GR);
+    mtile = g * GR + r % gm;
+    ntile = r / gm;
+  };
   if constexpr (GROUPED) {
-    // tiles in the order (expert, column tile, row block of the expert); every wave finds its own
+    // tiles expert by expert; every wave finds its own
     auto blocks_of = [&](int e) { return e < a.n_experts ? (a.offsets[e + 1] - a.offsets[e] + ROWS - 1) / ROWS : 0; };
     int total = 0;
     for (int base = 0; base < a.n_experts; base += 64) {
@@ -122,18 +133,10 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
       carry += __shfl(incl, 63, 64);
     }
     expert = __builtin_amdgcn_readfirstlane(found_e);
-    ntile = __builtin_amdgcn_readfirstlane(found_at / found_nb);
-    mtile = __builtin_amdgcn_readfirstlane(found_at % found_nb);
+    tile_in(__builtin_amdgcn_readfirstlane(found_at), __builtin_amdgcn_readfirstlane(found_nb));
     m_end = a.offsets[expert + 1];
   } else {
-    // tiles in groups of 1024 rows, inside a group column tile by column tile: an XCD works on about 1024 rows x 8 column
-    // tiles at a time (2048 or 4096 rows: the same at 16 row tiles, 3 to 20 % slower at 8)
-    constexpr int GR = 1024 / ROWS;
-    const int tile = xcd_tile((int)blockIdx.x, tiles_m * tiles_n), per_group = GR * tiles_n;
-    const int g = tile / per_group, r = tile % per_group;
-    const int gm = min(GR, tiles_m - g * GR);
-    mtile = g * GR + r % gm;
-    ntile = r / gm;
+    tile_in(xcd_tile((int)blockIdx.x, tiles_m * tiles_n), tiles_m);
   }
   // first row of the tile (GROUPED: first position in the sorted route list)
   const int64_t m0 = GROUPED ? (int64_t)a.offsets[expert] + (int64_t)mtile * ROWS : (int64_t)mtile * ROWS;

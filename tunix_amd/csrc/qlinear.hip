@@ -3,6 +3,8 @@
 // in gemm_tile.h.
 #include <string.h>
 
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "gemm_tile.h"
@@ -868,10 +870,18 @@ int launch_qgemm_pre_grouped_rt(hipStream_t st, const QLArgs& a) {
   TNX_REQUIRE(false, "experts over many rows: bad epilogue %d", a.epilogue);
 }
 
+// As launch_qgemm_pre, by rounds of the device, for experts of random loads: up to half a block of an expert's last one is empty (a
+// quarter counted for the low tiles: where their last round may yet be missing, they stay).  A tall tile costs some 400 k's worth besides its
+// contraction, so that it wins where a round is saved or K is long.  us at 256 | 128 rows: 8 experts of 512 rows x 12288 -> 2048: 244 | 320,
+// 4 x 512 x 8192 -> 4096: 160 | 206, 8 x 6000 x 8192 -> 2048: 1225 | 1410; 4 x 1000 x 8192 -> 4096: 328 | 278, 8 x 512 x 4096 -> 4096: 183 | 163,
+// 4 x 1300 x 4096 -> 4096: 206 | 144, 64 x 512 x 2048 -> 1536: 244 | 216 (below 4096 the low ones everywhere).
 int launch_qgemm_pre_grouped(hipStream_t st, const QLArgs& a) {
-  // as launch_qgemm_pre, with half a row block per expert left empty on average
-  const double avg = (double)a.M / (double)a.n_experts;
-  const bool tall = (avg + 128.0) * (double)(a.K + 150) < (avg + 64.0) * 1.09 * (double)a.K;
+  const double avg = (double)a.M / (double)a.n_experts, tn = (double)cdiv(a.N, kWideCols);
+  auto rounds = [&](double rows, double part) {
+    const double blocks = a.n_experts > 1 ? a.n_experts * (avg / rows + part) : std::ceil(avg / rows);
+    return std::ceil(blocks * tn / 256.0);
+  };
+  const bool tall = a.K >= 4096 && rounds(256.0, 0.5) * (double)(a.K + 400) < 0.5 * rounds(128.0, 0.25) * 1.15 * (double)a.K;
   return tall ? launch_qgemm_pre_grouped_rt<16>(st, a) : launch_qgemm_pre_grouped_rt<8>(st, a);
 }
 // Rows per expert from which the experts' converted copies beat the codes (four times the bytes, no conversion in the loop); 0: never.
