@@ -854,6 +854,9 @@ int launch_qgemm_pre(hipStream_t st, const QLArgs& a, const WideHead& h) {
   const int64_t tn = cdiv(a.N, kWideCols);
   const double tall = (double)cdiv(cdiv(a.M, 256) * tn, 256) * (double)(a.K + 150);
   const double low = 0.5 * (double)cdiv(cdiv(a.M, 128) * tn, 256) * 1.09 * (double)a.K;
+  // (the noise of a draw is vector work, which two work-groups per unit put under each other's loads: 2048 x 151936 over 400 rows 634 us at 256 rows
+  // of a tile, 468 at 128; 65536 x 2048 over 256 rows 144 | 130, over 160, more than a third of the second 128 missing, 108 | 137)
+  if (h.part_draw && a.M > 160) return launch_qgemm_pre_rt<8>(st, a, h);
   return tall < low ? launch_qgemm_pre_rt<16>(st, a, h) : launch_qgemm_pre_rt<8>(st, a, h);
 }
 

@@ -40,51 +40,65 @@ __device__ __forceinline__ void wide_tile_out(const QLArgs& a, const WideHead& h
   }
   if constexpr (HEAD) {
     // The whole-vocabulary draw: per column the logit plus the Gumbel noise of element row * N + col of
-    // rows_total * N; a block's best (first among equals), its id and its logit go to part_draw.  Sixteen lanes share a (row, half), one
-    // 16-byte chunk each: the noise is a hundred instructions per element, and with a thread per (row, half), as the statistics below
-    // are formed, a tile of 16 rows had 32 threads at it: 128256 columns x 4096, 16 rows 214 -> 172 us.
+    // rows_total * N; a block's best (first among equals), its id and its logit go to part_draw.  The noise is a hundred instructions per
+    // element, so the tile's (row, half) are spread over all threads: sixteen lanes share one, a 16-byte chunk each, or, where the rows alone
+    // occupy the threads and no merging between lanes is needed, two or one take its chunks in turn.  us, one lane | sixteen | as chosen, 70000
+    // columns x 512: 16 rows 109 | 39 | 39, 128 rows 92 | 100 | 92; 262144 x 1152: 16 rows 226 | 125 | 124, 256 rows 397 | 398 | 365.
     if (h.part_draw != nullptr) {
       uint32_t ks0 = 0u, ks1 = (uint32_t)(*h.step_ptr);
       threefry2x32(h.key0, h.key1, ks0, ks1);   // fold_in(key, step)
       const uint64_t total = (uint64_t)h.rows_total * (uint64_t)a.N;
-      for (int p = tid >> 4; p < 2 * rows_here; p += 16) {
-        const int row = p >> 1, hf = p & 1;
-        const int64_t pb = (int64_t)ntile * 2 + hf, grow = m0 + row, c0 = pb * 128 + (tid & 15) * 8;
-        if (pb >= h.nvb) continue;   // (the same for the sixteen lanes)
-        const u32x4 v = lds_ld128(stage + (uint32_t)((row * sld + hf * 128 + (tid & 15) * 8) * 2));
-        float gv = -__builtin_inff(), gl = gv;
-        int gi = 0x7fffffff;
+      auto draw = [&](auto lanes_c) {
+        constexpr int LANES = decltype(lanes_c)::value, STEP = 256 / LANES;
+        const int first = tid % LANES;
+        for (int p = tid / LANES; p < 2 * rows_here; p += STEP) {
+          const int row = p >> 1, hf = p & 1;
+          const int64_t pb = (int64_t)ntile * 2 + hf, grow = m0 + row;
+          if (pb >= h.nvb) continue;   // (the same for the lanes of a row half)
+          float gv = -__builtin_inff(), gl = gv;
+          int gi = 0x7fffffff;
+#pragma unroll 1
+          for (int c = 0; c < 16 / LANES; ++c) {   // (columns ascend: the first among equals of a lane stays)
+            const int64_t c0 = pb * 128 + (c * LANES + first) * 8;
+            const u32x4 v = lds_ld128(stage + (uint32_t)((row * sld + hf * 128 + (c * LANES + first) * 8) * 2));
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int64_t col = c0 + q;
-          if (col < a.N) {
-            const float raw = (q & 1) ? bfhi(v[q >> 1]) : bflo(v[q >> 1]);
-            const float l = __fdiv_rn(raw, h.temperature);
-            const float n = l + gumbel_from_bits(random_bits(ks0, ks1, (uint64_t)grow * (uint64_t)a.N + (uint64_t)col, total, h.variant));
-            if (n > gv) {
-              gv = n;
-              gi = (int)col;
-              gl = l;
+            for (int q = 0; q < 8; ++q) {
+              const int64_t col = c0 + q;
+              if (col < a.N) {
+                const float raw = (q & 1) ? bfhi(v[q >> 1]) : bflo(v[q >> 1]);
+                const float l = __fdiv_rn(raw, h.temperature);
+                const float n = l + gumbel_from_bits(random_bits(ks0, ks1, (uint64_t)grow * (uint64_t)a.N + (uint64_t)col, total, h.variant));
+                if (n > gv) {
+                  gv = n;
+                  gi = (int)col;
+                  gl = l;
+                }
+              }
             }
           }
-        }
 #pragma unroll
-        for (int o = 8; o > 0; o >>= 1) {
-          const float ov = __shfl_xor(gv, o, 64), ol = __shfl_xor(gl, o, 64);
-          const int oi = __shfl_xor(gi, o, 64);
-          if (ov > gv || (ov == gv && oi < gi)) {
-            gv = ov;
-            gi = oi;
-            gl = ol;
+          for (int o = LANES / 2; o > 0; o >>= 1) {
+            const float ov = __shfl_xor(gv, o, 64), ol = __shfl_xor(gl, o, 64);
+            const int oi = __shfl_xor(gi, o, 64);
+            if (ov > gv || (ov == gv && oi < gi)) {
+              gv = ov;
+              gi = oi;
+              gl = ol;
+            }
+          }
+          if (first == 0) {
+            float* q3 = h.part_draw + (grow * h.nvb + pb) * 3;
+            q3[0] = gv;
+            q3[1] = __int_as_float(gi);
+            q3[2] = gl;
           }
         }
-        if ((tid & 15) == 0) {
-          float* q3 = h.part_draw + (grow * h.nvb + pb) * 3;
-          q3[0] = gv;
-          q3[1] = __int_as_float(gi);
-          q3[2] = gl;
-        }
-      }
+      };
+      // (passes of 256 threads, the last one at least seven eighths full)
+      const int rest = rows_here & 127;
+      if (rows_here >= 112 && (rest == 0 || rest >= 112)) draw(std::integral_constant<int, 1>{});
+      else if (rows_here >= 56 && rows_here <= 64) draw(std::integral_constant<int, 2>{});
+      else draw(std::integral_constant<int, 16>{});
     }
     // lm_head: thread (row % 128, half) reduces the row's 128 staged logits of column block
     // 2 * ntile + half to (max, first arg-max, sum of exp(l - max), logit of the row's target)
