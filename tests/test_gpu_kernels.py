@@ -1865,13 +1865,15 @@ def test_rope_row_kernel_equals_the_per_head_kernel(gpu, family, dh, Hq, Hkv):
 @pytest.mark.parametrize("family,norm,Hq,Hkv,dh", [("qwen3", "qwen3", 32, 4, 128), ("gemma3", "gemma3", 4, 1, 256), ("llama3", "llama3", 3, 1, 16),
                                                    ("qwen3", "gemma3", 5, 2, 64), ("llama3", "qwen3", 2, 1, 512)])
 def test_normed_heads_over_many_rows_equal_the_per_head_kernel(gpu, family, norm, Hq, Hkv, dh):
-  """512 rows in one call (a head's squares summed over its own lanes) against 128 per call (over a work-group):
-  the fp32 sum runs in another order, so a rounded result may be the neighbouring bf16 value; columns that
+  """The fewest rows of the row kernel in one call (a head's squares summed over its own lanes) against a quarter per call (over a
+  work-group): the fp32 sum runs in another order, so a rounded result may be the neighbouring bf16 value; columns that
   wrap around the cache included."""
   from tunix_amd import _lib as L
   from tunix_amd import ops
   from tunix_amd.model import _NORM, _ROPE, rope_timescale
-  B, T, S, col = 4, 128, 132, 9
+  B = 4
+  T = (384 + 5120 // (Hq + 2 * Hkv) + B - 1) // B
+  S, col = T + 4, 9
   qkv = bf(rnd((B, T, (Hq + 2 * Hkv) * dh), 121)).to(gpu)
   pos = torch.randint(0, 2000, (B, col + T), generator=torch.Generator().manual_seed(122), dtype=torch.int32).to(gpu)
   ts = torch.from_numpy(rope_timescale(dh, 1e6)).to(gpu)

@@ -704,7 +704,12 @@ extern "C" int tnx_qknorm_rope_kvwrite(void* stream, const tnx_rope_desc* d) {
   const bool aligned = (((uintptr_t)d->qkv | (uintptr_t)d->q_out | (uintptr_t)d->kcache | (uintptr_t)d->vcache) & 15) == 0 &&
                        (!norm || (((uintptr_t)d->q_norm_w | (uintptr_t)d->k_norm_w) & 15) == 0);
   TNX_REQUIRE(d->B * d->T < (int64_t)1 << 31, "rope: too many rows");
-  if (!d->qkv_ws && d->B * d->T >= 256 && d->dh % 16 == 0 && 256 % chunks == 0 && aligned) {
+  // Normed heads: the per-head kernel has a work-group for every head, the row kernel one for a row, whose chain (sines, barrier, loads, the
+  // sum over lanes) is the longer; the fewer heads, the more rows it takes until the per-head one has enough of them.  us, per head | per row,
+  // 256, 512, 1024 rows: 32 + 2 x 4 heads of 128 6.3 | 8.6, 9.5 | 9.4, 16.1 | 12.0; 8 + 2 x 2 of 64 3.6 | 5.1, 4.4 | 5.4, 6.1 | 5.7;
+  // 4 + 2 x 1 of 256 3.7 | 5.5, 4.7 | 6.2, 6.7 | 6.6; 64 + 2 x 8 of 128 9.9 | 11.5, 16.1 | 13.3, 29.1 | 18.2.
+  const int64_t from = norm ? 384 + 5120 / (d->Hq + 2 * d->Hkv > 0 ? d->Hq + 2 * d->Hkv : 1) : 256;
+  if (!d->qkv_ws && d->B * d->T >= from && d->dh % 16 == 0 && 256 % chunks == 0 && aligned) {
     if (norm) hipLaunchKernelGGL(rope_rows_kernel<true>, dim3((unsigned)(d->B * d->T)), dim3(256), 0, as_stream(stream), a);
     else hipLaunchKernelGGL(rope_rows_kernel<false>, dim3((unsigned)(d->B * d->T)), dim3(256), 0, as_stream(stream), a);
     TNX_CHECK_LAUNCH("qknorm_rope_kvwrite (rows)");
