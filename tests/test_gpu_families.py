@@ -60,6 +60,22 @@ def test_gemma3_sliding_window_greedy(gpu):
   _greedy_case(cfg, gpu, B=4, P=24, T=24, seed=32, lp_tol=4e-2)
 
 
+@pytest.mark.parametrize("kw,linears,experts", [({}, True, True), (dict(expand_many_rows=True), True, False), (dict(expand_many_rows=False), False, False),
+                                                (dict(expand_many_rows=False, expand_experts=True), False, True),
+                                                (dict(expand_many_rows=True, expand_experts=True), True, True), (dict(expand_experts=False), True, False)])
+def test_copies_of_linears_and_experts_are_asked_for_apart(gpu, kw, linears, experts):
+  """expand_many_rows speaks for the dense linears, expand_experts for the experts, whose copies are several times as large; by default
+  both are kept where they fit."""
+  from tunix_amd import config, dummy_model
+  from tunix_amd.model import QLoRAModel
+  cfg = config.qwen3_30b_a3b(num_layers=1, vocab_size=512, embed_dim=256, hidden_dim=256, num_heads=4, num_kv_heads=2, head_dim=64,
+                             num_experts=4, num_experts_per_tok=2)
+  model = QLoRAModel(cfg, dummy_model.create_dummy_weights(cfg, seed=5), gpu, **kw)
+  assert [f.expanded is not None for f in model._linears()] == [linears] * len(model._linears())
+  bank = model.layers[0]["experts"]
+  assert (bank.gu_expanded is not None, bank.dn_expanded is not None) == (experts, experts)
+
+
 def test_qwen3_moe_greedy(gpu):
   from tunix_amd import config
   cfg = config.qwen3_30b_a3b(num_layers=2, vocab_size=8192, embed_dim=512, hidden_dim=256, num_heads=8,

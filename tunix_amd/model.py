@@ -231,10 +231,13 @@ class ExpertBank:
 class QLoRAModel:
   """Packed weights of one model on one GPU."""
 
-  def __init__(self, cfg: ModelConfig, weights: dict, device="cuda", expand_many_rows: bool | None = None):
+  def __init__(self, cfg: ModelConfig, weights: dict, device="cuda", expand_many_rows: bool | None = None,
+               expand_experts: bool | None = None):
     """expand_many_rows: keep the converted second copy of every dense quantised linear
-    (`FusedLinear.expand`) and of the experts for the calls with many rows.  None (default): when the copies take
-    less than a quarter of the device memory that is free once the model is built (experts: together with the others)."""
+    (`FusedLinear.expand`) for the calls with many rows.  None (default): when the copies take
+    less than a quarter of the device memory that is free once the model is built.
+    expand_experts: the same for the routed experts (`ExpertBank.expand`), four times the bytes of their codes.  None (default): with
+    expand_many_rows at its default too, when all copies together take less than that quarter; otherwise no."""
     L.lib()  # fail loudly when the HIP library is missing
     self.cfg = cfg
     self.device = torch.device(device)
@@ -279,12 +282,12 @@ class QLoRAModel:
       if head_need >= (1 << 31):
         head_need = 0
     banks = [ly["experts"] for ly in self.layers if "experts" in ly]
-    expand_experts = expand_many_rows
     if expand_many_rows is None:
       need = head_need + sum(f.expanded_bytes() for f in self._linears() if f.wants_expansion())
       room = torch.cuda.mem_get_info(dev)[0] // 4
       expand_many_rows = need <= room
-      expand_experts = need + sum(bank.expanded_bytes() for bank in banks) <= room
+      if expand_experts is None:
+        expand_experts = need + sum(bank.expanded_bytes() for bank in banks) <= room
     if expand_experts:
       for bank in banks:
         bank.expand()
