@@ -266,7 +266,7 @@ def write_traffic_profile(fetch_csv, write_csv):
 
 # The same for the many-row kernel on the standalone log-probability pass (one launch = 16384 rows
 # x 128256 columns): counter runs of `bench.py --fused-logps`.
-FUSED_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "qgemm_wide_kernel_fused_logps_131072rows.json")
+FUSED_TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "qgemm_pre_kernel_fused_logps_131072rows.json")
 FUSED_KERNEL_SOURCES = ("csrc/qgemm_pre.h", "csrc/wide_out.h", "csrc/gemm_tile.h", "csrc/common.h", "csrc/qlinear.hip",
                         "csrc/lmhead.hip")
 
@@ -1285,7 +1285,7 @@ def main():
   ap.add_argument("--summarize-trace", metavar="CSV", default=None,
                   help="no GPU work: tabulate one decode step of a rocprofv3 kernel-trace csv of this script")
   ap.add_argument("--write-fused-traffic-profile", nargs=2, metavar=("FETCH_CSV", "WRITE_CSV"), default=None,
-                  help="rebuild profiles/qgemm_wide_kernel_fused_logps_131072rows.json from the counter csv files "
+                  help="rebuild profiles/qgemm_pre_kernel_fused_logps_131072rows.json from the counter csv files "
                        "of two `rocprofv3 --pmc FETCH_SIZE | WRITE_SIZE -- python3 bench.py --fused-logps` runs")
   ap.add_argument("--write-traffic-profile", nargs=2, metavar=("FETCH_CSV", "WRITE_CSV"), default=None,
                   help="no GPU work: rebuild profiles/qgemm128_kernel_llama8b_decode_b128.json from the counter csvs "

@@ -1,7 +1,7 @@
 // Linears with dense weights (bf16 or fp32) for decoders whose weights are not quantised.
 //
 // bf16: the weights live in HBM once, in the fragment order of tnx_dense_expand.  Calls with many
-// rows take the 128 x 256 kernel of qgemm_wide.h; calls with few rows take dense_rows_kernel below,
+// rows take the kernel of qgemm_pre.h; calls with few rows take dense_rows_kernel below,
 // which streams the same copy.  fp32: a plain tiled kernel in true 32-bit arithmetic.
 //
 // Two forms run several weights of one shape in a launch: a batch (every row through every weight, e.g.
@@ -359,7 +359,7 @@ extern "C" int tnx_dense_linear(void* stream, const tnx_dense_desc* d) {
   const bool x32 = x_rows * (d->x_frag ? d->K : d->ldx) < (int64_t)1 << 31;
   const bool offsets32 = cdiv(d->N, 256) * (d->K / kDenseKT) * 65536 < (int64_t)1 << 31;
   if (experts) {
-    // rows per block: as many as an expert gets on average, and the 128 x 256 kernel from about 24 on (a
+    // rows per block: as many as an expert gets on average, and the many-row kernel from about 24 on (a
     // second block of an expert streams its weights again)
     const int64_t avg = cdiv(d->M, (int64_t)d->n_experts);
     TNX_REQUIRE(d->w_stride == cdiv(d->N, 256) * 256 * d->K, "dense_linear: an expert's weights are one fragment-order copy");
@@ -375,7 +375,7 @@ extern "C" int tnx_dense_linear(void* stream, const tnx_dense_desc* d) {
     TNX_CHECK_LAUNCH("dense_rows");
     return TNX_OK;
   }
-  // many rows: the 128 x 256 kernel (row-major operands, 32-bit offsets); a few columns would leave its tiles
+  // many rows: the kernel of qgemm_pre.h (row-major operands, 32-bit offsets); a few columns would leave its tiles
   // and the device mostly empty: 32 rows per work-group then
   const bool narrow = d->N <= 128 && !mul && d->M > 64 && d->M <= 32 * 65535;
   if (!batch && !narrow && !d->x_frag && !d->y_frag && split == 1 && d->M > 64 && d->ldx == d->K && d->N % 16 == 0 &&
