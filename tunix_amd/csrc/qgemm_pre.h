@@ -90,17 +90,15 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   const int lm = lane & 15, lq = lane >> 4;
   const int tiles_m = (int)((a.M + ROWS - 1) / ROWS), tiles_n = (int)((a.N + kWideCols - 1) / kWideCols);
   int mtile, ntile, expert = 0, m_end = 0;
-  // tile number `tile` of row blocks x column tiles: in groups of 1024 rows, inside a group column tile by column tile, so that an XCD works on
-  // about 1024 rows x 8 column tiles at a time (2048 or 4096 rows: the same at 16 row tiles, 3 to 20 % slower at 8).  An expert of many rows the
-  // same: with all its row blocks per column tile, 8 experts of 8000 rows x 4096 -> 4096 took 2340 us against 1710 (256-row tiles), 2395 against
-  // 1760 (128).
-  auto tile_in = [&](int tile, int row_blocks) {
-    constexpr int GR = 1024 / ROWS;
-    const int per_group = GR * tiles_n, g = tile / per_group, r = tile % per_group;
-    const int gm = min(GR, row_blocks - g * GR);
-    mtile = g * GR + r % gm;
+  // tile number `tile` of row blocks x column tiles: in groups of `group` row blocks, inside a group column tile by column tile.  With groups of
+  // 1024 rows an XCD works on about 1024 rows x 8 column tiles at a time (2048 or 4096 rows: the same at 16 row tiles, 3 to 20 % slower at 8).
+  auto tile_in = [&](int tile, int row_blocks, int group) {
+    const int per_group = group * tiles_n, g = tile / per_group, r = tile % per_group;
+    const int gm = min(group, row_blocks - g * group);
+    mtile = g * group + r % gm;
     ntile = r / gm;
   };
+  constexpr int GR = 1024 / ROWS;
   if constexpr (GROUPED) {
     // tiles expert by expert; every wave finds its own
     auto blocks_of = [&](int e) { return e < a.n_experts ? (a.offsets[e + 1] - a.offsets[e] + ROWS - 1) / ROWS : 0; };
@@ -133,10 +131,14 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
       carry += __shfl(incl, 63, 64);
     }
     expert = __builtin_amdgcn_readfirstlane(found_e);
-    tile_in(__builtin_amdgcn_readfirstlane(found_at), __builtin_amdgcn_readfirstlane(found_nb));
+    // an expert of many rows in groups of 1024 rows or near it, equal ones, or its few last blocks would draw all weights for themselves:
+    // 8 experts of 8000 rows x 4096 -> 4096 took 2340 us with all row blocks per column tile against 1710 (256-row tiles), 2395 against
+    // 1760 (128); 8 of 1300 rows, eleven blocks, 340 us in groups of eight and three against 318 in one of eleven.
+    const int nb = __builtin_amdgcn_readfirstlane(found_nb), groups = max(1, (nb + GR / 2) / GR);
+    tile_in(__builtin_amdgcn_readfirstlane(found_at), nb, (nb + groups - 1) / groups);
     m_end = a.offsets[expert + 1];
   } else {
-    tile_in(xcd_tile((int)blockIdx.x, tiles_m * tiles_n), tiles_m);
+    tile_in(xcd_tile((int)blockIdx.x, tiles_m * tiles_n), tiles_m, GR);
   }
   // first row of the tile (GROUPED: first position in the sorted route list)
   const int64_t m0 = GROUPED ? (int64_t)a.offsets[expert] + (int64_t)mtile * ROWS : (int64_t)mtile * ROWS;
