@@ -80,9 +80,10 @@ const char* tnx_last_error(void);
  * tnx_embed_rows, centred norms, a factor, an extra row and the depth average to tnx_residual_norm_desc, slopes and
  * chunks to tnx_sink_attn_desc, an ungated form and shared weights to tnx_gated_norm_desc, TNX_EPI_RELU2, and
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
- * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows. */
+ * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora and
+ * tnx_gqa_attn_lora. */
 #define TNX_ABI_VERSION_MAJOR 6
-#define TNX_ABI_VERSION_MINOR 2
+#define TNX_ABI_VERSION_MINOR 3
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
 int tnx_version(void);
 
@@ -244,6 +245,35 @@ int tnx_rmsnorm_pair(void* stream, const uint16_t* x, const float* ws, int split
                      const uint16_t* res_post, uint16_t* y, const uint16_t* w2, uint16_t* y2,
                      int64_t M, int64_t D, float eps, int flavor);
 
+/* The norm ahead of a linear with a LoRA adapter, and the adapter's down-projection of what it writes:
+ * one of tnx_rmsnorm (x), tnx_rmsnorm_splitk (ws, split_k), tnx_rmsnorm_moe_combine (y_route, topk_w, k) or,
+ * with w2 and y2, tnx_rmsnorm_pair, then t[:, :R] = bf16(rows . a_t^T) as tnx_lora_down forms it (a_t bf16 [R, D];
+ * the routing scores of an MoE layer are the same product).  Up to 256 rows this is one launch when D <= 4096 and
+ * no output (h_out, y, y2) overlaps an input; the sums of t are then added in another order than tnx_lora_down's.
+ * D % 32 == 0, R % 16 == 0. */
+typedef struct tnx_norm_lora_desc {
+  int64_t M, D;
+  float eps;
+  int flavor;               /* TNX_NORM_* */
+  const uint16_t* x;        /* the rows, or */
+  const float* ws;          /* the partial planes of a split-k linear, or */
+  const uint16_t* y_route;  /* the routed rows of an MoE layer */
+  const uint16_t* topk_w;
+  int split_k, k;
+  const uint16_t* res_pre;
+  uint16_t* h_out;
+  const uint16_t* w;
+  const uint16_t* res_post;
+  uint16_t* y;
+  const uint16_t* w2;       /* a second norm, of y, or null */
+  uint16_t* y2;
+  const uint16_t* a_t;
+  uint16_t* t;
+  int64_t t_ld;
+  int R;
+} tnx_norm_lora_desc;
+int tnx_norm_lora(void* stream, const tnx_norm_lora_desc* d);
+
 /* ---------------------------------------------------------------------------------------
  * Per-head q/k RMSNorm (optional) + RoPE + KV-cache write for T tokens per row.
  *   qkv: bf16 [B*T, (Hq+2*Hkv)*dh] (q heads, then k heads, then v heads)
@@ -339,6 +369,11 @@ typedef struct tnx_attn_desc {
 } tnx_attn_desc;
 size_t tnx_attn_ws_bytes(int64_t B, int64_t T, int64_t S, int Hq, int dh, int kv_chunk);
 int tnx_gqa_attn(void* stream, const tnx_attn_desc* h_desc);
+
+/* tnx_gqa_attn, then the LoRA down-projection of its output rows, t[:, :R] = bf16(out . a_t^T) as tnx_lora_down forms it
+ * (a_t bf16 [R, Hq * dh], R % 16 == 0).  Where the key range of a decode step is split over few chunks, the pass that
+ * merges them takes the product too, whose sums are then added in another order. */
+int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld);
 
 /* ---------------------------------------------------------------------------------------
  * Fused lm_head -> fp32 log-softmax statistics, never writing [M,V] logits:

@@ -1745,6 +1745,101 @@ def test_rmsnorm_pair_equals_two_norms(gpu, family, planes):
     ops.rmsnorm_pair(w1, h2, w2, xn2, 1e-6, _NORM[family], M, D, res_post=h2)   # neither x nor ws
 
 
+def assert_down_projection(t, x, a, what=""):
+  """t against the exact product of bf16 rows and adapter columns.  32-bit sums: at most 16 products behind each other per thread, then
+  two binary trees over 256 of them, i.e. 32 roundings of 2^-24 of the sum of magnitudes; and the rounding to bf16."""
+  ref, mag = x.double() @ a.double().T, x.double().abs() @ a.double().abs().T
+  bad = (t.double() - ref).abs() > 2.0 ** -8 * ref.abs() + 32 * 2.0 ** -24 * mag
+  assert not bool(bad.any()), f"{what}: {int(bad.sum())} of {bad.numel()}"
+
+
+@pytest.mark.parametrize("family", ["llama3", "qwen3", "gemma3"])
+@pytest.mark.parametrize("src,M,D,R,parts", [
+    ("rows", 1, 32, 16, 0), ("rows", 5, 4096, 48, 0),
+    ("planes", 3, 2048, 192, 8), ("planes", 16, 4096, 192, 5), ("planes", 17, 4096, 64, 2),   # 17 rows of 4096: two launches
+    ("planes", 8, 2080, 16, 11), ("planes", 64, 1152, 96, 8), ("planes", 256, 512, 32, 4), ("planes", 257, 512, 32, 4),
+    ("planes", 2, 4128, 64, 3),                                                               # past 4096: two launches
+    ("routes", 9, 2048, 128, 8), ("routes", 4, 3072, 48, 10),
+    ("pair", 7, 1152, 96, 0), ("pair", 128, 1152, 64, 8), ("pair", 1, 4096, 208, 8),
+])
+def test_norm_and_down_projection_in_one_launch(gpu, family, src, M, D, R, parts):
+  """tnx_norm_lora against the norm of its own (rows bit for bit) and the exact down-projection of what it wrote; with an output in
+  place of an input it takes two launches, with the same rows."""
+  from tunix_amd import ops
+  from tunix_amd.model import _NORM
+  fl, eps = _NORM[family], 1e-6
+  w, w2 = bf(rnd((D,), 95, 0.3) + 1.0).to(gpu), bf(rnd((D,), 96, 0.3) + 1.0).to(gpu)
+  a, res = bf(rnd((R, D), 97)).to(gpu), bf(rnd((M, D), 98)).to(gpu)
+  x = bf(rnd((M, D), 99)).to(gpu)
+  ws = rnd((max(parts, 1), M, D), 100).to(gpu)
+  routes, tw = bf(rnd((M * max(parts, 1), D), 101)).to(gpu), bf(rnd((M, max(parts, 1)), 102, 0.2)).to(gpu)
+  new = lambda: torch.full((M, D), float("nan"), dtype=torch.bfloat16, device=gpu)
+  h1, y1, h2, y2 = new(), new(), new(), new()
+  t = torch.full((M, R + 8), 7.0, dtype=torch.bfloat16, device=gpu)
+  kw = dict(ws=ws, split_k=parts) if src != "pair" or parts else dict(x=x)
+  if src == "rows":
+    ops.rmsnorm(x, w, y1, eps, fl)
+    one = lambda h_in, h_out, y: ops.norm_lora(a, t, w, y, eps, fl, M, D, x=x)
+  elif src == "planes":
+    ops.rmsnorm_splitk(ws, parts, w, y1, eps, fl, M, D, res_pre=res, h_out=h1)
+    one = lambda h_in, h_out, y: ops.norm_lora(a, t, w, y, eps, fl, M, D, res_pre=h_in, h_out=h_out, **kw)
+  elif src == "routes":
+    ops.rmsnorm_moe_combine(routes, tw, parts, w, y1, eps, fl, M, D, res_pre=res, h_out=h1)
+    one = lambda h_in, h_out, y: ops.norm_lora(a, t, w, y, eps, fl, M, D, y_route=routes, topk_w=tw, k=parts, res_pre=h_in, h_out=h_out)
+  else:
+    ops.rmsnorm_pair(w, h1, w2, y1, eps, fl, M, D, res_post=res, **kw)
+    one = lambda h_in, h_out, y: ops.norm_lora(a, t, w, h_out, eps, fl, M, D, res_post=h_in, w2=w2, y2=y, **kw)
+  one(res, h2, y2)
+  torch.cuda.synchronize()
+  assert torch.equal(y1, y2) and (src == "rows" or torch.equal(h1, h2))
+  assert_down_projection(t[:, :R], y2, a, "apart")
+  assert bool((t[:, R:] == 7.0).all())
+  t.fill_(7.0)
+  h3, y3 = res.clone(), new()
+  one(h3, h3, y3)
+  torch.cuda.synchronize()
+  assert torch.equal(y1, y3) and (src == "rows" or torch.equal(h1, h3))
+  assert_down_projection(t[:, :R], y3, a, "in place")
+  with pytest.raises(ValueError):
+    ops.norm_lora(a, t, w, y2, eps, fl, M, D)           # no input
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,dh,S,kv_chunk,R,window,at", [
+    (1, 8, 2, 64, 128, 32, 32, 0, 127), (3, 32, 8, 128, 128, 32, 64, 0, 40),     # chunks without a key
+    (70, 4, 1, 256, 288, 32, 32, 0, 280), (5, 4, 1, 256, 500, 32, 48, 100, 470),   # nine and sixteen chunks, a window
+    (2, 32, 8, 128, 160, 32, 64, 0, 150),                                           # five chunks of 4096: two launches
+    (4, 8, 8, 64, 96, 96, 16, 0, 90), (9, 40, 8, 128, 64, 32, 16, 0, 63),           # one chunk; 5120 outputs
+])
+def test_attention_and_down_projection(gpu, B, Hq, Hkv, dh, S, kv_chunk, R, window, at):
+  """tnx_gqa_attn_lora against tnx_gqa_attn (bit for bit) and the exact down-projection of its output."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  k, v = bf(rnd((B, Hkv, S, dh), 103)).to(gpu), bf(rnd((B, Hkv, S, dh), 104)).to(gpu)
+  q, a = bf(rnd((B, Hq * dh), 105)).to(gpu), bf(rnd((R, Hq * dh), 106)).to(gpu)
+  tokens = torch.ones(B, S, dtype=torch.int32, device=gpu)
+  tokens[:, :5] = 0
+  col = torch.full((1,), at, dtype=torch.int32, device=gpu)
+  outs = [torch.full((B, Hq * dh), float("nan"), dtype=torch.bfloat16, device=gpu) for _ in range(2)]
+  t = torch.full((B, R + 16), 7.0, dtype=torch.bfloat16, device=gpu)
+  for i, out in enumerate(outs):
+    ws = torch.full((max(ops.attn_ws_bytes(B, 1, S, Hq, dh, kv_chunk) // 4, 1),), float("nan"), device=gpu)
+    d = L.AttnDesc()
+    d.B, d.T, d.S, d.Hq, d.Hkv, d.dh = B, 1, S, Hq, Hkv, dh
+    d.scale, d.window, d.pad_id = dh ** -0.5, window, 0
+    d.q, d.kcache, d.vcache = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    d.tokens, d.tok_ld, d.col_ptr = tokens.data_ptr(), S, col.data_ptr()
+    d.kv_chunk, d.ws, d.out = kv_chunk, ws.data_ptr(), out.data_ptr()
+    if i:
+      ops.gqa_attn_lora(d, a, t)
+    else:
+      ops.gqa_attn(d)
+    torch.cuda.synchronize()
+  assert torch.equal(*outs)
+  assert bool(torch.isfinite(outs[0].float()).all())
+  assert_down_projection(t[:, :R], outs[1], a)
+  assert bool((t[:, R:] == 7.0).all())
+
+
 @pytest.mark.parametrize("kv_chunk,window,planes,Hq,split", [
     (0, 0, False, 8, 3), (32, 0, True, 8, 3), (0, 40, True, 8, 3), (64, 0, False, 8, 3),
     (0, 0, True, 16, 3),     # eight query heads per kv head: more than one set of plane loads

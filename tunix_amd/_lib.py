@@ -12,7 +12,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtunix_hip.so")
 
 # the ABI this binding was written against (TNX_ABI_VERSION_MAJOR / _MINOR of include/tunix_hip.h)
-ABI_VERSION = (6, 2)
+ABI_VERSION = (6, 3)
 
 TNX_Q_INT4, TNX_Q_NF4 = 0, 1
 TNX_NORM_LLAMA, TNX_NORM_QWEN3, TNX_NORM_GEMMA3 = 0, 1, 2
@@ -52,6 +52,15 @@ class RopeDesc(C.Structure):
       ("qkv", _p), ("positions", _p), ("pos_ld", _i64), ("col_ptr", _p),
       ("q_out", _p), ("kcache", _p), ("vcache", _p),
       ("qkv_ws", _p), ("split_k", _i32),
+  ]
+
+
+class NormLoraDesc(C.Structure):
+  _fields_ = [
+      ("M", _i64), ("D", _i64), ("eps", _f32), ("flavor", _i32),
+      ("x", _p), ("ws", _p), ("y_route", _p), ("topk_w", _p), ("split_k", _i32), ("k", _i32),
+      ("res_pre", _p), ("h_out", _p), ("w", _p), ("res_post", _p), ("y", _p), ("w2", _p), ("y2", _p),
+      ("a_t", _p), ("t", _p), ("t_ld", _i64), ("R", _i32),
   ]
 
 
@@ -295,10 +304,12 @@ SIGNATURES = {
     "tnx_rmsnorm_splitk": (_i32, [_p, _p, _i32, _p, _p, _p, _p, _p, _i64, _i64, _f32, _i32]),
     "tnx_rmsnorm_moe_combine": (_i32, [_p, _p, _p, _i32, _p, _p, _p, _p, _p, _i64, _i64, _f32, _i32]),
     "tnx_rmsnorm_pair": (_i32, [_p, _p, _p, _i32, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _f32, _i32]),
+    "tnx_norm_lora": (_i32, [_p, C.POINTER(NormLoraDesc)]),
     "tnx_qknorm_rope_kvwrite": (_i32, [_p, C.POINTER(RopeDesc)]),
     "tnx_rope_table": (_i32, [_p, _p, _i64, _p, _i64, _p, _i32, _p, _p]),
     "tnx_attn_ws_bytes": (C.c_size_t, [_i64, _i64, _i64, _i32, _i32, _i32]),
     "tnx_gqa_attn": (_i32, [_p, C.POINTER(AttnDesc)]),
+    "tnx_gqa_attn_lora": (_i32, [_p, C.POINTER(AttnDesc), _p, _i32, _p, _i64]),
     "tnx_lmhead_nblocks": (_i64, [_i64]),
     "tnx_lmhead_logp": (_i32, [_p, C.POINTER(LmHeadDesc)]),
     "tnx_sample_topk_ws_bytes": (C.c_size_t, [_i64, _i64, _i32]),

@@ -14,6 +14,7 @@
 
 #include "common.h"
 #include "gemm_tile.h"   // dma16, raw_rsrc, tnx_wait_vm
+#include "row_adapter.h"
 
 // Register stages of the key-block ring (head_dim <= 128).  Two: one block in flight while one is
 // computed.  A compute unit draws 21-28 GB/s from memory whatever its waves request, so a
@@ -55,6 +56,16 @@ struct AttnArgs {
 };
 
 constexpr float kNegBig = -1.0e30f;
+constexpr int kPartPad = 4;   // numbers in front of a partial's O[dh]: m, l, and two that keep the rest on 16 bytes
+
+// f over the four lanes lm + 16 {0, 1, 2, 3} that share a query, in all of them
+template <class F>
+__device__ __forceinline__ float across_quarters(float x, F f) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 
 // FUSE: 0 = q comes rotated, keys and values are in the cache; 1 = the fused rotation and cache
 // write of a decode step (below), qkv taken from the finished output or from any number of
@@ -208,9 +219,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
       sv[s] = x;
       if (kvalid[s]) bmax = fmaxf(bmax, x);
     }
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
-    const float m_new = fmaxf(m_run, bmax);
+    const float m_new = fmaxf(m_run, across_quarters(bmax, [](float x, float y) { return fmaxf(x, y); }));
     const float alpha = __expf(m_run - m_new);
     m_run = m_new;
     float p[8], psum = 0.f;
@@ -486,8 +495,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
     }
   }
 
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = across_quarters(l_run, [](float x, float y) { return x + y; });
 
   // O rows are query columns 4*lq + i; columns are d = h*128 + 8*lm + jj.
   const bool dvalid = 8 * lm < (DH < 128 ? DH : 128);
@@ -520,7 +528,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
     const int gi = n & (a.Gp - 1), ti = qt * PT + (n >> a.gp_shift);
     if (!(gi < a.G && ti < a.T)) continue;
     const int64_t qv = (b * a.T + ti) * a.Hq + hkv * a.G + gi;
-    float* p = a.ws + (qv * a.n_chunks + chunk) * (DH + 2);
+    float* p = a.ws + (qv * a.n_chunks + chunk) * (DH + kPartPad);
     if (lm == 0) {
       p[0] = m;
       p[1] = l;
@@ -529,7 +537,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
 #pragma unroll
     for (int h = 0; h < NH; ++h)
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) p[2 + h * 128 + 8 * lm + jj] = O[h][jj][i];
+      for (int jj = 0; jj < 8; jj += 4)
+        *reinterpret_cast<f32x4*>(p + kPartPad + h * 128 + 8 * lm + jj) = f32x4{O[h][jj][i], O[h][jj + 1][i], O[h][jj + 2][i], O[h][jj + 3][i]};
   }
 }
 
@@ -784,14 +793,6 @@ __device__ __forceinline__ u32x4 attn_lds128(uint32_t addr) {
 __device__ __forceinline__ void dma4(uint32_t lds, const u32x4& r, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(r) : "memory", "m0");
 }
-// f over the four lanes lm + 16 {0, 1, 2, 3} that share a query, in all of them
-template <class F>
-__device__ __forceinline__ float across_quarters(float x, F f) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
 // c += a . b with the accumulator in place (the compiler's form copies O at every branch of the loop).  The wait states between a
 // vector write of an operand and the MFMA that reads it stand inside, under the MFMA before; what reads c next has to lie eight
 // instruction slots behind (the compiler does not know that this is an MFMA: tests/test_mfma_wait_states.py checks the built code).
@@ -1044,8 +1045,8 @@ __global__ void attn_combine_kernel(const float* ws, int64_t n_qvec, int dh, int
   extern __shared__ float ml[];   // [n_chunks][2]
   const int64_t qv = blockIdx.x;
   const int d = threadIdx.x;
-  const float* p = ws + qv * n_chunks * (dh + 2);
-  for (int i = d; i < 2 * n_chunks; i += blockDim.x) ml[i] = p[(i >> 1) * (dh + 2) + (i & 1)];
+  const float* p = ws + qv * n_chunks * (dh + kPartPad);
+  for (int i = d; i < 2 * n_chunks; i += blockDim.x) ml[i] = p[(i >> 1) * (dh + kPartPad) + (i & 1)];
   __syncthreads();
   if (d >= dh) return;
   float M = kNegBig;
@@ -1055,7 +1056,7 @@ __global__ void attn_combine_kernel(const float* ws, int64_t n_qvec, int dh, int
   for (int c0 = 0; c0 < n_chunks; c0 += 8) {
     float v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = p[min(c0 + u, n_chunks - 1) * (dh + 2) + 2 + d];
+    for (int u = 0; u < 8; ++u) v[u] = p[min(c0 + u, n_chunks - 1) * (dh + kPartPad) + kPartPad + d];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int c = c0 + u;
@@ -1072,6 +1073,86 @@ __global__ void attn_combine_kernel(const float* ws, int64_t n_qvec, int dh, int
   out[qv * dh + d] = f2bf(L > 0.f ? o / L : 0.f);
 }
 
+// The same over whole rows of heads, with the LoRA down-projection of the row behind it (row_adapter.h): grid (groups of adapter
+// columns, rows); the first group writes the row.  The chunks' (max, sum) pairs of all heads go to LDS; a thread asks for its first eight
+// chunks' outputs and its first columns of A ahead of them.
+template <int MAXC, int NB, int NCH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void attn_combine_lora_kernel(const float* ws, int heads, int dh, int n_chunks, uint16_t* out,
+                                                                const RowAdapterArgs g) {
+  extern __shared__ float ml[];   // [heads][n_chunks][2]
+  __shared__ float sums[4 * NB];
+  const int64_t row = blockIdx.y;
+  const int K = heads * dh, pitch = dh + kPartPad;
+  const float* base = ws + row * (int64_t)heads * n_chunks * pitch;
+  RowAdapter<MAXC, NB> ad;
+  const float* p[MAXC];
+  int at[MAXC];
+  typedef float f32x2v __attribute__((ext_vector_type(2)));
+  f32x4 v[MAXC][NCH][2];
+  auto fetch = [&](int c, int c0) {
+#pragma unroll
+    for (int u = 0; u < NCH; ++u)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) v[c][u][q] = *reinterpret_cast<const f32x4*>(p[c] + min(c0 + u, n_chunks - 1) * pitch + 4 * q);
+  };
+  for (int i = threadIdx.x; i < heads * n_chunks; i += 256)
+    *reinterpret_cast<f32x2v*>(ml + 2 * i) = *reinterpret_cast<const f32x2v*>(base + (int64_t)i * pitch);
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int e = min(c * 256 + (int)threadIdx.x, K / 8 - 1) * 8, h = e / dh;
+    at[c] = h * n_chunks;
+    p[c] = base + (int64_t)h * n_chunks * pitch + kPartPad + (e - h * dh);
+    fetch(c, 0);
+  }
+  ad.load(g, blockIdx.x, K);
+  __syncthreads();
+  u32x4 x[MAXC];
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    x[c] = u32x4{0, 0, 0, 0};
+    const float* m = ml + 2 * at[c];
+    float M = kNegBig;
+    for (int i = 0; i < n_chunks; ++i)
+      if (m[2 * i + 1] > 0.f) M = fmaxf(M, m[2 * i]);
+    float L = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 0; c0 < n_chunks; c0 += NCH) {
+      if (c0 > 0) fetch(c, c0);
+#pragma unroll
+      for (int u = 0; u < NCH; ++u) {
+        const int i = c0 + u;
+        if (i < n_chunks) {
+          const float l = m[2 * i + 1];
+          if (l > 0.f) {   // (a chunk without a key: an O nobody wrote)
+            const float w = __expf(m[2 * i] - M);
+            L += w * l;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              o[q] += w * v[c][u][0][q];
+              o[4 + q] += w * v[c][u][1][q];
+            }
+          }
+        }
+      }
+    }
+    const int ch = c * 256 + threadIdx.x;
+    if (ch < K / 8) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[c][q] = L > 0.f ? pack2bf(o[2 * q] / L, o[2 * q + 1] / L) : 0u;
+      if (blockIdx.x == 0) *reinterpret_cast<u32x4*>(out + row * K + (int64_t)ch * 8) = x[c];
+    }
+  }
+  ad.finish(g, blockIdx.x, row, x, sums);
+}
+
+// Whether one launch merges the chunks and takes the adapter columns, sixteen per work-group: as long as a row's partials are 64 KB, which every
+// group of columns reads again, and two work-groups per compute unit hold them.  us, attention with two launches | one behind it: 32 heads of
+// 128, 64 columns, 4 chunks 32 rows 19.3 | 17.9, 6 chunks 3 rows 11.6 | 12.1, 8 chunks 16 rows 19.6 | 20.0; 2 chunks 100 rows 36.4 | 34.6; 4 heads of 256, 32
+// columns, 9 chunks 16 rows 12.2 | 10.8, 64 rows 15.5 | 13.6.
+constexpr int kCombineCols = 16;
+bool attn_lora_one_launch(int64_t rows, int64_t K, int n_chunks, int R) {
+  return K <= 8 * 256 * 2 && n_chunks * K * 4 <= 64 * 1024 && rows * cdiv(R, kCombineCols) <= 512;
+}
+
 int next_pow2(int x) {
   int p = 1;
   while (p < x) p <<= 1;
@@ -1084,10 +1165,11 @@ extern "C" size_t tnx_attn_ws_bytes(int64_t B, int64_t T, int64_t S, int Hq, int
                                     int kv_chunk) {
   if (kv_chunk <= 0) return 0;
   const int64_t n_chunks = cdiv(S, kv_chunk);
-  return (size_t)(B * T * Hq * n_chunks * (dh + 2)) * sizeof(float);
+  return (size_t)(B * T * Hq * n_chunks * (dh + kPartPad)) * sizeof(float);
 }
 
-extern "C" int tnx_gqa_attn(void* stream, const tnx_attn_desc* d) {
+// The attention launch; combine: and, of a split key range, the pass that merges its chunks.
+static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
   TNX_REQUIRE(d, "attn: null descriptor");
   TNX_REQUIRE(d->B > 0 && d->T > 0 && d->S > 0, "attn: B,T,S must be positive");
   TNX_REQUIRE(d->dh == 64 || d->dh == 128 || d->dh == 256, "attn: head_dim %d not in {64,128,256}", d->dh);
@@ -1190,11 +1272,33 @@ extern "C" int tnx_gqa_attn(void* stream, const tnx_attn_desc* d) {
   }
 #undef TNX_ATTN_LAUNCH
   TNX_CHECK_LAUNCH("gqa_attn");
-  if (a.n_chunks > 1) {
+  if (a.n_chunks > 1 && combine) {
     const int64_t nq = d->B * d->T * d->Hq;
     hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)nq), dim3(d->dh), (size_t)a.n_chunks * 2 * sizeof(float), st,
                        a.ws, nq, d->dh, a.n_chunks, a.out);
     TNX_CHECK_LAUNCH("gqa_attn_combine");
   }
+  return TNX_OK;
+}
+
+extern "C" int tnx_gqa_attn(void* stream, const tnx_attn_desc* d) { return gqa_attn(stream, d, true); }
+
+extern "C" int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld) {
+  TNX_REQUIRE(d && a_t && t, "attn_lora: null pointer");
+  TNX_REQUIRE(R > 0 && R % 16 == 0 && t_ld >= R, "attn_lora: R=%d must be a multiple of 16 and <= t_ld", R);
+  const int64_t K = (int64_t)d->Hq * d->dh;
+  TNX_REQUIRE(d->B > 0 && d->T > 0 && K > 0 && K % 32 == 0, "attn_lora: bad shape");
+  const int n_chunks = d->kv_chunk > 0 ? (int)cdiv(d->S, d->kv_chunk) : 1;
+  const bool one = d->T == 1 && n_chunks > 1 && attn_lora_one_launch(d->B, K, n_chunks, R);
+  const int rc = gqa_attn(stream, d, !one);
+  if (rc != TNX_OK) return rc;
+  if (!one) return tnx_lora_down(stream, d->out, d->B * d->T, K, a_t, R, t, t_ld);
+  const RowAdapterArgs g{a_t, R, kCombineCols, t, t_ld};
+  const dim3 grid((unsigned)cdiv(R, g.nc), (unsigned)d->B);
+  const size_t lds = (size_t)d->Hq * n_chunks * 2 * sizeof(float);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), lds, as_stream(stream), d->ws, d->Hq, d->dh, n_chunks, d->out, g); };
+  if (K <= 8 * 256) n_chunks <= 4 ? launch(attn_combine_lora_kernel<1, kCombineCols, 4>) : launch(attn_combine_lora_kernel<1, kCombineCols, 8>);
+  else n_chunks <= 4 ? launch(attn_combine_lora_kernel<2, kCombineCols, 4>) : launch(attn_combine_lora_kernel<2, kCombineCols, 8>);
+  TNX_CHECK_LAUNCH("gqa_attn_combine_lora");
   return TNX_OK;
 }

@@ -3,7 +3,10 @@
 // are written for exact dtype-flow parity and few launches, not for peak bandwidth.
 #include <string.h>
 
+#include <type_traits>
+
 #include "common.h"
+#include "row_adapter.h"
 
 namespace {
 
@@ -86,18 +89,35 @@ __device__ __forceinline__ void unpack8(const u32x4& p, float (&f)[8]) {
 // the split_k routed rows of a token, j ascending: the weighted combine of an MoE layer folded
 // into the norm (same arithmetic as moe_combine_vec_kernel).
 constexpr int kNormInRow = 0, kNormInPlanes = 1, kNormInRoutes = 2;
-template <int MAXC, int FLAVOR, int IN>
-__global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, const uint16_t* res_pre,
-                                                          uint16_t* h_out, const uint16_t* w,
-                                                          const uint16_t* res_post, uint16_t* y,
-                                                          int64_t D, float eps, int /*flavor*/,
-                                                          const float* ws, int split_k, int64_t plane,
-                                                          const uint16_t* w2, uint16_t* y2, const uint16_t* cw) {
+struct NormRow {
+  const uint16_t *x, *res_pre;
+  uint16_t* h_out;
+  const uint16_t *w, *res_post;
+  uint16_t* y;
+  int64_t D;
+  float eps;
+  const float* ws;
+  int split_k;
+  int64_t plane;
+  const uint16_t* w2;
+  uint16_t* y2;
+  const uint16_t* cw;
+};
+// One row: writes it (WRITE) and leaves the thread's chunks of the last norm, packed, in `last` (zeros past the row's end).
+// behind(): called once every load of the row has been asked for.
+template <int MAXC, int FLAVOR, int IN, class F>
+__device__ __forceinline__ void norm_row(const NormRow& n, int64_t row, bool write, float* red, u32x4 (&last)[MAXC], F behind) {
+  const uint16_t *x = n.x, *res_pre = n.res_pre, *w = n.w, *res_post = n.res_post, *w2 = n.w2, *cw = n.cw;
+  uint16_t *h_out = n.h_out, *y = n.y, *y2 = n.y2;
+  const float* ws = n.ws;
+  const int64_t D = n.D, plane = n.plane;
+  const float eps = n.eps;
+  const int split_k = n.split_k;
   constexpr bool PLANES = IN == kNormInPlanes, ROUTES = IN == kNormInRoutes;
-  __shared__ float red[4];
-  const int64_t row = blockIdx.x;
   const int nchunks = (int)(D / 8);
   float h[MAXC][8];
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) last[c] = u32x4{0, 0, 0, 0};
   float ss = 0.f;
   // The norm weights and the post-norm residual do not depend on the row: they are asked for ahead of its planes (a launch is a
   // few round trips to memory long, and one that starts behind the sums adds a whole one: 16 rows of 4096 from
@@ -118,13 +138,14 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, con
   // to eight planes per chunk at once, further planes in groups of eight): the kernel is a few
   // dependent memory round trips long, and each group of loads that waits for the previous sum
   // adds one.  The sum itself stays in split order.
+  constexpr int CS = MAXC < 2 ? 1 : 2;
 #pragma unroll
-  for (int c0 = 0; c0 < MAXC; c0 += 2) {
+  for (int c0 = 0; c0 < MAXC; c0 += CS) {
     if (c0 * 256 >= nchunks) break;   // uniform
-    f32x4 p0[2][8], p1[2][8];
-    u32x4 xin[2], rin[2], yin[2][8];
+    f32x4 p0[CS][8], p1[CS][8];
+    u32x4 xin[CS], rin[CS], yin[CS][8];
 #pragma unroll
-    for (int cc = 0; cc < 2; ++cc) {
+    for (int cc = 0; cc < CS; ++cc) {
       const int ch = (c0 + cc) * 256 + threadIdx.x;
       const int64_t o = row * D + (int64_t)min(ch, nchunks - 1) * 8;
       if (PLANES) {
@@ -144,8 +165,9 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, con
       }
       if (res_pre) rin[cc] = *reinterpret_cast<const u32x4*>(res_pre + o);
     }
+    if (c0 + CS >= MAXC || (c0 + CS) * 256 >= nchunks) behind();
 #pragma unroll
-    for (int cc = 0; cc < 2; ++cc) {
+    for (int cc = 0; cc < CS; ++cc) {
       const int c = c0 + cc;
       const int ch = c * 256 + threadIdx.x;
       if (ch < nchunks) {
@@ -222,7 +244,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, con
 #pragma unroll
           for (int j = 0; j < 8; ++j) h[c][j] = rbf(h[c][j] + r[j]);
         }
-        if (h_out) {
+        if (h_out && write) {
           u32x4 q;
 #pragma unroll
           for (int j = 0; j < 4; ++j) q[j] = pack2bf(h[c][2 * j], h[c][2 * j + 1]);
@@ -256,7 +278,8 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, con
       u32x4 q;
 #pragma unroll
       for (int j = 0; j < 4; ++j) q[j] = pack2bf(v[2 * j], v[2 * j + 1]);
-      *reinterpret_cast<u32x4*>(y + o) = q;
+      if (write) *reinterpret_cast<u32x4*>(y + o) = q;
+      last[c] = q;
       if (w2) {   // the row just written is the input of a second norm: keep it, as rounded
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -282,30 +305,72 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const uint16_t* x, con
       for (int j = 0; j < 4; ++j)
         q[j] = pack2bf(norm_elem(h[c][2 * j], wv[2 * j], ms2, eps, FLAVOR),
                        norm_elem(h[c][2 * j + 1], wv[2 * j + 1], ms2, eps, FLAVOR));
-      *reinterpret_cast<u32x4*>(y2 + row * D + (int64_t)ch * 8) = q;
+      if (write) *reinterpret_cast<u32x4*>(y2 + row * D + (int64_t)ch * 8) = q;
+      last[c] = q;
     }
   }
 }
-
-// The kernel is unrolled over its chunks (256 threads x 8 elements each): instantiated for 2, 4
-// and 8 chunks per thread so that the common widths (D <= 4096) run the small instance -- the
-// code a wave walks through once is fetched cold at every launch.
-template <int MAXC, class... Args>
-void launch_rmsnorm_vec_c(hipStream_t st, int64_t M, int flavor, int in, Args... args) {
-#define TNX_NORM_CASE(F)                                                                                   \
-  if (in == kNormInPlanes) hipLaunchKernelGGL((rmsnorm_vec_kernel<MAXC, F, kNormInPlanes>), dim3((unsigned)M), dim3(256), 0, st, args...); \
-  else if (in == kNormInRoutes) hipLaunchKernelGGL((rmsnorm_vec_kernel<MAXC, F, kNormInRoutes>), dim3((unsigned)M), dim3(256), 0, st, args...); \
-  else hipLaunchKernelGGL((rmsnorm_vec_kernel<MAXC, F, kNormInRow>), dim3((unsigned)M), dim3(256), 0, st, args...)
-  if (flavor == TNX_NORM_LLAMA) { TNX_NORM_CASE(TNX_NORM_LLAMA); }
-  else if (flavor == TNX_NORM_QWEN3) { TNX_NORM_CASE(TNX_NORM_QWEN3); }
-  else { TNX_NORM_CASE(TNX_NORM_GEMMA3); }
-#undef TNX_NORM_CASE
+template <int MAXC, int FLAVOR, int IN>
+__global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const NormRow n) {
+  __shared__ float red[4];
+  u32x4 last[MAXC];
+  norm_row<MAXC, FLAVOR, IN>(n, blockIdx.x, true, red, last, [] {});
 }
-template <class... Args>
-void launch_rmsnorm_vec(hipStream_t st, int64_t M, int64_t D, int flavor, int in, Args... args) {
-  if (D <= 8 * 256 * 2) launch_rmsnorm_vec_c<2>(st, M, flavor, in, args...);
-  else if (D <= 8 * 256 * 4) launch_rmsnorm_vec_c<4>(st, M, flavor, in, args...);
-  else launch_rmsnorm_vec_c<kNormMaxChunks>(st, M, flavor, in, args...);
+// The same with the LoRA down-projection of the row behind it (row_adapter.h): grid (groups of adapter columns, rows); the first
+// group writes the row.
+template <int MAXC, int FLAVOR, int IN, int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void rmsnorm_lora_kernel(const NormRow n, const RowAdapterArgs g) {
+  __shared__ float red[4], sums[4 * NB];
+  u32x4 last[MAXC];
+  RowAdapter<MAXC, NB> ad;
+  norm_row<MAXC, FLAVOR, IN>(n, blockIdx.y, blockIdx.x == 0, red, last, [&] { ad.load(g, blockIdx.x, n.D); });
+  ad.finish(g, blockIdx.x, blockIdx.y, last, sums);
+}
+
+// The kernel is unrolled over its chunks (256 threads x 8 elements each): instantiated for 1, 2, 4
+// and 8 chunks per thread so that the common widths (D <= 4096) run the small instances -- the
+// code a wave walks through once is fetched cold at every launch.
+template <class F>
+void with_flavor(int flavor, F f) {
+  if (flavor == TNX_NORM_LLAMA) f(std::integral_constant<int, TNX_NORM_LLAMA>{});
+  else if (flavor == TNX_NORM_QWEN3) f(std::integral_constant<int, TNX_NORM_QWEN3>{});
+  else f(std::integral_constant<int, TNX_NORM_GEMMA3>{});
+}
+template <class F>
+void with_input(int in, F f) {
+  if (in == kNormInPlanes) f(std::integral_constant<int, kNormInPlanes>{});
+  else if (in == kNormInRoutes) f(std::integral_constant<int, kNormInRoutes>{});
+  else f(std::integral_constant<int, kNormInRow>{});
+}
+void launch_rmsnorm_vec(hipStream_t st, int64_t M, int flavor, int in, const NormRow& n) {
+  with_flavor(flavor, [&](auto f) {
+    with_input(in, [&](auto i) {
+      constexpr int F = decltype(f)::value, IN = decltype(i)::value;
+      if (n.D <= 8 * 256) hipLaunchKernelGGL((rmsnorm_vec_kernel<1, F, IN>), dim3((unsigned)M), dim3(256), 0, st, n);
+      else if (n.D <= 8 * 256 * 2) hipLaunchKernelGGL((rmsnorm_vec_kernel<2, F, IN>), dim3((unsigned)M), dim3(256), 0, st, n);
+      else if (n.D <= 8 * 256 * 4) hipLaunchKernelGGL((rmsnorm_vec_kernel<4, F, IN>), dim3((unsigned)M), dim3(256), 0, st, n);
+      else hipLaunchKernelGGL((rmsnorm_vec_kernel<kNormMaxChunks, F, IN>), dim3((unsigned)M), dim3(256), 0, st, n);
+    });
+  });
+}
+// Whether the rows' work-groups take the adapter columns too: as long as there is at most one of them per compute unit.
+// us, two launches | one, eight planes: D 4096, 192 columns 1 row 8.6 | 5.8, 8 rows 9.2 | 6.5, 16 rows 9.6 | 8.9, 24 rows (24 columns each) 10.2 | 14;
+// D 2048, 128 columns 16 rows 7.3 | 4.8, 64 rows 7.9 | 7.4, 128 rows 9.3 | 11.5; two norms of 1152, 64 columns 64 rows 7.5 | 5.9, 128 rows 7.9 | 6.6.
+bool norm_lora_one_launch(int64_t M, int64_t D, int R) {
+  if (M > 256 || D > 8 * 256 * 2) return false;
+  return D > 8 * 256 ? M <= 16 && row_adapter_cols(M, R) <= 16 : row_adapter_cols(M, R) <= 32;
+}
+void launch_rmsnorm_lora(hipStream_t st, int64_t M, int flavor, int in, const NormRow& n, const RowAdapterArgs& g) {
+  const dim3 grid((unsigned)cdiv(g.R, g.nc), (unsigned)M);
+  with_flavor(flavor, [&](auto f) {
+    with_input(in, [&](auto i) {
+      constexpr int F = decltype(f)::value, IN = decltype(i)::value;
+      const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, n, g); };
+      if (n.D > 8 * 256) g.nc <= 8 ? launch(rmsnorm_lora_kernel<2, F, IN, 8>) : launch(rmsnorm_lora_kernel<2, F, IN, 16>);
+      else if (g.nc <= 16) g.nc <= 8 ? launch(rmsnorm_lora_kernel<1, F, IN, 8>) : launch(rmsnorm_lora_kernel<1, F, IN, 16>);
+      else g.nc <= 24 ? launch(rmsnorm_lora_kernel<1, F, IN, 24>) : launch(rmsnorm_lora_kernel<1, F, IN, 32>);
+    });
+  });
 }
 
 __global__ void embed_kernel(const uint16_t* table, int64_t V, int64_t D, const int32_t* ids,
@@ -610,9 +675,7 @@ extern "C" int tnx_rmsnorm(void* stream, const uint16_t* x, const uint16_t* res_
   TNX_REQUIRE(M > 0 && D > 0 && D <= 16384, "rmsnorm: D=%lld out of range (1..16384)", (long long)D);
   TNX_REQUIRE(flavor >= TNX_NORM_LLAMA && flavor <= TNX_NORM_GEMMA3, "rmsnorm: bad flavor %d", flavor);
   if (D % 8 == 0 && D <= 8 * 256 * kNormMaxChunks)
-    launch_rmsnorm_vec(as_stream(stream), M, D, flavor, kNormInRow, x, res_pre, h_out, w, res_post, y, D, eps, flavor,
-                       (const float*)nullptr, 0, (int64_t)0, (const uint16_t*)nullptr, (uint16_t*)nullptr,
-                       (const uint16_t*)nullptr);
+    launch_rmsnorm_vec(as_stream(stream), M, flavor, kNormInRow, NormRow{x, res_pre, h_out, w, res_post, y, D, eps});
   else
     hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)M), dim3(256), (size_t)D * sizeof(float),
                        as_stream(stream), x, res_pre, h_out, w, res_post, y, D, eps, flavor);
@@ -628,9 +691,8 @@ extern "C" int tnx_rmsnorm_splitk(void* stream, const float* ws, int split_k, co
   TNX_REQUIRE(M > 0 && D > 0 && D % 8 == 0 && D <= 8 * 256 * kNormMaxChunks,
               "rmsnorm_splitk: D=%lld must be a multiple of 8 and <= 16384", (long long)D);
   TNX_REQUIRE(flavor >= TNX_NORM_LLAMA && flavor <= TNX_NORM_GEMMA3, "rmsnorm_splitk: bad flavor %d", flavor);
-  launch_rmsnorm_vec(as_stream(stream), M, D, flavor, kNormInPlanes, (const uint16_t*)nullptr, res_pre, h_out, w, res_post, y,
-                     D, eps, flavor, ws, split_k, (int64_t)(M * D), (const uint16_t*)nullptr, (uint16_t*)nullptr,
-                     (const uint16_t*)nullptr);
+  launch_rmsnorm_vec(as_stream(stream), M, flavor, kNormInPlanes,
+                     NormRow{nullptr, res_pre, h_out, w, res_post, y, D, eps, ws, split_k, (int64_t)(M * D)});
   TNX_CHECK_LAUNCH("rmsnorm_splitk");
   return TNX_OK;
 }
@@ -644,8 +706,8 @@ extern "C" int tnx_rmsnorm_moe_combine(void* stream, const uint16_t* y_route, co
   TNX_REQUIRE(M > 0 && D > 0 && D % 8 == 0 && D <= 8 * 256 * kNormMaxChunks,
               "rmsnorm_moe_combine: D=%lld must be a multiple of 8 and <= 16384", (long long)D);
   TNX_REQUIRE(flavor >= TNX_NORM_LLAMA && flavor <= TNX_NORM_GEMMA3, "rmsnorm_moe_combine: bad flavor %d", flavor);
-  launch_rmsnorm_vec(as_stream(stream), M, D, flavor, kNormInRoutes, y_route, res_pre, h_out, w, res_post, y, D, eps, flavor,
-                     (const float*)nullptr, k, (int64_t)0, (const uint16_t*)nullptr, (uint16_t*)nullptr, topk_w);
+  launch_rmsnorm_vec(as_stream(stream), M, flavor, kNormInRoutes,
+                     NormRow{y_route, res_pre, h_out, w, res_post, y, D, eps, nullptr, k, 0, nullptr, nullptr, topk_w});
   TNX_CHECK_LAUNCH("rmsnorm_moe_combine");
   return TNX_OK;
 }
@@ -660,10 +722,43 @@ extern "C" int tnx_rmsnorm_pair(void* stream, const uint16_t* x, const float* ws
   TNX_REQUIRE(M > 0 && D > 0 && D % 8 == 0 && D <= 8 * 256 * kNormMaxChunks,
               "rmsnorm_pair: D=%lld must be a multiple of 8 and <= 16384", (long long)D);
   TNX_REQUIRE(flavor >= TNX_NORM_LLAMA && flavor <= TNX_NORM_GEMMA3, "rmsnorm_pair: bad flavor %d", flavor);
-  launch_rmsnorm_vec(as_stream(stream), M, D, flavor, ws ? kNormInPlanes : kNormInRow, x, res_pre, h_out, w, res_post, y, D,
-                     eps, flavor, ws, ws ? split_k : 0, (int64_t)(M * D), w2, y2, (const uint16_t*)nullptr);
+  launch_rmsnorm_vec(as_stream(stream), M, flavor, ws ? kNormInPlanes : kNormInRow,
+                     NormRow{x, res_pre, h_out, w, res_post, y, D, eps, ws, ws ? split_k : 0, (int64_t)(M * D), w2, y2});
   TNX_CHECK_LAUNCH("rmsnorm_pair");
   return TNX_OK;
+}
+
+extern "C" int tnx_norm_lora(void* stream, const tnx_norm_lora_desc* d) {
+  TNX_REQUIRE(d, "norm_lora: null descriptor");
+  TNX_REQUIRE((d->x != nullptr) + (d->ws != nullptr) + (d->y_route != nullptr) == 1, "norm_lora: exactly one of x, ws and y_route must be given");
+  TNX_REQUIRE(!d->w2 == !d->y2 && !(d->w2 && d->y_route), "norm_lora: the second norm takes w2 and y2, and rows or planes");
+  TNX_REQUIRE(d->w && d->y && d->a_t && d->t, "norm_lora: null pointer");
+  const int64_t M = d->M, D = d->D;
+  TNX_REQUIRE(M > 0 && D > 0 && D % 32 == 0 && D <= 8 * 256 * kNormMaxChunks, "norm_lora: D=%lld must be a multiple of 32 and <= 16384", (long long)D);
+  TNX_REQUIRE(d->R > 0 && d->R % 16 == 0 && d->t_ld >= d->R, "norm_lora: R=%d must be a multiple of 16 and <= t_ld", d->R);
+  TNX_REQUIRE(d->flavor >= TNX_NORM_LLAMA && d->flavor <= TNX_NORM_GEMMA3, "norm_lora: bad flavor %d", d->flavor);
+  if (d->ws) TNX_REQUIRE(d->split_k >= 1, "norm_lora: split_k must be >= 1");
+  if (d->y_route) TNX_REQUIRE(d->topk_w && d->k >= 1, "norm_lora: y_route needs topk_w and k >= 1");
+  const int in = d->ws ? kNormInPlanes : d->y_route ? kNormInRoutes : kNormInRow;
+  const int parts = d->ws ? d->split_k : d->y_route ? d->k : 0;
+  const NormRow n{d->y_route ? d->y_route : d->x, d->res_pre, d->h_out, d->w, d->res_post, d->y, D, d->eps, d->ws, parts, M * D, d->w2, d->y2, d->topk_w};
+  // A row's work-groups read it while the first of them writes: no output may lie in an input.
+  auto apart = [&](const void* out, const void* p, int64_t bytes) {
+    const char *o = (const char*)out, *q = (const char*)p;
+    return !o || !q || o + M * D * 2 <= q || q + bytes <= o;
+  };
+  bool separate = true;
+  for (const void* out : {(const void*)d->h_out, (const void*)d->y, (const void*)d->y2})
+    separate = separate && apart(out, d->x, M * D * 2) && apart(out, d->ws, parts * M * D * 4) && apart(out, d->y_route, parts * M * D * 2) &&
+               apart(out, d->res_pre, M * D * 2) && apart(out, d->res_post, M * D * 2);
+  if (separate && norm_lora_one_launch(M, D, d->R)) {
+    launch_rmsnorm_lora(as_stream(stream), M, d->flavor, in, n, RowAdapterArgs{d->a_t, d->R, row_adapter_cols(M, d->R), d->t, d->t_ld});
+    TNX_CHECK_LAUNCH("norm_lora");
+    return TNX_OK;
+  }
+  launch_rmsnorm_vec(as_stream(stream), M, d->flavor, in, n);
+  TNX_CHECK_LAUNCH("norm_lora");
+  return tnx_lora_down(stream, d->w2 ? d->y2 : d->y, M, D, d->a_t, d->R, d->t, d->t_ld);
 }
 
 extern "C" int tnx_rope_table(void* stream, const int32_t* positions, int64_t pos_ld, const int32_t* col_ptr,

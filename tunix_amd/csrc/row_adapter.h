@@ -1,0 +1,92 @@
+// The LoRA down-projection of a row that a work-group already holds: t[row, col0 .. col0 + n) = bf16(x[row] . A^T) by 256 threads, of
+// which thread i owns the 8-element chunks i, i + 256, ... of the bf16 row x in registers, as the norm and the attention combine leave it.
+//
+// A decode batch's down-projection as a launch of its own is a launch gap, a round trip for its operands and a reduction: 3.9-5 us, whatever
+// its size.  Behind the kernel that produces x it costs the product alone: the row's work-groups (one per group of `nc` adapter columns)
+// each form the row, redundantly, from operands that the L2 holds, and ask for their first columns of A before they wait for them.
+// What bounds it is the bytes of a work-group ((partial planes + nc * 2) * K at some 110 GB/s per compute unit): row_adapter_cols takes groups
+// that give every compute unit one work-group.  Measured: norm_rope.hip (tnx_norm_lora) and attention.hip (tnx_gqa_attn_lora).
+#pragma once
+#include "common.h"
+
+namespace {
+
+// sum of eight values over the wave's 64 lanes: lane l ends with the sum of value l / 8 of the eight
+__device__ __forceinline__ float wave_sum8(float (&v)[8], int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {   // the lower half takes values 0-3, the upper 4-7
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 4]), false, false);
+    v[i] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 2]), false, false);
+    v[i] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  }
+  const bool up = lane & 8;
+  float s = (up ? v[1] : v[0]) + lane_xor<8>(up ? v[0] : v[1]);
+  s += lane_xor<4>(s);
+  s += lane_xor<2>(s);
+  return s + lane_xor<1>(s);
+}
+
+struct RowAdapterArgs {
+  const uint16_t* a_t;   // bf16 [R, K]
+  int R, nc;             // adapter columns, and how many of them a work-group takes
+  uint16_t* t;
+  int64_t t_ld;
+};
+template <int MAXC, int NB>
+struct RowAdapter {   // NB: adapter columns of a work-group at most, all asked for at once (NB * MAXC loads of 16 bytes per thread)
+  u32x4 a[NB][MAXC];
+  int ncols;
+  // (columns past the last one repeat it, chunks past the row's end repeat its last one: their products are dropped)
+  __device__ __forceinline__ void load(const RowAdapterArgs& g, int group, int64_t K) {
+    const int nchunks = (int)(K / 8);
+    const uint16_t* base = g.a_t + (int64_t)group * g.nc * K;
+    ncols = min(g.nc, g.R - group * g.nc);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int c = 0; c < MAXC; ++c)
+        a[i][c] = *reinterpret_cast<const u32x4*>(base + (int64_t)min(i, ncols - 1) * K + (int64_t)min(c * 256 + (int)threadIdx.x, nchunks - 1) * 8);
+  }
+  // x: the thread's chunks of the row (zeros past its end); red: 4 * NB floats of LDS
+  __device__ __forceinline__ void finish(const RowAdapterArgs& g, int group, int64_t row, const u32x4 (&x)[MAXC], float* red) {
+    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int b = 0; b < NB; b += 8) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[i] = 0.f;
+#pragma unroll
+        for (int c = 0; c < MAXC; ++c)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t xq = x[c][q], aq = a[b + i][c][q];   // (a bit cast applied to the vector element itself reads element 0)
+            v[i] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, xq), __builtin_bit_cast(bf2, aq), v[i], false);
+          }
+      }
+      const float s = wave_sum8(v, lane);
+      if ((lane & 7) == 0) red[wave * NB + b + (lane >> 3)] = s;
+    }
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (i < ncols) {
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) s += red[w * NB + i];
+      g.t[row * g.t_ld + (int64_t)group * g.nc + i] = f2bf(s);
+    }
+  }
+};
+
+// Columns per work-group: whole batches of eight, as few as leave at most one work-group per compute unit.
+inline int row_adapter_cols(int64_t M, int R) {
+  const int64_t groups = M >= 256 ? 1 : 256 / M;
+  return (int)(cdiv(cdiv(R, groups), 8) * 8);
+}
+
+}  // namespace

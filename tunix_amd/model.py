@@ -522,7 +522,10 @@ class Runner(HeadRunner):
     D, F = cfg.embed_dim, cfg.hidden_dim
     nqkv = cfg.q_dim + 2 * cfg.kv_dim
     rp = _pad32(cfg.lora_rank)
+    # the residual stream and the buffer its next sum goes to (they trade places: a norm that shares a row among
+    # work-groups must not write where another of them reads)
     self.h = torch.empty(M, D, dtype=bf, device=dev)
+    self.h_next = torch.empty(M, D, dtype=bf, device=dev) if M <= 256 else self.h
     self.xn = torch.empty(M, D, dtype=bf, device=dev)
     self.tmp = torch.empty(M, D, dtype=bf, device=dev)
     self.qkv = torch.empty(M, nqkv, dtype=bf, device=dev)
@@ -629,27 +632,43 @@ class Runner(HeadRunner):
             and epilogue in (L.TNX_EPI_SILU_MUL, L.TNX_EPI_GELU_MUL) and (f.N // 2) % 8 == 0
             and self.next_tpart is not None)
 
-  def norm_after(self, pending: int, w, M):
+  def norm_after(self, pending: int, w, M, a_t=None, t=None) -> bool:
     """self.xn = norm(self.h) -- or, with the partial planes of a deferred linear pending,
-    self.h += bf16(sum of planes) first (the linear's residual epilogue) in the same kernel."""
+    self.h += bf16(sum of planes) first (the linear's residual epilogue) in the same kernel.  With a_t, t = self.xn . a_t^T
+    as well (the adapter's down-projection ahead of the next linear, or the router): returns whether it is there."""
     cfg = self.cfg
-    flavor = _NORM[cfg.family]
+    flavor, D = _NORM[cfg.family], cfg.embed_dim
     if pending == _MOE_PENDING:   # h += the weighted combine of the routed rows, in the same kernel
-      ops.rmsnorm_moe_combine(self.y_route, self.topk_w, cfg.num_experts_per_tok, w, self.xn, cfg.norm_eps,
-                              flavor, M, cfg.embed_dim, res_pre=self.h, h_out=self.h)
+      k = cfg.num_experts_per_tok
+      src, two = dict(y_route=self.y_route, topk_w=self.topk_w, k=k), lambda: ops.rmsnorm_moe_combine(
+          self.y_route, self.topk_w, k, w, self.xn, cfg.norm_eps, flavor, M, D, res_pre=self.h, h_out=self.h)
     elif pending > 1:
-      ops.rmsnorm_splitk(self.splitk_ws, pending, w, self.xn, cfg.norm_eps, flavor, M, cfg.embed_dim,
-                         res_pre=self.h, h_out=self.h)
+      src, two = dict(ws=self.splitk_ws, split_k=pending), lambda: ops.rmsnorm_splitk(
+          self.splitk_ws, pending, w, self.xn, cfg.norm_eps, flavor, M, D, res_pre=self.h, h_out=self.h)
     else:
-      ops.rmsnorm(self.h, w, self.xn, cfg.norm_eps, flavor, M=M)
+      src, two = dict(x=self.h), lambda: ops.rmsnorm(self.h, w, self.xn, cfg.norm_eps, flavor, M=M)
+    if a_t is None or D % 32:
+      two()
+      return False
+    if "x" not in src:
+      src.update(res_pre=self.h, h_out=self.h_next)
+    ops.norm_lora(a_t, t, w, self.xn, cfg.norm_eps, flavor, M, D, **src)
+    if "x" not in src:
+      self.h, self.h_next = self.h_next, self.h
+    return True
 
-  def norm_pair(self, pending: int, w, w2, M):
+  def norm_pair(self, pending: int, w, w2, M, a_t=None) -> bool:
     """self.h += norm(self.tmp) . w (self.tmp = a linear's output, or its `pending` partial planes);
-    self.xn = norm(self.h) . w2 -- Gemma-3's post-norm + residual + next pre-norm in one launch."""
+    self.xn = norm(self.h) . w2 -- Gemma-3's post-norm + residual + next pre-norm in one launch; a_t: as in `norm_after`, into self.t."""
     cfg = self.cfg
     kw = dict(ws=self.splitk_ws, split_k=pending) if pending > 1 else dict(x=self.tmp)
-    ops.rmsnorm_pair(w, self.h, w2, self.xn, cfg.norm_eps, _NORM[cfg.family], M, cfg.embed_dim,
-                     res_post=self.h, **kw)
+    if a_t is None or cfg.embed_dim % 32:
+      ops.rmsnorm_pair(w, self.h, w2, self.xn, cfg.norm_eps, _NORM[cfg.family], M, cfg.embed_dim,
+                       res_post=self.h, **kw)
+      return False
+    ops.norm_lora(a_t, self.t, w, self.h_next, cfg.norm_eps, _NORM[cfg.family], M, cfg.embed_dim, res_post=self.h, w2=w2, y2=self.xn, **kw)
+    self.h, self.h_next = self.h_next, self.h
+    return True
 
   def forward_hidden(self, tokens, positions, col_ptr, cache, B=None, T=None, segment_ids=None, starts=None):
     """Runs all layers for tokens[b, col .. col+T) of each row; leaves the final-normed hidden
@@ -672,12 +691,14 @@ class Runner(HeadRunner):
       # one table of this step's sines / cosines for all layers (they share theta)
       ops.rope_table(positions, col_ptr, B, m.layers[0]["timescale"], cfg.head_dim, self.rope_sin, self.rope_cos)
     xn_ready = False   # gemma3: the block before has already normed the residual stream into self.xn
+    t_ready = False    # ... and formed the qkv adapters' down-projection of it
+    adapter = lambda f: f.a_t if f.has_lora else None
     for i, ly in enumerate(m.layers):
       kv = cache.entries[i]
       if not xn_ready:
-        self.norm_after(pending, ly["attn_norm"], M)
+        t_ready = self.norm_after(pending, ly["attn_norm"], M, adapter(ly["qkv"]), self.t)
       pending, xn_ready = 1, False
-      qkv_split = self.linear(ly["qkv"], self.xn, self.qkv, M, defer=True)
+      qkv_split = self.linear(ly["qkv"], self.xn, self.qkv, M, defer=True, t_ready=t_ready)
       # decode step of a model without q/k norm and with the Llama rotation: the attention kernel
       # rotates q / k and writes the cache itself, and the stand-alone launch is dropped
       fuse_rope = (T == 1 and "q_norm" not in ly and _ROPE[cfg.family] == L.TNX_ROPE_LLAMA
@@ -719,39 +740,46 @@ class Runner(HeadRunner):
         else:
           ad.qkv = self.qkv.data_ptr()
         ad.rope_sin, ad.rope_cos = self.rope_sin.data_ptr(), self.rope_cos.data_ptr()
-      ops.gqa_attn(ad)
+      if ly["o"].has_lora:
+        ops.gqa_attn_lora(ad, ly["o"].a_t, self.t)
+      else:
+        ops.gqa_attn(ad)
+      mlp_adapter = None if cfg.num_experts else adapter(ly["gu"])
       if cfg.family == "gemma3":
         # h += post_attn_norm(o_proj); xn = mlp_norm(h): one launch, which also sums the
         # projection's partial planes when it ran split
-        po = self.linear(ly["o"], self.attn, self.tmp, M, defer=True)
-        self.norm_pair(po, ly["post_attn_norm"], ly["mlp_norm"], M)
+        po = self.linear(ly["o"], self.attn, self.tmp, M, defer=True, t_ready=True)
+        gu_ready = self.norm_pair(po, ly["post_attn_norm"], ly["mlp_norm"], M, mlp_adapter)
       else:
         po = self.linear(ly["o"], self.attn, self.h, M, epilogue=L.TNX_EPI_RESIDUAL, residual=self.h,
-                         defer=True)
-        self.norm_after(po, ly["mlp_norm"], M)
+                         defer=True, t_ready=True)
+        gu_ready = (self.norm_after(po, ly["mlp_norm"], M, ly["experts"].router_t, self.scores) if cfg.num_experts
+                    else self.norm_after(po, ly["mlp_norm"], M, mlp_adapter, self.t))
       if cfg.num_experts:
-        pending = self._moe(ly["experts"], M)
+        pending = self._moe(ly["experts"], M, gu_ready)
       elif cfg.family == "gemma3":
         fused = self.fuses_next(ly["gu"], ly["down"], M, L.TNX_EPI_GELU_MUL)
-        self.linear(ly["gu"], self.xn, self.act, M, epilogue=L.TNX_EPI_GELU_MUL, next_f=ly["down"])
+        self.linear(ly["gu"], self.xn, self.act, M, epilogue=L.TNX_EPI_GELU_MUL, next_f=ly["down"], t_ready=gu_ready)
         pd = self.linear(ly["down"], self.act, self.tmp, M, t_ready=fused, defer=True)
         # h += post_ffw_norm(down_proj); xn = the next block's attn_norm (or the final norm) of h
-        nxt = m.layers[i + 1]["attn_norm"] if i + 1 < len(m.layers) else m.final_norm
-        self.norm_pair(pd, ly["post_ffw_norm"], nxt, M)
+        last = i + 1 == len(m.layers)
+        nxt = m.final_norm if last else m.layers[i + 1]["attn_norm"]
+        t_ready = self.norm_pair(pd, ly["post_ffw_norm"], nxt, M, None if last else adapter(m.layers[i + 1]["qkv"]))
         xn_ready = True
       else:
         fused = self.fuses_next(ly["gu"], ly["down"], M, L.TNX_EPI_SILU_MUL)
-        self.linear(ly["gu"], self.xn, self.act, M, epilogue=L.TNX_EPI_SILU_MUL, next_f=ly["down"])
+        self.linear(ly["gu"], self.xn, self.act, M, epilogue=L.TNX_EPI_SILU_MUL, next_f=ly["down"], t_ready=gu_ready)
         pending = self.linear(ly["down"], self.act, self.h, M, epilogue=L.TNX_EPI_RESIDUAL,
                               residual=self.h, defer=True, t_ready=fused)
     if not xn_ready:
       self.norm_after(pending, m.final_norm, M)
     return self.xn
 
-  def _moe(self, ex: ExpertBank, M: int) -> int:
+  def _moe(self, ex: ExpertBank, M: int, scored: bool) -> int:
     cfg = self.cfg
     k, E = cfg.num_experts_per_tok, cfg.num_experts
-    ops.lora_down(self.xn, ex.router_t, self.scores, M=M)          # dense bf16 router
+    if not scored:
+      ops.lora_down(self.xn, ex.router_t, self.scores, M=M)          # dense bf16 router
     ops.moe_route_topk(self.scores[:M], k, self.topk_w, self.topk_id)
     ops.moe_sort_routes(self.topk_id[:M], E, self.counts, self.offsets, self.sorted_route)
     d = L.MoeGmmDesc()

@@ -171,6 +171,18 @@ def rmsnorm_pair(w, y, w2, y2, eps, flavor, M, D, x=None, ws=None, split_k=0, re
                                    flavor), "tnx_rmsnorm_pair")
 
 
+def norm_lora(a_t, t, w, y, eps, flavor, M, D, x=None, ws=None, split_k=0, y_route=None, topk_w=None, k=0, res_pre=None, h_out=None,
+              res_post=None, w2=None, y2=None):
+  """rmsnorm (x), rmsnorm_splitk (ws), rmsnorm_moe_combine (y_route) or, with w2, rmsnorm_pair, and lora_down of what it writes."""
+  d = L.NormLoraDesc()
+  d.M, d.D, d.eps, d.flavor, d.split_k, d.k = M, D, float(eps), flavor, split_k, k
+  d.x, d.ws, d.y_route, d.topk_w = _ptr(x), _ptr(ws), _ptr(y_route), _ptr(topk_w)
+  d.res_pre, d.h_out, d.w, d.res_post, d.y = _ptr(res_pre), _ptr(h_out), _ptr(w), _ptr(res_post), _ptr(y)
+  d.w2, d.y2 = _ptr(w2), _ptr(y2)
+  d.a_t, d.R, d.t, d.t_ld = _ptr(a_t), a_t.shape[0], _ptr(t), t.shape[1]
+  L.check(L.lib().tnx_norm_lora(_stream(), C.byref(d)), "tnx_norm_lora")
+
+
 def rope_kvwrite(desc: L.RopeDesc):
   L.check(L.lib().tnx_qknorm_rope_kvwrite(_stream(), C.byref(desc)), "tnx_qknorm_rope_kvwrite")
 
@@ -186,6 +198,11 @@ def attn_ws_bytes(B, T, S, Hq, dh, kv_chunk) -> int:
 
 def gqa_attn(desc: L.AttnDesc):
   L.check(L.lib().tnx_gqa_attn(_stream(), C.byref(desc)), "tnx_gqa_attn")
+
+
+def gqa_attn_lora(desc: L.AttnDesc, a_t, t):
+  """gqa_attn and lora_down of its output rows."""
+  L.check(L.lib().tnx_gqa_attn_lora(_stream(), C.byref(desc), _ptr(a_t), a_t.shape[0], _ptr(t), t.shape[1]), "tnx_gqa_attn_lora")
 
 
 def lmhead_nblocks(V: int) -> int:
