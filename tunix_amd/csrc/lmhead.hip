@@ -176,13 +176,13 @@ __global__ __launch_bounds__(DENSE && NT == 2 ? 512 : 256) void lmhead_kernel(co
       // arg-max over the 16 lanes of the row (columns grow with lm)
 #pragma unroll
       for (int o = 1; o < 16; o <<= 1) {
-        const float omx = __shfl_xor(mx, o, 64);
-        const int oidx = __shfl_xor(idx, o, 64);
+        const float omx = lane_xor(mx, o);
+        const int oidx = lane_xor(idx, o);
         if (omx > mx || (omx == mx && oidx < idx)) {
           mx = omx;
           idx = oidx;
         }
-        tgt = fmaxf(tgt, __shfl_xor(tgt, o, 64));
+        tgt = fmaxf(tgt, lane_xor(tgt, o));
       }
       float se = 0.f, we = 0.f;
       if (mx != kNegInf) {
@@ -195,8 +195,8 @@ __global__ __launch_bounds__(DENSE && NT == 2 ? 512 : 256) void lmhead_kernel(co
       }
 #pragma unroll
       for (int o = 1; o < 16; o <<= 1) {
-        se += __shfl_xor(se, o, 64);
-        we += __shfl_xor(we, o, 64);
+        se += lane_xor(se, o);
+        we += lane_xor(we, o);
       }
       // the draw: arg-max of logit + gumbel noise over this row's columns in the wave
       // (noise of element (row, v): counter row * V + v of M * V, one draw over [M, V])
@@ -216,8 +216,8 @@ __global__ __launch_bounds__(DENSE && NT == 2 ? 512 : 256) void lmhead_kernel(co
         }
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) {
-          const float ov = __shfl_xor(gv, o, 64), ol = __shfl_xor(gl, o, 64);
-          const int oi = __shfl_xor(gi, o, 64);
+          const float ov = lane_xor(gv, o), ol = lane_xor(gl, o);
+          const int oi = lane_xor(gi, o);
           if (ov > gv || (ov == gv && oi < gi)) {
             gv = ov;
             gi = oi;
@@ -264,46 +264,67 @@ __global__ __launch_bounds__(DENSE && NT == 2 ? 512 : 256) void lmhead_kernel(co
   }
 }
 
-// One wave per row merges the per-block statistics in column order.
-__global__ __launch_bounds__(64) void lmhead_finish_kernel(const float* part, int64_t nvb,
-                                                           int32_t* best_id, float* best_logp,
-                                                           float* target_logp, float* lse_out,
-                                                           const float* part_ent, float* entropy_out,
-                                                           const float* part_draw, int32_t* draw_id,
-                                                           float* draw_logp) {
+// A row's per-block statistics merged by one work-group, whose threads read them side by side, four blocks in flight each.
+// (One wave per row, each lane a run of neighbouring blocks one after the other: 16 rows x 1002 blocks 8.1 us, 8192 rows 185 us.)
+__global__ __launch_bounds__(256) void lmhead_finish_kernel(const float* part, int64_t nvb, int32_t* best_id, float* best_logp, float* target_logp,
+                                                            float* lse_out, const float* part_ent, float* entropy_out, const float* part_draw,
+                                                            int32_t* draw_id, float* draw_logp) {
+  typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
+  __shared__ Stat waves[4];
   const int64_t row = blockIdx.x;
-  const int lane = threadIdx.x;
-  const float* p = part + row * nvb * 4;
-  // lane l owns the contiguous block range [l*per, (l+1)*per): merges stay in column order
-  const int64_t per = (nvb + 63) / 64;
+  const int tid = threadIdx.x, T = blockDim.x;
+  const float *p = part + row * nvb * 4, *pe = part_ent ? part_ent + row * nvb : nullptr, *pd = part_draw ? part_draw + row * nvb * 3 : nullptr;
+  // (the columns come in any order: among equal maxima the lowest wins; a block without one, -inf, has no column)
+  auto merge_any = [](const Stat& a, const Stat& b) {
+    Stat r = merge(a, b);
+    if (b.mx == a.mx && b.idx < a.idx && b.mx > kNegInf) r.idx = b.idx;
+    return r;
+  };
   Stat r;
   r.mx = kNegInf; r.idx = 0x7fffffff; r.sum = 0.f; r.tgt = kNegInf; r.wsum = 0.f;
   r.gv = kNegInf; r.gi = 0x7fffffff; r.gl = kNegInf;
-  for (int64_t c = lane * per; c < min(nvb, (lane + 1) * per); ++c) {
-    Stat b;
-    b.mx = p[c * 4]; b.idx = __float_as_int(p[c * 4 + 1]); b.sum = p[c * 4 + 2]; b.tgt = p[c * 4 + 3];
-    b.wsum = part_ent ? part_ent[row * nvb + c] : 0.f;
-    b.gv = kNegInf; b.gi = 0x7fffffff; b.gl = kNegInf;
-    if (part_draw) {
-      const float* q = part_draw + (row * nvb + c) * 3;
-      b.gv = q[0]; b.gi = __float_as_int(q[1]); b.gl = q[2];
+  for (int64_t c0 = tid; c0 < nvb; c0 += 4 * T) {
+    f32x4 v[4];
+    float e[4], d[4][3];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t c = min(c0 + u * T, nvb - 1);
+      v[u] = *reinterpret_cast<const f32x4a*>(p + c * 4);
+      e[u] = pe ? pe[c] : 0.f;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) d[u][k] = pd ? pd[c * 3 + k] : 0.f;
     }
-    r = merge(r, b);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (c0 + u * T < nvb) {
+        Stat b;
+        const float idx = v[u][1], gi = d[u][1];   // (a bit cast applied to the vector element itself reads element 0)
+        b.mx = v[u][0]; b.idx = __float_as_int(idx); b.sum = v[u][2]; b.tgt = v[u][3];
+        b.wsum = e[u];
+        b.gv = pd ? d[u][0] : kNegInf; b.gi = pd ? __float_as_int(gi) : 0x7fffffff; b.gl = pd ? d[u][2] : kNegInf;
+        r = merge_any(r, b);
+      }
   }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     Stat b;
-    b.mx = __shfl_xor(r.mx, o, 64);
-    b.idx = __shfl_xor(r.idx, o, 64);
-    b.sum = __shfl_xor(r.sum, o, 64);
-    b.tgt = __shfl_xor(r.tgt, o, 64);
-    b.wsum = __shfl_xor(r.wsum, o, 64);
-    b.gv = __shfl_xor(r.gv, o, 64);
-    b.gi = __shfl_xor(r.gi, o, 64);
-    b.gl = __shfl_xor(r.gl, o, 64);
-    r = (lane & o) ? merge(b, r) : merge(r, b);  // the lower lane holds the lower columns
+    b.mx = lane_xor(r.mx, o);
+    b.idx = lane_xor(r.idx, o);
+    b.sum = lane_xor(r.sum, o);
+    b.tgt = lane_xor(r.tgt, o);
+    b.wsum = lane_xor(r.wsum, o);
+    b.gv = lane_xor(r.gv, o);
+    b.gi = lane_xor(r.gi, o);
+    b.gl = lane_xor(r.gl, o);
+    r = merge_any(r, b);
   }
-  if (lane == 0) {
+  if (T > 64) {
+    if ((tid & 63) == 0) waves[tid >> 6] = r;
+    __syncthreads();
+    for (int w = 1; w < (T >> 6); ++w)
+      if (tid == 0) r = merge_any(r, waves[w]);
+  }
+  if (tid == 0) {
     const float lse = r.mx + logf(r.sum);
     if (best_id) best_id[row] = r.idx;
     if (best_logp) best_logp[row] = r.mx - lse;
@@ -396,7 +417,7 @@ extern "C" int tnx_lmhead_logp(void* stream, const tnx_lmhead_desc* d) {
     else rc = dense ? launch_lmhead<8, true>(st, a) : launch_lmhead<8, false>(st, a);
   }
   if (rc) return rc;
-  hipLaunchKernelGGL(lmhead_finish_kernel, dim3((unsigned)d->M), dim3(64), 0, st, a.part, a.nvb,
+  hipLaunchKernelGGL(lmhead_finish_kernel, dim3((unsigned)d->M), dim3(a.nvb <= 64 ? 64 : 256), 0, st, a.part, a.nvb,
                      d->best_id, d->best_logp, d->target_logp, d->lse, a.part_ent, d->entropy, a.part_draw,
                      d->draw_id, d->draw_logp);
   TNX_CHECK_LAUNCH("lmhead_finish");
