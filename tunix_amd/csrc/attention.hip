@@ -672,8 +672,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         sv[s] = x;
         if (kvalid[s]) bmax = fmaxf(bmax, x);
       }
-      bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
-      bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
+      bmax = fmaxf(bmax, lane_xor(bmax, 16));
+      bmax = fmaxf(bmax, lane_xor(bmax, 32));
       const float m_new = fmaxf(m_run[w], bmax);
       const float alpha = __expf(m_run[w] - m_new);
       m_run[w] = m_new;
@@ -747,8 +747,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
     float lr = l_run[w];
-    lr += __shfl_xor(lr, 16, 64);
-    lr += __shfl_xor(lr, 32, 64);
+    lr += lane_xor(lr, 16);
+    lr += lane_xor(lr, 32);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = 4 * lq + i;
@@ -881,8 +881,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    lo_max = max(lo_max, __shfl_xor(lo_max, o, 64));
-    hi_min = min(hi_min, __shfl_xor(hi_min, o, 64));
+    lo_max = max(lo_max, lane_xor(lo_max, o));
+    hi_min = min(hi_min, lane_xor(hi_min, o));
   }
   lo_max = __builtin_amdgcn_readfirstlane(full ? lo_max : 0x7fffffff);
   hi_min = __builtin_amdgcn_readfirstlane(hi_min);

@@ -174,19 +174,32 @@ __device__ __forceinline__ u32x4 dequant8_scaled(uint32_t w, const uint32_t* lut
   return r;
 }
 
-// Lane l gets lane l ^ X's value, X = 1, 2, 4 or 8, by DPP (two of them for 4: l ^ 7 ^ 3): some eight cycles where the exchange through
-// LDS that __shfl_xor is takes a hundred.
-template <int CTRL>
-__device__ __forceinline__ float lane_dpp(float v) {
-  return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), CTRL, 0xf, 0xf, false));
+// Lane l gets lane (l ^ o)'s value, o a power of two that is a constant once the loop around the call is unrolled: by DPP within a row of
+// 16 lanes (two of them for 4: l ^ 7 ^ 3) and by the row and half swaps beyond it, some eight cycles where the exchange through LDS that __shfl_xor
+// is takes a hundred.
+template <int CTRL, class T>
+__device__ __forceinline__ T lane_dpp(T v) {
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0u, __builtin_bit_cast(uint32_t, v), CTRL, 0xf, 0xf, false));
 }
-template <int X>
-__device__ __forceinline__ float lane_xor(float v) {
-  static_assert(X == 1 || X == 2 || X == 4 || X == 8, "within a row of 16 lanes");
-  if constexpr (X == 1) return lane_dpp<0xb1>(v);                    // quad_perm 1 0 3 2
-  else if constexpr (X == 2) return lane_dpp<0x4e>(v);               // quad_perm 2 3 0 1
-  else if constexpr (X == 4) return lane_dpp<0x1b>(lane_dpp<0x141>(v));   // half mirror, quad_perm 3 2 1 0
-  else return lane_dpp<0x128>(v);                                    // row rotation by 8
+template <class T>
+__device__ __forceinline__ T lane_xor(T v, int o) {
+  static_assert(sizeof(T) == 4, "a register");
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  switch (o) {
+    case 1: return lane_dpp<0xb1>(v);                   // quad_perm 1 0 3 2
+    case 2: return lane_dpp<0x4e>(v);                   // quad_perm 2 3 0 1
+    case 4: return lane_dpp<0x1b>(lane_dpp<0x141>(v));  // half mirror, quad_perm 3 2 1 0
+    case 8: return lane_dpp<0x128>(v);                  // row rotation by 8
+    case 16: {
+      const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+      return __builtin_bit_cast(T, (uint32_t)(lane & 16 ? s[0] : s[1]));
+    }
+    default: {
+      const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      return __builtin_bit_cast(T, (uint32_t)(lane & 32 ? s[0] : s[1]));
+    }
+  }
 }
 // f over the wave's 64 lanes, in all of them, by halves: 32, 16, 8, 4, 2, 1 lanes apart (f commutes, and a kernel that calls it has whole waves).
 // A norm of a decode step is a chain of round trips of which this was one: with the down-projection behind it 16 rows of 4096 from eight planes
@@ -197,16 +210,40 @@ __device__ __forceinline__ float wave_all(float v, F f) {
   v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
   const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   v = f(__uint_as_float(b[0]), __uint_as_float(b[1]));
-  v = f(v, lane_xor<8>(v));
-  v = f(v, lane_xor<4>(v));
-  v = f(v, lane_xor<2>(v));
-  return f(v, lane_xor<1>(v));
+  v = f(v, lane_xor(v, 8));
+  v = f(v, lane_xor(v, 4));
+  v = f(v, lane_xor(v, 2));
+  return f(v, lane_xor(v, 1));
 }
 __device__ __forceinline__ float wave_sum(float v) {
   return wave_all(v, [](float x, float y) { return x + y; });
 }
 __device__ __forceinline__ float wave_max(float v) {
   return wave_all(v, [](float x, float y) { return fmaxf(x, y); });
+}
+
+// The k largest of a wave's values v[i], of index lane + 64 i, descending, the lowest index first among equals: pick(j, index, value) for each, the
+// same in every lane.  Values lie above -inf, which marks a place without one and a value taken.
+template <int N, class F>
+__device__ __forceinline__ void wave_largest(float (&v)[N], int k, F pick) {
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  for (int j = 0; j < k; ++j) {
+    float best = v[0];
+#pragma unroll
+    for (int i = 1; i < N; ++i) best = fmaxf(best, v[i]);
+    best = wave_max(best);
+    int id = -1;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const uint64_t at = __builtin_amdgcn_ballot_w64(v[i] == best);
+      if (id < 0 && at) {   // (uniform)
+        const int l = __builtin_ctzll(at);
+        id = l + 64 * i;
+        if (lane == l) v[i] = -__builtin_inff();
+      }
+    }
+    pick(j, id, best);
+  }
 }
 
 // cap * tanh(z / cap) with an absolute error of a few ulp of cap

@@ -1220,9 +1220,9 @@ int launch_act_mul(hipStream_t st, int dtype, const void* y, int64_t ld, int64_t
 // ---- choice of experts: the k largest logits (first among equals), softmax over them ---------------
 // One wave per token.  NaN logits rank below every number, so that k distinct experts are found whatever
 // the logits hold; they leave as NaN weights.
-// Up to 256 experts: every expert counts the ones ahead of it, which is its place among the chosen; more: one
-// pass over the logits per choice.
-constexpr int kRankExperts = 256;
+// Up to 256 experts: they stay in registers, a choice is a maximum over the wave and ballots; more: one pass over the logits
+// per choice.
+constexpr int kRegisterExperts = 256;
 __global__ __launch_bounds__(64) void route_softmax_kernel(const RowSrc<float> src, int E, int k, float* topk_w, int32_t* topk_id) {
   extern __shared__ __align__(16) float z[];   // logits [E], chosen logits [k]
   float* sel = z + E;
@@ -1237,25 +1237,19 @@ __global__ __launch_bounds__(64) void route_softmax_kernel(const RowSrc<float> s
   }
   bad = __any(bad);
   __syncthreads();
-  if (E <= kRankExperts) {   // (uniform)
-    for (int e = lane; e < E; e += 64) {
-      const float v = z[e];
-      int ahead = 0;
-      int o = 0;
-      for (; o + 4 <= E; o += 4) {
-        const f32x4 w = *reinterpret_cast<const f32x4*>(z + o);
+  if (E <= kRegisterExperts) {   // (uniform)
+    float c[kRegisterExperts / 64];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ahead += w[i] > v || (w[i] == v && o + i < e);
+    for (int i = 0; i < kRegisterExperts / 64; ++i) c[i] = lane + 64 * i < E ? z[lane + 64 * i] : ninf;
+    wave_largest(c, k, [&](int j, int id, float best) {
+      if (lane == 0) {
+        sel[j] = best;
+        topk_id[m * k + j] = id;
       }
-      for (; o < E; ++o) ahead += z[o] > v || (z[o] == v && o < e);
-      if (ahead < k) {
-        sel[ahead] = v;
-        topk_id[m * k + ahead] = e;
-      }
-    }
+    });
     __syncthreads();
   }
-  for (int j = 0; j < k && E > kRankExperts; ++j) {
+  for (int j = 0; j < k && E > kRegisterExperts; ++j) {
     float best = ninf;
     int bi = 0x7fffffff;
     for (int e = lane; e < E; e += 64)
@@ -1265,8 +1259,8 @@ __global__ __launch_bounds__(64) void route_softmax_kernel(const RowSrc<float> s
       }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const float ob = __shfl_xor(best, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
+      const float ob = lane_xor(best, o);
+      const int oi = lane_xor(bi, o);
       if (ob > best || (ob == best && oi < bi)) {
         best = ob;
         bi = oi;
@@ -1310,7 +1304,7 @@ __device__ __forceinline__ Best better(Best a, Best b) {   // larger value, then
 }
 __device__ __forceinline__ Best block_best(Best v, Best* red) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = better(v, Best{__shfl_xor(v.v, o, 64), __shfl_xor(v.i, o, 64)});
+  for (int o = 32; o > 0; o >>= 1) v = better(v, Best{lane_xor(v.v, o), lane_xor(v.i, o)});
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();

@@ -370,8 +370,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       sc[i] = key >= k_lo && key <= cn ? (st[0][i] + st[1][i]) * sc2 : -__builtin_inff();
       mx = fmaxf(mx, sc[i]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = fmaxf(mx, lane_xor(mx, 16));
+    mx = fmaxf(mx, lane_xor(mx, 32));
     if (lq == 0) redm[kg * 32 + hq] = mx;
     __syncthreads();
     {
@@ -428,8 +428,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
   }
-  l16 += __shfl_xor(l16, 16, 64);
-  l16 += __shfl_xor(l16, 32, 64);
+  l16 += lane_xor(l16, 16);
+  l16 += lane_xor(l16, 32);
   if (lq == 0) redl[kg * 32 + hq] = l16;
   __syncthreads();
   const float l = redl[l32] + redl[32 + l32] + redl[64 + l32] + redl[96 + l32];

@@ -361,8 +361,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, KT <= 4 
 #pragma unroll
         for (int r = 0; r < 4; ++r) dot += bflo(qv[r]) * ns[d + 2 * r] + bfhi(qv[r]) * ns[d + 2 * r + 1];
       }
-      dot += __shfl_xor(dot, 1, 64);
-      dot += __shfl_xor(dot, 2, 64);
+      dot += lane_xor(dot, 1);
+      dot += lane_xor(dot, 2);
       if ((tid & 3) == 0) tq[tok] = dot;
       __syncthreads();
     }
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, KT <= 4 
             O[qt] = mfma32(al, vf, O[qt]);
           }
         }
-        rs += __shfl_xor(rs, 32, 64);
+        rs += lane_xor(rs, 32);
         if (lh == 0) td[tq_] = 1.0f / (fmaxf(fabsf(te[tq_] * tq[tq_] + rs), tf[tq_]) + kFloor);
       }
       if (dok)

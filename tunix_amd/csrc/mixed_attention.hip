@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4))) voi
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[hf][i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = fmaxf(mx, lane_xor(mx, 32));
     const float m_new = fmaxf(m_run, mx), alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
     float psum = 0.f;
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4))) voi
       for (int i = 0; i < 16; ++i) psum += exp2_hw(st[hf][i] - m_new);   // (exp2(-inf) = 0: a masked key)
     l_run = l_run * alpha + psum;
   }
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run += lane_xor(l_run, 32);
   if (qrow < rows && lh == 0) a.lse[(b * a.T + tq) * a.H + head] = l_run > 0.f ? m_run + __log2f(l_run) : -kNegBig;
 }
 
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, KS > 4 ? 
   // a head's four lanes
 #pragma unroll
   for (int o = 16; o < 64; o <<= 1) {
-    const float om = __shfl_xor(m, o, 64), ol = __shfl_xor(l, o, 64), mn = fmaxf(m, om);
+    const float om = lane_xor(m, o), ol = lane_xor(l, o), mn = fmaxf(m, om);
     l = l * exp2_hw(m - mn) + ol * exp2_hw(om - mn);
     m = mn;
   }
@@ -578,7 +578,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
       }
 #pragma unroll
     for (int o = 1; o < 4; o <<= 1) {
-      const float om = __shfl_xor(m, o, 64), ol = __shfl_xor(l, o, 64), mn = fmaxf(m, om);
+      const float om = lane_xor(m, o), ol = lane_xor(l, o), mn = fmaxf(m, om);
       l = l * exp2_hw(m - mn) + ol * exp2_hw(om - mn);
       m = mn;
     }

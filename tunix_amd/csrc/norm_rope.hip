@@ -606,7 +606,9 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(const RopeArgs a) {
       float ss = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += sq_term(x1[e], a.qk_norm) + sq_term(x2[e], a.qk_norm);
-      for (int o = CH / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1)
+        if (o <= CH / 2) ss += lane_xor(ss, o);
       const float ms = finish_ms(ss, (float)a.dh, a.qk_norm);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {

@@ -106,7 +106,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
     for (int base = 0; base < a.n_experts; base += 64) {
       int nb = blocks_of(base + lane);
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) nb += __shfl_xor(nb, o, 64);
+      for (int o = 32; o > 0; o >>= 1) nb += lane_xor(nb, o);
       total += nb;
     }
     const int tile = xcd_tile((int)blockIdx.x, total * tiles_n);

@@ -24,10 +24,10 @@ __device__ __forceinline__ float wave_sum8(float (&v)[8], int lane) {
     v[i] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
   }
   const bool up = lane & 8;
-  float s = (up ? v[1] : v[0]) + lane_xor<8>(up ? v[0] : v[1]);
-  s += lane_xor<4>(s);
-  s += lane_xor<2>(s);
-  return s + lane_xor<1>(s);
+  float s = (up ? v[1] : v[0]) + lane_xor(up ? v[0] : v[1], 8);
+  s += lane_xor(s, 4);
+  s += lane_xor(s, 2);
+  return s + lane_xor(s, 1);
 }
 
 struct RowAdapterArgs {

@@ -27,8 +27,8 @@ __device__ ArgMax block_argmax(ArgMax x, ArgMax* red) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     ArgMax y;
-    y.v = __shfl_xor(x.v, o, 64);
-    y.i = __shfl_xor(x.i, o, 64);
+    y.v = lane_xor(x.v, o);
+    y.i = lane_xor(x.i, o);
     x = better(x, y);
   }
   __syncthreads();
@@ -325,8 +325,8 @@ __global__ __launch_bounds__(kSegThreads) void topk_segment_kernel(
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       ArgMax y;
-      y.v = __shfl_xor(g.v, o, 64);
-      y.i = __shfl_xor(g.i, o, 64);
+      y.v = lane_xor(g.v, o);
+      y.i = lane_xor(g.i, o);
       g = better(g, y);
     }
     if (lane == 0) red_g[wave] = g;
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(kSegThreads) void topk_segment_kernel(
     for (int size = 2; size <= 64; size <<= 1)               // bitonic in the wave, descending
 #pragma unroll
       for (int st = size >> 1; st > 0; st >>= 1) {
-        const float y = __shfl_xor(lm, st, 64);
+        const float y = lane_xor(lm, st);
         const bool up = (lane & size) == 0, low = (lane & st) == 0;
         lm = (up == low) ? fmaxf(lm, y) : fminf(lm, y);
       }
@@ -638,7 +638,7 @@ __device__ void select_best(const float* v, int n, int k, IdxFn gi, float* cv, i
   for (int size = 2; size <= 64; size <<= 1)
 #pragma unroll
     for (int st = size >> 1; st > 0; st >>= 1) {
-      const float y = __shfl_xor(lm, st, 64);
+      const float y = lane_xor(lm, st);
       const bool up = (lane & size) == 0, low = (lane & st) == 0;
       lm = (up == low) ? fmaxf(lm, y) : fminf(lm, y);
     }
@@ -813,8 +813,8 @@ __global__ __launch_bounds__(kBlkThreads) void topk_blocks_sample_kernel(
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       ArgMax y;
-      y.v = __shfl_xor(g.v, o, 64);
-      y.i = __shfl_xor(g.i, o, 64);
+      y.v = lane_xor(g.v, o);
+      y.i = lane_xor(g.i, o);
       g = better(g, y);
     }
     if (lane == 0) {

@@ -200,8 +200,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
       if constexpr (BIAS) sv[s] = __builtin_fmaf(slope2, (float)(key - c_n), sv[s]);
       if (ok[s]) bmax = fmaxf(bmax, sv[s]);
     }
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
+    bmax = fmaxf(bmax, lane_xor(bmax, 16));
+    bmax = fmaxf(bmax, lane_xor(bmax, 32));
     const float m_new = fmaxf(m_run, bmax), alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
     float p[8], psum = 0.f;
@@ -252,8 +252,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
       }
     }
   }
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run += lane_xor(l_run, 16);
+  l_run += lane_xor(l_run, 32);
   // lane: queries 4 lq + i (i = 0..3), value columns h * 16 NJ + NJ lm + j
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -436,7 +436,7 @@ void sink_attn_tile_kernel(const SinkArgs a) {
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[hf][i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = fmaxf(mx, lane_xor(mx, 32));
     const float m_new = fmaxf(m_run, mx * factor);
     const float alpha = exp2_hw(m_run - m_new);
     m_run = m_new;
@@ -483,7 +483,7 @@ void sink_attn_tile_kernel(const SinkArgs a) {
       }
   }
   if (!qvalid) return;
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run += lane_xor(l_run, 32);
   const float w = finish_scale(m_run, l_run, a.sinks != nullptr, a.sinks ? a.sinks[head] : 0.f);
   // register 4 b + e of O[j]: value column NV (8 b + 4 lh + e) + j: runs of 4 NV columns
   uint16_t* out = reinterpret_cast<uint16_t*>(a.out);

@@ -78,8 +78,8 @@ __device__ __forceinline__ void wide_tile_out(const QLArgs& a, const WideHead& h
           }
 #pragma unroll
           for (int o = LANES / 2; o > 0; o >>= 1) {
-            const float ov = __shfl_xor(gv, o, 64), ol = __shfl_xor(gl, o, 64);
-            const int oi = __shfl_xor(gi, o, 64);
+            const float ov = lane_xor(gv, o), ol = lane_xor(gl, o);
+            const int oi = lane_xor(gi, o);
             if (ov > gv || (ov == gv && oi < gi)) {
               gv = ov;
               gi = oi;
