@@ -80,8 +80,8 @@ const char* tnx_last_error(void);
  * tnx_embed_rows, centred norms, a factor, an extra row and the depth average to tnx_residual_norm_desc, slopes and
  * chunks to tnx_sink_attn_desc, an ungated form and shared weights to tnx_gated_norm_desc, TNX_EPI_RELU2, and
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
- * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora and
- * tnx_gqa_attn_lora. */
+ * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora,
+ * tnx_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric. */
 #define TNX_ABI_VERSION_MAJOR 6
 #define TNX_ABI_VERSION_MINOR 3
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
@@ -531,6 +531,10 @@ int tnx_moe_combine(void* stream, const uint16_t* y, const uint16_t* topk_w, int
 int tnx_grpo_ratio(void* stream, const float* logp, const float* old_logp, const float* adv,
                    int64_t N, int64_t tokens_per_seq, float eps_lo, float eps_hi, float* ratio,
                    float* loss, int32_t* clipped);
+/* The same with the clipped flags as bytes. */
+int tnx_grpo_ratio_flags(void* stream, const float* logp, const float* old_logp, const float* adv,
+                         int64_t N, int64_t tokens_per_seq, float eps_lo, float eps_hi, float* ratio,
+                         float* loss, uint8_t* clipped);
 
 /* Per-token KL estimators between the trained and the reference policy
  * (tunix/rl/common.py:135-184): TNX_KL_KL logp - ref; TNX_KL_MSE 0.5 * (logp - ref)^2;
@@ -555,6 +559,11 @@ enum {
 };
 int tnx_aggregate_loss(void* stream, const float* per_token_loss, const float* mask, int64_t B, int64_t T,
                        int mode, float norm, float* row_ws, float* out);
+
+/* out = sum * s, s = 0 where d = denom [+ eps, where has_eps] [raised to min_denom, where has_min] is 0, else 1 / d (one value each):
+ * WeightedMetric.compute in one launch. */
+int tnx_weighted_metric(void* stream, const float* sum, const float* denom, int has_eps, float eps,
+                        int has_min, float min_denom, float* out);
 
 /* The same over packed batches (the segment branch, tunix/rl/common.py:857-940 with the segment
  * sums of :704-760): a row holds several sequences, segment_ids int32 [B, T] tells them apart

@@ -338,6 +338,37 @@ def test_aggregate_loss_training_scale(gpu, mode):
   np.testing.assert_allclose(m16.unreduced_sum.item(), num16, rtol=1e-5, atol=1e-4)
 
 
+@pytest.mark.parametrize("mode", AGG_MODES)
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 63), (17, 65), (1024, 16), (1025, 3), (4, 4096), (5, 4096)])   # one launch up to 1024 rows and 16384 tokens
+def test_aggregate_loss_small(gpu, mode, B, T):
+  """One and two launches against the float64 oracle (32-bit sums of at most 20480 terms of order one: 1e-5), and compute()'s one launch against
+  the tensor operations it stands for, bit for bit."""
+  from tunix_amd.rl import common as C
+  rng = np.random.default_rng(B * 7 + T)
+  loss = rng.normal(0.3, 1.0, size=(B, T)).astype(np.float32)
+  mask = np.arange(T)[None, :] < rng.integers(0, T + 1, size=B)[:, None]
+  kwargs = {"norm": 37.5} if "norm" in mode or "scale" in mode else {}
+  m = C.aggregate_loss(torch.from_numpy(loss).to(gpu), torch.from_numpy(mask).to(gpu), mode, **kwargs)
+  num, den, min_denom = R.aggregate_loss(loss, mask, mode, **kwargs)
+  np.testing.assert_allclose(m.unreduced_sum.item(), num, rtol=1e-5, atol=1e-4)
+  np.testing.assert_allclose(m.denominator.item(), den, rtol=1e-7)
+  assert torch.equal(m.compute(), m.unreduced_sum * m.compute_scale())
+
+
+@pytest.mark.parametrize("total,denom", [(3.0, 0.0), (-2.0, 1e-7), (5.0, 3.0), (1.0, float("nan")), (float("inf"), 7.0), (2.0, -4.0)])
+def test_weighted_metric_in_one_launch(gpu, total, denom):
+  """Every rule of compute_scale (eps, minimum, zero, NaN), bit for bit; changed fields take the tensor operations."""
+  from tunix_amd.rl import common as C
+  for eps in (None, 0.25, -3.0):
+    for low in (None, 1.0, 1e-6):
+      m = C._metric(torch.tensor([total, denom], device=gpu), low)
+      m.eps = eps
+      want = m.unreduced_sum * m.compute_scale()
+      assert torch.equal(m.compute(), want) or bool(torch.isnan(want) & torch.isnan(m.compute()))
+      m.denominator = torch.tensor(8.0, device=gpu, dtype=torch.float64)
+      assert m.compute().item() == (m.unreduced_sum * m.compute_scale()).item()
+
+
 def test_aggregate_loss_argument_errors(gpu):
   from tunix_amd.rl import common as C
   x, k = torch.ones(2, 3, device=gpu), torch.ones(2, 3, device=gpu)

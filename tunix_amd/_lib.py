@@ -328,6 +328,8 @@ SIGNATURES = {
     "tnx_moe_combine": (_i32, [_p, _p, _p, _i64, _i32, _i64, _p, _p]),
     "tnx_grpo_ratio": (_i32, [_p, _p, _p, _p, _i64, _i64, _f32, _f32, _p, _p, _p]),
     "tnx_kl_divergence": (_i32, [_p, _p, _p, _i64, _i32, _f32, _p]),
+    "tnx_grpo_ratio_flags": (_i32, [_p, _p, _p, _p, _i64, _i64, _f32, _f32, _p, _p, _p]),
+    "tnx_weighted_metric": (_i32, [_p, _p, _p, _i32, _f32, _i32, _f32, _p]),
     "tnx_aggregate_loss": (_i32, [_p, _p, _p, _i64, _i64, _i32, _f32, _p, _p]),
     "tnx_aggregate_loss_segmented_ws_bytes": (C.c_size_t, [_i64, _i32]),
     "tnx_aggregate_loss_segmented": (_i32, [_p, _p, _p, _p, _i64, _i64, _i32, _i32, _f32, _p, _p]),

@@ -48,9 +48,10 @@ __global__ void sample_commit_kernel(const int32_t* ids, const float* logp, int6
   if (threadIdx.x == 0) *step_ptr = col + 1;
 }
 
+template <class Flag>
 __global__ void grpo_ratio_kernel(const float* logp, const float* old_logp, const float* adv,
                                   int64_t N, int64_t tokens_per_seq, float eps_lo, float eps_hi,
-                                  float* ratio, float* loss, int32_t* clipped) {
+                                  float* ratio, float* loss, Flag* clipped) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
   float lr = logp[i] - (old_logp ? old_logp[i] : logp[i]);
@@ -114,12 +115,11 @@ __global__ __launch_bounds__(256) void agg_rows_kernel(const float* loss, const 
   }
 }
 
-// The rows' sums -> (unreduced sum, denominator) of the aggregation mode.
-__global__ __launch_bounds__(256) void agg_finish_kernel(const float* row_ws, int64_t B, int mode,
-                                                         float norm, float* out) {
-  __shared__ float red[4];
+// The rows' sums -> (unreduced sum, denominator) of the aggregation mode, by the first 256 threads; every thread of the work-group calls it, red
+// holds a float per wave.
+__device__ __forceinline__ void agg_rows_to_mode(const float* row_ws, int64_t B, int mode, float norm, float* red, float* out) {
   float num = 0.f, den = 0.f;
-  for (int64_t b = threadIdx.x; b < B; b += 256) {
+  for (int64_t b = threadIdx.x; b < B && threadIdx.x < 256; b += 256) {
     const float s = row_ws[2 * b], c = row_ws[2 * b + 1];
     const float nonempty = c > 0.f ? 1.f : 0.f;
     if (mode == TNX_AGG_TOKEN_MEAN) {
@@ -144,6 +144,44 @@ __global__ __launch_bounds__(256) void agg_finish_kernel(const float* row_ws, in
     out[0] = num;
     out[1] = mode == TNX_AGG_SEQ_MEAN_TOKEN_SUM_NORM ? norm : den;
   }
+}
+__global__ __launch_bounds__(256) void agg_finish_kernel(const float* row_ws, int64_t B, int mode, float norm, float* out) {
+  __shared__ float red[4];
+  agg_rows_to_mode(row_ws, B, mode, norm, red, out);
+}
+
+// Both passes in one launch for a loss of a few thousand tokens, a wave per row at a time: what such a call costs is its launches.
+constexpr int kAggWaves = 16, kAggOneLaunchRows = 1024;
+constexpr int64_t kAggOneLaunch = 16384;   // tokens; one work-group reads them in some 4 us, a second launch costs the caller about 5
+__global__ __launch_bounds__(64 * kAggWaves) void agg_small_kernel(const float* loss, const float* mask, int64_t B, int64_t T, int mode, float norm,
+                                                                   float* row_ws, float* out) {
+  __shared__ float red[kAggWaves], rows[2 * kAggOneLaunchRows];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int64_t b = wave; b < B; b += kAggWaves) {
+    float s = 0.f, c = 0.f;
+#pragma unroll 4
+    for (int64_t t = lane; t < T; t += 64) {
+      const float m = mask[b * T + t];
+      s += loss[b * T + t] * m;
+      c += m;
+    }
+    s = wave_sum(s);
+    c = wave_sum(c);
+    if (lane == 0) {
+      rows[2 * b] = row_ws[2 * b] = s;
+      rows[2 * b + 1] = row_ws[2 * b + 1] = c;
+    }
+  }
+  __syncthreads();
+  agg_rows_to_mode(rows, B, mode, norm, red, out);
+}
+
+// WeightedMetric.compute: sum * (0 when denom + eps, at least min, is 0, else its reciprocal); NaNs pass the minimum, as they do torch's clamp.
+__global__ void weighted_metric_kernel(const float* sum, const float* denom, int has_eps, float eps, int has_min, float min_denom, float* out) {
+  float d = *denom;
+  if (has_eps) d = d + eps;
+  if (has_min && d < min_denom) d = min_denom;
+  *out = *sum * (d == 0.f ? 0.f : __fdiv_rn(1.0f, d));
 }
 
 // Packed batches: row b holds several sequences told apart by segment_ids[b][t] (0 = padding).
@@ -525,10 +563,26 @@ extern "C" int tnx_grpo_ratio(void* stream, const float* logp, const float* old_
                               const float* adv, int64_t N, int64_t tokens_per_seq, float eps_lo,
                               float eps_hi, float* ratio, float* loss, int32_t* clipped) {
   TNX_REQUIRE(logp && adv && N > 0 && tokens_per_seq > 0, "grpo_ratio: bad arguments");
-  hipLaunchKernelGGL(grpo_ratio_kernel, dim3((unsigned)cdiv(N, 256)), dim3(256), 0,
+  hipLaunchKernelGGL(grpo_ratio_kernel<int32_t>, dim3((unsigned)cdiv(N, 256)), dim3(256), 0,
                      as_stream(stream), logp, old_logp, adv, N, tokens_per_seq, eps_lo, eps_hi,
                      ratio, loss, clipped);
   TNX_CHECK_LAUNCH("grpo_ratio");
+  return TNX_OK;
+}
+
+extern "C" int tnx_grpo_ratio_flags(void* stream, const float* logp, const float* old_logp, const float* adv, int64_t N, int64_t tokens_per_seq,
+                                    float eps_lo, float eps_hi, float* ratio, float* loss, uint8_t* clipped) {
+  TNX_REQUIRE(logp && adv && N > 0 && tokens_per_seq > 0, "grpo_ratio: bad arguments");
+  hipLaunchKernelGGL(grpo_ratio_kernel<uint8_t>, dim3((unsigned)cdiv(N, 256)), dim3(256), 0, as_stream(stream), logp, old_logp, adv, N, tokens_per_seq,
+                     eps_lo, eps_hi, ratio, loss, clipped);
+  TNX_CHECK_LAUNCH("grpo_ratio");
+  return TNX_OK;
+}
+
+extern "C" int tnx_weighted_metric(void* stream, const float* sum, const float* denom, int has_eps, float eps, int has_min, float min_denom, float* out) {
+  TNX_REQUIRE(sum && denom && out, "weighted_metric: null pointer");
+  hipLaunchKernelGGL(weighted_metric_kernel, dim3(1), dim3(1), 0, as_stream(stream), sum, denom, has_eps, eps, has_min, min_denom, out);
+  TNX_CHECK_LAUNCH("weighted_metric");
   return TNX_OK;
 }
 
@@ -549,6 +603,11 @@ extern "C" int tnx_aggregate_loss(void* stream, const float* per_token_loss, con
   TNX_REQUIRE(mode >= TNX_AGG_TOKEN_MEAN && mode <= TNX_AGG_SEQ_MEAN_TOKEN_SUM_NORM, "aggregate_loss: bad mode %d", mode);
   if (mode == TNX_AGG_SEQ_MEAN_TOKEN_SCALE || mode == TNX_AGG_SEQ_MEAN_TOKEN_SUM_NORM)
     TNX_REQUIRE(norm > 0.f, "aggregate_loss: norm must be positive");
+  if (B <= kAggOneLaunchRows && B * T <= kAggOneLaunch) {
+    hipLaunchKernelGGL(agg_small_kernel, dim3(1), dim3(64 * kAggWaves), 0, as_stream(stream), per_token_loss, mask, B, T, mode, norm, row_ws, out);
+    TNX_CHECK_LAUNCH("aggregate_loss");
+    return TNX_OK;
+  }
   hipLaunchKernelGGL(agg_rows_kernel, dim3((unsigned)B), dim3(256), 0, as_stream(stream), per_token_loss, mask,
                      T, row_ws);
   TNX_CHECK_LAUNCH("aggregate_loss rows");

@@ -285,10 +285,17 @@ def moe_combine(y, topk_w, M, k, D, residual, out):
 
 def grpo_ratio(logp, old_logp, adv, tokens_per_seq, eps_lo, eps_hi, ratio=None, loss=None,
                clipped=None):
-  N = logp.numel()
-  L.check(L.lib().tnx_grpo_ratio(_stream(), _ptr(logp), _ptr(old_logp), _ptr(adv), N,
-                                 tokens_per_seq, float(eps_lo), float(eps_hi), _ptr(ratio),
-                                 _ptr(loss), _ptr(clipped)), "tnx_grpo_ratio")
+  """clipped: int32 or bool, as many values as logp."""
+  flags = clipped is not None and clipped.dtype == torch.bool
+  fn = L.lib().tnx_grpo_ratio_flags if flags else L.lib().tnx_grpo_ratio
+  L.check(fn(_stream(), _ptr(logp), _ptr(old_logp), _ptr(adv), logp.numel(), tokens_per_seq, float(eps_lo), float(eps_hi), _ptr(ratio),
+             _ptr(loss), _ptr(clipped)), "tnx_grpo_ratio")
+
+
+def weighted_metric(total, denom, eps, min_denom, out):
+  """out = total / denom of one value each, with `WeightedMetric.compute_scale`'s rules (eps, min_denom: numbers or None)."""
+  L.check(L.lib().tnx_weighted_metric(_stream(), _ptr(total), _ptr(denom), eps is not None, eps or 0.0, min_denom is not None,
+                                      min_denom or 0.0, _ptr(out)), "tnx_weighted_metric")
 
 
 KL_METHODS = {"kl": 0, "mse_kl": 1, "low_var_kl": 2}

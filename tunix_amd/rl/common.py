@@ -155,9 +155,9 @@ def grpo_clipped_ratio(logp: torch.Tensor, old_logp: torch.Tensor | None, advant
     raise ValueError("advantages must hold one value per sequence")
   ratio = torch.empty_like(lp)
   loss = torch.empty_like(lp)
-  clipped = torch.empty(B, T, dtype=torch.int32, device=lp.device)
+  clipped = torch.empty(B, T, dtype=torch.bool, device=lp.device)
   ops.grpo_ratio(lp, old, adv, T, epsilon, eps_hi, ratio=ratio, loss=loss, clipped=clipped)
-  return ratio, loss, clipped.bool()
+  return ratio, loss, clipped
 
 
 def compute_kl_divergence(per_token_logps: torch.Tensor, ref_per_token_logps: torch.Tensor,
@@ -198,7 +198,21 @@ class WeightedMetric:
     return torch.where(denom == 0, torch.zeros_like(denom), 1.0 / safe)
 
   def compute(self) -> torch.Tensor:
+    pair = self.__dict__.get("_pair")
+    # what `aggregate_loss` left here itself, plain 32-bit values on the device: one launch for nine
+    if pair is not None and self.unreduced_sum is pair[0] and self.denominator is pair[1] and not (
+        pair[0].requires_grad or pair[1].requires_grad):
+      out = torch.empty_like(pair[0])
+      ops.weighted_metric(pair[0], pair[1], self.eps, self.min_denom, out)
+      return out
     return self.unreduced_sum * self.compute_scale()
+
+
+def _metric(out: torch.Tensor, min_denom: float) -> WeightedMetric:
+  total, denom = out.unbind(0)
+  metric = WeightedMetric(total, denom, min_denom=min_denom)
+  metric._pair = total, denom
+  return metric
 
 
 def _check_get_norm(arguments: dict[str, Any], default: float) -> float:
@@ -231,7 +245,7 @@ def aggregate_loss(per_token_loss: torch.Tensor, completion_mask: torch.Tensor, 
   min_denom = 1e-6 if loss_agg_mode in ("seq-mean-token-sum", "sequence-mean-token-sum-norm") else 1.0
   loss = per_token_loss.to(torch.float32).contiguous()
   mask = completion_mask.to(torch.float32).contiguous()
-  out = torch.zeros(2, dtype=torch.float32, device=loss.device)
+  out = (torch.empty if B and T else torch.zeros)(2, dtype=torch.float32, device=loss.device)
   if segment_ids is not None:
     if num_segments is None:
       raise ValueError("num_segments must be provided when segment_ids is not None.")
@@ -252,7 +266,7 @@ def aggregate_loss(per_token_loss: torch.Tensor, completion_mask: torch.Tensor, 
       ops.aggregate_loss_segmented(loss, mask, seg, int(num_segments), ops.AGG_MODES[loss_agg_mode], norm, out)
     elif loss_agg_mode == "sequence-mean-token-sum-norm" and norm > 0:
       out[1] = norm
-    return WeightedMetric(out[0], out[1], min_denom=min_denom)
+    return _metric(out, min_denom)
   norm = 1.0
   if loss_agg_mode == "sequence-mean-token-scale":
     norm = _check_get_norm(kwargs, T)
@@ -263,7 +277,7 @@ def aggregate_loss(per_token_loss: torch.Tensor, completion_mask: torch.Tensor, 
     ops.aggregate_loss(loss, mask, ops.AGG_MODES[loss_agg_mode], norm, row_ws, out)
   elif loss_agg_mode == "sequence-mean-token-sum-norm":
     out[1] = norm
-  return WeightedMetric(out[0], out[1], min_denom=min_denom)
+  return _metric(out, min_denom)
 
 
 DRIFT_METRICS = ("sampler_trainer/logp_diff_mean", "sampler_trainer/logp_diff_max",
