@@ -12,7 +12,8 @@ from . import _lib as L
 
 
 def _stream() -> int:
-  return torch.cuda.current_stream().cuda_stream
+  # (the handle itself: building torch's stream object takes 2.9 us of a launch's 7.5, this 0.2)
+  return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
