@@ -218,6 +218,18 @@ class Sampler:
     """sampler.py:692-736: one token per row from the cached state."""
     self._sample(runner, self.forward_step(runner, st), st, mode)
 
+  def _captured(self, step) -> torch.cuda.CUDAGraph:
+    """One call of `step` as a graph.  (torch.cuda.graph would wait for the device and give the allocator's cache back first: the prompts'
+    forward pass and this call then run one after the other, and the next call allocates everything anew.)"""
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(torch.cuda.Stream(self._transformer.device)):   # (capture does not execute: nothing runs on this stream)
+      graph.capture_begin()
+      try:
+        step()
+      finally:
+        graph.capture_end()
+    return graph
+
   # ---- public entry --------------------------------------------------------------------------
   def __call__(
       self,
@@ -312,26 +324,18 @@ class Sampler:
           if (i & 15) == 15 and bool(st.done.all()):
             break
       else:
-        # the first step runs eagerly (lazy module load, attribute set-up), then one captured
-        # step is replayed; `done` is polled every 32 steps like the while_loop condition
-        self._decode_step(runner, st, mode)
-        steps_run = 1
+        # one step is captured, while the device still works on the prompts, and replayed for every token but the first; `done` is
+        # polled every 32 steps like the while_loop condition
+        step = lambda: self._decode_step(runner, st, mode)
         if n_decode > 1:
-          graph = torch.cuda.CUDAGraph()
-          side = torch.cuda.Stream()
-          side.wait_stream(torch.cuda.current_stream())
-          with torch.cuda.stream(side):
-            with torch.cuda.graph(graph, stream=side):
-              self._decode_step(runner, st, mode)
-          torch.cuda.current_stream().wait_stream(side)
-          # capture does not execute: replay n_decode - 1 times
-          while steps_run < n_decode:
-            burst = min(32, n_decode - steps_run)
-            for _ in range(burst):
-              graph.replay()
-            steps_run += burst
-            if bool(st.done.all()):
-              break
+          step = self._captured(step).replay
+        while steps_run < n_decode:
+          burst = min(32, n_decode - steps_run)
+          for _ in range(burst):
+            step()
+          steps_run += burst
+          if steps_run < n_decode and bool(st.done.all()):
+            break
     ev[2].record()
     torch.cuda.synchronize(dev)
     self.last_stats = {
@@ -344,11 +348,13 @@ class Sampler:
     eos_arr = np.asarray(eos_ids)
     out_tokens, out_logits, out_logprobs = [], [], []
     max_len = total_sampling_steps if echo else max_generation_steps
+    lengths = []
     for i in range(B):
       tb = token_buffers[i]
       start_idx = utils.np_find_first_non_pad_idx(tb, pad) if echo else max_prompt_length
       end_idx = utils.np_find_first_eos_idx(tb[max_prompt_length:], eos_arr) + max_prompt_length
       toks = tb[start_idx:end_idx]
+      lengths.append(int(end_idx - start_idx))
       if pad_output:
         length = end_idx - start_idx
         toks = utils.pad_to_length(toks, max_len, pad)[:max_len]
@@ -367,10 +373,6 @@ class Sampler:
           out_logprobs.append(logprobs_np[i][start_idx:end_idx].tolist())
       out_tokens.append(toks)
     if pad_output:
-      lengths = [utils.np_find_first_eos_idx(token_buffers[i][max_prompt_length:], eos_arr)
-                 + max_prompt_length
-                 - (utils.np_find_first_non_pad_idx(token_buffers[i], pad) if echo
-                    else max_prompt_length) for i in range(B)]
       decoded = [self.tokenizer.decode(t[:n].tolist()) for t, n in zip(out_tokens, lengths)]
     else:
       decoded = [self.tokenizer.decode(t.tolist()) for t in out_tokens]
