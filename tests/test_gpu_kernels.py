@@ -2301,3 +2301,58 @@ def test_many_rows_gated_and_residual_in_tiles_of_256_rows(gpu, epi, scale):
     got.append(y)
   assert torch.equal(got[0], got[1])
   assert_bf16_close(got[0], want, atol=1e-5, min_equal=0.9 if mul else 0.97, what=epi, mag=mag, ulps=3 if mul else 2)
+
+
+@pytest.mark.parametrize("B,T,S,Hq,Hkv,col,window,seg,scale", [
+    (2, 61, 61, 4, 1, 0, 0, False, 1.0),          # fewest tiles of the work-group form
+    (3, 131, 333, 6, 2, 77, 0, False, 0.0),       # three query heads in lanes of four, queries from column 77, odd slots, no scaling
+    (1, 259, 263, 4, 1, 3, 40, False, 0.0),       # a window inside two key blocks
+    (2, 150, 150, 2, 2, 0, 0, True, 0.0625),      # a packed batch of several segments, one head per kv head
+    (1, 45, 70, 16, 1, 5, 0, True, 0.0),           # sixteen heads per kv head: one position per tile
+])
+def test_gqa_attention_head_dim_256_many_positions(gpu, B, T, S, Hq, Hkv, col, window, seg, scale):
+  """Keys and values of 256 dimensions through LDS: bit for bit what calls of a few positions give (every wave loads its own), and
+  attention in 64 bits with the probabilities' bf16 rounding as the bound."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  dh, pad = 256, 0
+  g = torch.Generator().manual_seed(190 + T)
+  ids = torch.randint(1, 4 if seg else 100, (B, S), generator=g, dtype=torch.int32)
+  ids = torch.sort(ids, dim=1).values if seg else ids
+  if not seg:
+    ids[0, :5] = pad
+    ids[B - 1, 9] = pad
+  q = bf(rnd((B, T, Hq * dh), 191) * dh ** -0.5).to(gpu)
+  kc, vc = bf(rnd((B, Hkv, S, dh), 192)).to(gpu), bf(rnd((B, Hkv, S, dh), 193)).to(gpu)
+  gids = ids.to(gpu).contiguous()
+
+  def attn(t0, n):
+    qs = q[:, t0:t0 + n].contiguous()
+    out = torch.full((B, n, Hq * dh), 7.0, dtype=torch.bfloat16, device=gpu)
+    colp = torch.tensor([col + t0], dtype=torch.int32, device=gpu)
+    d = L.AttnDesc()
+    d.B, d.T, d.S, d.Hq, d.Hkv, d.dh = B, n, S, Hq, Hkv, dh
+    d.scale, d.window, d.pad_id = scale, window, pad
+    d.q, d.kcache, d.vcache, d.out = qs.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr()
+    if seg:
+      d.segment_ids = gids.data_ptr()
+    else:
+      d.tokens = gids.data_ptr()
+    d.tok_ld, d.col_ptr, d.kv_chunk = S, colp.data_ptr(), 0
+    ops.gqa_attn(d)
+    torch.cuda.synchronize()
+    return out
+
+  whole = attn(0, T)
+  few = 3 * max(1, 16 // (1 << (Hq // Hkv - 1).bit_length()))       # three tiles of queries
+  parts = torch.cat([attn(t0, min(few, T - t0)) for t0 in range(0, T, few)], dim=1)
+  assert torch.equal(whole.view(torch.int16), parts.view(torch.int16))
+  at, key = torch.arange(T)[:, None] + col, torch.arange(S)[None]
+  mask = ((key <= at) & (at - key < window) if window else key <= at)[None] & \
+      (ids[:, None, :] == ids[:, col:col + T, None] if seg else ids[:, None, :] != pad)
+  valid = mask.any(-1) & (ids[:, col:col + T] != pad)
+  heads = lambda x: x.cpu().repeat_interleave(Hq // Hkv, 1).double()
+  score = q.cpu().view(B, T, Hq, dh).permute(0, 2, 1, 3).double() @ heads(kc).transpose(2, 3) * (scale or 1.0)
+  ref = (torch.softmax(score.masked_fill(~mask[:, None], -1e30), -1) @ heads(vc)).permute(0, 2, 1, 3).reshape(B, T, -1).float()
+  diff = (whole.float().cpu() - ref).abs()[valid]
+  assert valid.float().mean() > 0.9 and diff.max().item() <= 2.0 ** -6 * max(1.0, ref[valid].abs().max().item()), diff.max().item()

@@ -769,12 +769,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   }
 }
 
-// The same for head_dim 128 with keys and values staged through LDS: a work-group of four waves
+// The same for head_dim 128 and 256 with keys and values staged through LDS: a work-group of four waves
 // takes 4 x QW consecutive query tiles of one (row, kv head), and every 32-key block is requested
 // once per work-group straight into LDS (16 bytes per lane, key rows with their 16-byte chunks
 // XOR-swizzled by row so that the fragment reads of 16 rows hit 16 bank groups; value rows as they
 // are; the block's 32 token / segment ids next to them, by the dword: rows of ids need no alignment),
-// three blocks in flight.  Every wave computes exactly the blocks attn_tiles_kernel would give it, in the same order
+// the next blocks in flight.  Every wave computes exactly the blocks attn_tiles_kernel would give it, in the same order
 // with the same arithmetic: outputs are bit-identical.
 //
 // What bounds it is vector work: per score 11 lane-instructions (two roundings to bf16 with a scale between them, maximum, exponential,
@@ -799,12 +799,17 @@ __device__ __forceinline__ void dma4(uint32_t lds, const u32x4& r, uint32_t voff
 __device__ __forceinline__ void mfma16_tied(u32x4 a, u32x4 b, f32x4& c) {
   asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
 }
-constexpr uint32_t kWgStageBytes = 8192 + 8192 + 256;   // 32 keys x 256 B, 32 values x 256 B, ids
-// blocks in LDS: one computed, three in flight
-constexpr int kWgStages = 4;
-template <int QW, bool SCALED>
+// 32 keys, 32 values, ids
+constexpr uint32_t wg_stage_bytes(int dh) { return 32u * (uint32_t)dh * 2u * 2u + 256u; }
+// Blocks in LDS: one computed, the others in flight; what two work-groups per compute unit have room for.
+constexpr int wg_stages(int dh) { return dh > 128 ? 2 : 4; }
+// Query tiles of a wave: O and the queries of two at head_dim 256 leave room for one wave per SIMD only, and a wave alone does not cover its own
+// softmax.
+constexpr int wg_tiles_per_wave(int dh) { return dh > 128 ? 1 : 2; }
+template <int DH, bool SCALED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_wg_kernel(const AttnArgs a) {
-  constexpr int DH = 128, KS = 4;
+  constexpr int KS = DH / 32, NH = DH / 128, QW = wg_tiles_per_wave(DH), kWgStages = wg_stages(DH);
+  constexpr uint32_t kWgStageBytes = wg_stage_bytes(DH), ROW = DH * 2, PASSES = DH / 64, VAT = 32 * ROW, IAT = 64 * ROW;
   extern __shared__ __align__(16) unsigned char smem_a[];
   const uint32_t lds0 = lds_addr(smem_a);
   const int tid = threadIdx.x, lane = tid & 63, lm = lane & 15, lq = lane >> 4;
@@ -846,15 +851,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int kb0 = k_lo & ~31, kb_last = k_hi & ~31;
   const bool any = wave_live && kb0 <= k_hi;
 
-  // O^T: lane (query lm, quarter lq) holds dimensions 32 lq + 8 i + jj in O[w][jj][i]
-  f32x4 O[QW][8];
+  // O^T: lane (query lm, quarter lq) holds dimensions 128 h + 32 lq + 8 i + jj in O[w][8 h + jj][i]
+  f32x4 O[QW][8 * NH];
   float m_run[QW], l_run[QW];
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
     m_run[w] = kNegBig;
     l_run[w] = 0.f;
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) O[w][jj] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int jj = 0; jj < 8 * NH; ++jj) O[w][jj] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
   const uint16_t* kbase = a.k + ((b * a.Hkv + hkv) * a.S) * DH;
@@ -889,39 +894,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const uint32_t slab_bytes = (uint32_t)a.S * DH * 2u;
   const u32x4 rk = raw_rsrc(kbase, slab_bytes), rv = raw_rsrc(vbase, slab_bytes);
   const u32x4 rtok = raw_rsrc(tok, (uint64_t)min(a.S, a.tok_ld) * 4);
-  // thread t requests, per 16-row half of a block, the 16 bytes that land at byte 16 t of the half:
-  // row t / 16, and of the key row the chunk (t % 16) ^ (row % 16)
-  const uint32_t krow = (uint32_t)(tid >> 4);
-  const uint32_t kreq = krow * 256u + ((uint32_t)(tid & 15) ^ krow) * 16u;
-  const uint32_t vreq = krow * 256u + (uint32_t)(tid & 15) * 16u;
-  auto request_block = [&](int i) {   // five requests per wave (the ids by every wave: same bytes, one count)
+  // thread t requests, per 4 KB pass over a block (16 rows | 8), the 16 bytes that land at byte 16 t of the pass:
+  // row t / 16 | t / 32, and of the key row the chunk (t % 16 | t % 32) ^ (row % 16)
+  constexpr int CH = DH / 8;   // chunks of a row
+  const uint32_t krow = (uint32_t)(tid / CH);
+  const uint32_t kreq = krow * ROW + ((uint32_t)(tid % CH) ^ krow) * 16u;
+  const uint32_t vreq = (uint32_t)tid * 16u;
+  auto request_block = [&](int i) {   // 2 PASSES + 1 requests per wave (the ids by every wave: same bytes, one count)
     const uint32_t base = lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes + (uint32_t)wave * 1024u;
-    const uint32_t kb_bytes = (uint32_t)(kb0_wg + 32 * i) * 256u;
+    const uint32_t kb_bytes = (uint32_t)(kb0_wg + 32 * i) * ROW;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      dma16(base + (uint32_t)c * 4096u, rk, kb_bytes + (uint32_t)c * 4096u + kreq, 0);
-      dma16(base + 8192u + (uint32_t)c * 4096u, rv, kb_bytes + (uint32_t)c * 4096u + vreq, 0);
+    for (uint32_t c = 0; c < PASSES; ++c) {   // (rows 8 .. 15 of a block of 512-byte rows come with the odd passes)
+      dma16(base + c * 4096u, rk, kb_bytes + c * 4096u + (DH > 128 ? kreq ^ ((c & 1u) * 128u) : kreq), 0);
+      dma16(base + VAT + c * 4096u, rv, kb_bytes + c * 4096u + vreq, 0);
     }
     // ids kb .. kb + 63 (the block's 32 and whatever follows them; past the row: zeros)
-    dma4(lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes + 16384u, rtok, (uint32_t)(kb0_wg + 32 * i + lane) * 4u);
+    dma4(lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes + IAT, rtok, (uint32_t)(kb0_wg + 32 * i + lane) * 4u);
   };
-  // this lane's places in a stage: key row lm (+ 16 tt), chunk 4 j + lq; value rows 4 lq + s (+ 16), chunk lm; ids 4 lq
+  // this lane's places in a stage: key row lm (+ 16 tt), chunk 4 j + lq; value rows 4 lq + s (+ 16), chunk lm (+ 16 h); ids 4 lq
   uint32_t kat[KS];
 #pragma unroll
-  for (int j = 0; j < KS; ++j) kat[j] = (uint32_t)(lm * 256) + (((uint32_t)(j * 4 + lq) ^ (uint32_t)lm) * 16u);
-  const uint32_t vat = 8192u + (uint32_t)(lq * 1024 + lm * 16), iat = 16384u + (uint32_t)(lq * 16);
+  for (int j = 0; j < KS; ++j) kat[j] = (uint32_t)lm * ROW + (((uint32_t)(j * 4 + lq) ^ (uint32_t)lm) * 16u);
+  const uint32_t vat = VAT + (uint32_t)lq * (4u * ROW) + (uint32_t)(lm * 16), iat = IAT + (uint32_t)(lq * 16);
   auto compute_block = [&](int kb, uint32_t base) {
     u32x4 kf[2][KS], vf[8];
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
       const uint32_t at = base + kat[j];
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) kf[tt][j] = attn_lds128(at + (uint32_t)(tt * 4096));
+      for (int tt = 0; tt < 2; ++tt) kf[tt][j] = attn_lds128(at + (uint32_t)tt * (16u * ROW));
     }
     const uint32_t va = base + vat, ia = base + iat;
     const u32x4 t0 = attn_lds128(ia), t1 = attn_lds128(ia + 64u);
 #pragma unroll
-    for (int s = 0; s < 8; ++s) vf[s] = attn_lds128(va + (uint32_t)((s < 4 ? s : 12 + s) * 256));
+    for (int s = 0; s < 8; ++s) vf[s] = attn_lds128(va + (uint32_t)(s < 4 ? s : 12 + s) * ROW);
     // (pad mode: a key counts when its id differs from pad_id; packed: when it is the query's)
     bool ids = true;
 #pragma unroll
@@ -985,19 +991,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int w = 0; w < QW; ++w)
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj)
+        for (int jj = 0; jj < 8 * NH; ++jj)
 #pragma unroll
           for (int i = 0; i < 4; ++i) O[w][jj][i] *= alpha[w];
     }
     // a value fragment is transposed once for all tiles
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) {
-      const uint32_t sel = (jj & 1) ? 0x07060302u : 0x05040100u;
-      u32x4 vt;
+    for (int h = 0; h < NH; ++h) {
+      if (h > 0)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vt[r] = __builtin_amdgcn_perm(vf[2 * r + 1][jj >> 1], vf[2 * r][jj >> 1], sel);
+        for (int s = 0; s < 8; ++s) vf[s] = attn_lds128(va + (uint32_t)(s < 4 ? s : 12 + s) * ROW + (uint32_t)h * 256u);
 #pragma unroll
-      for (int w = 0; w < QW; ++w) mfma16_tied(vt, pa[w], O[w][jj]);
+      for (int jj = 0; jj < 8; ++jj) {
+        const uint32_t sel = (jj & 1) ? 0x07060302u : 0x05040100u;
+        u32x4 vt;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vt[r] = __builtin_amdgcn_perm(vf[2 * r + 1][jj >> 1], vf[2 * r][jj >> 1], sel);
+#pragma unroll
+        for (int w = 0; w < QW; ++w) mfma16_tied(vt, pa[w], O[w][8 * h + jj]);
+      }
     }
   };
 #pragma unroll
@@ -1005,8 +1017,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (u < nblk_wg) request_block(u);
   for (int i = 0; i < nblk_wg; ++i) {
     // this wave's share of block i has landed (behind it: the requests of blocks i + 1 ..
-    // i + stages - 2, five each; near the end, where fewer follow, everything is waited for) ...
-    if (i + kWgStages - 2 < nblk_wg) tnx_wait_vm(5 * (kWgStages - 2));
+    // i + stages - 2; near the end, where fewer follow, everything is waited for) ...
+    if (i + kWgStages - 2 < nblk_wg) tnx_wait_vm((int)(2 * PASSES + 1) * (kWgStages - 2));
     else tnx_wait_vm(0);
     __syncthreads();    // ... and everyone's; every wave is also done reading block i - 1, whose stage is refilled
     if (i + kWgStages - 1 < nblk_wg) request_block(i + kWgStages - 1);
@@ -1017,7 +1029,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int w = 0; w < QW; ++w)
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) asm volatile("" : "+v"(O[w][jj]));
+    for (int jj = 0; jj < 8 * NH; ++jj) asm volatile("" : "+v"(O[w][jj]));
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
     const float l = across_quarters(l_run[w], [](float x, float y) { return x + y; });
@@ -1026,12 +1038,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     uint16_t* o = a.out + ((b * a.T + ti) * a.Hq + hkv * a.G + g) * DH + 32 * lq;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      u32x4 wv;
+    for (int h = 0; h < NH; ++h)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) wv[r] = pack2bf(O[w][2 * r][i] * inv, O[w][2 * r + 1][i] * inv);
-      *reinterpret_cast<u32x4*>(o + 8 * i) = wv;
-    }
+      for (int i = 0; i < 4; ++i) {
+        u32x4 wv;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) wv[r] = pack2bf(O[w][8 * h + 2 * r][i] * inv, O[w][8 * h + 2 * r + 1][i] * inv);
+        *reinterpret_cast<u32x4*>(o + 128 * h + 8 * i) = wv;
+      }
   }
 }
 
@@ -1224,27 +1238,33 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
     if (tv) hipLaunchKernelGGL((attn_kernel<DH, FUSE, true>), grid, dim3(64), 0, st, a);         \
     else hipLaunchKernelGGL((attn_kernel<DH, FUSE, false>), grid, dim3(64), 0, st, a);           \
   } while (0)
-  // many query positions at head_dim 128, no key split, no fused rotation: keys and values through
-  // LDS, eight query tiles per work-group
-  constexpr int kWgTilesPerWave = 2;
-  if (!a.rope_sin && a.n_chunks == 1 && d->dh == 128 && QT >= 2 * 4 * kWgTilesPerWave &&
-      (uint64_t)d->S * 256u < (1ull << 32) && d->B * cdiv(QT, 4 * kWgTilesPerWave) <= 65535) {
-    a.QTG = (unsigned)cdiv(QT, 4 * kWgTilesPerWave);
-    auto launch = [&](auto scaled_c) -> int {
+  // many query positions at head_dim 128 or 256, no key split, no fused rotation: keys and values through LDS, eight | four query tiles
+  // per work-group.  At 256 every wave's own loads of its keys and values are what bounds the other form; us, through LDS | per wave, positions
+  // x rows, 4 heads on one: 256 x 64 38.6 | 133.4, 1000 x 16 92 | 335, 3000 x 8 308 | 1334 (window of 512 117 | 490), 3000 x 1 117 | 210; 64 x 64
+  // 9.1 | 14.8, 64 x 1 6.7 | 6.1; of fewer tiles, 32 x 64 6.6 | 6.4, 32 x 1 5.5 | 4.6.
+  if (!a.rope_sin && a.n_chunks == 1 && d->dh >= 128) {
+    auto launch = [&](auto dh_c, auto scaled_c) -> int {
+      constexpr int DH = decltype(dh_c)::value;
       constexpr bool SCALED = decltype(scaled_c)::value;
       static std::once_flag wg_once;
       static hipError_t wg_rc = hipSuccess;
+      constexpr int kLds = (int)(wg_stages(DH) * wg_stage_bytes(DH));
       std::call_once(wg_once, [] {
-        wg_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_wg_kernel<kWgTilesPerWave, SCALED>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kWgStages * kWgStageBytes));
+        wg_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_wg_kernel<DH, SCALED>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
       });
       TNX_REQUIRE(wg_rc == hipSuccess, "attn: cannot raise the dynamic LDS limit");
-      hipLaunchKernelGGL((attn_wg_kernel<kWgTilesPerWave, SCALED>), dim3(1u, (unsigned)d->Hkv, (unsigned)(d->B * a.QTG)), dim3(256),
-                         kWgStages * kWgStageBytes, st, a);
+      hipLaunchKernelGGL((attn_wg_kernel<DH, SCALED>), dim3(1u, (unsigned)d->Hkv, (unsigned)(d->B * a.QTG)), dim3(256), kLds, st, a);
       TNX_CHECK_LAUNCH("gqa_attn (work-group tiles)");
       return TNX_OK;
     };
-    return a.scale_bf != 0.f ? launch(std::true_type{}) : launch(std::false_type{});
+    const int tiles = 4 * wg_tiles_per_wave(d->dh);   // of a work-group
+    if (QT >= 16 && (uint64_t)d->S * d->dh * 2u < (1ull << 32) && d->B * cdiv(QT, tiles) <= 65535) {
+      a.QTG = (unsigned)cdiv(QT, tiles);
+      const bool scaled = a.scale_bf != 0.f;
+      if (d->dh == 128) return scaled ? launch(std::integral_constant<int, 128>{}, std::true_type{}) : launch(std::integral_constant<int, 128>{}, std::false_type{});
+      return scaled ? launch(std::integral_constant<int, 256>{}, std::true_type{}) : launch(std::integral_constant<int, 256>{}, std::false_type{});
+    }
   }
   // many query positions, no key split, no fused rotation: two query tiles per wave
   constexpr int kTilesPerWave = 2;
