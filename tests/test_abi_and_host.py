@@ -248,3 +248,20 @@ def test_split_k_choice_of_the_decode_linears():
   assert m._split_k(lin("wq", 4096, 6144), 8192) == 1            # many rows
   m.split_k_override = {"w_gate": 3}
   assert m._split_k(lin("w_gate", 1152, 13824, True), 64) == 3
+
+
+def test_split_k_leaves_no_empty_split_and_goes_on_for_long_contractions():
+  import math
+  import types
+  from tunix_amd.model import Runner
+  m = Runner.__new__(Runner)
+  m.split_k_override = {}
+  lin = lambda name, K, N: types.SimpleNamespace(names=[f"l0.{name}"], K=K, N=N, interleave2=False)
+  assert m._split_k(lin("wq", 1152, 1536), 64) == 5            # nine k-tiles, two per split
+  assert m._split_k(lin("w_down", 6912, 1152), 64) == 14       # nine column blocks: 126 of 256 compute units, four k-tiles each
+  assert m._split_k(lin("w_down", 16384, 1152), 64) == 16
+  assert m._split_k(lin("wq", 8192, 512), 1) == 8              # the attention kernel takes eight planes in one round trip
+  for kt in range(1, 130):
+    for n in (128, 640, 1152, 4096, 12800):
+      s = m._split_k(lin("wo", 128 * kt, n), 8)
+      assert 1 <= s <= 16 and (s - 1) * math.ceil(kt / s) < kt

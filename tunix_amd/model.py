@@ -588,7 +588,14 @@ class Runner(HeadRunner):
     ktiles = f.K // 128
     if blocks >= 200 or M > 128:
       return 1
-    split = int(max(1, min(8, ktiles, 256 // blocks)))
+    # Eight splits, or so many that a split has four k-tiles, and as many as fill the device; more planes cost their consumer more
+    # than the shorter splits save (the q|k|v planes may go to the attention kernel, which takes eight in one round trip).  Then no more than leave
+    # none empty: nine k-tiles in eight splits of two are five splits and three planes of zeros.  Rollouts of Gemma3-1B (qkv 9, o 8, down 54
+    # k-tiles; splits 8 / 8 / 8 | 5 / 8 / 14), 32 tokens, ms: 64 rows 68.7 | 67.4, 128 rows 85.2 | 82.9, 16 rows 58.0 | 57.1, 1 row 50.4 | 49.8
+    # (down in 11 or 18 splits 0.5 to 1.4 more at 64 and 128 rows).
+    most = 8 if key == "wq" else 16
+    split = int(max(1, min(max(8, math.ceil(ktiles / 4)), most, ktiles, 256 // blocks)))
+    split = math.ceil(ktiles / math.ceil(ktiles / split))
     # A gate|up linear that runs unsplit applies its activation itself and can leave the next
     # linear's adapter down-projection behind: two launches fewer (finishing pass, LoRA down),
     # ≈ 9 us, against ≈ 1.1 us per k-tile the unsplit work-groups run longer.
