@@ -2356,3 +2356,57 @@ def test_gqa_attention_head_dim_256_many_positions(gpu, B, T, S, Hq, Hkv, col, w
   ref = (torch.softmax(score.masked_fill(~mask[:, None], -1e30), -1) @ heads(vc)).permute(0, 2, 1, 3).reshape(B, T, -1).float()
   diff = (whole.float().cpu() - ref).abs()[valid]
   assert valid.float().mean() > 0.9 and diff.max().item() <= 2.0 ** -6 * max(1.0, ref[valid].abs().max().item()), diff.max().item()
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,dh,chunk,window", [
+    (70, 8, 2, 128, 0, 0),        # three blocks for four waves; rows of ids read one by one
+    (300, 16, 1, 128, 128, 0),    # sixteen heads on one, chunks of a block per wave, the last ones empty for most columns
+    (300, 6, 2, 64, 0, 100),      # head_dim 64, three heads in lanes of four, a window over four or five blocks
+    (1300, 4, 1, 128, 672, 0),    # odd and even block counts
+])
+@pytest.mark.parametrize("packed", [False, True])
+def test_decode_attention_of_several_waves_per_chunk(gpu, S, Hq, Hkv, dh, chunk, window, packed):
+  """One query position whose key blocks are shared among the waves of a work-group, at columns on both sides of every share, against
+  attention in 64 bits (probabilities rounded to bf16: 2^-8 of values below 4)."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  B, pad = 3, 0
+  g = torch.Generator().manual_seed(300 + S)
+  ids = torch.sort(torch.randint(1, 4, (B, S), generator=g, dtype=torch.int32), 1).values if packed else \
+      torch.randint(1, 100, (B, S), generator=g, dtype=torch.int32)
+  if not packed:
+    ids[0, :40] = pad
+    ids[1, 7] = pad
+  q = bf(rnd((B, Hq * dh), 301)).to(gpu)
+  kc, vc = bf(rnd((B, Hkv, S, dh), 302)), bf(rnd((B, Hkv, S, dh), 303))
+  gids = ids.to(gpu).contiguous()
+  heads = lambda x: x.double().repeat_interleave(Hq // Hkv, 1)
+  for col in sorted({min(c, S - 1) for c in (0, 31, 32, 63, 64, 95, 127, 128, 129, 160, 255, 256, 299, 671, 672, 703, 1299)}):
+    kg, vg = kc.clone(), vc.clone()
+    kg[:, :, col + 1:], vg[:, :, col + 1:] = 1e4, 1e4          # slots not written yet
+    kg, vg = kg.to(gpu), vg.to(gpu)
+    out = torch.full((B, Hq * dh), 7.0, dtype=torch.bfloat16, device=gpu)
+    ws = torch.empty(max(ops.attn_ws_bytes(B, 1, S, Hq, dh, chunk) // 4, 1), dtype=torch.float32, device=gpu)
+    colp = torch.tensor([col], dtype=torch.int32, device=gpu)
+    d = L.AttnDesc()
+    d.B, d.T, d.S, d.Hq, d.Hkv, d.dh = B, 1, S, Hq, Hkv, dh
+    d.scale, d.window, d.pad_id = dh ** -0.5, window, pad
+    d.q, d.kcache, d.vcache, d.out, d.ws = q.data_ptr(), kg.data_ptr(), vg.data_ptr(), out.data_ptr(), ws.data_ptr()
+    if packed:
+      d.segment_ids = gids.data_ptr()
+    else:
+      d.tokens = gids.data_ptr()
+    d.tok_ld, d.col_ptr, d.kv_chunk = S, colp.data_ptr(), chunk
+    ops.gqa_attn(d)
+    torch.cuda.synchronize()
+    lo = max(0, col - window + 1) if window else 0
+    mask = torch.zeros(B, S, dtype=torch.bool)
+    mask[:, lo:col + 1] = True
+    mask &= (ids == ids[:, col:col + 1]) if packed else ids != pad
+    score = (q.cpu().view(B, Hq, 1, dh).double() @ heads(kc).transpose(2, 3)) * dh ** -0.5
+    ref = torch.softmax(score.masked_fill(~mask[:, None, None], -1e30), -1) @ heads(vc)
+    live = mask.any(1)
+    got = out.float().cpu().view(B, Hq, dh)
+    diff = (got - ref[:, :, 0].float()).abs()[live]
+    assert live.any() and diff.max().item() <= 2.0 ** -6 * max(1.0, ref[live].abs().max().item()), (col, diff.max().item())
+    assert (got[~live] == 0).all()

@@ -6,7 +6,7 @@
 // probabilities of ONE query column for 8 keys -- exactly the A fragment of the P.V MFMA --
 // and the max / sum of the online softmax are per-lane scalars reduced over 4 lanes.  V rows
 // are loaded in their natural [key][dh] layout (256 B contiguous per key) and transposed
-// inside each lane with v_perm_b32 to form B fragments; nothing goes through LDS.
+// inside each lane with v_perm_b32 to form B fragments; keys and values go through LDS only in the work-group form for many positions below.
 #include <string.h>
 
 #include <mutex>
@@ -71,12 +71,18 @@ __device__ __forceinline__ float across_quarters(float x, F f) {
 // write of a decode step (below), qkv taken from the finished output or from any number of
 // partial planes; 2 = the same from at most eight partial planes and at most four query heads per
 // kv head (one set of 3 x 64 lanes x 16 bytes per plane), all fetched in one round trip.
-template <int DH, int FUSE, bool TOKVEC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2 : 1, DH > 128 ? 2 : 1))) void attn_kernel(const AttnArgs a) {
+// W: waves of a work-group.  Of more than one (a decode step: T == 1) each takes an equal share of the key blocks that the work-group's
+// chunk of the cache holds by now, and they merge what they have through LDS: the pass that would merge them otherwise is a launch, and its partials
+// a round trip to memory.  32 heads on 8, with the o adapter's 64 columns behind it, us before | now: 16 rows x 192 keys 14.0 | 12.7, 700 keys 19.9 |
+// 16.9, 8 rows x 1000 18.8 | 15.5, 1 row x 732 15.6 | 13.3, 3 rows x 2940 22.8 | 18.7, 64 rows x 372 27.6 | 23.3.
+constexpr int kAttnWaves = 4;
+template <int DH, int FUSE, bool TOKVEC, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128 || W > 1 ? 2 : 1, DH > 128 || W > 1 ? 2 : 1))) void attn_kernel(const AttnArgs a) {
   constexpr int KS = DH / 32;                 // k-steps of the QK product
   constexpr int NH = DH > 128 ? DH / 128 : 1; // 128-column halves of V / O
   constexpr int NS = DH > 128 ? 1 : TNX_ATTN_NS;        // register stages of the key-block pipeline
-  const int lane = threadIdx.x, lm = lane & 15, lq = lane >> 4;
+  const int lane = threadIdx.x & 63, lm = lane & 15, lq = lane >> 4;
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
   const int chunk = blockIdx.x, hkv = blockIdx.y;
   // (shifts and one unsigned division: a general integer division costs some forty instructions,
   // and the chain in front of this kernel's first loads had several of them)
@@ -103,6 +109,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
   }
 
   constexpr bool fused = FUSE != 0;                         // T == 1: c_n = col0 for every lane
+  // the chunk that owns the new token (of its waves the last, which has the fewest blocks)
+  const bool writer = fused && col0 >= k_lo && col0 <= k_hi && wave == W - 1;
+  if constexpr (W > 1) {
+    if (fused) k_hi = min(k_hi, col0 - 1);
+    const int first = k_lo & ~31, each = (max(k_hi - first + 32, 0) / 32 + W - 1) / W * 32;
+    k_lo = max(k_lo, first + wave * each);
+    k_hi = min(k_hi, first + (wave + 1) * each - 1);
+  }
   u32x4 qf[KS];
 #pragma unroll
   for (int j = 0; j < KS; ++j) {
@@ -112,7 +126,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
   // in fused mode the step's own key / value never come from the cache: the loop stops one key
   // short and they are added from registers at the end
   int key_hi = fused ? c_n - 1 : c_n;
-  const bool writer = fused && col0 >= k_lo && col0 <= k_hi;   // the chunk that owns the new token
   if (fused) k_hi = min(k_hi, col0 - 1);
 
   f32x4 O[NH][8];
@@ -259,6 +272,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
         O[h][jj] = mfma16(pa, bfrag, O[h][jj]);
       }
   };
+  // a wave's staged q / k / v, later its part of the output
+  __shared__ __align__(16) float stage[FUSE || W > 1 ? W : 1][FUSE ? 18 * DH : W > 1 ? 16 * DH : 1];
   {
     Stage sg[NS];
     const int kb0 = k_lo & ~31;
@@ -280,7 +295,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
       fetch_query_id();
     }
     // the step's own key / value wait in LDS while the cached keys stream through the registers
-    __shared__ u32x4 park[FUSE ? KS + NH : 1][64];
+    __shared__ u32x4 park_w[W][FUSE ? KS + NH : 1][64];
+    auto& park = park_w[wave];
     if constexpr (fused) {
       u32x4 kn[KS], vn[NH];
       // ---- this step's q (G heads), k and v of the kv head from the qkv linear's output, RoPE
@@ -292,7 +308,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
       // values, are fetched once by the whole wave (16 bytes per lane and plane, all planes of
       // a group in flight together), summed in split order, rounded to bf16 and staged in LDS,
       // from where every lane picks the elements of its fragments.
-      __shared__ float xs[18 * DH];
+      float* xs = stage[wave];
       // sine / cosine of this row's position: a per-step table (tnx_rope_table), computed with
       // the arithmetic of the stand-alone kernel; fetched together with the planes
       float sn[KS / 2][8], cs[KS / 2][8];
@@ -388,7 +404,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
               *reinterpret_cast<f32x4*>(&xs[i4 * 4]) = f32x4{rbf(acc[0]), rbf(acc[1]), rbf(acc[2]), rbf(acc[3])};
           }
         }
-        // the work-group is this one wave: LDS executes a wave's accesses in order, so the staged
+        // only this wave reads them: LDS executes a wave's accesses in order, so the staged
         // values only need the compiler to keep the reads behind the writes (a work-group
         // barrier would also wait for the key / value loads in flight)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -458,21 +474,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
       // Whole turns of the ring without a branch inside (an exit in the middle of a turn makes
       // the compiler merge the stages' registers on the exit edges, and a copy of a register
       // that is still being loaded waits for everything in flight), then the last one or two
-      // blocks, whose loads were issued by the turn before them.
+      // blocks in code of their own: a load of the last block once more, that the turn would make to keep its
+      // count, is a block's worth of the memory's time (of two blocks per wave, half as much again).
       const int nblk = ((kb_last - kb0) >> 5) + 1;
-      int i = 0;
-      for (; i + NS <= nblk; i += NS) {
-#pragma unroll
-        for (int u = 0; u < NS; ++u) {
-          const int kbu = kb0 + 32 * (i + u);
-          load_block(min(kbu + 32 * (NS - 1), kb_last), sg[(u + NS - 1) % NS]);
+      if constexpr (NS == 1) {
+        for (int i = 0; i < nblk; ++i) {
+          load_block(kb0 + 32 * i, sg[0]);
           __builtin_amdgcn_sched_barrier(0);
-          compute_block(kbu, sg[u]);
+          compute_block(kb0 + 32 * i, sg[0]);
+        }
+      } else {
+        static_assert(NS <= 2, "the turns below are of two blocks");
+        auto step = [&](int i, Stage& now, Stage& next) {   // computes block i while i + 1 is on its way
+          load_block(kb0 + 32 * (i + 1), next);
+          __builtin_amdgcn_sched_barrier(0);
+          compute_block(kb0 + 32 * i, now);
+        };
+        int i = 0;
+        for (; i + 2 < nblk; i += 2) {
+          step(i, sg[0], sg[1]);
+          step(i + 1, sg[1], sg[0]);
+        }
+        if (i + 1 < nblk) {
+          step(i, sg[0], sg[1]);
+          compute_block(kb0 + 32 * (i + 1), sg[1]);
+        } else {
+          compute_block(kb0 + 32 * i, sg[0]);
         }
       }
-#pragma unroll
-      for (int u = 0; u < NS - 1; ++u)
-        if (i + u < nblk) compute_block(kb0 + 32 * (i + u), sg[u]);
     }
     if (writer) {
       // the step's own key / value as a block of one key (at position col0) from registers
@@ -489,6 +518,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
       const int own_tok = tok[col0];
 #pragma unroll
       for (int sidx = 0; sidx < 8; ++sidx) one.tk[sidx] = own_tok;
+      k_lo = min(k_lo, col0);   // (W > 1: a wave's share may lie behind it, with no block in it)
       k_hi = col0;
       key_hi = col0;
       compute_block(col0, one);
@@ -499,6 +529,55 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DH > 128 ? 2
 
   // O rows are query columns 4*lq + i; columns are d = h*128 + 8*lm + jj.
   const bool dvalid = 8 * lm < (DH < 128 ? DH : 128);
+  if constexpr (W > 1) {   // T == 1: the queries are columns 0 .. G - 1
+    __shared__ float ml[W][16][2];
+    if (lane < 16) {
+      ml[wave][lane][0] = m_run;
+      ml[wave][lane][1] = l_run;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int n = 4 * lq + i;
+      if (n >= a.G || !dvalid) continue;
+#pragma unroll
+      for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int jj = 0; jj < 8; jj += 4)
+          *reinterpret_cast<f32x4*>(&stage[wave][n * DH + h * 128 + 8 * lm + jj]) = f32x4{O[h][jj][i], O[h][jj + 1][i], O[h][jj + 2][i], O[h][jj + 3][i]};
+    }
+    __syncthreads();
+    for (int e = (int)threadIdx.x * 4; e < a.G * DH; e += 64 * W * 4) {
+      const int n = e / DH, d = e - n * DH;
+      float M = kNegBig, L = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; ++w)
+        if (ml[w][n][1] > 0.f) M = fmaxf(M, ml[w][n][0]);
+      f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const float l = ml[w][n][1], f = __expf(ml[w][n][0] - M);
+        if (l > 0.f) {   // (a wave without a key)
+          L += f * l;
+          const f32x4 v = *reinterpret_cast<const f32x4*>(&stage[w][e]);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) o[q] += f * v[q];
+        }
+      }
+      const int64_t qv = b * a.Hq + hkv * a.G + n;
+      if (a.n_chunks == 1) {
+        const float inv = L > 0.f ? 1.0f / L : 0.f;
+        *reinterpret_cast<u32x2*>(a.out + qv * DH + d) = u32x2{pack2bf(o[0] * inv, o[1] * inv), pack2bf(o[2] * inv, o[3] * inv)};
+      } else {
+        float* p = a.ws + (qv * a.n_chunks + chunk) * (DH + kPartPad);
+        if (d == 0) {
+          p[0] = M;
+          p[1] = L;
+        }
+        *reinterpret_cast<f32x4*>(p + kPartPad + d) = o;
+      }
+    }
+    return;
+  }
   if (a.kv_chunk <= 0 || a.n_chunks == 1) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1233,11 +1312,20 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
   dim3 grid((unsigned)a.n_chunks, (unsigned)d->Hkv, (unsigned)(d->B * QT));
   hipStream_t st = as_stream(stream);
   const bool tv = (d->tok_ld % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.tokens) & 15) == 0) && d->S % 4 == 0;
-#define TNX_ATTN_LAUNCH(DH, FUSE)                                                                \
-  do {                                                                                           \
-    if (tv) hipLaunchKernelGGL((attn_kernel<DH, FUSE, true>), grid, dim3(64), 0, st, a);         \
-    else hipLaunchKernelGGL((attn_kernel<DH, FUSE, false>), grid, dim3(64), 0, st, a);           \
-  } while (0)
+  auto launch_decode = [&](auto dh_c, auto fuse_c, auto waves_c) {
+    constexpr int DH = decltype(dh_c)::value, FUSE = decltype(fuse_c)::value, W = decltype(waves_c)::value;
+    if (tv) hipLaunchKernelGGL((attn_kernel<DH, FUSE, true, W>), grid, dim3(64 * W), 0, st, a);
+    else hipLaunchKernelGGL((attn_kernel<DH, FUSE, false, W>), grid, dim3(64 * W), 0, st, a);
+  };
+  // several waves per chunk: of more than two key blocks, as long as two work-groups per compute unit hold them all (beyond, waves enough of their own:
+  // 128 rows x 8 kv heads x 160 keys 21.9 us with one wave, 25.0 with four)
+  const int64_t chunk_keys = d->kv_chunk > 0 ? d->kv_chunk : d->S;
+  const bool waves = d->T == 1 && (d->window > 0 ? std::min<int64_t>(chunk_keys, d->window) : chunk_keys) > 64 && d->B * d->Hkv * a.n_chunks <= 512;
+  auto launch_head_dim = [&](auto dh_c, auto fuse_c) {
+    if (waves) launch_decode(dh_c, fuse_c, std::integral_constant<int, kAttnWaves>{});
+    else launch_decode(dh_c, fuse_c, std::integral_constant<int, 1>{});
+  };
+#define TNX_ATTN_LAUNCH(DH, FUSE) launch_head_dim(std::integral_constant<int, DH>{}, std::integral_constant<int, FUSE>{})
   // many query positions at head_dim 128 or 256, no key split, no fused rotation: keys and values through LDS, eight | four query tiles
   // per work-group.  At 256 every wave's own loads of its keys and values are what bounds the other form; us, through LDS | per wave, positions
   // x rows, 4 heads on one: 256 x 64 38.6 | 133.4, 1000 x 16 92 | 335, 3000 x 8 308 | 1334 (window of 512 117 | 490), 3000 x 1 117 | 210; 64 x 64
@@ -1288,7 +1376,7 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
       else if (a.rope_sin) TNX_ATTN_LAUNCH(128, 1);
       else TNX_ATTN_LAUNCH(128, 0);
       break;
-    default: TNX_ATTN_LAUNCH(256, 0); break;
+    default: launch_decode(std::integral_constant<int, 256>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}); break;
   }
 #undef TNX_ATTN_LAUNCH
   TNX_CHECK_LAUNCH("gqa_attn");
