@@ -2363,6 +2363,8 @@ def test_gqa_attention_head_dim_256_many_positions(gpu, B, T, S, Hq, Hkv, col, w
     (300, 16, 1, 128, 128, 0),    # sixteen heads on one, chunks of a block per wave, the last ones empty for most columns
     (300, 6, 2, 64, 0, 100),      # head_dim 64, three heads in lanes of four, a window over four or five blocks
     (1300, 4, 1, 128, 672, 0),    # odd and even block counts
+    (300, 4, 1, 256, 128, 0),     # head_dim 256
+    (200, 2, 2, 256, 0, 150),
 ])
 @pytest.mark.parametrize("packed", [False, True])
 def test_decode_attention_of_several_waves_per_chunk(gpu, S, Hq, Hkv, dh, chunk, window, packed):

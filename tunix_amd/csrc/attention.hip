@@ -74,7 +74,8 @@ __device__ __forceinline__ float across_quarters(float x, F f) {
 // W: waves of a work-group.  Of more than one (a decode step: T == 1) each takes an equal share of the key blocks that the work-group's
 // chunk of the cache holds by now, and they merge what they have through LDS: the pass that would merge them otherwise is a launch, and its partials
 // a round trip to memory.  32 heads on 8, with the o adapter's 64 columns behind it, us before | now: 16 rows x 192 keys 14.0 | 12.7, 700 keys 19.9 |
-// 16.9, 8 rows x 1000 18.8 | 15.5, 1 row x 732 15.6 | 13.3, 3 rows x 2940 22.8 | 18.7, 64 rows x 372 27.6 | 23.3.
+// 16.9, 8 rows x 1000 18.8 | 15.5, 1 row x 732 15.6 | 13.3, 3 rows x 2940 22.8 | 18.7, 64 rows x 372 27.6 | 23.3; 4 heads of 256 on one, 32 columns:
+// 64 rows x 288 14.7 | 12.0, 16 rows x 1200 21.7 | 14.6.
 constexpr int kAttnWaves = 4;
 template <int DH, int FUSE, bool TOKVEC, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128 || W > 1 ? 2 : 1, DH > 128 || W > 1 ? 2 : 1))) void attn_kernel(const AttnArgs a) {
@@ -1376,7 +1377,7 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
       else if (a.rope_sin) TNX_ATTN_LAUNCH(128, 1);
       else TNX_ATTN_LAUNCH(128, 0);
       break;
-    default: launch_decode(std::integral_constant<int, 256>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}); break;
+    default: TNX_ATTN_LAUNCH(256, 0); break;
   }
 #undef TNX_ATTN_LAUNCH
   TNX_CHECK_LAUNCH("gqa_attn");

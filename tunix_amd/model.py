@@ -562,19 +562,17 @@ class Runner(HeadRunner):
             need = max(need, sk * M * ly[key].N)
     self.splitk_ws = torch.empty(need, dtype=torch.float32, device=dev)
     if kv_chunk is None:
-      # decode: the key range of a (row, kv head) is split only as far as needed to put one work-group of four waves on every compute unit
-      # (at head_dim 256 about a thousand single waves on the device), in chunks of at least a key block per wave.  Attention with its merging
-      # pass and the o adapter, head_dim 128, us in 1 | 2 | 4 | 8 chunks or so: 16 rows x 8 kv heads x 700 keys 20.2 | 16.9 | 19.0 | 20.4, 1500 keys
-      # 32.8 | 24.7 | 25.8 | 27.6, 8 rows x 1000 24.2 | 18.0 | 15.5 | 17.1, 32 rows x 750 23.6 | 25.1 | 26.6 | 30.4.  Two to a unit, of many keys, are cut in
-      # halves, which even out what the units have: 40 rows x 1280 52.6 | 44.2, 60 rows 59.2 | 58.0 (32 rows 33.3 | 35.0).
+      # decode: the key range of a (row, kv head) is split only as far as needed to put one work-group of four waves on every compute unit,
+      # in chunks of at least a key block per wave or so.  Attention with its merging pass and the o adapter, us in 1 | 2 | 4 | 8 chunks or so:
+      # 8 kv heads of 128, 16 rows x 700 keys 20.2 | 16.9 | 19.0 | 20.4, 1500 keys 32.8 | 24.7 | 25.8 | 27.6, 8 rows x 1000 24.2 | 18.0 | 15.5 |
+      # 17.1, 32 rows x 750 23.6 | 25.1 | 26.6 | 30.4; one kv head of 256, 64 rows x 288 18.5 | 14.2 | 12.0 | 14.7, 16 rows x 1200 48 | 30 | 21.7 | 15.7
+      # (12 chunks 14.6).  Two to a unit, of many keys, are cut in halves, which even out what the units have: 40 rows x 8 x 1280 52.6 | 44.2,
+      # 60 rows 59.2 | 58.0 (32 rows 33.3 | 35.0).
       kv_chunk = 0
       waves = B * cfg.num_kv_heads
       if T == 1 and S > 64:
-        if cfg.head_dim > 128:
-          n_chunks = min(math.ceil(1024 / waves), S // 32)
-        else:
-          n_chunks = 2 if 256 <= waves <= 512 and S > 1024 else max(1, min(256 // waves, math.ceil(S / 128)))
-        kv_chunk = max(32 if cfg.head_dim > 128 else 128, math.ceil(S / n_chunks / 32) * 32)
+        n_chunks = 2 if 256 <= waves <= 512 and S > 1024 else max(1, min(256 // waves, math.ceil(S / 128)))
+        kv_chunk = math.ceil(S / n_chunks / 32) * 32
         if kv_chunk >= S:
           kv_chunk = 0
     self.kv_chunk = kv_chunk
