@@ -2412,3 +2412,54 @@ def test_decode_attention_of_several_waves_per_chunk(gpu, S, Hq, Hkv, dh, chunk,
     diff = (got - ref[:, :, 0].float()).abs()[live]
     assert live.any() and diff.max().item() <= 2.0 ** -6 * max(1.0, ref[live].abs().max().item()), (col, diff.max().item())
     assert (got[~live] == 0).all()
+
+
+@pytest.mark.parametrize("M,K,N,batch,ldx,ldy,relu2", [
+    (1, 16, 1, 1, 16, 1, False),             # one turn of the k range, one row and column
+    (16, 2048, 512, 1, 2048, 512, False),
+    (33, 144, 75, 1, 148, 77, True),         # ragged everywhere, output rows off 16-byte alignment
+    (70, 4112, 1000, 1, 4112, 1000, False),  # k turns that the waves do not share evenly
+    (1300, 48, 1664, 1, 48, 1664, False),    # tiles of 128: half a step of k at the end
+    (1537, 2064, 1025, 1, 2064, 1028, True),
+    (40, 64, 96, 9, 64, 96, False),          # a batch, few tiles and many
+    (300, 256, 640, 9, 256, 640, False),
+])
+def test_dense_linear_in_32_bits(gpu, M, K, N, batch, ldx, ldy, relu2):
+  """Few rows and many, against the products in 64 bits: every element within K roundings of its products' magnitudes."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  x, w = rnd((batch, M, ldx), 401).to(gpu), rnd((batch, N, K), 402).to(gpu)
+  y = torch.full((batch, M, ldy), float("nan"), device=gpu)
+  d = L.DenseDesc()
+  d.M, d.K, d.N, d.dtype, d.split_k, d.batch = M, K, N, ops.DTYPES[torch.float32], 1, batch
+  d.x, d.ldx, d.w, d.y, d.ldy = x.data_ptr(), ldx, w.data_ptr(), y.data_ptr(), ldy
+  d.epilogue = L.TNX_EPI_RELU2 if relu2 else L.TNX_EPI_F32
+  d.x_stride, d.w_stride, d.y_stride = M * ldx, N * K, M * ldy
+  ops.dense_linear(d)
+  xd, wd = x[..., :K].cpu().double(), w.cpu().double()
+  want, size = xd @ wd.transpose(1, 2).contiguous(), xd.abs() @ wd.abs().transpose(1, 2).contiguous()
+  bound = (K + 1) * 2.0 ** -24 * size
+  if relu2:
+    want, bound = want.clamp_min(0) ** 2, bound * (2 * want.abs() + bound) + 2.0 ** -23 * want ** 2
+  got = y.cpu().double()
+  assert ((got[..., :N] - want).abs() <= bound).all() and got[..., N:].isnan().all()
+
+
+@pytest.mark.parametrize("K,N,counts,x_div", [(48, 75, (0, 3, 17, 0, 1), 1), (256, 512, (130, 0, 1, 301), 1), (2048, 256, (9, 40, 31, 0), 2)])
+def test_dense_experts_in_32_bits(gpu, K, N, counts, x_div):
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  E, n = len(counts), sum(counts)
+  x, w = rnd(((n + x_div - 1) // x_div, K), 403).to(gpu), rnd((E, N, K), 404).to(gpu)
+  route = torch.randperm(n, generator=torch.Generator().manual_seed(1)).to(torch.int32).to(gpu)
+  offsets = torch.tensor([0] + [int(v) for v in np.cumsum(counts)], dtype=torch.int32, device=gpu)
+  y = torch.full((n, N), float("nan"), device=gpu)
+  d = L.DenseDesc()
+  d.M, d.K, d.N, d.dtype, d.batch, d.split_k = n, K, N, ops.DTYPES[torch.float32], 1, 1
+  d.x, d.ldx, d.w, d.w_stride, d.epilogue, d.y, d.ldy = x.data_ptr(), K, w.data_ptr(), N * K, L.TNX_EPI_F32, y.data_ptr(), N
+  d.n_experts, d.x_div, d.offsets, d.sorted_route = E, x_div, offsets.data_ptr(), route.data_ptr()
+  ops.dense_linear(d)
+  for e, (a0, a1) in enumerate(zip(offsets.tolist()[:-1], offsets.tolist()[1:])):
+    r = route[a0:a1].long()
+    xe, we = x[r // x_div].cpu().double(), w[e].cpu().double()
+    assert ((y[r].cpu().double() - xe @ we.T).abs() <= (K + 1) * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()

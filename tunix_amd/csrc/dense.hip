@@ -2,7 +2,7 @@
 //
 // bf16: the weights live in HBM once, in the fragment order of tnx_dense_expand.  Calls with many
 // rows take the kernel of qgemm_pre.h; calls with few rows take dense_rows_kernel below,
-// which streams the same copy.  fp32: a plain tiled kernel in true 32-bit arithmetic.
+// which streams the same copy.  fp32: the 32-bit MFMAs, true 32-bit arithmetic.
 //
 // Two forms run several weights of one shape in a launch: a batch (every row through every weight, e.g.
 // one per head) and experts (a row goes to the weights its routes name, rows sorted by expert).
@@ -240,62 +240,203 @@ void dense_rows_kernel(const DenseArgs a) {
   }
 }
 
-// fp32: 64 x 64 tile, 256 threads, 4 x 4 outputs each; K a multiple of 16
+// ---- fp32 ------------------------------------------------------------------------------------------
+// In the 32-bit MFMAs: 256 products and sums per clock and compute unit, twice what the vector unit does, each rounded as a fused multiply-add.
+// K is a multiple of 16, N and M are whatever they are: rows and columns past the end repeat the last one and are not stored.
+// Products are formed transposed (weights as the A operand): a lane owns four consecutive columns of one row.
+typedef float f32x16v __attribute__((ext_vector_type(16)));
+
+// the operands of this work-group, and its rows [m0, m_end); false: it has none
+struct F32Tile {
+  const float *x, *w;
+  float* y;
+  int64_t m0, m_end;
+};
 template <int MODE>
-__global__ __launch_bounds__(256) void dense_f32_kernel(const DenseArgs a) {
-  __shared__ float xs[16][68], wsh[16][68];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int64_t n0 = (int64_t)blockIdx.x * 64, K = a.K, N = a.N, ldy = a.ldy;
-  int64_t m0 = (int64_t)blockIdx.y * 64, M = a.M;
-  const float* x = reinterpret_cast<const float*>(a.x);
-  const float* w = reinterpret_cast<const float*>(a.w);
-  float* y = reinterpret_cast<float*>(a.y);
+__device__ __forceinline__ bool f32_tile(const DenseArgs& a, int rows, F32Tile& t) {
+  t.x = reinterpret_cast<const float*>(a.x);
+  t.w = reinterpret_cast<const float*>(a.w);
+  t.y = reinterpret_cast<float*>(a.y);
+  t.m0 = (int64_t)blockIdx.y * rows;
+  t.m_end = a.M;
   if constexpr (MODE == kBatch) {
-    x += blockIdx.z * a.x_stride;
-    w += blockIdx.z * a.w_stride;
-    y += blockIdx.z * a.y_stride;
+    t.x += blockIdx.z * a.x_stride;
+    t.w += blockIdx.z * a.w_stride;
+    t.y += blockIdx.z * a.y_stride;
   }
   if constexpr (MODE == kExperts) {
     int expert, first_row, end_row;
-    if (!find_block(a.offsets, a.n_experts, 64, (int)blockIdx.y, expert, first_row, end_row)) return;
-    m0 = first_row;
-    M = end_row;
-    w += expert * a.w_stride;
+    if (!find_block(a.offsets, a.n_experts, rows, (int)blockIdx.y, expert, first_row, end_row)) return false;
+    t.m0 = first_row;
+    t.m_end = end_row;
+    t.w += expert * a.w_stride;
   }
-  const int lr = tid >> 2, lk = (tid & 3) * 4;
-  int64_t xrow = m0 + lr;
-  if constexpr (MODE == kExperts) xrow = xrow < M ? a.sorted_route[xrow] / a.x_div : 0;
-  float acc[4][4] = {};
-  for (int64_t k0 = 0; k0 < K; k0 += 16) {
-    f32x4 xv = f32x4{0.f, 0.f, 0.f, 0.f}, wv = xv;
-    if (m0 + lr < M) xv = *reinterpret_cast<const f32x4*>(x + xrow * a.ldx + k0 + lk);
-    if (n0 + lr < N) wv = *reinterpret_cast<const f32x4*>(w + (n0 + lr) * K + k0 + lk);
-    __syncthreads();
+  return true;
+}
+// row of x that row m of the tile's range reads (experts: m counts sorted routes)
+template <int MODE>
+__device__ __forceinline__ const float* f32_x_row(const DenseArgs& a, const F32Tile& t, int64_t m) {
+  m = min(m, t.m_end - 1);
+  if constexpr (MODE == kExperts) m = a.sorted_route[m] / a.x_div;
+  return t.x + m * a.ldx;
+}
+template <int MODE>
+__device__ __forceinline__ void f32_store(const DenseArgs& a, const F32Tile& t, int64_t m, int64_t col, f32x4 v) {
+  if (m >= t.m_end) return;
+  if constexpr (MODE == kExperts) m = a.sorted_route[m];
+  if (a.epilogue == TNX_EPI_RELU2) v = square_relu(v);
+  float* y = t.y + m * a.ldy + col;
+  if (col + 4 <= a.N && ((uintptr_t)y & 15) == 0) {
+    *reinterpret_cast<f32x4*>(y) = v;
+  } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      xs[lk + e][lr] = xv[e];
-      wsh[lk + e][lr] = wv[e];
+    for (int e = 0; e < 4; ++e)
+      if (col + e < a.N) y[e] = v[e];
+  }
+}
+
+// Few rows: 16 * RT rows x 16 columns per work-group, whose waves take the k range in turns of 16 and meet through LDS.  Bound by the stream
+// of the weights, which go straight into registers, four turns ahead: the lanes of a quarter-wave hold four k each of 16 columns.
+template <int MODE, int RT, int KS>
+__global__ __launch_bounds__(64 * KS) void dense_f32_rows_kernel(const DenseArgs a) {
+  constexpr int P = 4;
+  __shared__ __align__(16) f32x4 red[KS][RT][64];
+  const int tid = threadIdx.x, lane = tid & 63, lm = lane & 15, lq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  F32Tile t;
+  if (!f32_tile<MODE>(a, 16 * RT, t)) return;
+  const int64_t n0 = (int64_t)blockIdx.x * 16;
+  const float* w = t.w + min(n0 + lm, a.N - 1) * a.K + 4 * lq;
+  const float* x[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) x[rt] = f32_x_row<MODE>(a, t, t.m0 + rt * 16 + lm) + 4 * lq;
+  const int turns = (int)(a.K / 16), n = wave < turns ? (turns - wave + KS - 1) / KS : 0;   // of this wave: wave, wave + KS, ...
+  f32x4 acc[RT], wr[P], xr[P][RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto load = [&](int i, int p) {
+    const int64_t k = (int64_t)(min(wave, turns - 1) + max(min(i, n - 1), 0) * KS) * 16;
+    wr[p] = *reinterpret_cast<const f32x4*>(w + k);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) xr[p][rt] = *reinterpret_cast<const f32x4*>(x[rt] + k);
+  };
+#pragma unroll
+  for (int p = 0; p < P - 1; ++p) load(p, p);
+  for (int i = 0; i < n; i += P) {
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      load(i + u + P - 1, (u + P - 1) % P);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i + u < n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[u][e], xr[u][rt][e], acc[rt], 0, 0, 0);
     }
-    __syncthreads();
+  }
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const f32x4 av = *reinterpret_cast<const f32x4*>(&xs[k][ty * 4]);
-      const f32x4 bv = *reinterpret_cast<const f32x4*>(&wsh[k][tx * 4]);
+  for (int rt = 0; rt < RT; ++rt) red[wave][rt][lane] = acc[rt];
+  __syncthreads();
+  if (wave >= RT) return;
+  f32x4 v = red[0][wave][lane];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+  for (int s = 1; s < KS; ++s) v += red[s][wave][lane];
+  if (n0 + 4 * lq < a.N) f32_store<MODE>(a, t, t.m0 + wave * 16 + lm, n0 + 4 * lq, v);
+}
+
+// Many rows: 128 x 128 per work-group of four waves, a wave 64 x 64; steps of 32 k through two LDS buffers (rows of 128 bytes, whose 16-byte
+// chunks are swizzled by the row so that sixteen rows' reads of one chunk hit all banks), the next one's operands in registers meanwhile.
+// Bound by the matrix pipe: 122 TFLOP/s at 2400 x 2048 -> 16384.
+template <int MODE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_f32_tile_kernel(const DenseArgs a) {
+  __shared__ __align__(16) f32x4 tile[2][2][128 * 8];   // buffer, [weights | x], [row][chunk]
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  F32Tile t;
+  if (!f32_tile<MODE>(a, 128, t)) return;
+  const int64_t n0 = (int64_t)blockIdx.x * 128;
+  // thread: chunk tid % 8 of rows tid / 8 + 32 c
+  const int ch = tid & 7, r0 = tid >> 3;
+  const float *wp[4], *xp[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += av[i] * bv[j];
+  for (int c = 0; c < 4; ++c) {
+    wp[c] = t.w + min(n0 + r0 + 32 * c, a.N - 1) * a.K + 4 * ch;
+    xp[c] = f32_x_row<MODE>(a, t, t.m0 + r0 + 32 * c) + 4 * ch;
+  }
+  f32x4 wv[4], xv[4];
+  auto fetch = [&](int64_t k0) {
+    const bool in = k0 + 4 * ch < a.K;   // (K is a multiple of 16: of the last step perhaps half)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      wv[c] = in ? *reinterpret_cast<const f32x4*>(wp[c] + k0) : f32x4{0.f, 0.f, 0.f, 0.f};
+      xv[c] = in ? *reinterpret_cast<const f32x4*>(xp[c] + k0) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
+  };
+  auto at = [](int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); };
+  f32x16v acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  fetch(0);
+  int buf = 0;
+  for (int64_t k0 = 0; k0 < a.K; k0 += 32) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      tile[buf][0][at(r0 + 32 * c, ch)] = wv[c];
+      tile[buf][1][at(r0 + 32 * c, ch)] = xv[c];
+    }
+    __syncthreads();   // (the other buffer's readers are behind this barrier by one step: it is free in the next)
+    if (k0 + 32 < a.K) fetch(k0 + 32);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      f32x4 wf[2], xf[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        wf[i] = tile[buf][0][at(wn * 64 + i * 32 + l32, 2 * u + lh)];
+        xf[i] = tile[buf][1][at(wm * 64 + i * 32 + l32, 2 * u + lh)];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j][e], xf[i][e], acc[i][j], 0, 0, 0);
+    }
+    buf ^= 1;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int64_t row = m0 + ty * 4 + i;
-    if (row >= M) break;
-    if constexpr (MODE == kExperts) row = a.sorted_route[row];
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (n0 + tx * 4 + j < N) y[row * ldy + n0 + tx * 4 + j] = a.epilogue == TNX_EPI_RELU2 ? fmaxf(acc[i][j], 0.f) * fmaxf(acc[i][j], 0.f) : acc[i][j];
-  }
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const int64_t col = n0 + wn * 64 + j * 32 + 8 * b + 4 * lh;
+        if (col < a.N)
+          f32_store<MODE>(a, t, t.m0 + wm * 64 + i * 32 + l32, col, f32x4{acc[i][j][4 * b], acc[i][j][4 * b + 1], acc[i][j][4 * b + 2], acc[i][j][4 * b + 3]});
+      }
+}
+
+// Which form: a round of 128 x 128 tiles over the device takes as long as some 2700 blocks of 32 x 16 (experts: a tile is as good as full from
+// 33 rows on).  us, few rows | tiles | the 64 x 64 tiles of the vector unit that were here before, K = 2048:
+//   N = 2048   8 rows 8.8 | 146 | 122   64: 15 | 147 | 122   400: 88 | 148 | 122   800: 163 | 149 | 129   2400: 472 | 263 | 282
+//   N = 16384  8 rows 36 | 149 | 138    64: 110 | 150 | 141  128: 210 | 151 | 154  400: 644 | 267 | 399   2400: 3725 | 1318 | 2043
+// K = 8192, N = 2048: 8 rows 31 | 578 | 528, 400 rows 302 | 583 | 527.  Error against 64 bits, K = 2048: 2.9e-7 | 8.1e-7 | 8.1e-7.
+template <int MODE>
+void launch_f32(hipStream_t st, const DenseArgs& a, int64_t batch) {
+  auto blocks = [&](int64_t rows) { return MODE == kExperts ? a.M / rows + std::min<int64_t>(a.n_experts, a.M) : cdiv(a.M, rows); };
+  const int64_t rows = MODE == kExperts ? cdiv(a.M, (int64_t)a.n_experts) : a.M;   // of a weight
+  const int64_t rounds = cdiv(cdiv(a.M, 128) * cdiv(a.N, 128) * batch, 256);
+  const bool few = (MODE == kExperts ? rows <= 32 : cdiv(a.M, 32) * cdiv(a.N, 16) * batch < 2700 * rounds) && blocks(rows <= 16 ? 16 : 32) <= 65535;
+  constexpr int KS = 8;   // (sixteen waves: 8.2 us for 7.1 at a row of 2048 -> 2048, the same at 8192 -> 2048)
+  auto launch = [&](auto kernel, int64_t tile_rows, int64_t tile_cols, int threads) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)cdiv(a.N, tile_cols), (unsigned)blocks(tile_rows), (unsigned)batch), dim3((unsigned)threads), 0, st, a);
+  };
+  if (!few) launch(dense_f32_tile_kernel<MODE>, 128, 128, 256);
+  else if (rows <= 16) launch(dense_f32_rows_kernel<MODE, 1, KS>, 16, 16, 64 * KS);
+  else launch(dense_f32_rows_kernel<MODE, 2, KS>, 32, 16, 64 * KS);
 }
 
 template <int MODE>
@@ -333,10 +474,9 @@ extern "C" int tnx_dense_linear(void* stream, const tnx_dense_desc* d) {
     const int64_t blocks = experts ? d->M / 64 + (d->n_experts < d->M ? d->n_experts : d->M) : cdiv(d->M, 64);
     TNX_REQUIRE(blocks <= 65535, "dense_linear: too many rows in one call");
     TNX_REQUIRE(d->x_stride % 4 == 0 && d->w_stride % 4 == 0, "dense_linear: operands of a batch must stay 16-byte aligned");
-    const dim3 grid((unsigned)cdiv(d->N, 64), (unsigned)blocks, batch ? (unsigned)d->batch : 1u);
-    if (experts) hipLaunchKernelGGL(dense_f32_kernel<kExperts>, grid, dim3(256), 0, st, a);
-    else if (batch) hipLaunchKernelGGL(dense_f32_kernel<kBatch>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(dense_f32_kernel<kPlain>, grid, dim3(256), 0, st, a);
+    if (experts) launch_f32<kExperts>(st, a, 1);
+    else if (batch) launch_f32<kBatch>(st, a, d->batch);
+    else launch_f32<kPlain>(st, a, 1);
     TNX_CHECK_LAUNCH("dense_f32");
     return TNX_OK;
   }
