@@ -6,12 +6,14 @@
 //   gated_chunk_kernel   prompts: 32 tokens at a time on MFMAs; a long prompt is cut into spans that run in
 //                        parallel, their start states formed by a scan over spans
 //   gated_step_kernel    one token per sequence: one pass over the state, optionally the heads' norms behind it
-//   gated_any_kernel     any sizes and fp32: token by token
+//   gated_token_kernel   fp32 prompts, and bf16 ones of odd sizes: token by token, the state in registers
+//   gated_any_kernel     any sizes: token by token
 #include <string.h>
 
 #include <mutex>
 
 #include "decoder.h"
+#include "state_scan.h"
 
 namespace {
 
@@ -83,6 +85,33 @@ __global__ __launch_bounds__(256) void gated_any_kernel(const GateArgs a, const 
   // rows in front of the sequence: defined values for the norms behind
   for (int64_t t = 0; t < min((int64_t)max(0, start - col0), a.T); ++t)
     for (int d = tid; d < a.dv; d += 256) a.o[(b * a.T + t) * a.o_ld + hv + d] = 0.f;
+}
+
+// Prompts token by token with the state in registers (state_scan.h); grid (H, columns / 64, B).  2 x 1200 tokens of 16 heads of 128 x 128 in fp32:
+// 25.2 ms before, when the state went through memory with every token, 0.96 now.
+template <int R, typename T>
+__global__ __launch_bounds__(256) void gated_token_kernel(const GateArgs a, const RowSrc<T> src, const RowSrc<float> fs) {
+  const int h = blockIdx.x, d0 = blockIdx.y * kScanCols;
+  const int64_t b = blockIdx.z, hk = (int64_t)h * a.dk, hv = (int64_t)h * a.dv;
+  const int col0 = *a.col_ptr, start = a.starts[b];
+  const int64_t t0 = min((int64_t)max(0, start - col0), a.T), row0 = b * a.T;
+  float* o = a.o + row0 * a.o_ld + hv;
+  // rows in front of the sequence: defined values for the norms behind
+  for (int64_t e = threadIdx.x; e < t0 * kScanCols; e += 256) {
+    const int d = d0 + (int)(e % kScanCols);
+    if (d < a.dv) o[e / kScanCols * a.o_ld + d] = 0.f;
+  }
+  if (t0 >= a.T) return;
+  state_scan<R, true>(
+      t0, a.T, a.dk, a.dv, d0, col0 <= start, 0.f, a.state + (b * a.H + h) * (int64_t)a.dk * a.dv,
+      [&](int64_t t, int i) {
+        return f32x4{src.get(row0 + t, a.q_off + hk + i), fs.get(row0 + t, a.f_off + hk + i) + a.bias[hk + i], a.lower[hk + i], 0.f};
+      },
+      [](const f32x4& raw, float& q, float& k, float& f) {
+        q = silu_f32(raw[0]);
+        forget<false>(raw[1], raw[2], f, k);
+      },
+      [&](int64_t t, int d) { return src.get(row0 + t, a.v_off + hv + d); }, [&](int64_t t, int d, float v) { o[t * a.o_ld + d] = v; });
 }
 
 // One token: a thread owns four value columns and every NG-th row of the state.
@@ -674,6 +703,14 @@ extern "C" int tnx_gated_state(void* stream, const tnx_gated_state_desc* d) {
     a.ws = d->ws;
     TNX_REQUIRE(a.n_spans == 1 || d->ws, "gated_state: a long prompt needs the workspace of tnx_gated_state_ws_bytes");
     return plain ? launch_chunk_any(st, a, s16, fs) : launch_chunk_any(st, a, s32, fs);
+  }
+  if (d->T > 1 && d->dk <= 256 && cdiv(d->dv, kScanCols) <= 65535) {
+    const dim3 grid((unsigned)d->H, (unsigned)cdiv(d->dv, kScanCols), (unsigned)d->B);
+    auto launch = [&](auto kernel, const auto& src) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, a, src, fs); };
+    if (y16) d->dk <= 128 ? launch(gated_token_kernel<32, uint16_t>, s16) : launch(gated_token_kernel<64, uint16_t>, s16);
+    else d->dk <= 128 ? launch(gated_token_kernel<32, float>, s32) : launch(gated_token_kernel<64, float>, s32);
+    TNX_CHECK_LAUNCH("gated_token");
+    return TNX_OK;
   }
   const size_t lds = (size_t)3 * d->dk * 4;
   if (y16) hipLaunchKernelGGL(gated_any_kernel<uint16_t>, per, dim3(256), lds, st, a, s16, fs);

@@ -6,12 +6,14 @@
 //   lightning_chunk_kernel   prompts: 64 tokens at a time on MFMAs; a long prompt is cut into spans
 //                            that run in parallel, their start states formed by a scan over spans
 //   lightning_step_kernel    one token per sequence: one pass over the state
-//   lightning_any_kernel     any sizes and fp32: token by token
+//   lightning_token_kernel   fp32 prompts, and bf16 ones of odd sizes: token by token, the state in registers
+//   lightning_any_kernel     any sizes: token by token
 #include <string.h>
 
 #include <mutex>
 
 #include "decoder.h"
+#include "state_scan.h"
 
 namespace {
 
@@ -69,6 +71,32 @@ __global__ __launch_bounds__(256) void lightning_any_kernel(const LightArgs a, c
   // rows in front of the sequence: defined values for the norms behind
   for (int64_t t = 0; t < min((int64_t)max(0, start - col0), a.T); ++t)
     for (int d = tid; d < a.dv; d += 256) a.o[(b * a.T + t) * a.o_ld + (int64_t)h * a.dv + d] = 0.f;
+}
+
+// Prompts token by token with the state in registers (state_scan.h); grid (H, columns / 64, B).  2 x 1200 tokens of 16 heads of 128 x 128 in fp32:
+// 25.4 ms before, when the state went through memory with every token, 0.75 now.
+template <int R, typename T>
+__global__ __launch_bounds__(256) void lightning_token_kernel(const LightArgs a, const RowSrc<T> src) {
+  const int h = blockIdx.x, d0 = blockIdx.y * kScanCols;
+  const int64_t b = blockIdx.z;
+  const int col0 = *a.col_ptr, start = a.starts[b];
+  const int64_t t0 = min((int64_t)max(0, start - col0), a.T), row0 = b * a.T;
+  float* o = a.o + row0 * a.o_ld + (int64_t)h * a.dv;
+  // rows in front of the sequence: defined values for the norms behind
+  for (int64_t e = threadIdx.x; e < t0 * kScanCols; e += 256) {
+    const int d = d0 + (int)(e % kScanCols);
+    if (d < a.dv) o[e / kScanCols * a.o_ld + d] = 0.f;
+  }
+  if (t0 >= a.T) return;
+  state_scan<R, false>(
+      t0, a.T, a.dk, a.dv, d0, col0 <= start, a.decay[h], a.state + (b * a.H + h) * (int64_t)a.dk * a.dv,
+      [&](int64_t t, int i) { return f32x4{src.get(row0 + t, (int64_t)h * a.dk + i), src.get(row0 + t, a.k_off + (int64_t)h * a.dk + i), 0.f, 0.f}; },
+      [](const f32x4& raw, float& q, float& k, float&) {
+        q = silu_f32(raw[0]);
+        k = silu_f32(raw[1]);
+      },
+      [&](int64_t t, int d) { return silu_f32(src.get(row0 + t, a.v_off + (int64_t)h * a.dv + d)); },
+      [&](int64_t t, int d, float v) { o[t * a.o_ld + d] = v; });
 }
 
 // One token: a thread owns four value columns and every NG-th row of the state.
@@ -483,6 +511,14 @@ extern "C" int tnx_lightning(void* stream, const tnx_lightning_desc* d) {
     if (d->dk <= 64) return launch_chunk<2>(st, a);
     if (d->dk <= 128) return launch_chunk<4>(st, a);
     return launch_chunk<8>(st, a);
+  }
+  if (d->T > 1 && d->dk <= 256 && cdiv(d->dv, kScanCols) <= 65535) {
+    const dim3 grid((unsigned)d->H, (unsigned)cdiv(d->dv, kScanCols), (unsigned)d->B);
+    auto launch = [&](auto kernel, const auto& src) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, a, src); };
+    if (bf) d->dk <= 128 ? launch(lightning_token_kernel<32, uint16_t>, s16) : launch(lightning_token_kernel<64, uint16_t>, s16);
+    else d->dk <= 128 ? launch(lightning_token_kernel<32, float>, s32) : launch(lightning_token_kernel<64, float>, s32);
+    TNX_CHECK_LAUNCH("lightning_token");
+    return TNX_OK;
   }
   const size_t lds = (size_t)2 * d->dk * 4;
   if (bf) hipLaunchKernelGGL(lightning_any_kernel<uint16_t>, per, dim3(256), lds, st, a, s16);
