@@ -938,9 +938,9 @@ int launch_qgemm_wide_grouped(hipStream_t st, const QLArgs& a) {
 // Shapes the many-row kernels take: enough rows to fill the device with its tiles, no k split,
 // a bf16 output whose rows can be written in 16-byte chunks, and an adapter (if any) of rank
 // <= 64 none of whose 256-column windows touches more than two segments.
-bool wide_shape(const QLArgs& a, int64_t min_rows = 512) {
+bool wide_shape(const QLArgs& a, int64_t min_rows = 512, int64_t min_tiles = 256) {
   if (a.split_k > 1 || a.next_tpart || a.M < min_rows) return false;
-  if (cdiv(a.M, kWideRows) * cdiv(a.N, kWideCols) < 256) return false;
+  if (cdiv(a.M, kWideRows) * cdiv(a.N, kWideCols) < min_tiles) return false;
   const bool mul = a.epilogue == TNX_EPI_SILU_MUL || a.epilogue == TNX_EPI_GELU_MUL;
   if (!mul && a.epilogue != TNX_EPI_STORE && a.epilogue != TNX_EPI_RESIDUAL) return false;
   if ((mul ? a.N / 2 : a.N) % 8 != 0 || ((uintptr_t)a.y & 15) != 0) return false;
@@ -1157,7 +1157,10 @@ int tnx_internal_wide_head(hipStream_t st, const tnx_lmhead_desc* d, float tempe
   // A dense head's copy is streamed at any row count: at a decode batch the launch is bound by
   // the weight stream, and this kernel re-reads the activations once per 256 columns where the
   // 128 x 128 head kernel re-reads them once per 128, as many bytes again as the weights.
-  if (!wide_shape(a, dense ? 1 : 512)) return 1;
+  // Short vocabularies leave part of the device without a tile, and the other kernel, whose tiles are half as wide, has its rows to re-read: us,
+  // that one | this, 32768 x 2048 16 rows 44.5 | 41.2, 32 rows 46.2 | 38.6, 128 rows 68 | 44; 50304 x 1024 32 rows 38.7 | 29.8; 16384 x 2048 16 rows
+  // 34.3 | 38.5, 32 rows 36.8 | 35.7, 64 rows 42.5 | 37.0; 32000 x 512 16 rows 17.8 | 21.7, 32 rows 20.3 | 18.5.
+  if (!(dense ? wide_shape(a, 1, a.M > 16 ? 1 : 128) : wide_shape(a))) return 1;
   a.y = nullptr;
   WideHead h{d->part, part_ent, d->targets, nvb, temperature, d->logits_out, nullptr, 0u, 0u, 0, nullptr, d->M, d->softcap};
   if (d->draw_id) {
