@@ -81,7 +81,7 @@ const char* tnx_last_error(void);
  * chunks to tnx_sink_attn_desc, an ungated form and shared weights to tnx_gated_norm_desc, TNX_EPI_RELU2, and
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
  * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora,
- * tnx_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric. */
+ * tnx_gqa_attn_lora, tnx_rope_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric. */
 #define TNX_ABI_VERSION_MAJOR 6
 #define TNX_ABI_VERSION_MINOR 3
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
@@ -374,6 +374,11 @@ int tnx_gqa_attn(void* stream, const tnx_attn_desc* h_desc);
  * (a_t bf16 [R, Hq * dh], R % 16 == 0).  Where the key range of a decode step is split over few chunks, the pass that
  * merges them takes the product too, whose sums are then added in another order. */
 int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld);
+/* tnx_qknorm_rope_kvwrite(r), then tnx_gqa_attn_lora (a_t null: tnx_gqa_attn) of the same rows, heads and caches; q lies in r->q_out.  A decode
+ * step whose qkv linear left up to eight partial planes takes one launch for the first two: q_out is not written then, and the step's own key
+ * enters the softmax as a block of its own. */
+int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t,
+                           int64_t t_ld);
 
 /* ---------------------------------------------------------------------------------------
  * Fused lm_head -> fp32 log-softmax statistics, never writing [M,V] logits:

@@ -2463,3 +2463,62 @@ def test_dense_experts_in_32_bits(gpu, K, N, counts, x_div):
     r = route[a0:a1].long()
     xe, we = x[r // x_div].cpu().double(), w[e].cpu().double()
     assert ((y[r].cpu().double() - xe @ we.T).abs() <= (K + 1) * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()
+
+
+@pytest.mark.parametrize("family,dh,Hq,Hkv,split,chunk,window,R", [
+    ("qwen3", 64, 4, 2, 4, 0, 0, 32),       # half a wave per head
+    ("qwen3", 128, 16, 2, 6, 96, 0, 16),    # ten heads of a pair of kv heads, split over chunks
+    ("gemma3", 256, 4, 1, 5, 128, 100, 32),
+    ("gemma3", 256, 16, 1, 8, 0, 0, 0),     # more heads than one batch of the waves takes, no adapter
+    ("llama3", 128, 6, 2, 3, 0, 0, 16),     # no norms, three heads in lanes of four
+    ("qwen3", 128, 8, 2, 9, 0, 0, 16),      # too many planes: the two launches
+])
+def test_norms_rotation_and_attention_in_one_launch(gpu, family, dh, Hq, Hkv, split, chunk, window, R):
+  """tnx_rope_gqa_attn_lora against the launches it stands for, at columns on both sides of the waves' shares: the cache bit for
+  bit, the output to a bf16 ulp (the step's own key enters the softmax as a block of its own)."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  from tunix_amd.model import rope_timescale
+  B, S = 3, 300
+  ld = (Hq + 2 * Hkv) * dh
+  g = torch.Generator().manual_seed(700 + dh)
+  ws = (torch.randn(split, B, ld, generator=g) * split ** -0.5).to(gpu)
+  norms = [(torch.randn(dh, generator=g) * 0.1 + (0.0 if family == "gemma3" else 1.0)).to(torch.bfloat16).to(gpu) for _ in range(2)]
+  ts = torch.from_numpy(rope_timescale(dh, 1e4)).to(gpu)
+  pos = torch.randint(0, 900, (B, S), generator=g, dtype=torch.int32).to(gpu)
+  tokens = torch.randint(1, 50, (B, S), generator=g, dtype=torch.int32)
+  tokens[1, :9] = 0
+  tokens = tokens.to(gpu)
+  kc0, vc0 = (torch.randn(B, Hkv, S, dh, generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+  a_t = torch.randn(R, Hq * dh, generator=g).to(torch.bfloat16).to(gpu) if R else None
+  for col in (0, 9, 31, 32, 127, 128, 160, 299):
+    colp = torch.tensor([col], dtype=torch.int32, device=gpu)
+    got = []
+    for one in (False, True):
+      kc, vc, q = kc0.clone(), vc0.clone(), torch.empty(B, Hq * dh, dtype=torch.bfloat16, device=gpu)
+      out, t = torch.empty_like(q), torch.zeros(B, 32, dtype=torch.bfloat16, device=gpu)
+      part = torch.empty(max(ops.attn_ws_bytes(B, 1, S, Hq, dh, chunk) // 4, 1), device=gpu)
+      rd, d = L.RopeDesc(), L.AttnDesc()
+      for x in (rd, d):
+        x.B, x.T, x.S, x.Hq, x.Hkv, x.dh = B, 1, S, Hq, Hkv, dh
+        x.kcache, x.vcache, x.col_ptr = kc.data_ptr(), vc.data_ptr(), colp.data_ptr()
+      rd.rope_flavor, rd.rope_scale, rd.timescale = {"llama3": L.TNX_ROPE_LLAMA, "qwen3": L.TNX_ROPE_QWEN3, "gemma3": L.TNX_ROPE_GEMMA3}[family], 2.0, ts.data_ptr()
+      rd.qk_norm = {"llama3": -1, "qwen3": L.TNX_NORM_QWEN3, "gemma3": L.TNX_NORM_GEMMA3}[family]
+      rd.norm_eps, rd.q_norm_w, rd.k_norm_w = 1e-6, norms[0].data_ptr(), norms[1].data_ptr()
+      rd.q_prescale = dh ** -0.5 if family == "gemma3" else 0.0
+      rd.qkv_ws, rd.split_k, rd.positions, rd.pos_ld, rd.q_out = ws.data_ptr(), split, pos.data_ptr(), S, q.data_ptr()
+      d.scale, d.window, d.q, d.out, d.ws = 0.0 if family == "gemma3" else dh ** -0.5, window, q.data_ptr(), out.data_ptr(), part.data_ptr()
+      d.tokens, d.tok_ld, d.kv_chunk = tokens.data_ptr(), S, chunk
+      if one:
+        ops.rope_gqa_attn_lora(rd, d, a_t, t)
+      else:
+        ops.rope_kvwrite(rd)
+        ops.gqa_attn(d)
+      torch.cuda.synchronize()
+      got.append((kc, vc, out.float(), t))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and not torch.equal(got[0][0], kc0), col
+    ref, out = got[0][2], got[1][2]
+    ulp = 2.0 ** (torch.floor(torch.log2(torch.maximum(ref.abs(), out.abs()).clamp_min(0.5))) - 7)
+    assert ((ref - out).abs() <= ulp).all(), (col, ((ref - out).abs() / ulp).max().item())
+    if R:
+      assert_down_projection(got[1][3][:, :R], got[1][2].to(torch.bfloat16), a_t)

@@ -310,6 +310,7 @@ SIGNATURES = {
     "tnx_attn_ws_bytes": (C.c_size_t, [_i64, _i64, _i64, _i32, _i32, _i32]),
     "tnx_gqa_attn": (_i32, [_p, C.POINTER(AttnDesc)]),
     "tnx_gqa_attn_lora": (_i32, [_p, C.POINTER(AttnDesc), _p, _i32, _p, _i64]),
+    "tnx_rope_gqa_attn_lora": (_i32, [_p, C.POINTER(RopeDesc), C.POINTER(AttnDesc), _p, _i32, _p, _i64]),
     "tnx_lmhead_nblocks": (_i64, [_i64]),
     "tnx_lmhead_logp": (_i32, [_p, C.POINTER(LmHeadDesc)]),
     "tnx_sample_topk_ws_bytes": (C.c_size_t, [_i64, _i64, _i32]),

@@ -14,6 +14,7 @@
 
 #include "common.h"
 #include "gemm_tile.h"   // dma16, raw_rsrc, tnx_wait_vm
+#include "rope_math.h"
 #include "row_adapter.h"
 
 // Register stages of the key-block ring (head_dim <= 128).  Two: one block in flight while one is
@@ -70,7 +71,8 @@ __device__ __forceinline__ float across_quarters(float x, F f) {
 // FUSE: 0 = q comes rotated, keys and values are in the cache; 1 = the fused rotation and cache
 // write of a decode step (below), qkv taken from the finished output or from any number of
 // partial planes; 2 = the same from at most eight partial planes and at most four query heads per
-// kv head (one set of 3 x 64 lanes x 16 bytes per plane), all fetched in one round trip.
+// kv head (one set of 3 x 64 lanes x 16 bytes per plane), all fetched in one round trip; 3 = any rotation, behind per-head norms or not, from
+// at most eight partial planes (RopeArgs), the heads divided among the work-group's waves.
 // W: waves of a work-group.  Of more than one (a decode step: T == 1) each takes an equal share of the key blocks that the work-group's
 // chunk of the cache holds by now, and they merge what they have through LDS: the pass that would merge them otherwise is a launch, and its partials
 // a round trip to memory.  32 heads on 8, with the o adapter's 64 columns behind it, us before | now: 16 rows x 192 keys 14.0 | 12.7, 700 keys 19.9 |
@@ -78,7 +80,8 @@ __device__ __forceinline__ float across_quarters(float x, F f) {
 // 64 rows x 288 14.7 | 12.0, 16 rows x 1200 21.7 | 14.6.
 constexpr int kAttnWaves = 4;
 template <int DH, int FUSE, bool TOKVEC, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128 || W > 1 ? 2 : 1, DH > 128 || W > 1 ? 2 : 1))) void attn_kernel(const AttnArgs a) {
+__device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) {
+  static_assert(FUSE != 3 || (W > 1 && DH <= 128), "the heads are divided among waves, a pair of dimensions per lane");
   constexpr int KS = DH / 32;                 // k-steps of the QK product
   constexpr int NH = DH > 128 ? DH / 128 : 1; // 128-column halves of V / O
   constexpr int NS = DH > 128 ? 1 : TNX_ATTN_NS;        // register stages of the key-block pipeline
@@ -91,6 +94,43 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128
   const unsigned bz = blockIdx.z;
   const int64_t b = FUSE != 0 ? bz : bz / a.QT;          // (the fused decode step has one query tile per row)
   const int qt = FUSE != 0 ? 0 : (int)(bz - (unsigned)b * a.QT);
+  // FUSE 3: this wave's first heads of the G + 2 of the (row, kv head), all planes at once, ahead of everything that waits for the column.
+  // Lane i has dimensions i and i + DH / 2.
+  constexpr int HB = 3, HALF = DH / 2;
+  const int il = min(lane, HALF - 1);
+  struct HeadPlanes {
+    float p1[HB][8], p2[HB][8];
+  };
+  auto load_heads = [&](int h0, HeadPlanes& hp) {
+    const int ld = (a.Hq + 2 * a.Hkv) * DH;
+    const int64_t plane = a.B * (int64_t)ld;
+#pragma unroll
+    for (int u = 0; u < HB; ++u) {
+      const int hs = min(h0 + u * W + wave, a.G + 1);
+      const int head = hs < a.G ? hkv * a.G + hs : (hs == a.G ? a.Hq + hkv : a.Hq + a.Hkv + hkv);
+      const float* src = r.ws + b * (int64_t)ld + (int64_t)head * DH + il;
+#pragma unroll
+      for (int z = 0; z < 8; ++z) {
+        const float* p = src + (int64_t)min(z, r.split_k - 1) * plane;
+        hp.p1[u][z] = p[0];
+        hp.p2[u][z] = p[HALF];
+      }
+    }
+  };
+  HeadPlanes hp;
+  float timescale = 1.f;
+  uint16_t wq[2] = {0, 0}, wk[2] = {0, 0};
+  if constexpr (FUSE == 3) {
+    load_heads(0, hp);
+    timescale = r.timescale[il];
+    if (r.qk_norm >= 0)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        wq[e] = r.q_norm_w[il + e * HALF];
+        wk[e] = r.k_norm_w[il + e * HALF];
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   const int col0 = *a.col_ptr;
 
   // query column of this lane (as B-fragment column and as softmax owner)
@@ -274,7 +314,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128
       }
   };
   // a wave's staged q / k / v, later its part of the output
-  __shared__ __align__(16) float stage[FUSE || W > 1 ? W : 1][FUSE ? 18 * DH : W > 1 ? 16 * DH : 1];
+  __shared__ __align__(16) float stage[FUSE || W > 1 ? W : 1][FUSE == 1 || FUSE == 2 ? 18 * DH : W > 1 ? 16 * DH : 1];
   {
     Stage sg[NS];
     const int kb0 = k_lo & ~31;
@@ -296,9 +336,63 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128
       fetch_query_id();
     }
     // the step's own key / value wait in LDS while the cached keys stream through the registers
-    __shared__ u32x4 park_w[W][FUSE ? KS + NH : 1][64];
-    auto& park = park_w[wave];
-    if constexpr (fused) {
+    constexpr bool parked = FUSE == 1 || FUSE == 2;
+    __shared__ u32x4 park_w[parked ? W : 1][parked ? KS + NH : 1][64];
+    auto& park = park_w[parked ? wave : 0];
+    __shared__ __align__(16) uint16_t rot[FUSE == 3 ? 18 * DH : 8];   // the rotated heads: queries, key, value
+    if constexpr (FUSE == 3) {
+      const float pos = (float)r.positions[b * r.pos_ld + col0];
+      load_block(min(k_lo & ~31, k_hi & ~31), sg[0]);
+      fetch_query_id();
+      float sn, cs;
+      rope_angle(r, pos, timescale, sn, cs);   // (while the planes arrive)
+      for (int h0 = 0; h0 < a.G + 2; h0 += HB * W) {
+        if (h0 > 0) load_heads(h0, hp);
+#pragma unroll
+        for (int u = 0; u < HB; ++u) {
+          const int hs = h0 + u * W + wave;
+          const bool is_v = hs > a.G, is_q = hs < a.G;
+          if (hs >= a.G + 2) continue;   // (uniform)
+          float x1 = 0.f, x2 = 0.f;
+#pragma unroll
+          for (int z = 0; z < 8; ++z)
+            if (z < r.split_k) {
+              x1 += hp.p1[u][z];
+              x2 += hp.p2[u][z];
+            }
+          x1 = rbf(x1);
+          x2 = rbf(x2);
+          if (!is_v) {
+            if (r.qk_norm >= 0) {
+              const float ms = finish_ms(wave_sum(lane < HALF ? sq_term(x1, r.qk_norm) + sq_term(x2, r.qk_norm) : 0.f), (float)DH, r.qk_norm);
+              x1 = norm_elem(x1, bf2f(is_q ? wq[0] : wk[0]), ms, r.norm_eps, r.qk_norm);
+              x2 = norm_elem(x2, bf2f(is_q ? wq[1] : wk[1]), ms, r.norm_eps, r.qk_norm);
+            }
+            float o1, o2;
+            rotate_pair(r, is_q, x1, x2, sn, cs, o1, o2);
+            x1 = o1;
+            x2 = o2;
+          }
+          if (lane < HALF) {
+            rot[hs * DH + lane] = f2bf(x1);
+            rot[hs * DH + lane + HALF] = f2bf(x2);
+          }
+        }
+      }
+      __syncthreads();
+      const u32x4* heads = reinterpret_cast<const u32x4*>(rot);
+#pragma unroll
+      for (int j = 0; j < KS; ++j)
+        if (qvalid) qf[j] = heads[(g * DH + j * 32 + lq * 8) / 8];
+      if (writer) {
+        const int64_t slot = ((b * a.Hkv + hkv) * a.S + ring_slot(col0, a.S)) * DH;
+        for (int c = lane; c < DH / 8; c += 64) {
+          *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(a.k) + slot + c * 8) = heads[a.G * DH / 8 + c];
+          *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(a.v) + slot + c * 8) = heads[(a.G + 1) * DH / 8 + c];
+        }
+      }
+    }
+    if constexpr (parked) {
       u32x4 kn[KS], vn[NH];
       // ---- this step's q (G heads), k and v of the kv head from the qkv linear's output, RoPE
       // applied as the stand-alone kernel does; the first key blocks are already in flight ----
@@ -509,13 +603,21 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128
       Stage& one = sg[0];
 #pragma unroll
       for (int j = 0; j < KS; ++j) {
-        one.kf[0][j] = park[j][lane];
+        if constexpr (parked) {
+          one.kf[0][j] = park[j][lane];
+        } else {   // (row 0 of the key fragment)
+          one.kf[0][j] = u32x4{0, 0, 0, 0};
+          if (lm == 0) one.kf[0][j] = *reinterpret_cast<const u32x4*>(&rot[FUSE == 3 ? a.G * DH + j * 32 + lq * 8 : 0]);
+        }
         one.kf[1][j] = u32x4{0, 0, 0, 0};
       }
 #pragma unroll
-      for (int h = 0; h < NH; ++h)
+      for (int h = 0; h < NH; ++h) {
 #pragma unroll
-        for (int sidx = 0; sidx < 8; ++sidx) one.vf[h][sidx] = sidx == 0 ? park[KS + h][lane] : u32x4{0, 0, 0, 0};
+        for (int sidx = 0; sidx < 8; ++sidx) one.vf[h][sidx] = u32x4{0, 0, 0, 0};
+        if constexpr (parked) one.vf[h][0] = park[KS + h][lane];
+        else if (lq == 0 && 8 * lm < (DH < 128 ? DH : 128)) one.vf[h][0] = *reinterpret_cast<const u32x4*>(&rot[FUSE == 3 ? (a.G + 1) * DH + h * 128 + 8 * lm : 0]);
+      }
       const int own_tok = tok[col0];
 #pragma unroll
       for (int sidx = 0; sidx < 8; ++sidx) one.tk[sidx] = own_tok;
@@ -620,6 +722,18 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128
       for (int jj = 0; jj < 8; jj += 4)
         *reinterpret_cast<f32x4*>(p + kPartPad + h * 128 + 8 * lm + jj) = f32x4{O[h][jj][i], O[h][jj + 1][i], O[h][jj + 2][i], O[h][jj + 3][i]};
   }
+}
+
+template <int DH, int FUSE, bool TOKVEC, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128 || W > 1 ? 2 : 1, DH > 128 || W > 1 ? 2 : 1))) void attn_kernel(const AttnArgs a) {
+  attn_body<DH, FUSE, TOKVEC, W>(a, RopeArgs{});
+}
+// Norms, rotation, the cache write and attention of a decode step in one launch: what it saves is the other one's gap and its trip through memory.
+// With the o adapter behind, us in two | one, 32 heads of 128 on 4, 160 keys: 1 row 12.9 | 12.7, 64 rows 16.1 | 14.8, 128 rows 21.7 | 19.0, 1000
+// keys 16 rows 18.6 | 18.6, 64 rows 33.2 | 31.8; 8 heads of 64 on 2: 1 row of 48 keys 10.2 | 9.1, 128 rows of 100 11.7 | 10.8.
+template <int DH, bool TOKVEC>
+__global__ __launch_bounds__(64 * kAttnWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_rope_kernel(const AttnArgs a, const RopeArgs r) {
+  attn_body<DH, 3, TOKVEC, kAttnWaves>(a, r);
 }
 
 // Many query positions per row (prefill, whole-sequence log-probability passes): the wave above
@@ -1262,8 +1376,16 @@ extern "C" size_t tnx_attn_ws_bytes(int64_t B, int64_t T, int64_t S, int Hq, int
   return (size_t)(B * T * Hq * n_chunks * (dh + kPartPad)) * sizeof(float);
 }
 
-// The attention launch; combine: and, of a split key range, the pass that merges its chunks.
-static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
+// Whether four waves share each chunk: of more than two key blocks, as long as two work-groups per compute unit hold them all (beyond, waves
+// enough of their own: 128 rows x 8 kv heads x 160 keys 21.9 us with one wave, 25.0 with four).
+static bool several_waves(const tnx_attn_desc* d, int n_chunks, int64_t keys_over) {
+  const int64_t chunk_keys = d->kv_chunk > 0 ? d->kv_chunk : d->S;
+  return d->T == 1 && (d->window > 0 ? std::min<int64_t>(chunk_keys, d->window) : chunk_keys) > keys_over && d->B * d->Hkv * n_chunks <= 512;
+}
+
+// The attention launch; combine: and, of a split key range, the pass that merges its chunks.  rope: what forms q and writes the step's
+// key and value in the same launch (checked by the caller), or null.
+static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine, const RopeArgs* rope = nullptr) {
   TNX_REQUIRE(d, "attn: null descriptor");
   TNX_REQUIRE(d->B > 0 && d->T > 0 && d->S > 0, "attn: B,T,S must be positive");
   TNX_REQUIRE(d->dh == 64 || d->dh == 128 || d->dh == 256, "attn: head_dim %d not in {64,128,256}", d->dh);
@@ -1318,10 +1440,7 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
     if (tv) hipLaunchKernelGGL((attn_kernel<DH, FUSE, true, W>), grid, dim3(64 * W), 0, st, a);
     else hipLaunchKernelGGL((attn_kernel<DH, FUSE, false, W>), grid, dim3(64 * W), 0, st, a);
   };
-  // several waves per chunk: of more than two key blocks, as long as two work-groups per compute unit hold them all (beyond, waves enough of their own:
-  // 128 rows x 8 kv heads x 160 keys 21.9 us with one wave, 25.0 with four)
-  const int64_t chunk_keys = d->kv_chunk > 0 ? d->kv_chunk : d->S;
-  const bool waves = d->T == 1 && (d->window > 0 ? std::min<int64_t>(chunk_keys, d->window) : chunk_keys) > 64 && d->B * d->Hkv * a.n_chunks <= 512;
+  const bool waves = several_waves(d, a.n_chunks, 64);
   auto launch_head_dim = [&](auto dh_c, auto fuse_c) {
     if (waves) launch_decode(dh_c, fuse_c, std::integral_constant<int, kAttnWaves>{});
     else launch_decode(dh_c, fuse_c, std::integral_constant<int, 1>{});
@@ -1370,7 +1489,15 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
     TNX_CHECK_LAUNCH("gqa_attn (tiles)");
     return TNX_OK;
   }
-  switch (d->dh) {
+  auto launch_rope = [&](auto dh_c) {
+    constexpr int DH = decltype(dh_c)::value;
+    if (tv) hipLaunchKernelGGL((attn_rope_kernel<DH, true>), grid, dim3(64 * kAttnWaves), 0, st, a, *rope);
+    else hipLaunchKernelGGL((attn_rope_kernel<DH, false>), grid, dim3(64 * kAttnWaves), 0, st, a, *rope);
+  };
+  if (rope) {
+    if (d->dh == 64) launch_rope(std::integral_constant<int, 64>{});
+    else launch_rope(std::integral_constant<int, 128>{});
+  } else switch (d->dh) {
     case 64: TNX_ATTN_LAUNCH(64, 0); break;
     case 128:
       if (a.rope_sin && a.qkv_ws && a.qkv_split <= 8 && G <= 4) TNX_ATTN_LAUNCH(128, 2);
@@ -1392,14 +1519,14 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine) {
 
 extern "C" int tnx_gqa_attn(void* stream, const tnx_attn_desc* d) { return gqa_attn(stream, d, true); }
 
-extern "C" int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld) {
+static int gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld, const RopeArgs* rope) {
   TNX_REQUIRE(d && a_t && t, "attn_lora: null pointer");
   TNX_REQUIRE(R > 0 && R % 16 == 0 && t_ld >= R, "attn_lora: R=%d must be a multiple of 16 and <= t_ld", R);
   const int64_t K = (int64_t)d->Hq * d->dh;
   TNX_REQUIRE(d->B > 0 && d->T > 0 && K > 0 && K % 32 == 0, "attn_lora: bad shape");
   const int n_chunks = d->kv_chunk > 0 ? (int)cdiv(d->S, d->kv_chunk) : 1;
   const bool one = d->T == 1 && n_chunks > 1 && attn_lora_one_launch(d->B, K, n_chunks, R);
-  const int rc = gqa_attn(stream, d, !one);
+  const int rc = gqa_attn(stream, d, !one, rope);
   if (rc != TNX_OK) return rc;
   if (!one) return tnx_lora_down(stream, d->out, d->B * d->T, K, a_t, R, t, t_ld);
   const RowAdapterArgs g{a_t, R, kCombineCols, t, t_ld};
@@ -1410,4 +1537,29 @@ extern "C" int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uin
   else n_chunks <= 4 ? launch(attn_combine_lora_kernel<2, kCombineCols, 4>) : launch(attn_combine_lora_kernel<2, kCombineCols, 8>);
   TNX_CHECK_LAUNCH("gqa_attn_combine_lora");
   return TNX_OK;
+}
+
+extern "C" int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld) {
+  return gqa_attn_lora(stream, d, a_t, R, t, t_ld, nullptr);
+}
+
+extern "C" int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t,
+                                      int64_t t_ld) {
+  TNX_REQUIRE(r && d, "rope_gqa_attn: null descriptor");
+  RopeArgs ra;
+  int rc = rope_args(r, ra);
+  if (rc) return rc;
+  TNX_REQUIRE(r->B == d->B && r->T == d->T && r->S == d->S && r->Hq == d->Hq && r->Hkv == d->Hkv && r->dh == d->dh && r->q_out == d->q &&
+                  r->kcache == d->kcache && r->vcache == d->vcache && r->col_ptr == d->col_ptr && !d->rope_sin,
+              "rope_gqa_attn: the two descriptors name different rows");
+  const int n_chunks = d->kv_chunk > 0 ? (int)cdiv(d->S, d->kv_chunk) : 1;
+  const bool aligned = (((uintptr_t)r->kcache | (uintptr_t)r->vcache) & 15) == 0;
+  // (heads of 256, which three chunks form again each: 1.0 us more per layer than in two launches, Gemma3-1B, 64 rows)
+  const bool one = r->qkv_ws && r->split_k <= 8 && aligned && (d->dh == 64 || d->dh == 128) && several_waves(d, n_chunks, 0);
+  if (!one) {
+    rc = tnx_qknorm_rope_kvwrite(stream, r);
+    if (rc) return rc;
+  }
+  const RopeArgs* rope = one ? &ra : nullptr;
+  return a_t ? gqa_attn_lora(stream, d, a_t, R, t, t_ld, rope) : gqa_attn(stream, d, true, rope);
 }

@@ -732,7 +732,8 @@ class Runner(HeadRunner):
           rd.qkv_ws, rd.split_k = self.splitk_ws.data_ptr(), qkv_split
         rd.col_ptr = col_ptr.data_ptr()
         rd.q_out, rd.kcache, rd.vcache = self.q.data_ptr(), kv.k.data_ptr(), kv.v.data_ptr()
-        ops.rope_kvwrite(rd)
+        if T > 1:
+          ops.rope_kvwrite(rd)
       ad = L.AttnDesc()
       ad.B, ad.T, ad.S = B, T, self.S
       ad.Hq, ad.Hkv, ad.dh = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
@@ -751,7 +752,9 @@ class Runner(HeadRunner):
         else:
           ad.qkv = self.qkv.data_ptr()
         ad.rope_sin, ad.rope_cos = self.rope_sin.data_ptr(), self.rope_cos.data_ptr()
-      if ly["o"].has_lora:
+      if T == 1 and not fuse_rope:
+        ops.rope_gqa_attn_lora(rd, ad, adapter(ly["o"]), self.t)
+      elif ly["o"].has_lora:
         ops.gqa_attn_lora(ad, ly["o"].a_t, self.t)
       else:
         ops.gqa_attn(ad)

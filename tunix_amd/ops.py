@@ -206,6 +206,12 @@ def gqa_attn_lora(desc: L.AttnDesc, a_t, t):
   L.check(L.lib().tnx_gqa_attn_lora(_stream(), C.byref(desc), _ptr(a_t), a_t.shape[0], _ptr(t), t.shape[1]), "tnx_gqa_attn_lora")
 
 
+def rope_gqa_attn_lora(rope: L.RopeDesc, desc: L.AttnDesc, a_t, t):
+  """rope_kvwrite, gqa_attn and, with a_t, lora_down of its output rows."""
+  L.check(L.lib().tnx_rope_gqa_attn_lora(_stream(), C.byref(rope), C.byref(desc), _ptr(a_t), 0 if a_t is None else a_t.shape[0], _ptr(t),
+                                         t.shape[1]), "tnx_rope_gqa_attn_lora")
+
+
 def lmhead_nblocks(V: int) -> int:
   return int(L.lib().tnx_lmhead_nblocks(V))
 
