@@ -1281,15 +1281,17 @@ __global__ void attn_combine_kernel(const float* ws, int64_t n_qvec, int dh, int
   out[qv * dh + d] = f2bf(L > 0.f ? o / L : 0.f);
 }
 
-// The same over whole rows of heads, with the LoRA down-projection of the row behind it (row_adapter.h): grid (groups of adapter
-// columns, rows); the first group writes the row.  The chunks' (max, sum) pairs of all heads go to LDS; a thread asks for its first eight
+// The same over whole rows of heads, with the LoRA down-projection of the row behind it (row_adapter.h); the first group of adapter columns
+// writes the row.  The chunks' (max, sum) pairs of all heads go to LDS; a thread asks for its first eight
 // chunks' outputs and its first columns of A ahead of them.
 template <int MAXC, int NB, int NCH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void attn_combine_lora_kernel(const float* ws, int heads, int dh, int n_chunks, uint16_t* out,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void attn_combine_lora_kernel(const float* ws, int64_t M, int heads, int dh, int n_chunks, uint16_t* out,
                                                                 const RowAdapterArgs g) {
   extern __shared__ float ml[];   // [heads][n_chunks][2]
   __shared__ float sums[4 * NB];
-  const int64_t row = blockIdx.y;
+  int group;
+  int64_t row;
+  if (!row_adapter_place(g, M, group, row)) return;
   const int K = heads * dh, pitch = dh + kPartPad;
   const float* base = ws + row * (int64_t)heads * n_chunks * pitch;
   RowAdapter<MAXC, NB> ad;
@@ -1312,7 +1314,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     p[c] = base + (int64_t)h * n_chunks * pitch + kPartPad + (e - h * dh);
     fetch(c, 0);
   }
-  ad.load(g, blockIdx.x, K);
+  ad.load(g, group, K);
   __syncthreads();
   u32x4 x[MAXC];
 #pragma unroll
@@ -1346,10 +1348,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     if (ch < K / 8) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) x[c][q] = L > 0.f ? pack2bf(o[2 * q] / L, o[2 * q + 1] / L) : 0u;
-      if (blockIdx.x == 0) *reinterpret_cast<u32x4*>(out + row * K + (int64_t)ch * 8) = x[c];
+      if (group == 0) *reinterpret_cast<u32x4*>(out + row * K + (int64_t)ch * 8) = x[c];
     }
   }
-  ad.finish(g, blockIdx.x, row, x, sums);
+  ad.finish(g, group, row, x, sums);
 }
 
 // Whether one launch merges the chunks and takes the adapter columns, sixteen per work-group: as long as a row's partials are 64 KB, which every
@@ -1529,10 +1531,10 @@ static int gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a
   const int rc = gqa_attn(stream, d, !one, rope);
   if (rc != TNX_OK) return rc;
   if (!one) return tnx_lora_down(stream, d->out, d->B * d->T, K, a_t, R, t, t_ld);
-  const RowAdapterArgs g{a_t, R, kCombineCols, t, t_ld};
-  const dim3 grid((unsigned)cdiv(R, g.nc), (unsigned)d->B);
+  RowAdapterArgs g{a_t, R, kCombineCols, t, t_ld, 0, 0};
+  const dim3 grid = row_adapter_grid(g, d->B, K, n_chunks * K * 4);
   const size_t lds = (size_t)d->Hq * n_chunks * 2 * sizeof(float);
-  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), lds, as_stream(stream), d->ws, d->Hq, d->dh, n_chunks, d->out, g); };
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), lds, as_stream(stream), d->ws, d->B, d->Hq, d->dh, n_chunks, d->out, g); };
   if (K <= 8 * 256) n_chunks <= 4 ? launch(attn_combine_lora_kernel<1, kCombineCols, 4>) : launch(attn_combine_lora_kernel<1, kCombineCols, 8>);
   else n_chunks <= 4 ? launch(attn_combine_lora_kernel<2, kCombineCols, 4>) : launch(attn_combine_lora_kernel<2, kCombineCols, 8>);
   TNX_CHECK_LAUNCH("gqa_attn_combine_lora");

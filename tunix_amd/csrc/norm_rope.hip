@@ -293,15 +293,17 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const NormRow n) {
   u32x4 last[MAXC];
   norm_row<MAXC, FLAVOR, IN>(n, blockIdx.x, true, red, last, [] {});
 }
-// The same with the LoRA down-projection of the row behind it (row_adapter.h): grid (groups of adapter columns, rows); the first
-// group writes the row.
+// The same with the LoRA down-projection of the row behind it (row_adapter.h); the first group of adapter columns writes the row.
 template <int MAXC, int FLAVOR, int IN, int NB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void rmsnorm_lora_kernel(const NormRow n, const RowAdapterArgs g) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void rmsnorm_lora_kernel(const NormRow n, int64_t M, const RowAdapterArgs g) {
   __shared__ float red[4], sums[4 * NB];
   u32x4 last[MAXC];
   RowAdapter<MAXC, NB> ad;
-  norm_row<MAXC, FLAVOR, IN>(n, blockIdx.y, blockIdx.x == 0, red, last, [&] { ad.load(g, blockIdx.x, n.D); });
-  ad.finish(g, blockIdx.x, blockIdx.y, last, sums);
+  int group;
+  int64_t row;
+  if (!row_adapter_place(g, M, group, row)) return;
+  norm_row<MAXC, FLAVOR, IN>(n, row, group == 0, red, last, [&] { ad.load(g, group, n.D); });
+  ad.finish(g, group, row, last, sums);
 }
 
 // The kernel is unrolled over its chunks (256 threads x 8 elements each): instantiated for 1, 2, 4
@@ -337,12 +339,12 @@ bool norm_lora_one_launch(int64_t M, int64_t D, int R) {
   if (M > 256 || D > 8 * 256 * 2) return false;
   return D > 8 * 256 ? M <= 16 && row_adapter_cols(M, R) <= 16 : row_adapter_cols(M, R) <= 32;
 }
-void launch_rmsnorm_lora(hipStream_t st, int64_t M, int flavor, int in, const NormRow& n, const RowAdapterArgs& g) {
-  const dim3 grid((unsigned)cdiv(g.R, g.nc), (unsigned)M);
+void launch_rmsnorm_lora(hipStream_t st, int64_t M, int flavor, int in, const NormRow& n, RowAdapterArgs g) {
+  const dim3 grid = row_adapter_grid(g, M, n.D, n.D * (in == kNormInPlanes ? 4 * n.split_k : in == kNormInRoutes ? 2 * n.split_k : 2));
   with_flavor(flavor, [&](auto f) {
     with_input(in, [&](auto i) {
       constexpr int F = decltype(f)::value, IN = decltype(i)::value;
-      const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, n, g); };
+      const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, n, M, g); };
       if (n.D > 8 * 256) g.nc <= 8 ? launch(rmsnorm_lora_kernel<2, F, IN, 8>) : launch(rmsnorm_lora_kernel<2, F, IN, 16>);
       else if (g.nc <= 16) g.nc <= 8 ? launch(rmsnorm_lora_kernel<1, F, IN, 8>) : launch(rmsnorm_lora_kernel<1, F, IN, 16>);
       else g.nc <= 24 ? launch(rmsnorm_lora_kernel<1, F, IN, 24>) : launch(rmsnorm_lora_kernel<1, F, IN, 32>);
@@ -671,7 +673,7 @@ extern "C" int tnx_norm_lora(void* stream, const tnx_norm_lora_desc* d) {
     separate = separate && apart(out, d->x, M * D * 2) && apart(out, d->ws, parts * M * D * 4) && apart(out, d->y_route, parts * M * D * 2) &&
                apart(out, d->res_pre, M * D * 2) && apart(out, d->res_post, M * D * 2);
   if (separate && norm_lora_one_launch(M, D, d->R)) {
-    launch_rmsnorm_lora(as_stream(stream), M, d->flavor, in, n, RowAdapterArgs{d->a_t, d->R, row_adapter_cols(M, d->R), d->t, d->t_ld});
+    launch_rmsnorm_lora(as_stream(stream), M, d->flavor, in, n, RowAdapterArgs{d->a_t, d->R, row_adapter_cols(M, d->R), d->t, d->t_ld, 0, 0});
     TNX_CHECK_LAUNCH("norm_lora");
     return TNX_OK;
   }

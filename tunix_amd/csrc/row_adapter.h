@@ -35,7 +35,17 @@ struct RowAdapterArgs {
   int R, nc;             // adapter columns, and how many of them a work-group takes
   uint16_t* t;
   int64_t t_ld;
+  int groups, c_shift;   // ceil(R / nc); log2 of the column sets (row_adapter_place)
 };
+// Which row and which group of columns a work-group takes.  Ids go round-robin to the eight XCDs, and the grid is a multiple of eight wide: XCD x has
+// column set x % c and row set x / c (c column sets, 8 / c row sets), so that its L2 fetches a part of the rows and a part of A and no
+// more.  (Shifts: with two divisions in front of the first load the gain was a third smaller.)  false: none.
+__device__ __forceinline__ bool row_adapter_place(const RowAdapterArgs& g, int64_t M, int& group, int64_t& row) {
+  const int x = blockIdx.x;
+  row = ((x & 7) >> g.c_shift) + ((int)blockIdx.y << (3 - g.c_shift));
+  group = (x & ((1 << g.c_shift) - 1)) + ((x >> 3) << g.c_shift);
+  return row < M && group < g.groups;
+}
 template <int MAXC, int NB>
 struct RowAdapter {   // NB: adapter columns of a work-group at most, all asked for at once (NB * MAXC loads of 16 bytes per thread)
   u32x4 a[NB][MAXC];
@@ -82,6 +92,24 @@ struct RowAdapter {   // NB: adapter columns of a work-group at most, all asked 
     }
   }
 };
+
+// The sets for operands of `row_bytes` per row, into g: those with which an XCD fetches least, as long as its 32 compute units have one
+// work-group each; and the grid.  (Every XCD with a part of the columns of all rows, as ids fall in a grid of groups x rows, Llama-8B layers of 16 rows
+// fetched 2.2 MB per norm and XCD instead of 1.3: the rollout of 16 rows 67.3 ms -> 65.4,
+// of Gemma3-1B, 64 rows, 90.2 -> 89.6, of Qwen3-MoE layers 27.4 -> 27.0; column sets alone 68.3, 96.4 and 27.8.)
+inline dim3 row_adapter_grid(RowAdapterArgs& g, int64_t M, int64_t K, int64_t row_bytes) {
+  g.groups = (int)cdiv(g.R, g.nc);
+  g.c_shift = 3;
+  int64_t least = -1;
+  for (int sh = 3; sh >= 0; --sh) {
+    const int64_t sets = 8 >> sh, bytes = M * row_bytes / sets + (int64_t)g.R * K * 2 * sets / 8;
+    if (cdiv(M, sets) * cdiv(g.groups, 1 << sh) <= 32 && (least < 0 || bytes < least)) {
+      g.c_shift = sh;
+      least = bytes;
+    }
+  }
+  return dim3((unsigned)(8 * cdiv(g.groups, 1 << g.c_shift)), (unsigned)cdiv(M, 8 >> g.c_shift));
+}
 
 // Columns per work-group: whole batches of eight, as few as leave at most one work-group per compute unit.
 inline int row_adapter_cols(int64_t M, int R) {
