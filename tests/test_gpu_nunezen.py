@@ -294,6 +294,21 @@ def test_attention_prompt_portions_and_steps(gpu, dtype, H, G, dk, dv, rot):
                   out_frag=dtype == BF and t % 4 == 0), t)
 
 
+@pytest.mark.parametrize("H,G,dk,dv,rot", [(8, 8, 32, 64, 0), (16, 1, 128, 128, 64), (6, 2, 192, 200, 48), (40, 2, 64, 64, 32)])
+@pytest.mark.parametrize("kv_chunk", [0, 96, 160])
+def test_one_position_shared_by_several_waves(gpu, H, G, dk, dv, rot, kv_chunk):
+  """Key blocks of a chunk divided among four waves (40 heads on 2: single waves), at columns on both sides of every share."""
+  S = 420
+  a = Attn(gpu, BF, H, G, dk, dv, rot, S, [0, 37, 300], sharp=3.0, seed=H)
+  a.run(0, 2)
+  col = 2
+  for t in (31, 32, 33, 64, 95, 96, 97, 128, 160, 161, 256, 319, 320, 383, 384, 419):
+    if t > col:
+      a.run(col, t - col)
+    a.check(a.run(t, 1, kv_chunk=kv_chunk), t)
+    col = t + 1
+
+
 @pytest.mark.parametrize("decoded", [False, True])
 @pytest.mark.parametrize("far", [0, 31, 32, 63, 64, 255, 298, 299])
 def test_one_key_stands_out(gpu, decoded, far):

@@ -426,14 +426,21 @@ class StackRunner(HeadRunner):
     return self._bufs[key]
 
   def _kv_chunk(self, m: AttentionMixer, given) -> int:
-    """Decode: split the key range only as far as needed to put about a thousand waves on the device."""
+    """Decode: split the key range only as far as needed to give every compute unit a work-group of four waves (more than sixteen heads per kv
+    head, whose tiles are single waves: to put about a thousand waves on the device)."""
     if given is not None:
       return given
     waves = self.B * m.kv_heads * math.ceil(self.T * (m.heads // m.kv_heads) / 16)
     S = min(self.S, m.chunk + 31) if m.chunk else self.S      # (columns that one position may see, from a block's edge on)
     if self.dtype != torch.bfloat16 or self.T != 1 or waves >= 1024 or S <= 64:
       return 0
-    n = min(math.ceil(1024 / waves), S // 32)
+    if m.heads // m.kv_heads > 16:
+      n = min(math.ceil(1024 / waves), S // 32)
+    else:
+      n = 2 if 256 <= waves <= 512 and S > 1024 else max(1, min(256 // waves, math.ceil(S / 128)))
+      # (the pass that merges chunks takes 3.8 us; a compute unit draws 28 KB of keys and values in one)
+      if S * (m.dim + m.vdim) * 2 / 28e3 * (1 - 1 / n) < 4.0:
+        n = 1
     chunk = max(32, _up(math.ceil(S / n), 32))
     return 0 if chunk >= S else chunk
 
