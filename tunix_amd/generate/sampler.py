@@ -220,7 +220,11 @@ class Sampler:
 
   def _captured(self, step) -> torch.cuda.CUDAGraph:
     """One call of `step` as a graph.  (torch.cuda.graph would wait for the device and give the allocator's cache back first: the prompts'
-    forward pass and this call then run one after the other, and the next call allocates everything anew.)"""
+    forward pass and this call then run one after the other, and the next call allocates everything anew.  Where the allocator's cache
+    holds nearly all of the memory it does have to come back: a capture allocates from the device.)"""
+    if torch.cuda.mem_get_info(self._transformer.device)[0] < 1 << 30:
+      torch.cuda.synchronize(self._transformer.device)
+      torch.cuda.empty_cache()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(torch.cuda.Stream(self._transformer.device)):   # (capture does not execute: nothing runs on this stream)
       graph.capture_begin()
