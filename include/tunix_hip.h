@@ -376,7 +376,7 @@ int tnx_gqa_attn(void* stream, const tnx_attn_desc* h_desc);
 int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld);
 /* tnx_qknorm_rope_kvwrite(r), then tnx_gqa_attn_lora (a_t null: tnx_gqa_attn) of the same rows, heads and caches; q lies in r->q_out.  A decode
  * step whose qkv linear left up to eight partial planes takes one launch for the first two: q_out is not written then, and the step's own key
- * enters the softmax as a block of its own. */
+ * enters the softmax as a block of its own where a chunk (or the window) holds more than 64 keys; of fewer the output is bit for bit that of the two. */
 int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t,
                            int64_t t_ld);
 

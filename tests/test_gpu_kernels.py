@@ -2466,6 +2466,8 @@ def test_dense_experts_in_32_bits(gpu, K, N, counts, x_div):
 
 
 @pytest.mark.parametrize("family,dh,Hq,Hkv,split,chunk,window,R", [
+    ("qwen3", 64, 8, 2, 4, 64, 0, 16),      # chunks of two key blocks, each by one wave
+    ("qwen3", 128, 6, 2, 5, 0, 50, 32),     # a window of up to three
     ("qwen3", 64, 4, 2, 4, 0, 0, 32),       # half a wave per head
     ("qwen3", 128, 16, 2, 6, 96, 0, 16),    # ten heads of a pair of kv heads, split over chunks
     ("gemma3", 256, 4, 1, 5, 128, 100, 32),
@@ -2475,7 +2477,7 @@ def test_dense_experts_in_32_bits(gpu, K, N, counts, x_div):
 ])
 def test_norms_rotation_and_attention_in_one_launch(gpu, family, dh, Hq, Hkv, split, chunk, window, R):
   """tnx_rope_gqa_attn_lora against the launches it stands for, at columns on both sides of the waves' shares: the cache bit for
-  bit, the output to a bf16 ulp (the step's own key enters the softmax as a block of its own)."""
+  bit, the output to a bf16 ulp (the step's own key enters the softmax as a block of its own), of one wave's keys bit for bit too."""
   from tunix_amd import _lib as L
   from tunix_amd import ops
   from tunix_amd.model import rope_timescale
@@ -2520,5 +2522,7 @@ def test_norms_rotation_and_attention_in_one_launch(gpu, family, dh, Hq, Hkv, sp
     ref, out = got[0][2], got[1][2]
     ulp = 2.0 ** (torch.floor(torch.log2(torch.maximum(ref.abs(), out.abs()).clamp_min(0.5))) - 7)
     assert ((ref - out).abs() <= ulp).all(), (col, ((ref - out).abs() / ulp).max().item())
+    if min(chunk or S, window or S) <= 64:
+      assert torch.equal(ref, out), col
     if R:
       assert_down_projection(got[1][3][:, :R], got[1][2].to(torch.bfloat16), a_t)

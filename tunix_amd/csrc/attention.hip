@@ -72,7 +72,7 @@ __device__ __forceinline__ float across_quarters(float x, F f) {
 // write of a decode step (below), qkv taken from the finished output or from any number of
 // partial planes; 2 = the same from at most eight partial planes and at most four query heads per
 // kv head (one set of 3 x 64 lanes x 16 bytes per plane), all fetched in one round trip; 3 = any rotation, behind per-head norms or not, from
-// at most eight partial planes (RopeArgs), the heads divided among the work-group's waves.
+// at most eight partial planes (RopeArgs), the heads divided among the work-group's waves; 4 = 3, the keys of at most two blocks by one wave.
 // W: waves of a work-group.  Of more than one (a decode step: T == 1) each takes an equal share of the key blocks that the work-group's
 // chunk of the cache holds by now, and they merge what they have through LDS: the pass that would merge them otherwise is a launch, and its partials
 // a round trip to memory.  32 heads on 8, with the o adapter's 64 columns behind it, us before | now: 16 rows x 192 keys 14.0 | 12.7, 700 keys 19.9 |
@@ -81,7 +81,12 @@ __device__ __forceinline__ float across_quarters(float x, F f) {
 constexpr int kAttnWaves = 4;
 template <int DH, int FUSE, bool TOKVEC, int W>
 __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) {
-  static_assert(FUSE != 3 || (W > 1 && DH <= 128), "the heads are divided among waves, a pair of dimensions per lane");
+  constexpr bool formed = FUSE >= 3;           // the heads come out of this launch's planes
+  // FUSE 4, few keys: one wave takes them all, the step's own among them, in the order and with the roundings of the launch without the
+  // rotation, for the same time (4.7 ms for a rollout of 32 steps at 48 columns, either way): divided, other last bits turned near-ties of
+  // a routed decoder's experts.
+  constexpr bool few = FUSE == 4;
+  static_assert(!formed || (W > 1 && DH <= 128), "the heads are divided among waves, a pair of dimensions per lane");
   constexpr int KS = DH / 32;                 // k-steps of the QK product
   constexpr int NH = DH > 128 ? DH / 128 : 1; // 128-column halves of V / O
   constexpr int NS = DH > 128 ? 1 : TNX_ATTN_NS;        // register stages of the key-block pipeline
@@ -94,7 +99,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
   const unsigned bz = blockIdx.z;
   const int64_t b = FUSE != 0 ? bz : bz / a.QT;          // (the fused decode step has one query tile per row)
   const int qt = FUSE != 0 ? 0 : (int)(bz - (unsigned)b * a.QT);
-  // FUSE 3: this wave's first heads of the G + 2 of the (row, kv head), all planes at once, ahead of everything that waits for the column.
+  // formed: this wave's first heads of the G + 2 of the (row, kv head), all planes at once, ahead of everything that waits for the column.
   // Lane i has dimensions i and i + DH / 2.
   constexpr int HB = 3, HALF = DH / 2;
   const int il = min(lane, HALF - 1);
@@ -120,7 +125,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
   HeadPlanes hp;
   float timescale = 1.f;
   uint16_t wq[2] = {0, 0}, wk[2] = {0, 0};
-  if constexpr (FUSE == 3) {
+  if constexpr (formed) {
     load_heads(0, hp);
     timescale = r.timescale[il];
     if (r.qk_norm >= 0)
@@ -153,8 +158,9 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
   // the chunk that owns the new token (of its waves the last, which has the fewest blocks)
   const bool writer = fused && col0 >= k_lo && col0 <= k_hi && wave == W - 1;
   if constexpr (W > 1) {
-    if (fused) k_hi = min(k_hi, col0 - 1);
-    const int first = k_lo & ~31, each = (max(k_hi - first + 32, 0) / 32 + W - 1) / W * 32;
+    constexpr int N = few ? 1 : W;
+    if (fused && !few) k_hi = min(k_hi, col0 - 1);
+    const int first = k_lo & ~31, each = (max(k_hi - first + 32, 0) / 32 + N - 1) / N * 32;
     k_lo = max(k_lo, first + wave * each);
     k_hi = min(k_hi, first + (wave + 1) * each - 1);
   }
@@ -166,8 +172,9 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
   }
   // in fused mode the step's own key / value never come from the cache: the loop stops one key
   // short and they are added from registers at the end
-  int key_hi = fused ? c_n - 1 : c_n;
-  if (fused) k_hi = min(k_hi, col0 - 1);
+  // (of few keys they take the place of what the cache held in their block)
+  int key_hi = fused && !few ? c_n - 1 : c_n;
+  if (fused && !few) k_hi = min(k_hi, col0 - 1);
 
   f32x4 O[NH][8];
 #pragma unroll
@@ -249,7 +256,20 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
             rtok, (uint32_t)(kb + (s < 4 ? 4 * lq + s : 16 + 4 * lq + (s - 4))) * 4u, 0, 0);
     }
   };
-  auto compute_block = [&](int kb, const Stage& sg) {
+  __shared__ __align__(16) uint16_t rot[formed ? 18 * DH : 8];   // the rotated heads: queries, key, value
+  auto compute_block = [&](int kb, Stage& sg) {
+    if constexpr (few) {
+      if (kb == (col0 & ~31)) {
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+          if (kb + tt * 16 + lm == col0)
+#pragma unroll
+            for (int j = 0; j < KS; ++j) sg.kf[tt][j] = *reinterpret_cast<const u32x4*>(&rot[a.G * DH + j * 32 + lq * 8]);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+          if (kb + 4 * lq + (s < 4 ? s : 12 + s) == col0) sg.vf[0][s] = *reinterpret_cast<const u32x4*>(&rot[(a.G + 1) * DH + vcol]);
+      }
+    }
     bool kvalid[8];
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
@@ -339,8 +359,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
     constexpr bool parked = FUSE == 1 || FUSE == 2;
     __shared__ u32x4 park_w[parked ? W : 1][parked ? KS + NH : 1][64];
     auto& park = park_w[parked ? wave : 0];
-    __shared__ __align__(16) uint16_t rot[FUSE == 3 ? 18 * DH : 8];   // the rotated heads: queries, key, value
-    if constexpr (FUSE == 3) {
+    if constexpr (formed) {
       const float pos = (float)r.positions[b * r.pos_ld + col0];
       load_block(min(k_lo & ~31, k_hi & ~31), sg[0]);
       fetch_query_id();
@@ -598,7 +617,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
         }
       }
     }
-    if (writer) {
+    if (writer && !few) {
       // the step's own key / value as a block of one key (at position col0) from registers
       Stage& one = sg[0];
 #pragma unroll
@@ -607,7 +626,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
           one.kf[0][j] = park[j][lane];
         } else {   // (row 0 of the key fragment)
           one.kf[0][j] = u32x4{0, 0, 0, 0};
-          if (lm == 0) one.kf[0][j] = *reinterpret_cast<const u32x4*>(&rot[FUSE == 3 ? a.G * DH + j * 32 + lq * 8 : 0]);
+          if (lm == 0) one.kf[0][j] = *reinterpret_cast<const u32x4*>(&rot[formed ? a.G * DH + j * 32 + lq * 8 : 0]);
         }
         one.kf[1][j] = u32x4{0, 0, 0, 0};
       }
@@ -616,7 +635,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
 #pragma unroll
         for (int sidx = 0; sidx < 8; ++sidx) one.vf[h][sidx] = u32x4{0, 0, 0, 0};
         if constexpr (parked) one.vf[h][0] = park[KS + h][lane];
-        else if (lq == 0 && 8 * lm < (DH < 128 ? DH : 128)) one.vf[h][0] = *reinterpret_cast<const u32x4*>(&rot[FUSE == 3 ? (a.G + 1) * DH + h * 128 + 8 * lm : 0]);
+        else if (lq == 0 && 8 * lm < (DH < 128 ? DH : 128)) one.vf[h][0] = *reinterpret_cast<const u32x4*>(&rot[formed ? (a.G + 1) * DH + h * 128 + 8 * lm : 0]);
       }
       const int own_tok = tok[col0];
 #pragma unroll
@@ -731,9 +750,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(DH > 128
 // Norms, rotation, the cache write and attention of a decode step in one launch: what it saves is the other one's gap and its trip through memory.
 // With the o adapter behind, us in two | one, 32 heads of 128 on 4, 160 keys: 1 row 12.9 | 12.7, 64 rows 16.1 | 14.8, 128 rows 21.7 | 19.0, 1000
 // keys 16 rows 18.6 | 18.6, 64 rows 33.2 | 31.8; 8 heads of 64 on 2: 1 row of 48 keys 10.2 | 9.1, 128 rows of 100 11.7 | 10.8.
-template <int DH, bool TOKVEC>
+template <int DH, bool TOKVEC, bool FEW>
 __global__ __launch_bounds__(64 * kAttnWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_rope_kernel(const AttnArgs a, const RopeArgs r) {
-  attn_body<DH, 3, TOKVEC, kAttnWaves>(a, r);
+  attn_body<DH, FEW ? 4 : 3, TOKVEC, kAttnWaves>(a, r);
 }
 
 // Many query positions per row (prefill, whole-sequence log-probability passes): the wave above
@@ -1491,14 +1510,19 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine, const Ro
     TNX_CHECK_LAUNCH("gqa_attn (tiles)");
     return TNX_OK;
   }
-  auto launch_rope = [&](auto dh_c) {
+  auto launch_rope = [&](auto dh_c, auto few_c) {
     constexpr int DH = decltype(dh_c)::value;
-    if (tv) hipLaunchKernelGGL((attn_rope_kernel<DH, true>), grid, dim3(64 * kAttnWaves), 0, st, a, *rope);
-    else hipLaunchKernelGGL((attn_rope_kernel<DH, false>), grid, dim3(64 * kAttnWaves), 0, st, a, *rope);
+    constexpr bool FEW = decltype(few_c)::value;
+    if (tv) hipLaunchKernelGGL((attn_rope_kernel<DH, true, FEW>), grid, dim3(64 * kAttnWaves), 0, st, a, *rope);
+    else hipLaunchKernelGGL((attn_rope_kernel<DH, false, FEW>), grid, dim3(64 * kAttnWaves), 0, st, a, *rope);
+  };
+  auto launch_rope_keys = [&](auto dh_c) {
+    if (waves) launch_rope(dh_c, std::false_type{});
+    else launch_rope(dh_c, std::true_type{});
   };
   if (rope) {
-    if (d->dh == 64) launch_rope(std::integral_constant<int, 64>{});
-    else launch_rope(std::integral_constant<int, 128>{});
+    if (d->dh == 64) launch_rope_keys(std::integral_constant<int, 64>{});
+    else launch_rope_keys(std::integral_constant<int, 128>{});
   } else switch (d->dh) {
     case 64: TNX_ATTN_LAUNCH(64, 0); break;
     case 128:
