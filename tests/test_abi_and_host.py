@@ -250,6 +250,25 @@ def test_split_k_choice_of_the_decode_linears():
   assert m._split_k(lin("w_gate", 1152, 13824, True), 64) == 3
 
 
+@pytest.mark.parametrize("override", [{}, {"wq": 4}])
+@pytest.mark.parametrize("rows", [1, 64, 127, 128, 129, 160, 1024, 16384])
+def test_partial_planes_have_room_at_every_row_count_of_a_runner(rows, override):
+  """A runner of many rows is called with fewer (the last group of prompts): the planes of a linear that splits there fit."""
+  import types
+  from tunix_amd.model import Runner
+  lin = lambda name, K, N, il=False: types.SimpleNamespace(names=[f"l0.{name}"], K=K, N=N, interleave2=il)
+  layers = [dict(qkv=lin("wq", 4096, 6144), o=lin("wo", 4096, 4096), gu=lin("w_gate", 4096, 28672, True), down=lin("w_down", 14336, 4096)),
+            dict(qkv=lin("wq", 512, 768), o=lin("wo", 512, 512), gu=lin("w_gate", 4096, 2048, True))]
+  r = Runner.__new__(Runner)
+  r.split_k_override, r.M, r.model = override, rows, types.SimpleNamespace(layers=layers)
+  room = r._split_floats()
+  for ly in layers:
+    for f in ly.values():
+      for M in list(range(1, min(rows, 300) + 1)) + [rows]:
+        split = r._split_k(f, M)
+        assert split == 1 or split * M * f.N <= room, (f.names, M, split)
+
+
 def test_split_k_leaves_no_empty_split_and_goes_on_for_long_contractions():
   import math
   import types

@@ -86,6 +86,10 @@ def test_per_token_logps_chunking_and_batching_are_invariant(tiny, gpu):
   # the fp32 summation order, far inside the tolerance of the path
   one_by_one = common.compute_per_token_logps(model, prompt, comp, pad_id=0, max_rows=40)
   assert (one_by_one - full).abs().max().item() <= 1e-2
+  # groups of 160 rows, whose linears run unsplit, and a last one of 40, whose linears split
+  again = np.concatenate([prompt, prompt[:1]]), np.concatenate([comp, comp[:1]])
+  ragged = common.compute_per_token_logps(model, *again, pad_id=0, max_rows=160)
+  assert torch.equal(ragged[:4], full) and (ragged[4] - full[0]).abs().max().item() <= 1e-2
 
 
 def test_packed_per_token_logps(tiny, gpu):

@@ -553,14 +553,7 @@ class Runner(HeadRunner):
     if M <= 1024 and not cfg.num_experts and model.layers and "gu" in model.layers[0]:
       n_planes = math.ceil(M / 128) * math.ceil(model.layers[0]["gu"].N / 128)
       self.next_tpart = torch.empty(n_planes * 8192, dtype=torch.float32, device=dev)
-    need = 1
-    for ly in model.layers:
-      for key in ("qkv", "o", "gu", "down"):
-        if key in ly:
-          sk = self._split_k(ly[key], M)
-          if sk > 1:
-            need = max(need, sk * M * ly[key].N)
-    self.splitk_ws = torch.empty(need, dtype=torch.float32, device=dev)
+    self.splitk_ws = torch.empty(self._split_floats(), dtype=torch.float32, device=dev)
     if kv_chunk is None:
       # decode: the key range of a (row, kv head) is split only as far as needed to put one work-group of four waves on every compute unit,
       # in chunks of at least a key block per wave or so.  Attention with its merging pass and the o adapter, us in 1 | 2 | 4 | 8 chunks or so:
@@ -582,6 +575,20 @@ class Runner(HeadRunner):
     self._init_head(B, D, bf, want_logits)
 
   # ---- building blocks -----------------------------------------------------------------------
+  SPLIT_ROWS = 128   # calls with more rows run unsplit
+
+  def _split_floats(self) -> int:
+    """Floats of the split linears' partial planes, for every row count up to the runner's own: a last group of prompts may have few enough rows
+    to split where a full one has not, and below SPLIT_ROWS the split does not depend on the rows."""
+    need = 1
+    for ly in self.model.layers:
+      for key in ("qkv", "o", "gu", "down"):
+        for M in {self.M, min(self.M, self.SPLIT_ROWS)} if key in ly else ():
+          sk = self._split_k(ly[key], M)
+          if sk > 1:
+            need = max(need, sk * M * ly[key].N)
+    return need
+
   def _split_k(self, f: FusedLinear, M: int) -> int:
     if f.names[0] in self.split_k_override:
       return self.split_k_override[f.names[0]]
@@ -590,7 +597,7 @@ class Runner(HeadRunner):
       return self.split_k_override[key]
     blocks = math.ceil(f.N / 128) * math.ceil(M / 128)
     ktiles = f.K // 128
-    if blocks >= 200 or M > 128:
+    if blocks >= 200 or M > self.SPLIT_ROWS:
       return 1
     # Eight splits, or so many that a split has four k-tiles, and as many as fill the device; more planes cost their consumer more
     # than the shorter splits save (the q|k|v planes may go to the attention kernel, which takes eight in one round trip).  Then no more than leave
