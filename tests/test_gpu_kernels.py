@@ -568,7 +568,9 @@ def test_rmsnorm_wide_rows_and_many_planes(gpu, family, D, split):
 
 
 @pytest.mark.parametrize("family,dh,Hq,Hkv", [("llama3", 128, 8, 2), ("qwen3", 64, 8, 2),
-                                               ("gemma3", 256, 4, 1)])
+                                               ("gemma3", 256, 4, 1),
+                                               # half a head is not whole waves
+                                               ("qwen3", 160, 3, 1), ("qwen3", 192, 4, 2), ("gemma3", 320, 2, 1), ("qwen3", 34, 2, 1)])
 def test_rope_kvwrite(gpu, family, dh, Hq, Hkv):
   from tunix_amd import _lib as L
   from tunix_amd import ops

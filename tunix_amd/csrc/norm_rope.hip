@@ -379,7 +379,7 @@ __global__ void embed_kernel(const uint16_t* table, int64_t V, int64_t D, const 
   }
 }
 
-// grid (B*T, Hq + 2*Hkv); max(64, dh/2) threads: thread i < dh/2 owns elements i and i + dh/2
+// grid (B*T, Hq + 2*Hkv); dh/2 threads, rounded up to whole waves (wave_sum): thread i < dh/2 owns elements i and i + dh/2
 // of one head; the other threads only take part in the reductions.
 // A decode step's launch is a chain of round trips to memory, so everything that needs no other load is asked for at
 // once, ahead of the first wait, and the angle is computed while the planes arrive.  64 rows of 4 + 2 heads of 256 from eight planes, us
@@ -714,7 +714,7 @@ extern "C" int tnx_qknorm_rope_kvwrite(void* stream, const tnx_rope_desc* d) {
     TNX_CHECK_LAUNCH("qknorm_rope_kvwrite (rows)");
     return TNX_OK;
   }
-  dim3 grid((unsigned)(d->B * d->T), (unsigned)(d->Hq + 2 * d->Hkv)), block(d->dh / 2 < 64 ? 64 : d->dh / 2);
+  dim3 grid((unsigned)(d->B * d->T), (unsigned)(d->Hq + 2 * d->Hkv)), block((unsigned)(cdiv(d->dh / 2, 64) * 64));
   if (d->qkv_ws) hipLaunchKernelGGL(rope_kernel<true>, grid, block, 0, as_stream(stream), a);
   else hipLaunchKernelGGL(rope_kernel<false>, grid, block, 0, as_stream(stream), a);
   TNX_CHECK_LAUNCH("qknorm_rope_kvwrite");
