@@ -14,6 +14,7 @@ from oracle import model_ref as MR
 from oracle import rl_ref
 from oracle import sampler_ref as SR
 from oracle import utils_ref as U
+from tests import kezolix_cases, kuzezen_cases, lapevik_cases, nunezen_cases
 
 pytestmark = pytest.mark.gpu
 
@@ -148,6 +149,39 @@ def test_graph_replay_equals_eager(tiny, gpu):
   for x, y in zip(a.tokens, b.tokens):
     np.testing.assert_array_equal(x, y)
   np.testing.assert_array_equal(np.asarray(a.logprobs), np.asarray(b.logprobs))
+
+
+@pytest.mark.parametrize("rows", [3, 130])
+@pytest.mark.parametrize("family,name,dtype", [("qlora", "tiny", "bf16")] + [
+    (f, n, t) for f, cases in (("nunezen", nunezen_cases), ("lapevik", lapevik_cases), ("kuzezen", kuzezen_cases), ("kezolix", kezolix_cases))
+    for n in sorted(cases.CONFIGS) for t in ("bf16", "fp32")])
+def test_a_captured_step_allocates_nothing(tiny, gpu, family, name, dtype, rows):
+  """Every buffer of a decode step is there before its capture: what the capture allocated (and filled) would be done again by
+  every replay."""
+  import importlib
+  from tunix_amd.generate import CacheConfig, Sampler
+  from tunix_amd.generate.utils import IdTokenizer
+  if family == "qlora":
+    model = tiny[2]
+  else:
+    model = importlib.import_module(f"tests.test_gpu_{family}").model_of(name, 3, torch.bfloat16 if dtype == "bf16" else torch.float32, gpu)[2]
+  counts = []
+
+  class Watched(Sampler):
+    def _captured(self, step):
+      def watched():
+        count = lambda: torch.cuda.memory_stats(gpu)["allocation.all.allocated"]
+        before = count()
+        step()
+        counts.append(count() - before)
+      return super()._captured(watched)
+
+  V = model.cfg.vocab_size
+  prompts = [np.arange(2 + b % 5, 9, dtype=np.int32) % V for b in range(rows)]
+  sampler = Watched(model, IdTokenizer(V, pad_id=0, eos_id=1), CacheConfig(64))
+  for kw in (dict(return_logprobs=True), dict(temperature=1.0, top_p=1.0), dict(temperature=1.0, top_p=0.9, top_k=10)):
+    sampler(prompts, 5, max_prompt_length=16, eos_tokens=[-1], **kw)
+  assert counts == [0, 0, 0]
 
 
 def test_sampler_contract(tiny, gpu):

@@ -413,6 +413,9 @@ class StackRunner(HeadRunner):
       self._head_logits = self.logits if self.logits is not None else torch.empty(
           B, cfg.vocab_size, dtype=torch.float32, device=dev)
     self.residual_sink = None   # called with the fp32 residual [M, D] behind every layer run
+    if T == 1:
+      for args in self._step_buffers():
+        self._buf(*args)
 
   # ---- building blocks -----------------------------------------------------------------------
   def _buf(self, name: str, cols: int, dtype=None, rows: int | None = None) -> torch.Tensor:
@@ -424,6 +427,49 @@ class StackRunner(HeadRunner):
         rows = _up(self.M, 128) if self.frag else self.M
       self._bufs[key] = torch.zeros(rows, cols, dtype=self.dtype if dtype is None else dtype, device=self.model.device)
     return self._bufs[key]
+
+  def _step_buffers(self):
+    """`_buf`'s arguments for everything that a pass over one token per row asks for: such a pass is captured, and a buffer made
+    meanwhile would be filled again by every replay."""
+    m, M, f32, pad = self.model, self.M, torch.float32, lambda n, value: ops.sink_attn_pad(n, value, self.dtype)
+    yield "h", m.Dp
+    if m.loop_in is not None:
+      yield "cat", m.loop_in.Kp
+    if self.cfg.parallel:
+      yield "h2", m.Dp
+    for ly in m.layers:
+      x, e = ly["spec"].mixer, ly["spec"].mlp
+      if isinstance(x, ParallelMixer):
+        yield "q", x.left.heads * pad(x.left.dim, True)
+        yield "mixed", ly["left"]["out"].Kp
+        yield "state_out", x.right.heads * x.right.vdim, f32
+        yield "gated", ly["right"]["out"].Kp
+      elif isinstance(x, AttentionMixer):
+        yield "q", x.heads * pad(x.dim, False)
+        yield "attn", ly["out"].Kp
+      elif isinstance(x, LatentMixer):
+        fk, fv = ly["absorb_k"], ly["absorb_v"]
+        yield "cq", ly["uq"].Kp
+        yield "q_un", x.heads * fk.Kp, None, M
+        yield "q", x.heads * ops.latent_row(x.kv_rank, x.rot_dim, self.dtype), None, M
+        yield "latent_out", x.heads * fv.Kp, None, M
+        yield "heads", x.heads * fv.N, None, M
+        yield "gated", ly["out"].Kp
+      else:
+        if isinstance(x, SsdMixer):
+          if not ops.ssd_step_ok(x.state, x.vdim):
+            yield "conv", _up(x.channels, 8), None, M
+          yield "state_out", x.inner, f32
+        elif not (isinstance(x, GatedStateMixer) and ops.gated_state_step_ok(x.dim, x.vdim)):
+          yield "state_out", x.heads * x.vdim, f32
+        yield "gated", ly["out"].Kp
+      if isinstance(e, ExpertsMlp):
+        yield "act", ly["down"].Kp, None, M * e.routes
+        yield "routes", ly["down"].N, None, M * e.routes
+        if "shared_up" in ly:
+          yield "shared", ly["shared_down"].Kp
+      elif "gu" in ly:
+        yield "act", ly["down"].Kp
 
   def _kv_chunk(self, m: AttentionMixer, given) -> int:
     """Decode: split the key range only as far as needed to give every compute unit a work-group of four waves (more than sixteen heads per kv
