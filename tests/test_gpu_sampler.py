@@ -184,6 +184,35 @@ def test_a_captured_step_allocates_nothing(tiny, gpu, family, name, dtype, rows)
   assert counts == [0, 0, 0]
 
 
+@pytest.mark.parametrize("free,given_back", [(64 << 20, True), (512 << 20, False)])
+def test_a_capture_gives_the_cache_back_only_where_a_graph_has_no_room(tiny, gpu, monkeypatch, free, given_back):
+  """A graph takes some MiB of the device, and no more than the room that a capture asks for."""
+  from tunix_amd.generate import CacheConfig, Sampler
+  from tunix_amd.generate.utils import IdTokenizer
+  cfg, w, model = tiny
+  taken, emptied = [], []
+
+  class Watched(Sampler):
+    def _captured(self, step):
+      torch.cuda.synchronize(gpu)
+      before = torch.cuda.mem_get_info(gpu)[0]
+      with monkeypatch.context() as m:
+        empty = torch.cuda.empty_cache
+        m.setattr(torch.cuda, "mem_get_info", lambda device=None: (free, 288 << 30))
+        m.setattr(torch.cuda, "empty_cache", lambda: (emptied.append(1), empty()))
+        graph = super()._captured(step)
+      taken.append(before - torch.cuda.mem_get_info(gpu)[0])
+      return graph
+
+  sampler = Watched(model, IdTokenizer(cfg.vocab_size, pad_id=0, eos_id=1), CacheConfig(64))
+  prompts = _prompts(4, 16, cfg.vocab_size, 7)
+  a = sampler(prompts, 20, eos_tokens=[-1])
+  assert bool(emptied) == given_back and taken[0] < Sampler.CAPTURE_ROOM
+  b = Sampler(model, sampler.tokenizer, CacheConfig(64), use_graph=False)(prompts, 20, eos_tokens=[-1])
+  for x, y in zip(a.tokens, b.tokens):
+    np.testing.assert_array_equal(x, y)
+
+
 def test_sampler_contract(tiny, gpu):
   """Errors, eos truncation, echo, pad_output, return_logits (tunix/generate/sampler.py:868-1011)."""
   from tunix_amd.generate import CacheConfig, Sampler

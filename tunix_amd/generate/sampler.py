@@ -218,11 +218,14 @@ class Sampler:
     """sampler.py:692-736: one token per row from the cached state."""
     self._sample(runner, self.forward_step(runner, st), st, mode)
 
+  CAPTURE_ROOM = 128 << 20
+
   def _captured(self, step) -> torch.cuda.CUDAGraph:
     """One call of `step` as a graph.  (torch.cuda.graph would wait for the device and give the allocator's cache back first: the prompts'
-    forward pass and this call then run one after the other, and the next call allocates everything anew.  Where the allocator's cache
-    holds nearly all of the memory it does have to come back: a capture allocates from the device.)"""
-    if torch.cuda.mem_get_info(self._transformer.device)[0] < 1 << 30:
+    forward pass and this call then run one after the other, and the next call allocates everything anew.  A step allocates nothing, its
+    runner's buffers are there; the graph itself takes 4 to 6 MiB from the device, of two or of 26 layers.  Only where the allocator's cache
+    leaves the device less than CAPTURE_ROOM does it have to come back.)"""
+    if torch.cuda.mem_get_info(self._transformer.device)[0] < self.CAPTURE_ROOM:
       torch.cuda.synchronize(self._transformer.device)
       torch.cuda.empty_cache()
     graph = torch.cuda.CUDAGraph()
