@@ -284,3 +284,16 @@ def test_split_k_leaves_no_empty_split_and_goes_on_for_long_contractions():
     for n in (128, 640, 1152, 4096, 12800):
       s = m._split_k(lin("wo", 128 * kt, n), 8)
       assert 1 <= s <= 16 and (s - 1) * math.ceil(kt / s) < kt
+
+
+def test_a_metric_takes_a_term_with_a_gradient_in_place():
+  """What aggregate_loss returns is added to in place by terms that ask for a gradient, and carries it."""
+  import torch
+  from tunix_amd.rl import common as C
+  aux = torch.tensor(2.0, requires_grad=True)
+  m = C._metric(torch.tensor([3.0, 4.0]), 1.0)
+  m.unreduced_sum += 0.5 * aux
+  total = m.compute()
+  assert total.item() == 1.0
+  total.backward()
+  assert aux.grad.item() == 0.125

@@ -209,7 +209,7 @@ class WeightedMetric:
 
 
 def _metric(out: torch.Tensor, min_denom: float) -> WeightedMetric:
-  total, denom = out.unbind(0)
+  total, denom = out[0], out[1]   # (two views of their own: an in-place sum with a term that asks for a gradient is refused for unbind's)
   metric = WeightedMetric(total, denom, min_denom=min_denom)
   metric._pair = total, denom
   return metric
