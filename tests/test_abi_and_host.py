@@ -297,3 +297,18 @@ def test_a_metric_takes_a_term_with_a_gradient_in_place():
   assert total.item() == 1.0
   total.backward()
   assert aux.grad.item() == 0.125
+
+
+def test_a_metric_that_left_the_device_is_computed_where_it_is():
+  """A saved metric whose numbers are loaded to the host (or were there, or changed their type) takes the tensor operations."""
+  import io
+  import torch
+  from tunix_amd.rl import common as C
+  m = C._metric(torch.tensor([3.0, 4.0]), 1.0)
+  assert m.compute().item() == 0.75
+  f = io.BytesIO()
+  torch.save(m, f)
+  f.seek(0)
+  assert torch.load(f, weights_only=False, map_location="cpu").compute().item() == 0.75   # (written above by this test)
+  m.unreduced_sum.data = m.unreduced_sum.data.double()
+  assert m.compute().item() == 0.75 and m.compute().dtype == torch.float64

@@ -373,6 +373,27 @@ def test_weighted_metric_in_one_launch(gpu, total, denom):
       assert m.compute().item() == (m.unreduced_sum * m.compute_scale()).item()
 
 
+def test_weighted_metric_off_the_one_launch(gpu):
+  """A metric loaded to the host, of another type, or with a forward-mode tangent: the tensor operations."""
+  import io
+  from torch.autograd import forward_ad
+  from tunix_amd.rl import common as C
+  new = lambda: C._metric(torch.tensor([3.0, 4.0], device=gpu), 1.0)
+  f = io.BytesIO()
+  torch.save(new(), f)
+  for where in ("cpu", gpu):
+    f.seek(0)
+    got = torch.load(f, weights_only=False, map_location=where).compute()   # (written above by this test)
+    assert got.item() == 0.75 and got.device.type == torch.device(where).type
+  m = new()
+  m.denominator.data = m.denominator.data.double()
+  assert m.compute().item() == 0.75 and m.compute().dtype == torch.float64
+  with forward_ad.dual_level():
+    m = new()
+    m.unreduced_sum.add_(forward_ad.make_dual(torch.tensor(1.0, device=gpu), torch.tensor(2.0, device=gpu)))
+    assert forward_ad.unpack_dual(m.compute()).tangent.item() == 0.5
+
+
 def test_aggregate_loss_argument_errors(gpu):
   from tunix_amd.rl import common as C
   x, k = torch.ones(2, 3, device=gpu), torch.ones(2, 3, device=gpu)

@@ -180,6 +180,13 @@ def compute_kl_divergence(per_token_logps: torch.Tensor, ref_per_token_logps: to
   return out
 
 
+def _plain(a: torch.Tensor, b: torch.Tensor) -> bool:
+  """Whether a kernel may read the two numbers in place of autograd, forward mode and other devices' operations."""
+  at, tangent = a.get_device(), torch.autograd.forward_ad.unpack_dual   # (-1: on the host)
+  return (at >= 0 and at == b.get_device() == torch._C._cuda_getDevice() and a.dtype is b.dtype is torch.float32
+          and not (a.requires_grad or b.requires_grad) and tangent(a)[1] is None and tangent(b)[1] is None)
+
+
 @dataclasses.dataclass
 class WeightedMetric:
   """A sum and the weight to divide it by (tunix/sft/utils.py:185-219); both stay on the device."""
@@ -199,9 +206,8 @@ class WeightedMetric:
 
   def compute(self) -> torch.Tensor:
     pair = self.__dict__.get("_pair")
-    # what `aggregate_loss` left here itself, plain 32-bit values on the device: one launch for nine
-    if pair is not None and self.unreduced_sum is pair[0] and self.denominator is pair[1] and not (
-        pair[0].requires_grad or pair[1].requires_grad):
+    # what `aggregate_loss` left here itself, as long as it is plain 32-bit values on the device: one launch for nine
+    if pair is not None and self.unreduced_sum is pair[0] and self.denominator is pair[1] and _plain(*pair):
       out = torch.empty_like(pair[0])
       ops.weighted_metric(pair[0], pair[1], self.eps, self.min_denom, out)
       return out
