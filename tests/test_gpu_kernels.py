@@ -1842,6 +1842,47 @@ def test_attention_and_down_projection(gpu, B, Hq, Hkv, dh, S, kv_chunk, R, wind
   assert bool((t[:, R:] == 7.0).all())
 
 
+@pytest.mark.parametrize("lora", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,dh,S,kv_chunk,where", [
+    (2, 8, 2, 128, 200, 0, "q"), (2, 8, 2, 64, 60, 0, "q"), (3, 4, 1, 256, 300, 0, "k"), (2, 8, 2, 128, 384, 96, "q"),
+    (2, 8, 2, 128, 384, 96, "k"), (2, 4, 2, 64, 128, 32, "k"), (2, 8, 2, 128, 256, 128, "v"), (600, 8, 1, 64, 128, 0, "k")])
+def test_decode_attention_keeps_a_nan(gpu, B, Hq, Hkv, dh, S, kv_chunk, where, lora):
+  """A NaN in a head's query, or in one key or value of its kv head, is in the output of those heads and of no other, however the keys are divided
+  among waves and chunks: a share whose sum is NaN is none without a key."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  k, v, q = bf(rnd((B, Hkv, S, dh), 113)), bf(rnd((B, Hkv, S, dh), 114)), bf(rnd((B, Hq, dh), 115))
+  want = torch.zeros(B, Hq, dh, dtype=torch.bool)
+  if where == "q":
+    q[1, 2, 5] = float("nan")
+    want[1, 2] = True
+  elif where == "k":
+    k[1, 0, 40, 3] = float("nan")
+    want[1, :Hq // Hkv] = True
+  else:
+    v[1, 0, 40, 3] = float("nan")
+    want[1, :Hq // Hkv, 3] = True
+  k, v, q = k.to(gpu), v.to(gpu), q.to(gpu)
+  tokens, col = torch.ones(B, S, dtype=torch.int32, device=gpu), torch.full((1,), S - 1, dtype=torch.int32, device=gpu)
+  ws = torch.full((max(ops.attn_ws_bytes(B, 1, S, Hq, dh, kv_chunk) // 4, 1),), float("nan"), device=gpu)
+  out = torch.zeros(B, Hq * dh, dtype=torch.bfloat16, device=gpu)
+  d = L.AttnDesc()
+  d.B, d.T, d.S, d.Hq, d.Hkv, d.dh = B, 1, S, Hq, Hkv, dh
+  d.scale, d.window, d.pad_id = dh ** -0.5, 0, 0
+  d.q, d.kcache, d.vcache = q.data_ptr(), k.data_ptr(), v.data_ptr()
+  d.tokens, d.tok_ld, d.col_ptr = tokens.data_ptr(), S, col.data_ptr()
+  d.kv_chunk, d.ws, d.out = kv_chunk, ws.data_ptr(), out.data_ptr()
+  if lora:
+    a, t = bf(rnd((16, Hq * dh), 116)).to(gpu), torch.zeros(B, 16, dtype=torch.bfloat16, device=gpu)
+    ops.gqa_attn_lora(d, a, t)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isnan(t).any(1).cpu(), want.flatten(1).any(1))
+  else:
+    ops.gqa_attn(d)
+    torch.cuda.synchronize()
+  assert torch.equal(torch.isnan(out).cpu().view(B, Hq, dh), want)
+
+
 @pytest.mark.parametrize("kv_chunk,window,planes,Hq,split", [
     (0, 0, False, 8, 3), (32, 0, True, 8, 3), (0, 40, True, 8, 3), (64, 0, False, 8, 3),
     (0, 0, True, 16, 3),     # eight query heads per kv head: more than one set of plane loads

@@ -673,12 +673,12 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
       float M = kNegBig, L = 0.f;
 #pragma unroll
       for (int w = 0; w < W; ++w)
-        if (ml[w][n][1] > 0.f) M = fmaxf(M, ml[w][n][0]);
+        if (ml[w][n][1] != 0.f) M = fmaxf(M, ml[w][n][0]);
       f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < W; ++w) {
         const float l = ml[w][n][1], f = __expf(ml[w][n][0] - M);
-        if (l > 0.f) {   // (a wave without a key)
+        if (l != 0.f) {   // (a wave without a key has 0; a NaN is no such wave)
           L += f * l;
           const f32x4 v = *reinterpret_cast<const f32x4*>(&stage[w][e]);
 #pragma unroll
@@ -1266,7 +1266,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // The (m, l) pairs of all chunks are fetched at once into LDS (one round trip instead of one
 // dependent load per chunk and pass); every thread then forms M, the weights and the sums in
 // chunk order, with its chunk outputs fetched eight at a time.  (Chunks without a key have
-// l = 0 and an O nobody wrote: selected away, never multiplied.)
+// l = 0 and an O nobody wrote: selected away, never multiplied.  l is a sum of exponentials: 0, positive, or the NaN of a
+// query or a key, which has to reach the output.)
 __global__ void attn_combine_kernel(const float* ws, int64_t n_qvec, int dh, int n_chunks,
                                     uint16_t* out) {
   extern __shared__ float ml[];   // [n_chunks][2]
@@ -1278,7 +1279,7 @@ __global__ void attn_combine_kernel(const float* ws, int64_t n_qvec, int dh, int
   if (d >= dh) return;
   float M = kNegBig;
   for (int c = 0; c < n_chunks; ++c)
-    if (ml[2 * c + 1] > 0.f) M = fmaxf(M, ml[2 * c]);
+    if (ml[2 * c + 1] != 0.f) M = fmaxf(M, ml[2 * c]);
   float L = 0.f, o = 0.f;
   for (int c0 = 0; c0 < n_chunks; c0 += 8) {
     float v[8];
@@ -1289,7 +1290,7 @@ __global__ void attn_combine_kernel(const float* ws, int64_t n_qvec, int dh, int
       const int c = c0 + u;
       if (c < n_chunks) {
         const float l = ml[2 * c + 1];
-        if (l > 0.f) {
+        if (l != 0.f) {
           const float w = __expf(ml[2 * c] - M);
           L += w * l;
           o += w * v[u];
@@ -1297,7 +1298,7 @@ __global__ void attn_combine_kernel(const float* ws, int64_t n_qvec, int dh, int
       }
     }
   }
-  out[qv * dh + d] = f2bf(L > 0.f ? o / L : 0.f);
+  out[qv * dh + d] = f2bf(L != 0.f ? o / L : 0.f);
 }
 
 // The same over whole rows of heads, with the LoRA down-projection of the row behind it (row_adapter.h); the first group of adapter columns
@@ -1342,7 +1343,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const float* m = ml + 2 * at[c];
     float M = kNegBig;
     for (int i = 0; i < n_chunks; ++i)
-      if (m[2 * i + 1] > 0.f) M = fmaxf(M, m[2 * i]);
+      if (m[2 * i + 1] != 0.f) M = fmaxf(M, m[2 * i]);
     float L = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int c0 = 0; c0 < n_chunks; c0 += NCH) {
       if (c0 > 0) fetch(c, c0);
@@ -1351,7 +1352,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
         const int i = c0 + u;
         if (i < n_chunks) {
           const float l = m[2 * i + 1];
-          if (l > 0.f) {   // (a chunk without a key: an O nobody wrote)
+          if (l != 0.f) {   // (a chunk without a key: an O nobody wrote)
             const float w = __expf(m[2 * i] - M);
             L += w * l;
 #pragma unroll
@@ -1366,7 +1367,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const int ch = c * 256 + threadIdx.x;
     if (ch < K / 8) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) x[c][q] = L > 0.f ? pack2bf(o[2 * q] / L, o[2 * q + 1] / L) : 0u;
+      for (int q = 0; q < 4; ++q) x[c][q] = L != 0.f ? pack2bf(o[2 * q] / L, o[2 * q + 1] / L) : 0u;
       if (group == 0) *reinterpret_cast<u32x4*>(out + row * K + (int64_t)ch * 8) = x[c];
     }
   }
