@@ -307,6 +307,26 @@ def test_slopes_alone_and_chunks_alone(gpu, dtype):
       a.check(a.run(t, 1, split=32 if dtype == BF else 0), t)
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("H,G,dk,dv,chunk,key", [(4, 2, 64, 24, 0, 45), (8, 2, 128, 128, 0, 97), (6, 1, 20, 100, 50, 63), (2, 2, 32, 32, 40, 79), (4, 1, 96, 64, 0, 149)])
+def test_a_value_that_is_no_number_reaches_the_positions_that_see_it_in_32_bits(gpu, H, G, dk, dv, chunk, key, value):
+  """An infinity or a NaN in one value of one kv head: in that column of its heads, at the positions from the key's on (in its chunk), and
+  nowhere else; what does not see it is what it is without it (the block's sums in another order: 32-bit sums of 150 terms)."""
+  S, col = 150, 7
+  a = Biased(gpu, F32, H, G, dk, dv, S, [0, 37], chunk, seed=3, sharp=1.0, scale=0.3)
+  for c, T in ((0, S), (90, 13), (S - 1, 1)):
+    a.vc[1, 0, key, col] = 0.25
+    clean = a.run(c, T)
+    a.vc[1, 0, key, col] = value
+    got = a.run(c, T)
+    at = torch.arange(c, c + T) - 37
+    seen = (at >= key - 37) & (at // chunk == (key - 37) // chunk if chunk else torch.ones(T, dtype=torch.bool))
+    hit = torch.zeros(2, T, H, dv, dtype=torch.bool)
+    hit[1, seen, :H // G, col] = True
+    assert bool(torch.isnan(got[hit]).all() if value != value else (got[hit] == value).all())
+    torch.testing.assert_close(got[~hit], clean[~hit], rtol=1e-5, atol=2e-6)
+
+
 @pytest.mark.parametrize("how", ["prompt", "portion", "decoded", "split"])
 @pytest.mark.parametrize("start", [0, 13])
 @pytest.mark.parametrize("chunk,at", [(120, 359), (120, 240), (120, 300), (64, 127), (64, 128), (63, 251), (63, 252), (31, 371), (400, 399), (397, 396), (397, 397), (5, 204), (1, 77)])

@@ -123,11 +123,12 @@ __global__ __launch_bounds__(256) void sink_attn_any_kernel(const SinkArgs a) {
 // leaves a lane with half of the keys of one query, the B operand of O^T = V^T . P^T; O keeps its query in the lane, so that rescaling
 // needs no exchange.  Key rows lie with their 16-byte chunks swizzled by row (sixteen rows' reads of one chunk hit all banks).  Bound by the matrix
 // pipe: 2 x 64 MFMAs of 64 clocks per block and wave at heads of 128.
-// Plain loops before | now: 2 x 1200 positions, 16 heads on 4 10.7 | 0.30 ms, one position of 8 rows over 224 keys 94 | 43 us.
+// Plain loops before | now: 2 x 1200 positions, 16 heads on 4 10.7 | 0.32 ms (0.31 while a value that is no number reached positions that do not see it).
 template <int KD, int VD>   // dk <= KD, dv <= VD, multiples of 32
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void sink_attn_f32_kernel(const SinkArgs a) {
   constexpr int KC = KD / 4, VC = VD / 4, KN = 32 * KC / 256, VN = 32 * VC / 256, NT = VD / 32;
   __shared__ __align__(16) f32x4 ks[2][32 * KC], vs[2][32 * VC];
+  __shared__ int odd;   // whether a value that some query sees is an infinity or a NaN
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = blockIdx.y;
@@ -173,6 +174,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   };
   if (lo_wg <= hi_wg) fetch(lo_wg);
+  if (tid == 0) odd = 0;
+  __syncthreads();
   int buf = 0;
   for (int kb = lo_wg; kb <= hi_wg; kb += 32, buf ^= 1) {
 #pragma unroll
@@ -180,8 +183,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int e = n * 256 + tid, row = e / KC, c = e % KC;
       ks[buf][row * KC + (c ^ (row & (KC < 16 ? KC - 1 : 15)))] = kr[n];
     }
+    // (a product takes every key of the block for every query, and 0 x NaN is a NaN: what is no number stays out, and is added in the end)
+    bool finite = true;
 #pragma unroll
-    for (int n = 0; n < VN; ++n) vs[buf][n * 256 + tid] = vr[n];
+    for (int n = 0; n < VN; ++n) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool ok = fabsf(vr[n][e]) < __builtin_inff();
+        finite = finite && ok;
+        vr[n][e] = ok ? vr[n][e] : 0.f;
+      }
+      vs[buf][n * 256 + tid] = vr[n];
+    }
+    if (!finite) odd = 1;
     __syncthreads();   // (the other buffer is read one step behind, in front of this barrier)
     if (kb + 32 <= hi_wg) fetch(kb + 32);
     if (kb > hi_w || kb + 31 < lo_w) continue;
@@ -225,7 +239,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int i = 0; i < NT; ++i)
         o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[(8 * (r >> 2) + 4 * lh + (r & 3)) * VD + 32 * i], st[r], o[i], 0, 0, 0);
   }
+  __syncthreads();
   if (qrow >= rows) return;
+  if (odd && valid)   // (the weight of a key that a query sees is above zero: the infinity or the NaN itself)
+    for (int key = max(first, 0); key <= last; ++key)
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int d = 32 * i + 8 * (e >> 2) + 4 * lh + (e & 3);
+          const float x = d < a.dv ? v[(int64_t)key * a.dvp + d] : 0.f;
+          if (!(fabsf(x) < __builtin_inff())) o[i][e] += x;
+        }
   float w;
   if (a.sinks) {
     const float s2 = a.sinks[h] * kLog2e, top = fmaxf(m, s2);
