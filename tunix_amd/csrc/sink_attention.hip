@@ -95,7 +95,18 @@ __global__ __launch_bounds__(256) void sink_attn_any_kernel(const SinkArgs a) {
         const int d = c * 256 + tid;
         if (d >= a.dv) break;
         float acc = o[c] * alpha;
-        for (int j = 0; j < n; ++j) acc += p[j] * ld_elem(v, (int64_t)(k0 + j) * a.dvp + d);
+        // (eight values asked for together: left to itself the scheduler waits for each where that saves registers for one more wave)
+        const T* vd = v + (int64_t)k0 * a.dvp + d;
+        int j = 0;
+        for (; j + 8 <= n; j += 8) {
+          float x[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) x[u] = ld_elem(vd, (int64_t)(j + u) * a.dvp);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int u = 0; u < 8; ++u) acc += p[j + u] * x[u];
+        }
+        for (; j < n; ++j) acc += p[j] * ld_elem(vd, (int64_t)j * a.dvp);
         o[c] = acc;
       }
     }
