@@ -307,6 +307,15 @@ def test_slopes_alone_and_chunks_alone(gpu, dtype):
       a.check(a.run(t, 1, split=32 if dtype == BF else 0), t)
 
 
+@pytest.mark.parametrize("H,G,dk,dv,chunk", [(9, 3, 64, 24, 0), (16, 8, 20, 33, 0), (16, 2, 128, 128, 40), (10, 5, 100, 64, 0)])
+def test_steps_of_many_rows_in_32_bits(gpu, H, G, dk, dv, chunk):
+  """One and three positions of so many rows that the tiles take them (of few, the plain loops do)."""
+  starts = [(7 * b) % 60 for b in range(40)]
+  a = Biased(gpu, F32, H, G, dk, dv, 70, starts, chunk, seed=9)
+  for col, T in ((69, 1), (33, 1), (60, 3)):
+    a.check(a.run(col, T), col)
+
+
 @pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
 @pytest.mark.parametrize("H,G,dk,dv,chunk,key", [(4, 2, 64, 24, 0, 45), (8, 2, 128, 128, 0, 97), (6, 1, 20, 100, 50, 63), (2, 2, 32, 32, 40, 79), (4, 1, 96, 64, 0, 149)])
 def test_a_value_that_is_no_number_reaches_the_positions_that_see_it_in_32_bits(gpu, H, G, dk, dv, chunk, key, value):

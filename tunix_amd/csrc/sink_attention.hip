@@ -8,7 +8,7 @@
 //                           staged through LDS, 32x32x16 MFMAs
 //   sink_attn_step_kernel   few query rows (decode): one wave per 16 query rows and key chunk,
 //                           keys and values streamed through registers, 16x16x32 MFMAs
-//   sink_attn_f32_kernel    fp32, heads of up to 128: 32-bit MFMAs
+//   sink_attn_f32_kernel    fp32, heads of up to 128, more than a few queries: 32-bit MFMAs
 //   sink_attn_any_kernel    any sizes: plain loops
 #include <string.h>
 
@@ -284,6 +284,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 bool f32_sizes(const SinkArgs& a) {
   return a.dk <= 128 && a.dv <= 128 && (a.dk | a.dv | a.dkp | a.dvp) % 4 == 0 && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0 &&
          a.G <= 65535 && a.T * a.R < (int64_t)1 << 30;
+}
+// Whether the plain loops are the faster form: a work-group per query there spends its time on that query's keys, whatever the other compute units
+// do, and a wave of the tiles on 32 queries, whether it has them or not.  Counted in work-groups of the plain loops, those of a prompt (T of S
+// slots) by the part of the slots that they see; a single row's share their keys.  us, plain | tiles, heads of 32, 64, 96, 128, 400 slots unless said:
+//   one position (256) 27 | 45, 35 | 46, 45 | 76, 49 | 77; (320) 34 | 45, 46 | 46, 66 | 76, 75 | 76; (511) 41 | 45, 61 | 46, 91 | 75, 110 | 76;
+//   four positions (318) 31 | 45, 44 | 46, 64 | 76, 71 | 76; (509) 38 | 45, 56 | 46, 87 | 76, 103 | 76;
+//   a row of 37 positions behind 963 (581) 55 | 107, 93 | 108, 138 | 181, 177 | 184; of 64 (512) 7.6 | 11.4, 10.2 | 13.2, 14.0 | 20.8, 17.4 | 22.1;
+//   of 100 (800) 10.8 | 17.0, 16.5 | 17.5, 22.5 | 27.8, 27.6 | 28.2; of 60 behind 440 (902) 37 | 56, 63 | 57, 91 | 95, 118 | 96;
+//   2 rows of 64 (512) 7.6 | 10.7, 10.3 | 11.5, 14.3 | 17.5, 17.7 | 18.0; 2 of 37 behind 463 (570) 43 | 55, 74 | 56, 118 | 91, 138 | 92, (1140)
+//   62 | 56, 115 | 58, 180 | 96, 223 | 98.
+bool f32_plain(const SinkArgs& a) {
+  const double groups = (double)a.B * a.T * a.H * (1.0 - 0.5 * (double)a.T / (double)a.S);
+  if (a.dk <= 32) return groups <= (a.T < 16 ? 600 : 1100);
+  return groups <= (a.T < 16 ? 320 : a.B == 1 ? 800 : 520);
 }
 void launch_f32(hipStream_t st, const SinkArgs& a) {
   const dim3 grid((unsigned)cdiv(a.T * a.R, 128), (unsigned)a.G, (unsigned)a.B);
@@ -835,7 +849,7 @@ extern "C" int tnx_sink_attn(void* stream, const tnx_sink_attn_desc* d) {
   if (!mfma) {
     // one work-group per (query position, head)
     TNX_REQUIRE(d->B * d->T <= 65535, "sink_attn: at most 65535 query rows per call at these sizes");
-    if (d->dtype == TNX_F32 && f32_sizes(a)) {
+    if (d->dtype == TNX_F32 && f32_sizes(a) && !f32_plain(a)) {
       launch_f32(st, a);
       TNX_CHECK_LAUNCH("sink_attn_f32");
       return TNX_OK;
