@@ -434,6 +434,22 @@ class Gated:
         assert rel(self.state[b], S) < (1e-5 if self.dtype == F32 else 1e-3), (b, col, T, rel(self.state[b], S))
 
 
+@pytest.mark.parametrize("H,dk,dv", [(2, 20, 33), (1, 96, 70), (2, 128, 16), (1, 129, 9), (1, 250, 40)])
+def test_an_infinite_value_stays_one_in_32_bits(gpu, H, dk, dv):
+  """Queries and weights above zero: from the token that brings an infinity on its column is infinite, not a NaN of the rows that fill a head's
+  size up, and every other column is bit for bit what it is without."""
+  outs = []
+  for value in (0.5, float("inf")):
+    a = Gated(gpu, F32, H, dk, dv, 30, [0, 11], seed=2, lower=0.25)
+    a.q = a.q.abs() + 0.5
+    a.v[1, 17, 0, 3] = value
+    outs.append(a.run(0, 30))
+  hit = torch.zeros(2, 30, H, dv, dtype=torch.bool)
+  hit[1, 17:, 0, 3] = True
+  assert bool((outs[1][hit] == float("inf")).all())
+  assert torch.equal(outs[1][~hit], outs[0][~hit])
+
+
 GATED = [(3, 32, 48), (2, 64, 40), (2, 128, 128), (5, 16, 16), (2, 11, 9), (1, 20, 30), (2, 200, 136), (1, 256, 264), (9, 8, 8), (4, 96, 24), (1, 40, 1032)]
 
 

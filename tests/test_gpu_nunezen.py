@@ -428,6 +428,22 @@ def test_lightning_prompt_portions_and_steps(gpu, dtype, H, dk, dv):
     b.check(b.run(t, 1), t)
 
 
+@pytest.mark.parametrize("H,dk,dv", [(2, 20, 33), (1, 96, 70), (2, 128, 16), (1, 129, 9), (1, 250, 40)])
+def test_an_infinite_value_stays_one_in_32_bits(gpu, H, dk, dv):
+  """Queries and keys above zero: from the token that brings an infinity on its column is infinite, not a NaN of the rows that fill a head's
+  size up, and every other column is bit for bit what it is without."""
+  outs = []
+  for value in (0.5, float("inf")):
+    a = Light(gpu, F32, H, dk, dv, 30, [0, 11], [0.9] * H, seed=2)
+    a.q, a.k = a.q.abs() + 0.5, a.k.abs() + 0.5
+    a.v[1, 17, 0, 3] = value
+    outs.append(a.run(0, 30))
+  hit = torch.zeros(2, 30, H, dv, dtype=torch.bool)
+  hit[1, 17:, 0, 3] = True
+  assert bool((outs[1][hit] == float("inf")).all())
+  assert torch.equal(outs[1][~hit], outs[0][~hit])
+
+
 def test_lightning_remembers_and_forgets(gpu):
   """One key-value pair far back: with decay 1 it returns whole after hundreds of tokens, with decay 0 it
   is gone with the next token; the last token of a chunk and the first of the next are the same to it."""

@@ -19,6 +19,7 @@ __device__ __forceinline__ void state_scan(int64_t t0, int64_t T, int dk, int dv
   constexpr int DK = 4 * R, TB = R > 32 ? 4 : 8, N = TB * DK / 256, NV = TB * kScanCols / 256;
   __shared__ __align__(16) float qs[2][TB][DK], ks[2][TB][DK], fs[FORGET ? 2 : 1][FORGET ? TB : 1][FORGET ? DK : 1];
   __shared__ float vs[2][TB][kScanCols], part[2][TB][4][kScanCols];
+  __shared__ int odd[kScanCols];   // whether a column's v holds an infinity or a NaN
   const int tid = threadIdx.x, lane = tid & 63;
   const int r0 = __builtin_amdgcn_readfirstlane(tid >> 6) * R, wave = r0 / R;
   const int d = d0 + lane;
@@ -52,11 +53,16 @@ __device__ __forceinline__ void state_scan(int64_t t0, int64_t T, int dk, int dv
     }
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
+      // (an infinity would make NaNs of the rows past the last, whose k is zero: it stays out, and its column is formed again in the end)
       const int e = n * 256 + tid;
-      vs[b][e / kScanCols][e % kScanCols] = rv[n];
+      const bool finite = fabsf(rv[n]) < __builtin_inff();
+      vs[b][e / kScanCols][e % kScanCols] = finite ? rv[n] : 0.f;
+      if (!finite) odd[e % kScanCols] = 1;
     }
   };
+  if (tid < kScanCols) odd[tid] = 0;
   fetch(t0);
+  __syncthreads();
   put(0);
   __syncthreads();
   int b = 0;
@@ -89,7 +95,24 @@ __device__ __forceinline__ void state_scan(int64_t t0, int64_t T, int dk, int dv
   }
 #pragma unroll
   for (int r = 0; r < R; ++r)
-    if (mine && r0 + r < dk) S[(int64_t)(r0 + r) * dv + d] = s[r];
+    if (mine && !odd[lane] && r0 + r < dk) S[(int64_t)(r0 + r) * dv + d] = s[r];
+  __syncthreads();   // (every output is written)
+  if (tid < kScanCols && mine && odd[lane]) {   // token by token, from the state as it was; the first wave's lane is the column
+    bool seen = false;
+    for (int64_t t = t0; t < T; ++t) {
+      const float v = load_v(t, d);
+      seen = seen || !(fabsf(v) < __builtin_inff());
+      float acc = 0.f;
+      for (int i = 0; i < dk; ++i) {
+        float q, k, f = decay;
+        make(load(t, i), q, k, f);
+        float& at = S[(int64_t)i * dv + d];
+        at = __builtin_fmaf(k, v, fresh && t == t0 ? 0.f : f * at);
+        acc = __builtin_fmaf(q, at, acc);
+      }
+      if (seen) out(t, d, acc);
+    }
+  }
 }
 
 }  // namespace
