@@ -2464,6 +2464,10 @@ def test_decode_attention_of_several_waves_per_chunk(gpu, S, Hq, Hkv, dh, chunk,
     (70, 4112, 1000, 1, 4112, 1000, False),  # k turns that the waves do not share evenly
     (1300, 48, 1664, 1, 48, 1664, False),    # tiles of 128: half a step of k at the end
     (1537, 2064, 1025, 1, 2064, 1028, True),
+    (400, 144, 1000, 1, 148, 1003, False),   # tiles of 64
+    (129, 16, 4100, 1, 16, 4100, True),
+    (1601, 80, 2050, 1, 80, 2053, True),     # tiles of 128 where those of 64 take four rounds
+    (65, 48, 72, 130, 48, 72, False),
     (40, 64, 96, 9, 64, 96, False),          # a batch, few tiles and many
     (300, 256, 640, 9, 256, 640, False),
 ])
@@ -2488,7 +2492,11 @@ def test_dense_linear_in_32_bits(gpu, M, K, N, batch, ldx, ldy, relu2):
   assert ((got[..., :N] - want).abs() <= bound).all() and got[..., N:].isnan().all()
 
 
-@pytest.mark.parametrize("K,N,counts,x_div", [(48, 75, (0, 3, 17, 0, 1), 1), (256, 512, (130, 0, 1, 301), 1), (2048, 256, (9, 40, 31, 0), 2)])
+@pytest.mark.parametrize("K,N,counts,x_div", [
+    (48, 75, (0, 3, 17, 0, 1), 1), (256, 512, (130, 0, 1, 301), 1), (2048, 256, (9, 40, 31, 0), 2),
+    (48, 1000, (80, 64, 65, 0, 3) * 8, 2),                  # tiles of 64
+    (80, 2040, (100, 96, 128, 129, 7, 99, 140, 101) * 2, 1),  # tiles of 128
+])
 def test_dense_experts_in_32_bits(gpu, K, N, counts, x_div):
   from tunix_amd import _lib as L
   from tunix_amd import ops

@@ -8,6 +8,8 @@
 // one per head) and experts (a row goes to the weights its routes name, rows sorted by expert).
 #include <string.h>
 
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -344,47 +346,49 @@ __global__ __launch_bounds__(64 * KS) void dense_f32_rows_kernel(const DenseArgs
   if (n0 + 4 * lq < a.N) f32_store<MODE>(a, t, t.m0 + wave * 16 + lm, n0 + 4 * lq, v);
 }
 
-// Many rows: 128 x 128 per work-group of four waves, a wave 64 x 64; steps of 32 k through two LDS buffers (rows of 128 bytes, whose 16-byte
+// Many rows: 64 TW x 64 TW (TW = 1, 2) per work-group of four waves, a wave a quarter of it; steps of 32 k through two LDS buffers (rows of 128 bytes, whose 16-byte
 // chunks are swizzled by the row so that sixteen rows' reads of one chunk hit all banks), the next one's operands in registers meanwhile.
-// Bound by the matrix pipe: 122 TFLOP/s at 2400 x 2048 -> 16384.
-template <int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_f32_tile_kernel(const DenseArgs a) {
-  __shared__ __align__(16) f32x4 tile[2][2][128 * 8];   // buffer, [weights | x], [row][chunk]
+// Bound by the matrix pipe: TW = 2 at 2400 x 2048 -> 16384 115 TFLOP/s, TW = 1 at 2400 x 2048 -> 2048, which leaves TW = 2 two rounds for a little more than
+// one, 97 (TW = 2: 77).
+template <int MODE, int TW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TW > 1 ? 2 : 4, TW > 1 ? 2 : 4))) void dense_f32_tile_kernel(const DenseArgs a) {
+  constexpr int SIDE = 64 * TW, C = SIDE / 32;
+  __shared__ __align__(16) f32x4 tile[2][2][SIDE * 8];   // buffer, [weights | x], [row][chunk]
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
   F32Tile t;
-  if (!f32_tile<MODE>(a, 128, t)) return;
-  const int64_t n0 = (int64_t)blockIdx.x * 128;
+  if (!f32_tile<MODE>(a, SIDE, t)) return;
+  const int64_t n0 = (int64_t)blockIdx.x * SIDE;
   // thread: chunk tid % 8 of rows tid / 8 + 32 c
   const int ch = tid & 7, r0 = tid >> 3;
-  const float *wp[4], *xp[4];
+  const float *wp[C], *xp[C];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < C; ++c) {
     wp[c] = t.w + min(n0 + r0 + 32 * c, a.N - 1) * a.K + 4 * ch;
     xp[c] = f32_x_row<MODE>(a, t, t.m0 + r0 + 32 * c) + 4 * ch;
   }
-  f32x4 wv[4], xv[4];
+  f32x4 wv[C], xv[C];
   auto fetch = [&](int64_t k0) {
     const bool in = k0 + 4 * ch < a.K;   // (K is a multiple of 16: of the last step perhaps half)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < C; ++c) {
       wv[c] = in ? *reinterpret_cast<const f32x4*>(wp[c] + k0) : f32x4{0.f, 0.f, 0.f, 0.f};
       xv[c] = in ? *reinterpret_cast<const f32x4*>(xp[c] + k0) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
   };
   auto at = [](int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); };
-  f32x16v acc[2][2];
+  f32x16v acc[TW][TW];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TW; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TW; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   fetch(0);
   int buf = 0;
   for (int64_t k0 = 0; k0 < a.K; k0 += 32) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < C; ++c) {
       tile[buf][0][at(r0 + 32 * c, ch)] = wv[c];
       tile[buf][1][at(r0 + 32 * c, ch)] = xv[c];
     }
@@ -392,51 +396,79 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (k0 + 32 < a.K) fetch(k0 + 32);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      f32x4 wf[2], xf[2];
+      f32x4 wf[TW], xf[TW];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        wf[i] = tile[buf][0][at(wn * 64 + i * 32 + l32, 2 * u + lh)];
-        xf[i] = tile[buf][1][at(wm * 64 + i * 32 + l32, 2 * u + lh)];
+      for (int i = 0; i < TW; ++i) {
+        wf[i] = tile[buf][0][at((wn * TW + i) * 32 + l32, 2 * u + lh)];
+        xf[i] = tile[buf][1][at((wm * TW + i) * 32 + l32, 2 * u + lh)];
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < TW; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j][e], xf[i][e], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < TW; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j][e], xf[i][e], acc[i][j], 0, 0, 0);
     }
     buf ^= 1;
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TW; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TW; ++j)
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        const int64_t col = n0 + wn * 64 + j * 32 + 8 * b + 4 * lh;
+        const int64_t col = n0 + (wn * TW + j) * 32 + 8 * b + 4 * lh;
         if (col < a.N)
-          f32_store<MODE>(a, t, t.m0 + wm * 64 + i * 32 + l32, col, f32x4{acc[i][j][4 * b], acc[i][j][4 * b + 1], acc[i][j][4 * b + 2], acc[i][j][4 * b + 3]});
+          f32_store<MODE>(a, t, t.m0 + (wm * TW + i) * 32 + l32, col, f32x4{acc[i][j][4 * b], acc[i][j][4 * b + 1], acc[i][j][4 * b + 2], acc[i][j][4 * b + 3]});
       }
 }
 
-// Which form: a round of 128 x 128 tiles over the device takes as long as some 2700 blocks of 32 x 16 (experts: a tile is as good as full from
-// 33 rows on).  us, few rows | tiles | the 64 x 64 tiles of the vector unit that were here before, K = 2048:
-//   N = 2048   8 rows 8.8 | 146 | 122   64: 15 | 147 | 122   400: 88 | 148 | 122   800: 163 | 149 | 129   2400: 472 | 263 | 282
-//   N = 16384  8 rows 36 | 149 | 138    64: 110 | 150 | 141  128: 210 | 151 | 154  400: 644 | 267 | 399   2400: 3725 | 1318 | 2043
-// K = 8192, N = 2048: 8 rows 31 | 578 | 528, 400 rows 302 | 583 | 527.  Error against 64 bits, K = 2048: 2.9e-7 | 8.1e-7 | 8.1e-7.
+// Blocks of h rows that a call brings, over its weights.  Experts: for routes that fall on them by chance (the sizes are on the device), of the
+// experts with a route the whole blocks that a Poisson number of routes fills.
+template <int MODE>
+double f32_row_blocks(const DenseArgs& a, int h) {
+  if (MODE != kExperts) return (double)cdiv(a.M, h);
+  const double r = (double)a.M / a.n_experts;
+  if (r > 16.0 * h) return a.n_experts * (r / h + 0.5);
+  double blocks = -std::expm1(-r);
+  for (int k = 1; k * h < r + 4.0 * std::sqrt(r) + 1.0; ++k) blocks += 0.5 * std::erfc((k * h + 0.5 - r) / std::sqrt(2.0 * r));
+  return a.n_experts * blocks;
+}
+// Which form.  In units of what a 64 x 64 tile per compute unit costs where there are many (40 us at K = 2048): the first round of them 1.4, a round of
+// 128 x 128 tiles 3.2 to 3.6, a round of blocks of 32 x 16 or 16 x 16 a third and less than a fifth, more where K is short, as every block adds up its waves' parts.
+// us, few rows | 64 x 64 | 128 x 128 | the 64 x 64 tiles of the vector unit that were here first, K = 2048:
+//   N = 2048   8 rows 8.9 | 56 | 145 | 121   200: 49 | 59 | 146 | 123   400: 86 | 59 | 146 | 122   800: 161 | 86 | 147 | 130   1600: 304 | 159 | 150 | 223
+//              2400: 466 | 208 | 263 | 288   4800: 935 | 410 | 422 | 543
+//   N = 16384  8 rows 36 | 59 | 146 | 137    64: 109 | 60 | 148 | 141   130: 233 | 122 | 152 | 190   400: 644 | 286 | 281 | 393   2400: 3756 | 1603 | 1400 | 2112
+// K = 512, N = 2048, 400 rows 33 | 17 | 40 | 34; K = 8192, 400 rows 305 | 229 | 573 | 503, 800 569 | 334 | 572 | 540.
+// 64 experts, 768 -> 2048, routes per expert: 1 71 | 88 | 173 | 102   12 161 | 122 | 202 | 151   64 549 | 188 | 228 | 246   100 863 | 267 | 240 | 336;
+// 2048 -> 1536: 4 176 | 244 | 526 | 311   32 433 | 253 | 537 | 340.  128 weights of 128 -> 512, 20 rows 61 | 14 | 21 | 19.
+// Error against 64 bits, K = 2048: 2.9e-7 | 8.1e-7 | 8.1e-7 | 8.1e-7.
 template <int MODE>
 void launch_f32(hipStream_t st, const DenseArgs& a, int64_t batch) {
   auto blocks = [&](int64_t rows) { return MODE == kExperts ? a.M / rows + std::min<int64_t>(a.n_experts, a.M) : cdiv(a.M, rows); };
   const int64_t rows = MODE == kExperts ? cdiv(a.M, (int64_t)a.n_experts) : a.M;   // of a weight
-  const int64_t rounds = cdiv(cdiv(a.M, 128) * cdiv(a.N, 128) * batch, 256);
-  const bool few = (MODE == kExperts ? rows <= 32 : cdiv(a.M, 32) * cdiv(a.N, 16) * batch < 2700 * rounds) && blocks(rows <= 16 ? 16 : 32) <= 65535;
+  const int few_rows = rows <= 16 ? 16 : 32;
+  auto rounds = [&](int h, int w) { return std::max(1.0, std::ceil(f32_row_blocks<MODE>(a, h) * (double)(cdiv(a.N, w) * batch) / 256 - 0.1)); };
+  const double few = rounds(few_rows, 16), K = (double)a.K;
+  double few_cost = 0, t64_cost = 0, t128_cost = 1;   // (one round of few rows: nothing is faster)
+  if (few > 1) {
+    few_cost = few * (few_rows == 16 ? 0.16 + 50 / K : 0.27 + 100 / K);
+    t64_cost = std::max(1.43, rounds(64, 64));
+    t128_cost = 3.2 * rounds(128, 128);
+  }
   constexpr int KS = 8;   // (sixteen waves: 8.2 us for 7.1 at a row of 2048 -> 2048, the same at 8192 -> 2048)
   auto launch = [&](auto kernel, int64_t tile_rows, int64_t tile_cols, int threads) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)cdiv(a.N, tile_cols), (unsigned)blocks(tile_rows), (unsigned)batch), dim3((unsigned)threads), 0, st, a);
   };
-  if (!few) launch(dense_f32_tile_kernel<MODE>, 128, 128, 256);
-  else if (rows <= 16) launch(dense_f32_rows_kernel<MODE, 1, KS>, 16, 16, 64 * KS);
-  else launch(dense_f32_rows_kernel<MODE, 2, KS>, 32, 16, 64 * KS);
+  if ((few > 1 && few_cost > std::min(t64_cost, t128_cost)) || blocks(few_rows) > 65535) {
+    if (t64_cost < t128_cost) launch(dense_f32_tile_kernel<MODE, 1>, 64, 64, 256);
+    else launch(dense_f32_tile_kernel<MODE, 2>, 128, 128, 256);
+  } else if (few_rows == 16) {
+    launch(dense_f32_rows_kernel<MODE, 1, KS>, 16, 16, 64 * KS);
+  } else {
+    launch(dense_f32_rows_kernel<MODE, 2, KS>, 32, 16, 64 * KS);
+  }
 }
 
 template <int MODE>
