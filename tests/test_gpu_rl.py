@@ -343,7 +343,7 @@ def test_aggregate_loss_training_scale(gpu, mode):
 
 
 @pytest.mark.parametrize("mode", AGG_MODES)
-@pytest.mark.parametrize("B,T", [(1, 1), (3, 63), (17, 65), (1024, 16), (1025, 3), (4, 4096), (5, 4096)])   # one launch up to 1024 rows and 16384 tokens
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 63), (17, 65), (128, 128), (129, 3), (1024, 16), (1025, 3), (4, 4096), (5, 4096)])   # one launch up to 128 rows and 16384 tokens
 def test_aggregate_loss_small(gpu, mode, B, T):
   """One and two launches against the float64 oracle (32-bit sums of at most 20480 terms of order one: 1e-5), and compute()'s one launch against
   the tensor operations it stands for, bit for bit."""
@@ -357,6 +357,22 @@ def test_aggregate_loss_small(gpu, mode, B, T):
   np.testing.assert_allclose(m.unreduced_sum.item(), num, rtol=1e-5, atol=1e-4)
   np.testing.assert_allclose(m.denominator.item(), den, rtol=1e-7)
   assert torch.equal(m.compute(), m.unreduced_sum * m.compute_scale())
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (2, 64), (3, 65), (16, 129), (8, 500), (5, 1023), (1, 16384), (33, 256), (70, 200), (128, 128)])
+def test_aggregate_loss_in_one_launch_gives_the_bits_of_two(gpu, B, T):
+  """A row's sums do not depend on the call's size: the rows of a small call against the same rows in one of many."""
+  from tunix_amd import ops
+  rng = np.random.default_rng(B + T)
+  loss = torch.from_numpy(rng.normal(0.3, 1.0, size=(B, T)).astype(np.float32)).to(gpu)
+  mask = torch.from_numpy((rng.random((B, T)) < 0.8).astype(np.float32)).to(gpu)
+  sums = []
+  for n in (1, -(-200 // B)):     # (200 rows and more: two launches)
+    x, m = loss.repeat(n, 1), mask.repeat(n, 1)
+    rows, out = torch.empty(2 * B * n, device=gpu), torch.empty(2, device=gpu)
+    ops.aggregate_loss(x, m, ops.AGG_MODES["token-mean"], 1.0, rows, out)
+    sums.append(rows[:2 * B].cpu())
+  assert torch.equal(*sums)
 
 
 @pytest.mark.parametrize("total,denom", [(3.0, 0.0), (-2.0, 1e-7), (5.0, 3.0), (1.0, float("nan")), (float("inf"), 7.0), (2.0, -4.0)])

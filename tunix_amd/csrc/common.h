@@ -221,6 +221,24 @@ __device__ __forceinline__ float wave_sum(float v) {
 __device__ __forceinline__ float wave_max(float v) {
   return wave_all(v, [](float x, float y) { return fmaxf(x, y); });
 }
+// sum of eight values over the wave's 64 lanes, each in the order of wave_sum: lane l ends with the sum of value l / 8 of the eight
+__device__ __forceinline__ float wave_sum8(float (&v)[8], int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {   // the lower half takes values 0-3, the upper 4-7
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 4]), false, false);
+    v[i] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 2]), false, false);
+    v[i] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  }
+  const bool up = lane & 8;
+  float s = (up ? v[1] : v[0]) + lane_xor(up ? v[0] : v[1], 8);
+  s += lane_xor(s, 4);
+  s += lane_xor(s, 2);
+  return s + lane_xor(s, 1);
+}
 
 // The k largest of a wave's values v[i], of index lane + 64 i, descending, the lowest index first among equals: pick(j, index, value) for each, the
 // same in every lane.  Values lie above -inf, which marks a place without one and a value taken.

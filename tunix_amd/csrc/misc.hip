@@ -150,28 +150,57 @@ __global__ __launch_bounds__(256) void agg_finish_kernel(const float* row_ws, in
   agg_rows_to_mode(row_ws, B, mode, norm, red, out);
 }
 
-// Both passes in one launch for a loss of a few thousand tokens, a wave per row at a time: what such a call costs is its launches.
-constexpr int kAggWaves = 16, kAggOneLaunchRows = 1024;
-constexpr int64_t kAggOneLaunch = 16384;   // tokens; one work-group reads them in some 4 us, a second launch costs the caller about 5
+// Both passes in one launch for a loss of a few thousand tokens, a wave per row, or two side by side, which adds the row's numbers as the four waves
+// of agg_rows_kernel do: the same bits.  Sixteen waves take the rows in turn, so there is a limit to them.  us, two launches | one: 8 x 512, 4 x 4096 6.7 |
+// 4.3, 1 x 16384 9.9 | 6.9, 64 x 256 6.8 | 4.9, 128 x 128 6.7 | 6.2, 160 x 100 6.7 | 7.3.
+constexpr int kAggWaves = 16, kAggOneLaunchRows = 128;
+constexpr int64_t kAggOneLaunch = 16384;   // tokens
 __global__ __launch_bounds__(64 * kAggWaves) void agg_small_kernel(const float* loss, const float* mask, int64_t B, int64_t T, int mode, float norm,
                                                                    float* row_ws, float* out) {
   __shared__ float red[kAggWaves], rows[2 * kAggOneLaunchRows];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int64_t b = wave; b < B; b += kAggWaves) {
-    float s = 0.f, c = 0.f;
-#pragma unroll 4
-    for (int64_t t = lane; t < T; t += 64) {
-      const float m = mask[b * T + t];
-      s += loss[b * T + t] * m;
-      c += m;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = (int)T;
+  // G rows b, b + kAggWaves, ...: their turns of 256 tokens first, then what is left, of which every wave of agg_rows_kernel has up to 64
+  auto add = [&](int64_t b, auto group) {
+    constexpr int G = decltype(group)::value;
+    float s[G][4] = {}, c[G][4] = {};
+    int t0 = 0;
+    if constexpr (G == 1) {
+      const float *lr = loss + b * T + lane, *mr = mask + b * T + lane;
+#pragma unroll 2
+      for (; t0 + 256 <= n; t0 += 256)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float m = mr[t0 + 64 * w];
+          s[0][w] += lr[t0 + 64 * w] * m;
+          c[0][w] += m;
+        }
     }
-    s = wave_sum(s);
-    c = wave_sum(c);
-    if (lane == 0) {
-      rows[2 * b] = row_ws[2 * b] = s;
-      rows[2 * b + 1] = row_ws[2 * b + 1] = c;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int64_t at = min(b + g * kAggWaves, B - 1) * T;
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        if (t0 + 64 * w < n) {   // (uniform)
+          const int t = t0 + 64 * w + lane;
+          const float m = t < n ? mask[at + t] : 0.f;
+          s[g][w] += loss[at + min(t, n - 1)] * m;
+          c[g][w] += m;
+        }
     }
-  }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float v[8] = {s[g][0], s[g][1], s[g][2], s[g][3], c[g][0], c[g][1], c[g][2], c[g][3]};
+      float x = wave_sum8(v, lane);   // lanes 0, 8, 16, 24: the loss, lanes 32 ...: the mask
+      x += lane_xor(x, 8);
+      x += lane_xor(x, 16);
+      const int64_t row = b + g * kAggWaves;
+      if ((lane & 31) == 0 && row < B) rows[2 * row + (lane >> 5)] = row_ws[2 * row + (lane >> 5)] = x;
+    }
+  };
+  if (n <= 256 && B > kAggWaves)
+    for (int64_t b = wave; b < B; b += 2 * kAggWaves) add(b, std::integral_constant<int, 2>{});
+  else
+    for (int64_t b = wave; b < B; b += kAggWaves) add(b, std::integral_constant<int, 1>{});
   __syncthreads();
   agg_rows_to_mode(rows, B, mode, norm, red, out);
 }
