@@ -104,6 +104,22 @@ def test_embed_gathers_rows_and_scales_in_bf16(gpu, B, T, D, V, scale):
   assert torch.equal(out.float().cpu(), want)
 
 
+@pytest.mark.parametrize("E,k", [(1, 1), (63, 5), (64, 8), (65, 3), (128, 64), (200, 8), (257, 8), (300, 16), (512, 4), (513, 9), (1024, 64)])
+def test_moe_route_picks_the_largest_lowest_first(gpu, E, k):
+  """Every number of experts per lane: ids in the order of the scores, the lower one first among equals, weights that add up."""
+  from tunix_amd import ops
+  M = 37
+  scores = bf(rnd((M, E), 121))
+  scores[3] = 0.25
+  scores[5, E // 2:] = 1.5
+  tw, ti = torch.empty(M, k, dtype=torch.bfloat16, device=gpu), torch.empty(M, k, dtype=torch.int32, device=gpu)
+  ops.moe_route_topk(scores.to(gpu), k, tw, ti)
+  val, idx = torch.sort(scores.float(), dim=-1, descending=True, stable=True)
+  assert torch.equal(ti.cpu().long(), idx[:, :k])
+  want = torch.softmax(val[:, :k], -1)
+  assert ((tw.float().cpu() - want).abs() <= 2.0 ** -8 * want + 1e-6).all()   # (rounded to bf16)
+
+
 def test_moe_route_keeps_ids_in_range_for_nan_scores(gpu):
   """A row of router scores with a NaN (a hidden state gone bad): the k ids stay distinct and
   inside [0, E) -- the route sort and the grouped GEMM index memory with them -- and the row's

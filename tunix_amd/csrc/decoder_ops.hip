@@ -1220,9 +1220,7 @@ int launch_act_mul(hipStream_t st, int dtype, const void* y, int64_t ld, int64_t
 // ---- choice of experts: the k largest logits (first among equals), softmax over them ---------------
 // One wave per token.  NaN logits rank below every number, so that k distinct experts are found whatever
 // the logits hold; they leave as NaN weights.
-// Up to 256 experts: they stay in registers, a choice is a maximum over the wave and ballots; more: one pass over the logits
-// per choice.
-constexpr int kRegisterExperts = 256;
+// (more than kChooseValues experts: one pass over the logits per choice)
 __global__ __launch_bounds__(64) void route_softmax_kernel(const RowSrc<float> src, int E, int k, float* topk_w, int32_t* topk_id) {
   extern __shared__ __align__(16) float z[];   // logits [E], chosen logits [k]
   float* sel = z + E;
@@ -1237,19 +1235,14 @@ __global__ __launch_bounds__(64) void route_softmax_kernel(const RowSrc<float> s
   }
   bad = __any(bad);
   __syncthreads();
-  if (E <= kRegisterExperts) {   // (uniform)
-    float c[kRegisterExperts / 64];
-#pragma unroll
-    for (int i = 0; i < kRegisterExperts / 64; ++i) c[i] = lane + 64 * i < E ? z[lane + 64 * i] : ninf;
-    wave_largest(c, k, [&](int j, int id, float best) {
-      if (lane == 0) {
-        sel[j] = best;
-        topk_id[m * k + j] = id;
-      }
+  if (E <= kChooseValues) {   // (uniform)
+    wave_choose(z, E, k, [&](int j, int id) {
+      sel[j] = z[id];
+      topk_id[m * k + j] = id;
     });
     __syncthreads();
   }
-  for (int j = 0; j < k && E > kRegisterExperts; ++j) {
+  for (int j = 0; j < k && E > kChooseValues; ++j) {
     float best = ninf;
     int bi = 0x7fffffff;
     for (int e = lane; e < E; e += 64)

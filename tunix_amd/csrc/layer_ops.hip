@@ -460,7 +460,6 @@ int launch_poly(hipStream_t st, int64_t M, const RowSrc<T>& src, int64_t F, cons
 // ---- choice of experts by corrected scores ------------------------------------------------------------
 // One wave per token: softmax over all logits, the k largest scores + correction (first among equals).  Whatever the
 // logits hold, k distinct experts are found; a row with a NaN leaves NaN weights.
-constexpr int kRegisterExperts = 256;   // up to here the choices stay in registers (64 experts, top 8, 8192 tokens: 13.0 us with every expert counting the ones ahead of it, 11.4 so)
 __global__ __launch_bounds__(64) void route_scores_kernel(const RowSrc<float> src, int E, int k, const float* correction, float scale, int64_t gate_off,
                                                           int ld, float* topk_w, int32_t* topk_id, float* gate_w) {
   extern __shared__ __align__(16) float lds[];   // choice scores [E rounded up to 4], scores [E], chosen scores [k]
@@ -502,19 +501,14 @@ __global__ __launch_bounds__(64) void route_scores_kernel(const RowSrc<float> sr
     choice[e] = c;
   }
   __syncthreads();
-  if (E <= kRegisterExperts) {   // (uniform)
-    float c[kRegisterExperts / 64];
-#pragma unroll
-    for (int i = 0; i < kRegisterExperts / 64; ++i) c[i] = lane + 64 * i < E ? choice[lane + 64 * i] : ninf;
-    wave_largest(c, k, [&](int j, int id, float) {
-      if (lane == 0) {
-        sel[j] = score[id];
-        topk_id[m * ld + j] = id;
-      }
+  if (E <= kChooseValues) {   // (uniform)
+    wave_choose(choice, E, k, [&](int j, int id) {
+      sel[j] = score[id];
+      topk_id[m * ld + j] = id;
     });
     __syncthreads();
   }
-  for (int j = 0; j < k && E > kRegisterExperts; ++j) {
+  for (int j = 0; j < k && E > kChooseValues; ++j) {
     float best = ninf;
     int bi = 0x7fffffff;
     for (int e = lane; e < E; e += 64)

@@ -745,6 +745,7 @@ extern "C" int tnx_moe_route_topk(void* stream, const uint16_t* scores, int64_t 
   if (E <= 64) launch(moe_route_kernel<1>);
   else if (E <= 128) launch(moe_route_kernel<2>);
   else if (E <= 256) launch(moe_route_kernel<4>);
+  else if (E <= 512) launch(moe_route_kernel<8>);
   else launch(moe_route_kernel<16>);
   TNX_CHECK_LAUNCH("moe_route");
   return TNX_OK;
