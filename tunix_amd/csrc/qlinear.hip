@@ -1158,9 +1158,10 @@ int tnx_internal_wide_head(hipStream_t st, const tnx_lmhead_desc* d, float tempe
   // the weight stream, and this kernel re-reads the activations once per 256 columns where the
   // 128 x 128 head kernel re-reads them once per 128, as many bytes again as the weights.
   // Short vocabularies leave part of the device without a tile, and the other kernel, whose tiles are half as wide, has its rows to re-read: us,
-  // that one | this, 32768 x 2048 16 rows 44.5 | 41.2, 32 rows 46.2 | 38.6, 128 rows 68 | 44; 50304 x 1024 32 rows 38.7 | 29.8; 16384 x 2048 16 rows
-  // 34.3 | 38.5, 32 rows 36.8 | 35.7, 64 rows 42.5 | 37.0; 32000 x 512 16 rows 17.8 | 21.7, 32 rows 20.3 | 18.5.
-  if (!(dense ? wide_shape(a, 1, a.M > 16 ? 1 : 128) : wide_shape(a))) return 1;
+  // that one | this, weights from memory, 32768 x 2048 16 rows 43.8 | 40.6, 32 rows 46.7 | 37.9; x 1024 16 rows 25.0 | 28.6, 32 rows 28.1 | 25.6;
+  // x 512 16 rows 18.4 | 22.1, 32 rows 21.7 | 19.5; 36864 x 1024 16 rows 33.9 | 29.2, x 512 23.9 | 22.4; 16384 x 2048 17 rows 35.3 | 35.3, 48 rows 43.5 |
+  // 36.2, x 512 17 rows 19.7 | 18.4.
+  if (!(dense ? wide_shape(a, 1, a.M > 16 ? 1 : a.K < 2048 ? 144 : 128) : wide_shape(a))) return 1;
   a.y = nullptr;
   WideHead h{d->part, part_ent, d->targets, nvb, temperature, d->logits_out, nullptr, 0u, 0u, 0, nullptr, d->M, d->softcap};
   if (d->draw_id) {
