@@ -1826,6 +1826,7 @@ def test_norm_and_down_projection_in_one_launch(gpu, family, src, M, D, R, parts
     (1, 8, 2, 64, 128, 32, 32, 0, 127), (3, 32, 8, 128, 128, 32, 64, 0, 40),     # chunks without a key
     (70, 4, 1, 256, 288, 32, 32, 0, 280), (5, 4, 1, 256, 500, 32, 48, 100, 470),   # nine and sixteen chunks, a window
     (2, 32, 8, 128, 160, 32, 64, 0, 150),                                           # five chunks of 4096: two launches
+    (128, 4, 1, 64, 96, 32, 32, 0, 90), (129, 4, 1, 64, 96, 32, 32, 0, 90),         # 256 work-groups of rows and columns, and more: two launches
     (4, 8, 8, 64, 96, 96, 16, 0, 90), (9, 40, 8, 128, 64, 32, 16, 0, 63),           # one chunk; 5120 outputs
 ])
 def test_attention_and_down_projection(gpu, B, Hq, Hkv, dh, S, kv_chunk, R, window, at):

@@ -1375,12 +1375,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 }
 
 // Whether one launch merges the chunks and takes the adapter columns, sixteen per work-group: as long as a row's partials are 64 KB, which every
-// group of columns reads again, and two work-groups per compute unit hold them.  us, attention with two launches | one behind it: 32 heads of
-// 128, 64 columns, 4 chunks 32 rows 19.3 | 17.9, 6 chunks 3 rows 11.6 | 12.1, 8 chunks 16 rows 19.6 | 20.0; 2 chunks 100 rows 36.4 | 34.6; 4 heads of 256, 32
-// columns, 9 chunks 16 rows 12.2 | 10.8, 64 rows 15.5 | 13.6.
+// group of columns reads again, and every compute unit has at most one work-group (beyond, two share its registers and its reads).  us, attention with two launches |
+// one behind it, K and the adapter from memory: 32 heads of 128, 64 columns, 2 chunks 16 rows (64 work-groups) 14.0 | 12.8, 64 rows (256) 22.5 | 20.5, 80 rows (320)
+// 30.8 | 34.8; 4 chunks 48 rows 32.6 | 31.0, 100 rows 51.9 | 59.7; 16 heads of 128 80 rows x 8 chunks 42.6 | 47.0.
 constexpr int kCombineCols = 16;
 bool attn_lora_one_launch(int64_t rows, int64_t K, int n_chunks, int R) {
-  return K <= 8 * 256 * 2 && n_chunks * K * 4 <= 64 * 1024 && rows * cdiv(R, kCombineCols) <= 512;
+  return K <= 8 * 256 * 2 && n_chunks * K * 4 <= 64 * 1024 && rows * cdiv(R, kCombineCols) <= 256;
 }
 
 int next_pow2(int x) {
