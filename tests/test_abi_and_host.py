@@ -269,6 +269,15 @@ def test_partial_planes_have_room_at_every_row_count_of_a_runner(rows, override)
         assert split == 1 or split * M * f.N <= room, (f.names, M, split)
 
 
+@pytest.mark.parametrize("groups,S,head_dim,chunks", [
+    (1, 4000, 128, 32), (1, 65, 128, 1), (64, 1000, 128, 4), (128, 129, 64, 2), (129, 4000, 128, 1), (255, 4000, 128, 1), (256, 1025, 128, 2), (257, 1024, 64, 1),
+    (400, 4000, 64, 2), (401, 4000, 64, 1), (128, 4000, 256, 2), (129, 257, 256, 3), (129, 256, 256, 1), (171, 1025, 256, 4), (171, 1024, 256, 1),
+    (200, 3000, 256, 6), (256, 3000, 256, 1), (264, 700, 256, 4), (384, 700, 256, 3), (512, 3000, 256, 1), (513, 700, 256, 3), (640, 700, 256, 2), (901, 3000, 256, 1)])
+def test_key_chunks_of_a_decode_step(groups, S, head_dim, chunks):
+  from tunix_amd.model import Runner
+  assert Runner._key_chunks(groups, S, head_dim) == chunks
+
+
 def test_split_k_leaves_no_empty_split_and_goes_on_for_long_contractions():
   import math
   import types

@@ -555,17 +555,9 @@ class Runner(HeadRunner):
       self.next_tpart = torch.empty(n_planes * 8192, dtype=torch.float32, device=dev)
     self.splitk_ws = torch.empty(self._split_floats(), dtype=torch.float32, device=dev)
     if kv_chunk is None:
-      # decode: the key range of a (row, kv head) is split only as far as needed to put one work-group of four waves on every compute unit,
-      # in chunks of at least a key block per wave or so.  Attention with its merging pass and the o adapter, us in 1 | 2 | 4 | 8 chunks or so:
-      # 8 kv heads of 128, 16 rows x 700 keys 20.2 | 16.9 | 19.0 | 20.4, 1500 keys 32.8 | 24.7 | 25.8 | 27.6, 8 rows x 1000 24.2 | 18.0 | 15.5 |
-      # 17.1, 32 rows x 750 23.6 | 25.1 | 26.6 | 30.4; one kv head of 256, 64 rows x 288 18.5 | 14.2 | 12.0 | 14.7, 16 rows x 1200 48 | 30 | 21.7 | 15.7
-      # (12 chunks 14.6).  Two to a unit, of many keys, are cut in halves, which even out what the units have: 40 rows x 8 x 1280 52.6 | 44.2,
-      # 60 rows 59.2 | 58.0 (32 rows 33.3 | 35.0).
       kv_chunk = 0
-      waves = B * cfg.num_kv_heads
       if T == 1 and S > 64:
-        n_chunks = 2 if 256 <= waves <= 512 and S > 1024 else max(1, min(256 // waves, math.ceil(S / 128)))
-        kv_chunk = math.ceil(S / n_chunks / 32) * 32
+        kv_chunk = math.ceil(S / self._key_chunks(B * cfg.num_kv_heads, S, cfg.head_dim) / 32) * 32
         if kv_chunk >= S:
           kv_chunk = 0
     self.kv_chunk = kv_chunk
@@ -573,6 +565,31 @@ class Runner(HeadRunner):
     self.attn_ws = torch.empty(max(nb // 4, 1), dtype=torch.float32, device=dev)
     self.zero = torch.zeros(1, dtype=torch.int32, device=dev)
     self._init_head(B, D, bf, want_logits)
+
+  @staticmethod
+  def _key_chunks(groups: int, S: int, head_dim: int) -> int:
+    """Chunks that a decode step's key range of `groups` (row, kv head) pairs is cut into."""
+    # Only as far as needed to put one work-group of four waves on every compute unit, in chunks of at least a key block per wave or so.
+    # Attention with its merging pass and the o adapter, us in 1 | 2 | 4 | 8 chunks or so: 8 kv heads of 128, 16 rows x 700 keys 20.2 | 16.9 | 19.0 | 20.4,
+    # 1500 keys 32.8 | 24.7 | 25.8 | 27.6, 8 rows x 1000 24.2 | 18.0 | 15.5 | 17.1; one kv head of 256, 64 rows x 288 18.5 | 14.2 | 12.0 | 14.7,
+    # 16 rows x 1200 48 | 30 | 21.7 | 15.7 (12 chunks 14.6).
+    if groups <= 128:
+      return max(1, min(256 // groups, math.ceil(S / 128)))
+    # More: two to a unit, of many keys, are cut in halves, which even out what the units have: 40 rows x 8 heads of 128 x 1280 52.6 | 44.2 (32 rows
+    # 33.3 | 35.0, 56 rows x 1500 63.7 | 67.9; heads of 64, 256 rows x 2 x 1500 37 | 49).
+    if head_dim <= 128:
+      return 2 if 256 <= groups <= 400 and S > 1024 else 1
+    # Heads of 256, whose work-groups take twice as long: as many as fill the units evenly, two or four at a time (more than 512 in all run as
+    # single waves).  4 kv heads, us in 1 | 2 | 3 | 4 | 6 chunks, 1500 keys: 34 rows 62 | 61 | 45 | 54 | 49, 44 rows 65 | 63 | 66 | 57 | 57, 52 rows 67 | 65 | 68 |
+    # 69 | 60, 66 rows 109 | 95 | 86 | 82 | 78, 86 rows 114 | 103 | 99 | 99 | 98, 112 rows 120 | 130 | 128 | 116 | 128, 136 rows 179 | 162 | 149 | 183 | 173, 160 rows
+    # 186 | 172 | 172 | 192 | 186, 200 rows 238 | 224 | 240 | 246 | 235, 250 rows 251 | 265 | 277 | 281 | 275.
+    if S <= 256:
+      return 1
+    many = S > 1024
+    for most, n in ((170, 3), (192, 4 if many else 1), (208, 6 if many else 1), (256, 1), (340, 4), (440, 3), (512, 1), (560, 3), (900, 2)):
+      if groups <= most:
+        return n
+    return 1
 
   # ---- building blocks -----------------------------------------------------------------------
   SPLIT_ROWS = 128   # calls with more rows run unsplit
