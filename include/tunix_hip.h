@@ -248,9 +248,10 @@ int tnx_rmsnorm_pair(void* stream, const uint16_t* x, const float* ws, int split
 /* The norm ahead of a linear with a LoRA adapter, and the adapter's down-projection of what it writes:
  * one of tnx_rmsnorm (x), tnx_rmsnorm_splitk (ws, split_k), tnx_rmsnorm_moe_combine (y_route, topk_w, k) or,
  * with w2 and y2, tnx_rmsnorm_pair, then t[:, :R] = bf16(rows . a_t^T) as tnx_lora_down forms it (a_t bf16 [R, D];
- * the routing scores of an MoE layer are the same product).  Up to 256 rows this is one launch when D <= 4096 and
- * no output (h_out, y, y2) overlaps an input; the sums of t are then added in another order than tnx_lora_down's.
- * D % 32 == 0, R % 16 == 0. */
+ * the routing scores of an MoE layer are the same product).  One launch when no output (h_out, y, y2, t) overlaps an
+ * input, nor t another output, and there is at most one work-group per compute unit: of n = R / floor(256 / M) adapter columns each, rounded
+ * up to eight, at most 256 rows with n <= 32 where D <= 2048, at most 16 rows with n <= 16 where D <= 4096; the sums of t are then added in
+ * another order than tnx_lora_down's.  D % 32 == 0, R % 16 == 0. */
 typedef struct tnx_norm_lora_desc {
   int64_t M, D;
   float eps;

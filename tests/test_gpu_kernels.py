@@ -1822,6 +1822,34 @@ def test_norm_and_down_projection_in_one_launch(gpu, family, src, M, D, R, parts
     ops.norm_lora(a, t, w, y2, eps, fl, M, D)           # no input
 
 
+@pytest.mark.parametrize("place", ["x", "ws", "y_route", "res_pre", "w", "h_out"])
+def test_norm_and_down_projection_over_an_input(gpu, place):
+  """tnx_norm_lora with t in the memory of an input, or of its other output, that row's other work-groups still read: two launches, whose bits it has."""
+  from tunix_amd import ops
+  M, D, R, parts = 16, 512, 32, 2
+  got = []
+  for one in (False, True):
+    x, res, h, y = bf(rnd((M, D), 99)).to(gpu), bf(rnd((M, D), 98)).to(gpu), *(torch.zeros(M, D, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    w = bf(torch.cat([rnd((D,), 95, 0.3) + 1.0, torch.zeros(M * R)])).to(gpu)
+    ws, routes = rnd((parts, M, D), 100).to(gpu), bf(rnd((M * parts, D), 101)).to(gpu)
+    tw, a = bf(rnd((M, parts), 102, 0.2)).to(gpu), bf(rnd((R, D), 97)).to(gpu)
+    t = {"x": x, "ws": ws.view(torch.bfloat16), "y_route": routes, "res_pre": res, "w": w, "h_out": h}[place].reshape(-1)[:M * R].view(M, R)
+    if place in ("x", "w"):
+      ops.norm_lora(a, t, w, y, 1e-6, 0, M, D, x=x) if one else ops.rmsnorm(x, w, y, 1e-6, 0)
+    elif place == "y_route":
+      kw = dict(res_pre=res, h_out=h)
+      ops.norm_lora(a, t, w, y, 1e-6, 0, M, D, y_route=routes, topk_w=tw, k=parts, **kw) if one else ops.rmsnorm_moe_combine(
+          routes, tw, parts, w, y, 1e-6, 0, M, D, **kw)
+    else:
+      kw = dict(res_pre=res, h_out=h)
+      ops.norm_lora(a, t, w, y, 1e-6, 0, M, D, ws=ws, split_k=parts, **kw) if one else ops.rmsnorm_splitk(ws, parts, w, y, 1e-6, 0, M, D, **kw)
+    if not one:
+      ops.lora_down(y, a, t)
+    torch.cuda.synchronize()
+    got.append((y.clone(), t.clone(), h.clone()))
+  assert all(torch.equal(p, q) for p, q in zip(*got))
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,dh,S,kv_chunk,R,window,at", [
     (1, 8, 2, 64, 128, 32, 32, 0, 127), (3, 32, 8, 128, 128, 32, 64, 0, 40),     # chunks without a key
     (70, 4, 1, 256, 288, 32, 32, 0, 280), (5, 4, 1, 256, 500, 32, 48, 100, 470),   # nine and sixteen chunks, a window

@@ -271,6 +271,10 @@ __device__ __forceinline__ float soft_cap_fast(float z, float cap) {
 
 static inline hipStream_t as_stream(void* s) { return (hipStream_t)s; }
 static inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// Whether two ranges of memory share no byte (a null pointer is no range).
+static inline bool apart(const void* p, int64_t p_bytes, const void* q, int64_t q_bytes) {
+  return !p || !q || (uintptr_t)p + p_bytes <= (uintptr_t)q || (uintptr_t)q + q_bytes <= (uintptr_t)p;
+}
 
 // Raw buffer resources: 32-bit byte offsets, and loads whose vector offset (plus the
 // immediate) lies past the size return zeros instead of faulting.

@@ -663,15 +663,18 @@ extern "C" int tnx_norm_lora(void* stream, const tnx_norm_lora_desc* d) {
   const int in = d->ws ? kNormInPlanes : d->y_route ? kNormInRoutes : kNormInRow;
   const int parts = d->ws ? d->split_k : d->y_route ? d->k : 0;
   const NormRow n{d->y_route ? d->y_route : d->x, d->res_pre, d->h_out, d->w, d->res_post, d->y, D, d->eps, d->ws, parts, M * D, d->w2, d->y2, d->topk_w};
-  // A row's work-groups read it while the first of them writes: no output may lie in an input.
-  auto apart = [&](const void* out, const void* p, int64_t bytes) {
-    const char *o = (const char*)out, *q = (const char*)p;
-    return !o || !q || o + M * D * 2 <= q || q + bytes <= o;
-  };
-  bool separate = true;
-  for (const void* out : {(const void*)d->h_out, (const void*)d->y, (const void*)d->y2})
-    separate = separate && apart(out, d->x, M * D * 2) && apart(out, d->ws, parts * M * D * 4) && apart(out, d->y_route, parts * M * D * 2) &&
-               apart(out, d->res_pre, M * D * 2) && apart(out, d->res_post, M * D * 2);
+  // A row's work-groups read it while the first of them writes it and each writes its adapter columns: no output may lie in an input, and t not
+  // in another output either.
+  const int64_t row_bytes = M * D * 2, t_bytes = ((M - 1) * d->t_ld + d->R) * 2;
+  struct Range { const void* p; int64_t bytes; };
+  const Range ins[] = {{d->x, row_bytes}, {d->ws, 2 * parts * row_bytes}, {d->y_route, parts * row_bytes}, {d->res_pre, row_bytes}, {d->res_post, row_bytes}};
+  const Range outs[] = {{d->h_out, row_bytes}, {d->y, row_bytes}, {d->y2, row_bytes}};
+  bool separate = apart(d->t, t_bytes, d->topk_w, M * parts * 2) && apart(d->t, t_bytes, d->w, D * 2) && apart(d->t, t_bytes, d->w2, D * 2);
+  for (const Range& in : ins) {
+    separate = separate && apart(d->t, t_bytes, in.p, in.bytes);
+    for (const Range& out : outs) separate = separate && apart(out.p, out.bytes, in.p, in.bytes);
+  }
+  for (const Range& out : outs) separate = separate && apart(d->t, t_bytes, out.p, out.bytes);
   if (separate && norm_lora_one_launch(M, D, d->R)) {
     launch_rmsnorm_lora(as_stream(stream), M, d->flavor, in, n, RowAdapterArgs{d->a_t, d->R, row_adapter_cols(M, d->R), d->t, d->t_ld, 0, 0});
     TNX_CHECK_LAUNCH("norm_lora");
