@@ -372,11 +372,13 @@ size_t tnx_attn_ws_bytes(int64_t B, int64_t T, int64_t S, int Hq, int dh, int kv
 int tnx_gqa_attn(void* stream, const tnx_attn_desc* h_desc);
 
 /* tnx_gqa_attn, then the LoRA down-projection of its output rows, t[:, :R] = bf16(out . a_t^T) as tnx_lora_down forms it
- * (a_t bf16 [R, Hq * dh], R % 16 == 0).  Where the key range of a decode step is split over few chunks, the pass that
- * merges them takes the product too, whose sums are then added in another order. */
+ * (a_t bf16 [R, Hq * dh], R % 16 == 0).  Where the key range of a decode step is split into chunks whose partials are at most 64 KB a row
+ * (Hq * dh <= 4096), and B * R / 16 is at most 256, the pass that merges them takes the product too, whose sums are then added in another
+ * order (unless t lies in ws). */
 int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld);
 /* tnx_qknorm_rope_kvwrite(r), then tnx_gqa_attn_lora (a_t null: tnx_gqa_attn) of the same rows, heads and caches; q lies in r->q_out.  A decode
- * step whose qkv linear left up to eight partial planes takes one launch for the first two: q_out is not written then, and the step's own key
+ * step of heads of 64 or 128 whose qkv linear left up to eight partial planes, in which neither out nor ws lies, takes one launch for the first
+ * two as long as two work-groups per compute unit hold it (B * Hkv * chunks <= 512): q_out is not written then, and the step's own key
  * enters the softmax as a block of its own where a chunk (or the window) holds more than 64 keys; of fewer the output is bit for bit that of the two. */
 int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t,
                            int64_t t_ld);

@@ -1887,6 +1887,54 @@ def test_attention_and_down_projection(gpu, B, Hq, Hkv, dh, S, kv_chunk, R, wind
   assert bool((t[:, R:] == 7.0).all())
 
 
+@pytest.mark.parametrize("chunk,place", [(32, "t in ws"), (0, "out in planes"), (64, "ws in planes")])
+def test_attention_outputs_over_what_it_reads(gpu, chunk, place):
+  """The adapter's output in the memory of the chunks' partials, or the attention's in that of the qkv linear's planes, which other work-groups of
+  the same row still read: separate launches, whose bits it has."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  from tunix_amd.model import rope_timescale
+  B, S, Hq, Hkv, dh, R, parts = 4, 128, 8, 2, 64, 32, 4
+  ts = torch.from_numpy(rope_timescale(dh, 1e4)).to(gpu)
+  pos = torch.arange(S, dtype=torch.int32, device=gpu).repeat(B, 1).contiguous()
+  tokens, col = torch.ones(B, S, dtype=torch.int32, device=gpu), torch.full((1,), 120, dtype=torch.int32, device=gpu)
+  a = bf(rnd((R, Hq * dh), 106)).to(gpu)
+  got = []
+  for one in (False, True):
+    k, v = bf(rnd((B, Hkv, S, dh), 103)).to(gpu), bf(rnd((B, Hkv, S, dh), 104)).to(gpu)
+    planes, q = rnd((parts, B, (Hq + 2 * Hkv) * dh), 107).to(gpu), bf(rnd((B, Hq * dh), 105)).to(gpu)
+    n_ws = max(ops.attn_ws_bytes(B, 1, S, Hq, dh, chunk) // 4, 1)
+    ws, out = torch.zeros(n_ws, device=gpu), torch.zeros(B, Hq * dh, dtype=torch.bfloat16, device=gpu)
+    t = torch.zeros(B, R, dtype=torch.bfloat16, device=gpu)
+    if place == "t in ws":
+      t = ws.view(torch.bfloat16)[:B * R].view(B, R)
+    elif place == "out in planes":
+      out = planes.view(torch.bfloat16).reshape(-1)[:B * Hq * dh].view(B, Hq * dh)
+    else:
+      assert n_ws <= planes.numel()
+      ws = planes.view(-1)[:n_ws]
+    rd, d = L.RopeDesc(), L.AttnDesc()
+    for x in (rd, d):
+      x.B, x.T, x.S, x.Hq, x.Hkv, x.dh = B, 1, S, Hq, Hkv, dh
+      x.kcache, x.vcache, x.col_ptr = k.data_ptr(), v.data_ptr(), col.data_ptr()
+    rd.rope_flavor, rd.rope_scale, rd.timescale, rd.qk_norm = L.TNX_ROPE_QWEN3, 1.0, ts.data_ptr(), -1
+    rd.qkv_ws, rd.split_k, rd.positions, rd.pos_ld, rd.q_out = planes.data_ptr(), parts, pos.data_ptr(), S, q.data_ptr()
+    d.scale, d.q, d.out, d.ws, d.kv_chunk = dh ** -0.5, q.data_ptr(), out.data_ptr(), ws.data_ptr(), chunk
+    d.tokens, d.tok_ld = tokens.data_ptr(), S
+    if place == "t in ws":
+      ops.gqa_attn_lora(d, a, t) if one else ops.gqa_attn(d)
+    elif one:
+      ops.rope_gqa_attn_lora(rd, d, a, t)
+    else:
+      ops.rope_kvwrite(rd)
+      ops.gqa_attn(d)
+    if not one:
+      ops.lora_down(out, a, t)
+    torch.cuda.synchronize()
+    got.append((out.clone(), t.clone(), k, v))
+  assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
 @pytest.mark.parametrize("lora", [False, True])
 @pytest.mark.parametrize("B,Hq,Hkv,dh,S,kv_chunk,where", [
     (2, 8, 2, 128, 200, 0, "q"), (2, 8, 2, 64, 60, 0, "q"), (3, 4, 1, 256, 300, 0, "k"), (2, 8, 2, 128, 384, 96, "q"),

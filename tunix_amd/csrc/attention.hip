@@ -1552,7 +1552,9 @@ static int gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a
   const int64_t K = (int64_t)d->Hq * d->dh;
   TNX_REQUIRE(d->B > 0 && d->T > 0 && K > 0 && K % 32 == 0, "attn_lora: bad shape");
   const int n_chunks = d->kv_chunk > 0 ? (int)cdiv(d->S, d->kv_chunk) : 1;
-  const bool one = d->T == 1 && n_chunks > 1 && attn_lora_one_launch(d->B, K, n_chunks, R);
+  // (the groups of columns of a row write t while others still read its partials)
+  const bool one = d->T == 1 && n_chunks > 1 && attn_lora_one_launch(d->B, K, n_chunks, R) &&
+                   apart(t, ((d->B - 1) * t_ld + R) * 2, d->ws, (int64_t)tnx_attn_ws_bytes(d->B, 1, d->S, d->Hq, d->dh, d->kv_chunk));
   const int rc = gqa_attn(stream, d, !one, rope);
   if (rc != TNX_OK) return rc;
   if (!one) return tnx_lora_down(stream, d->out, d->B * d->T, K, a_t, R, t, t_ld);
@@ -1582,7 +1584,11 @@ extern "C" int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, cons
   const int n_chunks = d->kv_chunk > 0 ? (int)cdiv(d->S, d->kv_chunk) : 1;
   const bool aligned = (((uintptr_t)r->kcache | (uintptr_t)r->vcache) & 15) == 0;
   // (heads of 256, which three chunks form again each: 1.0 us more per layer than in two launches, Gemma3-1B, 64 rows)
-  const bool one = r->qkv_ws && r->split_k <= 8 && aligned && (d->dh == 64 || d->dh == 128) && several_waves(d, n_chunks, 0);
+  // The chunks of a head read its planes while the first to end writes its output: neither output may lie in them.
+  const int64_t planes = (int64_t)r->split_k * r->B * (r->Hq + 2 * r->Hkv) * r->dh * 4;
+  const bool separate = apart(d->out, d->B * d->Hq * d->dh * 2, r->qkv_ws, planes) &&
+                        apart(d->ws, (int64_t)tnx_attn_ws_bytes(d->B, 1, d->S, d->Hq, d->dh, d->kv_chunk), r->qkv_ws, planes);
+  const bool one = r->qkv_ws && r->split_k <= 8 && aligned && separate && (d->dh == 64 || d->dh == 128) && several_waves(d, n_chunks, 0);
   if (!one) {
     rc = tnx_qknorm_rope_kvwrite(stream, r);
     if (rc) return rc;
