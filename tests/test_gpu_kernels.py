@@ -2618,6 +2618,7 @@ def test_dense_experts_in_32_bits(gpu, K, N, counts, x_div):
     ("gemma3", 256, 16, 1, 8, 0, 0, 0),     # more heads than one batch of the waves takes, no adapter
     ("llama3", 128, 6, 2, 3, 0, 0, 16),     # no norms, three heads in lanes of four
     ("qwen3", 128, 8, 2, 9, 0, 0, 16),      # too many planes: the two launches
+    ("qwen3", 128, 11, 1, 8, 64, 0, 16),    # of a few keys one head more than a batch of the waves: the two launches
 ])
 def test_norms_rotation_and_attention_in_one_launch(gpu, family, dh, Hq, Hkv, split, chunk, window, R):
   """tnx_rope_gqa_attn_lora against the launches it stands for, at columns on both sides of the waves' shares: the cache bit for

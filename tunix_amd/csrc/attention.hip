@@ -1588,7 +1588,12 @@ extern "C" int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, cons
   const int64_t planes = (int64_t)r->split_k * r->B * (r->Hq + 2 * r->Hkv) * r->dh * 4;
   const bool separate = apart(d->out, d->B * d->Hq * d->dh * 2, r->qkv_ws, planes) &&
                         apart(d->ws, (int64_t)tnx_attn_ws_bytes(d->B, 1, d->S, d->Hq, d->dh, d->kv_chunk), r->qkv_ws, planes);
-  const bool one = r->qkv_ws && r->split_k <= 8 && aligned && separate && (d->dh == 64 || d->dh == 128) && several_waves(d, n_chunks, 0);
+  // Of few keys the heads bound it, three a wave at a time, and a second batch of them pays with many rows of heads of 64 only.  us, two
+  // launches | one, 64 keys: 10 + 2 heads of 128 16 rows 11.9 | 12.2; 12 + 2 12.2 | 13.9, 2 x (16 + 2) 13.4 | 15.3, 64 rows 14.3 | 15.7; 4 x (12 + 2)
+  // heads of 64 16 rows 12.8 | 13.4, 100 rows 16.0 | 15.2, 4 x (16 + 2) of 128 70 rows 19.1 | 20.2; 90 keys: 12 + 2 of 128 16 rows 15.6 | 13.2.
+  const int64_t groups = (int64_t)d->B * d->Hkv;
+  const bool heads_fit = d->Hq <= (3 * kAttnWaves - 2) * d->Hkv || (d->dh == 64 && groups > 256) || several_waves(d, n_chunks, 64);
+  const bool one = r->qkv_ws && r->split_k <= 8 && aligned && separate && (d->dh == 64 || d->dh == 128) && heads_fit && several_waves(d, n_chunks, 0);
   if (!one) {
     rc = tnx_qknorm_rope_kvwrite(stream, r);
     if (rc) return rc;
