@@ -483,12 +483,29 @@ class StackRunner(HeadRunner):
     if m.heads // m.kv_heads > 16:
       n = min(math.ceil(1024 / waves), S // 32)
     else:
-      n = 2 if 256 <= waves <= 512 and S > 1024 else max(1, min(256 // waves, math.ceil(S / 128)))
-      # (the pass that merges chunks takes 3.8 us; a compute unit draws 28 KB of keys and values in one)
-      if S * (m.dim + m.vdim) * 2 / 28e3 * (1 - 1 / n) < 4.0:
-        n = 1
+      n = self._key_chunks(waves, S, m.dim + m.vdim)
     chunk = max(32, _up(math.ceil(S / n), 32))
     return 0 if chunk >= S else chunk
+
+  @staticmethod
+  def _key_chunks(groups: int, S: int, width: int) -> int:
+    """Chunks of the key range of `groups` (row, kv head) pairs, a key and its value `width` numbers."""
+    # As few as fill the units evenly.  One query head on a kv head or a few, us in 1 | 2 | 3 | 4 | 5 chunks: heads of 256, 60 pairs x 1000 keys 33 | 24 | 21 |
+    # 18 | 26, 96 x 2500 78 | 52 | 66 | 56 | 49, 128 x 2500 82 | 58 | 71 | 60 | 64, 140 x 2500 83 | 95 | 72 | 74 | 64, 176 x 4000 136 | 146 | 142 | 120 | 124, 208 x 2500
+    # 92 | 102 | 99 | 100 | 115, 320 x 2500 172 | 146 | 137 | 171 | 154, 360 x 1500 108 | 95 | 117 | 114 | 104, 440 x 1500 114 | 121 | 141 | 129 | 132; keys of 192 with values
+    # of 128, 96 x 2500 56 | 38 | 46 | 38 | 34, 140 x 2500 58 | 66 | 49 | 51 | 45, 280 x 1000 49 | 43 | 42 | 43 | 41; heads of 128, 140 x 4000 65 | 71 | 54 | 58 | 50.
+    many = S > 1024
+    if groups <= 128:
+      n = 5 if 85 < groups <= 102 and many else max(1, min(256 // groups, math.ceil(S / (96 if width >= 512 and S <= 512 else 128))))
+    else:
+      n = 1
+      for most, k in ((170, 3 if many else 1), (192, 4 if S > (1024 if width > 256 else 2048) else 1), (256, 1), (340, 3), (380, 2)):
+        if groups <= most:
+          n = k
+          break
+    # (the pass that merges chunks takes 3.8 us; a compute unit draws 28 KB of keys and values in one)
+    rounds = lambda k: math.ceil(groups * k / 256) / k
+    return n if S * width * 2 / 28e3 * (1 - rounds(n) / rounds(1)) >= 4.0 else 1
 
   def _latent_chunk(self, m: LatentMixer) -> int:
     """The same for latent attention, whose work-groups have a compute unit to themselves."""
