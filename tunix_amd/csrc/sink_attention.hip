@@ -314,10 +314,13 @@ void launch_f32(hipStream_t st, const SinkArgs& a) {
 // saves the pass that merges single waves' chunks and the trip of their partials through memory: 16 heads of 128 on 4, 32 rows x 304 keys 12.6 us
 // -> 8.7, the whole rollout of the Nunezen layers 25.6 ms -> 25.1.
 constexpr int kStepWaves = 4;
+constexpr int step_stages(int ks, int nh, int nj) { return ks * 8 + nh * 4 * nj <= 64 ? 2 : 1; }
 template <int KS, int NH, int NJ, bool BIAS, int W>   // 32-deep k-steps, halves of V, value columns per lane and half
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 2))) void sink_attn_step_kernel(const SinkArgs a) {
+// (two stages fit in the 256 registers that leave a SIMD two waves, if only just; heads of 128 with slopes or chunks took 260 without being told so: 1120
+// pairs of rows and kv heads, 531 keys, 64 against 56 us)
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(step_stages(KS, NH, NJ), 2))) void sink_attn_step_kernel(const SinkArgs a) {
   constexpr int DK = KS * 32, DV = NH * NJ * 16;
-  constexpr int NS = KS * 8 + NH * 4 * NJ <= 64 ? 2 : 1;
+  constexpr int NS = step_stages(KS, NH, NJ);
   typedef uint32_t vfrag __attribute__((ext_vector_type(NJ / 2)));
   const int lane = threadIdx.x & 63, lm = lane & 15, lq = lane >> 4;
   const int wave = W > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
