@@ -281,7 +281,7 @@ def test_key_chunks_of_a_decode_step(groups, S, head_dim, chunks):
 @pytest.mark.parametrize("groups,S,width,chunks", [
     (1, 4000, 256, 32), (40, 300, 512, 4), (40, 300, 256, 1), (60, 1000, 512, 4), (85, 2500, 512, 3), (86, 2500, 512, 5), (102, 1025, 512, 5), (96, 1024, 512, 2),
     (103, 2500, 512, 2), (128, 4000, 256, 2), (129, 2500, 512, 3), (129, 1024, 512, 1), (171, 1500, 512, 4), (171, 1500, 256, 1), (171, 2500, 256, 4),
-    (193, 4000, 512, 1), (256, 4000, 512, 1), (257, 1000, 512, 3), (257, 100, 128, 1), (340, 600, 512, 3), (341, 1500, 512, 2), (381, 4000, 512, 1)])
+    (32, 256, 512, 8), (8, 256, 320, 8), (8, 256, 256, 1), (33, 256, 512, 2), (32, 224, 512, 2), (32, 257, 512, 3), (193, 4000, 512, 1), (256, 4000, 512, 1), (257, 1000, 512, 3), (257, 100, 128, 1), (340, 600, 512, 3), (341, 1500, 512, 2), (381, 4000, 512, 1)])
 def test_key_chunks_of_a_layer_list_step(groups, S, width, chunks):
   from tunix_amd.stack_model import StackRunner
   assert StackRunner._key_chunks(groups, S, width) == chunks

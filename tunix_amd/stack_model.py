@@ -494,9 +494,12 @@ class StackRunner(HeadRunner):
     # 18 | 26, 96 x 2500 78 | 52 | 66 | 56 | 49, 128 x 2500 82 | 58 | 71 | 60 | 64, 140 x 2500 83 | 95 | 72 | 74 | 64, 176 x 4000 136 | 146 | 142 | 120 | 124, 208 x 2500
     # 92 | 102 | 99 | 100 | 115, 320 x 2500 172 | 146 | 137 | 171 | 154, 360 x 1500 108 | 95 | 117 | 114 | 104, 440 x 1500 114 | 121 | 141 | 129 | 132; keys of 192 with values
     # of 128, 96 x 2500 56 | 38 | 46 | 38 | 34, 140 x 2500 58 | 66 | 49 | 51 | 45, 280 x 1000 49 | 43 | 42 | 43 | 41; heads of 128, 140 x 4000 65 | 71 | 54 | 58 | 50.
+    # (wide heads and up to 256 keys: a block each, to single waves: heads of 256, 16 pairs x 256 keys 11.8 whole, 11.2 in halves, 9.4; of 192 | 128, 8 pairs 8.8, 9.2, 8.1)
+    if width >= 320 and 224 < S <= 256 and groups <= 32:
+      return 8
     many = S > 1024
     if groups <= 128:
-      n = 5 if 85 < groups <= 102 and many else max(1, min(256 // groups, math.ceil(S / (96 if width >= 512 and S <= 512 else 128))))
+      n = 5 if 85 < groups <= 102 and many else max(1, min(256 // groups, math.ceil(S / (96 if width >= 512 and 256 < S <= 512 else 128))))
     else:
       n = 1
       for most, k in ((170, 3 if many else 1), (192, 4 if S > (1024 if width > 256 else 2048) else 1), (256, 1), (340, 3), (380, 2)):
