@@ -1313,7 +1313,7 @@ def main():
     write_traffic_profile(*args.write_traffic_profile)
     return
   if args.gpus != 1:
-    print("bench.py measures one GPU: this build has no multi-GPU path (the decode path shards "
+    print("bench.py measures one GPU: there is no multi-GPU path (the decode path shards "
           "by batch rows with no exchange); run with --gpus 1", file=sys.stderr)
     sys.exit(2)
 

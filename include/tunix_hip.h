@@ -765,8 +765,11 @@ int tnx_rownorm_kvwrite(void* stream, const tnx_rownorm_kvwrite_desc* d);
  * holds exp(sinks[head]) (sinks null: none).  out[row, head * out_head ..] (out_head 0: dv).  kv_chunk > 0 splits the key range (few
  * query rows, workspace of tnx_sink_attn_ws_bytes).  slopes (null: none; [H]): slopes[head] times the distance of the
  * two positions is taken off a score.  chunk > 0: a position sees the keys of its own chunk alone, chunks of that many
- * positions counted from starts[b].  tnx_sink_attn_pad: the padded head size the
- * MFMA kernels take (other sizes, and fp32, run a plain kernel). */
+ * positions counted from starts[b].  tnx_sink_attn_pad: the padded head size the bf16 MFMA kernels take; fp32 runs 32-bit
+ * MFMAs at heads of up to 128, any multiple of 4, and more than a few queries, and everything else plain loops.
+ * The bf16 MFMA kernels multiply a masked key's value by its weight of zero: as for tnx_gqa_attn every slot that they read
+ * (columns up to the last position's block of 32, or the split's) must hold finite values.  In the fp32 kernels a value that is no
+ * number reaches only the positions that see it. */
 typedef struct {
   int64_t B, T, S;
   int H, G, dk, dv, dkp, dvp;

@@ -1,7 +1,7 @@
 """CPU oracle: a restatement of the reference's algorithm for the quantized rollout-decode path.
 
 TEST INFRASTRUCTURE ONLY.  Nothing in the product package may import this directory; only
-tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg use it, as the checker.
+tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg use it, to compare with.
 
 Every function cites the google/tunix file:line it follows (paths relative to the reference
 tree).  Pinning status of each part:

@@ -5,7 +5,7 @@ threefry2x32 (Salmon et al., SC'11; 20 rounds) as jax._src.prng uses it: PRNGKey
 the "partitionable" layout (counter (hi, lo) = 64-bit index, output x0 ^ x1) and in the
 original layout (counter array split in two halves); uniform / randint / gumbel / categorical.
 
-jax is not importable in this build, so this file is pinned by the golden arrays the
+jax is not importable here, so this file is pinned by the golden arrays the
 reference's own tests hold for jax.random.PRNGKey(0) inputs (tests/rl/common_test.py:35-108);
 see tests/test_oracle_rl.py (the threefry and golden-array tests) for which layout reproduces them.
 """

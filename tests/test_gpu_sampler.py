@@ -3,8 +3,8 @@
 Greedy ids: the oracle is teacher-forced with the ids the GPU produced; at every generated
 position the GPU id must be the oracle's arg-max, or lie within two bf16 ulps of it (the logits
 are bf16 values, so near-ties flip with the fp32 accumulation order; every such case is listed
-with its top-2 margin, and the counts go to a summary file next to the run's other outputs).  Log-probs: <= 2e-2 absolute against the oracle's bf16 flow and against
-the fp32 reference mode (the tolerance north_star states for bf16).
+with its top-2 margin, and the counts go to a summary file next to the run's other outputs).
+Log-probs: <= 2e-2 absolute against the oracle's bf16 flow and against the fp32 reference mode.
 """
 import numpy as np
 import pytest

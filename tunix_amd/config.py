@@ -61,7 +61,7 @@ class ModelConfig:
     if self.num_heads % self.num_kv_heads:
       raise ValueError("num_heads must be a multiple of num_kv_heads")
 
-  # ---- helpers shared by the engine and by checkers ----------------------------------------
+  # ---- helpers shared by the engine and by tests ----------------------------------------
   def is_local_layer(self, i: int) -> bool:
     return self.family == "gemma3" and (i % GEMMA3_PATTERN_LEN) != GEMMA3_PATTERN_LEN - 1
 

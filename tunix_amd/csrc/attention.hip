@@ -7,6 +7,7 @@
 // and the max / sum of the online softmax are per-lane scalars reduced over 4 lanes.  V rows
 // are loaded in their natural [key][dh] layout (256 B contiguous per key) and transposed
 // inside each lane with v_perm_b32 to form B fragments; keys and values go through LDS only in the work-group form for many positions below.
+// In a decode step of up to 512 work-groups four waves share a chunk's keys and merge what they have through LDS (several_waves).
 #include <string.h>
 
 #include <mutex>
@@ -203,13 +204,9 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
   // compile-time choice: a branch around loads would make every wait behind it assume that the
   // shorter side was taken.
 
-  // A ring of NS register stages: the loads of the next NS-1 key blocks are in flight while a
-  // block is computed, so the memory system is never left idle behind a wave's softmax and
-  // MFMAs.  One wave per SIMD owns the whole register file for this (nothing else hides the
-  // latency: a wave has no second wave to alternate with).  Prefetches past the last block are
-  // redirected to the last block (cache hits) rather than skipped: with every load issued
-  // unconditionally the number of loads in flight is static, and the wait for a stage's data
-  // does not have to drain the younger stages.
+  // NS register stages: the loads of the next key block are in flight while a block is computed, so the memory system is never left idle behind a
+  // wave's softmax and MFMAs.  No load of the loop stands behind a branch, so that the number in flight is static and the wait for a stage's data does
+  // not drain the younger one; the last one or two blocks have code of their own (below), and none is loaded twice.
   struct Stage {
     u32x4 kf[2][KS];
     u32x4 vf[NH][8];

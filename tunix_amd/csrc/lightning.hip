@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void lightning_any_kernel(const LightArgs a, c
 }
 
 // Prompts token by token with the state in registers (state_scan.h); grid (H, columns / 64, B).  2 x 1200 tokens of 16 heads of 128 x 128 in fp32:
-// 25.4 ms before, when the state went through memory with every token, 0.75 now.
+// 25.7 ms before, when the state went through memory with every token, 0.78 now.
 template <int R, typename T>
 __global__ __launch_bounds__(256) void lightning_token_kernel(const LightArgs a, const RowSrc<T> src) {
   const int h = blockIdx.x, d0 = blockIdx.y * kScanCols;

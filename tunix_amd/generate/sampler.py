@@ -258,7 +258,7 @@ class Sampler:
     """Samples a completion of the input prompts (sampler.py:738-1011).
 
     If top_p is provided the sampling mode is top_p (top_k alone does not enable sampling);
-    otherwise greedy.  Beam search is not part of this build.
+    otherwise greedy.  Beam search is not supported.
     """
     model, dev = self._transformer, self._transformer.device
     cfg = model.cfg
@@ -283,7 +283,7 @@ class Sampler:
     if beam_size is not None:
       if top_p is not None:
         utils.check_sampling_mode_conflict(["beam_search"], "top_p")
-      raise NotImplementedError("beam search is outside the rollout decode path of this build")
+      raise NotImplementedError("beam search is outside the rollout decode path")
     key = _threefry_seed(0 if seed is None else seed)
 
     B = all_input_ids.shape[0]
