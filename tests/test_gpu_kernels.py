@@ -272,6 +272,66 @@ def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank,
     assert (tf.float() - tm[:M].float()).abs().max().item() <= 2.0 ** -6 * tm.float().abs().max().item()
 
 
+@pytest.mark.parametrize("M,K,N,split,group,qtype,rank,mul", [
+    (1, 128, 16, 1, 64, Q.NF4, 0, False),        # one k-tile, one column tile
+    (8, 640, 272, 2, 32, Q.INT4, 64, False),     # three and two k-tiles; a last block of one column tile
+    (8, 6144, 128, 1, 64, Q.NF4, 64, False),     # 48 k-tiles: what LDS holds of eight rows
+    (5, 7296, 256, 1, 64, Q.NF4, 32, True),      # 57: two chunks of slots filled again, the last with one
+    (7, 10368, 128, 1, 128, Q.INT4, 96, False),  # 81: one more than without a table; a rank past 64
+    (9, 3072, 128, 1, 64, Q.NF4, 64, True),      # 24, of sixteen rows
+    (16, 4224, 144, 1, 32, Q.NF4, 64, False),    # 33
+    (13, 5248, 256, 1, 64, Q.INT4, 0, True),     # 41 (40 are held)
+    (17, 1536, 128, 1, 64, Q.NF4, 64, False),    # 12, of 32 rows
+    (32, 2176, 384, 1, 64, Q.NF4, 64, True),     # 17
+    (31, 2688, 160, 1, 128, Q.INT4, 64, True),   # 21 (20 are held)
+    (24, 8192, 128, 4, 32, Q.NF4, 32, False),    # sixteen per split
+])
+def test_few_rows_at_the_edges_of_what_lds_holds(gpu, M, K, N, split, group, qtype, rank, mul):
+  """Linears of at most 32 rows against 64 bits over the same weights, both rounded to bf16.  The fp32 sum of K products of about 0.03 is off by
+  some eps of the sum of their magnitudes, 2^-23 * 0.03 K (`off`, what a result near zero may differ by), a hundredth of a bf16 ulp of the usual
+  result of 0.03 sqrt(K): the rounded values are equal but for near ties.  Gated products are rounded at every step."""
+  off = 2.0 ** -23 * 0.03 * K
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  x, t = bf(rnd((M, K), 311)).to(gpu), bf(rnd((M, 2 * max(rank, 32)), 312)).to(gpu)
+  w = bf(rnd((K, N), 313, 0.03)).to(gpu)
+  c, s = ops.quantize_pack(w, group, qtype, mul)
+  lb = bf(rnd((N, max(rank, 32)), 314, 0.1)).to(gpu)
+  # (interleaved: column tile 2 i is gate tile i, 2 i + 1 up tile i; the dequantised weights come back as they went in)
+  deq = ops.qw_dequant(c, s, K, N, group, qtype, mul).double()
+  cols = torch.arange(N, device=gpu)
+  place = (cols % (N // 2)) // 16 * 32 + cols // (N // 2) * 16 + cols % 16 if mul else cols   # packed column of each
+  y64 = x.double() @ deq
+  if rank:
+    seg = cols // (N // 2) if mul else torch.zeros_like(cols)
+    td = t.double()
+    for g in range(2 if mul else 1):
+      at = torch.nonzero(seg == g)[:, 0]
+      y64[:, at] += 1.5 * (td[:, g * rank:(g + 1) * rank] @ lb.double()[place[at], :rank].T)
+  kw = dict(lora_rank=rank, lora_nseg=-1 if mul else 1, lora_seg_end=[N // 2, N] if mul else [N], lora_seg_toff=[0, rank] if mul else [0], t=t,
+            t_ld=t.shape[1], lora_b=lb, lora_scale=1.5) if rank else {}
+  y = torch.full((M, N // 2 if mul else N), 7.0, dtype=torch.bfloat16, device=gpu)
+  ws = torch.full((split * M * N,), float("nan"), device=gpu) if split > 1 else None
+  nxt = {}
+  if mul:
+    nxt = dict(next_a_t=bf(rnd((64, N // 2), 315, 0.05)).to(gpu), next_rank=64, next_tpart=torch.full(((N + 127) // 128 * 8192,), float("nan"), device=gpu))
+  ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=group, qtype=qtype, x=x, codes=c, scales=s, y=y, split_k=split, ws=ws,
+                                    epilogue=L.TNX_EPI_SILU_MUL if mul else L.TNX_EPI_STORE, **kw, **nxt))
+  torch.cuda.synchronize()
+  if mul:
+    r = lambda v: v.float().bfloat16().double()
+    g, u = r(y64[:, :N // 2]), r(y64[:, N // 2:])
+    assert_bf16_close(y, r(r(g * r(torch.sigmoid(g))) * u), min_equal=0.95, what="gated", ulps=3, atol=2 * off * g.abs().max().item())
+    tn = torch.zeros(M, 64, dtype=torch.bfloat16, device=gpu)
+    ops.lora_reduce(nxt["next_tpart"], M, (N + 127) // 128, 64, tn)
+    torch.cuda.synchronize()
+    want = y.double() @ nxt["next_a_t"].double().T
+    # (products of the same activations, summed in fp32 and rounded once)
+    assert_bf16_close(tn, r(want), min_equal=0.95, what="next adapter", atol=1e-5 * want.abs().max().item())
+  else:
+    assert_bf16_close(y, y64.float().bfloat16(), what="linear", atol=off)
+
+
 @pytest.mark.parametrize("rows,copy,split", [(65536, False, 1), (65536, True, 1), (100, False, 1), (100, False, 2), (16, False, 1)])
 def test_silu_of_every_gate(gpu, rows, copy, split):
   """Gates of every finite bf16 value (weights that pick one element of x), among them those whose sigmoid is not a normal fp32

@@ -1,6 +1,6 @@
 // The quantised GEMM (rollout batch, prefill, per-token logps): one work-group = 8 waves = two
-// per SIMD, output tile 16 * MT rows x (64 * NT) columns (MT = 8: 128 rows; 1, 2, 4 for decode
-// batches of up to 16, 32, 64 rows); a wave covers all rows x (16 * NT) columns over one half
+// per SIMD, output tile 16 * MT rows x (64 * NT) columns (MT = 8: 128 rows; 4 for decode
+// batches of 33 to 64 rows; fewer are qgemm_few.h's); a wave covers all rows x (16 * NT) columns over one half
 // of every k-tile.  At 128 rows the op sits past the MFMA/HBM ridge of the machine (2 * 128 flop
 // per 0.53 B of weights), so the loop is built around keeping the matrix pipe fed:
 //
@@ -92,12 +92,18 @@ __device__ __forceinline__ void fill_level_table(uint32_t base, int tid) {
 
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 constexpr uint32_t kRowsActBytes = 72 * 2;            // per row of the activation staging
+// byte offset of fragment j of columns [16 n, + 16) of the next linear's adapter, over this work-group's 64 activated columns
+__device__ __forceinline__ uint32_t next_a_off(const QLArgs& a, int n, int j, int lm, int lq) {
+  const int64_t ldy = a.N / 2, k = (int64_t)blockIdx.y * 64 + j * 32 + lq * 8;
+  return n * 16 < a.next_rank && k + 8 <= ldy ? (uint32_t)(((int64_t)(n * 16 + lm) * ldy + k) * 2) : 0xfffffff0u;
+}
 // The end of a work-group of eight waves over 16 * MT rows x 128 columns: wave wv holds in `out` the sums of row tiles
 // (wv / 4) * HM ... and column tiles 2 (wv % 4), + 1 (with one row tile waves 0-3 hold all of it).  act_lds: 16 MT rows of
-// kRowsActBytes; scr_lds (SCRATCH): 16 x 36 floats per wave; both idle for every wave by now.
-template <int MT, int NT, bool SCRATCH>
+// kRowsActBytes; scr_lds (SCRATCH): 16 x 36 floats per wave; both idle for every wave by now.  PRE (one row tile): wave n < 4 has asked for its
+// fragments of the next linear's adapter itself, `pre`.
+template <int MT, int NT, bool SCRATCH, bool PRE = false>
 __device__ __forceinline__ void quant_rows_out(const QLArgs& a, f32x4 (&out)[(MT + 1) / 2][NT], int64_t m0, int64_t ntile0, int wv,
-                                               uint32_t act_lds, uint32_t scr_lds) {
+                                               uint32_t act_lds, uint32_t scr_lds, const u32x4* pre = nullptr) {
   constexpr int HM = (MT + 1) / 2, ROWS = 16 * MT;
   const int tid = threadIdx.x, lane = tid & 63, lm = lane & 15, lq = lane >> 4, wn = wv & 3, kh = wv >> 2;
   const bool has_rows = MT > 1 || kh == 0;
@@ -113,16 +119,12 @@ __device__ __forceinline__ void quant_rows_out(const QLArgs& a, f32x4 (&out)[(MT
     const int64_t wgcol0 = (int64_t)blockIdx.y * 64;      // first act column of the work-group
     const bool fuse_next = a.next_tpart != nullptr;
     u32x4 bn[4][2];
-    if (fuse_next) {
+    if (fuse_next && !PRE) {
       const rsrc_t rn = make_rsrc(a.next_a_t, (uint64_t)a.next_rank * ldy * 2);
 #pragma unroll
       for (int n = 0; n < 4; ++n)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int64_t k = wgcol0 + j * 32 + lq * 8;
-          const bool ok = n * 16 < a.next_rank && k + 8 <= ldy;
-          bn[n][j] = buf_load128(rn, ok ? (uint32_t)(((int64_t)(n * 16 + lm) * ldy + k) * 2) : 0xfffffff0u);
-        }
+        for (int j = 0; j < 2; ++j) bn[n][j] = buf_load128(rn, next_a_off(a, n, j, lm, lq));
     }
     if (has_rows) {
 #pragma unroll
@@ -146,7 +148,14 @@ __device__ __forceinline__ void quant_rows_out(const QLArgs& a, f32x4 (&out)[(MT
       if (m0 + row < a.M && wgcol0 + ch * 8 + 8 <= ldy)
         __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(y + (m0 + row) * ldy + wgcol0 + ch * 8));
     }
-    if (fuse_next && wv < MT) {   // one row tile per wave; fewer rows leave plane slots unwritten
+    if (PRE && fuse_next && wv < 4) {
+      float* plane = a.next_tpart + (int64_t)blockIdx.y * 8192;
+      f32x4 pacc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 2; ++j) pacc = mfma16(lds_ld128(act_lds + (uint32_t)((lm * ACT_LD + j * 32 + lq * 8) * 2)), pre[j], pacc);
+      __builtin_nontemporal_store(pacc, reinterpret_cast<f32x4*>(plane + (wv * 64 + lane) * 4));
+    }
+    if (!PRE && fuse_next && wv < MT) {   // one row tile per wave; fewer rows leave plane slots unwritten
       float* plane = a.next_tpart + ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * 8192;
       {
         const int mt = wv;
@@ -205,9 +214,8 @@ __device__ __forceinline__ void quant_rows_out(const QLArgs& a, f32x4 (&out)[(MT
 
 // 512 threads: waves 0-3 and 4-7 share the four column groups and split every k-tile between
 // them (k-steps 0,1 | 2,3), which puts two waves on each SIMD at 256 registers each.
-// MT = row tiles of 16 (8 for 65+ rows; 1, 2, 4 for decode batches of up to 16, 32, 64 rows: the
-// weight stream and its dequantisation are the same, the MFMA, fragment and activation work
-// shrink with the rows).
+// MT = row tiles of 16 (8 for 65+ rows; 4 for decode batches of 33 to 64 rows: the weight stream
+// and its dequantisation are the same, the MFMA, fragment and activation work shrink with the rows).
 // INT4: integer codes, converted without the table (Int4Magic in common.h).
 template <int NT, int SPT, int MT, bool INT4 = false>
 __global__ __launch_bounds__(512)

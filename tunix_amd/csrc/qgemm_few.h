@@ -1,39 +1,53 @@
-// The quantised GEMM over at most 16 rows (a decode batch): one work-group = 8 waves = 16 rows x 128 columns of one k split, no
-// barrier between its first and its last load.
+// The quantised GEMM over at most 32 rows (a decode batch): one work-group = 8 waves = ROWS (8, 16 or 32) rows x 128 columns of one k split, a
+// wave a column tile of 16 over the whole of it.
 //
-// What bounds it is the round trip to memory, then the weight stream and the conversion of the codes (two lane-instructions per
-// weight).  So nothing is shared between waves that would have to be waited for: of CW x KW = 8 waves, wave (ch, ks) takes 128 / CW
-// columns over the k-tiles ks, ks + KW, ..., reads its activation fragments straight from memory (the rows of a decode batch live in the
-// L2; rows past M cost nothing), keeps PF k-tiles in flight in registers, and the KW partial sums of a column meet in LDS once,
-// at the end.  qgemm128_kernel shares the activations through LDS behind one barrier per k-tile: 24 KB per compute unit in flight and
-// its waves in step; here it is 64 to 96 KB, and every wave runs on as its own data arrives.
-// CW = 4: fewer sums to exchange, activations read four times over: for up to 8 rows.  CW = 2: twice over, for up to 16 rows and many
-// k-tiles.  CW = 1 pays a microsecond for the exchange of 64 KB; at 32 rows the shared form wins everywhere.  Which calls come here:
-// few_shape in qlinear.hip.  The planes of a split are stored as they lie in the accumulators and without the non-temporal policy:
-// with it the pass that sums them waits longer than this one gains (14336 -> 4096 in 8 splits, 8 rows, with that pass: 16.1 us
-// against 17.0, 4096 -> 4096 in 8: 11.6 against 12.5).
+// What bounds it is the launch and the round trip to memory, then the conversion of the codes: five instructions per pair of weights and lane
+// (address, look-up, two products, rounding), of which a compute unit finishes a k-tile (8192 pairs) in 0.36 us or so, looked up, converted and
+// multiplied, where vector instructions alone would take 0.28; 4096 -> 28672 has 32 of them per unit, 11.5 of its 18 us, and its 62 MB of codes
+// and scales take some 11 us.  So:
+//   * the activations, which all waves share, are requested once, as whole kilobytes straight into LDS, ahead of everything else.  (As fragments
+//     from memory, 16 bytes of 16 rows a load, they come at a third of that rate and once per wave: the first loads of 4096 -> 28672 over 16 rows
+//     took 6 us to be asked for, now 2.)  There is no barrier in the loop as long as LDS holds them, up to 12 to 80 k-tiles by rows and code book;
+//   * a wave has a column tile of its own over the whole k range: no sums to exchange, and little code (8 KB; a work-group's first pass over its
+//     instructions is part of every launch: the same kernel with six k-tiles in flight and a copy of the loop for the tiles left, 22 KB, is
+//     0.5 to 1 us slower at every size, with three tiles or two at long contractions 0.2 and 5 us).
+// us, before (activations as fragments from memory, or through LDS behind a barrier per k-tile) | now, weights from HBM, NF4 of group 64 with an
+// adapter of rank 64, splits without the pass that sums them:
+//                                   1 row        8 rows       16 rows       32 rows
+//   4096 -> 6144 in 5           8.5 |  6.6    9.1 |  6.7    9.4 |  7.1    9.9 |  8.6
+//   4096 -> 4096 in 8           7.5 |  5.4    7.7 |  5.6    7.8 |  5.8    8.3 |  6.9
+//   4096 -> 28672 gated        18.8 | 17.8   20.2 | 18.5   20.7 | 18.8   24.7 | 22.5
+//   14336 -> 4096 in 8         11.3 |  9.4   12.1 |  9.9   13.2 | 10.2   14.2 | 12.5
+//   int4 1152 -> 13824 gated    8.4 |  7.6    9.8 |  7.6    9.9 |  7.8   10.4 |  9.0
+//   int4 1024 -> 1152 in 8      5.0 |  3.3    5.2 |  3.7    5.2 |  3.9    5.5 |  4.7
+// Over 94 shapes (20 contractions x 5 forms of code book, group and adapter) the geometric mean is 0.80 at 1 to 16 rows and 0.88 at 17 to 32, and
+// none is slower but contractions of 64 k-tiles on eight work-groups (8192 -> 1024 unsplit, which the decoder splits: 27.4 | 29.3).  At 33 to 64 rows,
+// where eight waves read 128 KB of fragments per k-tile, the form was faster only up to three k-tiles, by 2 to 10 %: those calls are qgemm128_kernel's.
+// Also slower: sixteen waves with half a k-tile each (4096 -> 28672 over one row 23.0 us), column tiles in pairs over half of the k-tiles (the
+// sums meet: 4096 -> 4096 in 8 6.1).
 //
 // Included by qlinear.hip after qgemm128.h.
 #pragma once
 
 namespace {
 
-constexpr uint32_t few_out_base(bool int4, int cw) {
-  return int4 ? 65536u / (uint32_t)cw : kBigLutBase + (uint32_t)kBigLutBytes;
-}
-constexpr size_t few_smem_bytes(bool int4, int cw) {
-  return few_out_base(int4, cw) + 16 * kRowsActBytes;
-}
+// LDS: the activations of a work-group's k-tiles lie in slots of ROWS * 256 bytes from address 0 on, around the table of the code book (64 KiB to
+// 128 KiB; integer codes have none).  Behind the loop the sums of gated columns meet at 128 KiB, the activated tile leaves through the table's place.
+constexpr uint32_t kFewLds = 160u << 10, kFewMeet = 0x20000, kFewOut = 0x10000;
 
-template <int SPT, bool INT4, int CW>
+template <int SPT, bool INT4, int ROWS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void qgemm_few_kernel(const QLArgs a) {
-  constexpr int CT = 8 / CW, KW = 8 / CW, NT = 2;
-  constexpr int UC = CT < 4 ? CT : 4, UH = CT / UC;   // column tiles per unit of conversion, units per k-step
-  constexpr int PF = CW == 4 ? 4 : 3;          // k-tiles in flight
+  constexpr int MT = (ROWS + 15) / 16;
+  constexpr uint32_t SLOT = ROWS * 256;
+  constexpr int SLOTS = (int)((kFewLds - (INT4 ? 0u : (uint32_t)kBigLutBytes)) / SLOT);
+  constexpr int PF = 4;                        // k-tiles in flight: a turn of the ring
+  constexpr int TURNS = SLOTS >= 24 ? 2 : 1, CHUNK = TURNS * PF;   // turns, k-tiles whose slots are filled again together
+  constexpr int NB = SLOTS / CHUNK;            // chunks that LDS holds
+  static_assert(NB >= 2 && NB * CHUNK == SLOTS && 8 * MT * 1024 <= kFewLds - kFewMeet, "LDS");
   constexpr int SW = SPT / 2;                  // dwords of scales per column and k-tile
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), ch = wv % CW, ks = wv / CW;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lq = lane >> 4;
   // the whole argument block in one batch of scalar loads (left alone, each field is one memory round trip next to its first use)
   asm volatile("" ::"s"(a.M), "s"(a.K), "s"(a.N), "s"(a.x), "s"(a.codes), "s"(a.scales), "s"(a.ktiles_per_split), "s"(a.lora_rank),
@@ -47,184 +61,192 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int64_t ntiles = a.N / 16;
   const int ktiles = (int)(a.K / KTILE);
   const int kt_begin = blockIdx.z * a.ktiles_per_split;
-  const int kt_end = min(ktiles, kt_begin + a.ktiles_per_split);
+  const int kt_end = min(ktiles, kt_begin + a.ktiles_per_split), n = max(kt_end - kt_begin, 0);
   const uint64_t ntk = (uint64_t)ntiles * ktiles;
-  const uint32_t xbytes = (uint32_t)a.M * (uint32_t)a.K * 2u;
 
   // Per-lane offsets (32 bit: the host checks the 4 GiB limits); the k-tile enters as the scalar offset of a load.  Rows past M
   // and column tiles past N start beyond the buffer and read zeros.
-  uint32_t coff[CT], soff[CT];
-  const uint32_t xoff = ((uint32_t)lm * (uint32_t)a.K + (uint32_t)lq * 8u) * 2u;
-#pragma unroll
-  for (int ct = 0; ct < CT; ++ct) {
-    const uint32_t tile0 = ((uint32_t)blockIdx.y * 8u + (uint32_t)(ch * CT + ct)) * (uint32_t)ktiles;
-    coff[ct] = tile0 * 1024u + (uint32_t)lane * 16u;
-    soff[ct] = (tile0 * 16u + (uint32_t)lm) * (uint32_t)(SPT * 2);
-  }
-  u32x4 rc[PF][CT], xf[PF][4];
-  uint32_t rs[PF][CT][SW];
-  // (a k-tile past the wave's last one is asked of an empty buffer: zeros, and no traffic)
+  const int64_t my_tile = (int64_t)blockIdx.y * 8 + wv;
+  const uint32_t tile0 = (uint32_t)my_tile * (uint32_t)ktiles;
+  const uint32_t coff = tile0 * 1024u + (uint32_t)lane * 16u, soff = (tile0 * 16u + (uint32_t)lm) * (uint32_t)(SPT * 2);
+  u32x4 rc[PF];
+  uint32_t rs[PF][SW];
+  // (a k-tile past the last one is asked of an empty buffer: zeros, and no traffic)
   auto load_w = [&](int d, int kt) {
     const bool live = kt < kt_end;
     const rsrc_t qc = make_rsrc(a.codes, live ? ntk * 1024 : 0);
     const rsrc_t qs = make_rsrc(a.scales, live ? ntk * 16 * SPT * 2 : 0);
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) rc[d][ct] = __builtin_amdgcn_raw_buffer_load_b128(qc, coff[ct], kt * 1024, kStreamOnce);
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      if constexpr (SW == 1) {
-        rs[d][ct][0] = __builtin_amdgcn_raw_buffer_load_b32(qs, soff[ct], kt * (16 * SPT * 2), 0);
-      } else {
-        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(qs, soff[ct], kt * (16 * SPT * 2), 0);
-        rs[d][ct][0] = v[0];
-        rs[d][ct][1] = v[1];
-      }
+    rc[d] = __builtin_amdgcn_raw_buffer_load_b128(qc, coff, kt * 1024, kStreamOnce);
+    if constexpr (SW == 1) {
+      rs[d][0] = __builtin_amdgcn_raw_buffer_load_b32(qs, soff, kt * (16 * SPT * 2), 0);
+    } else {
+      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(qs, soff, kt * (16 * SPT * 2), 0);
+      rs[d][0] = v[0];
+      rs[d][1] = v[1];
     }
   };
-  auto load_x = [&](int d, int j, int kt) {
-    const rsrc_t q = make_rsrc(a.x, kt < kt_end ? xbytes : 0);
-    xf[d][j] = __builtin_amdgcn_raw_buffer_load_b128(q, xoff + (uint32_t)(j * 64), kt * 256, 0);
+  // Activations go from memory straight into LDS, a wave's 64 lanes 1 KB = four rows of a k-tile: chunk p of row r is k-chunk p ^ (r % 16), so
+  // that the rows a fragment is read from hit different banks.
+  constexpr int QUADS = ROWS / 4;   // quads of rows per k-tile
+  const u32x4 rx = raw_rsrc(a.x, (uint64_t)a.M * a.K * 2);
+  const int quad = wv % QUADS, xrow = quad * 4 + (lane >> 4);
+  const uint32_t xvoff = ((uint32_t)xrow * (uint32_t)a.K + (uint32_t)((lane & 15) ^ (xrow & 15)) * 8u) * 2u;
+  // k-tiles first .. first + count of this work-group into the slots from `slot` on
+  auto request_x = [&](int first, int count, int slot) {
+    for (int i = wv / QUADS; i < count; i += 8 / QUADS) {
+      const uint32_t at = (uint32_t)(slot + i) * SLOT;
+      dma16((INT4 || at < kBigLutBase ? at : at + (uint32_t)kBigLutBytes) + (uint32_t)quad * 1024u, rx, xvoff, (kt_begin + first + i) * (KTILE * 2));
+    }
   };
-  const int kt0 = kt_begin + ks;
+  request_x(0, min(n, NB * CHUNK), 0);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int d = 0; d < PF; ++d) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) load_x(d, j, kt0 + d * KW);
-    load_w(d, kt0 + d * KW);
-  }
+  for (int d = 0; d < PF; ++d) load_w(d, kt_begin + d);
   __builtin_amdgcn_sched_barrier(0);
 
-  // the adapter segment of the two column tiles this wave finishes
-  const int wn = wv & 3;
-  const int64_t ntile0 = ((int64_t)blockIdx.y * 4 + wn) * NT;
-  int toff[NT] = {0, 0};
+  // the adapter segment of this wave's columns
+  int toff = 0;
   if (a.lora_rank > 0) {
     if (a.lora_nseg < 0) {   // interleaved gate / up pair: even tiles segment 0, odd tiles segment 1
-      toff[1] = a.lora_rank;
+      toff = (wv & 1) * a.lora_rank;
     } else {
       // (N < 2^31: the host checks the 4 GiB limits; opaque copies, or the selects are folded back into loads from the arguments)
       int e0 = (int)a.lora_seg_end[0], e1 = (int)a.lora_seg_end[1], e2 = (int)a.lora_seg_end[2];
       int t0 = a.lora_seg_toff[0], t1 = a.lora_seg_toff[1], t2 = a.lora_seg_toff[2], t3 = a.lora_seg_toff[3];
       asm volatile("" : "+s"(e0), "+s"(e1), "+s"(e2), "+s"(t0), "+s"(t1), "+s"(t2), "+s"(t3));
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int col = (int)min(ntile0 + nt, ntiles - 1) * 16;
-        int t = t0;
-        t = a.lora_nseg > 1 && col >= e0 ? t1 : t;
-        t = a.lora_nseg > 2 && col >= e1 ? t2 : t;
-        t = a.lora_nseg > 3 && col >= e2 ? t3 : t;
-        toff[nt] = t;
-      }
+      const int col = (int)min(my_tile, ntiles - 1) * 16;
+      toff = t0;
+      toff = a.lora_nseg > 1 && col >= e0 ? t1 : toff;
+      toff = a.lora_nseg > 2 && col >= e1 ? t2 : toff;
+      toff = a.lora_nseg > 3 && col >= e2 ? t3 : toff;
     }
   }
-  // the adapter's fragments for the rows and columns this wave finishes: asked for here, needed last
-  const bool has_rows = wv < 4;
-  const bool lora = a.lora_rank > 0 && blockIdx.z == 0 && has_rows, lora_fast = lora && a.lora_rank <= 64;
-  u32x4 lb[NT][2], tf[NT][2];
+  if constexpr (!INT4) fill_level_table<512>(kBigLutBase, tid);   // while the first loads are in flight
+  __builtin_amdgcn_sched_barrier(0);
+  tnx_wait_vm(PF * 2);   // the activations, requested ahead of the ring's weights
+  __syncthreads();
+  // the adapter's fragments of this wave's columns, and those of the next linear's adapter: asked for here, needed last
+  const bool lora = a.lora_rank > 0 && blockIdx.z == 0, lora_fast = lora && a.lora_rank <= 64;
+  u32x4 lb[2], tf[MT][2], bn[2];
   if (lora_fast) {
     const rsrc_t rb = make_rsrc(a.lora_b, (uint64_t)a.N * a.lora_rank * 2), rt = make_rsrc(a.t, (uint64_t)a.M * a.t_ld * 2);
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int j = 0; j < 2; ++j) {
+      const bool on = j * 32 < a.lora_rank;
+      const uint32_t ko = (uint32_t)(j * 32 + lq * 8);
+      lb[j] = buf_load128(rb, on ? (((uint32_t)my_tile * 16u + (uint32_t)lm) * (uint32_t)a.lora_rank + ko) * 2u : 0xfffffff0u);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const bool on = j * 32 < a.lora_rank;
-        const uint32_t ko = (uint32_t)(j * 32 + lq * 8);
-        lb[nt][j] = buf_load128(rb, on ? (((uint32_t)(ntile0 + nt) * 16u + (uint32_t)lm) * (uint32_t)a.lora_rank + ko) * 2u : 0xfffffff0u);
-        tf[nt][j] = buf_load128(rt, on ? ((uint32_t)lm * (uint32_t)a.t_ld + (uint32_t)toff[nt] + ko) * 2u : 0xfffffff0u);
-      }
-  }
-  if constexpr (!INT4) {
-    fill_level_table<512>(kBigLutBase, tid);   // while the first loads are in flight
-    __syncthreads();
-  }
-
-  f32x4 acc[CT];
-#pragma unroll
-  for (int ct = 0; ct < CT; ++ct) zero_acc(acc[ct]);
-  // one k-tile of ring stage d = four k-steps: the look-ups of the next step are issued before this step's codes are converted
-  auto tile = [&](auto Dc, int kt) {
-    constexpr int d = decltype(Dc)::value;
-    uint32_t lp[2][UC][4];
-    auto look = [&](int u) {
-#pragma unroll
-      for (int c = 0; c < UC; ++c)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t w = rc[d][u % UH * UC + c][u / UH];
-          if constexpr (INT4) lp[u & 1][c][i] = int4_entry(magic, w, i);
-          else lp[u & 1][c][i] = lds_ld32(__builtin_amdgcn_perm(w, lane_off, 0x0c020400u + ((uint32_t)i << 8)));
-        }
-    };
-    look(0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < 4 * UH; ++u) {
-      const int j = u / UH;
-      if (u + 1 < 4 * UH) look(u + 1);
-#pragma unroll
-      for (int c = 0; c < UC; ++c) {
-        const int ct = u % UH * UC + c;
-        const uint32_t sw = rs[d][ct][SPT == 2 ? 0 : j >> 1];
-        const float s = (SPT == 2 ? j >> 1 : j & 1) ? bfhi(sw) : bflo(sw);
-        u32x4 w;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          _Float16 l0, l1;
-          level_pair<INT4>(lp[u & 1][c], b, l0, l1);
-          w[b] = cvt_pk_bf16(__builtin_fmaf((float)l0, s, 0.0f), __builtin_fmaf((float)l1, s, 0.0f));
-        }
-        acc[ct] = mfma16(xf[d][j], w, acc[ct]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      if (u % UH == UH - 1) load_x(d, j, kt + PF * KW);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int m = 0; m < MT; ++m)
+        tf[m][j] = buf_load128(rt, on ? ((uint32_t)(m * 16 + lm) * (uint32_t)a.t_ld + (uint32_t)toff + ko) * 2u : 0xfffffff0u);
     }
-    load_w(d, kt + PF * KW);
-    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (MT == 1 && a.next_tpart && wv < 4) {
+    const rsrc_t rn = make_rsrc(a.next_a_t, (uint64_t)a.next_rank * a.N);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bn[j] = buf_load128(rn, next_a_off(a, wv, j, lm, lq));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  f32x4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) zero_acc(acc[m]);
+  // LDS address of this lane's activation fragment of k-step 0 in a slot; k-step j lies 64 j bytes away under XOR, row tile m 4096 m bytes on.
+  // (Rows past the slot's read others: what they give stays in rows past M.)
+  const uint32_t xrd = (uint32_t)(lm % ROWS) * 256u + (uint32_t)(lq ^ (lm % ROWS)) * 16u;
+  // Entries of the code dwords (four code bytes: eight weights of a column, one k-step) are looked up kAhead dwords before the dword is
+  // converted, one at a time between the conversions: the LDS pipe takes an entry in two cycles and gets one of every wave in some
+  // sixteen; the counter of LDS accesses tells fifteen apart.
+  constexpr int kAhead = 3;
+  uint32_t lp[kAhead + 1][4];
+  u32x4 xf[2][MT];
+  auto entry_addr = [&](uint32_t w, int i) -> uint32_t { return INT4 ? 0u : __builtin_amdgcn_perm(w, lane_off, 0x0c020400u + ((uint32_t)i << 8)); };
+  auto entry = [&](uint32_t w, uint32_t at, int i) -> uint32_t {
+    if constexpr (INT4) return int4_entry(magic, w, i);
+    else return lds_ld32(at);
   };
-  // whole turns of the ring without a branch inside (behind one, the compiler's counted waits would assume that its loads never
-  // happened), then the tiles left
-  int kt = kt0;
-  for (; kt + (PF - 1) * KW < kt_end; kt += PF * KW) {
-    tile(ic<0>{}, kt);
-    tile(ic<1>{}, kt + KW);
-    tile(ic<2>{}, kt + 2 * KW);
-    if constexpr (PF > 3) tile(ic<(PF > 3 ? 3 : 0)>{}, kt + 3 * KW);
-  }
-  if (kt < kt_end) {
-    tile(ic<0>{}, kt);
-    if (kt + KW < kt_end) {
-      tile(ic<1>{}, kt + KW);
-      if (PF > 3 && kt + 2 * KW < kt_end) tile(ic<2>{}, kt + 2 * KW);
-    }
-  }
-
-  // The four k slices of a column meet: every wave leaves its sums, then takes the tiles it finishes from the four waves that hold
-  // a share of them.
+  auto read_x = [&](u32x4 (&to)[MT], uint32_t slot, int j) {
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) lds_st128((uint32_t)(wv * CT + ct) * 1024u + (uint32_t)lane * 16u, __builtin_bit_cast(u32x4, acc[ct]));
-  __syncthreads();
-  f32x4 out[1][NT];
+    for (int m = 0; m < MT; ++m) to[m] = lds_ld128(((xrd + slot) ^ (uint32_t)(j * 64)) + (uint32_t)(m * 4096));
+  };
+  int kt = kt_begin;
+  uint32_t here = 0;   // LDS address of the k-tile's slot
+  auto tile = [&](auto Dc) {   // one k-tile, of ring stage d
+    constexpr int d = decltype(Dc)::value, dn = (d + 1) % PF;
+    uint32_t next = here + SLOT;
+    if (!INT4) next = next == kBigLutBase ? kBigLutBase + (uint32_t)kBigLutBytes : next;
+    next = next == (uint32_t)(NB * CHUNK) * SLOT + (INT4 ? 0u : (uint32_t)kBigLutBytes) ? 0 : next;
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) zero_acc(out[0][nt]);
-  if (has_rows) {
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t ahead = j + kAhead < 4 ? rc[d][(j + kAhead) & 3] : rc[dn][(j + kAhead) & 3];
+      const uint32_t sw = rs[d][SPT == 2 ? 0 : j >> 1];
+      const float s = (SPT == 2 ? j >> 1 : j & 1) ? bfhi(sw) : bflo(sw);
+      uint32_t (&now)[4] = lp[(j + 4 * d) % (kAhead + 1)], (&later)[4] = lp[(j + 4 * d + kAhead) % (kAhead + 1)];
+      u32x4 q;
+      // two pairs at a time, an instruction between each and what needs its result
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int k = 0; k < KW; ++k) {
-        const uint32_t from = (uint32_t)((CW * k + 2 * wn / CT) * CT + (2 * wn) % CT + nt);
-        out[0][nt] += __builtin_bit_cast(f32x4, lds_ld128(from * 1024u + (uint32_t)lane * 16u));
+      for (int b = 0; b < 4; b += 2) {
+        const uint32_t at0 = entry_addr(ahead, b), at1 = entry_addr(ahead, b + 1);
+        _Float16 l0, l1, h0, h1;
+        level_pair<INT4>(now, b, l0, l1);
+        level_pair<INT4>(now, b + 1, h0, h1);
+        __builtin_amdgcn_sched_barrier(0);
+        const float p0 = __builtin_fmaf((float)l0, s, 0.0f), p1 = __builtin_fmaf((float)l1, s, 0.0f);
+        later[b] = entry(ahead, at0, b);
+        __builtin_amdgcn_sched_barrier(0);
+        const float r0 = __builtin_fmaf((float)h0, s, 0.0f), r1 = __builtin_fmaf((float)h1, s, 0.0f);
+        later[b + 1] = entry(ahead, at1, b + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b == 0) read_x(xf[(j + 1) & 1], j < 3 ? here : next, (j + 1) & 3);
+        q[b] = cvt_pk_bf16(p0, p1);
+        q[b + 1] = cvt_pk_bf16(r0, r1);
+        __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[m] = mfma16(xf[j & 1][m], q, acc[m]);
+    }
+    here = next;
+  };
+  static_assert(PF * 4 % (kAhead + 1) == 0, "a turn of the ring is whole turns of the look-ups");
+  auto turn = [&](auto self, auto Dc) -> void {
+    constexpr int d = decltype(Dc)::value;
+    if constexpr (d < PF) {
+      if (kt < kt_end) tile(Dc);   // (its loads, unconditional, stand behind it: the compiler's counted waits stay exact)
+      load_w(d, kt + PF);
+      __builtin_amdgcn_sched_barrier(0);
+      ++kt;
+      self(self, ic<d + 1>{});
+    }
+  };
+  read_x(xf[0], 0, 0);
+#pragma unroll
+  for (int w = 0; w < kAhead; ++w)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) lp[w][b] = entry(rc[0][w], entry_addr(rc[0][w], b), b);
+  __builtin_amdgcn_sched_barrier(0);
+  // Where LDS does not hold the activations of all k-tiles, the end of chunk c frees its slots for those of chunk c + NB, which have NB - 1 chunks
+  // to arrive in: the loads of those are the ones that may still be in flight at the wait.
+  for (int c = 0, into = 0; kt < kt_end; ++c) {
+#pragma unroll 1
+    for (int t = 0; t < TURNS; ++t) turn(turn, ic<0>{});
+    const int left = n - (c + NB) * CHUNK;   // k-tiles behind the chunks that are there
+    if (n > NB * CHUNK && (left > 0 || c + 1 >= NB)) {
+      constexpr int kYounger = (NB - 1) * CHUNK * 2;
+      tnx_wait_vm(kYounger < 60 ? kYounger : 60);
+      __syncthreads();
+      if (left > 0) request_x((c + NB) * CHUNK, min(CHUNK, left), into);
+      into = into + CHUNK == NB * CHUNK ? 0 : into + CHUNK;
+      read_x(xf[0], here, 0);   // (what the chunk before read may not have been there)
+    }
   }
   if (lora_fast) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
+    for (int m = 0; m < MT; ++m) {
       f32x4 part;
       zero_acc(part);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) part = mfma16(tf[nt][j], lb[nt][j], part);
+      for (int j = 0; j < 2; ++j) part = mfma16(tf[m][j], lb[j], part);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) out[0][nt][i] += a.lora_scale * part[i];
+      for (int i = 0; i < 4; ++i) acc[m][i] += a.lora_scale * part[i];
     }
   } else if (lora) {
     TileSrc s;
@@ -232,9 +254,37 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     s.w_bf16 = nullptr; s.codes = a.codes; s.scales = a.scales; s.group = a.group; s.qtype = a.qtype;
     s.ntiles = ntiles; s.lora_rank = a.lora_rank; s.t = a.t; s.t_ld = a.t_ld; s.lora_b = a.lora_b;
     s.lora_scale = a.lora_scale;
-    tile_lora<1, NT>(s, 0, ntile0, toff, out);
+    f32x4 out[MT][1];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) out[m][0] = acc[m];
+    const int toffs[1] = {toff};
+    tile_lora<MT, 1>(s, 0, my_tile, toffs, out);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = out[m][0];
   }
-  quant_rows_out<1, NT, false>(a, out, 0, ntile0, wv, few_out_base(INT4, CW), 0u);
+  const bool mul = a.epilogue == TNX_EPI_SILU_MUL || a.epilogue == TNX_EPI_GELU_MUL;
+  if (!mul || a.split_k > 1) {
+    // The planes of a split are stored as they lie in the accumulators and without the non-temporal policy: with it the pass that sums them waits
+    // longer than this one gains (14336 -> 4096 in 8 splits, 8 rows, with that pass: 16.1 us against 17.0, 4096 -> 4096 in 8: 11.6 against 12.5).
+    f32x4 out[MT][1];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) out[m][0] = acc[m];
+    store_tile<MT, 1>(a, 0, a.M, my_tile, ntiles, out, [](int64_t r) { return r; });
+    return;
+  }
+  // Gate and up columns meet: every wave leaves its sums and takes the two column tiles and the row tile it finishes.
+  __syncthreads();   // (activations and table lie there)
+#pragma unroll
+  for (int m = 0; m < MT; ++m) lds_st128(kFewMeet + (uint32_t)(wv * MT + m) * 1024u + (uint32_t)lane * 16u, __builtin_bit_cast(u32x4, acc[m]));
+  __syncthreads();
+  const int wn = wv & 3, rt = wv >> 2;
+  f32x4 out[1][2];
+  if (rt < MT) {
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+      out[0][nt] = __builtin_bit_cast(f32x4, lds_ld128(kFewMeet + (uint32_t)((2 * wn + nt) * MT + rt) * 1024u + (uint32_t)lane * 16u));
+  }
+  quant_rows_out<MT, 2, false, (MT == 1)>(a, out, 0, (int64_t)blockIdx.y * 8 + 2 * wn, wv, kFewOut, 0u, bn);
 }
 
 }  // namespace

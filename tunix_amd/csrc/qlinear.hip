@@ -745,45 +745,20 @@ int launch_qgemm128(hipStream_t st, const QLArgs& a) {
   return a.qtype == TNX_Q_INT4 ? launch_qgemm128_as<NT, SPT, MT, true>(st, a) : launch_qgemm128_as<NT, SPT, MT, false>(st, a);
 }
 
-template <int SPT, bool INT4, int CW>
+template <int SPT, bool INT4, int ROWS>
 int launch_qgemm_few_as(hipStream_t st, const QLArgs& a) {
   static std::once_flag once;
   static int attr_rc = TNX_OK;
-  constexpr size_t kSmem = few_smem_bytes(INT4, CW);
-  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, CW>, kSmem); });
+  constexpr size_t kSmem = kFewLds;
+  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, ROWS>, kSmem); });
   if (attr_rc) return attr_rc;
-  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, CW>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kSmem, st, a);
+  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, ROWS>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kSmem, st, a);
   TNX_CHECK_LAUNCH("qgemm_few");
   return TNX_OK;
 }
-template <int SPT, int CW>
+template <int SPT, int ROWS>
 int launch_qgemm_few(hipStream_t st, const QLArgs& a) {
-  return a.qtype == TNX_Q_INT4 ? launch_qgemm_few_as<SPT, true, CW>(st, a) : launch_qgemm_few_as<SPT, false, CW>(st, a);
-}
-
-// Calls whose activations come straight from memory (qgemm_few.h) instead of through LDS.  A wave's k-tiles have to be many enough for its
-// stream to run, more of them the more rows there are, whose fragments are fetched 16 bytes a lane; fewer k-tiles do where the sum over
-// the splits follows or the work-groups fill the device.  us, through LDS | from memory, weights from HBM, NF4 of group 64 with an adapter of
-// rank 64, splits with the pass that sums them (int4: the same within 3 %, groups of 32, whose scales take twice the loads, up to 6 % less
-// gain):             1 row          4 rows         8 rows         16 rows
-//   4 k-tiles     5.9 |  6.3     6.1 |  6.6     6.1 |  6.8     6.1 |  7.1   512 -> 3072 gated
-//   4 per split  11.1 | 10.8    11.5 | 11.4    11.7 | 11.7    11.9 | 12.3   4096 -> 4096 in 8
-//   7 per split  12.2 | 11.1    12.7 | 11.7    13.0 | 12.1    13.3 | 13.4   4096 -> 6144 in 5
-//   8             9.7 |  9.2     9.7 |  9.3     9.7 |  9.6     9.8 | 10.2   1024 -> 28672 (224 work-groups)
-//   9             9.0 |  8.7     8.9 |  8.9     9.0 |  9.3     9.0 | 10.2   1152 -> 13824 gated (108)
-//   14 per split 17.4 | 15.5    17.3 | 15.7    17.3 | 16.1    17.5 | 17.2   14336 -> 4096 in 8
-//   16           11.8 | 10.9    12.3 | 11.7    12.3 | 12.2    12.3 | 13.1   2048 -> 4096 (32)
-//   16           13.3 | 11.3    13.3 | 11.6    13.3 | 12.0    13.3 | 13.0   2048 -> 12288 gated (96)
-//   40           30.4 | 24.9    29.7 | 24.8    28.4 | 25.8    28.5 | 25.4   5120 -> 27648 gated
-// One row of int4, whose conversion needs no table to be filled first, is faster from memory from four k-tiles on (512 -> 3072 gated 5.7 | 5.3).
-bool few_shape(const QLArgs& a, bool two_scales) {
-  const int kt = a.ktiles_per_split;
-  const bool split = a.split_k > 1;
-  const int64_t groups = cdiv(a.N, 128) * a.split_k;
-  if (a.M == 1 && a.qtype == TNX_Q_INT4 && two_scales) return kt >= 4;
-  if (a.M <= 4) return kt >= (split ? 7 : groups >= 200 ? 8 : two_scales ? 9 : 10);
-  if (a.M <= 8) return split ? kt >= 10 || (kt >= 7 && groups >= 160) : (kt >= 8 && groups >= 200) || (kt >= 16 && (two_scales || groups >= 64));
-  return a.M <= 16 && (split ? kt >= 14 : (kt >= 16 && groups >= 96) || (kt >= 18 && groups >= 64));
+  return a.qtype == TNX_Q_INT4 ? launch_qgemm_few_as<SPT, true, ROWS>(st, a) : launch_qgemm_few_as<SPT, false, ROWS>(st, a);
 }
 
 template <int SPT, int MODE>
@@ -1109,19 +1084,15 @@ extern "C" int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* d) {
   if (rc) return rc;
   const QLArgs a = to_args(d);
   hipStream_t st = as_stream(stream);
-  // One kernel for every row count: 128 x 128 work-group tiles at 65+ rows, 16 / 32 / 64 rows for
-  // decode batches that small (the weight stream and its dequantisation are the same; MFMA,
-  // fragment and activation work shrink with the rows).  The 256-column variant (NT = 4) is not
+  // 128 x 128 work-group tiles at 65+ rows, 64 x 128 below, and up to 32 rows, where what a call waits for is not the matrix pipe, a kernel
+  // of its own (qgemm_few.h has both sides).  The 256-column variant of qgemm128_kernel (NT = 4) is not
   // dispatched: its accumulators need AGPRs, and the compiler wraps loops over AGPR accumulators
   // in register copies that cost more than the halved LDS traffic gains.
   const bool s2 = scales_per_tile(a.group) == 2;
   if (wide_shape(a)) return s2 ? launch_qgemm_wide<2>(st, a) : launch_qgemm_wide<4>(st, a);
-  if (few_shape(a, s2)) {
-    if (a.M <= 8) return s2 ? launch_qgemm_few<2, 4>(st, a) : launch_qgemm_few<4, 4>(st, a);
-    return s2 ? launch_qgemm_few<2, 2>(st, a) : launch_qgemm_few<4, 2>(st, a);
-  }
-  if (a.M <= 16) return s2 ? launch_qgemm128<2, 2, 1>(st, a) : launch_qgemm128<2, 4, 1>(st, a);
-  if (a.M <= 32) return s2 ? launch_qgemm128<2, 2, 2>(st, a) : launch_qgemm128<2, 4, 2>(st, a);
+  if (a.M <= 8) return s2 ? launch_qgemm_few<2, 8>(st, a) : launch_qgemm_few<4, 8>(st, a);
+  if (a.M <= 16) return s2 ? launch_qgemm_few<2, 16>(st, a) : launch_qgemm_few<4, 16>(st, a);
+  if (a.M <= 32) return s2 ? launch_qgemm_few<2, 32>(st, a) : launch_qgemm_few<4, 32>(st, a);
   if (a.M <= 64) return s2 ? launch_qgemm128<2, 2, 4>(st, a) : launch_qgemm128<2, 4, 4>(st, a);
   return s2 ? launch_qgemm128<2, 2, 8>(st, a) : launch_qgemm128<2, 4, 8>(st, a);
 }
