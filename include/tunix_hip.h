@@ -81,9 +81,10 @@ const char* tnx_last_error(void);
  * chunks to tnx_sink_attn_desc, an ungated form and shared weights to tnx_gated_norm_desc, TNX_EPI_RELU2, and
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
  * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora,
- * tnx_gqa_attn_lora, tnx_rope_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric. */
+ * tnx_gqa_attn_lora, tnx_rope_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric; 6.4 adds tnx_qlinear_inner and
+ * tnx_qlinear_inner_rows. */
 #define TNX_ABI_VERSION_MAJOR 6
-#define TNX_ABI_VERSION_MINOR 3
+#define TNX_ABI_VERSION_MINOR 4
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
 int tnx_version(void);
 
@@ -188,6 +189,11 @@ typedef struct tnx_qlinear_desc {
 } tnx_qlinear_desc;
 
 int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* h_desc);
+/* The same over at most tnx_qlinear_inner_rows(K, N, lora_rank) rows (0: a shape it does not take), with the adapter's down-projection formed inside:
+ * desc's t is not read (tnx_splitk_finish wants one all the same), one adapter segment, no *_MUL epilogue.  t is not rounded to bf16 on the way.  a_frag: A in the order it is multiplied in,
+ * bf16 [K / 32][lora_rank / 16][4][16][8]: element (g, n, q, c, i) is A[32 g + 8 q + i][16 n + c].                                      */
+int tnx_qlinear_inner(void* stream, const tnx_qlinear_desc* h_desc, const uint16_t* a_frag);
+int64_t tnx_qlinear_inner_rows(int64_t K, int64_t N, int lora_rank);
 /* Epilogue for split_k > 1 (same desc): y = epi(sum_z ws[z]). */
 int tnx_splitk_finish(void* stream, const tnx_qlinear_desc* h_desc);
 

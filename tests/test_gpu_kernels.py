@@ -332,6 +332,65 @@ def test_few_rows_at_the_edges_of_what_lds_holds(gpu, M, K, N, split, group, qty
     assert_bf16_close(y, y64.float().bfloat16(), what="linear", atol=off)
 
 
+@pytest.mark.parametrize("M,K,N,split,group,qtype,rank,epi", [
+    (1, 128, 16, 1, 64, Q.INT4, 32, "store"),        # one k-tile, one column tile, half of the ranks
+    (8, 1024, 1152, 8, 128, Q.INT4, 64, "store"),    # one k-tile per split
+    (5, 1152, 272, 5, 32, Q.NF4, 64, "store"),       # two per split, one in the last; a last block of one column tile
+    (9, 512, 256, 1, 64, Q.NF4, 64, "residual"),     # four, unsplit
+    (16, 1920, 384, 3, 64, Q.NF4, 32, "store"),      # five per split: past the form for few
+    (13, 4224, 128, 1, 64, Q.NF4, 64, "f32"),        # 33: slots are filled again
+    (17, 384, 128, 1, 128, Q.INT4, 64, "store"),     # two row tiles, three k-tiles
+    (32, 2176, 256, 1, 32, Q.NF4, 64, "residual"),   # 17 of 32 rows: slots are filled again
+])
+def test_few_rows_form_the_adapters_down_projection(gpu, M, K, N, split, group, qtype, rank, epi):
+  """y = x . W + 1.5 (x . A) . B with x . A formed inside, against 64 bits: x . A is a pair of bf16, 2^-17 of itself off, so the result is the
+  rounded one but for near ties (`off`: the fp32 sums, as above, and those 2^-17 of the adapter's share)."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  x, w, res = bf(rnd((M, K), 411)).to(gpu), bf(rnd((K, N), 412, 0.03)).to(gpu), bf(rnd((M, N), 413)).to(gpu)
+  a_t, lb = bf(rnd((rank, K), 414, 0.03)).to(gpu), bf(rnd((N, rank), 415, 0.1)).to(gpu)
+  c, s = ops.quantize_pack(w, group, qtype)
+  share = 1.5 * (x.double() @ a_t.double().T) @ lb.double().T
+  ref = x.double() @ ops.qw_dequant(c, s, K, N, group, qtype).double() + share
+  off = 2.0 ** -23 * 0.03 * K + 2.0 ** -17 * share.abs().max().item()
+  y = torch.full((M, N), 7.0, dtype=torch.float32 if epi == "f32" else torch.bfloat16, device=gpu)
+  ws = torch.full((split * M * N,), float("nan"), device=gpu) if split > 1 else None
+  t = torch.full((M, rank), float("nan"), dtype=torch.bfloat16, device=gpu)   # (not read)
+  d = ops.make_qlinear_desc(M=M, K=K, N=N, group=group, qtype=qtype, x=x, codes=c, scales=s, y=y, split_k=split, ws=ws, lora_rank=rank, lora_nseg=1,
+                            lora_seg_end=[N], lora_seg_toff=[0], t=t, t_ld=rank, lora_b=lb, lora_scale=1.5, residual=res if epi == "residual" else None,
+                            epilogue={"store": L.TNX_EPI_STORE, "residual": L.TNX_EPI_RESIDUAL, "f32": L.TNX_EPI_F32}[epi])
+  assert ops.qlinear_inner_rows(K, N, rank) >= M
+  ops.qlinear(d, a_frag=ops.lora_frag(a_t))
+  torch.cuda.synchronize()
+  if epi == "f32":
+    assert (y.double() - ref).abs().max().item() <= off
+  elif epi == "residual":
+    ref = ref.float().bfloat16()
+    assert_bf16_close(y, (ref.float() + res.float()).bfloat16(), what=epi, atol=off, mag=torch.maximum(ref.float().abs(), res.float().abs()))
+  else:
+    assert_bf16_close(y, ref.float().bfloat16(), what=epi, atol=off)
+
+
+def test_adapter_inside_refuses_other_shapes(gpu):
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  assert ops.qlinear_inner_rows(512, 256, 96) == 0 and ops.qlinear_inner_rows(500, 256, 64) == 0 and ops.qlinear_inner_rows(512, 256, 64) == 32
+  w = bf(rnd((512, 256), 421, 0.03)).to(gpu)
+  c, s = ops.quantize_pack(w, 64, Q.NF4)
+  a_t, lb = bf(rnd((64, 512), 422)).to(gpu), bf(rnd((256, 64), 423)).to(gpu)
+
+  def call(M=4, rank=64, nseg=1, epi=L.TNX_EPI_STORE):
+    x, y = bf(rnd((M, 512), 424)).to(gpu), torch.empty(M, 256, dtype=torch.bfloat16, device=gpu)
+    ops.qlinear(ops.make_qlinear_desc(M=M, K=512, N=256, group=64, qtype=Q.NF4, x=x, codes=c, scales=s, y=y, lora_rank=rank, lora_nseg=nseg,
+                                      lora_seg_end=[128, 256][-abs(nseg):], lora_seg_toff=[0, 64][:abs(nseg)], lora_b=lb, lora_scale=1.0, epilogue=epi),
+                a_frag=ops.lora_frag(a_t))
+
+  call()
+  for bad in (dict(M=33), dict(rank=96), dict(rank=0), dict(nseg=2), dict(nseg=-1, epi=L.TNX_EPI_SILU_MUL)):
+    with pytest.raises(ValueError):
+      call(**bad)
+
+
 @pytest.mark.parametrize("rows,copy,split", [(65536, False, 1), (65536, True, 1), (100, False, 1), (100, False, 2), (16, False, 1)])
 def test_silu_of_every_gate(gpu, rows, copy, split):
   """Gates of every finite bf16 value (weights that pick one element of x), among them those whose sigmoid is not a normal fp32

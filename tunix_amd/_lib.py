@@ -12,7 +12,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtunix_hip.so")
 
 # the ABI this binding was written against (TNX_ABI_VERSION_MAJOR / _MINOR of include/tunix_hip.h)
-ABI_VERSION = (6, 3)
+ABI_VERSION = (6, 4)
 
 TNX_Q_INT4, TNX_Q_NF4 = 0, 1
 TNX_NORM_LLAMA, TNX_NORM_QWEN3, TNX_NORM_GEMMA3 = 0, 1, 2
@@ -324,6 +324,8 @@ SIGNATURES = {
     "tnx_moe_route_topk": (_i32, [_p, _p, _i64, _i32, _i32, _p, _p]),
     "tnx_moe_sort_routes": (_i32, [_p, _p, _i64, _i32, _i32, _p, _p, _p]),
     "tnx_moe_int4_gmm": (_i32, [_p, C.POINTER(MoeGmmDesc)]),
+    "tnx_qlinear_inner": (_i32, [_p, C.POINTER(QLinearDesc), _p]),
+    "tnx_qlinear_inner_rows": (_i64, [_i64, _i64, _i32]),
     "tnx_moe_gmm_expanded": (_i32, [_p, C.POINTER(MoeGmmDesc), _p]),
     "tnx_moe_expanded_rows": (_i64, [_i64, _i64, _i32]),
     "tnx_moe_combine": (_i32, [_p, _p, _p, _i64, _i32, _i64, _p, _p]),

@@ -35,7 +35,17 @@ namespace {
 // 128 KiB; integer codes have none).  Behind the loop the sums of gated columns meet at 128 KiB, the activated tile leaves through the table's place.
 constexpr uint32_t kFewLds = 160u << 10, kFewMeet = 0x20000, kFewOut = 0x10000;
 
-template <int SPT, bool INT4, int ROWS>
+// INNER: the adapter's down-projection t = x . A is formed here (a.inner_a, its fragments in order) instead of ahead of the launch: a work-group
+// multiplies the activations it holds with its k range of A (wave (rank tile, half of each k-tile): the fragments of x are there already), and its share
+// of t, as a pair of bf16 (to 2^-17 of itself), with B: t is linear, so no sum over the splits has to be waited for, nor is one rounded to bf16 on the
+// way (against 64 bits 6e-7 of the result where a rounded t gave 4e-4).  us, down-projection and this kernel in two launches | in one, 16 rows, rank 64:
+// 4096 -> 4096 in 8 10.7 | 7.2, 14336 -> 4096 in 8 20.0 | 13.1, int4 1024 -> 1152 in 8 7.6 | 4.4, 2048 -> 4096 unsplit 13.8 | 12.9; 32 rows 11.9 | 8.2,
+// 22.5 | 15.8, 8.6 | 5.0, 16.4 | 15.0.  (The fragments of A are 16 KB a k-tile and work-group, from the L2, next to 9 of codes and scales: a pair of
+// adapters over a long unsplit range, gate | up's, would be a megabyte for each.)
+// SHORT: at most PF k-tiles per split, none of them asked for in vain.  (A load that is not needed still takes its turn in the memory pipe; with the
+// adapter's there are twice as many: 1024 -> 1152 in 8, one k-tile each, 5.8 -> 4.1 us with the adapter inside, 4096 -> 4096 in 8 7.7 -> 6.9; without
+// it the waits behind the branches cost as much as the loads, 1152 -> 1536 in 5 3.5 | 3.7.)
+template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void qgemm_few_kernel(const QLArgs a) {
   constexpr int MT = (ROWS + 15) / 16;
   constexpr uint32_t SLOT = ROWS * 256;
@@ -69,8 +79,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int64_t my_tile = (int64_t)blockIdx.y * 8 + wv;
   const uint32_t tile0 = (uint32_t)my_tile * (uint32_t)ktiles;
   const uint32_t coff = tile0 * 1024u + (uint32_t)lane * 16u, soff = (tile0 * 16u + (uint32_t)lm) * (uint32_t)(SPT * 2);
-  u32x4 rc[PF];
+  u32x4 rc[PF], ra[PF][2];
   uint32_t rs[PF][SW];
+  const int a_tile = wv & 3, a_half = wv >> 2, a_tiles = a.lora_rank / 16;
+  const uint32_t aoff = (uint32_t)(a_half * 2 * a_tiles + a_tile) * 1024u + (uint32_t)lane * 16u;
+  constexpr int LOADS = INNER ? 4 : 2;   // per k-tile and wave
   // (a k-tile past the last one is asked of an empty buffer: zeros, and no traffic)
   auto load_w = [&](int d, int kt) {
     const bool live = kt < kt_end;
@@ -83,6 +96,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(qs, soff, kt * (16 * SPT * 2), 0);
       rs[d][0] = v[0];
       rs[d][1] = v[1];
+    }
+    if constexpr (INNER) {
+      const rsrc_t qa = make_rsrc(a.inner_a, live && a_tile < a_tiles ? (uint64_t)a.K * a.lora_rank * 2 : 0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) ra[d][j] = __builtin_amdgcn_raw_buffer_load_b128(qa, aoff + (uint32_t)(j * a_tiles) * 1024u, kt * 4 * a_tiles * 1024, 0);
     }
   };
   // Activations go from memory straight into LDS, a wave's 64 lanes 1 KB = four rows of a k-tile: chunk p of row r is k-chunk p ^ (r % 16), so
@@ -101,7 +119,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   request_x(0, min(n, NB * CHUNK), 0);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int d = 0; d < PF; ++d) load_w(d, kt_begin + d);
+  for (int d = 0; d < PF; ++d)
+    if (!SHORT || d < n) load_w(d, kt_begin + d);
   __builtin_amdgcn_sched_barrier(0);
 
   // the adapter segment of this wave's columns
@@ -123,10 +142,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   if constexpr (!INT4) fill_level_table<512>(kBigLutBase, tid);   // while the first loads are in flight
   __builtin_amdgcn_sched_barrier(0);
-  tnx_wait_vm(PF * 2);   // the activations, requested ahead of the ring's weights
+  // the activations, requested ahead of the ring's weights
+  if (!SHORT || n >= 4) tnx_wait_vm(4 * LOADS);
+  else if (n == 3) tnx_wait_vm(3 * LOADS);
+  else if (n == 2) tnx_wait_vm(2 * LOADS);
+  else tnx_wait_vm(LOADS);
+  static_assert(PF == 4, "the waits above");
   __syncthreads();
   // the adapter's fragments of this wave's columns, and those of the next linear's adapter: asked for here, needed last
-  const bool lora = a.lora_rank > 0 && blockIdx.z == 0, lora_fast = lora && a.lora_rank <= 64;
+  const bool lora = a.lora_rank > 0 && (INNER || blockIdx.z == 0), lora_fast = lora && a.lora_rank <= 64;
   u32x4 lb[2], tf[MT][2], bn[2];
   if (lora_fast) {
     const rsrc_t rb = make_rsrc(a.lora_b, (uint64_t)a.N * a.lora_rank * 2), rt = make_rsrc(a.t, (uint64_t)a.M * a.t_ld * 2);
@@ -137,7 +161,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       lb[j] = buf_load128(rb, on ? (((uint32_t)my_tile * 16u + (uint32_t)lm) * (uint32_t)a.lora_rank + ko) * 2u : 0xfffffff0u);
 #pragma unroll
       for (int m = 0; m < MT; ++m)
-        tf[m][j] = buf_load128(rt, on ? ((uint32_t)(m * 16 + lm) * (uint32_t)a.t_ld + (uint32_t)toff + ko) * 2u : 0xfffffff0u);
+        if constexpr (!INNER) tf[m][j] = buf_load128(rt, on ? ((uint32_t)(m * 16 + lm) * (uint32_t)a.t_ld + (uint32_t)toff + ko) * 2u : 0xfffffff0u);
     }
   }
   if (MT == 1 && a.next_tpart && wv < 4) {
@@ -147,9 +171,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   __builtin_amdgcn_sched_barrier(0);
 
-  f32x4 acc[MT];
+  f32x4 acc[MT], tacc[MT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) zero_acc(acc[m]);
+  for (int m = 0; m < MT; ++m) {
+    zero_acc(acc[m]);
+    zero_acc(tacc[m]);
+  }
   // LDS address of this lane's activation fragment of k-step 0 in a slot; k-step j lies 64 j bytes away under XOR, row tile m 4096 m bytes on.
   // (Rows past the slot's read others: what they give stays in rows past M.)
   const uint32_t xrd = (uint32_t)(lm % ROWS) * 256u + (uint32_t)(lq ^ (lm % ROWS)) * 16u;
@@ -203,6 +230,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[m] = mfma16(xf[j & 1][m], q, acc[m]);
+      if (INNER && a_half == j >> 1)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) tacc[m] = mfma16(xf[j & 1][m], ra[d][j & 1], tacc[m]);
     }
     here = next;
   };
@@ -211,8 +241,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int d = decltype(Dc)::value;
     if constexpr (d < PF) {
       if (kt < kt_end) tile(Dc);   // (its loads, unconditional, stand behind it: the compiler's counted waits stay exact)
-      load_w(d, kt + PF);
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!SHORT) {
+        load_w(d, kt + PF);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       ++kt;
       self(self, ic<d + 1>{});
     }
@@ -225,12 +257,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   __builtin_amdgcn_sched_barrier(0);
   // Where LDS does not hold the activations of all k-tiles, the end of chunk c frees its slots for those of chunk c + NB, which have NB - 1 chunks
   // to arrive in: the loads of those are the ones that may still be in flight at the wait.
-  for (int c = 0, into = 0; kt < kt_end; ++c) {
+  if constexpr (SHORT) turn(turn, ic<0>{});
+  for (int c = 0, into = 0; !SHORT && kt < kt_end; ++c) {
 #pragma unroll 1
     for (int t = 0; t < TURNS; ++t) turn(turn, ic<0>{});
     const int left = n - (c + NB) * CHUNK;   // k-tiles behind the chunks that are there
     if (n > NB * CHUNK && (left > 0 || c + 1 >= NB)) {
-      constexpr int kYounger = (NB - 1) * CHUNK * 2;
+      constexpr int kYounger = (NB - 1) * CHUNK * LOADS;
       tnx_wait_vm(kYounger < 60 ? kYounger : 60);
       __syncthreads();
       if (left > 0) request_x((c + NB) * CHUNK, min(CHUNK, left), into);
@@ -238,7 +271,44 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       read_x(xf[0], here, 0);   // (what the chunk before read may not have been there)
     }
   }
-  if (lora_fast) {
+  if constexpr (INNER) {
+    // the shares of t meet as rows in LDS, padded by four ranks
+    constexpr uint32_t T_LD = 68 * 4, T_HALF = 16 * MT * T_LD;
+    static_assert(2 * T_HALF <= kFewLds - kFewMeet, "LDS");
+    if ((uint32_t)n * SLOT > (INT4 ? kFewMeet : kBigLutBase)) __syncthreads();   // (activations lie there)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = tacc[m][i];
+        *reinterpret_cast<lds_u32*>(static_cast<uintptr_t>(kFewMeet + (uint32_t)a_half * T_HALF + (uint32_t)(m * 16 + lq * 4 + i) * T_LD +
+                                                           (uint32_t)(a_tile * 16 + lm) * 4u)) = __float_as_uint(v);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      f32x4 part;
+      zero_acc(part);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {   // (ranks past the adapter's are zeros: nothing was asked for them, neither of A nor of B)
+        const uint32_t at = kFewMeet + (uint32_t)(m * 16 + lm) * T_LD + (uint32_t)(j * 32 + lq * 8) * 4u;
+        u32x4 hi, lo;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 v = __builtin_bit_cast(f32x4, lds_ld128(at + h * 16u)) + __builtin_bit_cast(f32x4, lds_ld128(at + T_HALF + h * 16u));
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            hi[2 * h + i] = cvt_pk_bf16(v[2 * i], v[2 * i + 1]);
+            lo[2 * h + i] = cvt_pk_bf16(v[2 * i] - bflo(hi[2 * h + i]), v[2 * i + 1] - bfhi(hi[2 * h + i]));
+          }
+        }
+        part = mfma16(lo, lb[j], part);
+        part = mfma16(hi, lb[j], part);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[m][i] += a.lora_scale * part[i];
+    }
+  } else if (lora_fast) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       f32x4 part;

@@ -45,6 +45,8 @@ struct QLArgs {
   const uint16_t* w_pre;
   // row stride of the stored output in elements, 0: the output's width (many-row kernel only)
   int64_t ldy;
+  // the adapter's A in fragment order (few-row kernel only)
+  const uint16_t* inner_a;
 };
 // gate | up with the activation and the product in fp32 and one rounding (dense-weight decoders;
 // many-row kernel only)
@@ -541,6 +543,7 @@ QLArgs to_args(const tnx_qlinear_desc* d) {
   a.next_a_t = d->next_a_t; a.next_rank = d->next_rank; a.next_tpart = d->next_tpart;
   a.w_pre = d->w_expanded;
   a.ldy = 0;
+  a.inner_a = nullptr;
   return a;
 }
 
@@ -745,20 +748,32 @@ int launch_qgemm128(hipStream_t st, const QLArgs& a) {
   return a.qtype == TNX_Q_INT4 ? launch_qgemm128_as<NT, SPT, MT, true>(st, a) : launch_qgemm128_as<NT, SPT, MT, false>(st, a);
 }
 
-template <int SPT, bool INT4, int ROWS>
+template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT>
 int launch_qgemm_few_as(hipStream_t st, const QLArgs& a) {
   static std::once_flag once;
   static int attr_rc = TNX_OK;
-  constexpr size_t kSmem = kFewLds;
-  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, ROWS>, kSmem); });
+  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT>, kFewLds); });
   if (attr_rc) return attr_rc;
-  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, ROWS>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kSmem, st, a);
+  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kFewLds, st, a);
   TNX_CHECK_LAUNCH("qgemm_few");
   return TNX_OK;
 }
-template <int SPT, int ROWS>
-int launch_qgemm_few(hipStream_t st, const QLArgs& a) {
-  return a.qtype == TNX_Q_INT4 ? launch_qgemm_few_as<SPT, true, ROWS>(st, a) : launch_qgemm_few_as<SPT, false, ROWS>(st, a);
+template <int SPT, int ROWS, bool INNER, bool SHORT>
+int launch_qgemm_few_book(hipStream_t st, const QLArgs& a) {
+  return a.qtype == TNX_Q_INT4 ? launch_qgemm_few_as<SPT, true, ROWS, INNER, SHORT>(st, a) : launch_qgemm_few_as<SPT, false, ROWS, INNER, SHORT>(st, a);
+}
+template <int SPT, int ROWS, bool INNER>
+int launch_qgemm_few_rows(hipStream_t st, const QLArgs& a) {
+  if constexpr (INNER)
+    if (a.ktiles_per_split <= 4) return launch_qgemm_few_book<SPT, ROWS, INNER, true>(st, a);
+  return launch_qgemm_few_book<SPT, ROWS, INNER, false>(st, a);
+}
+constexpr int64_t kFewRows = 32;
+template <bool INNER>
+int launch_qgemm_few(hipStream_t st, const QLArgs& a, bool two_scales) {
+  if (a.M <= 8) return two_scales ? launch_qgemm_few_rows<2, 8, INNER>(st, a) : launch_qgemm_few_rows<4, 8, INNER>(st, a);
+  if (a.M <= 16) return two_scales ? launch_qgemm_few_rows<2, 16, INNER>(st, a) : launch_qgemm_few_rows<4, 16, INNER>(st, a);
+  return two_scales ? launch_qgemm_few_rows<2, 32, INNER>(st, a) : launch_qgemm_few_rows<4, 32, INNER>(st, a);
 }
 
 template <int SPT, int MODE>
@@ -1090,11 +1105,29 @@ extern "C" int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* d) {
   // in register copies that cost more than the halved LDS traffic gains.
   const bool s2 = scales_per_tile(a.group) == 2;
   if (wide_shape(a)) return s2 ? launch_qgemm_wide<2>(st, a) : launch_qgemm_wide<4>(st, a);
-  if (a.M <= 8) return s2 ? launch_qgemm_few<2, 8>(st, a) : launch_qgemm_few<4, 8>(st, a);
-  if (a.M <= 16) return s2 ? launch_qgemm_few<2, 16>(st, a) : launch_qgemm_few<4, 16>(st, a);
-  if (a.M <= 32) return s2 ? launch_qgemm_few<2, 32>(st, a) : launch_qgemm_few<4, 32>(st, a);
+  if (a.M <= kFewRows) return launch_qgemm_few<false>(st, a, s2);
   if (a.M <= 64) return s2 ? launch_qgemm128<2, 2, 4>(st, a) : launch_qgemm128<2, 4, 4>(st, a);
   return s2 ? launch_qgemm128<2, 2, 8>(st, a) : launch_qgemm128<2, 4, 8>(st, a);
+}
+
+extern "C" int64_t tnx_qlinear_inner_rows(int64_t K, int64_t N, int lora_rank) {
+  return K > 0 && K % KTILE == 0 && N > 0 && N % 16 == 0 && (lora_rank == 32 || lora_rank == 64) ? kFewRows : 0;
+}
+
+extern "C" int tnx_qlinear_inner(void* stream, const tnx_qlinear_desc* d, const uint16_t* a_frag) {
+  TNX_REQUIRE(d != nullptr, "qlinear_inner: null descriptor");
+  tnx_qlinear_desc c = *d;
+  c.t = c.x;   // (not read)
+  c.t_ld = 8;
+  const int rc = check_desc(&c);
+  if (rc) return rc;
+  TNX_REQUIRE(d->lora_rank > 0 && d->M <= tnx_qlinear_inner_rows(d->K, d->N, d->lora_rank), "qlinear_inner: %lld rows, rank %d: not a shape it takes",
+              (long long)d->M, d->lora_rank);
+  TNX_REQUIRE(d->lora_nseg == 1 && d->epilogue != TNX_EPI_SILU_MUL && d->epilogue != TNX_EPI_GELU_MUL, "qlinear_inner: one adapter, no *_MUL epilogue");
+  TNX_REQUIRE(a_frag && ((uintptr_t)a_frag & 15) == 0, "qlinear_inner: the adapter's fragments must be there and 16-byte aligned");
+  QLArgs a = to_args(&c);
+  a.inner_a = a_frag;
+  return launch_qgemm_few<true>(as_stream(stream), a, scales_per_tile(a.group) == 2);
 }
 
 // The lm_head over many rows on the many-row kernels: per 128-column block statistics

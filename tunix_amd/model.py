@@ -52,6 +52,7 @@ class FusedLinear:
     self.load_base(weights)
     r = cfg.lora_rank
     self.has_lora = any((n + ".lora_a") in weights for n in names)
+    self.inner_rows = 0   # rows up to which the linear forms its adapter's down-projection itself
     self.rp = _pad32(r) if self.has_lora else 0
     self.r = r
     self.lora_scale = float(cfg.lora_alpha) / float(r) if self.has_lora else 0.0
@@ -64,6 +65,11 @@ class FusedLinear:
     if self.has_lora:
       self.a_t = torch.zeros(len(names) * self.rp, self.K, dtype=torch.bfloat16, device=device)
       self.b_t = torch.zeros(self.N, self.rp, dtype=torch.bfloat16, device=device)
+      # a single adapter's A once more, in the order that few rows multiply it in inside the linear
+      self.a_frag = None
+      self.inner_rows = ops.qlinear_inner_rows(self.K, self.N, self.rp) if len(names) == 1 else 0
+      if self.inner_rows:
+        self.a_frag = ops.lora_frag(self.a_t)
       self._row_perm = None
       if interleave2:
         c = torch.arange(self.N, device=device)
@@ -144,6 +150,8 @@ class FusedLinear:
         self.a_t[i * self.rp: i * self.rp + self.r].copy_(a.to(self.a_t.device, torch.bfloat16).t())
         b_full[off: off + wd, : self.r].copy_(b.to(self.b_t.device, torch.bfloat16).t())
       off += wd
+    if self.a_frag is not None:
+      self.a_frag.copy_(ops.lora_frag(self.a_t))
     if self._row_perm is not None:
       self.b_t[self._row_perm] = b_full
     else:
@@ -557,7 +565,9 @@ class Runner(HeadRunner):
     if kv_chunk is None:
       kv_chunk = 0
       if T == 1 and S > 64:
-        kv_chunk = math.ceil(S / self._key_chunks(B * cfg.num_kv_heads, S, cfg.head_dim) / 32) * 32
+        o = model.layers[0]["o"] if model.layers else None
+        behind = o is not None and o.has_lora and not self.inner(o, M)
+        kv_chunk = math.ceil(S / self._key_chunks(B * cfg.num_kv_heads, S, cfg.head_dim, behind) / 32) * 32
         if kv_chunk >= S:
           kv_chunk = 0
     self.kv_chunk = kv_chunk
@@ -567,12 +577,17 @@ class Runner(HeadRunner):
     self._init_head(B, D, bf, want_logits)
 
   @staticmethod
-  def _key_chunks(groups: int, S: int, head_dim: int) -> int:
-    """Chunks that a decode step's key range of `groups` (row, kv head) pairs is cut into."""
+  def _key_chunks(groups: int, S: int, head_dim: int, adapter_behind: bool = True) -> int:
+    """Chunks that a decode step's key range of `groups` (row, kv head) pairs is cut into.  adapter_behind: the pass that merges them forms the
+    o adapter's down-projection too, and so would have to run for one chunk."""
     # Only as far as needed to put one work-group of four waves on every compute unit, in chunks of at least a key block per wave or so.
     # Attention with its merging pass and the o adapter, us in 1 | 2 | 4 | 8 chunks or so: 8 kv heads of 128, 16 rows x 700 keys 20.2 | 16.9 | 19.0 | 20.4,
     # 1500 keys 32.8 | 24.7 | 25.8 | 27.6, 8 rows x 1000 24.2 | 18.0 | 15.5 | 17.1; one kv head of 256, 64 rows x 288 18.5 | 14.2 | 12.0 | 14.7,
     # 16 rows x 1200 48 | 30 | 21.7 | 15.7 (12 chunks 14.6).
+    # Without the adapter behind it one chunk saves the merging pass, us in 1 | 2 | 4 chunks: heads of 128, 1 row x 256 keys 6.3 | 8.1 | 8.1, 16 rows x 256 8.0 |
+    # 9.6 | 10.2, 8 rows x 384 9.7 | 9.8 | 9.2; heads of 64, 16 rows x 384 7.4 | 8.4 | 7.7, x 512 8.6 | 8.8 | 8.1; heads of 256, 16 rows x 256 12.2 | 10.7 | 10.3.
+    if not adapter_behind and S <= (384 if head_dim <= 64 else 256 if head_dim <= 128 else 0):
+      return 1
     if groups <= 128:
       return max(1, min(256 // groups, math.ceil(S / 128)))
     # More: two to a unit, of many keys, are cut in halves, which even out what the units have: 40 rows x 8 heads of 128 x 1280 52.6 | 44.2 (32 rows
@@ -637,7 +652,8 @@ class Runner(HeadRunner):
     returns split_k (> 1): the caller hands the partial planes in self.splitk_ws to the kernel
     that consumes them (`norm_after` for a RESIDUAL linear of model width, the rope / cache
     write for a plain STORE); otherwise returns 1 with y complete."""
-    if f.has_lora and not t_ready:
+    inner = self.inner(f, M) and not t_ready
+    if f.has_lora and not t_ready and not inner:
       ops.lora_down(x, f.a_t, self.t, M=M)
     split = self._split_k(f, M)
     # a gate|up linear can leave the down-projection of the next linear's adapter behind
@@ -659,11 +675,16 @@ class Runner(HeadRunner):
     deferred = defer and split > 1 and (
         epilogue == L.TNX_EPI_STORE
         or (epilogue == L.TNX_EPI_RESIDUAL and f.N == self.cfg.embed_dim and f.N % 8 == 0))
-    ops.qlinear(d, finish=not deferred)
+    ops.qlinear(d, finish=not deferred, a_frag=f.a_frag if inner else None)
     return split if deferred else 1
 
+  @staticmethod
+  def inner(f: FusedLinear, M: int) -> bool:
+    """Whether `linear` of M rows forms the adapter's down-projection of its input itself: then nothing ahead of it has to."""
+    return M <= f.inner_rows
+
   def fuses_next(self, f: FusedLinear, next_f: FusedLinear, M: int, epilogue: int) -> bool:
-    return (next_f.has_lora and next_f.rp <= 64 and M <= 1024 and self._split_k(f, M) == 1
+    return (next_f.has_lora and not self.inner(next_f, M) and next_f.rp <= 64 and M <= 1024 and self._split_k(f, M) == 1
             and epilogue in (L.TNX_EPI_SILU_MUL, L.TNX_EPI_GELU_MUL) and (f.N // 2) % 8 == 0
             and self.next_tpart is not None)
 
@@ -776,9 +797,10 @@ class Runner(HeadRunner):
         else:
           ad.qkv = self.qkv.data_ptr()
         ad.rope_sin, ad.rope_cos = self.rope_sin.data_ptr(), self.rope_cos.data_ptr()
+      o_ready = not self.inner(ly["o"], M)
       if T == 1 and not fuse_rope:
-        ops.rope_gqa_attn_lora(rd, ad, adapter(ly["o"]), self.t)
-      elif ly["o"].has_lora:
+        ops.rope_gqa_attn_lora(rd, ad, adapter(ly["o"]) if o_ready else None, self.t)
+      elif ly["o"].has_lora and o_ready:
         ops.gqa_attn_lora(ad, ly["o"].a_t, self.t)
       else:
         ops.gqa_attn(ad)
@@ -786,11 +808,11 @@ class Runner(HeadRunner):
       if cfg.family == "gemma3":
         # h += post_attn_norm(o_proj); xn = mlp_norm(h): one launch, which also sums the
         # projection's partial planes when it ran split
-        po = self.linear(ly["o"], self.attn, self.tmp, M, defer=True, t_ready=True)
+        po = self.linear(ly["o"], self.attn, self.tmp, M, defer=True, t_ready=o_ready)
         gu_ready = self.norm_pair(po, ly["post_attn_norm"], ly["mlp_norm"], M, mlp_adapter)
       else:
         po = self.linear(ly["o"], self.attn, self.h, M, epilogue=L.TNX_EPI_RESIDUAL, residual=self.h,
-                         defer=True, t_ready=True)
+                         defer=True, t_ready=o_ready)
         gu_ready = (self.norm_after(po, ly["mlp_norm"], M, ly["experts"].router_t, self.scores) if cfg.num_experts
                     else self.norm_after(po, ly["mlp_norm"], M, mlp_adapter, self.t))
       if cfg.num_experts:

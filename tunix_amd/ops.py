@@ -112,10 +112,24 @@ def dense_expand(w):
   return out
 
 
-def qlinear(desc: L.QLinearDesc, finish: bool = True):
+def lora_frag(a_t):
+  """The adapter a_t [R, K] in the order that a linear multiplies it in when it forms x . A itself (`qlinear`'s a_frag)."""
+  R, K = a_t.shape
+  return a_t.view(R // 16, 16, K // 32, 4, 8).permute(2, 0, 3, 1, 4).contiguous()
+
+
+def qlinear_inner_rows(K: int, N: int, rank: int) -> int:
+  """Rows up to which `qlinear` takes an a_frag; 0: none."""
+  return int(L.lib().tnx_qlinear_inner_rows(K, N, rank))
+
+
+def qlinear(desc: L.QLinearDesc, finish: bool = True, a_frag=None):
   """finish=False leaves the split-k partial planes in desc.ws for a consumer that sums them
-  itself (rmsnorm_splitk)."""
-  L.check(L.lib().tnx_qlinear_lora(_stream(), C.byref(desc)), "tnx_qlinear_lora")
+  itself (rmsnorm_splitk).  a_frag (`lora_frag`): the adapter's down-projection is formed inside, desc.t is not read."""
+  if a_frag is not None:
+    L.check(L.lib().tnx_qlinear_inner(_stream(), C.byref(desc), _ptr(a_frag)), "tnx_qlinear_inner")
+  else:
+    L.check(L.lib().tnx_qlinear_lora(_stream(), C.byref(desc)), "tnx_qlinear_lora")
   if desc.split_k > 1 and finish:
     L.check(L.lib().tnx_splitk_finish(_stream(), C.byref(desc)), "tnx_splitk_finish")
 
