@@ -285,9 +285,11 @@ def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank,
     (32, 2176, 384, 1, 64, Q.NF4, 64, True),     # 17
     (31, 2688, 160, 1, 128, Q.INT4, 64, True),   # 21 (20 are held)
     (24, 8192, 128, 4, 32, Q.NF4, 32, False),    # sixteen per split
+    (33, 512, 144, 1, 64, Q.NF4, 64, False),     # four row tiles, four k-tiles
+    (64, 2048, 272, 8, 32, Q.INT4, 96, False),   # two per split
 ])
 def test_few_rows_at_the_edges_of_what_lds_holds(gpu, M, K, N, split, group, qtype, rank, mul):
-  """Linears of at most 32 rows against 64 bits over the same weights, both rounded to bf16.  The fp32 sum of K products of about 0.03 is off by
+  """Linears of few rows against 64 bits over the same weights, both rounded to bf16.  The fp32 sum of K products of about 0.03 is off by
   some eps of the sum of their magnitudes, 2^-23 * 0.03 K (`off`, what a result near zero may differ by), a hundredth of a bf16 ulp of the usual
   result of 0.03 sqrt(K): the rounded values are equal but for near ties.  Gated products are rounded at every step."""
   off = 2.0 ** -23 * 0.03 * K
@@ -341,6 +343,9 @@ def test_few_rows_at_the_edges_of_what_lds_holds(gpu, M, K, N, split, group, qty
     (13, 4224, 128, 1, 64, Q.NF4, 64, "f32"),        # 33: slots are filled again
     (17, 384, 128, 1, 128, Q.INT4, 64, "store"),     # two row tiles, three k-tiles
     (32, 2176, 256, 1, 32, Q.NF4, 64, "residual"),   # 17 of 32 rows: slots are filled again
+    (33, 384, 144, 1, 64, Q.NF4, 64, "store"),       # four row tiles, three k-tiles
+    (64, 1152, 384, 3, 128, Q.INT4, 32, "store"),    # three per split
+    (57, 512, 272, 1, 32, Q.NF4, 64, "residual"),    # four
 ])
 def test_few_rows_form_the_adapters_down_projection(gpu, M, K, N, split, group, qtype, rank, epi):
   """y = x . W + 1.5 (x . A) . B with x . A formed inside, against 64 bits: x . A is a pair of bf16, 2^-17 of itself off, so the result is the
@@ -359,7 +364,7 @@ def test_few_rows_form_the_adapters_down_projection(gpu, M, K, N, split, group, 
   d = ops.make_qlinear_desc(M=M, K=K, N=N, group=group, qtype=qtype, x=x, codes=c, scales=s, y=y, split_k=split, ws=ws, lora_rank=rank, lora_nseg=1,
                             lora_seg_end=[N], lora_seg_toff=[0], t=t, t_ld=rank, lora_b=lb, lora_scale=1.5, residual=res if epi == "residual" else None,
                             epilogue={"store": L.TNX_EPI_STORE, "residual": L.TNX_EPI_RESIDUAL, "f32": L.TNX_EPI_F32}[epi])
-  assert ops.qlinear_inner_rows(K, N, rank) >= M
+  assert ops.qlinear_inner_rows(K, N, rank, split) >= M
   ops.qlinear(d, a_frag=ops.lora_frag(a_t))
   torch.cuda.synchronize()
   if epi == "f32":
@@ -374,7 +379,8 @@ def test_few_rows_form_the_adapters_down_projection(gpu, M, K, N, split, group, 
 def test_adapter_inside_refuses_other_shapes(gpu):
   from tunix_amd import _lib as L
   from tunix_amd import ops
-  assert ops.qlinear_inner_rows(512, 256, 96) == 0 and ops.qlinear_inner_rows(500, 256, 64) == 0 and ops.qlinear_inner_rows(512, 256, 64) == 32
+  assert ops.qlinear_inner_rows(512, 256, 96) == 0 and ops.qlinear_inner_rows(500, 256, 64) == 0
+  assert ops.qlinear_inner_rows(512, 256, 64) == 64 and ops.qlinear_inner_rows(640, 256, 64) == 32 and ops.qlinear_inner_rows(640, 256, 64, 2) == 64
   w = bf(rnd((512, 256), 421, 0.03)).to(gpu)
   c, s = ops.quantize_pack(w, 64, Q.NF4)
   a_t, lb = bf(rnd((64, 512), 422)).to(gpu), bf(rnd((256, 64), 423)).to(gpu)
@@ -386,7 +392,7 @@ def test_adapter_inside_refuses_other_shapes(gpu):
                 a_frag=ops.lora_frag(a_t))
 
   call()
-  for bad in (dict(M=33), dict(rank=96), dict(rank=0), dict(nseg=2), dict(nseg=-1, epi=L.TNX_EPI_SILU_MUL)):
+  for bad in (dict(M=65), dict(rank=96), dict(rank=0), dict(nseg=2), dict(nseg=-1, epi=L.TNX_EPI_SILU_MUL)):
     with pytest.raises(ValueError):
       call(**bad)
 

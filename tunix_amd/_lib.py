@@ -325,7 +325,7 @@ SIGNATURES = {
     "tnx_moe_sort_routes": (_i32, [_p, _p, _i64, _i32, _i32, _p, _p, _p]),
     "tnx_moe_int4_gmm": (_i32, [_p, C.POINTER(MoeGmmDesc)]),
     "tnx_qlinear_inner": (_i32, [_p, C.POINTER(QLinearDesc), _p]),
-    "tnx_qlinear_inner_rows": (_i64, [_i64, _i64, _i32]),
+    "tnx_qlinear_inner_rows": (_i64, [_i64, _i64, _i32, _i32]),
     "tnx_moe_gmm_expanded": (_i32, [_p, C.POINTER(MoeGmmDesc), _p]),
     "tnx_moe_expanded_rows": (_i64, [_i64, _i64, _i32]),
     "tnx_moe_combine": (_i32, [_p, _p, _p, _i64, _i32, _i64, _p, _p]),

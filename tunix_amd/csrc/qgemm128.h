@@ -100,8 +100,8 @@ __device__ __forceinline__ uint32_t next_a_off(const QLArgs& a, int n, int j, in
 // The end of a work-group of eight waves over 16 * MT rows x 128 columns: wave wv holds in `out` the sums of row tiles
 // (wv / 4) * HM ... and column tiles 2 (wv % 4), + 1 (with one row tile waves 0-3 hold all of it).  act_lds: 16 MT rows of
 // kRowsActBytes; scr_lds (SCRATCH): 16 x 36 floats per wave; both idle for every wave by now.  PRE (one row tile): wave n < 4 has asked for its
-// fragments of the next linear's adapter itself, `pre`.
-template <int MT, int NT, bool SCRATCH, bool PRE = false>
+// fragments of the next linear's adapter itself, `pre`.  POLICY: of the stores of a plane.
+template <int MT, int NT, bool SCRATCH, bool PRE = false, int POLICY = kStreamOnce>
 __device__ __forceinline__ void quant_rows_out(const QLArgs& a, f32x4 (&out)[(MT + 1) / 2][NT], int64_t m0, int64_t ntile0, int wv,
                                                uint32_t act_lds, uint32_t scr_lds, const u32x4* pre = nullptr) {
   constexpr int HM = (MT + 1) / 2, ROWS = 16 * MT;
@@ -203,7 +203,7 @@ __device__ __forceinline__ void quant_rows_out(const QLArgs& a, f32x4 (&out)[(MT
         const int r = (lane >> 3) + 8 * j, c4 = (lane & 7) * 4;
         const u32x4 v = lds_ld128(scr + (uint32_t)((r * T_LD + c4) * 4));
         const uint32_t off = ((uint32_t)(m0w + mt * 16 + r) * (uint32_t)a.N + col0 + (uint32_t)c4) * 4u;
-        __builtin_amdgcn_raw_buffer_store_b128(v, rp, off, 0, kStreamOnce);
+        __builtin_amdgcn_raw_buffer_store_b128(v, rp, off, 0, POLICY);
       }
       asm volatile("" ::: "memory");
     }

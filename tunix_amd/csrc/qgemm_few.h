@@ -1,4 +1,4 @@
-// The quantised GEMM over at most 32 rows (a decode batch): one work-group = 8 waves = ROWS (8, 16 or 32) rows x 128 columns of one k split, a
+// The quantised GEMM over at most 32 rows, or 64 of a few k-tiles (a decode batch): one work-group = 8 waves = ROWS (8, 16, 32 or 64) rows x 128 columns of one k split, a
 // wave a column tile of 16 over the whole of it.
 //
 // What bounds it is the launch and the round trip to memory, then the conversion of the codes: five instructions per pair of weights and lane
@@ -21,8 +21,8 @@
 //   int4 1152 -> 13824 gated    8.4 |  7.6    9.8 |  7.6    9.9 |  7.8   10.4 |  9.0
 //   int4 1024 -> 1152 in 8      5.0 |  3.3    5.2 |  3.7    5.2 |  3.9    5.5 |  4.7
 // Over 94 shapes (20 contractions x 5 forms of code book, group and adapter) the geometric mean is 0.80 at 1 to 16 rows and 0.88 at 17 to 32, and
-// none is slower but contractions of 64 k-tiles on eight work-groups (8192 -> 1024 unsplit, which the decoder splits: 27.4 | 29.3).  At 33 to 64 rows,
-// where eight waves read 128 KB of fragments per k-tile, the form was faster only up to three k-tiles, by 2 to 10 %: those calls are qgemm128_kernel's.
+// none is slower but contractions of 64 k-tiles on eight work-groups (8192 -> 1024 unsplit, which the decoder splits: 27.4 | 29.3).  33 to 64 rows:
+// kFewKtiles64 in qlinear.hip.
 // Also slower: sixteen waves with half a k-tile each (4096 -> 28672 over one row 23.0 us), column tiles in pairs over half of the k-tiles (the
 // sums meet: 4096 -> 4096 in 8 6.1).
 //
@@ -33,7 +33,7 @@ namespace {
 
 // LDS: the activations of a work-group's k-tiles lie in slots of ROWS * 256 bytes from address 0 on, around the table of the code book (64 KiB to
 // 128 KiB; integer codes have none).  Behind the loop the sums of gated columns meet at 128 KiB, the activated tile leaves through the table's place.
-constexpr uint32_t kFewLds = 160u << 10, kFewMeet = 0x20000, kFewOut = 0x10000;
+constexpr uint32_t kFewLds = 160u << 10, kFewMeet = 0x20000, kFewOut = 0x10000, kFewScratch = 0x14000;
 
 // INNER: the adapter's down-projection t = x . A is formed here (a.inner_a, its fragments in order) instead of ahead of the launch: a work-group
 // multiplies the activations it holds with its k range of A (wave (rank tile, half of each k-tile): the fragments of x are there already), and its share
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int PF = 4;                        // k-tiles in flight: a turn of the ring
   constexpr int TURNS = SLOTS >= 24 ? 2 : 1, CHUNK = TURNS * PF;   // turns, k-tiles whose slots are filled again together
   constexpr int NB = SLOTS / CHUNK;            // chunks that LDS holds
-  static_assert(NB >= 2 && NB * CHUNK == SLOTS && 8 * MT * 1024 <= kFewLds - kFewMeet, "LDS");
+  static_assert((SHORT ? NB >= 1 : NB >= 2 && NB * CHUNK == SLOTS) && 8 * MT * 1024 <= kFewLds - kFewMeet, "LDS");
   constexpr int SW = SPT / 2;                  // dwords of scales per column and k-tile
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -105,15 +105,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
   // Activations go from memory straight into LDS, a wave's 64 lanes 1 KB = four rows of a k-tile: chunk p of row r is k-chunk p ^ (r % 16), so
   // that the rows a fragment is read from hit different banks.
-  constexpr int QUADS = ROWS / 4;   // quads of rows per k-tile
+  constexpr int QUADS = ROWS / 4, QW = QUADS > 8 ? QUADS / 8 : 1;   // quads of rows per k-tile, and of them per wave
   const u32x4 rx = raw_rsrc(a.x, (uint64_t)a.M * a.K * 2);
   const int quad = wv % QUADS, xrow = quad * 4 + (lane >> 4);
   const uint32_t xvoff = ((uint32_t)xrow * (uint32_t)a.K + (uint32_t)((lane & 15) ^ (xrow & 15)) * 8u) * 2u;
   // k-tiles first .. first + count of this work-group into the slots from `slot` on
   auto request_x = [&](int first, int count, int slot) {
-    for (int i = wv / QUADS; i < count; i += 8 / QUADS) {
+    for (int i = wv / QUADS; i < count; i += QW > 1 ? 1 : 8 / QUADS) {
       const uint32_t at = (uint32_t)(slot + i) * SLOT;
-      dma16((INT4 || at < kBigLutBase ? at : at + (uint32_t)kBigLutBytes) + (uint32_t)quad * 1024u, rx, xvoff, (kt_begin + first + i) * (KTILE * 2));
+#pragma unroll
+      for (int q = 0; q < QW; ++q)
+        dma16((INT4 || at < kBigLutBase ? at : at + (uint32_t)kBigLutBytes) + (uint32_t)(quad + 8 * q) * 1024u, rx,
+              xvoff + (uint32_t)(32 * q) * (uint32_t)a.K * 2u, (kt_begin + first + i) * (KTILE * 2));
     }
   };
   request_x(0, min(n, NB * CHUNK), 0);
@@ -273,15 +276,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   if constexpr (INNER) {
     // the shares of t meet as rows in LDS, padded by four ranks
-    constexpr uint32_t T_LD = 68 * 4, T_HALF = 16 * MT * T_LD;
-    static_assert(2 * T_HALF <= kFewLds - kFewMeet, "LDS");
-    if ((uint32_t)n * SLOT > (INT4 ? kFewMeet : kBigLutBase)) __syncthreads();   // (activations lie there)
+    constexpr uint32_t T_LD = 68 * 4, T_HALF = 16 * MT * T_LD, T_AT = 2 * T_HALF <= kFewLds - kFewMeet ? kFewMeet : 0;
+    static_assert(2 * T_HALF <= kBigLutBase, "LDS");
+    if (T_AT == 0 || (uint32_t)n * SLOT > (INT4 ? kFewMeet : kBigLutBase)) __syncthreads();   // (activations lie there)
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float v = tacc[m][i];
-        *reinterpret_cast<lds_u32*>(static_cast<uintptr_t>(kFewMeet + (uint32_t)a_half * T_HALF + (uint32_t)(m * 16 + lq * 4 + i) * T_LD +
+        *reinterpret_cast<lds_u32*>(static_cast<uintptr_t>(T_AT + (uint32_t)a_half * T_HALF + (uint32_t)(m * 16 + lq * 4 + i) * T_LD +
                                                            (uint32_t)(a_tile * 16 + lm) * 4u)) = __float_as_uint(v);
       }
     __syncthreads();
@@ -291,7 +294,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       zero_acc(part);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {   // (ranks past the adapter's are zeros: nothing was asked for them, neither of A nor of B)
-        const uint32_t at = kFewMeet + (uint32_t)(m * 16 + lm) * T_LD + (uint32_t)(j * 32 + lq * 8) * 4u;
+        const uint32_t at = T_AT + (uint32_t)(m * 16 + lm) * T_LD + (uint32_t)(j * 32 + lq * 8) * 4u;
         u32x4 hi, lo;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int m = 0; m < MT; ++m) acc[m] = out[m][0];
   }
   const bool mul = a.epilogue == TNX_EPI_SILU_MUL || a.epilogue == TNX_EPI_GELU_MUL;
-  if (!mul || a.split_k > 1) {
+  if (MT < 4 && (!mul || a.split_k > 1)) {
     // The planes of a split are stored as they lie in the accumulators and without the non-temporal policy: with it the pass that sums them waits
     // longer than this one gains (14336 -> 4096 in 8 splits, 8 rows, with that pass: 16.1 us against 17.0, 4096 -> 4096 in 8: 11.6 against 12.5).
     f32x4 out[MT][1];
@@ -342,19 +345,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     store_tile<MT, 1>(a, 0, a.M, my_tile, ntiles, out, [](int64_t r) { return r; });
     return;
   }
-  // Gate and up columns meet: every wave leaves its sums and takes the two column tiles and the row tile it finishes.
+  // Gate and up columns meet, and the rows of a plane of many rows (whole lines of 128 bytes instead of four-byte stores: 4096 -> 4096 in 8 over 64 rows
+  // 9.5 -> 8.8 us): every wave leaves its sums and takes the two column tiles and the row tiles it finishes.
   __syncthreads();   // (activations and table lie there)
 #pragma unroll
   for (int m = 0; m < MT; ++m) lds_st128(kFewMeet + (uint32_t)(wv * MT + m) * 1024u + (uint32_t)lane * 16u, __builtin_bit_cast(u32x4, acc[m]));
   __syncthreads();
-  const int wn = wv & 3, rt = wv >> 2;
-  f32x4 out[1][2];
-  if (rt < MT) {
+  constexpr int HM = (MT + 1) / 2;
+  const int wn = wv & 3, rh = wv >> 2;
+  f32x4 out[HM][2];
+  if (MT > 1 || rh == 0) {
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-      out[0][nt] = __builtin_bit_cast(f32x4, lds_ld128(kFewMeet + (uint32_t)((2 * wn + nt) * MT + rt) * 1024u + (uint32_t)lane * 16u));
+    for (int m = 0; m < HM; ++m)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+        out[m][nt] = __builtin_bit_cast(f32x4, lds_ld128(kFewMeet + (uint32_t)((2 * wn + nt) * MT + rh * HM + m) * 1024u + (uint32_t)lane * 16u));
   }
-  quant_rows_out<MT, 2, false, (MT == 1)>(a, out, 0, (int64_t)blockIdx.y * 8 + 2 * wn, wv, kFewOut, 0u, bn);
+  quant_rows_out<MT, 2, (MT >= 4), (MT == 1), 0>(a, out, 0, (int64_t)blockIdx.y * 8 + 2 * wn, wv, kFewOut, kFewScratch, bn);
 }
 
 }  // namespace

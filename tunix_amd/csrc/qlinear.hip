@@ -764,16 +764,24 @@ int launch_qgemm_few_book(hipStream_t st, const QLArgs& a) {
 }
 template <int SPT, int ROWS, bool INNER>
 int launch_qgemm_few_rows(hipStream_t st, const QLArgs& a) {
-  if constexpr (INNER)
+  if constexpr (INNER || ROWS > 32)
     if (a.ktiles_per_split <= 4) return launch_qgemm_few_book<SPT, ROWS, INNER, true>(st, a);
-  return launch_qgemm_few_book<SPT, ROWS, INNER, false>(st, a);
+  if constexpr (ROWS <= 32) return launch_qgemm_few_book<SPT, ROWS, INNER, false>(st, a);
+  tnx_set_error("qgemm_few: %d k-tiles per split are too many for %d rows", a.ktiles_per_split, ROWS);   // (the callers see to that)
+  return TNX_EINVAL;
 }
 constexpr int64_t kFewRows = 32;
+// 33 to 64 rows too, of few k-tiles per split: what such a call waits for is its first loads (the waves read 128 KB of fragments per k-tile: at more of
+// them the form of 64 x 128 tiles shares those better, 4 | 7 | 9 | 14 k-tiles 0.96 | 1.00 | 1.06 | 1.02 of its time at 64 rows).  33 | 64 rows, us before and
+// now: int4 1024 -> 1152 in 8 5.9 -> 5.1 | 6.0 -> 5.8, 2048 -> 5120 in 6 7.9 -> 7.4 | 8.0 -> 7.9, NF4 1152 -> 1536 in 5 6.5 -> 5.9 | 6.7 -> 6.6.  Unsplit ones of 64 rows are up
+// to 8 % slower.
+constexpr int kFewKtiles64 = 4;
 template <bool INNER>
 int launch_qgemm_few(hipStream_t st, const QLArgs& a, bool two_scales) {
   if (a.M <= 8) return two_scales ? launch_qgemm_few_rows<2, 8, INNER>(st, a) : launch_qgemm_few_rows<4, 8, INNER>(st, a);
   if (a.M <= 16) return two_scales ? launch_qgemm_few_rows<2, 16, INNER>(st, a) : launch_qgemm_few_rows<4, 16, INNER>(st, a);
-  return two_scales ? launch_qgemm_few_rows<2, 32, INNER>(st, a) : launch_qgemm_few_rows<4, 32, INNER>(st, a);
+  if (a.M <= 32) return two_scales ? launch_qgemm_few_rows<2, 32, INNER>(st, a) : launch_qgemm_few_rows<4, 32, INNER>(st, a);
+  return two_scales ? launch_qgemm_few_rows<2, 64, INNER>(st, a) : launch_qgemm_few_rows<4, 64, INNER>(st, a);
 }
 
 template <int SPT, int MODE>
@@ -1105,13 +1113,15 @@ extern "C" int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* d) {
   // in register copies that cost more than the halved LDS traffic gains.
   const bool s2 = scales_per_tile(a.group) == 2;
   if (wide_shape(a)) return s2 ? launch_qgemm_wide<2>(st, a) : launch_qgemm_wide<4>(st, a);
-  if (a.M <= kFewRows) return launch_qgemm_few<false>(st, a, s2);
+  if (a.M <= kFewRows || (a.M <= 64 && a.ktiles_per_split <= kFewKtiles64 && a.split_k > 1))
+    return launch_qgemm_few<false>(st, a, s2);
   if (a.M <= 64) return s2 ? launch_qgemm128<2, 2, 4>(st, a) : launch_qgemm128<2, 4, 4>(st, a);
   return s2 ? launch_qgemm128<2, 2, 8>(st, a) : launch_qgemm128<2, 4, 8>(st, a);
 }
 
-extern "C" int64_t tnx_qlinear_inner_rows(int64_t K, int64_t N, int lora_rank) {
-  return K > 0 && K % KTILE == 0 && N > 0 && N % 16 == 0 && (lora_rank == 32 || lora_rank == 64) ? kFewRows : 0;
+extern "C" int64_t tnx_qlinear_inner_rows(int64_t K, int64_t N, int lora_rank, int split_k) {
+  if (K <= 0 || K % KTILE != 0 || N <= 0 || N % 16 != 0 || (lora_rank != 32 && lora_rank != 64)) return 0;
+  return cdiv(K / KTILE, split_k < 1 ? 1 : split_k) <= kFewKtiles64 ? 64 : kFewRows;
 }
 
 extern "C" int tnx_qlinear_inner(void* stream, const tnx_qlinear_desc* d, const uint16_t* a_frag) {
@@ -1121,7 +1131,7 @@ extern "C" int tnx_qlinear_inner(void* stream, const tnx_qlinear_desc* d, const 
   c.t_ld = 8;
   const int rc = check_desc(&c);
   if (rc) return rc;
-  TNX_REQUIRE(d->lora_rank > 0 && d->M <= tnx_qlinear_inner_rows(d->K, d->N, d->lora_rank), "qlinear_inner: %lld rows, rank %d: not a shape it takes",
+  TNX_REQUIRE(d->lora_rank > 0 && d->M <= tnx_qlinear_inner_rows(d->K, d->N, d->lora_rank, d->split_k), "qlinear_inner: %lld rows, rank %d: not a shape it takes",
               (long long)d->M, d->lora_rank);
   TNX_REQUIRE(d->lora_nseg == 1 && d->epilogue != TNX_EPI_SILU_MUL && d->epilogue != TNX_EPI_GELU_MUL, "qlinear_inner: one adapter, no *_MUL epilogue");
   TNX_REQUIRE(a_frag && ((uintptr_t)a_frag & 15) == 0, "qlinear_inner: the adapter's fragments must be there and 16-byte aligned");

@@ -52,7 +52,6 @@ class FusedLinear:
     self.load_base(weights)
     r = cfg.lora_rank
     self.has_lora = any((n + ".lora_a") in weights for n in names)
-    self.inner_rows = 0   # rows up to which the linear forms its adapter's down-projection itself
     self.rp = _pad32(r) if self.has_lora else 0
     self.r = r
     self.lora_scale = float(cfg.lora_alpha) / float(r) if self.has_lora else 0.0
@@ -66,10 +65,7 @@ class FusedLinear:
       self.a_t = torch.zeros(len(names) * self.rp, self.K, dtype=torch.bfloat16, device=device)
       self.b_t = torch.zeros(self.N, self.rp, dtype=torch.bfloat16, device=device)
       # a single adapter's A once more, in the order that few rows multiply it in inside the linear
-      self.a_frag = None
-      self.inner_rows = ops.qlinear_inner_rows(self.K, self.N, self.rp) if len(names) == 1 else 0
-      if self.inner_rows:
-        self.a_frag = ops.lora_frag(self.a_t)
+      self.a_frag = ops.lora_frag(self.a_t) if self.inner_rows(1) else None
       self._row_perm = None
       if interleave2:
         c = torch.arange(self.N, device=device)
@@ -156,6 +152,10 @@ class FusedLinear:
       self.b_t[self._row_perm] = b_full
     else:
       self.b_t.copy_(b_full)
+
+  def inner_rows(self, split_k: int) -> int:
+    """Rows up to which the linear forms its adapter's down-projection itself (0: never)."""
+    return ops.qlinear_inner_rows(self.K, self.N, self.rp, split_k) if self.has_lora and len(self.names) == 1 else 0
 
   @property
   def t_cols(self) -> int:
@@ -678,10 +678,9 @@ class Runner(HeadRunner):
     ops.qlinear(d, finish=not deferred, a_frag=f.a_frag if inner else None)
     return split if deferred else 1
 
-  @staticmethod
-  def inner(f: FusedLinear, M: int) -> bool:
+  def inner(self, f: FusedLinear, M: int) -> bool:
     """Whether `linear` of M rows forms the adapter's down-projection of its input itself: then nothing ahead of it has to."""
-    return M <= f.inner_rows
+    return M <= self.SPLIT_ROWS and M <= f.inner_rows(self._split_k(f, M))
 
   def fuses_next(self, f: FusedLinear, next_f: FusedLinear, M: int, epilogue: int) -> bool:
     return (next_f.has_lora and not self.inner(next_f, M) and next_f.rp <= 64 and M <= 1024 and self._split_k(f, M) == 1

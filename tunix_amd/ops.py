@@ -118,9 +118,9 @@ def lora_frag(a_t):
   return a_t.view(R // 16, 16, K // 32, 4, 8).permute(2, 0, 3, 1, 4).contiguous()
 
 
-def qlinear_inner_rows(K: int, N: int, rank: int) -> int:
+def qlinear_inner_rows(K: int, N: int, rank: int, split_k: int = 1) -> int:
   """Rows up to which `qlinear` takes an a_frag; 0: none."""
-  return int(L.lib().tnx_qlinear_inner_rows(K, N, rank))
+  return int(L.lib().tnx_qlinear_inner_rows(K, N, rank, split_k))
 
 
 def qlinear(desc: L.QLinearDesc, finish: bool = True, a_frag=None):
