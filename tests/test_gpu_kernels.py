@@ -949,6 +949,14 @@ def test_gqa_attention_many_positions_equals_few(gpu, B, T, S, Hq, Hkv, col, win
   assert torch.equal(whole.view(torch.int16), parts.view(torch.int16))
 
 
+@pytest.mark.parametrize("T,col,window", [(62, 0, 0), (62, 2, 0), (62, 3, 0), (62, 35, 0), (62, 66, 0), (62, 67, 0),   # 2, 2, 3, 4, 4, 5 key blocks
+                                          (93, 31, 30), (93, 33, 33), (64, 64, 1)])    # windows that start on either block of a pair
+def test_attention_key_blocks_in_pairs(gpu, T, col, window):
+  """Numbers of key blocks around the pair that a work-group takes behind one barrier, its waves starting and ending at either of the two.  (No
+  number of positions that leaves a single one for the last of the calls compared with: one position's keys are divided among waves.)"""
+  test_gqa_attention_many_positions_equals_few(gpu, 2, T, col + T + 1, 8, 2, col, window, False, None)
+
+
 @pytest.mark.parametrize("M,D,V,temperature", [(1, 128, 65536, 1.0), (17, 384, 65552, 0.7), (64, 256, 66000, 1.0),
                                                (65, 256, 65536, 1.0), (128, 128, 65600, 1.0)])
 def test_dense_head_over_few_rows_equals_many(gpu, M, D, V, temperature):

@@ -982,36 +982,54 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 // The same for head_dim 128 and 256 with keys and values staged through LDS: a work-group of four waves
 // takes 4 x QW consecutive query tiles of one (row, kv head), and every 32-key block is requested
 // once per work-group straight into LDS (16 bytes per lane, key rows with their 16-byte chunks
-// XOR-swizzled by row so that the fragment reads of 16 rows hit 16 bank groups; value rows as they
-// are; the block's 32 token / segment ids next to them, by the dword: rows of ids need no alignment),
+// XOR-swizzled by row so that the fragment reads of 16 rows hit 16 bank groups, value rows by pairs of chunks, which the transposing
+// reads take whole; the block's 32 token / segment ids next to them, by the dword: rows of ids need no alignment),
 // the next blocks in flight.  Every wave computes exactly the blocks attn_tiles_kernel would give it, in the same order
 // with the same arithmetic: outputs are bit-identical.
 //
-// What bounds it is vector work: per score 11 lane-instructions (two roundings to bf16 with a scale between them, maximum, exponential,
-// sum, rounding of P) against half a clock of matrix pipe.  So the tiles of a wave run through one straight line of code, whose
-// chains hide each other's latency, with two such work-groups per compute unit; values are rounded in pairs; maxima cross the
-// lanes in registers (permlane swaps) instead of through LDS; and O is kept transposed (P.V formed as V^T . P^T: the same operand
-// registers with the operands exchanged), so that a query's rescaling factor is already in the lanes that need it.
-// 32 heads of 128 over 8 kv heads, us: 2 x 6144 positions 1369 -> 1110 (451 -> 557 TFLOP/s), 13 x 1024 packed 395 -> 306; rows of ids
-// off 16-byte alignment, which took attn_tiles_kernel, 7 x 1023 over 4 kv heads: 363 -> 167.
+// What bounds it is vector work and the waits between its steps: per score 9 lane-instructions (two roundings to bf16 with a scale between
+// them, maximum, exponential, sum, rounding of P) against half a clock of matrix pipe.  So the tiles of a wave run through one straight line of
+// code, whose chains hide each other's latency, with two such work-groups per compute unit; the values leave LDS transposed
+// (ds_read_tr: no packing of rows by the vector unit); maxima cross the lanes in registers (permlane swaps) instead of through LDS; O is kept
+// transposed (P.V formed as V^T . P^T: the same operand registers with the operands exchanged), so that a query's rescaling
+// factor is already in the lanes that need it; the ids of a block are tested by one read and one ballot, and read key by key only where one
+// differs; and head_dim 128 meets at a barrier every second block.
+// 32 heads of 128 over 8 kv heads, us before (values rounded in pairs by the vector unit, a barrier per block) and now:
+//   2 x 6144 positions 895 -> 826 (691 -> 750 TFLOP/s)   3 x 2900: 337 -> 311   13 x 1024: 221 -> 208   7 x 1023 over 4: 135 -> 132
+//   64 x 256: 119.5 -> 119.5   16 x 128: 16.3 -> 15.6    head_dim 256, 4 heads over 1: 3 x 3000 135 -> 116, 64 x 256 40.8 -> 39.2
+// Two blocks in one line of code (both blocks' scores, then both softmaxes, then both blocks' values): 1030 for the first.
 typedef uint32_t __attribute__((address_space(3))) lds_word_t;
 typedef u32x4 __attribute__((address_space(3))) lds_vec_t;
 __device__ __forceinline__ u32x4 attn_lds128(uint32_t addr) {
   return *reinterpret_cast<const lds_vec_t*>(static_cast<uintptr_t>(addr));
 }
+__device__ __forceinline__ uint32_t attn_lds32(uint32_t addr) { return *reinterpret_cast<const lds_word_t*>(static_cast<uintptr_t>(addr)); }
+// Of each 16 lanes, which point at four rows of 16 16-bit elements, 8 bytes a lane (row lane / 4, elements 4 (lane % 4) ..), lane i gets element i of
+// the four rows.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x2 attn_lds_tr16(uint32_t addr) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                       (__attribute__((address_space(3))) s16x4*)static_cast<uintptr_t>(addr)));
+}
+// Maxima of numbers that no operation left as signalling NaNs (fmaxf quiets each operand first, an instruction more).  What a permlane swap reads
+// of them is a copy and its source, at least the copy and the distance that the compiler keeps behind it away.
+__device__ __forceinline__ float max_plain(float x, float y) {
+  float d;
+  asm("v_max_f32 %0, %1, %2" : "=v"(d) : "v"(x), "v"(y));
+  return d;
+}
+__device__ __forceinline__ float max3_plain(float x, float y, float z) {
+  float d;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(x), "v"(y), "v"(z));
+  return d;
+}
 // four bytes per lane straight into LDS, at `lds` + 4 * lane (as dma16 of gemm_tile.h)
 __device__ __forceinline__ void dma4(uint32_t lds, const u32x4& r, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(r) : "memory", "m0");
 }
-// c += a . b with the accumulator in place (the compiler's form copies O at every branch of the loop).  The wait states between a
-// vector write of an operand and the MFMA that reads it stand inside, under the MFMA before; what reads c next has to lie eight
-// instruction slots behind (the compiler does not know that this is an MFMA: tests/test_mfma_wait_states.py checks the built code).
-__device__ __forceinline__ void mfma16_tied(u32x4 a, u32x4 b, f32x4& c) {
-  asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
-}
 // 32 keys, 32 values, ids
 constexpr uint32_t wg_stage_bytes(int dh) { return 32u * (uint32_t)dh * 2u * 2u + 256u; }
-// Blocks in LDS: one computed, the others in flight; what two work-groups per compute unit have room for.
+// Blocks in LDS, half of them computed and half in flight; what two work-groups per compute unit have room for.
 constexpr int wg_stages(int dh) { return dh > 128 ? 2 : 4; }
 // Query tiles of a wave: O and the queries of two at head_dim 256 leave room for one wave per SIMD only, and a wave alone does not cover its own
 // softmax.
@@ -1061,7 +1079,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int kb0 = k_lo & ~31, kb_last = k_hi & ~31;
   const bool any = wave_live && kb0 <= k_hi;
 
-  // O^T: lane (query lm, quarter lq) holds dimensions 128 h + 32 lq + 8 i + jj in O[w][8 h + jj][i]
+  // O^T: lane (query lm, quarter lq) holds dimensions 128 h + 16 jj + 4 lq + i in O[w][8 h + jj][i]
   f32x4 O[QW][8 * NH];
   float m_run[QW], l_run[QW];
 #pragma unroll
@@ -1105,12 +1123,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const u32x4 rk = raw_rsrc(kbase, slab_bytes), rv = raw_rsrc(vbase, slab_bytes);
   const u32x4 rtok = raw_rsrc(tok, (uint64_t)min(a.S, a.tok_ld) * 4);
   // thread t requests, per 4 KB pass over a block (16 rows | 8), the 16 bytes that land at byte 16 t of the pass:
-  // row t / 16 | t / 32, and of the key row the chunk (t % 16 | t % 32) ^ (row % 16)
+  // row t / 16 | t / 32, and of the key row the chunk (t % 16 | t % 32) ^ (row % 16), of the value row the one whose pair of chunks is that of
+  // this place ^ (row % 8)
   constexpr int CH = DH / 8;   // chunks of a row
   const uint32_t krow = (uint32_t)(tid / CH);
   const uint32_t kreq = krow * ROW + ((uint32_t)(tid % CH) ^ krow) * 16u;
-  const uint32_t vreq = (uint32_t)tid * 16u;
-  auto request_block = [&](int i) {   // 2 PASSES + 1 requests per wave (the ids by every wave: same bytes, one count)
+  const uint32_t vreq = krow * ROW + ((uint32_t)(tid % CH) ^ ((krow & 7u) * 2u)) * 16u;
+  auto request_block = [&](int i) {   // (the ids by every wave: the same bytes)
     const uint32_t base = lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes + (uint32_t)wave * 1024u;
     const uint32_t kb_bytes = (uint32_t)(kb0_wg + 32 * i) * ROW;
 #pragma unroll
@@ -1121,28 +1140,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // ids kb .. kb + 63 (the block's 32 and whatever follows them; past the row: zeros)
     dma4(lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes + IAT, rtok, (uint32_t)(kb0_wg + 32 * i + lane) * 4u);
   };
-  // this lane's places in a stage: key row lm (+ 16 tt), chunk 4 j + lq; value rows 4 lq + s (+ 16), chunk lm (+ 16 h); ids 4 lq
+  // this lane's places in a stage: key row lm (+ 16 tt), chunk 4 j + lq; value row 4 lq + lm / 4 (+ 16 tt), 8 bytes lm % 4 of dimensions 16 jj (+ 128 h)
+  // .. + 16, jj under XOR; ids 4 lq, and of key lane % 32
   uint32_t kat[KS];
 #pragma unroll
   for (int j = 0; j < KS; ++j) kat[j] = (uint32_t)lm * ROW + (((uint32_t)(j * 4 + lq) ^ (uint32_t)lm) * 16u);
-  const uint32_t vat = VAT + (uint32_t)lq * (4u * ROW) + (uint32_t)(lm * 16), iat = IAT + (uint32_t)(lq * 16);
+  const uint32_t vrow = (uint32_t)(4 * lq + (lm >> 2));
+  const uint32_t vat = VAT + vrow * ROW + (vrow & 7u) * 32u + (uint32_t)(lm & 3) * 8u, iat = IAT + (uint32_t)(lq * 16);
+  const uint32_t one_at = IAT + (uint32_t)(lane & 31) * 4u;
   auto compute_block = [&](int kb, uint32_t base) {
-    u32x4 kf[2][KS], vf[8];
+    u32x4 kf[2][KS];
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
       const uint32_t at = base + kat[j];
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) kf[tt][j] = attn_lds128(at + (uint32_t)tt * (16u * ROW));
     }
-    const uint32_t va = base + vat, ia = base + iat;
-    const u32x4 t0 = attn_lds128(ia), t1 = attn_lds128(ia + 64u);
-#pragma unroll
-    for (int s = 0; s < 8; ++s) vf[s] = attn_lds128(va + (uint32_t)(s < 4 ? s : 12 + s) * ROW);
     // (pad mode: a key counts when its id differs from pad_id; packed: when it is the query's)
-    bool ids = true;
-#pragma unroll
-    for (int s = 0; s < 4; ++s) ids = ids & (((int)t0[s] == one_id) == id_equal) & (((int)t1[s] == one_id) == id_equal);
-    const bool inside = kb >= lo_max && kb + 31 <= hi_min && __builtin_amdgcn_ballot_w64(ids) == ~0ull;
+    const bool inside = kb >= lo_max && kb + 31 <= hi_min &&
+                        __builtin_amdgcn_ballot_w64(((int)attn_lds32(base + one_at) == one_id) == id_equal) == ~0ull;
     f32x4 st[QW][2];
 #pragma unroll
     for (int w = 0; w < QW; ++w)
@@ -1166,6 +1182,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     if (!inside) {
       asm volatile("");   // (a branch, not selects in every block)
+      const u32x4 t0 = attn_lds128(base + iat), t1 = attn_lds128(base + iat + 64u);
 #pragma unroll
       for (int w = 0; w < QW; ++w)
 #pragma unroll
@@ -1180,9 +1197,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     u32x4 pa[QW];
 #pragma unroll
     for (int w = 0; w < QW; ++w) {
-      const float lo = fmaxf(fmaxf(fmaxf(sv[w][0], sv[w][1]), sv[w][2]), sv[w][3]);
-      const float hi = fmaxf(fmaxf(fmaxf(sv[w][4], sv[w][5]), sv[w][6]), sv[w][7]);
-      const float m_new = fmaxf(m_run[w], across_quarters(fmaxf(lo, hi), [](float x, float y) { return fmaxf(x, y); }));
+      const float m_blk = max3_plain(max3_plain(sv[w][0], sv[w][1], sv[w][2]), max3_plain(sv[w][3], sv[w][4], sv[w][5]), max_plain(sv[w][6], sv[w][7]));
+      const float m_new = max_plain(m_run[w], across_quarters(m_blk, [](float x, float y) { return max_plain(x, y); }));
       alpha[w] = __expf(m_run[w] - m_new);
       moved = moved || alpha[w] != 1.0f;
       m_run[w] = m_new;
@@ -1205,57 +1221,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
           for (int i = 0; i < 4; ++i) O[w][jj][i] *= alpha[w];
     }
-    // a value fragment is transposed once for all tiles
+    // value fragments come out of LDS transposed, once for all tiles: four keys of a dimension per lane and read
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
-      if (h > 0)
-#pragma unroll
-        for (int s = 0; s < 8; ++s) vf[s] = attn_lds128(va + (uint32_t)(s < 4 ? s : 12 + s) * ROW + (uint32_t)h * 256u);
+    for (int h = 0; h < NH; ++h)
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj) {
-        const uint32_t sel = (jj & 1) ? 0x07060302u : 0x05040100u;
-        u32x4 vt;
+        const uint32_t at = ((base + vat) ^ (uint32_t)(jj * 32)) + (uint32_t)h * 256u;
+        const u32x2 v0 = attn_lds_tr16(at), v1 = attn_lds_tr16(at + 16u * ROW);
+        const u32x4 vt = {v0[0], v0[1], v1[0], v1[1]};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) vt[r] = __builtin_amdgcn_perm(vf[2 * r + 1][jj >> 1], vf[2 * r][jj >> 1], sel);
-#pragma unroll
-        for (int w = 0; w < QW; ++w) mfma16_tied(vt, pa[w], O[w][8 * h + jj]);
+        for (int w = 0; w < QW; ++w) O[w][8 * h + jj] = mfma16(vt, pa[w], O[w][8 * h + jj]);
       }
-    }
   };
+  // BATCH blocks behind a barrier; the next ones are on their way meanwhile, into the stages that the ones before were read from.  (A barrier per
+  // block: 828 us instead of 815 for 2 x 6144 positions, the rest alike.)
+  constexpr int BATCH = kWgStages / 2;
 #pragma unroll
-  for (int u = 0; u < kWgStages - 1; ++u)
+  for (int u = 0; u < BATCH; ++u)
     if (u < nblk_wg) request_block(u);
-  for (int i = 0; i < nblk_wg; ++i) {
-    // this wave's share of block i has landed (behind it: the requests of blocks i + 1 ..
-    // i + stages - 2; near the end, where fewer follow, everything is waited for) ...
-    if (i + kWgStages - 2 < nblk_wg) tnx_wait_vm((int)(2 * PASSES + 1) * (kWgStages - 2));
-    else tnx_wait_vm(0);
-    __syncthreads();    // ... and everyone's; every wave is also done reading block i - 1, whose stage is refilled
-    if (i + kWgStages - 1 < nblk_wg) request_block(i + kWgStages - 1);
-    const int kb = kb0_wg + 32 * i;
-    if (any && kb >= kb0 && kb <= kb_last) compute_block(kb, lds0 + (uint32_t)(i % kWgStages) * kWgStageBytes);
+  for (int i = 0; i < nblk_wg; i += BATCH) {
+    tnx_wait_vm(0);     // this wave's share of the blocks has landed ...
+    __syncthreads();    // ... and everyone's; every wave is also done reading the blocks before
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u)
+      if (i + BATCH + u < nblk_wg) request_block(i + BATCH + u);
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) {
+      const int kb = kb0_wg + 32 * (i + u);
+      if (any && kb >= kb0 && kb <= kb_last) compute_block(kb, lds0 + (uint32_t)((i + u) % kWgStages) * kWgStageBytes);
+    }
   }
-  asm volatile("s_nop 15\n\ts_nop 7");
-#pragma unroll
-  for (int w = 0; w < QW; ++w)
-#pragma unroll
-    for (int jj = 0; jj < 8 * NH; ++jj) asm volatile("" : "+v"(O[w][jj]));
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
     const float l = across_quarters(l_run[w], [](float x, float y) { return x + y; });
     const int ti = (qt0 + w) * PT + (lm >> a.gp_shift);
     if (!qvalid[w]) continue;
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t* o = a.out + ((b * a.T + ti) * a.Hq + hkv * a.G + g) * DH + 32 * lq;
+    uint16_t* o = a.out + ((b * a.T + ti) * a.Hq + hkv * a.G + g) * DH + 4 * lq;
 #pragma unroll
-    for (int h = 0; h < NH; ++h)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        u32x4 wv;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) wv[r] = pack2bf(O[w][8 * h + 2 * r][i] * inv, O[w][8 * h + 2 * r + 1][i] * inv);
-        *reinterpret_cast<u32x4*>(o + 128 * h + 8 * i) = wv;
-      }
+    for (int jj = 0; jj < 8 * NH; ++jj)
+      *reinterpret_cast<u32x2*>(o + 16 * jj) = u32x2{pack2bf(O[w][jj][0] * inv, O[w][jj][1] * inv), pack2bf(O[w][jj][2] * inv, O[w][jj][3] * inv)};
   }
 }
 
