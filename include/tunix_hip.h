@@ -82,9 +82,9 @@ const char* tnx_last_error(void);
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
  * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora,
  * tnx_gqa_attn_lora, tnx_rope_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric; 6.4 adds tnx_qlinear_inner and
- * tnx_qlinear_inner_rows. */
+ * tnx_qlinear_inner_rows; 6.5 adds tnx_lmhead_commit. */
 #define TNX_ABI_VERSION_MAJOR 6
-#define TNX_ABI_VERSION_MINOR 4
+#define TNX_ABI_VERSION_MINOR 5
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
 int tnx_version(void);
 
@@ -499,6 +499,21 @@ int tnx_sample_topk_head(void* stream, const float* logits, const float* part, c
 int tnx_sample_commit(void* stream, const int32_t* ids, const float* logp, int64_t B,
                       int32_t* tokens, int64_t tok_ld, float* logprobs, int32_t* done,
                       const int32_t* eos, int n_eos, int32_t* step_ptr);
+
+/* tnx_lmhead_logp and the bookkeeping of what it chose (its draw_id, or best_id where nothing is drawn; logprobs from draw_logp or
+ * best_logp), without a launch of its own.  The fields mean what they mean in tnx_sample_commit; tickets: a word that holds 0 before
+ * the first call and between calls, one for each step counter. */
+typedef struct tnx_commit_desc {
+  int32_t* tokens;
+  int64_t tok_ld;
+  float* logprobs;        /* or NULL */
+  int32_t* done;          /* or NULL */
+  const int32_t* eos;
+  int n_eos;
+  int32_t* step_ptr;
+  uint32_t* tickets;
+} tnx_commit_desc;
+int tnx_lmhead_commit(void* stream, const tnx_lmhead_desc* h_desc, const tnx_commit_desc* h_commit);
 
 /* ---------------------------------------------------------------------------------------
  * MoE (qwen3/model.py:787-832): router softmax -> top-k -> renormalise (weights bf16), and an

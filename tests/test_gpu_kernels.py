@@ -1588,6 +1588,51 @@ def test_sample_commit_and_fill(gpu):
   assert buf.sum().item() == 0
 
 
+@pytest.mark.parametrize("M,V,draw,lists", [(1, 640, False, True), (1, 640, True, False), (5, 9008, False, False), (17, 8256, True, True),
+                                            (64, 640, False, True), (130, 9008, True, True), (1000, 640, False, True)])
+def test_head_enters_its_own_choice(gpu, M, V, draw, lists):
+  """tnx_lmhead_commit against tnx_lmhead_logp and tnx_sample_commit behind it, over several steps from one state each (the tickets are as they
+  were after every call); all whole numbers and the same bits."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  D, steps, dev = 128, 3, gpu
+  w = bf(rnd((V, D), 501)).to(dev)
+  eos = torch.arange(0, V, 3, dtype=torch.int32, device=dev)
+  states = []
+  for fused in (False, True):
+    tokens = torch.zeros(M, 4 + steps, dtype=torch.int32, device=dev)
+    lps = torch.zeros(M, 4 + steps, dtype=torch.float32, device=dev) if lists else None
+    done = torch.zeros(M, dtype=torch.int32, device=dev) if lists else None
+    step, tickets = torch.tensor([2], dtype=torch.int32, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
+    ids, lp = torch.empty(M, dtype=torch.int32, device=dev), torch.empty(M, dtype=torch.float32, device=dev)
+    nvb = ops.lmhead_nblocks(V)
+    part, part_draw = torch.empty(M * nvb * 4, device=dev), torch.empty(M * nvb * 3, device=dev)
+    for i in range(steps):
+      x = bf(rnd((M, D), 510 + i)).to(dev)
+      d = L.LmHeadDesc()
+      d.M, d.D, d.V, d.x, d.w_bf16, d.part, d.temperature = M, D, V, x.data_ptr(), w.data_ptr(), part.data_ptr(), 0.8 if draw else 1.0
+      if draw:
+        d.part_draw, d.draw_key0, d.draw_key1, d.draw_step_ptr = part_draw.data_ptr(), 5, 6, step.data_ptr()
+        d.draw_id, d.draw_logp = ids.data_ptr(), lp.data_ptr()
+      else:
+        d.best_id, d.best_logp = ids.data_ptr(), lp.data_ptr()
+      if fused:
+        ops.lmhead_commit(d, ops.make_commit_desc(tokens, lps, done, eos if lists else None, step, tickets))
+      else:
+        ops.lmhead(d)
+        ops.sample_commit(ids, lp if lists else None, tokens, lps, done, eos if lists else None, step)
+    assert step.item() == 2 + steps and tickets.item() == 0
+    states.append([t.cpu() for t in (tokens, lps, done, ids, lp) if t is not None])
+  for a, b in zip(*states):
+    assert torch.equal(a, b)
+  if lists and M > 16:
+    assert 0 < states[1][2].sum() < M
+  c = ops.make_commit_desc(tokens, lps, done, None, step, tickets)
+  d.draw_id, d.best_id = None, None
+  with pytest.raises(ValueError, match="chooses nothing"):
+    ops.lmhead_commit(d, c)
+
+
 def test_grpo_ratio_matches_oracle(gpu):
   from tunix_amd import ops
   N, T = 4096, 64

@@ -12,7 +12,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtunix_hip.so")
 
 # the ABI this binding was written against (TNX_ABI_VERSION_MAJOR / _MINOR of include/tunix_hip.h)
-ABI_VERSION = (6, 4)
+ABI_VERSION = (6, 5)
 
 TNX_Q_INT4, TNX_Q_NF4 = 0, 1
 TNX_NORM_LLAMA, TNX_NORM_QWEN3, TNX_NORM_GEMMA3 = 0, 1, 2
@@ -91,6 +91,10 @@ class LmHeadDesc(C.Structure):
       ("draw_step_ptr", _p), ("draw_id", _p), ("draw_logp", _p), ("logits_fp32", _i32),
       ("w_expanded", _p), ("softcap", _f32),
   ]
+
+
+class CommitDesc(C.Structure):
+  _fields_ = [("tokens", _p), ("tok_ld", _i64), ("logprobs", _p), ("done", _p), ("eos", _p), ("n_eos", _i32), ("step_ptr", _p), ("tickets", _p)]
 
 
 class MoeGmmDesc(C.Structure):
@@ -313,6 +317,7 @@ SIGNATURES = {
     "tnx_rope_gqa_attn_lora": (_i32, [_p, C.POINTER(RopeDesc), C.POINTER(AttnDesc), _p, _i32, _p, _i64]),
     "tnx_lmhead_nblocks": (_i64, [_i64]),
     "tnx_lmhead_logp": (_i32, [_p, C.POINTER(LmHeadDesc)]),
+    "tnx_lmhead_commit": (_i32, [_p, C.POINTER(LmHeadDesc), C.POINTER(CommitDesc)]),
     "tnx_sample_topk_ws_bytes": (C.c_size_t, [_i64, _i64, _i32]),
     "tnx_sample_fullsort_ws_bytes": (C.c_size_t, [_i64, _i64]),
     "tnx_sample_topk": (_i32, [_p, _p, _i64, _i64, _i32, _f32, _f32, C.c_uint32, C.c_uint32, _i32,

@@ -82,6 +82,7 @@ class _SamplingState:
     self.done = torch.zeros(B, dtype=torch.int32, device=dev)
     # decoding_step: column of the last committed token
     self.step = torch.full((1,), P - 1, dtype=torch.int32, device=dev)
+    self.tickets = torch.zeros(1, dtype=torch.int32, device=dev)   # tnx_commit_desc's
     # column of each row's first token
     self.starts = torch.tensor([P - n for n in lengths], dtype=torch.int32, device=dev)
     self.cache = model.new_cache(B, cache_size)
@@ -148,9 +149,11 @@ class Sampler:
   def _sample(self, runner, x, st: _SamplingState, mode: dict):
     """lm_head + sampling + bookkeeping for the B rows in x (sampler.py:474-552)."""
     want_lp = st.logprobs_buffer is not None
+    # where the head itself chooses, it enters its choice too
+    entered = dict(commit=ops.make_commit_desc(st.token_buffer, st.logprobs_buffer, st.done, mode["eos"], st.step, st.tickets)) if runner.commits else {}
     if mode["name"] == "greedy":
       runner.run_head(x, runner.B, best_id=runner.best_id, best_logp=runner.best_logp,
-                      forbidden=mode["forbidden"], logits_out=runner.logits)
+                      forbidden=mode["forbidden"], logits_out=runner.logits, **entered)
       ids, lp = runner.best_id, (runner.best_logp if want_lp else None)
     elif mode["top_k"] == 0 and mode["top_p"] >= 1.0:
       # the plain categorical draw (the reference's default rollout configuration) happens inside
@@ -158,11 +161,12 @@ class Sampler:
       runner.run_head(x, runner.B, temperature=mode["temperature"], forbidden=mode["forbidden"],
                       logits_out=runner.logits,
                       draw=dict(part=mode["part_draw"], key=mode["key"], variant=self.rng_variant,
-                                step=st.step, ids=mode["ids"], logp=mode["logp"]))
+                                step=st.step, ids=mode["ids"], logp=mode["logp"]), **entered)
       ids, lp = mode["ids"], (mode["logp"] if want_lp else None)
     elif mode.get("head_lse") is not None:
       # top-k of at most 64: the head runs at the sampling temperature and leaves per-block
       # maxima and the row's log-sum-exp; the draw then reads only the k best blocks' logits
+      entered = {}
       runner.run_head(x, runner.B, temperature=mode["temperature"], forbidden=mode["forbidden"],
                       lse=mode["head_lse"], logits_out=runner.logits)
       ops.sample_topk_head(runner.logits, runner.part, mode["head_lse"], mode["top_k"], mode["top_p"],
@@ -170,12 +174,14 @@ class Sampler:
                            mode["logp"], forbidden=mode["forbidden"])
       ids, lp = mode["ids"], (mode["logp"] if want_lp else None)
     else:
+      entered = {}
       runner.run_head(x, runner.B, best_id=runner.best_id, logits_out=runner.logits)
       ops.sample_topk(runner.logits, mode["top_k"], mode["top_p"], mode["temperature"], mode["key"],
                       self.rng_variant, st.step, mode["ws"], mode["ids"], mode["logp"],
                       forbidden=mode["forbidden"])
       ids, lp = mode["ids"], (mode["logp"] if want_lp else None)
-    ops.sample_commit(ids, lp, st.token_buffer, st.logprobs_buffer, st.done, mode["eos"], st.step)
+    if not entered:
+      ops.sample_commit(ids, lp, st.token_buffer, st.logprobs_buffer, st.done, mode["eos"], st.step)
 
   def forward_prompt(self, st: _SamplingState, on_rows):
     """Forward over the padded prompts (sampler.py:554-616), filling the cache, in groups of rows:

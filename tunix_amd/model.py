@@ -503,11 +503,15 @@ class HeadRunner:
         d.draw_logp = draw["logp"].data_ptr()
     return d
 
-  def run_head(self, x, rows, **kw):
+  commits = True   # run_head takes `commit`
+
+  def run_head(self, x, rows, commit=None, **kw):
+    """commit: what ops.make_commit_desc gives, the choice of this call is then entered into it."""
     m = self.model
     if m.head is not None and m.head.has_lora:
       ops.lora_down(x, m.head.a_t, self.t, M=rows)
-    ops.lmhead(self.head_desc(x, rows, self.part, **kw))
+    d = self.head_desc(x, rows, self.part, **kw)
+    ops.lmhead(d) if commit is None else ops.lmhead_commit(d, commit)
 
 
 class Runner(HeadRunner):

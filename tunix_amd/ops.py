@@ -234,6 +234,10 @@ def lmhead(desc: L.LmHeadDesc):
   L.check(L.lib().tnx_lmhead_logp(_stream(), C.byref(desc)), "tnx_lmhead_logp")
 
 
+def lmhead_commit(desc: L.LmHeadDesc, commit: L.CommitDesc):
+  L.check(L.lib().tnx_lmhead_commit(_stream(), C.byref(desc), C.byref(commit)), "tnx_lmhead_commit")
+
+
 def sample_topk_ws_bytes(M, V, k) -> int:
   return int(L.lib().tnx_sample_topk_ws_bytes(M, V, 0 if k is None else int(k)))
 
@@ -277,6 +281,13 @@ def sample_commit(ids, logp, tokens, logprobs, done, eos, step_ptr):
                                     tokens.shape[1], _ptr(logprobs), _ptr(done), _ptr(eos),
                                     0 if eos is None else eos.numel(), _ptr(step_ptr)),
           "tnx_sample_commit")
+
+
+def make_commit_desc(tokens, logprobs, done, eos, step_ptr, tickets) -> L.CommitDesc:
+  c = L.CommitDesc()
+  c.tokens, c.tok_ld, c.logprobs, c.done = _ptr(tokens), tokens.shape[1], _ptr(logprobs), _ptr(done)
+  c.eos, c.n_eos, c.step_ptr, c.tickets = _ptr(eos), 0 if eos is None else eos.numel(), _ptr(step_ptr), _ptr(tickets)
+  return c
 
 
 def moe_route_topk(scores, k, topk_w, topk_id):

@@ -1114,11 +1114,15 @@ class StackRunner(HeadRunner):
     d.softcap = self.cfg.logit_softcap
     return d
 
+  @property
+  def commits(self):
+    return self.model.block_head
+
   def run_head(self, x, rows, temperature=1.0, targets=None, best_id=None, best_logp=None, target_logp=None, lse=None,
-               logits_out=None, forbidden=None, entropy=None, part_entropy=None, draw=None, logits_fp32=False):
+               logits_out=None, forbidden=None, entropy=None, part_entropy=None, draw=None, logits_fp32=False, commit=None):
     m = self.model
     if m.block_head:
-      return super().run_head(x, rows, temperature=temperature, targets=targets, best_id=best_id, best_logp=best_logp,
+      return super().run_head(x, rows, commit=commit, temperature=temperature, targets=targets, best_id=best_id, best_logp=best_logp,
                               target_logp=target_logp, lse=lse, logits_out=logits_out, forbidden=forbidden,
                               entropy=entropy, part_entropy=part_entropy, draw=draw, logits_fp32=logits_fp32)
     V, f = self.cfg.vocab_size, m.head_linear
