@@ -82,7 +82,7 @@ const char* tnx_last_error(void);
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
  * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora,
  * tnx_gqa_attn_lora, tnx_rope_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric; 6.4 adds tnx_qlinear_inner and
- * tnx_qlinear_inner_rows; 6.5 adds tnx_lmhead_commit. */
+ * tnx_qlinear_inner_rows; 6.5 adds tnx_lmhead_commit and tnx_embed_norm. */
 #define TNX_ABI_VERSION_MAJOR 6
 #define TNX_ABI_VERSION_MINOR 5
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
@@ -280,6 +280,25 @@ typedef struct tnx_norm_lora_desc {
   int R;
 } tnx_norm_lora_desc;
 int tnx_norm_lora(void* stream, const tnx_norm_lora_desc* d);
+
+/* tnx_embed of M = B * T rows into h_out and tnx_norm_lora of them (x, ws, y_route, res_pre, res_post and w2 null; a_t null: the norm alone)
+ * in the launches of the latter, and with sin_out tnx_rope_table too (a step's: T tokens share the row's first position). */
+typedef struct tnx_embed_desc {
+  const uint16_t* table;    /* bf16 [V, D] */
+  int64_t V;
+  const int32_t* ids;
+  int64_t ids_ld;
+  const int32_t* col_ptr;
+  int64_t B, T;
+  float scale;
+  const int32_t* positions; /* the rope table, or nulls */
+  int64_t pos_ld;
+  const float* timescale;
+  int dh;
+  float* sin_out;
+  float* cos_out;
+} tnx_embed_desc;
+int tnx_embed_norm(void* stream, const tnx_embed_desc* e, const tnx_norm_lora_desc* d);
 
 /* ---------------------------------------------------------------------------------------
  * Per-head q/k RMSNorm (optional) + RoPE + KV-cache write for T tokens per row.

@@ -92,7 +92,7 @@ def test_struct_layouts_match_the_header(tmp_path):
            "tnx_latent_kv_desc": L.LatentKvDesc, "tnx_latent_attn_desc": L.LatentAttnDesc, "tnx_gate_mul_desc": L.GateMulDesc,
            "tnx_parallel_step_desc": L.ParallelStepDesc, "tnx_conv_kvwrite_desc": L.ConvKvDesc, "tnx_mixed_attn_desc": L.MixedAttnDesc,
            "tnx_memory_desc": L.MemoryDesc, "tnx_rownorm_kvwrite_desc": L.RowNormKvDesc, "tnx_gated_state_desc": L.GatedStateDesc,
-           "tnx_norm_lora_desc": L.NormLoraDesc, "tnx_commit_desc": L.CommitDesc}
+           "tnx_norm_lora_desc": L.NormLoraDesc, "tnx_commit_desc": L.CommitDesc, "tnx_embed_desc": L.EmbedDesc}
   lines = ['#include <stdio.h>', '#include <stddef.h>', '#include "tunix_hip.h"', 'int main(void) {']
   for cname, cls in pairs.items():
     lines.append(f'  printf("{cname} %zu\\n", sizeof({cname}));')

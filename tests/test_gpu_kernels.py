@@ -1588,6 +1588,41 @@ def test_sample_commit_and_fill(gpu):
   assert buf.sum().item() == 0
 
 
+@pytest.mark.parametrize("B,T,D,R,scale,dh,flavor", [
+    (1, 1, 256, 32, 1.0, 0, 1), (1, 1, 4096, 192, 1.0, 128, 0), (16, 1, 4096, 192, 1.0, 128, 0),   # one launch, the table's rows behind the last
+    (17, 1, 4096, 192, 1.0, 128, 0), (130, 1, 4096, 0, 1.0, 128, 0), (300, 1, 2048, 64, 1.0, 64, 1),   # the norm's launch has the table
+    (64, 1, 1152, 64, 34.0, 0, 2), (3, 37, 1152, 64, 34.0, 0, 2), (2, 5, 96, 16, 1.0, 2, 1), (1, 3, 16384, 0, 1.0, 0, 0)])
+def test_embedding_in_the_first_norm(gpu, B, T, D, R, scale, dh, flavor):
+  """tnx_embed_norm against tnx_embed, tnx_norm_lora (or tnx_rmsnorm) and tnx_rope_table, bit for bit; ids outside the vocabulary included."""
+  from tunix_amd import ops
+  V, L, col, M = 77, T + 3, 2, B * T
+  table, w = bf(rnd((V, D), 601)).to(gpu), bf(rnd((D,), 602)).to(gpu)
+  a_t = bf(rnd((R, D), 603)).to(gpu) if R else None
+  ids = torch.randint(-2, V + 2, (B, L), generator=torch.Generator().manual_seed(604), dtype=torch.int32).to(gpu)
+  positions = torch.randint(0, 5000, (B, L), generator=torch.Generator().manual_seed(605), dtype=torch.int32).to(gpu)
+  timescale = (10000.0 ** (torch.arange(max(dh // 2, 1)) / max(dh // 2, 1))).to(gpu)
+  colp = torch.tensor([col], dtype=torch.int32, device=gpu)
+  outs = []
+  for fused in (False, True):
+    h, y = (torch.full((M, D), 7.0, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    t = torch.full((M, R + 16), 7.0, dtype=torch.bfloat16, device=gpu)
+    sn, cs = (torch.full((B, max(dh // 2, 1)), 7.0, device=gpu) for _ in range(2))
+    if fused:
+      ops.embed_norm(table, ids, colp, B, T, scale, h, w, y, 1e-6, flavor, a_t, t, (positions, timescale, dh, sn, cs) if dh else None)
+    else:
+      ops.embed(table, ids, colp, B, T, scale, h)
+      if R:
+        ops.norm_lora(a_t, t, w, y, 1e-6, flavor, M, D, x=h)
+      else:
+        ops.rmsnorm(h, w, y, 1e-6, flavor)
+      if dh:
+        ops.rope_table(positions, colp, B, timescale, dh, sn, cs)
+    outs.append([v.cpu() for v in (h, y, t, sn, cs)])
+  for a, b in zip(*outs):
+    assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+  assert (outs[1][1] != 7.0).any() and (not dh or (outs[1][3] != 7.0).all())
+
+
 @pytest.mark.parametrize("M,V,draw,lists", [(1, 640, False, True), (1, 640, True, False), (5, 9008, False, False), (17, 8256, True, True),
                                             (64, 640, False, True), (130, 9008, True, True), (1000, 640, False, True)])
 def test_head_enters_its_own_choice(gpu, M, V, draw, lists):

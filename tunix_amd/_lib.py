@@ -64,6 +64,13 @@ class NormLoraDesc(C.Structure):
   ]
 
 
+class EmbedDesc(C.Structure):
+  _fields_ = [
+      ("table", _p), ("V", _i64), ("ids", _p), ("ids_ld", _i64), ("col_ptr", _p), ("B", _i64), ("T", _i64), ("scale", _f32),
+      ("positions", _p), ("pos_ld", _i64), ("timescale", _p), ("dh", _i32), ("sin_out", _p), ("cos_out", _p),
+  ]
+
+
 class AttnDesc(C.Structure):
   _fields_ = [
       ("B", _i64), ("T", _i64), ("S", _i64),
@@ -309,6 +316,7 @@ SIGNATURES = {
     "tnx_rmsnorm_moe_combine": (_i32, [_p, _p, _p, _i32, _p, _p, _p, _p, _p, _i64, _i64, _f32, _i32]),
     "tnx_rmsnorm_pair": (_i32, [_p, _p, _p, _i32, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _f32, _i32]),
     "tnx_norm_lora": (_i32, [_p, C.POINTER(NormLoraDesc)]),
+    "tnx_embed_norm": (_i32, [_p, C.POINTER(EmbedDesc), C.POINTER(NormLoraDesc)]),
     "tnx_qknorm_rope_kvwrite": (_i32, [_p, C.POINTER(RopeDesc)]),
     "tnx_rope_table": (_i32, [_p, _p, _i64, _p, _i64, _p, _i32, _p, _p]),
     "tnx_attn_ws_bytes": (C.c_size_t, [_i64, _i64, _i64, _i32, _i32, _i32]),

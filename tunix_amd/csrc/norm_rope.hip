@@ -64,8 +64,34 @@ __device__ __forceinline__ void unpack8(const u32x4& p, float (&f)[8]) {
 // planes ws[z][row][:]) of a split-k linear, added in split order: the linear's own finishing
 // pass folded into the norm; kNormInRoutes -- bf16(sum_j cw[row, j] * x[row * split_k + j]) over
 // the split_k routed rows of a token, j ascending: the weighted combine of an MoE layer folded
-// into the norm (same arithmetic as moe_combine_vec_kernel).
-constexpr int kNormInRow = 0, kNormInPlanes = 1, kNormInRoutes = 2;
+// into the norm (same arithmetic as moe_combine_vec_kernel); kNormInTable -- the embedding of the row's token, x[id] * scale.
+constexpr int kNormInRow = 0, kNormInPlanes = 1, kNormInRoutes = 2, kNormInTable = 3;
+// sin / cos of angle = position / timescale[i] for the token in column *col_ptr of row b: the
+// values rope_kernel computes for the Llama rotation, once per decode step instead of per layer.
+struct RopeTable {
+  const int32_t* positions;   // null: none asked for
+  int64_t pos_ld, B;
+  const float* timescale;
+  int half;
+  float *sin_out, *cos_out;
+};
+__device__ __forceinline__ void rope_table_row(const RopeTable& r, int64_t b, int col) {
+  for (int i = threadIdx.x; i < r.half; i += blockDim.x) {
+    const float ang = __fdiv_rn((float)r.positions[b * r.pos_ld + col], r.timescale[i]);
+    r.sin_out[b * r.half + i] = sinf(ang);
+    r.cos_out[b * r.half + i] = cosf(ang);
+  }
+}
+struct EmbedSrc {
+  const int32_t* ids;
+  int64_t ids_ld;
+  const int32_t* col_ptr;
+  int64_t V;
+  uint32_t T;
+  float scale_bf;
+  RopeTable rope;
+  int64_t first_table_row;   // of the grid: its rows (rmsnorm_lora_kernel) or its work-groups from there on have a row of the rope table
+};
 struct NormRow {
   const uint16_t *x, *res_pre;
   uint16_t* h_out;
@@ -79,7 +105,13 @@ struct NormRow {
   const uint16_t* w2;
   uint16_t* y2;
   const uint16_t* cw;
+  EmbedSrc e;
 };
+__device__ __forceinline__ int64_t embed_id(const EmbedSrc& e, int64_t row) {
+  const uint32_t b = (uint32_t)row / e.T, t = (uint32_t)row - b * e.T;
+  const int64_t id = e.ids[b * e.ids_ld + (e.col_ptr ? *e.col_ptr : 0) + t];
+  return id < 0 || id >= e.V ? 0 : id;   // pad sentinels outside the vocabulary read row 0 (masked later)
+}
 // One row: writes it (WRITE) and leaves the thread's chunks of the last norm, packed, in `last` (zeros past the row's end).
 // behind(): called once every load of the row has been asked for.
 template <int MAXC, int FLAVOR, int IN, class F>
@@ -90,7 +122,7 @@ __device__ __forceinline__ void norm_row(const NormRow& n, int64_t row, bool wri
   const int64_t D = n.D, plane = n.plane;
   const float eps = n.eps;
   const int split_k = n.split_k;
-  constexpr bool PLANES = IN == kNormInPlanes, ROUTES = IN == kNormInRoutes;
+  constexpr bool PLANES = IN == kNormInPlanes, ROUTES = IN == kNormInRoutes, TABLE = IN == kNormInTable;
   const int nchunks = (int)(D / 8);
   float h[MAXC][8];
 #pragma unroll
@@ -111,6 +143,7 @@ __device__ __forceinline__ void norm_row(const NormRow& n, int64_t row, bool wri
     }
   };
   if constexpr (MAXC <= 2) fetch_weights();
+  if constexpr (TABLE) x += embed_id(n.e, row) * D;
   // Chunks are taken two at a time with every load of the pair issued before the first sum (up
   // to eight planes per chunk at once, further planes in groups of eight): the kernel is a few
   // dependent memory round trips long, and each group of loads that waits for the previous sum
@@ -138,7 +171,7 @@ __device__ __forceinline__ void norm_row(const NormRow& n, int64_t row, bool wri
           yin[cc][u] = *reinterpret_cast<const u32x4*>(
               x + (row * split_k + min(u, split_k - 1)) * D + (int64_t)min(ch, nchunks - 1) * 8);
       } else {
-        xin[cc] = *reinterpret_cast<const u32x4*>(x + o);
+        xin[cc] = *reinterpret_cast<const u32x4*>(x + (TABLE ? o - row * D : o));
       }
       if (res_pre) rin[cc] = *reinterpret_cast<const u32x4*>(res_pre + o);
     }
@@ -214,6 +247,10 @@ __device__ __forceinline__ void norm_row(const NormRow& n, int64_t row, bool wri
           for (int j = 0; j < 8; ++j) h[c][j] = rbf(h[c][j]);
         } else {
           unpack8(xin[cc], h[c]);
+          if (TABLE && n.e.scale_bf != 1.0f) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) h[c][j] = rbf(h[c][j] * n.e.scale_bf);
+          }
         }
         if (res_pre) {
           float r[8];
@@ -291,6 +328,12 @@ template <int MAXC, int FLAVOR, int IN>
 __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const NormRow n) {
   __shared__ float red[4];
   u32x4 last[MAXC];
+  if constexpr (IN == kNormInTable) {
+    if ((int64_t)blockIdx.x >= n.e.first_table_row) {
+      rope_table_row(n.e.rope, blockIdx.x - n.e.first_table_row, n.e.col_ptr ? *n.e.col_ptr : 0);
+      return;
+    }
+  }
   norm_row<MAXC, FLAVOR, IN>(n, blockIdx.x, true, red, last, [] {});
 }
 // The same with the LoRA down-projection of the row behind it (row_adapter.h); the first group of adapter columns writes the row.
@@ -301,6 +344,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   RowAdapter<MAXC, NB> ad;
   int group;
   int64_t row;
+  if constexpr (IN == kNormInTable) {
+    if ((int64_t)blockIdx.y >= n.e.first_table_row) {
+      const int64_t b = (blockIdx.y - n.e.first_table_row) * gridDim.x + blockIdx.x;
+      if (b < n.e.rope.B) rope_table_row(n.e.rope, b, n.e.col_ptr ? *n.e.col_ptr : 0);
+      return;
+    }
+  }
   if (!row_adapter_place(g, M, group, row)) return;
   norm_row<MAXC, FLAVOR, IN>(n, row, group == 0, red, last, [&] { ad.load(g, group, n.D); });
   ad.finish(g, group, row, last, sums);
@@ -319,9 +369,13 @@ template <class F>
 void with_input(int in, F f) {
   if (in == kNormInPlanes) f(std::integral_constant<int, kNormInPlanes>{});
   else if (in == kNormInRoutes) f(std::integral_constant<int, kNormInRoutes>{});
+  else if (in == kNormInTable) f(std::integral_constant<int, kNormInTable>{});
   else f(std::integral_constant<int, kNormInRow>{});
 }
-void launch_rmsnorm_vec(hipStream_t st, int64_t M, int flavor, int in, const NormRow& n) {
+void launch_rmsnorm_vec(hipStream_t st, int64_t rows, int flavor, int in, const NormRow& given) {
+  NormRow n = given;
+  n.e.first_table_row = rows;
+  const int64_t M = rows + (n.e.rope.positions ? n.e.rope.B : 0);
   with_flavor(flavor, [&](auto f) {
     with_input(in, [&](auto i) {
       constexpr int F = decltype(f)::value, IN = decltype(i)::value;
@@ -339,8 +393,11 @@ bool norm_lora_one_launch(int64_t M, int64_t D, int R) {
   if (M > 256 || D > 8 * 256 * 2) return false;
   return D > 8 * 256 ? M <= 16 && row_adapter_cols(M, R) <= 16 : row_adapter_cols(M, R) <= 32;
 }
-void launch_rmsnorm_lora(hipStream_t st, int64_t M, int flavor, int in, const NormRow& n, RowAdapterArgs g) {
-  const dim3 grid = row_adapter_grid(g, M, n.D, n.D * (in == kNormInPlanes ? 4 * n.split_k : in == kNormInRoutes ? 2 * n.split_k : 2));
+void launch_rmsnorm_lora(hipStream_t st, int64_t M, int flavor, int in, const NormRow& given, RowAdapterArgs g) {
+  NormRow n = given;
+  dim3 grid = row_adapter_grid(g, M, n.D, n.D * (in == kNormInPlanes ? 4 * n.split_k : in == kNormInRoutes ? 2 * n.split_k : 2));
+  n.e.first_table_row = grid.y;
+  if (n.e.rope.positions) grid.y += (unsigned)cdiv(n.e.rope.B, grid.x);
   with_flavor(flavor, [&](auto f) {
     with_input(in, [&](auto i) {
       constexpr int F = decltype(f)::value, IN = decltype(i)::value;
@@ -563,18 +620,7 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(const RopeArgs a) {
   }
 }
 
-// sin / cos of angle = position / timescale[i] for the token in column *col_ptr of every row: the
-// values rope_kernel computes for the Llama rotation, once per decode step instead of per layer.
-__global__ void rope_table_kernel(const int32_t* positions, int64_t pos_ld, const int32_t* col_ptr,
-                                  const float* timescale, int half, float* sin_out, float* cos_out) {
-  const int64_t b = blockIdx.x;
-  const int i = threadIdx.x;
-  if (i >= half) return;
-  const float pos = (float)positions[b * pos_ld + *col_ptr];
-  const float ang = __fdiv_rn(pos, timescale[i]);
-  sin_out[b * half + i] = sinf(ang);
-  cos_out[b * half + i] = cosf(ang);
-}
+__global__ void rope_table_kernel(const RopeTable r, const int32_t* col_ptr) { rope_table_row(r, blockIdx.x, *col_ptr); }
 
 }  // namespace
 
@@ -649,25 +695,30 @@ extern "C" int tnx_rmsnorm_pair(void* stream, const uint16_t* x, const float* ws
   return TNX_OK;
 }
 
-extern "C" int tnx_norm_lora(void* stream, const tnx_norm_lora_desc* d) {
-  TNX_REQUIRE(d, "norm_lora: null descriptor");
-  TNX_REQUIRE((d->x != nullptr) + (d->ws != nullptr) + (d->y_route != nullptr) == 1, "norm_lora: exactly one of x, ws and y_route must be given");
+// e: the rows come from a table, which `d` names as its x
+static int norm_lora(void* stream, const tnx_norm_lora_desc* d, const EmbedSrc* e) {
   TNX_REQUIRE(!d->w2 == !d->y2 && !(d->w2 && d->y_route), "norm_lora: the second norm takes w2 and y2, and rows or planes");
-  TNX_REQUIRE(d->w && d->y && d->a_t && d->t, "norm_lora: null pointer");
+  TNX_REQUIRE(d->w && d->y && (e || d->a_t) && (!d->a_t || d->t), "norm_lora: null pointer");
   const int64_t M = d->M, D = d->D;
   TNX_REQUIRE(M > 0 && D > 0 && D % 32 == 0 && D <= 8 * 256 * kNormMaxChunks, "norm_lora: D=%lld must be a multiple of 32 and <= 16384", (long long)D);
-  TNX_REQUIRE(d->R > 0 && d->R % 16 == 0 && d->t_ld >= d->R, "norm_lora: R=%d must be a multiple of 16 and <= t_ld", d->R);
+  if (d->a_t) TNX_REQUIRE(d->R > 0 && d->R % 16 == 0 && d->t_ld >= d->R, "norm_lora: R=%d must be a multiple of 16 and <= t_ld", d->R);
   TNX_REQUIRE(d->flavor >= TNX_NORM_LLAMA && d->flavor <= TNX_NORM_GEMMA3, "norm_lora: bad flavor %d", d->flavor);
   if (d->ws) TNX_REQUIRE(d->split_k >= 1, "norm_lora: split_k must be >= 1");
   if (d->y_route) TNX_REQUIRE(d->topk_w && d->k >= 1, "norm_lora: y_route needs topk_w and k >= 1");
-  const int in = d->ws ? kNormInPlanes : d->y_route ? kNormInRoutes : kNormInRow;
+  const int in = e ? kNormInTable : d->ws ? kNormInPlanes : d->y_route ? kNormInRoutes : kNormInRow;
   const int parts = d->ws ? d->split_k : d->y_route ? d->k : 0;
-  const NormRow n{d->y_route ? d->y_route : d->x, d->res_pre, d->h_out, d->w, d->res_post, d->y, D, d->eps, d->ws, parts, M * D, d->w2, d->y2, d->topk_w};
+  const NormRow n{d->y_route ? d->y_route : d->x, d->res_pre, d->h_out, d->w, d->res_post, d->y, D, d->eps, d->ws, parts, M * D, d->w2, d->y2, d->topk_w,
+                  e ? *e : EmbedSrc{}};
+  if (!d->a_t) {
+    launch_rmsnorm_vec(as_stream(stream), M, d->flavor, in, n);
+    TNX_CHECK_LAUNCH("norm_lora");
+    return TNX_OK;
+  }
   // A row's work-groups read it while the first of them writes it and each writes its adapter columns: no output may lie in an input, and t not
   // in another output either.
   const int64_t row_bytes = M * D * 2, t_bytes = ((M - 1) * d->t_ld + d->R) * 2;
   struct Range { const void* p; int64_t bytes; };
-  const Range ins[] = {{d->x, row_bytes}, {d->ws, 2 * parts * row_bytes}, {d->y_route, parts * row_bytes}, {d->res_pre, row_bytes}, {d->res_post, row_bytes}};
+  const Range ins[] = {{d->x, e ? e->V * D * 2 : row_bytes}, {d->ws, 2 * parts * row_bytes}, {d->y_route, parts * row_bytes}, {d->res_pre, row_bytes}, {d->res_post, row_bytes}};
   const Range outs[] = {{d->h_out, row_bytes}, {d->y, row_bytes}, {d->y2, row_bytes}};
   bool separate = apart(d->t, t_bytes, d->topk_w, M * parts * 2) && apart(d->t, t_bytes, d->w, D * 2) && apart(d->t, t_bytes, d->w2, D * 2);
   for (const Range& in : ins) {
@@ -685,12 +736,36 @@ extern "C" int tnx_norm_lora(void* stream, const tnx_norm_lora_desc* d) {
   return tnx_lora_down(stream, d->w2 ? d->y2 : d->y, M, D, d->a_t, d->R, d->t, d->t_ld);
 }
 
+extern "C" int tnx_norm_lora(void* stream, const tnx_norm_lora_desc* d) {
+  TNX_REQUIRE(d, "norm_lora: null descriptor");
+  TNX_REQUIRE((d->x != nullptr) + (d->ws != nullptr) + (d->y_route != nullptr) == 1, "norm_lora: exactly one of x, ws and y_route must be given");
+  return norm_lora(stream, d, nullptr);
+}
+
+// A launch less ahead of the first layer, two where the step wants a rope table: 2.8 + 3.9 us of the tiny model's step, 4.6 + 4.6 + 5.2 of 16 rows of 4096.
+extern "C" int tnx_embed_norm(void* stream, const tnx_embed_desc* e, const tnx_norm_lora_desc* d) {
+  TNX_REQUIRE(e && d, "embed_norm: null descriptor");
+  TNX_REQUIRE(e->table && e->ids && d->h_out, "embed_norm: null pointer");
+  TNX_REQUIRE(!d->x && !d->ws && !d->y_route && !d->res_pre && !d->res_post && !d->w2, "embed_norm: the rows come from the table, with one norm behind them");
+  TNX_REQUIRE(e->V > 0 && e->B > 0 && e->T > 0 && d->M == e->B * e->T && d->M < (1ll << 31), "embed_norm: bad shape");
+  RopeTable rope{};
+  if (e->sin_out) {
+    TNX_REQUIRE(e->positions && e->col_ptr && e->timescale && e->cos_out, "embed_norm: null pointer");
+    TNX_REQUIRE(e->dh % 2 == 0 && e->dh >= 2 && e->dh <= 2048, "embed_norm: bad shape");
+    rope = RopeTable{e->positions, e->pos_ld, e->B, e->timescale, e->dh / 2, e->sin_out, e->cos_out};
+  }
+  const EmbedSrc src{e->ids, e->ids_ld, e->col_ptr, e->V, (uint32_t)e->T, host_round_bf16(e->scale), rope, 0};
+  tnx_norm_lora_desc rows = *d;
+  rows.x = e->table;
+  return norm_lora(stream, &rows, &src);
+}
+
 extern "C" int tnx_rope_table(void* stream, const int32_t* positions, int64_t pos_ld, const int32_t* col_ptr,
                               int64_t B, const float* timescale, int dh, float* sin_out, float* cos_out) {
   TNX_REQUIRE(positions && col_ptr && timescale && sin_out && cos_out, "rope_table: null pointer");
   TNX_REQUIRE(B > 0 && dh % 2 == 0 && dh >= 2 && dh <= 2048, "rope_table: bad shape");
-  hipLaunchKernelGGL(rope_table_kernel, dim3((unsigned)B), dim3((unsigned)(dh / 2 < 64 ? 64 : dh / 2)), 0,
-                     as_stream(stream), positions, pos_ld, col_ptr, timescale, dh / 2, sin_out, cos_out);
+  hipLaunchKernelGGL(rope_table_kernel, dim3((unsigned)B), dim3((unsigned)(dh / 2 < 64 ? 64 : dh / 2)), 0, as_stream(stream),
+                     RopeTable{positions, pos_ld, B, timescale, dh / 2, sin_out, cos_out}, col_ptr);
   TNX_CHECK_LAUNCH("rope_table");
   return TNX_OK;
 }

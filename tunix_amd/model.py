@@ -743,15 +743,24 @@ class Runner(HeadRunner):
     M = B * T
     flavor = _NORM[cfg.family]
     emb_scale = math.sqrt(cfg.embed_dim) if cfg.family == "gemma3" else 1.0
-    ops.embed(m.embed, tokens, col_ptr, B, T, emb_scale, self.h)
     pending = 1  # split count of a down-projection whose partial planes still await their sum
+    rope = None
     if (T == 1 and self.fuse_rope and m.layers and "q_norm" not in m.layers[0]
         and _ROPE[cfg.family] == L.TNX_ROPE_LLAMA and cfg.head_dim == 128):
       # one table of this step's sines / cosines for all layers (they share theta)
-      ops.rope_table(positions, col_ptr, B, m.layers[0]["timescale"], cfg.head_dim, self.rope_sin, self.rope_cos)
-    xn_ready = False   # gemma3: the block before has already normed the residual stream into self.xn
-    t_ready = False    # ... and formed the qkv adapters' down-projection of it
+      rope = positions, m.layers[0]["timescale"], cfg.head_dim, self.rope_sin, self.rope_cos
     adapter = lambda f: f.a_t if f.has_lora else None
+    # whether the first layer's rows are already normed into self.xn (gemma3: and any layer's, by the block before) and the qkv adapters'
+    # down-projection of them formed
+    xn_ready = t_ready = False
+    if m.layers and cfg.embed_dim % 32 == 0:
+      a_t = adapter(m.layers[0]["qkv"])
+      ops.embed_norm(m.embed, tokens, col_ptr, B, T, emb_scale, self.h, m.layers[0]["attn_norm"], self.xn, cfg.norm_eps, flavor, a_t, self.t, rope)
+      xn_ready, t_ready = True, a_t is not None
+    else:
+      ops.embed(m.embed, tokens, col_ptr, B, T, emb_scale, self.h)
+      if rope is not None:
+        ops.rope_table(rope[0], col_ptr, B, *rope[1:])
     for i, ly in enumerate(m.layers):
       kv = cache.entries[i]
       if not xn_ready:

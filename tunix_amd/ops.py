@@ -198,6 +198,21 @@ def norm_lora(a_t, t, w, y, eps, flavor, M, D, x=None, ws=None, split_k=0, y_rou
   L.check(L.lib().tnx_norm_lora(_stream(), C.byref(d)), "tnx_norm_lora")
 
 
+def embed_norm(table, ids, col_ptr, B, T, scale, h, w, y, eps, flavor, a_t=None, t=None, rope=None):
+  """embed into h, rmsnorm of its rows into y and, with a_t, lora_down of these into t; rope: (positions, timescale, dh, sin_out, cos_out), a
+  decode step's table as `rope_table` forms it."""
+  e, d = L.EmbedDesc(), L.NormLoraDesc()
+  e.table, (e.V, d.D) = _ptr(table), table.shape
+  e.ids, e.ids_ld, e.col_ptr, e.B, e.T, e.scale = _ptr(ids), ids.shape[1], _ptr(col_ptr), B, T, float(scale)
+  if rope is not None:
+    positions, timescale, e.dh, sin_out, cos_out = rope
+    e.positions, e.pos_ld, e.timescale, e.sin_out, e.cos_out = _ptr(positions), positions.shape[1], _ptr(timescale), _ptr(sin_out), _ptr(cos_out)
+  d.M, d.eps, d.flavor, d.h_out, d.w, d.y = B * T, float(eps), flavor, _ptr(h), _ptr(w), _ptr(y)
+  if a_t is not None:
+    d.a_t, d.R, d.t, d.t_ld = _ptr(a_t), a_t.shape[0], _ptr(t), t.shape[1]
+  L.check(L.lib().tnx_embed_norm(_stream(), C.byref(e), C.byref(d)), "tnx_embed_norm")
+
+
 def rope_kvwrite(desc: L.RopeDesc):
   L.check(L.lib().tnx_qknorm_rope_kvwrite(_stream(), C.byref(desc)), "tnx_qknorm_rope_kvwrite")
 
