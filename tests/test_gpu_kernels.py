@@ -1871,6 +1871,18 @@ def test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul):
   assert_bf16_close(y, ref, atol=1e-5, min_equal=0.9 if mul else 0.97, what="moe gmm", ulps=3 if mul else 1)
 
 
+@pytest.mark.parametrize("E,n_tok,k,K,N,group,qtype,mul", [
+    (16, 48, 2, 128, 128, 64, Q.NF4, True),       # four rows to a kilobyte of LDS, fewer k-tiles than the ring has
+    (256, 256, 4, 128, 576, 32, Q.INT4, False),   # runs that span two blocks, work-groups of three
+    (16, 48, 2, 4480, 96, 128, Q.INT4, False),    # the most that LDS holds of sixteen rows, and beyond it the form without
+    (16, 48, 2, 5120, 96, 128, Q.INT4, False),
+    (16, 48, 2, 3072, 64, 64, Q.NF4, True),
+])
+def test_moe_gmm_rows_in_lds(gpu, E, n_tok, k, K, N, group, qtype, mul):
+  """The decode-sized grouped GEMM at the edges of its form that stages the rows."""
+  test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul)
+
+
 def test_argument_errors_raise(gpu):
   from tunix_amd import ops
   with pytest.raises(ValueError, match="K % 128"):

@@ -1,10 +1,10 @@
 // Grouped GEMM over routed tokens for decode-sized expert batches: at most 16 rows per row block,
 // i.e. a weight stream with almost no arithmetic per byte.  What such a launch costs is (a) the
 // bytes in flight towards HBM and (b) the dequantisation (two VALU instructions per weight), so
-// the kernel is built as 8 * (compute units) independent waves that each stream their share of
+// the kernel is built as 8 or 16 * (compute units) independent waves that each stream their share of
 // the packed weights without ever meeting another wave after the prologue:
 //
-//   * one persistent work-group of eight waves per compute unit copies the expert offsets and the
+//   * one persistent work-group per compute unit copies the expert offsets and the
 //     sorted routes to LDS (the only dependent global round trip of the prologue), builds the
 //     code-book table (the f16 level pairs of qgemm128.h: one v_perm_b32 per look-up address, one
 //     v_fma_mix_f32 per weight, one v_cvt_pk_bf16_f32 per pair) and a list of the non-empty
@@ -17,9 +17,10 @@
 //   * a run never spans more than two blocks (the host only picks this kernel when there are at
 //     most as many blocks as waves), so the routes of a wave's rows -- the gather of the
 //     activation fragments and the scatter of the outputs -- are looked up once, up front;
-//   * activation fragments come straight from global memory in MFMA layout (the eight waves of a
-//     work-group work on the same expert's rows, the requests meet in L1); rows the block does
-//     not have are out-of-range buffer offsets, which read zeros and move no data;
+//   * the rows of a work-group's blocks are staged in LDS, whole rows of K (STAGED: sixteen waves, four to a SIMD, which the registers that a
+//     ring of fragments took allow; the work-groups then get even shares of the items instead of whole waves' runs).  Where LDS may not hold what
+//     the routes could give a work-group, eight waves take the fragments straight from global memory in MFMA layout (the requests of a
+//     work-group meet in L1); rows the block does not have are out-of-range buffer offsets there, which read zeros and move no data;
 //   * the loop has no barrier and no memory instruction behind a branch: the counted waits on
 //     the ring are the minimum over the paths that reach them, so a tile stored only in the step
 //     that finishes it would make the waits of the steps behind it stricter than the ring needs.
@@ -32,11 +33,18 @@
 // Included by qlinear.hip after qgemm128.h.
 #pragma once
 
+// What bounds it beside the stream is the conversion (32 pairs of weights, 17 to 20 cycles each, per k-tile and SIMD: 25 us of the 45 of
+// the first line's 64 tokens; with codes that L2 holds it takes 44).  128 experts, top 8, us, fragments from memory | staged, by tokens:
+//   int4 2048 -> 2 x 768, SiLU  1: 17.5 | 14.0   16: 42.3 | 35.7   40: 45.7 | 43.4   64: 52.4 | 44.6   128: 57.9 | 48.9
+//   int4 768 -> 2048            1: 11.5 | 9.9    16: 22.0 | 21.0   40: 26.4 | 25.7   64: 27.2 | 26.8   128: 42.4 | 27.6
+//   nf4 768 -> 2048, 64 tokens 29.9 | 28.4; 8 experts, top 2, 1024 -> 2 x 1024, 16 tokens 12.0 | 9.6.
+// (Staged with eight waves: 48.1 and 28.1 for 64 tokens; rings of eight k-tiles then 50.1 and 29.1.)
 namespace {
 
 constexpr int kMoeRing = 4;                 // k-tiles in flight per wave
-constexpr int kMoeWaves = 8;                // waves per work-group
+constexpr int kMoeWaves = 8, kMoeStagedWaves = 16;   // waves per work-group
 constexpr int kMoeMaxRun = 8;               // items (tile pairs) a wave takes at most
+constexpr size_t kMoeLds = 160 * 1024;      // of a work-group: a compute unit's
 // LDS behind the table: expert offsets [E + 1], sorted routes [n_routes], the block list
 // ([0] = number of blocks, [2 + 2b] = expert, [3 + 2b] = row block), each rounded up to 16
 // bytes, then 1 KiB per wave and item of its run for finished tiles.
@@ -47,6 +55,10 @@ constexpr size_t moe16_meta_bytes(int64_t E, int64_t n_routes) {
 }
 constexpr size_t moe16_smem_bytes(int64_t E, int64_t n_routes) {
   return kBigLutBytes + moe16_meta_bytes(E, n_routes) + (size_t)kMoeWaves * kMoeMaxRun * 1024;
+}
+// ... of the staged form, `items` and `rows` to a work-group: the table only for codes that look their levels up, a place for every item, the rows
+constexpr size_t moe16_staged_bytes(bool int4, bool mul, int64_t E, int64_t n_routes, int64_t items, int64_t rows, int64_t K) {
+  return (int4 ? 0 : kBigLutBytes) + moe16_meta_bytes(E, n_routes) + (size_t)items * (mul ? 512 : 1024) + ((size_t)rows * K * 2 + 1023) / 1024 * 1024;
 }
 
 template <int I, int N, class F>
@@ -59,26 +71,24 @@ __device__ __forceinline__ void moe_static_for(F&& f) {
 
 // MUL: the SiLU(gate) * up epilogue over interleaved gate / up tiles; SPT: scale slots per k-tile
 // INT4: integer codes, converted without the table (Int4Magic in common.h; the level offsets are
-// subtracted in the scale multiply-add)
-template <bool MUL, int SPT, bool INT4>
-__global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs a, const int E) {
-  constexpr int R = kMoeRing;
+// subtracted in the scale multiply-add): the table's place is the activations' too
+template <bool MUL, int SPT, bool INT4, bool STAGED>
+__global__ __launch_bounds__((STAGED ? kMoeStagedWaves : kMoeWaves) * 64) void moe_gmm16_kernel(const QLArgs a, const int E) {
+  constexpr int R = kMoeRing, WAVES = STAGED ? kMoeStagedWaves : kMoeWaves;
+  constexpr uint32_t TILE = STAGED && MUL ? 512 : 1024;   // bytes of a finished item
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lq = lane >> 4;
   const int n_routes = (int)a.M;
-  int* offs = reinterpret_cast<int*>(smem + kBigLutBytes);
-  int* routes = reinterpret_cast<int*>(smem + kBigLutBytes + moe16_round16((size_t)(E + 1) * 4));
-  int* list = reinterpret_cast<int*>(smem + kBigLutBytes + moe16_round16((size_t)(E + 1) * 4) +
-                                     moe16_round16((size_t)n_routes * 4));
-  const uint32_t stage_lds =
-      (uint32_t)(kBigLutBytes + moe16_meta_bytes(E, n_routes)) + (uint32_t)wv * (uint32_t)(kMoeMaxRun * 1024);
+  constexpr uint32_t kMeta = INT4 && STAGED ? 0u : (uint32_t)kBigLutBytes;
+  int* offs = reinterpret_cast<int*>(smem + kMeta);
+  int* routes = reinterpret_cast<int*>(smem + kMeta + moe16_round16((size_t)(E + 1) * 4));
+  int* list = reinterpret_cast<int*>(smem + kMeta + moe16_round16((size_t)(E + 1) * 4) + moe16_round16((size_t)n_routes * 4));
   // offsets and routes -> LDS, requested first; the table is built while they are in flight
-  for (int i = tid; i <= E; i += kMoeWaves * 64) offs[i] = a.offsets[i];
-  for (int i = tid; i < n_routes; i += kMoeWaves * 64) routes[i] = a.sorted_route[i];
-  static_assert(kMoeWaves == 8, "the table is written by 512 threads");
-  if constexpr (!INT4) fill_level_table<512>(0u, tid);
+  for (int i = tid; i <= E; i += WAVES * 64) offs[i] = a.offsets[i];
+  for (int i = tid; i < n_routes; i += WAVES * 64) routes[i] = a.sorted_route[i];
+  if constexpr (!INT4) fill_level_table<WAVES * 64>(0u, tid);
   __syncthreads();
   if (wv == 0) {  // non-empty (expert, row block) pairs in expert order: a running sum over the experts
     int carry = 0;
@@ -106,13 +116,44 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs 
   const int ktiles = (int)(a.K / KTILE), tp = (int)(a.N / 32);
   const int nblocks = __builtin_amdgcn_readfirstlane(list[0]);
   const int total = nblocks * tp;
-  const int nw = (int)gridDim.x * kMoeWaves;
-  const int per = (total + nw - 1) / nw;
-  const int i0 = ((int)blockIdx.x * kMoeWaves + wv) * per, i1 = min(i0 + per, total);
-  if (i0 >= i1) return;   // (no barrier below)
+  const uint32_t stage_all = kMeta + (uint32_t)moe16_meta_bytes(E, n_routes);
+  uint32_t stage_lds, x_lds = 0;
+  int i0, i1, begF = 0, bL = 0;
+  if constexpr (STAGED) {
+    // an even share to every work-group and to its waves, the longer ones one per SIMD and turn
+    const int w0 = (int)((int64_t)total * blockIdx.x / gridDim.x), w1 = (int)((int64_t)total * (blockIdx.x + 1) / gridDim.x);
+    if (w0 >= w1) return;   // (the whole work-group)
+    const int share = (w1 - w0) / WAVES, longer = (w1 - w0) % WAVES;
+    i0 = w0 + wv * share + min(wv, longer);
+    i1 = i0 + share + (wv < longer ? 1 : 0);
+    stage_lds = stage_all + (uint32_t)(i0 - w0) * TILE;
+    x_lds = (stage_all + (uint32_t)(w1 - w0) * TILE + 15u) & ~15u;
+    // The work-group's rows, those of its blocks, lie side by side in the sorted routes: whole rows of K to LDS, 16-byte chunk c of row r in the
+    // place c ^ (r % 16) of each sixteen.
+    const int bF = w0 / tp;
+    bL = (w1 - 1) / tp;
+    const int eF = list[2 + 2 * bF], eL = list[2 + 2 * bL];
+    begF = __builtin_amdgcn_readfirstlane(offs[eF] + list[3 + 2 * bF] * 16);
+    const int rows = __builtin_amdgcn_readfirstlane(min(offs[eL + 1], offs[eL] + list[3 + 2 * bL] * 16 + 16)) - begF;
+    const u32x4 xr = raw_rsrc(a.x, (uint64_t)(a.M / a.x_div) * a.K * 2);
+    const uint32_t row_bytes = (uint32_t)a.K * 2u, chunks = row_bytes / 16u, pieces = ((uint32_t)rows * row_bytes + 1023u) / 1024u;
+    for (uint32_t p = (uint32_t)wv; p < pieces; p += WAVES) {
+      const uint32_t f = p * 64u + (uint32_t)lane, r = f / chunks, c = f - r * chunks;
+      const bool in = r < (uint32_t)rows;
+      const uint32_t src = (uint32_t)(routes[begF + (in ? (int)r : 0)] / a.x_div);
+      dma16(x_lds + p * 1024u, xr, in ? src * row_bytes + (c ^ (r & 15u)) * 16u : 0xfffffff0u, 0);
+    }
+  } else {
+    const int nw = (int)gridDim.x * WAVES;
+    const int per = (total + nw - 1) / nw;
+    i0 = ((int)blockIdx.x * WAVES + wv) * per;
+    i1 = min(i0 + per, total);
+    if (i0 >= i1) return;   // (no barrier below)
+    stage_lds = stage_all + (uint32_t)(wv * kMoeMaxRun) * TILE;
+  }
 
   // the one or two blocks of this wave's run
-  const int bA = i0 / tp, bB = min(bA + 1, nblocks - 1);
+  const int bA = min(i0, total - 1) / tp, bB = min(bA + 1, nblocks - 1);
   const int iA = bA * tp, iB = iA + tp;   // first items of the two blocks
   const int eA = __builtin_amdgcn_readfirstlane(list[2 + 2 * bA]), rbA = __builtin_amdgcn_readfirstlane(list[3 + 2 * bA]);
   const int eB = __builtin_amdgcn_readfirstlane(list[2 + 2 * bB]), rbB = __builtin_amdgcn_readfirstlane(list[3 + 2 * bB]);
@@ -140,7 +181,16 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs 
   const uint32_t ctile = (uint32_t)ktiles * 1024u, stile = (uint32_t)ktiles * (uint32_t)(16 * SPT * 2);
   const uint32_t cexp = (uint32_t)(a.codes_stride * 4), sexp = (uint32_t)(a.scales_stride * 2);
 
-  u32x4 ring_c[R][2], ring_x[R][4];
+  // where this lane finds its fragments in LDS; of a row the block does not have (its products are dropped) those of the first
+  uint32_t xA[4], xB[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int rA = begA - begF + (lm < rowsA ? lm : 0), rB = bA + 1 <= bL ? begB - begF + (lm < rowsB ? lm : 0) : rA;
+    xA[j] = x_lds + (uint32_t)rA * (uint32_t)a.K * 2u + (((uint32_t)(j * 4 + lq)) ^ ((uint32_t)rA & 15u)) * 16u;
+    xB[j] = x_lds + (uint32_t)rB * (uint32_t)a.K * 2u + (((uint32_t)(j * 4 + lq)) ^ ((uint32_t)rB & 15u)) * 16u;
+  }
+
+  u32x4 ring_c[R][2], ring_x[STAGED ? 1 : R][4];
   // (a lane's scales: one 4-byte word for two slots, one 8-byte word for four; never a register
   // the lane does not use, which the allocator would hand to something else while the load that
   // writes it is still in flight -- a wait for everything outstanding)
@@ -161,9 +211,11 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs 
     const uint32_t ss = (uint32_t)e * sexp + (uint32_t)(2 * p) * stile + (uint32_t)q_kt * (uint32_t)(16 * SPT * 2);
     const uint32_t xo = inB ? xoffB : xoffA;
     __builtin_amdgcn_sched_barrier(0);   // the loads of a step stay in this order, here and before the loop
+    if constexpr (!STAGED) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      ring_x[D][j] = __builtin_amdgcn_raw_buffer_load_b128(rx, xo, q_kt * (KTILE * 2) + j * 64, 0);
+      for (int j = 0; j < 4; ++j)
+        ring_x[D][j] = __builtin_amdgcn_raw_buffer_load_b128(rx, xo, q_kt * (KTILE * 2) + j * 64, 0);
+    }
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
       ring_c[D][nt] = __builtin_amdgcn_raw_buffer_load_b128(rc, cvoff, cs + (uint32_t)nt * ctile, kStreamOnce);
@@ -184,8 +236,18 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs 
   };
 
   int c_i = i0, c_kt = 0;
+  u32x4 xf[2][4];   // staged: the fragments of this k-tile and, asked for meanwhile, of the next
+  auto fragments = [&](u32x4 (&f)[4], int i, int kt) {
+    const bool inB = i >= iB;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f[j] = lds_ld128((inB ? xB[j] : xA[j]) + (uint32_t)kt * (KTILE * 2));
+  };
   auto consume = [&](auto Dc) {
     constexpr int D = decltype(Dc)::value;
+    if constexpr (STAGED) {
+      const bool wrap = c_kt == ktiles - 1;
+      fragments(xf[(D + 1) & 1], c_i + (wrap ? 1 : 0), wrap ? 0 : c_kt + 1);
+    }
     // group g = (k-step g / 2, column tile g % 2): scale, code word, look-ups, conversion, MFMA
     auto scale_of = [&](int g) {
       const int j = g >> 1;
@@ -230,13 +292,13 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs 
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
-      acc[g & 1] = mfma16(ring_x[D][g >> 1], bw[g & 1], acc[g & 1]);
+      acc[g & 1] = mfma16(STAGED ? xf[D & 1][g >> 1] : ring_x[STAGED ? 0 : D][g >> 1], bw[g & 1], acc[g & 1]);
       if (g + 1 < 8) conv(g + 1);
       if (g + 3 < 8) look(g + 3);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (c_kt == ktiles - 1 && c_i < i1) {   // the item's tile pair is complete (no global access in here)
-      uint16_t* stage = reinterpret_cast<uint16_t*>(smem + stage_lds + (uint32_t)(c_i - i0) * 1024u);
+      uint16_t* stage = reinterpret_cast<uint16_t*>(smem + stage_lds + (uint32_t)(c_i - i0) * TILE);
       if constexpr (MUL) {   // even tile = gate, odd tile = up: one tile of act = f(gate) * up
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -257,7 +319,19 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs 
     c_i += wrap ? 1 : 0;
   };
 
-  moe_static_for<0, R>([&](auto d) { issue(d); });
+  if constexpr (STAGED) {
+    if (i0 < i1) {
+      moe_static_for<0, R>([&](auto d) { issue(d); });
+      tnx_wait_vm(4 * R);   // (the ring's codes and scales are younger)
+    } else {
+      tnx_wait_vm(0);
+    }
+    __syncthreads();
+    if (i0 >= i1) return;
+    fragments(xf[0], c_i, 0);
+  } else {
+    moe_static_for<0, R>([&](auto d) { issue(d); });
+  }
   // whole turns of the ring, the steps past the run's end included: no branch around a load or a wait
   const int steps = (i1 - i0) * ktiles;
   for (int s = 0; s < steps; s += R) {
@@ -275,7 +349,7 @@ __global__ __launch_bounds__(kMoeWaves * 64) void moe_gmm16_kernel(const QLArgs 
     const bool inB = i >= iB;
     const int p = i - (inB ? iB : iA);
     const int rt = inB ? rfB : rfA;
-    const uint32_t src = stage_lds + (uint32_t)(i - i0) * 1024u;
+    const uint32_t src = stage_lds + (uint32_t)(i - i0) * TILE;
     if constexpr (MUL) {
       const u32x2 v = *reinterpret_cast<const __attribute__((address_space(3))) u32x2*>(
           static_cast<uintptr_t>(src + (uint32_t)(frow * 32 + fch * 8)));

@@ -984,18 +984,30 @@ bool moe16_shape(const QLArgs& a, int E, size_t codes_bytes, size_t scales_bytes
   if (max_blocks > waves || max_blocks * (a.N / 32) > waves * kMoeMaxRun) return false;
   const bool mul = a.epilogue == TNX_EPI_SILU_MUL;
   if ((uint64_t)a.M * (uint64_t)(mul ? a.N / 2 : a.N) * 2 >= (1ull << 32) || ((uintptr_t)a.y & 15) != 0) return false;
-  return moe16_smem_bytes(E, a.M) <= 160 * 1024;
+  return moe16_smem_bytes(E, a.M) <= kMoeLds;
 }
 
-template <bool MUL, int SPT, bool INT4>
-int launch_moe16_t(hipStream_t st, const QLArgs& a, int E, int cus) {
+// Whether whatever rows may fall to a work-group of the staged form fit its LDS: a run of n items is of at most (n - 2) / (items of a block) + 2 blocks.
+bool moe16_staged(const QLArgs& a, int E, bool int4, bool mul, int cus) {
+  const int64_t tp = a.N / 32, blocks = std::min<int64_t>(E, a.M) + a.M / 16, items = cdiv(blocks * tp, cus);
+  const int64_t rows = std::min<int64_t>(a.M, 16 * ((items + tp - 2) / tp + 1));
+  return moe16_staged_bytes(int4, mul, E, a.M, items, rows, a.K) <= kMoeLds;
+}
+
+template <bool MUL, int SPT, bool INT4, bool STAGED>
+int launch_moe16_k(hipStream_t st, const QLArgs& a, int E, int cus) {
   static std::once_flag once;
   static int attr_rc = TNX_OK;
-  std::call_once(once, [] { attr_rc = prepare_qgemm128(&moe_gmm16_kernel<MUL, SPT, INT4>, 160 * 1024); });
+  std::call_once(once, [] { attr_rc = prepare_qgemm128(&moe_gmm16_kernel<MUL, SPT, INT4, STAGED>, kMoeLds); });
   if (attr_rc) return attr_rc;
-  hipLaunchKernelGGL((moe_gmm16_kernel<MUL, SPT, INT4>), dim3((unsigned)cus), dim3(kMoeWaves * 64), moe16_smem_bytes(E, a.M), st, a, E);
+  hipLaunchKernelGGL((moe_gmm16_kernel<MUL, SPT, INT4, STAGED>), dim3((unsigned)cus), dim3((STAGED ? kMoeStagedWaves : kMoeWaves) * 64),
+                     STAGED ? kMoeLds : moe16_smem_bytes(E, a.M), st, a, E);
   TNX_CHECK_LAUNCH("moe_gmm16");
   return TNX_OK;
+}
+template <bool MUL, int SPT, bool INT4>
+int launch_moe16_t(hipStream_t st, const QLArgs& a, int E, int cus) {
+  return moe16_staged(a, E, INT4, MUL, cus) ? launch_moe16_k<MUL, SPT, INT4, true>(st, a, E, cus) : launch_moe16_k<MUL, SPT, INT4, false>(st, a, E, cus);
 }
 
 template <bool MUL, int SPT>
