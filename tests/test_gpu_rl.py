@@ -528,3 +528,23 @@ def test_segmented_aggregate_loss_matches_oracle(gpu, mode):
     unpacked = C.aggregate_loss(-torch.tensor([[1.5, 1.5, 1.5], [3.0, 0.0, 0.0]], device=gpu),
                                 torch.tensor([[1.0, 1, 1], [1, 0, 0]], device=gpu), mode).compute().item()
     np.testing.assert_allclose(packed, unpacked, rtol=1e-6)
+
+
+@pytest.mark.parametrize("B,T", [(1, 5), (9, 300), (130, 200)])
+def test_loss_terms_take_any_layout(gpu, B, T):
+  """Transposed, strided and 64-bit operands give the bits of contiguous 32-bit ones; advantages of any shape that holds one per row."""
+  from tunix_amd.rl import common
+  g = torch.Generator().manual_seed(B + T)
+  old, mask = -torch.rand(B, T, generator=g), (torch.rand(B, T, generator=g) < 0.7).float()
+  logp, adv = old + 0.1 * torch.randn(B, T, generator=g), torch.randn(B, generator=g)
+
+  def terms(place, adv):
+    lp, od, mk = (place(t.to(gpu)) for t in (logp, old, mask))
+    ratio, loss, clipped = common.grpo_clipped_ratio(lp, od, adv.to(gpu), 0.2)
+    metric = common.aggregate_loss(place(loss), mk, "sequence-mean-token-mean")
+    return ratio, loss, clipped, common.compute_kl_divergence(lp, od), metric.unreduced_sum, metric.denominator, metric.compute()
+
+  want = terms(lambda t: t, adv)
+  for place in (lambda t: t.t().contiguous().t(), lambda t: torch.stack([t, -t], -1)[..., 0], lambda t: t.double()):
+    for a, b in zip(want, terms(place, adv.view(B, 1))):
+      assert torch.equal(a, b)

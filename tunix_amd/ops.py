@@ -356,9 +356,13 @@ def kl_divergence(logp, ref_logp, method: int, clamp: float, out):
 
 
 def aggregate_loss(per_token_loss, mask, mode: int, norm: float, row_ws, out):
+  """row_ws None: `out` has 2 + 2 B numbers, the rows' behind the results."""
   B, T = per_token_loss.shape
+  if row_ws is None and out.numel() < 2 + 2 * B:
+    raise ValueError(f"out holds {out.numel()} numbers, not the rows' of {B} rows too")
+  rows = _ptr(out) + 8 if row_ws is None else _ptr(row_ws)
   L.check(L.lib().tnx_aggregate_loss(_stream(), _ptr(per_token_loss), _ptr(mask), B, T, mode,
-                                     float(norm), _ptr(row_ws), _ptr(out)), "tnx_aggregate_loss")
+                                     float(norm), rows, _ptr(out)), "tnx_aggregate_loss")
 
 
 def aggregate_loss_segmented(per_token_loss, mask, segment_ids, num_segments: int, mode: int, norm: float, out):
