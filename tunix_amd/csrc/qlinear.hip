@@ -987,11 +987,11 @@ bool moe16_shape(const QLArgs& a, int E, size_t codes_bytes, size_t scales_bytes
   return moe16_smem_bytes(E, a.M) <= kMoeLds;
 }
 
-// Whether whatever rows may fall to a work-group of the staged form fit its LDS: a run of n items is of at most (n - 2) / (items of a block) + 2 blocks.
+// Whether rows of x are whole 16-byte pieces, and whatever of them may fall to a work-group of the staged form fits its LDS: a run of n items is of at most (n - 2) / (items of a block) + 2 blocks.
 bool moe16_staged(const QLArgs& a, int E, bool int4, bool mul, int cus) {
   const int64_t tp = a.N / 32, blocks = std::min<int64_t>(E, a.M) + a.M / 16, items = cdiv(blocks * tp, cus);
   const int64_t rows = std::min<int64_t>(a.M, 16 * ((items + tp - 2) / tp + 1));
-  return moe16_staged_bytes(int4, mul, E, a.M, items, rows, a.K) <= kMoeLds;
+  return ((uintptr_t)a.x & 15) == 0 && moe16_staged_bytes(int4, mul, E, a.M, items, rows, a.K) <= kMoeLds;
 }
 
 template <bool MUL, int SPT, bool INT4, bool STAGED>
