@@ -1588,6 +1588,29 @@ def test_sample_commit_and_fill(gpu):
   assert buf.sum().item() == 0
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5])
+def test_head_of_the_fewest_rows(gpu, M):
+  """A row's statistics, log-probabilities and raw logits do not depend on how many rows of its tile there are."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  D, V = 256, 1040
+  x, w = bf(rnd((16, D), 701)).to(gpu), bf(rnd((V, D), 702)).to(gpu)
+  targets = torch.arange(5, 5 + 16, dtype=torch.int32, device=gpu) * 40
+  outs = []
+  for rows in (16, M):
+    ids, best, tgt, lse = (torch.full((16,), -7, dtype=t, device=gpu) for t in (torch.int32, torch.float32, torch.float32, torch.float32))
+    ent, part, part_ent = torch.zeros(16, device=gpu), torch.empty(16 * 9 * 4, device=gpu), torch.empty(16 * 9, device=gpu)
+    logits = torch.zeros(16, V, device=gpu)
+    d = L.LmHeadDesc()
+    d.M, d.D, d.V, d.x, d.w_bf16, d.part, d.temperature, d.targets = rows, D, V, x.data_ptr(), w.data_ptr(), part.data_ptr(), 0.9, targets.data_ptr()
+    d.best_id, d.best_logp, d.target_logp, d.lse = ids.data_ptr(), best.data_ptr(), tgt.data_ptr(), lse.data_ptr()
+    d.entropy, d.part_entropy, d.logits_out = ent.data_ptr(), part_ent.data_ptr(), logits.data_ptr()
+    ops.lmhead(d)
+    outs.append([t.cpu() for t in (ids, best, tgt, lse, ent, logits)])
+  for a, b in zip(*outs):
+    assert torch.equal(a[:M], b[:M]) and (b[M:] == b[M:].flatten()[0]).all()
+
+
 @pytest.mark.parametrize("B,T,D,R,scale,dh,flavor", [
     (1, 1, 256, 32, 1.0, 0, 1), (1, 1, 4096, 192, 1.0, 128, 0), (16, 1, 4096, 192, 1.0, 128, 0),   # one launch, the table's rows behind the last
     (17, 1, 4096, 192, 1.0, 128, 0), (130, 1, 4096, 0, 1.0, 128, 0), (300, 1, 2048, 64, 1.0, 64, 1),   # the norm's launch has the table
