@@ -376,6 +376,36 @@ def test_few_rows_form_the_adapters_down_projection(gpu, M, K, N, split, group, 
     assert_bf16_close(y, ref.float().bfloat16(), what=epi, atol=off)
 
 
+@pytest.mark.parametrize("off", [1, 2, 4])
+@pytest.mark.parametrize("M,K,N,split,qtype,rank,inside", [
+    (1, 512, 144, 1, Q.INT4, 0, False),       # four k-tiles
+    (16, 4224, 128, 1, Q.NF4, 64, False),     # 33: slots are filled again
+    (31, 2688, 160, 1, Q.INT4, 32, True),     # 21 of 32 rows: here too, with the adapter inside
+    (5, 1152, 272, 5, Q.NF4, 64, True),       # two per split
+    (57, 1024, 256, 8, Q.INT4, 0, False),     # four row tiles, one k-tile per split
+])
+def test_few_rows_of_any_alignment(gpu, M, K, N, split, qtype, rank, inside, off):
+  """Rows that start `off` elements behind a 16-byte boundary, which loads straight into LDS ask for: the bits of the same rows on one."""
+  from tunix_amd import ops
+  x = bf(rnd((M, K), 431)).to(gpu)
+  c, s = ops.quantize_pack(bf(rnd((K, N), 432, 0.03)).to(gpu), 64, qtype)
+  a_t, lb, t = bf(rnd((max(rank, 32), K), 433, 0.03)).to(gpu), bf(rnd((N, max(rank, 32)), 434, 0.1)).to(gpu), bf(rnd((M, 64), 435)).to(gpu)
+
+  def run(rows):
+    y = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=gpu)
+    ws = torch.full((split * M * N,), float("nan"), device=gpu) if split > 1 else None
+    kw = dict(lora_rank=rank, lora_nseg=1, lora_seg_end=[N], lora_seg_toff=[0], t=t, t_ld=64, lora_b=lb, lora_scale=1.5) if rank else {}
+    d = ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=qtype, x=rows, codes=c, scales=s, y=y, split_k=split, ws=ws, **kw)
+    ops.qlinear(d, a_frag=ops.lora_frag(a_t) if inside else None)
+    torch.cuda.synchronize()
+    return y
+
+  shifted = torch.full((M * K + 16,), float("nan"), dtype=torch.bfloat16, device=gpu)
+  assert shifted.data_ptr() % 16 == 0
+  shifted[off:off + M * K] = x.view(-1)
+  assert torch.equal(run(shifted[off:off + M * K].view(M, K)), run(x))
+
+
 def test_adapter_inside_refuses_other_shapes(gpu):
   from tunix_amd import _lib as L
   from tunix_amd import ops

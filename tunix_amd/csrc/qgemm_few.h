@@ -45,7 +45,10 @@ constexpr uint32_t kFewLds = 160u << 10, kFewMeet = 0x20000, kFewOut = 0x10000, 
 // SHORT: at most PF k-tiles per split, none of them asked for in vain.  (A load that is not needed still takes its turn in the memory pipe; with the
 // adapter's there are twice as many: 1024 -> 1152 in 8, one k-tile each, 5.8 -> 4.1 us with the adapter inside, 4096 -> 4096 in 8 7.7 -> 6.9; without
 // it the waits behind the branches cost as much as the loads, 1152 -> 1536 in 5 3.5 | 3.7.)
-template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT>
+// WHOLE: rows of x are whole 16-byte pieces, as loads straight into LDS ask for; otherwise they go by way of registers.  (A form of its own: as a branch
+// beside those loads it costs every launch 0.2 us, 0.9 % of a rollout of 16 rows.)
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT, bool WHOLE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void qgemm_few_kernel(const QLArgs a) {
   constexpr int MT = (ROWS + 15) / 16;
   constexpr uint32_t SLOT = ROWS * 256;
@@ -111,12 +114,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const uint32_t xvoff = ((uint32_t)xrow * (uint32_t)a.K + (uint32_t)((lane & 15) ^ (xrow & 15)) * 8u) * 2u;
   // k-tiles first .. first + count of this work-group into the slots from `slot` on
   auto request_x = [&](int first, int count, int slot) {
+#pragma unroll(WHOLE ? 1 : 4)
     for (int i = wv / QUADS; i < count; i += QW > 1 ? 1 : 8 / QUADS) {
       const uint32_t at = (uint32_t)(slot + i) * SLOT;
 #pragma unroll
-      for (int q = 0; q < QW; ++q)
-        dma16((INT4 || at < kBigLutBase ? at : at + (uint32_t)kBigLutBytes) + (uint32_t)(quad + 8 * q) * 1024u, rx,
-              xvoff + (uint32_t)(32 * q) * (uint32_t)a.K * 2u, (kt_begin + first + i) * (KTILE * 2));
+      for (int q = 0; q < QW; ++q) {
+        const uint32_t lds = (INT4 || at < kBigLutBase ? at : at + (uint32_t)kBigLutBytes) + (uint32_t)(quad + 8 * q) * 1024u;
+        const uint32_t voff = xvoff + (uint32_t)(32 * q) * (uint32_t)a.K * 2u, koff = (uint32_t)(kt_begin + first + i) * (KTILE * 2);
+        if constexpr (WHOLE) {
+          dma16(lds, rx, voff, (int)koff);
+        } else {
+          u32x4 v = {0, 0, 0, 0};
+          if (xrow + 32 * q < a.M) v = *reinterpret_cast<const u32x4_any*>(reinterpret_cast<const char*>(a.x) + ((uint64_t)voff + koff));
+          lds_st128(lds + (uint32_t)lane * 16u, v);
+        }
+      }
     }
   };
   request_x(0, min(n, NB * CHUNK), 0);

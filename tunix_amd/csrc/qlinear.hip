@@ -748,25 +748,25 @@ int launch_qgemm128(hipStream_t st, const QLArgs& a) {
   return a.qtype == TNX_Q_INT4 ? launch_qgemm128_as<NT, SPT, MT, true>(st, a) : launch_qgemm128_as<NT, SPT, MT, false>(st, a);
 }
 
-template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT>
+template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT, bool WHOLE>
 int launch_qgemm_few_as(hipStream_t st, const QLArgs& a) {
   static std::once_flag once;
   static int attr_rc = TNX_OK;
-  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT>, kFewLds); });
+  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT, WHOLE>, kFewLds); });
   if (attr_rc) return attr_rc;
-  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kFewLds, st, a);
+  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT, WHOLE>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kFewLds, st, a);
   TNX_CHECK_LAUNCH("qgemm_few");
   return TNX_OK;
 }
-template <int SPT, int ROWS, bool INNER, bool SHORT>
+template <int SPT, int ROWS, bool INNER, bool SHORT, bool WHOLE>
 int launch_qgemm_few_book(hipStream_t st, const QLArgs& a) {
-  return a.qtype == TNX_Q_INT4 ? launch_qgemm_few_as<SPT, true, ROWS, INNER, SHORT>(st, a) : launch_qgemm_few_as<SPT, false, ROWS, INNER, SHORT>(st, a);
+  return a.qtype == TNX_Q_INT4 ? launch_qgemm_few_as<SPT, true, ROWS, INNER, SHORT, WHOLE>(st, a) : launch_qgemm_few_as<SPT, false, ROWS, INNER, SHORT, WHOLE>(st, a);
 }
-template <int SPT, int ROWS, bool INNER>
+template <int SPT, int ROWS, bool INNER, bool WHOLE = true>
 int launch_qgemm_few_rows(hipStream_t st, const QLArgs& a) {
-  if constexpr (INNER || ROWS > 32)
-    if (a.ktiles_per_split <= 4) return launch_qgemm_few_book<SPT, ROWS, INNER, true>(st, a);
-  if constexpr (ROWS <= 32) return launch_qgemm_few_book<SPT, ROWS, INNER, false>(st, a);
+  if constexpr ((INNER && WHOLE) || ROWS > 32)
+    if (a.ktiles_per_split <= 4) return launch_qgemm_few_book<SPT, ROWS, INNER, true, WHOLE>(st, a);
+  if constexpr (ROWS <= 32) return launch_qgemm_few_book<SPT, ROWS, INNER, false, WHOLE>(st, a);
   tnx_set_error("qgemm_few: %d k-tiles per split are too many for %d rows", a.ktiles_per_split, ROWS);   // (the callers see to that)
   return TNX_EINVAL;
 }
@@ -778,6 +778,10 @@ constexpr int64_t kFewRows = 32;
 constexpr int kFewKtiles64 = 4;
 template <bool INNER>
 int launch_qgemm_few(hipStream_t st, const QLArgs& a, bool two_scales) {
+  if (((uintptr_t)a.x & 15) != 0) {   // (the widest form only, of whatever rows there are)
+    if (a.M <= 32) return two_scales ? launch_qgemm_few_rows<2, 32, INNER, false>(st, a) : launch_qgemm_few_rows<4, 32, INNER, false>(st, a);
+    return two_scales ? launch_qgemm_few_rows<2, 64, INNER, false>(st, a) : launch_qgemm_few_rows<4, 64, INNER, false>(st, a);
+  }
   if (a.M <= 8) return two_scales ? launch_qgemm_few_rows<2, 8, INNER>(st, a) : launch_qgemm_few_rows<4, 8, INNER>(st, a);
   if (a.M <= 16) return two_scales ? launch_qgemm_few_rows<2, 16, INNER>(st, a) : launch_qgemm_few_rows<4, 16, INNER>(st, a);
   if (a.M <= 32) return two_scales ? launch_qgemm_few_rows<2, 32, INNER>(st, a) : launch_qgemm_few_rows<4, 32, INNER>(st, a);
