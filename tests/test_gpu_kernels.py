@@ -406,6 +406,44 @@ def test_few_rows_of_any_alignment(gpu, M, K, N, split, qtype, rank, inside, off
   assert torch.equal(run(shifted[off:off + M * K].view(M, K)), run(x))
 
 
+@pytest.mark.parametrize("M,K,N,split,qtype,rank", [
+    (3, 1152, 272, 5, Q.NF4, 64),      # short splits
+    (16, 2176, 128, 1, Q.INT4, 32),    # a ring of k-tiles, half of the ranks
+    (32, 1024, 144, 2, Q.NF4, 32),
+    (57, 512, 128, 1, Q.NF4, 64),
+])
+def test_adapter_inside_of_infinite_rows(gpu, M, K, N, split, qtype, rank):
+  """x . A formed inside, of rows with an infinite element or with products of A near the largest number: where the rounded t of
+  a launch ahead gives an infinite result or none, so does this form; every other row keeps its bits."""
+  from tunix_amd import ops
+  sign = torch.where(torch.arange(N) % 3 == 0, -1.0, 1.0)
+  w, a, lb = rnd((K, N), 441, 0.03), rnd((rank, K), 442, 0.03), rnd((N, rank), 443, 0.1).abs() * sign[:, None]
+  w[7], a[:, 7], a[:, 8] = 0.05 * sign, 1.9921875, 1.0   # (both products of element 7 have one sign in a column)
+  c, s = ops.quantize_pack(bf(w).to(gpu), 64, qtype)
+  a_t, lb, x = bf(a).to(gpu), bf(lb).to(gpu), bf(rnd((M, K), 444)).to(gpu)
+  odd = x.clone()
+  odd[0, 7], odd[1, 7], odd[1, 8] = float("inf"), 2.0 ** 127, 1.5 * 2.0 ** 119   # (row 1: t past the largest bf16, in 32 bits finite)
+  odd[2, 7] = float("nan")
+
+  def run(rows, inside):
+    y = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=gpu)
+    ws = torch.full((split * M * N,), 7.0, device=gpu) if split > 1 else None
+    t = torch.full((M, rank), 7.0, dtype=torch.bfloat16, device=gpu)
+    if not inside:
+      ops.lora_down(rows, a_t, t, M=M)
+    ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=qtype, x=rows, codes=c, scales=s, y=y, split_k=split, ws=ws, lora_rank=rank,
+                                      lora_nseg=1, lora_seg_end=[N], lora_seg_toff=[0], t=t, t_ld=rank, lora_b=lb, lora_scale=1.5),
+                a_frag=ops.lora_frag(a_t) if inside else None)
+    torch.cuda.synchronize()
+    return y
+
+  got, ahead, plain = run(odd, True), run(odd, False), run(x, True)
+  assert torch.isposinf(ahead[0]).sum() == (sign > 0).sum() and torch.isneginf(ahead[0]).sum() == (sign < 0).sum()
+  assert torch.isinf(ahead[1]).all() and torch.isnan(ahead[2]).all()
+  assert torch.equal(got[:2], ahead[:2]) and torch.isnan(got[2]).all()
+  assert torch.equal(got[3:], plain[3:])
+
+
 def test_adapter_inside_refuses_other_shapes(gpu):
   from tunix_amd import _lib as L
   from tunix_amd import ops

@@ -35,6 +35,12 @@ namespace {
 // 128 KiB; integer codes have none).  Behind the loop the sums of gated columns meet at 128 KiB, the activated tile leaves through the table's place.
 constexpr uint32_t kFewLds = 160u << 10, kFewMeet = 0x20000, kFewOut = 0x10000, kFewScratch = 0x14000;
 
+// What the upper of a pair of bf16 leaves of v; nothing where that is infinite or no number and says it all.
+__device__ __forceinline__ float rest_of(float v, float upper) {
+  const float d = v - upper;
+  return __builtin_fabsf(d) < __builtin_inff() ? d : 0.0f;
+}
+
 // INNER: the adapter's down-projection t = x . A is formed here (a.inner_a, its fragments in order) instead of ahead of the launch: a work-group
 // multiplies the activations it holds with its k range of A (wave (rank tile, half of each k-tile): the fragments of x are there already), and its share
 // of t, as a pair of bf16 (to 2^-17 of itself), with B: t is linear, so no sum over the splits has to be waited for, nor is one rounded to bf16 on the
@@ -295,7 +301,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float v = tacc[m][i];
+        const float v = a_tile < a_tiles ? tacc[m][i] : 0.0f;   // (zeros times an infinite x are none)
         *reinterpret_cast<lds_u32*>(static_cast<uintptr_t>(T_AT + (uint32_t)a_half * T_HALF + (uint32_t)(m * 16 + lq * 4 + i) * T_LD +
                                                            (uint32_t)(a_tile * 16 + lm) * 4u)) = __float_as_uint(v);
       }
@@ -314,7 +320,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
           for (int i = 0; i < 2; ++i) {
             hi[2 * h + i] = cvt_pk_bf16(v[2 * i], v[2 * i + 1]);
-            lo[2 * h + i] = cvt_pk_bf16(v[2 * i] - bflo(hi[2 * h + i]), v[2 * i + 1] - bfhi(hi[2 * h + i]));
+            lo[2 * h + i] = cvt_pk_bf16(rest_of(v[2 * i], bflo(hi[2 * h + i])), rest_of(v[2 * i + 1], bfhi(hi[2 * h + i])));
           }
         }
         part = mfma16(lo, lb[j], part);
