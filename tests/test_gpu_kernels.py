@@ -285,8 +285,11 @@ def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank,
     (32, 2176, 384, 1, 64, Q.NF4, 64, True),     # 17
     (31, 2688, 160, 1, 128, Q.INT4, 64, True),   # 21 (20 are held)
     (24, 8192, 128, 4, 32, Q.NF4, 32, False),    # sixteen per split
-    (33, 512, 144, 1, 64, Q.NF4, 64, False),     # four row tiles, four k-tiles
+    (33, 512, 144, 1, 64, Q.NF4, 64, False),     # four row tiles: unsplit, the form of 64 x 128 tiles
     (64, 2048, 272, 8, 32, Q.INT4, 96, False),   # two per split
+    (48, 1024, 1024, 8, 64, Q.NF4, 64, False),   # one, 64 work-groups: the most that come here
+    (48, 1024, 1040, 8, 64, Q.NF4, 64, False),   # 72
+    (57, 1152, 384, 3, 128, Q.INT4, 0, False),   # three per split
 ])
 def test_few_rows_at_the_edges_of_what_lds_holds(gpu, M, K, N, split, group, qtype, rank, mul):
   """Linears of few rows against 64 bits over the same weights, both rounded to bf16.  The fp32 sum of K products of about 0.03 is off by

@@ -22,7 +22,7 @@
 //   int4 1024 -> 1152 in 8      5.0 |  3.3    5.2 |  3.7    5.2 |  3.9    5.5 |  4.7
 // Over 94 shapes (20 contractions x 5 forms of code book, group and adapter) the geometric mean is 0.80 at 1 to 16 rows and 0.88 at 17 to 32, and
 // none is slower but contractions of 64 k-tiles on eight work-groups (8192 -> 1024 unsplit, which the decoder splits: 27.4 | 29.3).  33 to 64 rows:
-// kFewKtiles64 in qlinear.hip.
+// few_shape in qlinear.hip.
 // Also slower: sixteen waves with half a k-tile each (4096 -> 28672 over one row 23.0 us), column tiles in pairs over half of the k-tiles (the
 // sums meet: 4096 -> 4096 in 8 6.1).
 //

@@ -771,11 +771,20 @@ int launch_qgemm_few_rows(hipStream_t st, const QLArgs& a) {
   return TNX_EINVAL;
 }
 constexpr int64_t kFewRows = 32;
-// 33 to 64 rows too, of few k-tiles per split: what such a call waits for is its first loads (the waves read 128 KB of fragments per k-tile: at more of
-// them the form of 64 x 128 tiles shares those better, 4 | 7 | 9 | 14 k-tiles 0.96 | 1.00 | 1.06 | 1.02 of its time at 64 rows).  33 | 64 rows, us before and
-// now: int4 1024 -> 1152 in 8 5.9 -> 5.1 | 6.0 -> 5.8, 2048 -> 5120 in 6 7.9 -> 7.4 | 8.0 -> 7.9, NF4 1152 -> 1536 in 5 6.5 -> 5.9 | 6.7 -> 6.6.  Unsplit ones of 64 rows are up
-// to 8 % slower.
+// 33 to 64 rows too, where a call is little more than its first loads: at most two k-tiles per split and a work-group for a quarter of the compute
+// units at most.  (The waves read 128 KB of fragments per k-tile, which the form of 64 x 128 tiles shares better, and each work-group fetches 64 rows
+// of its k-tiles.)  us in decode steps, that form | this one, 33, 48, 64 rows:
+//   int4, 2 k-tiles, 60 groups (1152 -> 1536 in 5)  6.4 | 5.8, -, 6.7 | 6.5      1, 64 (1024 -> 1024 in 8)   6.3 | 5.7, -, 7.3 | 6.8
+//   int4, 2, 64 (2048 -> 1024 in 8)   6.9 | 6.9, 7.3 | 7.0, 7.2 | 6.9            nf4 7.1 | 6.9, 7.1 | 7.1, 7.3 | 7.3
+//   int4, 1, 96 (1024 -> 1536 in 8)   6.8 | 6.4, 7.0 | 7.1, 7.0 | 7.7            nf4, 2, 192 7.5 | 7.9, 7.4 | 8.1, 7.5 | 9.2
+//   int4, 3, 64 (3072 -> 1024 in 8)   7.8 | 7.7, 7.9 | 8.1, 8.0 | 8.6            int4, 3, 240 (2048 -> 5120 in 6) 7.5 | 7.3, -, 7.9 | 8.2
+//   nf4, 4, 192 (4096 -> 3072 in 8)   9.1 | 9.1, 9.4 | 10.1, 9.6 | 11.4
+// With the adapter inside, up to kFewKtiles64 k-tiles of any number of groups, at 64 rows: nf4 2048 -> 2048 in 8 7.8 | 8.8 and 8192 -> 2048 in 16, the least
+// gain, 10.0 | 15.2, next to 3.7 to 6 of the launch that formed t, its gap, and 1.1 of a gate | up that leaves the planes for it.
 constexpr int kFewKtiles64 = 4;
+bool few_shape(const QLArgs& a) {
+  return a.M <= kFewRows || (a.M <= 64 && a.split_k > 1 && a.ktiles_per_split <= 2 && cdiv(a.N, 128) * a.split_k <= 64);
+}
 template <bool INNER>
 int launch_qgemm_few(hipStream_t st, const QLArgs& a, bool two_scales) {
   if (((uintptr_t)a.x & 15) != 0) {   // (the widest form only, of whatever rows there are)
@@ -1129,8 +1138,7 @@ extern "C" int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* d) {
   // in register copies that cost more than the halved LDS traffic gains.
   const bool s2 = scales_per_tile(a.group) == 2;
   if (wide_shape(a)) return s2 ? launch_qgemm_wide<2>(st, a) : launch_qgemm_wide<4>(st, a);
-  if (a.M <= kFewRows || (a.M <= 64 && a.ktiles_per_split <= kFewKtiles64 && a.split_k > 1))
-    return launch_qgemm_few<false>(st, a, s2);
+  if (few_shape(a)) return launch_qgemm_few<false>(st, a, s2);
   if (a.M <= 64) return s2 ? launch_qgemm128<2, 2, 4>(st, a) : launch_qgemm128<2, 4, 4>(st, a);
   return s2 ? launch_qgemm128<2, 2, 8>(st, a) : launch_qgemm128<2, 4, 8>(st, a);
 }
