@@ -190,11 +190,11 @@ typedef struct tnx_qlinear_desc {
 
 int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* h_desc);
 /* The same over at most tnx_qlinear_inner_rows(K, N, lora_rank, split_k) rows (0: a shape it does not take), with the adapter's down-projection formed inside:
- * desc's t is not read (tnx_splitk_finish wants one all the same), one adapter segment, no *_MUL epilogue.  t is not rounded to bf16 on the way.  a_frag: A in the order it is multiplied in,
+ * desc's t is not read, one adapter segment, no *_MUL epilogue.  t is not rounded to bf16 on the way.  a_frag: A in the order it is multiplied in,
  * bf16 [K / 32][lora_rank / 16][4][16][8]: element (g, n, q, c, i) is A[32 g + 8 q + i][16 n + c].                                      */
 int tnx_qlinear_inner(void* stream, const tnx_qlinear_desc* h_desc, const uint16_t* a_frag);
 int64_t tnx_qlinear_inner_rows(int64_t K, int64_t N, int lora_rank, int split_k);
-/* Epilogue for split_k > 1 (same desc): y = epi(sum_z ws[z]). */
+/* Epilogue for split_k > 1 (same desc, whose t is not read): y = epi(sum_z ws[z]). */
 int tnx_splitk_finish(void* stream, const tnx_qlinear_desc* h_desc);
 
 /* t[M, :R] = bf16(sum over the n_col_blocks fragment planes that tnx_qlinear_lora left in

@@ -447,6 +447,23 @@ def test_adapter_inside_of_infinite_rows(gpu, M, K, N, split, qtype, rank):
   assert torch.equal(got[3:], plain[3:])
 
 
+def test_adapter_inside_needs_no_t(gpu):
+  """A descriptor without t, which the form with the adapter inside does not read, split: the call and the pass that sums its planes."""
+  from tunix_amd import ops
+  M, K, N = 5, 1024, 256
+  x, a_t, lb = bf(rnd((M, K), 451)).to(gpu), bf(rnd((64, K), 452, 0.03)).to(gpu), bf(rnd((N, 64), 453, 0.1)).to(gpu)
+  c, s = ops.quantize_pack(bf(rnd((K, N), 454, 0.03)).to(gpu), 64, Q.NF4)
+  out = []
+  for t in (None, torch.zeros(M, 64, dtype=torch.bfloat16, device=gpu)):
+    y, ws = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=gpu), torch.full((4 * M * N,), float("nan"), device=gpu)
+    ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=Q.NF4, x=x, codes=c, scales=s, y=y, split_k=4, ws=ws, lora_rank=64, lora_nseg=1,
+                                      lora_seg_end=[N], lora_seg_toff=[0], t=t, t_ld=0 if t is None else 64, lora_b=lb, lora_scale=1.5),
+                a_frag=ops.lora_frag(a_t))
+    torch.cuda.synchronize()
+    out.append(y)
+  assert torch.equal(*out) and torch.isfinite(out[0].float()).all()
+
+
 def test_adapter_inside_refuses_other_shapes(gpu):
   from tunix_amd import _lib as L
   from tunix_amd import ops

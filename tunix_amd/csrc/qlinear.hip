@@ -1237,7 +1237,14 @@ int tnx_internal_wide_dense_grouped(hipStream_t st, int64_t n_routes, int64_t K,
   return launch_qgemm_pre_grouped(st, a);
 }
 
-extern "C" int tnx_splitk_finish(void* stream, const tnx_qlinear_desc* d) {
+extern "C" int tnx_splitk_finish(void* stream, const tnx_qlinear_desc* given) {
+  TNX_REQUIRE(given != nullptr, "splitk_finish: null descriptor");
+  tnx_qlinear_desc c = *given;
+  const tnx_qlinear_desc* d = &c;
+  if (!c.t) {   // (not read: the adapter is in the planes, and tnx_qlinear_inner takes none)
+    c.t = c.x;
+    c.t_ld = 8;
+  }
   int rc = check_desc(d);
   if (rc) return rc;
   TNX_REQUIRE(d->ws, "splitk_finish: null workspace");
