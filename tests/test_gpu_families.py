@@ -137,3 +137,15 @@ def test_gemma3_temperature_topk_sampling(gpu):
       mag = max(abs(float(logits[b, c - 1, tb[b, c]])), 1e-30)
       tol = max(4e-2, 2.0 * 2.0 ** (np.floor(np.log2(mag)) - 7))
       assert abs(lps[b, c] - float(lp_full[b, tb[b, c]])) <= tol
+
+
+def test_only_linears_of_the_layers_keep_a_second_copy_of_their_adapter(gpu):
+  """The order that few rows multiply A in inside a linear: kept for o and down, whose adapter it is, not for an lm_head, which runs a kernel of its own."""
+  from tunix_amd import config, dummy_model
+  from tunix_amd.model import QLoRAModel
+  cfg = config.tiny_qwen3(quantize_head=True, head_lora=True)
+  m = QLoRAModel(cfg, dummy_model.create_dummy_weights(cfg, seed=3), gpu)
+  assert m.head.has_lora and m.head.a_frag is None and m.head.inner_rows(1) == 0
+  for ly in m.layers:
+    assert ly["qkv"].a_frag is None and ly["gu"].a_frag is None
+    assert ly["o"].a_frag.numel() == ly["o"].a_t.numel() and ly["down"].a_frag.numel() == ly["down"].a_t.numel()

@@ -39,8 +39,10 @@ class FusedLinear:
   LoRA tensors in kernel layout."""
 
   def __init__(self, cfg: ModelConfig, weights: dict, names: list[str], device,
-               interleave2: bool = False):
+               interleave2: bool = False, head: bool = False):
+    """head: an lm_head, which `HeadRunner.run_head` runs, not `Runner.linear`."""
     self.names = names
+    self.head = head
     self.K = weights[names[0]].shape[0]
     self.widths = [weights[n].shape[1] for n in names]
     self.N = sum(self.widths)
@@ -155,7 +157,7 @@ class FusedLinear:
 
   def inner_rows(self, split_k: int) -> int:
     """Rows up to which the linear forms its adapter's down-projection itself (0: never)."""
-    return ops.qlinear_inner_rows(self.K, self.N, self.rp, split_k) if self.has_lora and len(self.names) == 1 else 0
+    return ops.qlinear_inner_rows(self.K, self.N, self.rp, split_k) if self.has_lora and len(self.names) == 1 and not self.head else 0
 
   @property
   def t_cols(self) -> int:
@@ -256,7 +258,7 @@ class QLoRAModel:
     self.head_w = None
     if not cfg.tied_embedding:
       if cfg.quantize_head:
-        self.head = FusedLinear(cfg, weights, ["lm_head"], dev)
+        self.head = FusedLinear(cfg, weights, ["lm_head"], dev, head=True)
       else:
         self.head_w = weights["lm_head"].to(dev, bf).t().contiguous()  # [V, D]
     self.layers = []
