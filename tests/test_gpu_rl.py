@@ -410,6 +410,17 @@ def test_weighted_metric_off_the_one_launch(gpu):
     assert forward_ad.unpack_dual(m.compute()).tangent.item() == 0.5
 
 
+@pytest.mark.parametrize("B,segmented", [(1, False), (62, False), (63, False), (4096, False), (300, True)])
+def test_a_metric_keeps_no_memory_of_the_rows(gpu, B, segmented):
+  """What a metric's two numbers keep alive is at most the 512 bytes that they would take alone."""
+  from tunix_amd.rl import common as C
+  x, mask = torch.randn(B, 5, device=gpu), torch.ones(B, 5, device=gpu)
+  kw = dict(segment_ids=torch.ones(B, 5, dtype=torch.int32, device=gpu), num_segments=1) if segmented else {}
+  m = C.aggregate_loss(x, mask, "token-mean", **kw)
+  assert m.unreduced_sum.untyped_storage().nbytes() <= 512
+  torch.testing.assert_close(m.unreduced_sum.double(), x.double().sum(), rtol=1e-5, atol=1e-5 * 5 * B)
+
+
 def test_aggregate_loss_argument_errors(gpu):
   from tunix_amd.rl import common as C
   x, k = torch.ones(2, 3, device=gpu), torch.ones(2, 3, device=gpu)

@@ -255,8 +255,10 @@ def aggregate_loss(per_token_loss: torch.Tensor, completion_mask: torch.Tensor, 
   B, T = per_token_loss.shape
   min_denom = 1e-6 if loss_agg_mode in ("seq-mean-token-sum", "sequence-mean-token-sum-norm") else 1.0
   loss, mask = _fp32(per_token_loss), _fp32(completion_mask)
-  # (behind the sum and its weight: the rows')
-  out = (torch.empty if B and T else torch.zeros)(2 + 2 * B, dtype=torch.float32, device=loss.device)
+  # Of few rows the kernel's numbers for each lie behind the sum and its weight, in the 512 bytes that the allocator gives these anyway (an
+  # allocation less); more would stay as long as the metric does.
+  behind = segment_ids is None and B <= 62
+  out = (torch.empty if B and T else torch.zeros)(2 + 2 * B if behind else 2, dtype=torch.float32, device=loss.device)
   if segment_ids is not None:
     if num_segments is None:
       raise ValueError("num_segments must be provided when segment_ids is not None.")
@@ -284,7 +286,8 @@ def aggregate_loss(per_token_loss: torch.Tensor, completion_mask: torch.Tensor, 
   elif loss_agg_mode == "sequence-mean-token-sum-norm":
     norm = _check_get_norm(kwargs, B)
   if B and T:
-    ops.aggregate_loss(loss, mask, ops.AGG_MODES[loss_agg_mode], norm, None, out)
+    rows = None if behind else torch.empty(B, 2, dtype=torch.float32, device=loss.device)
+    ops.aggregate_loss(loss, mask, ops.AGG_MODES[loss_agg_mode], norm, rows, out)
   elif loss_agg_mode == "sequence-mean-token-sum-norm":
     out[1] = norm
   return _metric(out, min_denom)
