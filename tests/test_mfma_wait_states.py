@@ -1,10 +1,11 @@
-"""Wait states around the MFMAs that are written in assembly (qgemm_pre.h, attention.hip), in the listing of the built library.
+"""Wait states around vector instructions that are written in assembly, in the listing of the built library: the MFMAs of qgemm_pre.h, and the
+maxima of attention.hip, which lane swaps read.
 
 The compiler does not look inside assembly: it keeps no distance between such an MFMA and the vector instructions that it places around
-it itself (copies of an operand, reads of a finished accumulator).  Required, in instruction slots of which `s_nop N` is N + 1:
-two between a vector write and an MFMA that reads it, eight between a 16x16x32 bf16 MFMA (four passes) and anything else that
-reads or overwrites its result, three until its addend's registers are overwritten.  These are the distances that the compiler
-keeps around its own MFMAs of this shape.
+it itself (copies of an operand, reads of a finished accumulator), nor between such a maximum and a swap.  Required, in instruction slots of
+which `s_nop N` is N + 1: two between a vector write and an MFMA that reads it, eight between a 16x16x32 bf16 MFMA (four passes) and anything
+else that reads or overwrites its result, three until its addend's registers are overwritten; two between a vector write and a permlane swap
+of the register.  These are the distances that the compiler keeps around its own instructions.
 """
 import os
 import re
@@ -18,7 +19,7 @@ from tunix_amd import _lib
 
 OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
 KERNELS = ("qgemm_pre_kernel", "attn_wg_kernel")
-VALU_TO_MFMA, MFMA_TO_OTHER, ADDEND_TO_WRITE = 2, 8, 3
+VALU_TO_MFMA, MFMA_TO_OTHER, ADDEND_TO_WRITE, VALU_TO_SWAP = 2, 8, 3, 2
 
 LINE = re.compile(r"^\s+([a-z_]\w+)\s*(.*?)\s*//\s*([0-9A-Fa-f]+):")
 TARGET = re.compile(r"<[^>+]+(?:\+0x([0-9a-f]+))?>\s*$")
@@ -92,6 +93,8 @@ def too_close(code):
           need = ADDEND_TO_WRITE
       elif p.mfma and c.mfma and p.writes & c.ab:
         need = MFMA_TO_OTHER
+      elif c.op.startswith("v_permlane") and p.valu and p.writes & touches:
+        need = VALU_TO_SWAP
       if slots < need:
         found.append((slots, need, p.text, c.text))
       if slots + p.slots < MFMA_TO_OTHER:
@@ -125,6 +128,7 @@ def test_wait_states_around_assembly_mfmas(listings, kernel):
   for name, text in mine.items():
     code = parse(text)
     assert sum(c.mfma for c in code) >= 32, name
+    assert kernel != "attn_wg_kernel" or sum(c.op.startswith("v_permlane") for c in code) >= 4, name
     assert not too_close(code), (name, too_close(code)[:3])
 
 
@@ -140,6 +144,10 @@ def test_wait_states_around_assembly_mfmas(listings, kernel):
     ("accumulators in turn", ["v_mfma_f32_16x16x32_bf16 a[0:3], v[4:7], v[8:11], a[0:3]"] * 3, 0),
     ("operand reloaded", ["v_mfma_f32_16x16x32_bf16 a[0:3], v[4:7], v[8:11], a[0:3]", "ds_read_b128 v[4:7], v20"], 0),
     ("addend reused", ["v_mfma_f32_16x16x32_bf16 v[0:3], v[4:7], v[8:11], v[12:15]", "s_nop 1", "v_mov_b32_e32 v12, v40"], 1),
+    ("swap of a maximum", ["v_max_f32 v8, v1, v2", "v_permlane16_swap_b32_e32 v8, v9"], 1),
+    ("swap with its copy", ["v_max3_f32 v8, v1, v2, v3", "v_mov_b32_e32 v9, v8", "s_nop 0", "v_permlane32_swap_b32_e32 v8, v9"], 1),
+    ("the same with its wait", ["v_max3_f32 v8, v1, v2, v3", "v_mov_b32_e32 v9, v8", "s_nop 1", "v_permlane32_swap_b32_e32 v8, v9"], 0),
+    ("swap of other registers", ["v_max_f32 v8, v1, v2", "v_permlane16_swap_b32_e32 v10, v9"], 0),
     ("round a loop", ["v_mfma_f32_16x16x32_bf16 a[0:3], v[4:7], v[8:11], a[0:3]", "v_add_u32_e32 v4, v20, v21",
                       "s_cbranch_scc1 65533 // 0000000000000008: BF85FFFD <f>"], 1),
 ])
