@@ -278,6 +278,15 @@ def test_key_chunks_of_a_decode_step(groups, S, head_dim, chunks):
   assert Runner._key_chunks(groups, S, head_dim) == chunks
 
 
+@pytest.mark.parametrize("groups,S,head_dim,chunks", [
+    (1, 256, 128, 1), (1, 257, 128, 3), (128, 256, 128, 1), (128, 257, 128, 2), (1, 384, 64, 1), (1, 385, 64, 4), (128, 384, 64, 1), (128, 385, 64, 2),
+    (1, 256, 256, 2), (64, 288, 256, 3), (256, 1025, 128, 2), (200, 3000, 256, 6)])
+def test_key_chunks_of_a_decode_step_without_an_adapter_behind(groups, S, head_dim, chunks):
+  """Short contexts are not cut where the merging pass would have nothing else to do; longer ones as ever."""
+  from tunix_amd.model import Runner
+  assert Runner._key_chunks(groups, S, head_dim, adapter_behind=False) == chunks
+
+
 @pytest.mark.parametrize("groups,S,width,chunks", [
     (1, 4000, 256, 32), (40, 300, 512, 4), (40, 300, 256, 1), (60, 1000, 512, 4), (85, 2500, 512, 3), (86, 2500, 512, 5), (102, 1025, 512, 5), (96, 1024, 512, 2),
     (103, 2500, 512, 2), (128, 4000, 256, 2), (129, 2500, 512, 3), (129, 1024, 512, 1), (171, 1500, 512, 4), (171, 1500, 256, 1), (171, 2500, 256, 4),
