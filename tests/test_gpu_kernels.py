@@ -212,25 +212,28 @@ def test_qlinear_lora_matches_oracle(gpu, M, K, N, group, qtype, r, split):
 
 
 @pytest.mark.parametrize("M,K,N,split,group,qtype,rank,nseg,epi", [
-    (1, 512, 128, 1, 64, Q.INT4, 64, 1, "store"),         # one row of int4: four k-tiles, half a turn of the four-way form
+    (1, 512, 128, 1, 64, Q.INT4, 64, 1, "store"),         # one row of int4, a turn of the ring
     (3, 1280, 208, 1, 32, Q.NF4, 32, 1, "residual"),      # a last column block of five tiles, four scales per k-tile
     (8, 3584, 512, 3, 64, Q.INT4, 64, 3, "store"),        # 28 k-tiles in splits of 10, 10, 8; three adapter segments
     (4, 1792, 512, 2, 64, Q.NF4, 64, 1, "residual"),      # seven per split: two turns less one
     (5, 2176, 768, 1, 128, Q.NF4, 64, -1, "silu"),        # 17 k-tiles, gate | up with the next adapter's planes
     (7, 1024, 25600, 1, 64, Q.INT4, 64, -1, "gelu"),      # eight k-tiles, work-groups for most of the device
-    (9, 2048, 12288, 1, 64, Q.NF4, 0, 1, "f32"),          # 16 k-tiles: the two-way form's first
+    (9, 2048, 12288, 1, 64, Q.NF4, 0, 1, "f32"),          # 16 k-tiles of sixteen rows
     (16, 3712, 384, 2, 64, Q.INT4, 96, 1, "store"),       # 15 and 14; an adapter of more than 64 ranks
     (12, 4096, 320, 2, 256, Q.NF4, 64, -1, "gelu"),       # sixteen per split
     (16, 2304, 8192, 1, 64, Q.NF4, 64, -1, "silu"),       # eighteen
+    (20, 1280, 208, 1, 32, Q.INT4, 64, 1, "f32"),         # two row tiles
+    (32, 2688, 512, 3, 64, Q.NF4, 64, 3, "residual"),     # seven per split
+    (27, 1536, 768, 1, 128, Q.INT4, 64, -1, "gelu"),
 ])
 def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank, nseg, epi):
-  """At most 16 rows (activations straight from memory, sums of the k slices at the end) against the same rows
-  in a call of 24 (activations through LDS).  Same products; a column's fp32 sum of K terms in another order, so a
+  """At most 32 rows (a column tile per wave, all activations in LDS) against the same rows in a call of 72, which runs on another kernel (tiles of
+  128 x 128, the waves sharing a k-tile behind a barrier).  Same products; a column's fp32 sum of K terms in another order, so a
   rounded result may be the neighbouring bf16 value."""
   from tunix_amd import _lib as L
   from tunix_amd import ops
   mul = epi in ("silu", "gelu")
-  x, t, res = bf(rnd((24, K), 111)).to(gpu), bf(rnd((24, 320), 112)).to(gpu), bf(rnd((24, N), 113)).to(gpu)
+  x, t, res = bf(rnd((72, K), 111)).to(gpu), bf(rnd((72, 320), 112)).to(gpu), bf(rnd((72, N), 113)).to(gpu)
   c, s = ops.quantize_pack(bf(rnd((K, N), 114, 0.03)).to(gpu), group, qtype, mul)
   lb = bf(rnd((N, max(rank, 32)), 115, 0.1)).to(gpu)
   ends = [N] if nseg < 2 else [N // 2, N * 3 // 4 // 16 * 16, N][:nseg]
@@ -257,7 +260,7 @@ def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank,
     torch.cuda.synchronize()
     return y, tn
 
-  (few, tf), (many, tm) = run(M), run(24)
+  (few, tf), (many, tm) = run(M), run(72)
   # (magnitude of a result's terms: gated products and sums with a residual are rounded more than once)
   ulps = 3 if mul else 1
   if epi == "f32":
@@ -287,6 +290,9 @@ def test_few_rows_equal_the_shared_form(gpu, M, K, N, split, group, qtype, rank,
     (24, 8192, 128, 4, 32, Q.NF4, 32, False),    # sixteen per split
     (33, 512, 144, 1, 64, Q.NF4, 64, False),     # four row tiles: unsplit, the form of 64 x 128 tiles
     (64, 2048, 272, 8, 32, Q.INT4, 96, False),   # two per split
+    (5, 1152, 144, 8, 64, Q.NF4, 64, False),     # nine k-tiles in eight splits of two: three splits of none
+    (16, 4480, 128, 8, 64, Q.INT4, 64, False),   # 35 in eight of five: one of none
+    (40, 1152, 144, 8, 64, Q.NF4, 64, False),
     (48, 1024, 1024, 8, 64, Q.NF4, 64, False),   # one, 64 work-groups: the most that come here
     (48, 1024, 1040, 8, 64, Q.NF4, 64, False),   # 72
     (57, 1152, 384, 3, 128, Q.INT4, 0, False),   # three per split
@@ -349,6 +355,9 @@ def test_few_rows_at_the_edges_of_what_lds_holds(gpu, M, K, N, split, group, qty
     (33, 384, 144, 1, 64, Q.NF4, 64, "store"),       # four row tiles, three k-tiles
     (64, 1152, 384, 3, 128, Q.INT4, 32, "store"),    # three per split
     (57, 512, 272, 1, 32, Q.NF4, 64, "residual"),    # four
+    (5, 1152, 144, 8, 64, Q.NF4, 64, "store"),       # nine k-tiles in eight splits of two: three splits of none
+    (16, 4480, 128, 8, 64, Q.INT4, 32, "store"),     # 35 in eight of five: one of none
+    (40, 1152, 144, 8, 64, Q.INT4, 64, "f32"),
 ])
 def test_few_rows_form_the_adapters_down_projection(gpu, M, K, N, split, group, qtype, rank, epi):
   """y = x . W + 1.5 (x . A) . B with x . A formed inside, against 64 bits: x . A is a pair of bf16, 2^-17 of itself off, so the result is the
@@ -697,11 +706,12 @@ def test_qlinear_invariants(gpu):
   assert torch.equal(run(w * 4.0), base * 4.0)
 
 
+@pytest.mark.parametrize("M", [1, 8, 16, 32, 40])
 @pytest.mark.parametrize("epi", ["silu", "gelu", "residual"])
-def test_qlinear_epilogues(gpu, epi):
+def test_qlinear_epilogues(gpu, epi, M):
   from tunix_amd import _lib as L
   from tunix_amd import ops
-  M, K, F, g = 40, 512, 256, 64
+  K, F, g = 512, 256, 64
   x = rnd((M, K), 8)
   if epi == "residual":
     w = rnd((K, F), 9, 0.02)
@@ -1920,7 +1930,7 @@ def test_moe_route_sort_gmm_combine(gpu, M, E, k, D, F):
     (8, 64, 2, 384, 96, 64, Q.NF4, False),        # 16 rows per expert on average: the 32-row tile kernel, whose
     (8, 128, 2, 256, 96, 128, Q.INT4, False),     # activation rows are gathered straight into LDS; 32: its 64-row form
 ])
-def test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul):
+def test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul, off=0):
   """The grouped GEMM alone, on routes built by hand: experts with no rows, with one row, with
   exactly one row block and with more (several row blocks of one expert), gathered through a
   shuffled route order; k-tile counts below the streaming kernel's ring depth; both code books,
@@ -1969,7 +1979,8 @@ def test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul):
   y = torch.full((n_routes, ncol), 7.0, dtype=torch.bfloat16, device=gpu)
   d = L.MoeGmmDesc()
   d.n_routes, d.E, d.k, d.K, d.N, d.group, d.qtype = n_routes, E, k, K, N, group, qtype
-  gx = bf(x).to(gpu)
+  buf = torch.zeros(x.numel() + 8, dtype=torch.bfloat16, device=gpu)   # (on a boundary; x starts `off` elements behind it)
+  gx = buf[off:off + x.numel()].view(x.shape).copy_(x)
   d.x, d.x_div, d.codes, d.scales = gx.data_ptr(), x_div, gc.data_ptr(), gs.data_ptr()
   go, gr = torch.from_numpy(offs).to(gpu), torch.from_numpy(sorted_route).to(gpu)
   d.offsets, d.sorted_route = go.data_ptr(), gr.data_ptr()
@@ -1982,16 +1993,21 @@ def test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul):
   assert_bf16_close(y, ref, atol=1e-5, min_equal=0.9 if mul else 0.97, what="moe gmm", ulps=3 if mul else 1)
 
 
-@pytest.mark.parametrize("E,n_tok,k,K,N,group,qtype,mul", [
-    (16, 48, 2, 128, 128, 64, Q.NF4, True),       # four rows to a kilobyte of LDS, fewer k-tiles than the ring has
-    (256, 256, 4, 128, 576, 32, Q.INT4, False),   # runs that span two blocks, work-groups of three
-    (16, 48, 2, 4480, 96, 128, Q.INT4, False),    # the most that LDS holds of sixteen rows, and beyond it the form without
-    (16, 48, 2, 5120, 96, 128, Q.INT4, False),
-    (16, 48, 2, 3072, 64, 64, Q.NF4, True),
+@pytest.mark.parametrize("E,n_tok,k,K,N,group,qtype,mul,off", [
+    (16, 48, 2, 128, 128, 64, Q.NF4, True, 0),        # four rows to a kilobyte of LDS, fewer k-tiles than the ring has
+    (256, 256, 4, 128, 576, 32, Q.INT4, False, 0),    # runs that span two blocks, work-groups of three
+    (16, 48, 2, 4992, 96, 128, Q.INT4, False, 0),     # (256 compute units) the most that LDS holds of sixteen rows, and beyond it the form without
+    (16, 48, 2, 5120, 96, 128, Q.INT4, False, 0),
+    (16, 48, 2, 2944, 64, 64, Q.NF4, True, 0),        # the same next to a table of levels
+    (16, 48, 2, 3072, 64, 64, Q.NF4, True, 0),
+    (256, 256, 4, 2304, 32, 128, Q.INT4, False, 0),   # of two blocks
+    (256, 256, 4, 2432, 32, 128, Q.INT4, False, 0),
+    (16, 48, 2, 512, 256, 128, Q.INT4, True, 1),      # rows off a 16-byte boundary: the form without
+    (16, 48, 2, 512, 256, 64, Q.NF4, False, 4),
 ])
-def test_moe_gmm_rows_in_lds(gpu, E, n_tok, k, K, N, group, qtype, mul):
+def test_moe_gmm_rows_in_lds(gpu, E, n_tok, k, K, N, group, qtype, mul, off):
   """The decode-sized grouped GEMM at the edges of its form that stages the rows."""
-  test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul)
+  test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul, off)
 
 
 def test_argument_errors_raise(gpu):
