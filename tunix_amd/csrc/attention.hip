@@ -987,8 +987,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 // the next blocks in flight.  Every wave computes exactly the blocks attn_tiles_kernel would give it, in the same order
 // with the same arithmetic: outputs are bit-identical.
 //
-// What bounds it is vector work and the waits between its steps: per score 9 lane-instructions (two roundings to bf16 with a scale between
-// them, maximum, exponential, sum, rounding of P) against half a clock of matrix pipe.  So the tiles of a wave run through one straight line of
+// What bounds it is vector work and the waits between its steps: per score 11 lane-instructions in the straight line of the loop
+// (two roundings to bf16 with a scale between them, maximum, exponential, sum, rounding of P; 9 without a scale), 16.7 by counters with masks, rescaling,
+// addresses and the two matrix instructions (2 x 6144 positions: the vector unit at work for 72 % of the cycles, the matrix pipe for 32 %).  So the tiles of a wave run through one straight line of
 // code, whose chains hide each other's latency, with two such work-groups per compute unit; the values leave LDS transposed
 // (ds_read_tr: no packing of rows by the vector unit); maxima cross the lanes in registers (permlane swaps) instead of through LDS; O is kept
 // transposed (P.V formed as V^T . P^T: the same operand registers with the operands exchanged), so that a query's rescaling
@@ -996,6 +997,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 // differs; and head_dim 128 meets at a barrier every second block.
 // 32 heads of 128 over 8 kv heads, us before (values rounded in pairs by the vector unit, a barrier per block) and now:
 //   2 x 6144 positions 895 -> 826 (691 -> 750 TFLOP/s)   3 x 2900: 337 -> 311   13 x 1024: 221 -> 208   7 x 1023 over 4: 135 -> 132
+//   (3 x 2900 inside a pass, under the clock that its GEMMs leave: 434 -> 377 to 407)
 //   64 x 256: 119.5 -> 119.5   16 x 128: 16.3 -> 15.6    head_dim 256, 4 heads over 1: 3 x 3000 135 -> 116, 64 x 256 40.8 -> 39.2
 // Two blocks in one line of code (both blocks' scores, then both softmaxes, then both blocks' values): 1030 for the first.
 typedef uint32_t __attribute__((address_space(3))) lds_word_t;

@@ -33,8 +33,9 @@
 // Included by qlinear.hip after qgemm128.h.
 #pragma once
 
-// What bounds it beside the stream is the conversion (32 pairs of weights, 17 to 20 cycles each, per k-tile and SIMD: 25 us of the 45 of
-// the first line's 64 tokens; with codes that L2 holds it takes 44).  128 experts, top 8, us, fragments from memory | staged, by tokens:
+// What bounds it beside the stream is the conversion (32 pairs of weights per k-tile and wave, by counters 5.6 vector instructions or 22 cycles each: some
+// 25 us of the 45 of the first line's 64 tokens, which have vector instructions at work for 76 % of their cycles; with codes that L2 holds it takes
+// 44).  128 experts, top 8, us, one shape after another, fragments from memory | staged, by tokens (64 of them inside a rollout: 48.3 | 44.2 and 28.0 | 27.7):
 //   int4 2048 -> 2 x 768, SiLU  1: 17.5 | 14.0   16: 42.3 | 35.7   40: 45.7 | 43.4   64: 52.4 | 44.6   128: 57.9 | 48.9
 //   int4 768 -> 2048            1: 11.5 | 9.9    16: 22.0 | 21.0   40: 26.4 | 25.7   64: 27.2 | 26.8   128: 42.4 | 27.6
 //   nf4 768 -> 2048, 64 tokens 29.9 | 28.4; 8 experts, top 2, 1024 -> 2 x 1024, 16 tokens 12.0 | 9.6.

@@ -2,13 +2,14 @@
 // wave a column tile of 16 over the whole of it.
 //
 // What bounds it is the launch and the round trip to memory, then the conversion of the codes: five instructions per pair of weights and lane
-// (address, look-up, two products, rounding), of which a compute unit finishes a k-tile (8192 pairs) in 0.36 us or so, looked up, converted and
+// (address, look-up, two products, rounding; by counters over 4096 -> 28672 and 16 rows 5.1 of the vector unit and 1.3 of
+// LDS, the vector unit at work for 49 % of the launch's cycles), of which a compute unit finishes a k-tile (8192 pairs) in 0.36 us or so, looked up, converted and
 // multiplied, where vector instructions alone would take 0.28; 4096 -> 28672 has 32 of them per unit, 11.5 of its 18 us, and its 62 MB of codes
 // and scales take some 11 us.  So:
 //   * the activations, which all waves share, are requested once, as whole kilobytes straight into LDS, ahead of everything else.  (As fragments
 //     from memory, 16 bytes of 16 rows a load, they come at a third of that rate and once per wave: the first loads of 4096 -> 28672 over 16 rows
 //     took 6 us to be asked for, now 2.)  There is no barrier in the loop as long as LDS holds them, up to 12 to 80 k-tiles by rows and code book;
-//   * a wave has a column tile of its own over the whole k range: no sums to exchange, and little code (8 KB; a work-group's first pass over its
+//   * a wave has a column tile of its own over the whole k range: no sums to exchange, and little code (9 to 10 KB up to 16 rows; a work-group's first pass over its
 //     instructions is part of every launch: the same kernel with six k-tiles in flight and a copy of the loop for the tiles left, 22 KB, is
 //     0.5 to 1 us slower at every size, with three tiles or two at long contractions 0.2 and 5 us).
 // us, before (activations as fragments from memory, or through LDS behind a barrier per k-tile) | now, weights from HBM, NF4 of group 64 with an
