@@ -155,7 +155,7 @@ int tnx_dense_expand(void* stream, const uint16_t* w_bf16, int64_t K, int64_t N,
 typedef struct tnx_qlinear_desc {
   int64_t M, K, N;          /* N counts packed columns (after interleave2 it is 2*F)        */
   int group, qtype;
-  const uint16_t* x;        /* bf16 [M,K]                                                   */
+  const uint16_t* x;        /* bf16 [M,K], on a 16-byte boundary (calls of up to 32 rows take any) */
   const uint32_t* codes;    /* QW codes                                                     */
   const uint16_t* scales;   /* QW scales                                                    */
   /* LoRA (optional: lora_rank == 0 disables). t = bf16(x . A) comes from tnx_lora_down.    */
