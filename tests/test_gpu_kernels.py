@@ -2667,6 +2667,37 @@ def test_many_rows_experts_from_expanded_copies(gpu, K, N, counts):
     assert ((y[route[a0:a1].long()].double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()
 
 
+@pytest.mark.parametrize("E,x_div", [(1, 3), (64, 1), (65, 2), (256, 1), (257, 3), (520, 4)])
+def test_many_rows_experts_are_found_among_any_number(gpu, E, x_div):
+  """The search for a tile's expert, 256 of them at a time, and the rows of routes for divisors that are and are no powers of two: most experts
+  without a row, some with several blocks, the first and the last with some."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  K, N = 128, 256
+  rng = np.random.default_rng(E)
+  counts = np.where(rng.random(E) < 0.6, 0, rng.integers(1, 300, size=E))
+  counts[0], counts[-1] = 130, 257
+  counts[0] += -int(counts.sum()) % x_div
+  n = int(counts.sum())
+  g = torch.Generator(device=gpu).manual_seed(n)
+  x = torch.randn(n // x_div, K, generator=g, device=gpu).bfloat16()
+  w = (torch.randn(E, N, K, generator=g, device=gpu) * K ** -0.5).bfloat16()
+  bank = torch.stack([ops.dense_expand(e) for e in w])
+  route = torch.randperm(n, generator=torch.Generator().manual_seed(2)).to(torch.int32).to(gpu)
+  offsets = torch.tensor([0] + [int(v) for v in np.cumsum(counts)], dtype=torch.int32, device=gpu)
+  y = torch.full((n, N), float("nan"), dtype=torch.bfloat16, device=gpu)
+  d = L.DenseDesc()
+  d.M, d.K, d.N, d.dtype, d.batch, d.split_k = n, K, N, ops.DTYPES[torch.bfloat16], 1, 1
+  d.x, d.ldx, d.w, d.w_stride, d.epilogue, d.y, d.ldy = x.data_ptr(), K, bank.data_ptr(), bank[0].numel(), L.TNX_EPI_STORE, y.data_ptr(), N
+  d.n_experts, d.x_div, d.offsets, d.sorted_route = E, x_div, offsets.data_ptr(), route.data_ptr()
+  ops.dense_linear(d)
+  for e, (a0, a1) in enumerate(zip(offsets.tolist()[:-1], offsets.tolist()[1:])):
+    at = route[a0:a1].long()
+    xe, we = x[at // x_div].double(), w[e].double()
+    want = xe @ we.T
+    assert ((y[at].double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()
+
+
 @pytest.mark.parametrize("M,counts_scale,K,N", [(36, 1, 256, 512), (320, 1, 256, 512), (333, 2, 256, 512), (2601, 1, 4096, 2048)])
 @pytest.mark.parametrize("qtype", [Q.INT4, Q.NF4])
 def test_moe_from_the_experts_copies(gpu, M, counts_scale, K, N, qtype):

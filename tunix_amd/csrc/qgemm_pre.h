@@ -78,6 +78,17 @@ constexpr bool pre_mul(int kind) { return kind == kPreSilu || kind == kPreGelu |
 // the delta is summed onto the accumulators directly; kLoraScaled: any scale.
 constexpr int kLoraInPlace = 1, kLoraScaled = 2;
 
+// sum over the lanes up to and with each one, by DPP: one, two, four, eight lanes on in a row of sixteen, the last lane of each row and of the lower half on
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
 template <int RT, bool GROUPED, int KIND, int LORA>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(RT == 16 ? 1 : RT == 8 ? 2 : 3, RT == 16 ? 1 : RT == 8 ? 2 : 3)))
@@ -89,7 +100,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   const int wn = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lq = lane >> 4;
   const int tiles_m = (int)((a.M + ROWS - 1) / ROWS), tiles_n = (int)((a.N + kWideCols - 1) / kWideCols);
-  int mtile, ntile, expert = 0, m_end = 0;
+  int mtile, ntile, expert = 0, m_from = 0, m_end = 0;
   // tile number `tile` of row blocks x column tiles: in groups of `group` row blocks, inside a group column tile by column tile.  With groups of
   // 1024 rows an XCD works on about 1024 rows x 8 column tiles at a time (2048 or 4096 rows: the same at 16 row tiles, 3 to 20 % slower at 8).
   auto tile_in = [&](int tile, int row_blocks, int group) {
@@ -100,48 +111,60 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   };
   constexpr int GR = 1024 / ROWS;
   if constexpr (GROUPED) {
-    // tiles expert by expert; every wave finds its own
-    auto blocks_of = [&](int e) { return e < a.n_experts ? (a.offsets[e + 1] - a.offsets[e] + ROWS - 1) / ROWS : 0; };
-    int total = 0;
-    for (int base = 0; base < a.n_experts; base += 64) {
-      int nb = blocks_of(base + lane);
+    // Tiles expert by expert; every wave finds its own: 256 experts at a time, four to a lane, from one round trip for all their offsets and a running
+    // sum by DPP: it stands in front of a work-group's first load, a tenth of its time at short contractions (clock stamps).  With the places of the stored rows asked for
+    // at once (wide_out.h), us before (a round trip and a chain of exchanges through LDS per 64 experts, twice) | now: 57288 routes of 128 experts
+    // 768 -> 2048 286 | 262, 2048 -> 1536 gated 428 | 424; 65536 of 64 768 -> 2048 302 | 283, 2048 -> 768 232 | 225.
+    const int E = a.n_experts;
+    int from[4], to[4], nb[4], end[4];   // an expert's routes and its blocks; the blocks up to its last one
+    auto count = [&](int base, int before) -> int {   // returns `before` and the blocks of these experts
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) nb += lane_xor(nb, o);
-      total += nb;
-    }
+      for (int c = 0; c < 4; ++c) {
+        from[c] = a.offsets[min(base + 64 * c + lane, E)];
+        to[c] = a.offsets[min(base + 64 * c + lane + 1, E)];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        nb[c] = (to[c] - from[c] + ROWS - 1) / ROWS;
+        end[c] = wave_scan(nb[c]) + before;
+        before = __builtin_amdgcn_readlane(end[c], 63);
+      }
+      return before;
+    };
+    int total = 0;
+    for (int base = 0; base < E; base += 256) total = count(base, total);
     const int tile = xcd_tile((int)blockIdx.x, total * tiles_n);
     if (tile < 0) return;   // past the last block (the grid covers an upper bound)
-    int carry = 0, found_e = 0, found_at = 0, found_nb = 1;
-    for (int base = 0; base < a.n_experts; base += 64) {
-      const int nb = blocks_of(base + lane);
-      int incl = nb;
+    const int block = tile / tiles_n;
+    int found_at = 0, found_nb = 1;
+    for (int base = 0, before = 0; base < E; base += 256) {
+      if (E > 256) before = count(base, before);
+      bool found = false;
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += t;
+      for (int c = 0; c < 4; ++c) {
+        const uint64_t hit = __ballot(block < end[c] && block >= end[c] - nb[c]);   // (one lane: the blocks of an expert are its own)
+        if (hit) {
+          const int l = __builtin_ctzll(hit);
+          expert = base + 64 * c + l;
+          found_nb = __builtin_amdgcn_readlane(nb[c], l);
+          found_at = tile - (__builtin_amdgcn_readlane(end[c], l) - found_nb) * tiles_n;
+          m_from = __builtin_amdgcn_readlane(from[c], l);
+          m_end = __builtin_amdgcn_readlane(to[c], l);
+          found = true;
+        }
       }
-      const int first = (carry + incl - nb) * tiles_n;
-      const uint64_t hit = __ballot(nb > 0 && tile >= first && tile < first + nb * tiles_n);
-      if (hit) {
-        const int l = __ffsll((long long)hit) - 1;
-        found_e = base + l;
-        found_at = tile - __shfl(first, l, 64);
-        found_nb = __shfl(nb, l, 64);
-      }
-      carry += __shfl(incl, 63, 64);
+      if (found) break;
     }
-    expert = __builtin_amdgcn_readfirstlane(found_e);
     // an expert of many rows in groups of 1024 rows or near it, equal ones, or its few last blocks would draw all weights for themselves:
     // 8 experts of 8000 rows x 4096 -> 4096 took 2340 us with all row blocks per column tile against 1710 (256-row tiles), 2395 against
     // 1760 (128); 8 of 1300 rows, eleven blocks, 340 us in groups of eight and three against 318 in one of eleven.
-    const int nb = __builtin_amdgcn_readfirstlane(found_nb), groups = max(1, (nb + GR / 2) / GR);
-    tile_in(__builtin_amdgcn_readfirstlane(found_at), nb, (nb + groups - 1) / groups);
-    m_end = a.offsets[expert + 1];
+    const int groups = max(1, (found_nb + GR / 2) / GR);
+    tile_in(found_at, found_nb, (found_nb + groups - 1) / groups);
   } else {
     tile_in(xcd_tile((int)blockIdx.x, tiles_m * tiles_n), tiles_m, GR);
   }
   // first row of the tile (GROUPED: first position in the sorted route list)
-  const int64_t m0 = GROUPED ? (int64_t)a.offsets[expert] + (int64_t)mtile * ROWS : (int64_t)mtile * ROWS;
+  const int64_t m0 = (int64_t)m_from + (int64_t)mtile * ROWS;
   const int rows_here = (int)min((int64_t)ROWS, (GROUPED ? (int64_t)m_end : a.M) - m0);
   const int ktiles = (int)(a.K / KTILE), ksteps = 2 * ktiles;
   const int64_t ntiles = a.N / 16, ntile0 = ((int64_t)ntile * 4 + wn) * 4;   // first 16-column tile of this wave
@@ -159,11 +182,13 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   const uint32_t dma_wave = (uint32_t)wn * 1024u;
   uint32_t xrow[GROUPED ? PASSES : 1];   // GROUPED: byte offsets of this thread's rows (rows the block does not have: beyond the buffer)
   if constexpr (GROUPED) {
+    const bool whole_shift = (a.x_div & (a.x_div - 1)) == 0;   // (a division is some thirty instructions in front of the first load)
+    const int x_shift = __builtin_ctz((uint32_t)a.x_div);
 #pragma unroll
     for (int c = 0; c < PASSES; ++c) {
       const int r = (tid >> 3) + 32 * c;
-      const int route = r < rows_here ? a.sorted_route[m0 + r] : -1;
-      xrow[c] = route >= 0 ? ((uint32_t)(route / a.x_div) * (uint32_t)a.K + chs * 8u) * 2u : 0xfffff000u;
+      const uint32_t route = (uint32_t)a.sorted_route[m0 + min(r, rows_here - 1)], src = whole_shift ? route >> x_shift : route / (uint32_t)a.x_div;
+      xrow[c] = r < rows_here ? (src * (uint32_t)a.K + chs * 8u) * 2u : 0xfffff000u;
     }
   }
   // (dma16 of gemm_tile.h: the compiler does not count these loads, the waits for them are written by hand)

@@ -212,10 +212,20 @@ __device__ __forceinline__ void wide_tile_out(const QLArgs& a, const WideHead& h
     const int ch = tid % chunks, r0 = tid / chunks, rstep = 256 / chunks;
     uint16_t* y = reinterpret_cast<uint16_t*>(a.y);
     const bool col_ok = col0 + ch * 8 + 8 <= width;
-    for (int row = r0; row < ROWS; row += rstep) {
+    // The places of all rows at once: y may lie anywhere for all the compiler knows, so that row by row every store stood behind a round trip to the L2
+    // of its own (57288 routes of 128 experts, 768 -> 2048, 286 -> 271 us).
+    constexpr int PER = ROWS / rstep;
+    int route[GROUPED ? PER : 1];
+    if constexpr (GROUPED) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) route[i] = a.sorted_route[m0 + min(r0 + i * rstep, rows_here - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int row = r0 + i * rstep;
       if (row >= rows_here || !col_ok) continue;
       u32x4 v = lds_ld128(stage + (uint32_t)((row * sld + ch * 8) * 2));
-      const int64_t orow = GROUPED ? (int64_t)a.sorted_route[m0 + row] : m0 + row;
+      const int64_t orow = GROUPED ? (int64_t)route[GROUPED ? i : 0] : m0 + row;
       const int64_t o = orow * ldy + col0 + ch * 8;
       if (a.epilogue == TNX_EPI_RESIDUAL) {
         const u32x4 res = *reinterpret_cast<const u32x4*>(a.residual + o);
