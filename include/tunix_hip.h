@@ -82,9 +82,10 @@ const char* tnx_last_error(void);
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
  * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora,
  * tnx_gqa_attn_lora, tnx_rope_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric; 6.4 adds tnx_qlinear_inner and
- * tnx_qlinear_inner_rows; 6.5 adds tnx_lmhead_commit and tnx_embed_norm. */
+ * tnx_qlinear_inner_rows; 6.5 adds tnx_lmhead_commit and tnx_embed_norm; 6.6 adds tnx_gqa_attn_parts, tnx_qlinear_merged and
+ * tnx_qlinear_merged_ok. */
 #define TNX_ABI_VERSION_MAJOR 6
-#define TNX_ABI_VERSION_MINOR 5
+#define TNX_ABI_VERSION_MINOR 6
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
 int tnx_version(void);
 
@@ -194,6 +195,11 @@ int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* h_desc);
  * bf16 [K / 32][lora_rank / 16][4][16][8]: element (g, n, q, c, i) is A[32 g + 8 q + i][16 n + c].                                      */
 int tnx_qlinear_inner(void* stream, const tnx_qlinear_desc* h_desc, const uint16_t* a_frag);
 int64_t tnx_qlinear_inner_rows(int64_t K, int64_t N, int lora_rank, int split_k);
+/* tnx_qlinear_inner whose x (not read) is the output of tnx_gqa_attn_parts, merged on its way in, bit for bit as tnx_gqa_attn's pass does: parts is that
+ * call's ws, n_chunks its chunks, dh its head size (K = heads * dh), M its rows.  The linear's output lies outside parts.  tnx_qlinear_merged_ok: whether
+ * it takes the shape (1) or not (0: the work-groups would read more partials than a launch of its own takes). */
+int tnx_qlinear_merged(void* stream, const tnx_qlinear_desc* h_desc, const uint16_t* a_frag, const float* parts, int dh, int n_chunks);
+int tnx_qlinear_merged_ok(int64_t M, int64_t K, int64_t N, int lora_rank, int split_k, int dh, int n_chunks);
 /* Epilogue for split_k > 1 (same desc, whose t is not read): y = epi(sum_z ws[z]). */
 int tnx_splitk_finish(void* stream, const tnx_qlinear_desc* h_desc);
 
@@ -395,6 +401,10 @@ typedef struct tnx_attn_desc {
 } tnx_attn_desc;
 size_t tnx_attn_ws_bytes(int64_t B, int64_t T, int64_t S, int Hq, int dh, int kv_chunk);
 int tnx_gqa_attn(void* stream, const tnx_attn_desc* h_desc);
+/* tnx_gqa_attn of a decode step (T == 1) with several key chunks, or with r tnx_rope_gqa_attn_lora (a_t null), without the pass that merges the chunks: out is not
+ * written, ws holds for every query vector (row, head) and chunk dh + 4 numbers: a maximum m, a sum l, two of no meaning and O[dh]; the output is
+ * sum_c e^(m_c - max m) O_c / sum_c e^(m_c - max m) l_c over the chunks whose l is not 0. */
+int tnx_gqa_attn_parts(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d);
 
 /* tnx_gqa_attn, then the LoRA down-projection of its output rows, t[:, :R] = bf16(out . a_t^T) as tnx_lora_down forms it
  * (a_t bf16 [R, Hq * dh], R % 16 == 0).  Where the key range of a decode step is split into chunks whose partials are at most 64 KB a row

@@ -2667,6 +2667,75 @@ def test_many_rows_experts_from_expanded_copies(gpu, K, N, counts):
     assert ((y[route[a0:a1].long()].double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()
 
 
+@pytest.mark.parametrize("dh,Hkv,G,M,S,chunk,window,qtype,group", [
+    (128, 8, 4, 1, 160, 32, 0, Q.NF4, 64),       # 5 chunks, 32 k-tiles in 8 splits of 4
+    (128, 8, 4, 3, 384, 32, 100, Q.NF4, 64),     # 12, some before the window
+    (128, 8, 4, 8, 128, 32, 0, Q.INT4, 32),      # 4
+    (128, 8, 4, 9, 96, 64, 0, Q.INT4, 128),      # 2, rows of the next tile
+    (128, 8, 4, 16, 64, 32, 20, Q.NF4, 32),
+    (64, 2, 4, 33, 96, 32, 0, Q.INT4, 64),       # two heads a k-tile
+    (64, 2, 4, 64, 64, 32, 40, Q.INT4, 64),
+    (256, 1, 4, 17, 288, 96, 0, Q.INT4, 128),    # half a head a k-tile
+    (256, 1, 4, 40, 64, 32, 0, Q.NF4, 64),
+    (256, 1, 3, 2, 200, 32, 33, Q.INT4, 128),    # 6 k-tiles, three a split
+])
+def test_linear_that_merges_key_chunks(gpu, dh, Hkv, G, M, S, chunk, window, qtype, group):
+  """gqa_attn_parts and a linear that merges its chunks against gqa_attn and the linear with its adapter inside, bit for bit: chunks without a key (padding in
+  front, a window), whose outputs nobody writes, included."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  bf = torch.bfloat16
+  g = torch.Generator(device=gpu).manual_seed(dh + M)
+  K, N, rank = Hkv * G * dh, 272, 32
+  r = lambda *s: torch.randn(*s, generator=g, device=gpu)
+  col = S - 3
+  tokens = torch.ones(M, S, dtype=torch.int32, device=gpu)
+  for b in range(M):
+    tokens[b, :(b * 37) % (col + 1)] = 0
+  q, kc, vc = r(M, Hkv * G, dh).to(bf), r(M, Hkv, S, dh).to(bf), r(M, Hkv, S, dh).to(bf)
+  n_chunks = -(-S // chunk)
+  ws = torch.full((ops.attn_ws_bytes(M, 1, S, Hkv * G, dh, chunk) // 4,), float("nan"), device=gpu)
+  out = torch.empty(M, K, dtype=bf, device=gpu)
+  ad = L.AttnDesc()
+  ad.B, ad.T, ad.S, ad.Hq, ad.Hkv, ad.dh = M, 1, S, Hkv * G, Hkv, dh
+  ad.scale, ad.window, ad.pad_id, ad.kv_chunk = dh ** -0.5, window, 0, chunk
+  at = torch.tensor([col], dtype=torch.int32, device=gpu)
+  ad.q, ad.kcache, ad.vcache, ad.tokens, ad.tok_ld, ad.col_ptr = q.data_ptr(), kc.data_ptr(), vc.data_ptr(), tokens.data_ptr(), S, at.data_ptr()
+  ad.ws, ad.out = ws.data_ptr(), out.data_ptr()
+  split = {4096: 8, 768: 2}.get(K, K // 128)
+  codes, scales = ops.quantize_pack((r(K, N) * 0.05).to(bf), group, qtype)
+  a_t, b = (r(rank, K) * K ** -0.5).to(bf), (r(N, rank) * 0.3).to(bf)
+  frag = ops.lora_frag(a_t)
+  assert ops.qlinear_merged_ok(M, K, N, rank, split, dh, n_chunks)
+  got = []
+  for merged in (False, True):
+    y = torch.full((M, N), float("nan"), dtype=bf, device=gpu)
+    planes = torch.full((split, M, N), float("nan"), device=gpu)
+    d = ops.make_qlinear_desc(M=M, K=K, N=N, group=group, qtype=qtype, x=out, codes=codes, scales=scales, y=y, lora_rank=rank, lora_nseg=1,
+                              lora_seg_end=[N], lora_seg_toff=[0], lora_b=b, lora_scale=0.5, split_k=split, ws=planes)
+    ws.fill_(float("nan"))
+    if merged:   # (x is not read)
+      out.fill_(float("nan"))
+      ops.gqa_attn_parts(None, ad)
+      ops.qlinear(d, a_frag=frag, parts=(ws, dh, n_chunks))
+    else:
+      ops.gqa_attn(ad)
+      ops.qlinear(d, a_frag=frag)
+    got += [y, planes]
+  assert got[0].isfinite().all()
+  assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3])
+
+
+def test_linear_that_merges_key_chunks_refuses(gpu):
+  """More rows, chunks or bytes than it takes, and an output in the partials."""
+  from tunix_amd import ops
+  ok = ops.qlinear_merged_ok
+  assert ok(16, 4096, 4096, 64, 8, 128, 2) and not ok(32, 4096, 4096, 64, 8, 128, 2)      # bytes
+  assert ok(1, 4096, 4096, 64, 8, 128, 12) and not ok(1, 4096, 4096, 64, 8, 128, 13)      # chunks
+  assert not ok(1, 4096, 4096, 64, 4, 128, 2)        # eight k-tiles a split
+  assert not ok(1, 4096, 4096, 48, 8, 128, 2) and not ok(1, 4096, 4096, 64, 8, 96, 2) and not ok(65, 1024, 1024, 32, 8, 256, 2)
+
+
 @pytest.mark.parametrize("E,x_div", [(1, 3), (64, 1), (65, 2), (256, 1), (257, 3), (520, 4)])
 def test_many_rows_experts_are_found_among_any_number(gpu, E, x_div):
   """The search for a tile's expert, 256 of them at a time, and the rows of routes for divisors that are and are no powers of two: most experts

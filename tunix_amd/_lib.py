@@ -12,7 +12,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtunix_hip.so")
 
 # the ABI this binding was written against (TNX_ABI_VERSION_MAJOR / _MINOR of include/tunix_hip.h)
-ABI_VERSION = (6, 5)
+ABI_VERSION = (6, 6)
 
 TNX_Q_INT4, TNX_Q_NF4 = 0, 1
 TNX_NORM_LLAMA, TNX_NORM_QWEN3, TNX_NORM_GEMMA3 = 0, 1, 2
@@ -321,6 +321,7 @@ SIGNATURES = {
     "tnx_rope_table": (_i32, [_p, _p, _i64, _p, _i64, _p, _i32, _p, _p]),
     "tnx_attn_ws_bytes": (C.c_size_t, [_i64, _i64, _i64, _i32, _i32, _i32]),
     "tnx_gqa_attn": (_i32, [_p, C.POINTER(AttnDesc)]),
+    "tnx_gqa_attn_parts": (_i32, [_p, C.POINTER(RopeDesc), C.POINTER(AttnDesc)]),
     "tnx_gqa_attn_lora": (_i32, [_p, C.POINTER(AttnDesc), _p, _i32, _p, _i64]),
     "tnx_rope_gqa_attn_lora": (_i32, [_p, C.POINTER(RopeDesc), C.POINTER(AttnDesc), _p, _i32, _p, _i64]),
     "tnx_lmhead_nblocks": (_i64, [_i64]),
@@ -339,6 +340,8 @@ SIGNATURES = {
     "tnx_moe_int4_gmm": (_i32, [_p, C.POINTER(MoeGmmDesc)]),
     "tnx_qlinear_inner": (_i32, [_p, C.POINTER(QLinearDesc), _p]),
     "tnx_qlinear_inner_rows": (_i64, [_i64, _i64, _i32, _i32]),
+    "tnx_qlinear_merged": (_i32, [_p, C.POINTER(QLinearDesc), _p, _p, _i32, _i32]),
+    "tnx_qlinear_merged_ok": (_i32, [_i64, _i64, _i64, _i32, _i32, _i32, _i32]),
     "tnx_moe_gmm_expanded": (_i32, [_p, C.POINTER(MoeGmmDesc), _p]),
     "tnx_moe_expanded_rows": (_i64, [_i64, _i64, _i32]),
     "tnx_moe_combine": (_i32, [_p, _p, _p, _i64, _i32, _i64, _p, _p]),

@@ -13,6 +13,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "attn_parts.h"
 #include "common.h"
 #include "gemm_tile.h"   // dma16, raw_rsrc, tnx_wait_vm
 #include "rope_math.h"
@@ -57,8 +58,6 @@ struct AttnArgs {
   const float* rope_cos;
 };
 
-constexpr float kNegBig = -1.0e30f;
-constexpr int kPartPad = 4;   // numbers in front of a partial's O[dh]: m, l, and two that keep the rest on 16 bytes
 
 // f over the four lanes lm + 16 {0, 1, 2, 3} that share a query, in all of them
 template <class F>
@@ -1576,8 +1575,8 @@ extern "C" int tnx_gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uin
   return gqa_attn_lora(stream, d, a_t, R, t, t_ld, nullptr);
 }
 
-extern "C" int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t,
-                                      int64_t t_ld) {
+// combine: see gqa_attn
+static int rope_gqa_attn(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld, bool combine) {
   TNX_REQUIRE(r && d, "rope_gqa_attn: null descriptor");
   RopeArgs ra;
   int rc = rope_args(r, ra);
@@ -1603,5 +1602,15 @@ extern "C" int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, cons
     if (rc) return rc;
   }
   const RopeArgs* rope = one ? &ra : nullptr;
-  return a_t ? gqa_attn_lora(stream, d, a_t, R, t, t_ld, rope) : gqa_attn(stream, d, true, rope);
+  return a_t ? gqa_attn_lora(stream, d, a_t, R, t, t_ld, rope) : gqa_attn(stream, d, combine, rope);
+}
+
+extern "C" int tnx_rope_gqa_attn_lora(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t,
+                                      int64_t t_ld) {
+  return rope_gqa_attn(stream, r, d, a_t, R, t, t_ld, true);
+}
+
+extern "C" int tnx_gqa_attn_parts(void* stream, const tnx_rope_desc* r, const tnx_attn_desc* d) {
+  TNX_REQUIRE(d && d->T == 1 && d->kv_chunk > 0 && d->S > d->kv_chunk, "gqa_attn_parts: a decode step whose key range is cut into chunks");
+  return r ? rope_gqa_attn(stream, r, d, nullptr, 0, nullptr, 0, false) : gqa_attn(stream, d, false);
 }

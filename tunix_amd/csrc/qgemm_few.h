@@ -49,7 +49,13 @@ constexpr uint32_t kFewLds = 160u << 10, kFewMeet = 0x20000, kFewOut = 0x10000, 
 // WHOLE: rows of x are whole 16-byte pieces, as loads straight into LDS ask for; otherwise they go by way of registers.  (A form of its own: as a branch
 // beside those loads it costs every launch 0.2 us, 0.9 % of a rollout of 16 rows.)
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
-template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT, bool WHOLE>
+// MERGE: x is what a decode step's attention left of its key chunks (attn_parts.h), merged here on its way to LDS: a launch less, for a read of the
+// partials per column of work-groups and some hundred instructions a wave.  us a layer, with the merging pass | merged here: 32 heads of 128 on 8,
+// 4 k-tiles a split: 1 row x 600 keys (5 chunks) 71.0 | 66.1, 2 x 800 (7) 69.2 | 66.9, 3 x 2940 (10) 77.8 | 74.4, 8 x 400 (4) 72.2 | 70.1, 16 x 700 (2) 80.9 | 79.4;
+// 4 heads of 256 on one, one k-tile: 1 x 600 (5) 48.4 | 46.4, 16 x 1200 (10) 51.3 | 50.2.  Beyond kMergeBytes of partials a work-group (qlinear.hip) or
+// kMergeChunks chunks, a second round trip, nothing is left of it.
+constexpr int kMergeChunks = 12;
+template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT, bool WHOLE, bool MERGE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void qgemm_few_kernel(const QLArgs a) {
   constexpr int MT = (ROWS + 15) / 16;
   constexpr uint32_t SLOT = ROWS * 256;
@@ -132,7 +138,79 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
   };
-  request_x(0, min(n, NB * CHUNK), 0);
+  // The same from partials: a thread takes eight columns of a row of a k-tile, U such pieces at a time, NC chunks of them at once.  (Vector instructions
+  // are what it costs, some 0.3 us per hundred of a wave: few, and no rows or chunks that are not there.)
+  auto merge_x = [&](auto Uc, auto NCc) {
+    constexpr int U = decltype(Uc)::value, NC = decltype(NCc)::value;
+    const uint32_t C = (uint32_t)a.parts_n, dh = 1u << a.parts_shift, pitch = (dh + kPartPad) * 4u, heads = (uint32_t)(a.K >> a.parts_shift);
+    const uint32_t pieces = (uint32_t)a.M * (uint32_t)n * 16u;
+    const rsrc_t rp = make_rsrc(a.parts, (uint64_t)a.M * heads * C * pitch);
+    for (uint32_t e0 = (uint32_t)tid; e0 < pieces; e0 += 512u * U) {
+      uint32_t at[U], off[U], to[U];
+      u32x2 ml[U][NC];
+      u32x4 v[U][NC][2];
+      auto fetch = [&](int k, uint32_t c0) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          if (c0 + c < C) {
+            ml[k][c] = __builtin_amdgcn_raw_buffer_load_b64(rp, at[k], (int)((c0 + c) * pitch), 0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[k][c][h] = __builtin_amdgcn_raw_buffer_load_b128(rp, off[k] + 16u * h, (int)((c0 + c) * pitch), 0);
+          }
+      };
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const uint32_t e = e0 + 512u * k, row = n == 1 ? e >> 4 : n == 2 ? e >> 5 : n == 4 ? e >> 6 : e / 48u, i = (e >> 4) - row * (uint32_t)n, p = e & 15u;
+        const uint32_t col = ((uint32_t)kt_begin + i) * KTILE + p * 8u;
+        at[k] = e < pieces ? (row * heads + (col >> a.parts_shift)) * (C * pitch) : 0xf0000000u;
+        off[k] = at[k] + (kPartPad + (col & (dh - 1u))) * 4u;
+        const uint32_t slot = i * SLOT;
+        to[k] = (INT4 || slot < kBigLutBase ? slot : slot + (uint32_t)kBigLutBytes) + row * 256u + (p ^ (row & 15u)) * 16u;
+        fetch(k, 0);
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        float top = kNegBig, L = 0.0f, o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          if (c < (int)C) top = __uint_as_float(ml[k][c][1]) != 0.0f ? fmaxf(top, __uint_as_float(ml[k][c][0])) : top;
+        for (uint32_t c = NC; c < C; ++c) {
+          const u32x2 m = __builtin_amdgcn_raw_buffer_load_b64(rp, at[k], (int)(c * pitch), 0);
+          top = __uint_as_float(m[1]) != 0.0f ? fmaxf(top, __uint_as_float(m[0])) : top;
+        }
+        for (uint32_t c0 = 0; c0 < C; c0 += NC) {
+          if (c0 > 0) fetch(k, c0);
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+            if (c0 + c < C) {
+              const float l = __uint_as_float(ml[k][c][1]);
+              if (l != 0.0f) {   // (a chunk without a key: an O nobody wrote)
+                const float w = __expf(__uint_as_float(ml[k][c][0]) - top);
+                L += w * l;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] += w * __uint_as_float(v[k][c][e >> 2][e & 3]);
+              }
+            }
+        }
+        if (e0 + 512u * k < pieces) {
+          // o / L: the quotient by a reciprocal, corrected by its remainder
+          const float inv = L != 0.0f ? 1.0f / L : 0.0f;
+          u32x4 x;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float t = o[e] * inv;
+            o[e] = __builtin_fmaf(__builtin_fmaf(-t, L, o[e]), inv, t);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = pack2bf(o[2 * e], o[2 * e + 1]);
+          lds_st128(to[k], x);
+        }
+      }
+    }
+  };
+  if constexpr (!MERGE) request_x(0, min(n, NB * CHUNK), 0);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int d = 0; d < PF; ++d)
@@ -158,8 +236,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   if constexpr (!INT4) fill_level_table<512>(kBigLutBase, tid);   // while the first loads are in flight
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (MERGE) {
+    static_assert(SHORT && INNER, "all k-tiles in LDS at once");
+    if (a.parts_n <= 4 && a.M * n > 32) merge_x(ic<2>{}, ic<4>{});
+    else merge_x(ic<1>{}, ic<kMergeChunks>{});
+  }
   // the activations, requested ahead of the ring's weights
-  if (!SHORT || n >= 4) tnx_wait_vm(4 * LOADS);
+  if (MERGE) {
+    // (they are in registers and stored)
+  } else if (!SHORT || n >= 4) tnx_wait_vm(4 * LOADS);
   else if (n == 3) tnx_wait_vm(3 * LOADS);
   else if (n == 2) tnx_wait_vm(2 * LOADS);
   else tnx_wait_vm(LOADS);

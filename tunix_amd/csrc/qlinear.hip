@@ -7,6 +7,7 @@
 #include <cmath>
 #include <mutex>
 
+#include "attn_parts.h"
 #include "gemm_tile.h"
 #include "rng.h"
 
@@ -47,6 +48,9 @@ struct QLArgs {
   int64_t ldy;
   // the adapter's A in fragment order (few-row kernel only)
   const uint16_t* inner_a;
+  // x as the partials of a decode step's attention (few-row kernel only): chunks, log2 of the head size
+  const float* parts;
+  int parts_n, parts_shift;
 };
 // gate | up with the activation and the product in fp32 and one rounding (dense-weight decoders;
 // many-row kernel only)
@@ -544,6 +548,8 @@ QLArgs to_args(const tnx_qlinear_desc* d) {
   a.w_pre = d->w_expanded;
   a.ldy = 0;
   a.inner_a = nullptr;
+  a.parts = nullptr;
+  a.parts_n = a.parts_shift = 0;
   return a;
 }
 
@@ -748,13 +754,13 @@ int launch_qgemm128(hipStream_t st, const QLArgs& a) {
   return a.qtype == TNX_Q_INT4 ? launch_qgemm128_as<NT, SPT, MT, true>(st, a) : launch_qgemm128_as<NT, SPT, MT, false>(st, a);
 }
 
-template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT, bool WHOLE>
+template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT, bool WHOLE, bool MERGE = false>
 int launch_qgemm_few_as(hipStream_t st, const QLArgs& a) {
   static std::once_flag once;
   static int attr_rc = TNX_OK;
-  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT, WHOLE>, kFewLds); });
+  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT, WHOLE, MERGE>, kFewLds); });
   if (attr_rc) return attr_rc;
-  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT, WHOLE>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kFewLds, st, a);
+  hipLaunchKernelGGL((qgemm_few_kernel<SPT, INT4, ROWS, INNER, SHORT, WHOLE, MERGE>), dim3(1u, (unsigned)cdiv(a.N, 128), (unsigned)a.split_k), dim3(512), kFewLds, st, a);
   TNX_CHECK_LAUNCH("qgemm_few");
   return TNX_OK;
 }
@@ -782,6 +788,10 @@ constexpr int64_t kFewRows = 32;
 // With the adapter inside, up to kFewKtiles64 k-tiles of any number of groups, at 64 rows: nf4 2048 -> 2048 in 8 7.8 | 8.8 and 8192 -> 2048 in 16, the least
 // gain, 10.0 | 15.2, next to 3.7 to 6 of the launch that formed t, its gap, and 1.1 of a gate | up that leaves the planes for it.
 constexpr int kFewKtiles64 = 4;
+// Partials of a decode step's attention that a work-group of the linear behind it merges itself.  us a layer, with the merging pass | in the linear: 4 heads of 256 on one,
+// 80 KB (16 rows x 10 chunks) 51.3 | 50.2, 96 KB (64 x 3) 63.4 | 63.6, 120 KB (48 x 5) 63.8 | 63.6, 128 KB (32 x 8) 55.8 | 55.9, (64 x 4) 72.9 | 73.0; 32 heads of 128 on 8, 64 KB
+// (16 x 2) 77.1 | 75.9, 128 KB (32 x 2) 111.9 | 112.6, 160 KB (40 x 2) 144.8 | 146.7; of few bytes in more chunks: 24 x 1 row 72.0 | 72.6, 23 x 3 rows of 256 51.7 | 52.9.
+constexpr int64_t kMergeBytes = 80 << 10;
 bool few_shape(const QLArgs& a) {
   return a.M <= kFewRows || (a.M <= 64 && a.split_k > 1 && a.ktiles_per_split <= 2 && cdiv(a.N, 128) * a.split_k <= 64);
 }
@@ -1162,6 +1172,40 @@ extern "C" int tnx_qlinear_inner(void* stream, const tnx_qlinear_desc* d, const 
   QLArgs a = to_args(&c);
   a.inner_a = a_frag;
   return launch_qgemm_few<true>(as_stream(stream), a, scales_per_tile(a.group) == 2);
+}
+
+extern "C" int tnx_qlinear_merged_ok(int64_t M, int64_t K, int64_t N, int lora_rank, int split_k, int dh, int n_chunks) {
+  if ((dh != 64 && dh != 128 && dh != 256) || K % dh != 0 || n_chunks < 1 || n_chunks > kMergeChunks || M < 1 || M > tnx_qlinear_inner_rows(K, N, lora_rank, split_k)) return 0;
+  const int64_t per = cdiv(K / KTILE, split_k < 1 ? 1 : split_k);
+  return per <= 4 && M * per * KTILE * n_chunks * 4 <= kMergeBytes;
+}
+
+extern "C" int tnx_qlinear_merged(void* stream, const tnx_qlinear_desc* d, const uint16_t* a_frag, const float* parts, int dh, int n_chunks) {
+  TNX_REQUIRE(d != nullptr, "qlinear_merged: null descriptor");
+  tnx_qlinear_desc c = *d;
+  c.t = c.x = (const uint16_t*)parts;   // (not read)
+  c.t_ld = 8;
+  const int rc = check_desc(&c);
+  if (rc) return rc;
+  TNX_REQUIRE(tnx_qlinear_merged_ok(d->M, d->K, d->N, d->lora_rank, d->split_k, dh, n_chunks), "qlinear_merged: %lld rows, %d chunks: not a shape it takes",
+              (long long)d->M, n_chunks);
+  TNX_REQUIRE(d->lora_nseg == 1 && d->epilogue != TNX_EPI_SILU_MUL && d->epilogue != TNX_EPI_GELU_MUL, "qlinear_merged: one adapter, no *_MUL epilogue");
+  TNX_REQUIRE(a_frag && ((uintptr_t)a_frag & 15) == 0 && ((uintptr_t)parts & 15) == 0, "qlinear_merged: fragments and partials must be 16-byte aligned");
+  const int64_t bytes = d->M * (d->K / dh) * n_chunks * (dh + kPartPad) * 4;
+  TNX_REQUIRE(apart(parts, bytes, d->split_k > 1 ? (const void*)d->ws : d->y, d->split_k > 1 ? (int64_t)d->split_k * d->M * d->N * 4 : d->M * d->N * 4),
+              "qlinear_merged: the output lies in the partials");
+  QLArgs a = to_args(&c);
+  a.inner_a = a_frag;
+  a.parts = parts;
+  a.parts_n = n_chunks;
+  a.parts_shift = dh == 64 ? 6 : dh == 128 ? 7 : 8;
+  hipStream_t st = as_stream(stream);
+  const auto rows = [&](auto spt_c, auto rows_c) {
+    constexpr int SPT = decltype(spt_c)::value, ROWS = decltype(rows_c)::value;
+    return a.qtype == TNX_Q_INT4 ? launch_qgemm_few_as<SPT, true, ROWS, true, true, true, true>(st, a) : launch_qgemm_few_as<SPT, false, ROWS, true, true, true, true>(st, a);
+  };
+  const auto book = [&](auto spt_c) { return a.M <= 8 ? rows(spt_c, ic<8>{}) : a.M <= 16 ? rows(spt_c, ic<16>{}) : a.M <= 32 ? rows(spt_c, ic<32>{}) : rows(spt_c, ic<64>{}); };
+  return scales_per_tile(a.group) == 2 ? book(ic<2>{}) : book(ic<4>{});
 }
 
 // The lm_head over many rows on the many-row kernels: per 128-column block statistics

@@ -595,7 +595,10 @@ class Runner(HeadRunner):
     if not adapter_behind and S <= (384 if head_dim <= 64 else 256 if head_dim <= 128 else 0):
       return 1
     if groups <= 128:
-      return max(1, min(256 // groups, math.ceil(S / 128)))
+      # (merged in the linear behind: no more than it takes in one round trip; heads of 256 gain more from more of them.  us a layer in 24 chunks with the merging
+      # pass | in 10 without, one row x 3000, 8 kv heads of 128 72.0 | 70.6, one of 256 50.8 | 53.4; 2 x 2000 in 16 | 9 72.0 | 69.0)
+      most = 12 if not adapter_behind and head_dim <= 128 else 256
+      return max(1, min(256 // groups, math.ceil(S / 128), most))
     # More: two to a unit, of many keys, are cut in halves, which even out what the units have: 40 rows x 8 heads of 128 x 1280 52.6 | 44.2 (32 rows
     # 33.3 | 35.0, 56 rows x 1500 63.7 | 67.9; heads of 64, 256 rows x 2 x 1500 37 | 49).
     if head_dim <= 128:
@@ -653,11 +656,12 @@ class Runner(HeadRunner):
     return split
 
   def linear(self, f: FusedLinear, x, y, M, epilogue=L.TNX_EPI_STORE, residual=None, defer=False,
-             next_f: FusedLinear | None = None, t_ready: bool = False):
+             next_f: FusedLinear | None = None, t_ready: bool = False, parts=None):
     """Runs one fused linear.  With defer=True a split-k linear skips its finishing pass and
     returns split_k (> 1): the caller hands the partial planes in self.splitk_ws to the kernel
     that consumes them (`norm_after` for a RESIDUAL linear of model width, the rope / cache
-    write for a plain STORE); otherwise returns 1 with y complete."""
+    write for a plain STORE); otherwise returns 1 with y complete.  parts: x is what `merges` says the
+    attention left in its workspace."""
     inner = self.inner(f, M) and not t_ready
     if f.has_lora and not t_ready and not inner:
       ops.lora_down(x, f.a_t, self.t, M=M)
@@ -681,12 +685,18 @@ class Runner(HeadRunner):
     deferred = defer and split > 1 and (
         epilogue == L.TNX_EPI_STORE
         or (epilogue == L.TNX_EPI_RESIDUAL and f.N == self.cfg.embed_dim and f.N % 8 == 0))
-    ops.qlinear(d, finish=not deferred, a_frag=f.a_frag if inner else None)
+    ops.qlinear(d, finish=not deferred, a_frag=f.a_frag if inner else None, parts=parts)
     return split if deferred else 1
 
   def inner(self, f: FusedLinear, M: int) -> bool:
     """Whether `linear` of M rows forms the adapter's down-projection of its input itself: then nothing ahead of it has to."""
     return M <= self.SPLIT_ROWS and M <= f.inner_rows(self._split_k(f, M))
+
+  def merges(self, f: FusedLinear, M: int) -> tuple | None:
+    """What `linear` takes as its parts where it merges the key chunks of a decode step's attention itself (a launch less), else None."""
+    n = math.ceil(self.S / self.kv_chunk) if self.kv_chunk else 1
+    dh = self.cfg.head_dim
+    return (self.attn_ws, dh, n) if n > 1 and self.inner(f, M) and ops.qlinear_merged_ok(M, f.K, f.N, f.rp, self._split_k(f, M), dh, n) else None
 
   def fuses_next(self, f: FusedLinear, next_f: FusedLinear, M: int, epilogue: int) -> bool:
     return (next_f.has_lora and not self.inner(next_f, M) and next_f.rp <= 64 and M <= 1024 and self._split_k(f, M) == 1
@@ -811,8 +821,10 @@ class Runner(HeadRunner):
         else:
           ad.qkv = self.qkv.data_ptr()
         ad.rope_sin, ad.rope_cos = self.rope_sin.data_ptr(), self.rope_cos.data_ptr()
-      o_ready = not self.inner(ly["o"], M)
-      if T == 1 and not fuse_rope:
+      o_ready, parts = not self.inner(ly["o"], M), self.merges(ly["o"], M) if T == 1 else None
+      if parts is not None:
+        ops.gqa_attn_parts(None if fuse_rope else rd, ad)
+      elif T == 1 and not fuse_rope:
         ops.rope_gqa_attn_lora(rd, ad, adapter(ly["o"]) if o_ready else None, self.t)
       elif ly["o"].has_lora and o_ready:
         ops.gqa_attn_lora(ad, ly["o"].a_t, self.t)
@@ -822,11 +834,11 @@ class Runner(HeadRunner):
       if cfg.family == "gemma3":
         # h += post_attn_norm(o_proj); xn = mlp_norm(h): one launch, which also sums the
         # projection's partial planes when it ran split
-        po = self.linear(ly["o"], self.attn, self.tmp, M, defer=True, t_ready=o_ready)
+        po = self.linear(ly["o"], self.attn, self.tmp, M, defer=True, t_ready=o_ready, parts=parts)
         gu_ready = self.norm_pair(po, ly["post_attn_norm"], ly["mlp_norm"], M, mlp_adapter)
       else:
         po = self.linear(ly["o"], self.attn, self.h, M, epilogue=L.TNX_EPI_RESIDUAL, residual=self.h,
-                         defer=True, t_ready=o_ready)
+                         defer=True, t_ready=o_ready, parts=parts)
         gu_ready = (self.norm_after(po, ly["mlp_norm"], M, ly["experts"].router_t, self.scores) if cfg.num_experts
                     else self.norm_after(po, ly["mlp_norm"], M, mlp_adapter, self.t))
       if cfg.num_experts:

@@ -123,10 +123,18 @@ def qlinear_inner_rows(K: int, N: int, rank: int, split_k: int = 1) -> int:
   return int(L.lib().tnx_qlinear_inner_rows(K, N, rank, split_k))
 
 
-def qlinear(desc: L.QLinearDesc, finish: bool = True, a_frag=None):
+def qlinear_merged_ok(M: int, K: int, N: int, rank: int, split_k: int, head_dim: int, n_chunks: int) -> bool:
+  """Whether `qlinear` takes the chunks that `gqa_attn_parts` left as its parts."""
+  return bool(L.lib().tnx_qlinear_merged_ok(M, K, N, rank, split_k, head_dim, n_chunks))
+
+
+def qlinear(desc: L.QLinearDesc, finish: bool = True, a_frag=None, parts=None):
   """finish=False leaves the split-k partial planes in desc.ws for a consumer that sums them
-  itself (rmsnorm_splitk).  a_frag (`lora_frag`): the adapter's down-projection is formed inside, desc.t is not read."""
-  if a_frag is not None:
+  itself (rmsnorm_splitk).  a_frag (`lora_frag`): the adapter's down-projection is formed inside, desc.t is not read.  parts: (workspace, head size,
+  chunks) of `gqa_attn_parts`, whose output is the input."""
+  if parts is not None:
+    L.check(L.lib().tnx_qlinear_merged(_stream(), C.byref(desc), _ptr(a_frag), _ptr(parts[0]), *parts[1:]), "tnx_qlinear_merged")
+  elif a_frag is not None:
     L.check(L.lib().tnx_qlinear_inner(_stream(), C.byref(desc), _ptr(a_frag)), "tnx_qlinear_inner")
   else:
     L.check(L.lib().tnx_qlinear_lora(_stream(), C.byref(desc)), "tnx_qlinear_lora")
@@ -228,6 +236,11 @@ def attn_ws_bytes(B, T, S, Hq, dh, kv_chunk) -> int:
 
 def gqa_attn(desc: L.AttnDesc):
   L.check(L.lib().tnx_gqa_attn(_stream(), C.byref(desc)), "tnx_gqa_attn")
+
+
+def gqa_attn_parts(rope: L.RopeDesc | None, desc: L.AttnDesc):
+  """gqa_attn, or with rope rope_gqa_attn_lora, of a decode step up to what its key chunks leave in desc.ws."""
+  L.check(L.lib().tnx_gqa_attn_parts(_stream(), rope, C.byref(desc)), "tnx_gqa_attn_parts")
 
 
 def gqa_attn_lora(desc: L.AttnDesc, a_t, t):
