@@ -653,6 +653,45 @@ def test_qlinear_many_rows_matches_oracle(gpu, M, K, N, group, qtype, r, seg_wid
                     ulps=3 if mul else 2 if epi == "residual" else 1)
 
 
+@pytest.mark.parametrize("M,K,N,group,qtype,r,epi,reads", [
+    (128, 256, 33024, 64, Q.NF4, 0, "store", False),      # 258 tiles of 128 x 128, but one row block
+    (129, 256, 16384, 64, Q.NF4, 32, "residual", False),  # 256 tiles: one turn of the device
+    (129, 256, 16400, 64, Q.NF4, 32, "store", True),      # 258, a ragged last column tile and a row block of one row
+    (300, 128, 11008, 32, Q.INT4, 64, "silu", True),      # 258
+    (1300, 1152, 3072, 128, Q.INT4, 0, "residual", True),  # 264
+    (1024, 384, 4096, 64, Q.INT4, 64, "gelu", False),     # 256
+])
+def test_linears_between_the_kernels_read_their_copy(gpu, M, K, N, group, qtype, r, epi, reads):
+  """Fewer rows and tiles than the many-row kernel takes from the codes: a linear with a converted copy goes there as soon as
+  128 x 128 tiles no longer fit the device in one turn (a copy of NaN shows which calls read it), with the sums of the codes."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  mul = epi in ("silu", "gelu")
+  c, s = ops.quantize_pack(bf(rnd((K, N), 702, 0.02)).to(gpu), group, qtype, mul)
+  kw = {}
+  if epi == "residual":
+    kw["residual"] = bf(rnd((M, N), 703)).to(gpu)
+  if r:
+    widths = [N // 2, N // 2] if mul else [N]
+    kw.update(lora_rank=r, lora_nseg=-1 if mul else 1, lora_seg_end=[int(e) for e in np.cumsum(widths)], lora_seg_toff=[i * r for i in range(len(widths))],
+              t=bf(rnd((M, len(widths) * r), 704)).to(gpu), t_ld=len(widths) * r, lora_b=bf(rnd((N, r), 705, 0.1)).to(gpu), lora_scale=0.5)
+  e = {"store": L.TNX_EPI_STORE, "residual": L.TNX_EPI_RESIDUAL, "silu": L.TNX_EPI_SILU_MUL, "gelu": L.TNX_EPI_GELU_MUL}[epi]
+  x = bf(rnd((M, K), 701)).to(gpu)
+  copy = ops.qw_expand(c, s, K, N, group, qtype)
+  outs = []
+  for exp in (None, copy, torch.full_like(copy, float("nan"))):
+    y = torch.full((M, N // 2 if mul else N), float("nan"), dtype=torch.bfloat16, device=gpu)
+    ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=group, qtype=qtype, x=x, codes=c, scales=s, y=y, epilogue=e, w_expanded=exp, **kw))
+    outs.append(y)
+  torch.cuda.synchronize()
+  assert bool(outs[2].isnan().any()) == reads
+  assert not outs[0].isnan().any()
+  # the same bf16 products in another order of the float32 sum: one step of bf16 where a sum lies between two, which the gate and
+  # the residual's own rounding can make two and three
+  assert_bf16_close(outs[1], outs[0].float().cpu(), atol=1e-5 if mul else 1e-6, min_equal=0.9, what=f"copy {epi}",
+                    mag=(outs[0].float() - kw["residual"].float()).cpu() if epi == "residual" else None, ulps=3 if mul else 2 if epi == "residual" else 1)
+
+
 @pytest.mark.parametrize("M,K,R", [(12300, 256, 192), (6200, 384, 128), (700, 128, 32)])
 def test_lora_down_many_rows(gpu, M, K, R):
   """The MFMA flavours of the LoRA down-projection (128-, 64- and 32-row tiles, chosen by how many

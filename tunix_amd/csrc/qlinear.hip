@@ -924,12 +924,14 @@ int64_t moe_expanded_rows(int64_t K, int64_t N, int qtype) {
   return K <= 1024 ? 144 : K <= 8192 ? 176 + std::max<int64_t>(0, K - 2048) / 16 : 0;
 }
 
+// There is a converted copy, and its block offsets fit the kernel's 32 bits.
+bool copy_fits(const QLArgs& a) { return a.w_pre && cdiv(a.N, kWideCols) * (a.K / KTILE) * 65536 < (int64_t)1 << 31; }
+
 template <int SPT>
 int launch_qgemm_wide(hipStream_t st, const QLArgs& a, const WideHead& h = kNoHead) {
-  // the converted copy when the caller keeps one (its block offsets are 32-bit); else integer
-  // codes take the instantiation that converts them without the table
-  if (a.w_pre && cdiv(a.N, kWideCols) * (a.K / KTILE) * 65536 < (int64_t)1 << 31)
-    return launch_qgemm_pre(st, a, h);
+  // the converted copy when the caller keeps one; else integer codes take the instantiation that
+  // converts them without the table
+  if (copy_fits(a)) return launch_qgemm_pre(st, a, h);
   TNX_REQUIRE(a.codes && a.scales, "quantised GEMM: no packed weights and no usable expanded copy");
   return a.qtype == TNX_Q_INT4 ? launch_qgemm_wide_as<SPT, kWideInt4>(st, a, h)
                                : launch_qgemm_wide_as<SPT, kWideTable>(st, a, h);
@@ -981,6 +983,19 @@ bool wide_shape(const QLArgs& a, int64_t min_rows = 512, int64_t min_tiles = 256
     }
   }
   return true;
+}
+
+// Which linears take them: those whose 128 x 128 tiles of qgemm128_kernel no longer fit the device's
+// compute units in one turn, for its second turn costs as much as its first and tiles of 128 x 256
+// still need only one.  From 512 rows, and with a converted copy from the second row block on (below
+// that the codes' quarter of the bytes decides, and on two row blocks their conversion does).  us,
+// qgemm128_kernel | from the codes | from the copy: Llama-3.1-8B's o 44.9 | 60.7 | 51.6 at 1000 rows
+// (256 tiles), 81.8 | 63.1 | 54.4 at 1300; its down 129 | 173 | 179, 216 | 174 | 168, and 229 | 206 |
+// 178 at 1800; its q|k|v 37.5 | 55.4 | 58.0 at 512 rows (192), 69.3 | 56.4 | 55.6 at 700; its gate|up
+// 73.4 | 75.1 | 73.3 at 256 rows (448), 106 | 126 | 96 at 384; gemma-3-1b's gate|up 15.3 | 22.5 | 19.7
+// at 256 (216), 27.0 | 23.7 | 20.3 at 384 (324).
+bool many_rows(const QLArgs& a) {
+  return cdiv(a.M, 128) * cdiv(a.N, 128) > 256 && wide_shape(a, copy_fits(a) ? kWideRows + 1 : 512, 1);
 }
 
 template <int MT, int NT>
@@ -1147,7 +1162,7 @@ extern "C" int tnx_qlinear_lora(void* stream, const tnx_qlinear_desc* d) {
   // dispatched: its accumulators need AGPRs, and the compiler wraps loops over AGPR accumulators
   // in register copies that cost more than the halved LDS traffic gains.
   const bool s2 = scales_per_tile(a.group) == 2;
-  if (wide_shape(a)) return s2 ? launch_qgemm_wide<2>(st, a) : launch_qgemm_wide<4>(st, a);
+  if (many_rows(a)) return s2 ? launch_qgemm_wide<2>(st, a) : launch_qgemm_wide<4>(st, a);
   if (few_shape(a)) return launch_qgemm_few<false>(st, a, s2);
   if (a.M <= 64) return s2 ? launch_qgemm128<2, 2, 4>(st, a) : launch_qgemm128<2, 4, 4>(st, a);
   return s2 ? launch_qgemm128<2, 2, 8>(st, a) : launch_qgemm128<2, 4, 8>(st, a);

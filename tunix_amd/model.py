@@ -125,7 +125,7 @@ class FusedLinear:
   def expand(self):
     """Keeps a second copy of the frozen weight, converted to bf16 in the many-row kernel's
     fragment order (2 bytes per weight): prefill and per-token-logps passes then load it instead
-    of converting codes in their loop.  Decode steps never read it."""
+    of converting codes in their loop.  Decode steps of up to 128 rows never read it."""
     if self.expanded is None and self.wants_expansion():
       self.expanded = ops.qw_expand(self.codes, self.scales, self.K, self.N, self.group, self.qtype)
 
