@@ -82,8 +82,8 @@ const char* tnx_last_error(void);
  * tnx_rownorm_kvwrite, tnx_gated_state, tnx_poly_norm and tnx_route_scores; 6.1 adds
  * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora,
  * tnx_gqa_attn_lora, tnx_rope_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric; 6.4 adds tnx_qlinear_inner and
- * tnx_qlinear_inner_rows; 6.5 adds tnx_lmhead_commit and tnx_embed_norm; 6.6 adds tnx_gqa_attn_parts, tnx_qlinear_merged and
- * tnx_qlinear_merged_ok. */
+ * tnx_qlinear_inner_rows; 6.5 adds tnx_lmhead_commit and tnx_embed_norm; 6.6 adds tnx_gqa_attn_parts, tnx_qlinear_merged,
+ * tnx_qlinear_merged_ok, tnx_embed_packed, tnx_qknorm_rope_kvwrite_packed and tnx_gqa_attn_packed. */
 #define TNX_ABI_VERSION_MAJOR 6
 #define TNX_ABI_VERSION_MINOR 6
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
@@ -222,6 +222,17 @@ int tnx_lora_down(void* stream, const uint16_t* x, int64_t M, int64_t K, const u
 int tnx_embed(void* stream, const uint16_t* table, int64_t V, int64_t D, const int32_t* ids,
               int64_t ids_ld, const int32_t* col_ptr, int64_t B, int64_t T, float scale,
               uint16_t* out);
+/* Prompts padded on the left, without the padding: of prompt b only columns starts[b] .. T - 1 are rows, row row_base[b] + t that of column t; row_base[b] is what makes the
+ * prompts follow each other (the sum of the lengths before b, less starts[b]), rows the sum of all lengths, 0 <= starts[b] < T.  The *_packed entry points read and
+ * write activations in those rows, ids, positions and caches as ever; cache slots of padding are not written (a zero-filled cache keeps its zeros). */
+typedef struct tnx_packed_rows {
+  const int32_t* row_base;  /* [B] */
+  const int32_t* starts;    /* [B] */
+  int64_t rows;
+} tnx_packed_rows;
+int tnx_embed_packed(void* stream, const uint16_t* table, int64_t V, int64_t D, const int32_t* ids, int64_t ids_ld, int64_t B, int64_t T, float scale,
+                     const tnx_packed_rows* rows, uint16_t* out);
+
 
 /* RMSNorm over the last axis, three dtype flows.
  *   h = (res_pre ? bf16(x + res_pre) : x);  if (h_out) h_out = h;
@@ -341,6 +352,7 @@ typedef struct tnx_rope_desc {
   int split_k;
 } tnx_rope_desc;
 int tnx_qknorm_rope_kvwrite(void* stream, const tnx_rope_desc* h_desc);
+int tnx_qknorm_rope_kvwrite_packed(void* stream, const tnx_rope_desc* h_desc, const tnx_packed_rows* rows);
 /* sin / cos of positions[b, *col_ptr] / timescale[i], fp32 [B, dh/2] each: the angles of the
  * Llama rotation above for one decode step, shared by all layers (input of the fused mode of
  * tnx_gqa_attn). */
@@ -401,6 +413,8 @@ typedef struct tnx_attn_desc {
 } tnx_attn_desc;
 size_t tnx_attn_ws_bytes(int64_t B, int64_t T, int64_t S, int Hq, int dh, int kv_chunk);
 int tnx_gqa_attn(void* stream, const tnx_attn_desc* h_desc);
+/* The same for packed rows: kv_chunk 0, no rope_sin, no segment_ids, *col_ptr 0; slots in front of starts[b], whose ids are padding, are not looked at. */
+int tnx_gqa_attn_packed(void* stream, const tnx_attn_desc* h_desc, const tnx_packed_rows* rows);
 /* tnx_gqa_attn of a decode step (T == 1) with several key chunks, or with r tnx_rope_gqa_attn_lora (a_t null), without the pass that merges the chunks: out is not
  * written, ws holds for every query vector (row, head) and chunk dh + 4 numbers: a maximum m, a sum l, two of no meaning and O[dh]; the output is
  * sum_c e^(m_c - max m) O_c / sum_c e^(m_c - max m) l_c over the chunks whose l is not 0. */

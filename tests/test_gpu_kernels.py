@@ -2775,6 +2775,77 @@ def test_linear_that_merges_key_chunks_refuses(gpu):
   assert not ok(1, 4096, 4096, 48, 8, 128, 2) and not ok(1, 4096, 4096, 64, 8, 96, 2) and not ok(65, 1024, 1024, 32, 8, 256, 2)
 
 
+@pytest.mark.parametrize("dh,Hkv,G,T,B,window,family,split", [
+    (64, 2, 4, 5, 3, 0, "qwen3", 4),        # fewer positions than a tile pair; planes
+    (64, 2, 4, 64, 4, 0, "qwen3", 1),       # two tiles a wave, prompts that begin inside a tile of the one before's last rows
+    (64, 1, 3, 131, 3, 20, "qwen3", 1),
+    (128, 2, 4, 3, 5, 0, "llama3", 2),
+    (128, 2, 4, 200, 3, 0, "llama3", 1),    # work-groups of 32 positions
+    (128, 1, 16, 97, 4, 33, "llama3", 1),
+    (256, 1, 4, 70, 5, 16, "gemma3", 1),
+    (256, 1, 4, 300, 2, 0, "gemma3", 1),
+])
+def test_prompts_without_their_padding(gpu, dh, Hkv, G, T, B, window, family, split):
+  """Embedding, rotation with the cache write and attention of packed prompts against the padded ones, bit for bit in every row that is there; nothing else is
+  written: prompts of all columns, of one, and such as begin at and around the edges of tiles."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  from tunix_amd.model import _NORM, _ROPE
+  bf = torch.bfloat16
+  g = torch.Generator(device=gpu).manual_seed(T)
+  r = lambda *s: torch.randn(*s, generator=g, device=gpu)
+  Hq, S, V = Hkv * G, T + 7, 50
+  first = [0, T - 1, min(8, T - 2), min(33, T - 2), min(16, T - 1)][:B]
+  lengths = [T - f for f in first]
+  base = [sum(lengths[:b]) - first[b] for b in range(B)]
+  M, W = sum(lengths), (Hq + 2 * Hkv) * dh
+  at = torch.tensor([b * T + t for b in range(B) for t in range(first[b], T)], device=gpu)
+  i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)
+  starts, row_base, zero = i32(first), i32(base), i32([0])
+  packed = ops.packed_rows(row_base, starts, M)
+  ids = torch.randint(1, V, (B, S), generator=g, device=gpu, dtype=torch.int32)
+  for b, f in enumerate(first):
+    ids[b, :f] = 0
+  positions = (torch.arange(S, device=gpu, dtype=torch.int32)[None] - starts[:, None]).clamp(min=0).contiguous()
+  nan = lambda *s: torch.full(s, float("nan"), dtype=bf, device=gpu)
+  table = r(V, 96).to(bf)
+  e0, e1 = nan(B * T, 96), nan(M, 96)
+  ops.embed(table, ids, zero, B, T, 1.5, e0)
+  ops.embed(table, ids, zero, B, T, 1.5, e1, packed)
+  assert torch.equal(e0[at], e1)
+  src = r(split, B * T, W) * 0.5
+  full, part = src.contiguous(), src[:, at].contiguous()
+  wq, wk = r(dh).to(bf), r(dh).to(bf)
+  scale = 0.0 if family == "gemma3" else dh ** -0.5
+  ts = (10000.0 ** (torch.arange(dh // 2, device=gpu, dtype=torch.float32) * 2 / dh)).contiguous()
+  got = []
+  for rows, x, p in ((B * T, full, None), (M, part, packed)):
+    q, out = nan(rows, Hq * dh), nan(rows, Hq * dh)
+    kc, vc = torch.zeros(B, Hkv, S, dh, dtype=bf, device=gpu), torch.zeros(B, Hkv, S, dh, dtype=bf, device=gpu)
+    y = x[0].to(bf).contiguous()
+    rd = L.RopeDesc()
+    rd.B, rd.T, rd.S, rd.Hq, rd.Hkv, rd.dh = B, T, S, Hq, Hkv, dh
+    rd.rope_flavor, rd.rope_scale, rd.timescale = _ROPE[family], 1.0, ts.data_ptr()
+    rd.qk_norm, rd.norm_eps, rd.q_norm_w, rd.k_norm_w = (-1 if family == "llama3" else _NORM[family]), 1e-6, wq.data_ptr(), wk.data_ptr()
+    rd.q_prescale = dh ** -0.5 if family == "gemma3" else 0.0
+    rd.qkv, rd.positions, rd.pos_ld, rd.col_ptr = y.data_ptr(), positions.data_ptr(), S, zero.data_ptr()
+    if split > 1:
+      rd.qkv_ws, rd.split_k = x.data_ptr(), split
+    rd.q_out, rd.kcache, rd.vcache = q.data_ptr(), kc.data_ptr(), vc.data_ptr()
+    ops.rope_kvwrite(rd, p)
+    ad = L.AttnDesc()
+    ad.B, ad.T, ad.S, ad.Hq, ad.Hkv, ad.dh, ad.scale, ad.window, ad.pad_id = B, T, S, Hq, Hkv, dh, scale, window, 0
+    ad.q, ad.kcache, ad.vcache, ad.tokens, ad.tok_ld, ad.col_ptr, ad.out = (q.data_ptr(), kc.data_ptr(), vc.data_ptr(), ids.data_ptr(), S, zero.data_ptr(),
+                                                                            out.data_ptr())
+    ops.gqa_attn(ad, p)
+    got.append((q, out, kc, vc))
+  (q0, o0, k0, v0), (q1, o1, k1, v1) = got
+  assert torch.equal(q0[at], q1) and o1.isfinite().all() and torch.equal(o0[at], o1)
+  for b, f in enumerate(first):
+    assert torch.equal(k0[b, :, f:], k1[b, :, f:]) and torch.equal(v0[b, :, f:], v1[b, :, f:])
+    assert not k1[b, :, :f].any() and not v1[b, :, :f].any()
+
+
 @pytest.mark.parametrize("E,x_div", [(1, 3), (64, 1), (65, 2), (256, 1), (257, 3), (520, 4)])
 def test_many_rows_experts_are_found_among_any_number(gpu, E, x_div):
   """The search for a tile's expert, 256 of them at a time, and the rows of routes for divisors that are and are no powers of two: most experts

@@ -465,3 +465,35 @@ def test_top_k_equal_to_the_vocabulary_sorts_the_row(tiny, gpu):
   assert not all(np.array_equal(x, y) for x, y in zip(out.tokens, plain.tokens))
   with pytest.raises(ValueError, match="top_k"):
     sampler(prompts, T, max_prompt_length=P, temperature=0.8, top_p=1.0, top_k=V + 1, seed=3)
+
+
+@pytest.mark.parametrize("name,kw,P,lens,rows", [
+    ("tiny_qwen3", {}, 64, (64, 40, 1, 57, 0), 16384),
+    ("tiny_qwen3", {}, 64, (3, 40, 64, 57, 33), 130),          # groups of two prompts
+    ("gemma3_1b", dict(num_layers=2, vocab_size=2048), 40, (40, 17, 33), 16384),
+    ("llama31_8b", dict(num_layers=2, vocab_size=2048), 300, (290, 300), 16384),
+    ("qwen3_30b_a3b", dict(num_layers=1, vocab_size=2048, num_experts=16), 33, (9, 30, 33), 16384),
+])
+def test_prompts_packed_and_padded_give_the_same(gpu, monkeypatch, name, kw, P, lens, rows):
+  """The prompts' forward pass over their tokens alone and over the padded rows: the same tokens and the same bits of their log-probabilities.  (Groups of so few
+  rows that the linears take another kernel: the first token's log-probability within what the greedy tests allow against the oracle.)"""
+  from tunix_amd import config, dummy_model
+  from tunix_amd.generate.sampler import CacheConfig, Sampler
+  from tunix_amd.generate.utils import IdTokenizer
+  from tunix_amd.model import QLoRAModel
+  cfg = getattr(config, name)(**kw)
+  model = QLoRAModel(cfg, dummy_model.create_dummy_weights(cfg, seed=3), "cuda:0")
+  rng = np.random.default_rng(P)
+  prompts = [rng.integers(2, cfg.vocab_size, size=n).astype(np.int32) for n in lens]
+  sampler = Sampler(model, IdTokenizer(cfg.vocab_size), CacheConfig(P + 6), prefill_rows=rows)
+  outs, packed = [], []
+  packs = Sampler.packs
+  for on in (True, False):
+    monkeypatch.setattr(Sampler, "packs", staticmethod(lambda st, r: packed.append(packs(st, r)) or (packed[-1] and on)))
+    outs.append(sampler(prompts, 6, max_prompt_length=P, return_logprobs=True, eos_tokens=[-1]))
+  assert packed == [True, True]
+  first = [np.asarray([lp[0] for lp in o.logprobs]) for o in outs]
+  assert np.abs(first[0] - first[1]).max() <= 2e-2
+  if rows > 1000:
+    for a, b in zip(*(list(zip(o.tokens, o.logprobs)) for o in outs)):
+      assert np.array_equal(a[0], b[0]) and np.array_equal(np.asarray(a[1]), np.asarray(b[1]))

@@ -55,6 +55,10 @@ class RopeDesc(C.Structure):
   ]
 
 
+class PackedRows(C.Structure):
+  _fields_ = [("row_base", _p), ("starts", _p), ("rows", _i64)]
+
+
 class NormLoraDesc(C.Structure):
   _fields_ = [
       ("M", _i64), ("D", _i64), ("eps", _f32), ("flavor", _i32),
@@ -321,6 +325,9 @@ SIGNATURES = {
     "tnx_rope_table": (_i32, [_p, _p, _i64, _p, _i64, _p, _i32, _p, _p]),
     "tnx_attn_ws_bytes": (C.c_size_t, [_i64, _i64, _i64, _i32, _i32, _i32]),
     "tnx_gqa_attn": (_i32, [_p, C.POINTER(AttnDesc)]),
+    "tnx_embed_packed": (_i32, [_p, _p, _i64, _i64, _p, _i64, _i64, _i64, _f32, C.POINTER(PackedRows), _p]),
+    "tnx_qknorm_rope_kvwrite_packed": (_i32, [_p, C.POINTER(RopeDesc), C.POINTER(PackedRows)]),
+    "tnx_gqa_attn_packed": (_i32, [_p, C.POINTER(AttnDesc), C.POINTER(PackedRows)]),
     "tnx_gqa_attn_parts": (_i32, [_p, C.POINTER(RopeDesc), C.POINTER(AttnDesc)]),
     "tnx_gqa_attn_lora": (_i32, [_p, C.POINTER(AttnDesc), _p, _i32, _p, _i64]),
     "tnx_rope_gqa_attn_lora": (_i32, [_p, C.POINTER(RopeDesc), C.POINTER(AttnDesc), _p, _i32, _p, _i64]),

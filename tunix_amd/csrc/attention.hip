@@ -56,6 +56,7 @@ struct AttnArgs {
   int qkv_split;
   const float* rope_sin;      // fp32 [B, dh/2] of this step's positions; non-null switches the mode on
   const float* rope_cos;
+  PackedRows rows;             // prompts (T > 1) without their padding
 };
 
 
@@ -140,15 +141,19 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
 
   // query column of this lane (as B-fragment column and as softmax owner)
   const int g = lm & (a.Gp - 1), tq = qt * PT + (lm >> a.gp_shift);
-  const bool qvalid = g < a.G && tq < a.T;
+  const bool packed = FUSE == 0 && W == 1 && a.rows.base != nullptr;
+  const int start = packed ? a.rows.starts[b] : 0;
+  const int64_t row0 = packed ? a.rows.base[b] : b * a.T;   // a row's position 0
+  if (packed && qt * PT + PT <= start) return;
+  const bool qvalid = g < a.G && tq < a.T && tq >= start;
   const int c_n = col0 + tq;                              // cache slot of the query token
   const int lo_n = a.window > 0 ? max(0, c_n - a.window + 1) : 0;
-  const int64_t qvec = (b * a.T + (qvalid ? tq : 0)) * a.Hq + hkv * a.G + (qvalid ? g : 0);
+  const int64_t qvec = (row0 + (qvalid ? tq : a.T - 1)) * a.Hq + hkv * a.G + (qvalid ? g : 0);
 
   // key range of the tile
   const int t_last = min((int)a.T - 1, qt * PT + PT - 1);
   int k_hi = col0 + t_last;                               // inclusive
-  int k_lo = a.window > 0 ? max(0, col0 + qt * PT - a.window + 1) : 0;
+  int k_lo = max(start, a.window > 0 ? col0 + qt * PT - a.window + 1 : 0);
   if (a.kv_chunk > 0) {
     k_lo = max(k_lo, chunk * a.kv_chunk);
     k_hi = min(k_hi, chunk * a.kv_chunk + a.kv_chunk - 1);
@@ -702,9 +707,9 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const RopeArgs& r) 
       const int n = 4 * lq + i;
       const float l = __shfl(l_run, n, 64);
       const int gi = n & (a.Gp - 1), ti = qt * PT + (n >> a.gp_shift);
-      if (!(gi < a.G && ti < a.T) || !dvalid) continue;
+      if (!(gi < a.G && ti < a.T && ti >= start) || !dvalid) continue;
       const float inv = l > 0.f ? 1.0f / l : 0.f;
-      uint16_t* o = a.out + ((b * a.T + ti) * a.Hq + hkv * a.G + gi) * DH;
+      uint16_t* o = a.out + ((row0 + ti) * a.Hq + hkv * a.G + gi) * DH;
 #pragma unroll
       for (int h = 0; h < NH; ++h) {
         u32x4 w;
@@ -772,6 +777,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   const int64_t b = bz / a.QTG;
   // (the longest tiles of a row are handed out first: a tile's work grows with its position)
   const int qt0 = ((int)a.QTG - 1 - (int)(bz - (unsigned)b * a.QTG)) * QW;
+  const int start = a.rows.base ? a.rows.starts[b] : 0;
+  const int64_t row0 = a.rows.base ? a.rows.base[b] : b * a.T;   // a row's position 0
+  if ((qt0 + QW) * PT <= start) return;
   const int col0 = *a.col_ptr;
   const int g = lm & (a.Gp - 1);
 
@@ -781,10 +789,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
     const int tq = (qt0 + w) * PT + (lm >> a.gp_shift);
-    qvalid[w] = g < a.G && tq < a.T;
+    qvalid[w] = g < a.G && tq < a.T && tq >= start;
     c_n[w] = col0 + tq;
     lo_n[w] = a.window > 0 ? max(0, c_n[w] - a.window + 1) : 0;
-    const int64_t qvec = (b * a.T + (qvalid[w] ? tq : 0)) * a.Hq + hkv * a.G + (qvalid[w] ? g : 0);
+    const int64_t qvec = (row0 + (qvalid[w] ? tq : a.T - 1)) * a.Hq + hkv * a.G + (qvalid[w] ? g : 0);
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
       qf[w][j] = u32x4{0, 0, 0, 0};
@@ -794,7 +802,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
   // key range of the QW tiles together
   const int t_last = min((int)a.T - 1, (qt0 + QW) * PT - 1);
   const int k_hi = col0 + t_last;
-  const int k_lo = a.window > 0 ? max(0, col0 + qt0 * PT - a.window + 1) : 0;
+  const int k_lo = max(start, a.window > 0 ? col0 + qt0 * PT - a.window + 1 : 0);
 
   f32x4 O[QW][NH][8];
   float m_run[QW], l_run[QW];
@@ -963,9 +971,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
       const int n = 4 * lq + i;
       const float l = __shfl(lr, n, 64);
       const int gi = n & (a.Gp - 1), ti = (qt0 + w) * PT + (n >> a.gp_shift);
-      if (!(gi < a.G && ti < a.T) || !dvalid) continue;
+      if (!(gi < a.G && ti < a.T && ti >= start) || !dvalid) continue;
       const float inv = l > 0.f ? 1.0f / l : 0.f;
-      uint16_t* o = a.out + ((b * a.T + ti) * a.Hq + hkv * a.G + gi) * DH;
+      uint16_t* o = a.out + ((row0 + ti) * a.Hq + hkv * a.G + gi) * DH;
 #pragma unroll
       for (int h = 0; h < NH; ++h) {
         u32x4 wv;
@@ -1050,6 +1058,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // (the longest groups of a row are handed out first: a tile's work grows with its position)
   const int qt_wg = ((int)a.QTG - 1 - (int)(bz - (unsigned)b * a.QTG)) * (4 * QW);
   const int qt0 = qt_wg + wave * QW;
+  const int start = a.rows.base ? a.rows.starts[b] : 0;
+  const int64_t row0 = a.rows.base ? a.rows.base[b] : b * a.T;   // a row's position 0
+  if ((qt_wg + 4 * QW) * PT <= start) return;                   // (the whole work-group)
   const int col0 = *a.col_ptr;
   const int g = lm & (a.Gp - 1);
 
@@ -1059,10 +1070,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
     const int tq = (qt0 + w) * PT + (lm >> a.gp_shift);
-    qvalid[w] = g < a.G && tq < a.T;
+    qvalid[w] = g < a.G && tq < a.T && tq >= start;
     c_n[w] = col0 + tq;
     lo_n[w] = a.window > 0 ? max(0, c_n[w] - a.window + 1) : 0;
-    const int64_t qvec = (b * a.T + (qvalid[w] ? tq : 0)) * a.Hq + hkv * a.G + (qvalid[w] ? g : 0);
+    const int64_t qvec = (row0 + (qvalid[w] ? tq : a.T - 1)) * a.Hq + hkv * a.G + (qvalid[w] ? g : 0);
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
       qf[w][j] = u32x4{0, 0, 0, 0};
@@ -1070,11 +1081,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
   // key range of this wave's QW tiles (as in attn_tiles_kernel) and of the work-group's 4 QW
-  const bool wave_live = qt0 * PT < a.T;
+  const bool wave_live = qt0 * PT < a.T && (qt0 + QW) * PT > start;
   const int k_hi = col0 + min((int)a.T - 1, (qt0 + QW) * PT - 1);
-  const int k_lo = a.window > 0 ? max(0, col0 + qt0 * PT - a.window + 1) : 0;
+  const int k_lo = max(start, a.window > 0 ? col0 + qt0 * PT - a.window + 1 : 0);
   const int k_hi_wg = col0 + min((int)a.T - 1, (qt_wg + 4 * QW) * PT - 1);
-  const int k_lo_wg = a.window > 0 ? max(0, col0 + qt_wg * PT - a.window + 1) : 0;
+  const int k_lo_wg = max(start, a.window > 0 ? col0 + qt_wg * PT - a.window + 1 : 0);
   const int kb0_wg = k_lo_wg & ~31;
   const int nblk_wg = (((k_hi_wg & ~31) - kb0_wg) >> 5) + 1;
   const int kb0 = k_lo & ~31, kb_last = k_hi & ~31;
@@ -1258,7 +1269,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int ti = (qt0 + w) * PT + (lm >> a.gp_shift);
     if (!qvalid[w]) continue;
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t* o = a.out + ((b * a.T + ti) * a.Hq + hkv * a.G + g) * DH + 4 * lq;
+    uint16_t* o = a.out + ((row0 + ti) * a.Hq + hkv * a.G + g) * DH + 4 * lq;
 #pragma unroll
     for (int jj = 0; jj < 8 * NH; ++jj)
       *reinterpret_cast<u32x2*>(o + 16 * jj) = u32x2{pack2bf(O[w][jj][0] * inv, O[w][jj][1] * inv), pack2bf(O[w][jj][2] * inv, O[w][jj][3] * inv)};
@@ -1410,7 +1421,7 @@ static bool several_waves(const tnx_attn_desc* d, int n_chunks, int64_t keys_ove
 
 // The attention launch; combine: and, of a split key range, the pass that merges its chunks.  rope: what forms q and writes the step's
 // key and value in the same launch (checked by the caller), or null.
-static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine, const RopeArgs* rope = nullptr) {
+static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine, const RopeArgs* rope = nullptr, const tnx_packed_rows* packed = nullptr) {
   TNX_REQUIRE(d, "attn: null descriptor");
   TNX_REQUIRE(d->B > 0 && d->T > 0 && d->S > 0, "attn: B,T,S must be positive");
   TNX_REQUIRE(d->dh == 64 || d->dh == 128 || d->dh == 256, "attn: head_dim %d not in {64,128,256}", d->dh);
@@ -1441,7 +1452,12 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine, const Ro
   a.col_ptr = d->col_ptr; a.kv_chunk = d->kv_chunk;
   a.n_chunks = d->kv_chunk > 0 ? (int)cdiv(d->S, d->kv_chunk) : 1;
   a.ws = d->ws; a.out = d->out;
-  a.qkv_ws = nullptr; a.qkv = nullptr; a.qkv_split = 0; a.rope_sin = nullptr; a.rope_cos = nullptr;
+  a.qkv_ws = nullptr; a.qkv = nullptr; a.qkv_split = 0; a.rope_sin = nullptr; a.rope_cos = nullptr; a.rows = kAllRows;
+  if (packed) {
+    TNX_REQUIRE(d->kv_chunk == 0 && !d->rope_sin && !d->segment_ids, "attn: packed rows take no key chunks, rotation or segments");
+    const int rc = packed_args(packed, d->B, d->T, a.rows);
+    if (rc) return rc;
+  }
   if (d->rope_sin) {
     TNX_REQUIRE(d->T == 1 && d->dh == 128, "attn: the fused RoPE / cache write needs T == 1 and head_dim 128");
     TNX_REQUIRE(d->rope_cos && (d->qkv || d->qkv_ws), "attn: fused RoPE needs the sine / cosine table and the qkv output");
@@ -1465,7 +1481,7 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine, const Ro
     if (tv) hipLaunchKernelGGL((attn_kernel<DH, FUSE, true, W>), grid, dim3(64 * W), 0, st, a);
     else hipLaunchKernelGGL((attn_kernel<DH, FUSE, false, W>), grid, dim3(64 * W), 0, st, a);
   };
-  const bool waves = several_waves(d, a.n_chunks, 64);
+  const bool waves = !packed && several_waves(d, a.n_chunks, 64);
   auto launch_head_dim = [&](auto dh_c, auto fuse_c) {
     if (waves) launch_decode(dh_c, fuse_c, std::integral_constant<int, kAttnWaves>{});
     else launch_decode(dh_c, fuse_c, std::integral_constant<int, 1>{});
@@ -1548,6 +1564,10 @@ static int gqa_attn(void* stream, const tnx_attn_desc* d, bool combine, const Ro
 }
 
 extern "C" int tnx_gqa_attn(void* stream, const tnx_attn_desc* d) { return gqa_attn(stream, d, true); }
+extern "C" int tnx_gqa_attn_packed(void* stream, const tnx_attn_desc* d, const tnx_packed_rows* rows) {
+  TNX_REQUIRE(rows, "attn: null packed rows");
+  return gqa_attn(stream, d, true, nullptr, rows);
+}
 
 static int gqa_attn_lora(void* stream, const tnx_attn_desc* d, const uint16_t* a_t, int R, uint16_t* t, int64_t t_ld, const RopeArgs* rope) {
   TNX_REQUIRE(d && a_t && t, "attn_lora: null pointer");

@@ -411,9 +411,10 @@ void launch_rmsnorm_lora(hipStream_t st, int64_t M, int flavor, int in, const No
 
 __global__ void embed_kernel(const uint16_t* table, int64_t V, int64_t D, const int32_t* ids,
                              int64_t ids_ld, const int32_t* col_ptr, int64_t T, float scale_bf,
-                             uint16_t* out) {
-  const int64_t row = blockIdx.x;  // b*T + t
-  const int64_t b = row / T, t = row % T;
+                             uint16_t* out, const PackedRows rows) {
+  const int64_t b = blockIdx.x / T, t = blockIdx.x % T;
+  if (rows.base && t < rows.starts[b]) return;
+  const int64_t row = rows.base ? rows.base[b] + t : blockIdx.x;
   const int col = col_ptr ? *col_ptr : 0;
   int64_t id = ids[b * ids_ld + col + t];
   if (id < 0 || id >= V) id = 0;  // pad sentinels outside the vocabulary read row 0 (masked later)
@@ -444,8 +445,9 @@ __global__ void embed_kernel(const uint16_t* table, int64_t V, int64_t D, const 
 template <bool PLANES>
 __global__ void rope_kernel(const RopeArgs a) {
   __shared__ float red[4];
-  const uint32_t row = blockIdx.x;
-  const uint32_t b = row / (uint32_t)a.T, t = row - b * (uint32_t)a.T;
+  const uint32_t b = blockIdx.x / (uint32_t)a.T, t = blockIdx.x - b * (uint32_t)a.T;
+  if (a.rows.base && (int)t < a.rows.starts[b]) return;
+  const uint32_t row = a.rows.base ? (uint32_t)a.rows.base[b] + t : blockIdx.x;
   const int head = blockIdx.y;
   const int half = a.dh / 2, i = threadIdx.x, il = min(i, half - 1);
   const bool live = i < half, is_v = head >= a.Hq + a.Hkv, is_q = head < a.Hq, normed = a.qk_norm >= 0 && !is_v;
@@ -457,7 +459,7 @@ __global__ void rope_kernel(const RopeArgs a) {
   float x1, x2;
   float p1[8], p2[8];
   uint16_t h1 = 0, h2 = 0;
-  const int64_t plane = a.B * a.T * (int64_t)ld;
+  const int64_t plane = (a.rows.base ? a.rows.rows : a.B * a.T) * (int64_t)ld;
   if constexpr (PLANES) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -539,8 +541,9 @@ __global__ void rope_kernel(const RopeArgs a) {
 template <bool NORM>
 __global__ __launch_bounds__(256) void rope_rows_kernel(const RopeArgs a) {
   __shared__ float trig[2][256];   // [sine, cosine][pair]: head_dim at most 512
-  const uint32_t row = blockIdx.x;
-  const uint32_t b = row / (uint32_t)a.T, t = row - b * (uint32_t)a.T;
+  const uint32_t b = blockIdx.x / (uint32_t)a.T, t = blockIdx.x - b * (uint32_t)a.T;
+  if (a.rows.base && (int)t < a.rows.starts[b]) return;   // (uniform)
+  const uint32_t row = a.rows.base ? (uint32_t)a.rows.base[b] + t : blockIdx.x;
   const int half = a.dh / 2, CH = half / 8, heads = a.Hq + 2 * a.Hkv;
   const int ch = threadIdx.x % CH, h0 = threadIdx.x / CH, hstep = 256 / CH;
   const int col = *a.col_ptr;
@@ -630,8 +633,20 @@ extern "C" int tnx_embed(void* stream, const uint16_t* table, int64_t V, int64_t
   TNX_REQUIRE(table && ids && out, "embed: null pointer");
   TNX_REQUIRE(V > 0 && D > 0 && B > 0 && T > 0, "embed: bad shape");
   hipLaunchKernelGGL(embed_kernel, dim3((unsigned)(B * T)), dim3(256), 0, as_stream(stream), table,
-                     V, D, ids, ids_ld, col_ptr, T, host_round_bf16(scale), out);
+                     V, D, ids, ids_ld, col_ptr, T, host_round_bf16(scale), out, kAllRows);
   TNX_CHECK_LAUNCH("embed");
+  return TNX_OK;
+}
+
+extern "C" int tnx_embed_packed(void* stream, const uint16_t* table, int64_t V, int64_t D, const int32_t* ids, int64_t ids_ld, int64_t B, int64_t T, float scale,
+                                const tnx_packed_rows* packed, uint16_t* out) {
+  TNX_REQUIRE(table && ids && out, "embed: null pointer");
+  TNX_REQUIRE(V > 0 && D > 0 && B > 0 && T > 0, "embed: bad shape");
+  PackedRows rows;
+  const int rc = packed_args(packed, B, T, rows);
+  if (rc) return rc;
+  hipLaunchKernelGGL(embed_kernel, dim3((unsigned)(B * T)), dim3(256), 0, as_stream(stream), table, V, D, ids, ids_ld, nullptr, T, host_round_bf16(scale), out, rows);
+  TNX_CHECK_LAUNCH("embed_packed");
   return TNX_OK;
 }
 
@@ -770,9 +785,10 @@ extern "C" int tnx_rope_table(void* stream, const int32_t* positions, int64_t po
   return TNX_OK;
 }
 
-extern "C" int tnx_qknorm_rope_kvwrite(void* stream, const tnx_rope_desc* d) {
+static int qknorm_rope_kvwrite(void* stream, const tnx_rope_desc* d, const tnx_packed_rows* packed) {
   RopeArgs a;
-  const int rc = rope_args(d, a);
+  int rc = rope_args(d, a);
+  if (rc == TNX_OK && packed) rc = packed_args(packed, d->B, d->T, a.rows);
   if (rc) return rc;
   // many rows, from the finished linear output: the row kernel.  Its thread groups are a head's dh / 16 lanes, whole ones in a
   // work-group and, where they add up a head's squares, inside a wave and a power of two.
@@ -797,4 +813,9 @@ extern "C" int tnx_qknorm_rope_kvwrite(void* stream, const tnx_rope_desc* d) {
   else hipLaunchKernelGGL(rope_kernel<false>, grid, block, 0, as_stream(stream), a);
   TNX_CHECK_LAUNCH("qknorm_rope_kvwrite");
   return TNX_OK;
+}
+extern "C" int tnx_qknorm_rope_kvwrite(void* stream, const tnx_rope_desc* d) { return qknorm_rope_kvwrite(stream, d, nullptr); }
+extern "C" int tnx_qknorm_rope_kvwrite_packed(void* stream, const tnx_rope_desc* d, const tnx_packed_rows* rows) {
+  TNX_REQUIRE(rows, "rope: null packed rows");
+  return qknorm_rope_kvwrite(stream, d, rows);
 }

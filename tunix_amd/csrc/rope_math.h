@@ -4,6 +4,7 @@
 #include <string.h>
 
 #include "common.h"
+#include "packed_rows.h"
 
 namespace {
 
@@ -51,6 +52,7 @@ struct RopeArgs {
   uint16_t* vcache;
   const float* ws;   // split-k partial planes of the qkv linear instead of qkv, or null
   int split_k;
+  PackedRows rows;
 };
 
 // The rotated pair (x1, x2) of a q or k head, as bf16 values.
@@ -111,7 +113,7 @@ inline int rope_args(const tnx_rope_desc* d, RopeArgs& a) {
   a.q_prescale_bf = d->q_prescale != 0.f ? host_round_bf16(d->q_prescale) : 0.f;
   a.qkv = d->qkv; a.positions = d->positions; a.pos_ld = d->pos_ld; a.col_ptr = d->col_ptr;
   a.timescale = d->timescale; a.q_out = d->q_out; a.kcache = d->kcache; a.vcache = d->vcache;
-  a.ws = d->qkv_ws; a.split_k = d->split_k;
+  a.ws = d->qkv_ws; a.split_k = d->split_k; a.rows = kAllRows;
   return TNX_OK;
 }
 

@@ -63,7 +63,7 @@ class Replay:
     utils.check_positions(self.model, P)
     ids = np.array([utils.pad_to_length(np.asarray(e["tokens"], dtype=np.int32), P, PAD_ID, left=True) for e in entries])
     S = utils.next_power_of_2(P + 64)
-    st = _SamplingState(self.model, ids, S, S, PAD_ID, False, False, lengths=lengths)
+    st = _SamplingState(self.model, ids, S, S, PAD_ID, False, False, lengths=lengths, prefill_rows=self.sampler.prefill_rows)
     batch = _Batch([e["id"] for e in entries], st)
     out: list = [None] * len(entries)
 

@@ -64,7 +64,7 @@ class _SamplingState:
 
   def __init__(self, model, all_input_ids: np.ndarray, total_sampling_steps: int,
                cache_size: int, pad_id: int, include_logits: bool, include_logprobs: bool,
-               lengths: Sequence[int] | None = None):
+               lengths: Sequence[int] | None = None, prefill_rows: int = 16384):
     """lengths: tokens of each left-padded prompt (default: what follows the leading pad ids)."""
     cfg, dev = model.cfg, model.device
     B, P = all_input_ids.shape
@@ -84,7 +84,17 @@ class _SamplingState:
     self.step = torch.full((1,), P - 1, dtype=torch.int32, device=dev)
     self.tickets = torch.zeros(1, dtype=torch.int32, device=dev)   # tnx_commit_desc's
     # column of each row's first token
-    self.starts = torch.tensor([P - n for n in lengths], dtype=torch.int32, device=dev)
+    first = [P - n for n in lengths]
+    self.group = max(1, min(B, prefill_rows // max(P, 1)))   # prompts of one forward pass (`forward_prompt`)
+    self.padded = P > 1 and any(first)
+    if self.padded:
+      # and, of the pass without padding, a row's first column (a prompt of no token at all keeps its last one), the row of its column 0 and that of its last
+      self.first = np.minimum(first, P - 1)
+      base = np.concatenate([np.cumsum(P - f) - P for f in np.split(self.first, range(self.group, B, self.group))])
+      self.starts, self.prompt_starts, self.prompt_base, self.prompt_last = torch.from_numpy(
+          np.stack([first, self.first, base, base + P - 1]).astype(np.int32)).to(dev).unbind()
+    else:
+      self.starts = torch.tensor(first, dtype=torch.int32, device=dev)
     self.cache = model.new_cache(B, cache_size)
     self.logits_buffer = (torch.zeros(B, L, cfg.vocab_size, dtype=torch.float32, device=dev)
                           if include_logits else None)
@@ -183,17 +193,26 @@ class Sampler:
     if not entered:
       ops.sample_commit(ids, lp, st.token_buffer, st.logprobs_buffer, st.done, mode["eos"], st.step)
 
-  def forward_prompt(self, st: _SamplingState, on_rows):
+  def forward_prompt(self, st: _SamplingState, on_rows, packed: bool = False):
     """Forward over the padded prompts (sampler.py:554-616), filling the cache, in groups of rows:
-    on_rows(b0, nb, runner, xn) gets the final hidden states [nb * P, width] of rows b0 .. b0 + nb - 1."""
+    on_rows(b0, nb, runner, xn) gets the final hidden states [nb * P, width] of rows b0 .. b0 + nb - 1; packed: of their tokens only, without the padding,
+    that of a row's last token in row st.prompt_last[b]."""
     B, P = st.token_buffer.shape[0], st.num_input_tokens
-    rows = max(1, min(B, self.prefill_rows // max(P, 1)))
+    rows = st.group
     runner = self._transformer.new_runner(rows, P, st.cache.S, self.tokenizer.pad_id(), kv_chunk=0)
     for b0 in range(0, B, rows):
       nb = min(rows, B - b0)
+      kw = {}
+      if packed:
+        kw = dict(packed=ops.packed_rows(st.prompt_base[b0:b0 + nb], st.prompt_starts[b0:b0 + nb], int((P - st.first[b0:b0 + nb]).sum())))
       xn = runner.forward_hidden(st.token_buffer[b0:b0 + nb], st.positions[b0:b0 + nb], runner.zero,
-                                 st.cache.rows(b0, nb), B=nb, T=P, starts=st.starts[b0:b0 + nb])
+                                 st.cache.rows(b0, nb), B=nb, T=P, starts=st.starts[b0:b0 + nb], **kw)
       on_rows(b0, nb, runner, xn)
+
+  @staticmethod
+  def packs(st: _SamplingState, runner) -> bool:
+    """Whether the prompts' forward pass leaves their padding out."""
+    return getattr(runner, "packs_prompts", False) and st.padded
 
   def forward_step(self, runner, st: _SamplingState):
     """Forward over the one token per row in column `st.step`, from the cached state."""
@@ -203,9 +222,13 @@ class Sampler:
     """sampler.py:554-673: forward over the padded prompts, fill the cache, sample one token."""
     model = self._transformer
     P = st.num_input_tokens
+    packed = self.packs(st, runner_dec) and not return_logits
 
     def on_rows(b0, nb, runner, xn):
-      runner_dec.xlast[b0:b0 + nb].copy_(xn[: nb * P].view(nb, P, -1)[:, P - 1])
+      if packed:
+        torch.index_select(xn, 0, st.prompt_last[b0:b0 + nb], out=runner_dec.xlast[b0:b0 + nb])
+      else:
+        runner_dec.xlast[b0:b0 + nb].copy_(xn[: nb * P].view(nb, P, -1)[:, P - 1])
       if return_logits:
         # logits of every prompt position go to logits_buffer[:, 1:P+1] (sampler.py:617-625)
         part = torch.empty(nb * P * runner.nvb * 4, dtype=torch.float32, device=model.device)
@@ -217,7 +240,7 @@ class Sampler:
         n_fit = min(P, L - 1)
         st.logits_buffer[b0:b0 + nb, 1:1 + n_fit].copy_(lg[:, :n_fit])
 
-    self.forward_prompt(st, on_rows)
+    self.forward_prompt(st, on_rows, packed)
     self._sample(runner_dec, runner_dec.xlast, st, mode)
 
   def _decode_step(self, runner, st: _SamplingState, mode: dict):
@@ -295,7 +318,7 @@ class Sampler:
     B = all_input_ids.shape[0]
     S = self.cache_config.cache_size
     st = _SamplingState(model, all_input_ids, total_sampling_steps, S, pad, return_logits,
-                        return_logprobs, lengths=[len(x) for x in tokens])
+                        return_logprobs, lengths=[len(x) for x in tokens], prefill_rows=self.prefill_rows)
     mode = {"name": "greedy", "forbidden": None,
             "eos": torch.tensor(eos_ids, dtype=torch.int32, device=dev)}
     if forbidden:

@@ -741,18 +741,21 @@ class Runner(HeadRunner):
     self.h, self.h_next = self.h_next, self.h
     return True
 
-  def forward_hidden(self, tokens, positions, col_ptr, cache, B=None, T=None, segment_ids=None, starts=None):
+  packs_prompts = True   # forward_hidden takes `packed`
+
+  def forward_hidden(self, tokens, positions, col_ptr, cache, B=None, T=None, segment_ids=None, starts=None, packed=None):
     """Runs all layers for tokens[b, col .. col+T) of each row; leaves the final-normed hidden
     state in self.xn[:B*T].  cache: a SequenceCache of [B,Hkv,S,dh] slabs.  segment_ids (int32,
     the shape of `tokens`): a packed batch, attention stays inside a token's own segment.
-    starts: not read here, padding is told by its token id."""
+    starts: not read here, padding is told by its token id.  packed (`ops.packed_rows`): prompts from
+    column 0 on (T > 1) without the padding in front of them, their rows one behind the other in self.xn."""
     if segment_ids is not None and (tuple(segment_ids.shape) != tuple(tokens.shape)
                                     or segment_ids.dtype != torch.int32 or not segment_ids.is_contiguous()):
       raise ValueError("segment_ids must be a contiguous int32 tensor of the token buffer's shape")
     cfg, m = self.cfg, self.model
     B = self.B if B is None else B
     T = self.T if T is None else T
-    M = B * T
+    M = B * T if packed is None else packed.rows
     flavor = _NORM[cfg.family]
     emb_scale = math.sqrt(cfg.embed_dim) if cfg.family == "gemma3" else 1.0
     pending = 1  # split count of a down-projection whose partial planes still await their sum
@@ -765,12 +768,12 @@ class Runner(HeadRunner):
     # whether the first layer's rows are already normed into self.xn (gemma3: and any layer's, by the block before) and the qkv adapters'
     # down-projection of them formed
     xn_ready = t_ready = False
-    if m.layers and cfg.embed_dim % 32 == 0:
+    if m.layers and cfg.embed_dim % 32 == 0 and packed is None:
       a_t = adapter(m.layers[0]["qkv"])
       ops.embed_norm(m.embed, tokens, col_ptr, B, T, emb_scale, self.h, m.layers[0]["attn_norm"], self.xn, cfg.norm_eps, flavor, a_t, self.t, rope)
       xn_ready, t_ready = True, a_t is not None
     else:
-      ops.embed(m.embed, tokens, col_ptr, B, T, emb_scale, self.h)
+      ops.embed(m.embed, tokens, col_ptr, B, T, emb_scale, self.h, packed)
       if rope is not None:
         ops.rope_table(rope[0], col_ptr, B, *rope[1:])
     for i, ly in enumerate(m.layers):
@@ -802,7 +805,7 @@ class Runner(HeadRunner):
         rd.col_ptr = col_ptr.data_ptr()
         rd.q_out, rd.kcache, rd.vcache = self.q.data_ptr(), kv.k.data_ptr(), kv.v.data_ptr()
         if T > 1:
-          ops.rope_kvwrite(rd)
+          ops.rope_kvwrite(rd, packed)
       ad = L.AttnDesc()
       ad.B, ad.T, ad.S = B, T, self.S
       ad.Hq, ad.Hkv, ad.dh = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
@@ -822,7 +825,10 @@ class Runner(HeadRunner):
           ad.qkv = self.qkv.data_ptr()
         ad.rope_sin, ad.rope_cos = self.rope_sin.data_ptr(), self.rope_cos.data_ptr()
       o_ready, parts = not self.inner(ly["o"], M), self.merges(ly["o"], M) if T == 1 else None
-      if parts is not None:
+      if packed is not None:
+        o_ready = False   # (the adapter's down-projection of the packed rows is the linear's)
+        ops.gqa_attn(ad, packed)
+      elif parts is not None:
         ops.gqa_attn_parts(None if fuse_rope else rd, ad)
       elif T == 1 and not fuse_rope:
         ops.rope_gqa_attn_lora(rd, ad, adapter(ly["o"]) if o_ready else None, self.t)

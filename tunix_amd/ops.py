@@ -157,8 +157,20 @@ def lora_down(x, a_t, t, M=None):
           "tnx_lora_down")
 
 
-def embed(table, ids, col_ptr, B, T, scale, out):
+def packed_rows(row_base, starts, rows: int) -> L.PackedRows:
+  """B left-padded prompts without their padding: position t of prompt b, t >= starts[b], is row row_base[b] + t of `rows`."""
+  _expect(row_base, torch.int32, "packed_rows")
+  _expect(starts, torch.int32, "packed_rows")
+  p = L.PackedRows()
+  p.row_base, p.starts, p.rows = _ptr(row_base), _ptr(starts), rows
+  return p
+
+
+def embed(table, ids, col_ptr, B, T, scale, out, packed=None):
   V, D = table.shape
+  if packed is not None:   # (from column 0)
+    L.check(L.lib().tnx_embed_packed(_stream(), _ptr(table), V, D, _ptr(ids), ids.shape[1], B, T, float(scale), packed, _ptr(out)), "tnx_embed_packed")
+    return
   L.check(L.lib().tnx_embed(_stream(), _ptr(table), V, D, _ptr(ids), ids.shape[1], _ptr(col_ptr),
                             B, T, float(scale), _ptr(out)), "tnx_embed")
 
@@ -221,7 +233,10 @@ def embed_norm(table, ids, col_ptr, B, T, scale, h, w, y, eps, flavor, a_t=None,
   L.check(L.lib().tnx_embed_norm(_stream(), C.byref(e), C.byref(d)), "tnx_embed_norm")
 
 
-def rope_kvwrite(desc: L.RopeDesc):
+def rope_kvwrite(desc: L.RopeDesc, packed=None):
+  if packed is not None:
+    L.check(L.lib().tnx_qknorm_rope_kvwrite_packed(_stream(), C.byref(desc), packed), "tnx_qknorm_rope_kvwrite_packed")
+    return
   L.check(L.lib().tnx_qknorm_rope_kvwrite(_stream(), C.byref(desc)), "tnx_qknorm_rope_kvwrite")
 
 
@@ -234,7 +249,10 @@ def attn_ws_bytes(B, T, S, Hq, dh, kv_chunk) -> int:
   return int(L.lib().tnx_attn_ws_bytes(B, T, S, Hq, dh, kv_chunk))
 
 
-def gqa_attn(desc: L.AttnDesc):
+def gqa_attn(desc: L.AttnDesc, packed=None):
+  if packed is not None:
+    L.check(L.lib().tnx_gqa_attn_packed(_stream(), C.byref(desc), packed), "tnx_gqa_attn_packed")
+    return
   L.check(L.lib().tnx_gqa_attn(_stream(), C.byref(desc)), "tnx_gqa_attn")
 
 
