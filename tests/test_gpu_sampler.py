@@ -467,6 +467,31 @@ def test_top_k_equal_to_the_vocabulary_sorts_the_row(tiny, gpu):
     sampler(prompts, T, max_prompt_length=P, temperature=0.8, top_p=1.0, top_k=V + 1, seed=3)
 
 
+def test_captures_of_a_thread_share_a_stream(tiny, gpu):
+  """One stream per thread to capture on, whatever became of the capture before."""
+  import threading
+  from tunix_amd.generate.sampler import CacheConfig, Sampler, _capture_stream
+  from tunix_amd.generate.utils import IdTokenizer
+  cfg, _, model = tiny[:3]
+  sampler = Sampler(model, IdTokenizer(cfg.vocab_size), CacheConfig(32))
+  generate = lambda: sampler([[5, 6, 7]], 8, max_prompt_length=8, eos_tokens=[-1]).tokens[0]
+  want = generate()
+  mine, other = _capture_stream(gpu), []
+  x = torch.zeros(4, device=gpu)
+
+  def fails():
+    x.add_(1.0)
+    raise ValueError("a step that fails")
+
+  with pytest.raises(ValueError, match="a step that fails"):
+    sampler._captured(fails)
+  assert np.array_equal(generate(), want) and _capture_stream(gpu) is mine
+  t = threading.Thread(target=lambda: other.extend([_capture_stream(gpu), generate()]))
+  t.start()
+  t.join()
+  assert other[0] is not mine and np.array_equal(other[1], want)
+
+
 @pytest.mark.parametrize("name,kw,P,lens,rows", [
     ("tiny_qwen3", {}, 64, (64, 40, 1, 57, 0), 16384),
     ("tiny_qwen3", {}, 64, (3, 40, 64, 57, 33), 130),          # groups of two prompts
