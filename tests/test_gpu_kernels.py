@@ -2651,6 +2651,37 @@ def test_many_rows_from_the_expanded_copy(gpu, M, K, N):
     assert ((got - act * up).norm() / (act * up).norm()) < 2.0 ** -8, epilogue
 
 
+@pytest.mark.parametrize("M,K,N,rank,scale,residual", [
+    (4000, 256, 1152, 32, 1.0, False),     # 128 columns in the last tile, a ragged last row block
+    (3970, 640, 1152, 64, 0.75, True),     # an adapter's scale that is no power of two; two rows in the last block
+    (4097, 128, 1040, 64, 0.5, True),      # 16 columns, one row, one k-tile
+    (30000, 128, 144, 0, 1.0, False),      # one whole column tile's worth less: 144 = none whole, one of 144
+    (33000, 128, 80, 32, 1.0, True),       # no whole tile at all
+    (4100, 256, 1168, 32, 1.0, False),     # 144 columns in the last tile: no half
+])
+def test_last_column_tiles_of_half_the_width(gpu, M, K, N, rank, scale, residual):
+  """Calls whose last column tile has at most 128 columns, from the converted copy: the bits of the codes, which go through whole tiles."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  g = torch.Generator(device=gpu).manual_seed(N + M)
+  r = lambda *s: torch.randn(*s, generator=g, device=gpu)
+  c, s = ops.quantize_pack((r(K, N) * 0.02).bfloat16(), 64, Q.NF4)
+  x = r(M, K).bfloat16()
+  kw = {}
+  if residual:
+    kw["residual"] = r(M, N).bfloat16()
+  if rank:
+    kw.update(lora_rank=rank, lora_nseg=1, lora_seg_end=[N], lora_seg_toff=[0], t=r(M, rank).bfloat16(), t_ld=rank, lora_b=(r(N, rank) * 0.1).bfloat16(), lora_scale=scale)
+  outs = []
+  for copy in (ops.qw_expand(c, s, K, N, 64, Q.NF4), None):
+    y = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=gpu)
+    ops.qlinear(ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=Q.NF4, x=x, codes=c, scales=s, y=y, w_expanded=copy,
+                                      epilogue=L.TNX_EPI_RESIDUAL if residual else L.TNX_EPI_STORE, **kw))
+    outs.append(y)
+  torch.cuda.synchronize()
+  assert torch.equal(outs[0][:M].view(torch.int16), outs[1][:M].view(torch.int16)) and bool((outs[0][M] == 7.0).all())
+
+
 @pytest.mark.parametrize("M,K,widths", [(600, 256, (3968, 4112, 16)), (1000, 2048, (8176, 4096, 4112))])
 @pytest.mark.parametrize("rank", [32, 64])
 @pytest.mark.parametrize("scale", [1.0, 0.25, 0.75])

@@ -89,85 +89,24 @@ __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 
-template <int RT, bool GROUPED, int KIND, int LORA>
-__global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(RT == 16 ? 1 : RT == 8 ? 2 : 3, RT == 16 ? 1 : RT == 8 ? 2 : 3)))
-void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
-  constexpr int ROWS = 16 * RT, CT = 4, S = kPreStages, PASSES = RT / 2, HALF = RT / 4;   // PASSES: LDS loads of a step per thread
+// The tile of row block mtile and column tile ntile.  CT: 16-column tiles of a wave, four, or two in a last column tile with at most 128
+// columns (HALVES), which are divided among all four waves: half the MFMAs and weights of a whole tile, where two waves worked on columns that
+// are not there.  us, 14322 rows 6912 -> 1152 214 | 184, 1024 -> 1152 44.1 | 39.5 (448 whole tiles and 112 halves on 512 places); 8000 rows of the
+// second 29.9 | 26.4; where all fit in one turn (13000 rows) the same.  (The four waves by two halves of the rows, which reads the
+// weights twice: 194.)
+template <int RT, bool GROUPED, int KIND, int LORA, int CT>
+__device__ __forceinline__ void pre_tile(const QLArgs& a, const WideHead& h, int mtile, int ntile, int expert, int m_from, int m_end) {
+  constexpr int ROWS = 16 * RT, S = kPreStages, PASSES = RT / 2, HALF = RT / 4;   // PASSES: LDS loads of a step per thread
   constexpr uint32_t SB = pre_step_bytes<RT>();
-  extern __shared__ __align__(16) unsigned char smem[];   // (addressed absolutely: no static LDS in this kernel, checked by the host)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wn = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lq = lane >> 4;
-  const int tiles_m = (int)((a.M + ROWS - 1) / ROWS), tiles_n = (int)((a.N + kWideCols - 1) / kWideCols);
-  int mtile, ntile, expert = 0, m_from = 0, m_end = 0;
-  // tile number `tile` of row blocks x column tiles: in groups of `group` row blocks, inside a group column tile by column tile.  With groups of
-  // 1024 rows an XCD works on about 1024 rows x 8 column tiles at a time (2048 or 4096 rows: the same at 16 row tiles, 3 to 20 % slower at 8).
-  auto tile_in = [&](int tile, int row_blocks, int group) {
-    const int per_group = group * tiles_n, g = tile / per_group, r = tile % per_group;
-    const int gm = min(group, row_blocks - g * group);
-    mtile = g * group + r % gm;
-    ntile = r / gm;
-  };
-  constexpr int GR = 1024 / ROWS;
-  if constexpr (GROUPED) {
-    // Tiles expert by expert; every wave finds its own: 256 experts at a time, four to a lane, from one round trip for all their offsets and a running
-    // sum by DPP: it stands in front of a work-group's first load, a tenth of its time at short contractions (clock stamps).  With the places of the stored rows asked for
-    // at once (wide_out.h), us before (a round trip and a chain of exchanges through LDS per 64 experts, twice) | now: 57288 routes of 128 experts
-    // 768 -> 2048 286 | 262, 2048 -> 1536 gated 428 | 424; 65536 of 64 768 -> 2048 302 | 283, 2048 -> 768 232 | 225.
-    const int E = a.n_experts;
-    int from[4], to[4], nb[4], end[4];   // an expert's routes and its blocks; the blocks up to its last one
-    auto count = [&](int base, int before) -> int {   // returns `before` and the blocks of these experts
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        from[c] = a.offsets[min(base + 64 * c + lane, E)];
-        to[c] = a.offsets[min(base + 64 * c + lane + 1, E)];
-      }
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        nb[c] = (to[c] - from[c] + ROWS - 1) / ROWS;
-        end[c] = wave_scan(nb[c]) + before;
-        before = __builtin_amdgcn_readlane(end[c], 63);
-      }
-      return before;
-    };
-    int total = 0;
-    for (int base = 0; base < E; base += 256) total = count(base, total);
-    const int tile = xcd_tile((int)blockIdx.x, total * tiles_n);
-    if (tile < 0) return;   // past the last block (the grid covers an upper bound)
-    const int block = tile / tiles_n;
-    int found_at = 0, found_nb = 1;
-    for (int base = 0, before = 0; base < E; base += 256) {
-      if (E > 256) before = count(base, before);
-      bool found = false;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint64_t hit = __ballot(block < end[c] && block >= end[c] - nb[c]);   // (one lane: the blocks of an expert are its own)
-        if (hit) {
-          const int l = __builtin_ctzll(hit);
-          expert = base + 64 * c + l;
-          found_nb = __builtin_amdgcn_readlane(nb[c], l);
-          found_at = tile - (__builtin_amdgcn_readlane(end[c], l) - found_nb) * tiles_n;
-          m_from = __builtin_amdgcn_readlane(from[c], l);
-          m_end = __builtin_amdgcn_readlane(to[c], l);
-          found = true;
-        }
-      }
-      if (found) break;
-    }
-    // an expert of many rows in groups of 1024 rows or near it, equal ones, or its few last blocks would draw all weights for themselves:
-    // 8 experts of 8000 rows x 4096 -> 4096 took 2340 us with all row blocks per column tile against 1710 (256-row tiles), 2395 against
-    // 1760 (128); 8 of 1300 rows, eleven blocks, 340 us in groups of eight and three against 318 in one of eleven.
-    const int groups = max(1, (found_nb + GR / 2) / GR);
-    tile_in(found_at, found_nb, (found_nb + groups - 1) / groups);
-  } else {
-    tile_in(xcd_tile((int)blockIdx.x, tiles_m * tiles_n), tiles_m, GR);
-  }
+  const int tiles_n = (int)((a.N + kWideCols - 1) / kWideCols);
   // first row of the tile (GROUPED: first position in the sorted route list)
   const int64_t m0 = (int64_t)m_from + (int64_t)mtile * ROWS;
   const int rows_here = (int)min((int64_t)ROWS, (GROUPED ? (int64_t)m_end : a.M) - m0);
   const int ktiles = (int)(a.K / KTILE), ksteps = 2 * ktiles;
-  const int64_t ntiles = a.N / 16, ntile0 = ((int64_t)ntile * 4 + wn) * 4;   // first 16-column tile of this wave
+  const int64_t ntiles = a.N / 16, ntile0 = (int64_t)ntile * 16 + wn * CT;   // first 16-column tile of this wave
 
   // the activation resource starts at this work-group's first row: offsets stay small whatever M is, and rows past M
   // lie beyond the resource and read zeros (GROUPED: the whole buffer, rows are gathered)
@@ -205,7 +144,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
 #pragma unroll
     for (int c = 0; c < PASSES; ++c) dma(Src{rx, xbase, xstride, st * 128}, c, (uint32_t)st * SB);
   __builtin_amdgcn_sched_barrier(0);
-  const uint32_t evoff = (uint32_t)(wn * 16384 + (lq >> 1) * 1024 + (lq & 1) * 512 + lm * 16);
+  const uint32_t evoff = (uint32_t)(wn * (CT * 4096) + (lq >> 1) * 1024 + (lq & 1) * 512 + lm * 16);
   const int wt0 = ntile * ktiles;
 
   // LoRA: the two steps behind the last are the row block of t = bf16(x . A), columns [toff_a, +64) and [toff_b, +64) (the
@@ -306,14 +245,14 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
     for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
-        const int ct = (rt & 1) ? 3 - j : j;
+        const int ct = (rt & 1) ? CT - 1 - j : j;
         // (three waves per unit leave the weights of some slabs in accumulator registers, from which the compiler copies them right in front of
         // their use; the stream of the weights, which bounds this form, hides the wait states)
         if constexpr (RT == 4) mfma16_acc_wait(wr[U % S][ct], xf[rt], acc[rt][ct]);
         else mfma16_acc(wr[U % S][ct], xf[rt], acc[rt][ct]);
-        if (j == 1 && rt % HALF == HALF - 1) load_w(ic<UL>{}, rt / HALF, kt + ((U + 3) >> 2));
-        if (j == 2 && (rt & 3) == 1) dma(src, ((U & 1) ? 0 : HALF) + (rt >> 2), dbuf);
-        if (j == 3) xf[rt] = lds_ld128(xaddr[UN & 1] + (uint32_t)(rt * 2048) + ((UN >> 1) ? SB : 0u));
+        if (j == 1 && rt % (RT / CT) == RT / CT - 1) load_w(ic<UL>{}, rt / (RT / CT), kt + ((U + 3) >> 2));
+        if (j == CT / 2 && (rt & 3) == 1) dma(src, ((U & 1) ? 0 : HALF) + (rt >> 2), dbuf);
+        if (j == CT - 1) xf[rt] = lds_ld128(xaddr[UN & 1] + (uint32_t)(rt * 2048) + ((UN >> 1) ? SB : 0u));
         __builtin_amdgcn_sched_barrier(0);   // in the order written
       }
     }
@@ -335,13 +274,13 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) load_w(ic<2>{}, ct, 0);
   // step 0 has landed: behind it 2 PASSES + HALF loads into LDS and twelve fragments
-  tnx_wait_vm(2 * PASSES + HALF + 12);
+  tnx_wait_vm(2 * PASSES + HALF + 3 * CT);
   __syncthreads();
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) xf[rt] = lds_ld128(xaddr[0] + (uint32_t)(rt * 2048));
   // A barrier stands in front of the first read of a step.  The last load of that step was issued in the first slab of two steps
   // before; behind it a slab issues its last fragment load, and then come four slabs of HALF + 4 loads each.
-  constexpr int kBehind = 4 * (HALF + 4);
+  constexpr int kBehind = 4 * (HALF + CT);
   uint32_t b3 = 3 * SB, b4 = 0, b5 = SB;   // buffers of steps 2 kt + 3, + 4, + 5
   int kt = 0;
   do {   // (at least one k-tile: a loop that may not run would merge its accumulators with the zeros before it, copy by copy)
@@ -437,7 +376,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
       if (rt * 16 + lm >= rows_here) continue;
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        const int64_t col = (int64_t)ntile * kWideCols + wn * 64 + ct * 16 + 4 * lq;
+        const int64_t col = (int64_t)ntile * kWideCols + wn * (16 * CT) + ct * 16 + 4 * lq;
         float* o = y + (m0 + rt * 16 + lm) * a.ldy + col;
         if (col + 4 <= a.N && (a.ldy & 3) == 0) {
           *reinterpret_cast<f32x4*>(o) = acc[rt][ct];
@@ -466,7 +405,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         const f32x4 g = acc[rt][2 * c], u = acc[rt][2 * c + 1];
-        put((rt * 16 + lm) * sld + wn * 32 + c * 16 + 4 * lq, gated(g[0], u[0]), gated(g[1], u[1]), gated(g[2], u[2]), gated(g[3], u[3]));
+        put((rt * 16 + lm) * sld + wn * (8 * CT) + c * 16 + 4 * lq, gated(g[0], u[0]), gated(g[1], u[1]), gated(g[2], u[2]), gated(g[3], u[3]));
       }
   } else {
     auto stage_tile = [&](auto f) {
@@ -475,7 +414,7 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           const f32x4 v = acc[rt][ct];
-          put((rt * 16 + lm) * sld + wn * 64 + ct * 16 + 4 * lq, f(v[0]), f(v[1]), f(v[2]), f(v[3]));
+          put((rt * 16 + lm) * sld + wn * (16 * CT) + ct * 16 + 4 * lq, f(v[0]), f(v[1]), f(v[2]), f(v[3]));
         }
     };
     if constexpr (KIND == kPreRelu2) {
@@ -489,6 +428,96 @@ void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   }
   __syncthreads();
   wide_tile_out<ROWS, GROUPED, pre_head(KIND), mul>(a, h, ntile, m0, rows_here);
+}
+
+
+template <int RT, bool GROUPED, int KIND, int LORA, bool HALVES>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(RT == 16 ? 1 : RT == 8 ? 2 : 3, RT == 16 ? 1 : RT == 8 ? 2 : 3)))
+void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
+  constexpr int ROWS = 16 * RT;
+  extern __shared__ __align__(16) unsigned char smem[];   // (addressed absolutely: no static LDS in this kernel, checked by the host)
+  const int lane = threadIdx.x & 63;
+  const int tiles_m = (int)((a.M + ROWS - 1) / ROWS), tiles_n = (int)((a.N + kWideCols - 1) / kWideCols);
+  int mtile, ntile, expert = 0, m_from = 0, m_end = 0;
+  // tile number `tile` of row blocks x column tiles: in groups of `group` row blocks, inside a group column tile by column tile.  With groups of
+  // 1024 rows an XCD works on about 1024 rows x 8 column tiles at a time (2048 or 4096 rows: the same at 16 row tiles, 3 to 20 % slower at 8).
+  auto tile_in = [&](int tile, int row_blocks, int group) {
+    const int per_group = group * tiles_n, g = tile / per_group, r = tile % per_group;
+    const int gm = min(group, row_blocks - g * group);
+    mtile = g * group + r % gm;
+    ntile = r / gm;
+  };
+  constexpr int GR = 1024 / ROWS;
+  if constexpr (GROUPED) {
+    // Tiles expert by expert; every wave finds its own: 256 experts at a time, four to a lane, from one round trip for all their offsets and a running
+    // sum by DPP: it stands in front of a work-group's first load, a tenth of its time at short contractions (clock stamps).  With the places of the stored rows asked for
+    // at once (wide_out.h), us before (a round trip and a chain of exchanges through LDS per 64 experts, twice) | now: 57288 routes of 128 experts
+    // 768 -> 2048 286 | 262, 2048 -> 1536 gated 428 | 424; 65536 of 64 768 -> 2048 302 | 283, 2048 -> 768 232 | 225.
+    const int E = a.n_experts;
+    int from[4], to[4], nb[4], end[4];   // an expert's routes and its blocks; the blocks up to its last one
+    auto count = [&](int base, int before) -> int {   // returns `before` and the blocks of these experts
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        from[c] = a.offsets[min(base + 64 * c + lane, E)];
+        to[c] = a.offsets[min(base + 64 * c + lane + 1, E)];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        nb[c] = (to[c] - from[c] + ROWS - 1) / ROWS;
+        end[c] = wave_scan(nb[c]) + before;
+        before = __builtin_amdgcn_readlane(end[c], 63);
+      }
+      return before;
+    };
+    int total = 0;
+    for (int base = 0; base < E; base += 256) total = count(base, total);
+    const int tile = xcd_tile((int)blockIdx.x, total * tiles_n);
+    if (tile < 0) return;   // past the last block (the grid covers an upper bound)
+    const int block = tile / tiles_n;
+    int found_at = 0, found_nb = 1;
+    for (int base = 0, before = 0; base < E; base += 256) {
+      if (E > 256) before = count(base, before);
+      bool found = false;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint64_t hit = __ballot(block < end[c] && block >= end[c] - nb[c]);   // (one lane: the blocks of an expert are its own)
+        if (hit) {
+          const int l = __builtin_ctzll(hit);
+          expert = base + 64 * c + l;
+          found_nb = __builtin_amdgcn_readlane(nb[c], l);
+          found_at = tile - (__builtin_amdgcn_readlane(end[c], l) - found_nb) * tiles_n;
+          m_from = __builtin_amdgcn_readlane(from[c], l);
+          m_end = __builtin_amdgcn_readlane(to[c], l);
+          found = true;
+        }
+      }
+      if (found) break;
+    }
+    // an expert of many rows in groups of 1024 rows or near it, equal ones, or its few last blocks would draw all weights for themselves:
+    // 8 experts of 8000 rows x 4096 -> 4096 took 2340 us with all row blocks per column tile against 1710 (256-row tiles), 2395 against
+    // 1760 (128); 8 of 1300 rows, eleven blocks, 340 us in groups of eight and three against 318 in one of eleven.
+    const int groups = max(1, (found_nb + GR / 2) / GR);
+    tile_in(found_at, found_nb, (found_nb + groups - 1) / groups);
+  } else if constexpr (HALVES) {
+    // every XCD's share of the whole tiles, and behind it its share of the halves: the slots that the whole ones leave over take those,
+    // two in turn
+    const int id = (int)blockIdx.x, whole = tiles_m * (tiles_n - 1);
+    const int mine = (whole >> 3) + (int)((id & 7) < (whole & 7)), s = id >> 3;
+    if (s >= mine) {
+      const int half = xcd_tile((s - mine) * 8 + (id & 7), tiles_m);
+      if (half < 0) return;
+      pre_tile<RT, false, KIND, LORA, 2>(a, h, half, tiles_n - 1, 0, 0, 0);
+      return;
+    }
+    const int tile = xcd_tile(id, whole), per_group = GR * (tiles_n - 1), g = tile / per_group, r = tile % per_group;
+    const int gm = min(GR, tiles_m - g * GR);
+    mtile = g * GR + r % gm;
+    ntile = r / gm;
+  } else {
+    tile_in(xcd_tile((int)blockIdx.x, tiles_m * tiles_n), tiles_m, GR);
+  }
+  pre_tile<RT, GROUPED, KIND, LORA, 4>(a, h, mtile, ntile, expert, m_from, m_end);
 }
 
 }  // namespace

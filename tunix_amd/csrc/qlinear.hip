@@ -822,23 +822,34 @@ int launch_qgemm_wide_as(hipStream_t st, const QLArgs& a, const WideHead& h) {
 
 constexpr WideHead kNoHead{nullptr, nullptr, nullptr, 0, 1.0f, nullptr};
 
-template <int RT, bool GROUPED, int KIND, int LORA>
+template <int RT, bool GROUPED, int KIND, int LORA, bool HALVES = false>
 int launch_qgemm_pre_as(hipStream_t st, const QLArgs& a, const WideHead& h) {
   static std::once_flag once;
   static int attr_rc = TNX_OK;
   constexpr size_t kSmem = pre_smem_bytes<RT>();
-  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_pre_kernel<RT, GROUPED, KIND, LORA>, kSmem); });
+  std::call_once(once, [] { attr_rc = prepare_qgemm128(&qgemm_pre_kernel<RT, GROUPED, KIND, LORA, HALVES>, kSmem); });
   if (attr_rc) return attr_rc;
   // grouped: an upper bound of the row blocks, sum over the experts of ceil(rows / ROWS) <= n_routes / ROWS + E (work-groups
   // past the last block exit at once)
   const int64_t blocks = GROUPED ? a.M / (16 * RT) + a.n_experts : cdiv(a.M, 16 * RT);
-  hipLaunchKernelGGL((qgemm_pre_kernel<RT, GROUPED, KIND, LORA>), dim3((unsigned)(blocks * cdiv(a.N, kWideCols))), dim3(256), kSmem, st, a, h);
+  // HALVES: a multiple of eight, of what an XCD has at most of either kind
+  const int64_t tn = cdiv(a.N, kWideCols), wgs = HALVES ? 8 * (cdiv(blocks * (tn - 1), 8) + cdiv(blocks, 8)) : blocks * tn;
+  hipLaunchKernelGGL((qgemm_pre_kernel<RT, GROUPED, KIND, LORA, HALVES>), dim3((unsigned)wgs), dim3(256), kSmem, st, a, h);
   TNX_CHECK_LAUNCH("qgemm_pre");
   return TNX_OK;
 }
 
+// Whether the last column tile has at most 128 columns.
+bool half_column(int64_t N) { return N % kWideCols > 0 && N % kWideCols <= kWideCols / 2; }
+
 template <int RT, int KIND>
 int launch_qgemm_pre_lora(hipStream_t st, const QLArgs& a, const WideHead& h) {
+  if constexpr (RT == 8 && KIND == kPreStore)
+    if (half_column(a.N)) {
+      if (a.lora_rank <= 0) return launch_qgemm_pre_as<RT, false, KIND, 0, true>(st, a, h);
+      return lora_in_place(a.lora_scale) ? launch_qgemm_pre_as<RT, false, KIND, kLoraInPlace, true>(st, a, h)
+                                         : launch_qgemm_pre_as<RT, false, KIND, kLoraScaled, true>(st, a, h);
+    }
   if (a.lora_rank <= 0) return launch_qgemm_pre_as<RT, false, KIND, 0>(st, a, h);
   return lora_in_place(a.lora_scale) ? launch_qgemm_pre_as<RT, false, KIND, kLoraInPlace>(st, a, h)
                                      : launch_qgemm_pre_as<RT, false, KIND, kLoraScaled>(st, a, h);
@@ -874,7 +885,8 @@ int launch_qgemm_pre(hipStream_t st, const QLArgs& a, const WideHead& h) {
     return a.M <= 64 ? launch_qgemm_pre_as<4, false, kPreHeadOnce, 0>(st, a, h) : launch_qgemm_pre_as<8, false, kPreHeadOnce, 0>(st, a, h);
   const int64_t tn = cdiv(a.N, kWideCols);
   const double tall = (double)cdiv(cdiv(a.M, 256) * tn, 256) * (double)(a.K + 150);
-  const double low = 0.5 * (double)cdiv(cdiv(a.M, 128) * tn, 256) * 1.09 * (double)a.K;
+  const bool halves = half_column(a.N) && !h.part && (a.epilogue == TNX_EPI_STORE || a.epilogue == TNX_EPI_RESIDUAL);
+  const double low = 0.5 * (double)cdiv(cdiv(a.M, 128) * (2 * tn - halves), 512) * 1.09 * (double)a.K;
   // (the noise of a draw is vector work, which two work-groups per unit put under each other's loads: 2048 x 151936 over 400 rows 634 us at 256 rows
   // of a tile, 468 at 128; 65536 x 2048 over 256 rows 144 | 130, over 160, more than a third of the second 128 missing, 108 | 137)
   if (h.part_draw && a.M > 160) return launch_qgemm_pre_rt<8>(st, a, h);
