@@ -83,7 +83,8 @@ const char* tnx_last_error(void);
  * tnx_moe_gmm_expanded and tnx_qw_expand_bank; 6.2 adds tnx_moe_expanded_rows; 6.3 adds tnx_norm_lora,
  * tnx_gqa_attn_lora, tnx_rope_gqa_attn_lora, tnx_grpo_ratio_flags and tnx_weighted_metric; 6.4 adds tnx_qlinear_inner and
  * tnx_qlinear_inner_rows; 6.5 adds tnx_lmhead_commit and tnx_embed_norm; 6.6 adds tnx_gqa_attn_parts, tnx_qlinear_merged,
- * tnx_qlinear_merged_ok, tnx_embed_packed, tnx_qknorm_rope_kvwrite_packed and tnx_gqa_attn_packed. */
+ * tnx_qlinear_merged_ok, tnx_embed_packed, tnx_qknorm_rope_kvwrite_packed, tnx_gqa_attn_packed, tnx_moe_gmm_unsorted and
+ * tnx_moe_gmm_unsorted_ok. */
 #define TNX_ABI_VERSION_MAJOR 6
 #define TNX_ABI_VERSION_MINOR 6
 #define TNX_ABI_VERSION ((TNX_ABI_VERSION_MAJOR << 16) | TNX_ABI_VERSION_MINOR)
@@ -587,6 +588,10 @@ typedef struct tnx_moe_gmm_desc {
   uint16_t* y;               /* bf16 [n_routes, N or N/2], indexed by route                  */
 } tnx_moe_gmm_desc;
 int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* h_desc);
+/* The same from the expert ids themselves, topk_id int32 [n_routes / k, k], distinct within a row: offsets and sorted_route are not read, and
+ * no tnx_moe_sort_routes is needed in front.  For the calls of which tnx_moe_gmm_unsorted_ok says 1 (decode steps of up to 128 rows). */
+int tnx_moe_gmm_unsorted(void* stream, const tnx_moe_gmm_desc* h_desc, const int32_t* topk_id);
+int tnx_moe_gmm_unsorted_ok(const tnx_moe_gmm_desc* h_desc);
 /* The same with a second copy of the weights: every expert's tnx_qw_expand output, behind each other
  * (tnx_qw_expanded_bytes(K, N) apart).  Calls with enough rows per expert read the copy, others the codes. */
 int tnx_moe_gmm_expanded(void* stream, const tnx_moe_gmm_desc* h_desc, const uint16_t* w_expanded);

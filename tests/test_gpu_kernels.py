@@ -2049,6 +2049,63 @@ def test_moe_gmm_rows_in_lds(gpu, E, n_tok, k, K, N, group, qtype, mul, off):
   test_moe_gmm_skewed_routes(gpu, E, n_tok, k, K, N, group, qtype, mul, off)
 
 
+@pytest.mark.parametrize("E,M,k,K,N,group,qtype,mul", [
+    (128, 64, 8, 256, 128, 128, Q.INT4, True),
+    (128, 1, 8, 256, 128, 64, Q.NF4, False),
+    (65, 63, 3, 128, 96, 64, Q.NF4, True),
+    (16, 65, 2, 256, 64, 32, Q.INT4, False),      # rows in both words of an expert's bits; experts of several blocks
+    (300, 128, 8, 128, 64, 128, Q.INT4, True),    # 1024 routes, several turns of 64 experts
+    (200, 128, 16, 128, 32, 64, Q.NF4, False),    # 2048: more than the work-group has threads
+    (3, 2, 3, 128, 32, 64, Q.INT4, False),        # every expert for every row
+    (64, 16, 4, 128, 64, 64, Q.INT4, True),
+])
+def test_moe_linears_that_sort_the_routes(gpu, E, M, k, K, N, group, qtype, mul):
+  """The experts' linear from the ids alone against the sorted routes: the same bits, also where most rows choose the same experts."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  g = torch.Generator(device=gpu).manual_seed(E + M)
+  w = [ops.quantize_pack((torch.randn(K, N, generator=g, device=gpu) * 0.05).bfloat16(), group, qtype, mul) for _ in range(min(E, 8))]
+  codes, scales = (torch.cat([w[e % len(w)][i].reshape(-1) for e in range(E)]) for i in (0, 1))
+  x = torch.randn(M if mul else M * k, K, generator=g, device=gpu).bfloat16()
+  for skew in (0.0, 4.0):
+    scores = torch.randn(M, E, generator=g, device=gpu) - skew * torch.arange(E, device=gpu) / E
+    ids = scores.topk(k, dim=1).indices.int().contiguous()
+    cnt, offs, sr = (torch.empty(n, dtype=torch.int32, device=gpu) for n in (E, E + 1, M * k))
+    ops.moe_sort_routes(ids, E, cnt, offs, sr)
+    outs = []
+    for unsorted in (False, True):
+      y = torch.full((M * k, N // 2 if mul else N), float("nan"), dtype=torch.bfloat16, device=gpu)
+      d = L.MoeGmmDesc()
+      d.n_routes, d.E, d.k, d.K, d.N, d.group, d.qtype = M * k, E, k, K, N, group, qtype
+      d.x, d.x_div, d.codes, d.scales = x.data_ptr(), k if mul else 1, codes.data_ptr(), scales.data_ptr()
+      d.epilogue, d.y = (L.TNX_EPI_SILU_MUL if mul else L.TNX_EPI_STORE), y.data_ptr()
+      assert ops.moe_gmm_unsorted_ok(d)
+      if unsorted:
+        ops.moe_gmm_unsorted(d, ids)
+      else:
+        d.offsets, d.sorted_route = offs.data_ptr(), sr.data_ptr()
+        ops.moe_gmm(d)
+      outs.append(y)
+    torch.cuda.synchronize()
+    assert not outs[0].isnan().any() and torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16)), skew
+
+
+def test_moe_linears_that_sort_refuse(gpu):
+  """More than 128 rows, a part of a row, more rows per expert than the streaming kernel takes, and ids of another number."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  z = torch.zeros(1 << 16, dtype=torch.int32, device=gpu)
+  for E, n_routes, k in ((64, 129 * 2, 2), (64, 127, 2), (4, 128, 2)):
+    d = L.MoeGmmDesc()
+    d.n_routes, d.E, d.k, d.K, d.N, d.group, d.qtype, d.x_div = n_routes, E, k, 128, 64, 64, Q.INT4, 1
+    d.x = d.codes = d.scales = d.y = z.data_ptr()
+    assert not ops.moe_gmm_unsorted_ok(d)
+    with pytest.raises(ValueError, match="not a shape it takes"):
+      ops.moe_gmm_unsorted(d, z[:n_routes])
+  with pytest.raises(ValueError, match="all routes"):
+    ops.moe_gmm_unsorted(d, z[:n_routes + 1])
+
+
 def test_argument_errors_raise(gpu):
   from tunix_amd import ops
   with pytest.raises(ValueError, match="K % 128"):

@@ -350,6 +350,8 @@ SIGNATURES = {
     "tnx_qlinear_merged": (_i32, [_p, C.POINTER(QLinearDesc), _p, _p, _i32, _i32]),
     "tnx_qlinear_merged_ok": (_i32, [_i64, _i64, _i64, _i32, _i32, _i32, _i32]),
     "tnx_moe_gmm_expanded": (_i32, [_p, C.POINTER(MoeGmmDesc), _p]),
+    "tnx_moe_gmm_unsorted": (_i32, [_p, C.POINTER(MoeGmmDesc), _p]),
+    "tnx_moe_gmm_unsorted_ok": (_i32, [C.POINTER(MoeGmmDesc)]),
     "tnx_moe_expanded_rows": (_i64, [_i64, _i64, _i32]),
     "tnx_moe_combine": (_i32, [_p, _p, _p, _i64, _i32, _i64, _p, _p]),
     "tnx_grpo_ratio": (_i32, [_p, _p, _p, _p, _i64, _i64, _f32, _f32, _p, _p, _p]),

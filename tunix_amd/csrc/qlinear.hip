@@ -37,6 +37,7 @@ struct QLArgs {
   const int32_t* sorted_route;
   int x_div;
   int n_experts;
+  int top_k;   // offsets null: sorted_route holds the expert ids of every row's top_k routes, and the kernel sorts them (moe_gmm16.h)
   int64_t codes_stride, scales_stride;  // per-expert strides in elements
   // fused down-projection of the next linear's adapter (*_MUL epilogue of qgemm128)
   const uint16_t* next_a_t;
@@ -1044,6 +1045,15 @@ bool moe16_staged(const QLArgs& a, int E, bool int4, bool mul, int cus) {
   return ((uintptr_t)a.x & 15) == 0 && moe16_staged_bytes(int4, mul, E, a.M, items, rows, a.K) <= kMoeLds;
 }
 
+// Whether the staged form, which sorts the routes of at most 128 rows for itself, takes the call: what falls to a work-group in LDS has to hold the
+// experts' bits of them.
+bool moe16_unsorted(const QLArgs& a, int E, int k, int cus) {
+  if (a.M % k != 0 || a.M / k > 128 || a.M > 4096) return false;
+  const bool int4 = a.qtype == TNX_Q_INT4;
+  return moe16_staged(a, E, int4, a.epilogue == TNX_EPI_SILU_MUL, cus) &&
+         (int4 ? 0 : kBigLutBytes) + moe16_meta_bytes(E, a.M) + (size_t)E * 16 <= kMoeLds;
+}
+
 template <bool MUL, int SPT, bool INT4, bool STAGED>
 int launch_moe16_k(hipStream_t st, const QLArgs& a, int E, int cus) {
   static std::once_flag once;
@@ -1431,13 +1441,15 @@ extern "C" int tnx_lora_down(void* stream, const uint16_t* x, int64_t M, int64_t
   return TNX_OK;
 }
 
-static int moe_gmm(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_expanded) {
+// topk_id: instead of the sorted routes, for the kernel that sorts for itself (moe16_unsorted), or null.  dry: only whether that kernel
+// would take the call, 1 or 0
+static int moe_gmm(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_expanded, const int32_t* topk_id = nullptr, bool dry = false) {
   TNX_REQUIRE(d, "moe_gmm: null descriptor");
   TNX_REQUIRE(d->n_routes > 0 && d->E > 0 && d->k > 0, "moe_gmm: bad shape");
   size_t cb = 0, sb = 0;
   int rc = tnx_qw_sizes(d->K, d->N, d->group, &cb, &sb);
   if (rc) return rc;
-  TNX_REQUIRE(d->x && d->codes && d->scales && d->offsets && d->sorted_route && d->y, "moe_gmm: null pointer");
+  TNX_REQUIRE(d->x && d->codes && d->scales && ((d->offsets && d->sorted_route) || topk_id || dry) && d->y, "moe_gmm: null pointer");
   TNX_REQUIRE(d->x_div >= 1, "moe_gmm: x_div must be >= 1");
   TNX_REQUIRE((uint64_t)(d->n_routes + 128) * (uint64_t)d->K * 2 < (1ull << 32),
               "moe_gmm: activations must stay below 4 GiB (32-bit buffer offsets)");
@@ -1466,7 +1478,7 @@ static int moe_gmm(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_ex
   // A3B shape, gate|up + down: 134 + 82 us against 152 + 102 us at 32 rows, 144 + 93 against
   // 271 + 179 us at 64; at 16 rows the 32-row tiles win, 97 + 60 against 130 + 76 us).
   const bool mul = d->epilogue == TNX_EPI_SILU_MUL;
-  if (avg_rows > 24 && d->N % kWideCols == 0 && (mul ? d->N / 2 : d->N) % 8 == 0 && ((uintptr_t)d->y & 15) == 0 &&
+  if (avg_rows > 24 && !topk_id && !dry && d->N % kWideCols == 0 && (mul ? d->N / 2 : d->N) % 8 == 0 && ((uintptr_t)d->y & 15) == 0 &&
       (uint64_t)(d->n_routes / d->x_div) * (uint64_t)d->K * 2 < 0xfffff000ull && d->n_routes % d->x_div == 0)
   {
     // from the experts' converted copies where those are worth four times the bytes
@@ -1482,14 +1494,32 @@ static int moe_gmm(void* stream, const tnx_moe_gmm_desc* d, const uint16_t* w_ex
   // at 10 rows per expert, 90 + 49 against 96 + 58 us at 12, 112 + 54 against 98 + 60 us at 16.
   if (max_rows <= 16 || avg_rows <= 12) {
     const int cus = device_cus();
-    if (moe16_shape(a, d->E, cb, sb, cus)) return launch_moe16(st, a, d->E, cus);
+    const bool streamed = moe16_shape(a, d->E, cb, sb, cus);
+    if (topk_id || dry) {
+      const bool takes = streamed && moe16_unsorted(a, d->E, d->k, cus);
+      if (dry) return takes;
+      TNX_REQUIRE(takes, "moe_gmm_unsorted: not a shape it takes");
+      a.offsets = nullptr;
+      a.sorted_route = topk_id;
+      a.top_k = d->k;
+    }
+    if (streamed) return launch_moe16(st, a, d->E, cus);
   }
+  if (dry) return 0;
+  TNX_REQUIRE(!topk_id, "moe_gmm_unsorted: not a shape it takes");
   if (max_rows <= 16 || avg_rows <= 8) return launch_moe<1, 2>(st, a, d->E, max_rows);
   if (max_rows <= 32 || avg_rows <= 24) return launch_moe<2, 2>(st, a, d->E, max_rows);
   return launch_moe<4, 2>(st, a, d->E, max_rows);
 }
 
 extern "C" int tnx_moe_int4_gmm(void* stream, const tnx_moe_gmm_desc* d) { return moe_gmm(stream, d, nullptr); }
+
+extern "C" int tnx_moe_gmm_unsorted_ok(const tnx_moe_gmm_desc* d) { return d && moe_gmm(nullptr, d, nullptr, nullptr, true) == 1; }
+
+extern "C" int tnx_moe_gmm_unsorted(void* stream, const tnx_moe_gmm_desc* d, const int32_t* topk_id) {
+  TNX_REQUIRE(topk_id, "moe_gmm_unsorted: null pointer");
+  return moe_gmm(stream, d, nullptr, topk_id);
+}
 
 extern "C" int64_t tnx_moe_expanded_rows(int64_t K, int64_t N, int qtype) {
   return K > 0 && N > 0 && K % KTILE == 0 ? moe_expanded_rows(K, N, qtype) : 0;

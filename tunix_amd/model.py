@@ -873,7 +873,6 @@ class Runner(HeadRunner):
     if not scored:
       ops.lora_down(self.xn, ex.router_t, self.scores, M=M)          # dense bf16 router
     ops.moe_route_topk(self.scores[:M], k, self.topk_w, self.topk_id)
-    ops.moe_sort_routes(self.topk_id[:M], E, self.counts, self.offsets, self.sorted_route)
     d = L.MoeGmmDesc()
     d.n_routes, d.E, d.k, d.K, d.N = M * k, E, k, ex.D, 2 * ex.F
     d.group, d.qtype = cfg.group, cfg.qtype
@@ -881,7 +880,6 @@ class Runner(HeadRunner):
     d.codes, d.scales = ex.gu_codes.data_ptr(), ex.gu_scales.data_ptr()
     d.offsets, d.sorted_route = self.offsets.data_ptr(), self.sorted_route.data_ptr()
     d.epilogue, d.y = L.TNX_EPI_SILU_MUL, self.act.data_ptr()
-    ops.moe_gmm(d, ex.gu_expanded)
     d2 = L.MoeGmmDesc()
     d2.n_routes, d2.E, d2.k, d2.K, d2.N = M * k, E, k, ex.F, ex.D
     d2.group, d2.qtype = cfg.group, cfg.qtype
@@ -889,7 +887,13 @@ class Runner(HeadRunner):
     d2.codes, d2.scales = ex.dn_codes.data_ptr(), ex.dn_scales.data_ptr()
     d2.offsets, d2.sorted_route = self.offsets.data_ptr(), self.sorted_route.data_ptr()
     d2.epilogue, d2.y = L.TNX_EPI_STORE, self.y_route.data_ptr()
-    ops.moe_gmm(d2, ex.dn_expanded)
+    if M <= 128 and ops.moe_gmm_unsorted_ok(d) and ops.moe_gmm_unsorted_ok(d2):   # (the linears of a decode step sort the routes for themselves)
+      ops.moe_gmm_unsorted(d, self.topk_id[:M])
+      ops.moe_gmm_unsorted(d2, self.topk_id[:M])
+    else:
+      ops.moe_sort_routes(self.topk_id[:M], E, self.counts, self.offsets, self.sorted_route)
+      ops.moe_gmm(d, ex.gu_expanded)
+      ops.moe_gmm(d2, ex.dn_expanded)
     if cfg.embed_dim % 8 == 0:   # the next norm adds the weighted combine to the residual stream
       return _MOE_PENDING
     ops.moe_combine(self.y_route, self.topk_w, M, k, cfg.embed_dim, self.h, self.h)

@@ -356,6 +356,17 @@ def moe_gmm(desc: L.MoeGmmDesc, w_expanded=None):
     L.check(L.lib().tnx_moe_gmm_expanded(_stream(), C.byref(desc), _ptr(w_expanded)), "tnx_moe_gmm_expanded")
 
 
+def moe_gmm_unsorted_ok(desc: L.MoeGmmDesc) -> bool:
+  return L.lib().tnx_moe_gmm_unsorted_ok(C.byref(desc)) == 1
+
+
+def moe_gmm_unsorted(desc: L.MoeGmmDesc, topk_id):
+  """`moe_gmm` of a decode step from the expert ids [rows, k], without `moe_sort_routes` in front."""
+  if topk_id.numel() != desc.n_routes or topk_id.dtype != torch.int32 or not topk_id.is_contiguous():
+    raise ValueError("topk_id must hold the int32 expert ids of all routes")
+  L.check(L.lib().tnx_moe_gmm_unsorted(_stream(), C.byref(desc), _ptr(topk_id)), "tnx_moe_gmm_unsorted")
+
+
 def moe_combine(y, topk_w, M, k, D, residual, out):
   L.check(L.lib().tnx_moe_combine(_stream(), _ptr(y), _ptr(topk_w), M, k, D, _ptr(residual),
                                   _ptr(out)), "tnx_moe_combine")
