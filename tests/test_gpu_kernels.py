@@ -2669,7 +2669,8 @@ def test_mul_epilogue_fuses_next_adapter_projection(gpu, M, F, r):
 
 
 # (the second half of the shapes runs 256-row tiles, the first 128-row ones: what fills the device better)
-PRE_SHAPES = [(65, 128, 16), (128, 256, 272), (129, 384, 48), (255, 128, 528), (769, 2048, 16304), (1024, 2048, 16384), (1023, 2176, 16144)]
+PRE_SHAPES = [(65, 128, 16), (128, 256, 272), (129, 384, 48), (255, 128, 528), (769, 2048, 16304), (1024, 2048, 16384), (1023, 2176, 16144),
+              (1000, 256, 4096), (1025, 256, 4096)]   # (the last two: 256 tiles of 64 rows, and 272)
 
 
 @pytest.mark.parametrize("M,K,N", PRE_SHAPES)

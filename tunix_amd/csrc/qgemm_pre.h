@@ -12,6 +12,7 @@
 //   * RT = 4 (three work-groups per unit) is for an lm_head over at most 64 rows, which is bound by the stream of its weights: the
 //     MFMAs of 64 rows stay below that.  128256 x 4096 at 16 rows 203 -> 172 us
 //     (1.05 GB: 6.1 TB/s with the finishing launch), 262144 x 1152 at 64 rows 143 -> 109 us, 151936 x 2048 at 64 rows 150 -> 120 us.
+//     With two waves to a SIMD it is the form of all calls with no more tiles of 64 rows than units (launch_qgemm_pre).
 //   * activations go from memory straight into LDS, in steps of 64 k (rows of 128 bytes, 16-byte chunks swizzled by row)
 //     through four buffers, two steps ahead of their use and spread evenly over the loop: a burst of such loads would
 //     stand between a weight fragment and the compiler's wait for it, which does not count them.
@@ -72,6 +73,8 @@ enum PreKind { kPreStore, kPreF32, kPreRelu2, kPreSilu, kPreGelu, kPreSiluF32, k
 // without it, 128256 x 4096 over 128 rows 181 | 197, 262144 x 1152 123 | 136; with a second block of rows the weights come from L2 and the
 // policy loses: 151936 x 2048 over 256 rows 194 | 183.
 constexpr bool pre_head(int kind) { return kind == kPreHead || kind == kPreHeadOnce; }
+// work-groups per unit, i.e. waves per SIMD
+constexpr int pre_waves(int rt, int kind) { return rt == 16 ? 1 : rt == 4 && pre_head(kind) ? 3 : 2; }
 constexpr bool pre_mul(int kind) { return kind == kPreSilu || kind == kPreGelu || kind == kPreSiluF32 || kind == kPreGeluF32; }
 
 // LORA: 0 no adapter, kLoraInPlace: its scale is a power of two near one (1 where alpha is the rank): B times the scale is exact, and
@@ -248,7 +251,7 @@ __device__ __forceinline__ void pre_tile(const QLArgs& a, const WideHead& h, int
         const int ct = (rt & 1) ? CT - 1 - j : j;
         // (three waves per unit leave the weights of some slabs in accumulator registers, from which the compiler copies them right in front of
         // their use; the stream of the weights, which bounds this form, hides the wait states)
-        if constexpr (RT == 4) mfma16_acc_wait(wr[U % S][ct], xf[rt], acc[rt][ct]);
+        if constexpr (pre_waves(RT, KIND) == 3) mfma16_acc_wait(wr[U % S][ct], xf[rt], acc[rt][ct]);
         else mfma16_acc(wr[U % S][ct], xf[rt], acc[rt][ct]);
         if (j == 1 && rt % (RT / CT) == RT / CT - 1) load_w(ic<UL>{}, rt / (RT / CT), kt + ((U + 3) >> 2));
         if (j == CT / 2 && (rt & 3) == 1) dma(src, ((U & 1) ? 0 : HALF) + (rt >> 2), dbuf);
@@ -433,7 +436,7 @@ __device__ __forceinline__ void pre_tile(const QLArgs& a, const WideHead& h, int
 
 template <int RT, bool GROUPED, int KIND, int LORA, bool HALVES>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(RT == 16 ? 1 : RT == 8 ? 2 : 3, RT == 16 ? 1 : RT == 8 ? 2 : 3)))
+__attribute__((amdgpu_waves_per_eu(pre_waves(RT, KIND), pre_waves(RT, KIND))))
 void qgemm_pre_kernel(const QLArgs a, const WideHead h) {
   constexpr int ROWS = 16 * RT;
   extern __shared__ __align__(16) unsigned char smem[];   // (addressed absolutely: no static LDS in this kernel, checked by the host)

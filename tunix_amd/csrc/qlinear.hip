@@ -891,6 +891,10 @@ int launch_qgemm_pre(hipStream_t st, const QLArgs& a, const WideHead& h) {
   // (the noise of a draw is vector work, which two work-groups per unit put under each other's loads: 2048 x 151936 over 400 rows 634 us at 256 rows
   // of a tile, 468 at 128; 65536 x 2048 over 256 rows 144 | 130, over 160, more than a third of the second 128 missing, 108 | 137)
   if (h.part_draw && a.M > 160) return launch_qgemm_pre_rt<8>(st, a, h);
+  // No more tiles of 64 rows than units: one work-group to a unit either way, and a tile of half the rows takes two thirds of the time.  us at 64 |
+  // 128 rows: 8192 -> 2048 over 65 to 512 rows 51 | 73, over 2048 (256 tiles of 64) 69 | 82; 2048 -> 2048 16.7 | 23.2, 21.6 | 25.7; 4096 -> 4096 over
+  // 1024 37.8 | 46.2, over 1500 (384) 60 | 46.
+  if (!h.part && cdiv(a.M, 64) * tn <= 256) return launch_qgemm_pre_rt<4>(st, a, h);
   return tall < low ? launch_qgemm_pre_rt<16>(st, a, h) : launch_qgemm_pre_rt<8>(st, a, h);
 }
 
@@ -1002,11 +1006,13 @@ bool wide_shape(const QLArgs& a, int64_t min_rows = 512, int64_t min_tiles = 256
 // compute units in one turn, for its second turn costs as much as its first and tiles of 128 x 256
 // still need only one.  From 512 rows, and with a converted copy from the second row block on (below
 // that the codes' quarter of the bytes decides, and on two row blocks their conversion does).  us,
-// qgemm128_kernel | from the codes | from the copy: Llama-3.1-8B's o 44.9 | 60.7 | 51.6 at 1000 rows
-// (256 tiles), 81.8 | 63.1 | 54.4 at 1300; its down 129 | 173 | 179, 216 | 174 | 168, and 229 | 206 |
-// 178 at 1800; its q|k|v 37.5 | 55.4 | 58.0 at 512 rows (192), 69.3 | 56.4 | 55.6 at 700; its gate|up
-// 73.4 | 75.1 | 73.3 at 256 rows (448), 106 | 126 | 96 at 384; gemma-3-1b's gate|up 15.3 | 22.5 | 19.7
-// at 256 (216), 27.0 | 23.7 | 20.3 at 384 (324).
+// qgemm128_kernel | from the codes | from the copy: Llama-3.1-8B's o 81.8 | 63.1 | 54.4 at 1300 rows
+// (352 tiles); its down 216 | 174 | 168, and 229 | 206 | 178 at 1800; its q|k|v 69.3 | 56.4 | 55.6 at
+// 700; its gate|up 73.4 | 75.1 | 73.3 at 256 rows, 106 | 126 | 96 at 384; gemma-3-1b's gate|up 27.0 |
+// 23.7 | 20.3 at 384.
+// (Of fewer tiles the codes stay the better ones, although tiles of 64 rows from the copy take less where the weight is in cache, gemma's o
+// 14.4 | 11.7 us: in a model, whose copies no cache holds, log-probabilities over 320 rows took 5.03 | 5.45 ms, 1500 rows 6.67 | 7.32,
+// Llama-3.1-8B's eight layers over 500 rows 3.94 | 4.11.)
 bool many_rows(const QLArgs& a) {
   return cdiv(a.M, 128) * cdiv(a.N, 128) > 256 && wide_shape(a, copy_fits(a) ? kWideRows + 1 : 512, 1);
 }
