@@ -2740,6 +2740,12 @@ def test_last_column_tiles_of_half_the_width(gpu, M, K, N, rank, scale, residual
   assert torch.equal(outs[0][:M].view(torch.int16), outs[1][:M].view(torch.int16)) and bool((outs[0][M] == 7.0).all())
 
 
+@pytest.mark.parametrize("K,rank,scale,residual", [(256, 64, 0.75, True), (128, 32, 1.0, False), (384, 0, 1.0, True)])
+def test_linears_in_tiles_of_64_rows(gpu, K, rank, scale, residual):
+  """A converted copy in tiles of 64 rows (234 of them, the last row block of one row), next to the codes in tiles of 128."""
+  test_last_column_tiles_of_half_the_width(gpu, 513, K, 6656, rank, scale, residual)
+
+
 @pytest.mark.parametrize("M,K,widths", [(600, 256, (3968, 4112, 16)), (1000, 2048, (8176, 4096, 4112))])
 @pytest.mark.parametrize("rank", [32, 64])
 @pytest.mark.parametrize("scale", [1.0, 0.25, 0.75])
