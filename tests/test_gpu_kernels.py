@@ -2669,8 +2669,7 @@ def test_mul_epilogue_fuses_next_adapter_projection(gpu, M, F, r):
 
 
 # (the second half of the shapes runs 256-row tiles, the first 128-row ones: what fills the device better)
-PRE_SHAPES = [(65, 128, 16), (128, 256, 272), (129, 384, 48), (255, 128, 528), (769, 2048, 16304), (1024, 2048, 16384), (1023, 2176, 16144),
-              (1000, 256, 4096), (1025, 256, 4096)]   # (the last two: 256 tiles of 64 rows, and 272)
+PRE_SHAPES = [(65, 128, 16), (128, 256, 272), (129, 384, 48), (255, 128, 528), (769, 2048, 16304), (1024, 2048, 16384), (1023, 2176, 16144)]
 
 
 @pytest.mark.parametrize("M,K,N", PRE_SHAPES)
@@ -2738,6 +2737,12 @@ def test_last_column_tiles_of_half_the_width(gpu, M, K, N, rank, scale, residual
     outs.append(y)
   torch.cuda.synchronize()
   assert torch.equal(outs[0][:M].view(torch.int16), outs[1][:M].view(torch.int16)) and bool((outs[0][M] == 7.0).all())
+
+
+@pytest.mark.parametrize("M", [1000, 1025])
+def test_expanded_copy_at_the_line_of_64_row_tiles(gpu, M):
+  """256 tiles of 64 rows, one to a compute unit, and 272."""
+  test_many_rows_from_the_expanded_copy(gpu, M, 256, 4096)
 
 
 @pytest.mark.parametrize("K,rank,scale,residual", [(256, 64, 0.75, True), (128, 32, 1.0, False), (384, 0, 1.0, True)])
