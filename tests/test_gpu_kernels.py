@@ -2806,32 +2806,23 @@ def test_many_rows_experts_from_expanded_copies(gpu, K, N, counts):
     assert ((y[route[a0:a1].long()].double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (xe.abs() @ we.abs().T)).all()
 
 
-@pytest.mark.parametrize("dh,Hkv,G,M,S,chunk,window,qtype,group", [
-    (128, 8, 4, 1, 160, 32, 0, Q.NF4, 64),       # 5 chunks, 32 k-tiles in 8 splits of 4
-    (128, 8, 4, 3, 384, 32, 100, Q.NF4, 64),     # 12, some before the window
-    (128, 8, 4, 8, 128, 32, 0, Q.INT4, 32),      # 4
-    (128, 8, 4, 9, 96, 64, 0, Q.INT4, 128),      # 2, rows of the next tile
-    (128, 8, 4, 16, 64, 32, 20, Q.NF4, 32),
-    (64, 2, 4, 33, 96, 32, 0, Q.INT4, 64),       # two heads a k-tile
-    (64, 2, 4, 64, 64, 32, 40, Q.INT4, 64),
-    (256, 1, 4, 17, 288, 96, 0, Q.INT4, 128),    # half a head a k-tile
-    (256, 1, 4, 40, 64, 32, 0, Q.NF4, 64),
-    (256, 1, 3, 2, 200, 32, 33, Q.INT4, 128),    # 6 k-tiles, three a split
-])
-def test_linear_that_merges_key_chunks(gpu, dh, Hkv, G, M, S, chunk, window, qtype, group):
-  """gqa_attn_parts and a linear that merges its chunks against gqa_attn and the linear with its adapter inside, bit for bit: chunks without a key (padding in
-  front, a window), whose outputs nobody writes, included."""
+def merged_and_apart(gpu, dh, Hkv, G, M, S, chunk, window, qtype, group, cache=None, positive=False):
+  """(y, planes) of gqa_attn and the linear with its adapter inside, then of gqa_attn_parts and the linear that merges its chunks; cache(k, v, column): changes to
+  the caches; positive: no weight below zero, so that an infinite value stays one."""
   from tunix_amd import _lib as L
   from tunix_amd import ops
   bf = torch.bfloat16
   g = torch.Generator(device=gpu).manual_seed(dh + M)
   K, N, rank = Hkv * G * dh, 272, 32
   r = lambda *s: torch.randn(*s, generator=g, device=gpu)
+  w_of = lambda t: t.abs() + t.abs().mean() if positive else t
   col = S - 3
   tokens = torch.ones(M, S, dtype=torch.int32, device=gpu)
   for b in range(M):
     tokens[b, :(b * 37) % (col + 1)] = 0
   q, kc, vc = r(M, Hkv * G, dh).to(bf), r(M, Hkv, S, dh).to(bf), r(M, Hkv, S, dh).to(bf)
+  if cache is not None:
+    cache(kc, vc, col)
   n_chunks = -(-S // chunk)
   ws = torch.full((ops.attn_ws_bytes(M, 1, S, Hkv * G, dh, chunk) // 4,), float("nan"), device=gpu)
   out = torch.empty(M, K, dtype=bf, device=gpu)
@@ -2842,8 +2833,8 @@ def test_linear_that_merges_key_chunks(gpu, dh, Hkv, G, M, S, chunk, window, qty
   ad.q, ad.kcache, ad.vcache, ad.tokens, ad.tok_ld, ad.col_ptr = q.data_ptr(), kc.data_ptr(), vc.data_ptr(), tokens.data_ptr(), S, at.data_ptr()
   ad.ws, ad.out = ws.data_ptr(), out.data_ptr()
   split = {4096: 8, 768: 2}.get(K, K // 128)
-  codes, scales = ops.quantize_pack((r(K, N) * 0.05).to(bf), group, qtype)
-  a_t, b = (r(rank, K) * K ** -0.5).to(bf), (r(N, rank) * 0.3).to(bf)
+  codes, scales = ops.quantize_pack(w_of(r(K, N) * 0.05).to(bf), group, qtype)
+  a_t, b = w_of(r(rank, K) * K ** -0.5).to(bf), w_of(r(N, rank) * 0.3).to(bf)
   frag = ops.lora_frag(a_t)
   assert ops.qlinear_merged_ok(M, K, N, rank, split, dh, n_chunks)
   got = []
@@ -2861,8 +2852,48 @@ def test_linear_that_merges_key_chunks(gpu, dh, Hkv, G, M, S, chunk, window, qty
       ops.gqa_attn(ad)
       ops.qlinear(d, a_frag=frag)
     got += [y, planes]
+  return got
+
+
+@pytest.mark.parametrize("dh,Hkv,G,M,S,chunk,window,qtype,group", [
+    (128, 8, 4, 1, 160, 32, 0, Q.NF4, 64),       # 5 chunks, 32 k-tiles in 8 splits of 4
+    (128, 8, 4, 3, 384, 32, 100, Q.NF4, 64),     # 12, some before the window
+    (128, 8, 4, 8, 128, 32, 0, Q.INT4, 32),      # 4
+    (128, 8, 4, 9, 96, 64, 0, Q.INT4, 128),      # 2, rows of the next tile
+    (128, 8, 4, 16, 64, 32, 20, Q.NF4, 32),
+    (64, 2, 4, 33, 96, 32, 0, Q.INT4, 64),       # two heads a k-tile
+    (64, 2, 4, 64, 64, 32, 40, Q.INT4, 64),
+    (256, 1, 4, 17, 288, 96, 0, Q.INT4, 128),    # half a head a k-tile
+    (256, 1, 4, 40, 64, 32, 0, Q.NF4, 64),
+    (256, 1, 3, 2, 200, 32, 33, Q.INT4, 128),    # 6 k-tiles, three a split
+])
+def test_linear_that_merges_key_chunks(gpu, dh, Hkv, G, M, S, chunk, window, qtype, group):
+  """gqa_attn_parts and a linear that merges its chunks against gqa_attn and the linear with its adapter inside, bit for bit: chunks without a key (padding in
+  front, a window), whose outputs nobody writes, included."""
+  got = merged_and_apart(gpu, dh, Hkv, G, M, S, chunk, window, qtype, group)
   assert got[0].isfinite().all()
   assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3])
+
+
+@pytest.mark.parametrize("dh,Hkv,G,M,S,chunk,qtype,group", [
+    (128, 8, 4, 3, 384, 32, Q.NF4, 64),       # 12 chunks, all of them at once
+    (128, 8, 4, 9, 96, 64, Q.INT4, 128),      # 2, two pieces of a row at once
+    (64, 2, 4, 33, 96, 32, Q.INT4, 64),
+    (256, 1, 4, 17, 288, 96, Q.INT4, 128),
+])
+def test_linear_that_merges_key_chunks_keeps_infinities(gpu, dh, Hkv, G, M, S, chunk, qtype, group):
+  """An infinite value in the cache (row 0), sums that overflow (row 1) and a key of NaN (row 2, by way of its maximum and sum) reach the output as they do through
+  the pass that merges; no other row sees them."""
+  def cache(kc, vc, col):
+    vc[0, 0, col, 5] = float("inf")
+    kc[1, -1], vc[1, -1, :, 7] = 0.0, 3.38e38
+    kc[2, 0, col] = float("nan")
+
+  y, planes, y_m, planes_m = merged_and_apart(gpu, dh, Hkv, G, M, S, chunk, 0, qtype, group, cache, positive=True)
+  assert (y[:2] == float("inf")).all() and y[2].isnan().all() and y[3:].isfinite().all()
+  same = lambda u, v: torch.testing.assert_close(u, v, rtol=0, atol=0, equal_nan=True)
+  same(y_m, y)
+  same(planes_m, planes)
 
 
 def test_linear_that_merges_key_chunks_refuses(gpu):
