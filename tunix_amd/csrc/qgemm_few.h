@@ -195,13 +195,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
         }
         if (e0 + 512u * k < pieces) {
-          // o / L: the quotient by a reciprocal, corrected by its remainder, which an infinite o does not have (no key at all: o is 0)
-          const float by = L != 0.0f ? L : 1.0f, inv = 1.0f / by;
+          // o / L: the quotient by a reciprocal, corrected by its remainder.  An infinite o has none (inf - inf): the maximum makes a finite number of it, and the
+          // quotient stays infinite
+          const float inv = L != 0.0f ? 1.0f / L : 0.0f;
           u32x4 x;
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float t = o[e] * inv;
-            o[e] = __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-t, by, o[e]), inv, t), by, o[e]);
+            const float t = o[e] * inv, rest = fmaxf(__builtin_fmaf(-t, L, o[e]), -3.0e38f);
+            o[e] = __builtin_fmaf(rest, inv, t);
           }
 #pragma unroll
           for (int e = 0; e < 4; ++e) x[e] = pack2bf(o[2 * e], o[2 * e + 1]);
