@@ -53,7 +53,7 @@ typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
 // partials per column of work-groups and some hundred instructions a wave.  us a layer, with the merging pass | merged here: 32 heads of 128 on 8,
 // 4 k-tiles a split: 1 row x 600 keys (5 chunks) 71.0 | 66.1, 2 x 800 (7) 69.2 | 66.9, 3 x 2940 (10) 77.8 | 74.4, 8 x 400 (4) 72.2 | 70.1, 16 x 700 (2) 80.9 | 79.4;
 // 4 heads of 256 on one, one k-tile: 1 x 600 (5) 48.4 | 46.4, 16 x 1200 (10) 51.3 | 50.2.  Beyond kMergeBytes of partials a work-group (qlinear.hip) or
-// kMergeChunks chunks, a second round trip, nothing is left of it.
+// kMergeChunks chunks, which would take a second round trip, nothing is left of it.
 constexpr int kMergeChunks = 12;
 template <int SPT, bool INT4, int ROWS, bool INNER, bool SHORT, bool WHOLE, bool MERGE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void qgemm_few_kernel(const QLArgs a) {
@@ -138,8 +138,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
   };
-  // The same from partials: a thread takes eight columns of a row of a k-tile, U such pieces at a time, NC chunks of them at once.  (Vector instructions
-  // are what it costs, some 0.3 us per hundred of a wave: few, and no rows or chunks that are not there.)
+  // The same from partials: a thread takes eight columns of a row of a k-tile, U such pieces at a time, all of its chunks at once, NC of them at most.  (Vector
+  // instructions are what it costs, some 0.3 us per hundred of a wave: few, and no rows or chunks that are not there.)
   auto merge_x = [&](auto Uc, auto NCc) {
     constexpr int U = decltype(Uc)::value, NC = decltype(NCc)::value;
     const uint32_t C = (uint32_t)a.parts_n, dh = 1u << a.parts_shift, pitch = (dh + kPartPad) * 4u, heads = (uint32_t)(a.K >> a.parts_shift);
@@ -149,15 +149,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       uint32_t at[U], off[U], to[U];
       u32x2 ml[U][NC];
       u32x4 v[U][NC][2];
-      auto fetch = [&](int k, uint32_t c0) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-          if (c0 + c < C) {
-            ml[k][c] = __builtin_amdgcn_raw_buffer_load_b64(rp, at[k], (int)((c0 + c) * pitch), 0);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) v[k][c][h] = __builtin_amdgcn_raw_buffer_load_b128(rp, off[k] + 16u * h, (int)((c0 + c) * pitch), 0);
-          }
-      };
 #pragma unroll
       for (int k = 0; k < U; ++k) {
         const uint32_t e = e0 + 512u * k, row = n == 1 ? e >> 4 : n == 2 ? e >> 5 : n == 4 ? e >> 6 : e / 48u, i = (e >> 4) - row * (uint32_t)n, p = e & 15u;
@@ -166,7 +157,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         off[k] = at[k] + (kPartPad + (col & (dh - 1u))) * 4u;
         const uint32_t slot = i * SLOT;
         to[k] = (INT4 || slot < kBigLutBase ? slot : slot + (uint32_t)kBigLutBytes) + row * 256u + (p ^ (row & 15u)) * 16u;
-        fetch(k, 0);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          if (c < (int)C) {
+            ml[k][c] = __builtin_amdgcn_raw_buffer_load_b64(rp, at[k], (int)(c * pitch), 0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[k][c][h] = __builtin_amdgcn_raw_buffer_load_b128(rp, off[k] + 16u * h, (int)(c * pitch), 0);
+          }
       }
 #pragma unroll
       for (int k = 0; k < U; ++k) {
@@ -176,24 +173,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int c = 0; c < NC; ++c)
           if (c < (int)C) top = __uint_as_float(ml[k][c][1]) != 0.0f ? fmaxf(top, __uint_as_float(ml[k][c][0])) : top;
-        for (uint32_t c = NC; c < C; ++c) {
-          const u32x2 m = __builtin_amdgcn_raw_buffer_load_b64(rp, at[k], (int)(c * pitch), 0);
-          top = __uint_as_float(m[1]) != 0.0f ? fmaxf(top, __uint_as_float(m[0])) : top;
-        }
-        for (uint32_t c0 = 0; c0 < C; c0 += NC) {
-          if (c0 > 0) fetch(k, c0);
 #pragma unroll
-          for (int c = 0; c < NC; ++c)
-            if (c0 + c < C) {
-              const float l = __uint_as_float(ml[k][c][1]);
-              if (l != 0.0f) {   // (a chunk without a key: an O nobody wrote)
-                const float w = __expf(__uint_as_float(ml[k][c][0]) - top);
-                L += w * l;
+        for (int c = 0; c < NC; ++c)
+          if (c < (int)C) {
+            const float l = __uint_as_float(ml[k][c][1]);
+            if (l != 0.0f) {   // (a chunk without a key: an O nobody wrote)
+              const float w = __expf(__uint_as_float(ml[k][c][0]) - top);
+              L += w * l;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) o[e] += w * __uint_as_float(v[k][c][e >> 2][e & 3]);
-              }
+              for (int e = 0; e < 8; ++e) o[e] += w * __uint_as_float(v[k][c][e >> 2][e & 3]);
             }
-        }
+          }
         if (e0 + 512u * k < pieces) {
           // o / L: the quotient by a reciprocal, corrected by its remainder.  An infinite o has none (inf - inf): the maximum makes a finite number of it, and the
           // quotient stays infinite
@@ -237,7 +227,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   if constexpr (!INT4) fill_level_table<512>(kBigLutBase, tid);   // while the first loads are in flight
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (MERGE) {
+  if constexpr (MERGE) {   // (parts_n <= kMergeChunks: tnx_qlinear_merged_ok)
     static_assert(SHORT && INNER, "all k-tiles in LDS at once");
     if (a.parts_n <= 4 && a.M * n > 32) merge_x(ic<2>{}, ic<4>{});
     else merge_x(ic<1>{}, ic<kMergeChunks>{});
