@@ -2896,8 +2896,41 @@ def test_linear_that_merges_key_chunks_keeps_infinities(gpu, dh, Hkv, G, M, S, c
   same(planes_m, planes)
 
 
+@pytest.mark.parametrize("K,split,epilogue", [(128, 1, "TNX_EPI_STORE"), (512, 1, "TNX_EPI_RESIDUAL"), (512, 1, "TNX_EPI_F32"), (512, 4, "TNX_EPI_STORE")])
+def test_linear_that_merges_key_chunks_beside_its_output(gpu, K, split, epilogue):
+  """Partials that begin where the output ends, or end where it begins, give what they give anywhere else; an output that reaches into them raises."""
+  from tunix_amd import _lib as L
+  from tunix_amd import ops
+  bf, M, N, dh, n_chunks, rank = torch.bfloat16, 4, 272, 128, 3, 32
+  g = torch.Generator(device=gpu).manual_seed(K + split)
+  r = lambda *s: torch.randn(*s, generator=g, device=gpu)
+  parts = r(M, K // dh, n_chunks, dh + 4)
+  parts[..., 1] = parts[..., 1].abs() + 1.0
+  codes, scales = ops.quantize_pack((r(K, N) * 0.05).to(bf), 64, L.TNX_Q_INT4)
+  frag, b, x = ops.lora_frag((r(rank, K) * K ** -0.5).to(bf)), (r(N, rank) * 0.3).to(bf), r(M, N).to(bf)
+  wide = split > 1 or epilogue == "TNX_EPI_F32"
+  out_bytes, part_bytes = split * M * N * (4 if wide else 2), parts.numel() * 4
+  got = []
+  for o0, p0, free in ((0, out_bytes, True), (part_bytes, 0, True), (part_bytes + 4096, 0, True), (part_bytes - 16, 0, False), (0, out_bytes - 16, False)):
+    room = torch.zeros(part_bytes + out_bytes + 4096, dtype=torch.uint8, device=gpu)
+    room[p0:p0 + part_bytes] = parts.view(torch.uint8).flatten()
+    out = room[o0:o0 + out_bytes].view(torch.float32 if wide else bf)
+    y = torch.empty(M, N, dtype=bf, device=gpu) if split > 1 else out
+    d = ops.make_qlinear_desc(M=M, K=K, N=N, group=64, qtype=L.TNX_Q_INT4, x=x, codes=codes, scales=scales, y=y, epilogue=getattr(L, epilogue), residual=x, lora_rank=rank,
+                              lora_nseg=1, lora_seg_end=[N], lora_seg_toff=[0], lora_b=b, lora_scale=0.5, split_k=split, ws=out if split > 1 else None)
+    run = lambda: ops.qlinear(d, finish=False, a_frag=frag, parts=(room[p0:], dh, n_chunks))
+    if free:
+      run()
+      got.append(out.clone())
+      assert torch.equal(room[p0:p0 + part_bytes], parts.view(torch.uint8).flatten())
+    else:
+      with pytest.raises(ValueError, match="in the partials"):
+        run()
+  assert got[0].isfinite().all() and got[0].any() and all(torch.equal(got[0], v) for v in got[1:])
+
+
 def test_linear_that_merges_key_chunks_refuses(gpu):
-  """More rows, chunks or bytes than it takes, and an output in the partials."""
+  """More rows, chunks or bytes than it takes."""
   from tunix_amd import ops
   ok = ops.qlinear_merged_ok
   assert ok(16, 4096, 4096, 64, 8, 128, 2) and not ok(32, 4096, 4096, 64, 8, 128, 2)      # bytes

@@ -1235,7 +1235,7 @@ extern "C" int tnx_qlinear_merged(void* stream, const tnx_qlinear_desc* d, const
   TNX_REQUIRE(d->lora_nseg == 1 && d->epilogue != TNX_EPI_SILU_MUL && d->epilogue != TNX_EPI_GELU_MUL, "qlinear_merged: one adapter, no *_MUL epilogue");
   TNX_REQUIRE(a_frag && ((uintptr_t)a_frag & 15) == 0 && ((uintptr_t)parts & 15) == 0, "qlinear_merged: fragments and partials must be 16-byte aligned");
   const int64_t bytes = d->M * (d->K / dh) * n_chunks * (dh + kPartPad) * 4;
-  TNX_REQUIRE(apart(parts, bytes, d->split_k > 1 ? (const void*)d->ws : d->y, d->split_k > 1 ? (int64_t)d->split_k * d->M * d->N * 4 : d->M * d->N * 4),
+  TNX_REQUIRE(apart(parts, bytes, d->split_k > 1 ? (const void*)d->ws : d->y, d->split_k > 1 ? (int64_t)d->split_k * d->M * d->N * 4 : d->M * d->N * (d->epilogue == TNX_EPI_F32 ? 4 : 2)),
               "qlinear_merged: the output lies in the partials");
   QLArgs a = to_args(&c);
   a.inner_a = a_frag;
