@@ -287,6 +287,39 @@ def test_key_chunks_of_a_decode_step_without_an_adapter_behind(groups, S, head_d
   assert Runner._key_chunks(groups, S, head_dim, adapter_behind=False) == chunks
 
 
+def test_chunks_that_a_linear_merges():
+  from tunix_amd import ops
+  from tunix_amd.model import Runner
+  ok = lambda n: ops.qlinear_merged_ok(1, 4096, 4096, 64, 8, 128, n)
+  assert ok(Runner.MERGED_CHUNKS) and not ok(Runner.MERGED_CHUNKS + 1)
+
+
+@pytest.mark.parametrize("M,heads,kv_heads,head_dim,D,S,rank,chunks", [
+    (1, 32, 8, 128, 4096, 1536, 64, 12), (1, 32, 8, 128, 4096, 3000, 64, 12), (1, 32, 8, 128, 4096, 8192, 64, 12), (1, 32, 8, 128, 4096, 8193, 64, 29),   # (of 288)
+    (1, 32, 8, 128, 4096, 16384, 64, 32), (2, 32, 8, 128, 4096, 8192, 64, 12), (2, 32, 8, 128, 4096, 16384, 64, 16), (3, 32, 8, 128, 4096, 16384, 64, 10),
+    (1, 8, 2, 64, 512, 16384, 32, 12), (1, 8, 2, 64, 512, 32768, 32, 12), (1, 8, 2, 64, 512, 32769, 32, 114), (2, 8, 2, 64, 512, 16384, 32, 64),
+    (1, 32, 8, 128, 4096, 3000, 0, 24),       # no adapter: the merging pass runs
+    (1, 32, 8, 128, 4096, 256, 0, 1),
+    (1, 64, 8, 128, 8192, 3000, 64, 24),      # sixteen k-tiles a split
+    (4, 32, 4, 128, 2048, 3000, 64, 16),      # twelve are more bytes than it merges
+    (4, 32, 4, 128, 2048, 1600, 64, 10),      # ... ten, of 160 keys, are not
+    (1, 4, 1, 256, 1152, 3000, 32, 24),       # heads of 256
+    (1, 32, 8, 128, 4096, 65, 64, 1),
+])
+def test_key_chunks_in_front_of_the_linear_that_merges_them(M, heads, kv_heads, head_dim, D, S, rank, chunks):
+  """Twelve where o merges that many by itself and they are not too long; otherwise as many as fill the device."""
+  import math
+  import types
+  from tunix_amd.model import FusedLinear, Runner
+  o = FusedLinear.__new__(FusedLinear)
+  o.names, o.K, o.N, o.rp, o.has_lora, o.head, o.interleave2 = ["l0.wo"], heads * head_dim, D, rank, rank > 0, False, False
+  r = Runner.__new__(Runner)
+  r.split_k_override, r.cfg, r.S = {}, types.SimpleNamespace(num_kv_heads=kv_heads, head_dim=head_dim), S
+  r.kv_chunk, r.attn_ws = r._decode_chunk(o, M, S), None
+  assert (math.ceil(S / r.kv_chunk) if r.kv_chunk else 1) == chunks
+  assert r.kv_chunk % 32 == 0 and (r.merges(o, M) is not None) == (rank > 0 and 1 < chunks <= 12 and o.K < 8192)
+
+
 @pytest.mark.parametrize("groups,S,width,chunks", [
     (1, 4000, 256, 32), (40, 300, 512, 4), (40, 300, 256, 1), (60, 1000, 512, 4), (85, 2500, 512, 3), (86, 2500, 512, 5), (102, 1025, 512, 5), (96, 1024, 512, 2),
     (103, 2500, 512, 2), (128, 4000, 256, 2), (129, 2500, 512, 3), (129, 1024, 512, 1), (171, 1500, 512, 4), (171, 1500, 256, 1), (171, 2500, 256, 4),

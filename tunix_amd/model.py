@@ -569,18 +569,30 @@ class Runner(HeadRunner):
       self.next_tpart = torch.empty(n_planes * 8192, dtype=torch.float32, device=dev)
     self.splitk_ws = torch.empty(self._split_floats(), dtype=torch.float32, device=dev)
     if kv_chunk is None:
-      kv_chunk = 0
-      if T == 1 and S > 64:
-        o = model.layers[0]["o"] if model.layers else None
-        behind = o is not None and o.has_lora and not self.inner(o, M)
-        kv_chunk = math.ceil(S / self._key_chunks(B * cfg.num_kv_heads, S, cfg.head_dim, behind) / 32) * 32
-        if kv_chunk >= S:
-          kv_chunk = 0
+      kv_chunk = self._decode_chunk(model.layers[0]["o"] if model.layers else None, B, S) if T == 1 and S > 64 else 0
     self.kv_chunk = kv_chunk
     nb = ops.attn_ws_bytes(B, T, S, cfg.num_heads, cfg.head_dim, kv_chunk)
     self.attn_ws = torch.empty(max(nb // 4, 1), dtype=torch.float32, device=dev)
     self.zero = torch.zeros(1, dtype=torch.int32, device=dev)
     self._init_head(B, D, bf, want_logits)
+
+  MERGED_CHUNKS = 12   # chunks that a linear merges at most (kMergeChunks of csrc/qgemm_few.h)
+
+  def _decode_chunk(self, o: FusedLinear | None, M: int, S: int) -> int:
+    """Keys of a chunk of a decode step of M rows over a cache of S slots, in front of the linear o; 0: all of them."""
+    cfg = self.cfg
+    groups, adapter = M * cfg.num_kv_heads, o is not None and o.has_lora
+    n = self._key_chunks(groups, S, cfg.head_dim, adapter and not self.inner(o, M))
+    size = lambda n: math.ceil(S / n / 32) * 32
+    # Where o merges them itself, no more than it takes, as long as the longer chunks cost less than the merging pass; heads of 256 gain more from more of
+    # them.  us a layer in that many chunks with the pass | in 12 without: 8 kv heads of 128, 1 row x 3000 keys (24) 72.8 | 69.7, x 8192 (32) 77.8 | 76.4, x 16384 82.1 |
+    # 86.6, x 32768 92.0 | 106.8, 2 rows (16) x 8192 80.2 | 78.2, x 16384 89.1 | 89.3; 4, 2 rows (32) x 8192 72.9 | 71.9, x 16384 77.6 | 82.5; 2 of 64, 4 rows
+    # (32) x 8192 45.7 | 43.6, x 16384 48.3 | 49.9, 1 row (128) x 16384 64.3 | 48.0, x 32768 65.5 | 59.1; one of 256, 1 row x 3000 in 24 | 10 50.8 | 53.4.
+    # Where the pass runs all the same, an o without an adapter, 1 row x 8 heads of 128 in 32 | 12 chunks, x 8192 68.1 | 70.1, x 16384 73.1 | 80.3.
+    if (n > self.MERGED_CHUNKS and cfg.head_dim <= 128 and S <= (32768 if groups <= 2 else 8192) and adapter
+        and self._merges(o, M, math.ceil(S / size(self.MERGED_CHUNKS)))):
+      n = self.MERGED_CHUNKS
+    return size(n) if size(n) < S else 0
 
   @staticmethod
   def _key_chunks(groups: int, S: int, head_dim: int, adapter_behind: bool = True) -> int:
@@ -595,10 +607,7 @@ class Runner(HeadRunner):
     if not adapter_behind and S <= (384 if head_dim <= 64 else 256 if head_dim <= 128 else 0):
       return 1
     if groups <= 128:
-      # (merged in the linear behind: no more than it takes in one round trip; heads of 256 gain more from more of them.  us a layer in 24 chunks with the merging
-      # pass | in 10 without, one row x 3000, 8 kv heads of 128 72.0 | 70.6, one of 256 50.8 | 53.4; 2 x 2000 in 16 | 9 72.0 | 69.0)
-      most = 12 if not adapter_behind and head_dim <= 128 else 256
-      return max(1, min(256 // groups, math.ceil(S / 128), most))
+      return max(1, min(256 // groups, math.ceil(S / 128)))
     # More: two to a unit, of many keys, are cut in halves, which even out what the units have: 40 rows x 8 heads of 128 x 1280 52.6 | 44.2 (32 rows
     # 33.3 | 35.0, 56 rows x 1500 63.7 | 67.9; heads of 64, 256 rows x 2 x 1500 37 | 49).
     if head_dim <= 128:
@@ -695,8 +704,10 @@ class Runner(HeadRunner):
   def merges(self, f: FusedLinear, M: int) -> tuple | None:
     """What `linear` takes as its parts where it merges the key chunks of a decode step's attention itself (a launch less), else None."""
     n = math.ceil(self.S / self.kv_chunk) if self.kv_chunk else 1
-    dh = self.cfg.head_dim
-    return (self.attn_ws, dh, n) if n > 1 and self.inner(f, M) and ops.qlinear_merged_ok(M, f.K, f.N, f.rp, self._split_k(f, M), dh, n) else None
+    return (self.attn_ws, self.cfg.head_dim, n) if self._merges(f, M, n) else None
+
+  def _merges(self, f: FusedLinear, M: int, n: int) -> bool:
+    return n > 1 and self.inner(f, M) and ops.qlinear_merged_ok(M, f.K, f.N, f.rp, self._split_k(f, M), self.cfg.head_dim, n)
 
   def fuses_next(self, f: FusedLinear, next_f: FusedLinear, M: int, epilogue: int) -> bool:
     return (next_f.has_lora and not self.inner(next_f, M) and next_f.rp <= 64 and M <= 1024 and self._split_k(f, M) == 1
