@@ -296,8 +296,9 @@ def test_chunks_that_a_linear_merges():
 
 @pytest.mark.parametrize("M,heads,kv_heads,head_dim,D,S,rank,chunks", [
     (1, 32, 8, 128, 4096, 1536, 64, 12), (1, 32, 8, 128, 4096, 3000, 64, 12), (1, 32, 8, 128, 4096, 8192, 64, 12), (1, 32, 8, 128, 4096, 8193, 64, 29),   # (of 288)
-    (1, 32, 8, 128, 4096, 16384, 64, 32), (2, 32, 8, 128, 4096, 8192, 64, 12), (2, 32, 8, 128, 4096, 16384, 64, 16), (3, 32, 8, 128, 4096, 16384, 64, 10),
-    (1, 8, 2, 64, 512, 16384, 32, 12), (1, 8, 2, 64, 512, 32768, 32, 12), (1, 8, 2, 64, 512, 32769, 32, 114), (2, 8, 2, 64, 512, 16384, 32, 64),
+    (1, 32, 8, 128, 4096, 16384, 64, 32), (2, 32, 8, 128, 4096, 16384, 64, 12), (2, 32, 8, 128, 4096, 16385, 64, 16), (3, 32, 8, 128, 4096, 16384, 64, 10),
+    (1, 8, 2, 64, 512, 16384, 32, 12), (1, 8, 2, 64, 512, 32768, 32, 12), (1, 8, 2, 64, 512, 32769, 32, 114), (2, 8, 2, 64, 512, 16384, 32, 12), (2, 8, 2, 64, 512, 16385, 32, 57),
+    (3, 8, 2, 64, 512, 8192, 32, 12), (3, 8, 2, 64, 512, 8193, 32, 37),
     (1, 32, 8, 128, 4096, 3000, 0, 24),       # no adapter: the merging pass runs
     (1, 32, 8, 128, 4096, 256, 0, 1),
     (1, 64, 8, 128, 8192, 3000, 64, 24),      # sixteen k-tiles a split

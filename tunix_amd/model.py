@@ -585,11 +585,13 @@ class Runner(HeadRunner):
     n = self._key_chunks(groups, S, cfg.head_dim, adapter and not self.inner(o, M))
     size = lambda n: math.ceil(S / n / 32) * 32
     # Where o merges them itself, no more than it takes, as long as the longer chunks cost less than the merging pass; heads of 256 gain more from more of
-    # them.  us a layer in that many chunks with the pass | in 12 without: 8 kv heads of 128, 1 row x 3000 keys (24) 72.8 | 69.7, x 8192 (32) 77.8 | 76.4, x 16384 82.1 |
-    # 86.6, x 32768 92.0 | 106.8, 2 rows (16) x 8192 80.2 | 78.2, x 16384 89.1 | 89.3; 4, 2 rows (32) x 8192 72.9 | 71.9, x 16384 77.6 | 82.5; 2 of 64, 4 rows
-    # (32) x 8192 45.7 | 43.6, x 16384 48.3 | 49.9, 1 row (128) x 16384 64.3 | 48.0, x 32768 65.5 | 59.1; one of 256, 1 row x 3000 in 24 | 10 50.8 | 53.4.
-    # Where the pass runs all the same, an o without an adapter, 1 row x 8 heads of 128 in 32 | 12 chunks, x 8192 68.1 | 70.1, x 16384 73.1 | 80.3.
-    if (n > self.MERGED_CHUNKS and cfg.head_dim <= 128 and S <= (32768 if groups <= 2 else 8192) and adapter
+    # them.  us a layer in that many chunks with the pass | in 12 without, 8192 keys, 16384, 32768: 8 kv heads of 128, 1 row (32) 77.8 | 76.4, 82.1 | 86.6, 92.0 | 106.8,
+    # 2 rows (16) 80.2 | 78.2, 89.1 | 89.3, 110.5 | 111.9; of 64, 2 rows (16) 72.6 | 71.3, 78.0 | 78.4, 88.6 | 90.8; 4 of 128, 1 row (64) 76.1 | 69.3, 78.6 | 79.1, 82.8 | 99.6;
+    # 2 of 64, 2 rows (64) 50.6 | 42.5, 53.6 | 49.2, 56.3 | 60.1, 1 row (up to 128) 49.4 | 42.0, 64.3 | 48.0, 65.5 | 59.1.  1 row x 3000 keys, 8 of 128 in 24 | 12 72.8 | 69.7, one
+    # head of 256 in 24 | 10 50.8 | 53.4.
+    # Where the pass runs all the same, an o without an adapter, 1 row on 8 heads of 128 in 32 | 12 chunks 68.1 | 70.1, 73.1 | 80.3, 83.2 | 101.1.
+    longest = 32768 if groups <= 2 else 16384 if groups <= 4 or groups >= 16 else 8192
+    if (n > self.MERGED_CHUNKS and cfg.head_dim <= 128 and S <= longest and adapter
         and self._merges(o, M, math.ceil(S / size(self.MERGED_CHUNKS)))):
       n = self.MERGED_CHUNKS
     return size(n) if size(n) < S else 0
