@@ -330,6 +330,23 @@ def test_key_chunks_of_a_layer_list_step(groups, S, width, chunks):
   assert StackRunner._key_chunks(groups, S, width) == chunks
 
 
+@pytest.mark.parametrize("name,P,first,group,packs", [
+    ("tiny_qwen3", 16, (0, 1), 2, False), ("tiny_qwen3", 16, (0, 15), 2, False), ("tiny_qwen3", 256, (0,) * 30 + (200, 200), 32, False),
+    ("tiny_qwen3", 256, (0,) * 30 + (240, 240), 32, True),
+    ("gemma3_1b", 256, (0, 4), 2, False), ("gemma3_1b", 256, (0, 5), 2, True), ("gemma3_1b", 256, (0, 5), 1, False), ("gemma3_1b", 256, (3, 6), 1, True),
+    ("llama31_8b", 128, (0, 1), 2, True), ("llama31_8b", 128, (0, 0), 2, False), ("llama31_8b", 128, (1,), 1, True),
+])
+def test_prompts_are_packed_where_their_padding_is_worth_a_launch(name, P, first, group, packs):
+  import types
+  from tunix_amd.generate.sampler import Sampler
+  from tunix_amd.model import Runner
+  r = Runner.__new__(Runner)
+  r.cfg = getattr(config, name)()
+  st = types.SimpleNamespace(padded=any(first), first=np.array(first), group=group, num_input_tokens=P)
+  assert Sampler.packs(st, r) is packs
+  assert not Sampler.packs(st, object())      # a runner that knows padded rows alone
+
+
 def test_split_k_leaves_no_empty_split_and_goes_on_for_long_contractions():
   import math
   import types

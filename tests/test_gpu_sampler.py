@@ -512,6 +512,7 @@ def test_prompts_packed_and_padded_give_the_same(gpu, monkeypatch, name, kw, P, 
   prompts = [rng.integers(2, cfg.vocab_size, size=n).astype(np.int32) for n in lens]
   sampler = Sampler(model, IdTokenizer(cfg.vocab_size), CacheConfig(P + 6), prefill_rows=rows)
   outs, packed = [], []
+  monkeypatch.setattr(Sampler, "PACK_FROM", 0)
   packs = Sampler.packs
   for on in (True, False):
     monkeypatch.setattr(Sampler, "packs", staticmethod(lambda st, r: packed.append(packs(st, r)) or (packed[-1] and on)))

@@ -126,6 +126,11 @@ class _SamplingState:
 class Sampler:
   """Sampler for transformer model."""
 
+  # Multiplications that the padding of a group of prompts has to cost before its pass leaves it out: that takes a launch more (the embedding without the first
+  # layer's norm), 4 to 6 us, in which the device does 3e9 to 5e9.  us, padded | packed: small test model (6e6 a row), 2 x 16 columns, 4 of them padding 78 | 82, 64 x 64, 512 282 |
+  # 282, 32 x 256, 512 434 | 437, 1024 434 | 420; eight Gemma3-1B layers (2.2e8) 16 x 64, 15 1672 | 1677, 64 x 64, 63 2827 | 2807; four of Llama-3.1-8B (8.7e8) 8 x 256, 1 3596 | 3603, 32 3600 | 3589.
+  PACK_FROM = 3e9
+
   def __init__(self, transformer, tokenizer, cache_config: CacheConfig,
                use_graph: bool = True, prefill_rows: int = 16384):
     self._transformer = transformer
@@ -224,8 +229,10 @@ class Sampler:
 
   @staticmethod
   def packs(st: _SamplingState, runner) -> bool:
-    """Whether the prompts' forward pass leaves their padding out."""
-    return getattr(runner, "packs_prompts", False) and st.padded
+    """Whether the prompts' forward pass leaves their padding out: where that is worth a launch."""
+    if not (st.padded and getattr(runner, "packs_prompts", False)):
+      return False
+    return int(st.first.sum()) * runner.row_work(st.num_input_tokens) >= Sampler.PACK_FROM * -(-len(st.first) // st.group)
 
   def forward_step(self, runner, st: _SamplingState):
     """Forward over the one token per row in column `st.step`, from the cached state."""

@@ -756,6 +756,12 @@ class Runner(HeadRunner):
 
   packs_prompts = True   # forward_hidden takes `packed`
 
+  def row_work(self, T: int) -> int:
+    """Multiplications of a row of a prompt of T columns: its linears' weights, and half of the keys in front of the last one."""
+    cfg = self.cfg
+    mlp = 3 * cfg.embed_dim * cfg.hidden_dim * max(cfg.num_experts_per_tok, 1)
+    return cfg.num_layers * (2 * cfg.embed_dim * (cfg.q_dim + cfg.kv_dim) + mlp + cfg.q_dim * T)
+
   def forward_hidden(self, tokens, positions, col_ptr, cache, B=None, T=None, segment_ids=None, starts=None, packed=None):
     """Runs all layers for tokens[b, col .. col+T) of each row; leaves the final-normed hidden
     state in self.xn[:B*T].  cache: a SequenceCache of [B,Hkv,S,dh] slabs.  segment_ids (int32,
