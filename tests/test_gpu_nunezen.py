@@ -192,6 +192,49 @@ def test_gated_norm(gpu, dtype, W, split):
     assert rel((unfrag(out, M) if fr else out[:M])[:, :W], want) < (1e-6 if dtype == F32 else 4e-3)
 
 
+# ---- rotation of few rows -----------------------------------------------------------------------
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("split", [1, 2, 4, 5, 7, 8])    # (four planes at a time: one round, a whole second one, ragged ones)
+@pytest.mark.parametrize("B,T,H,G,dk,dv,dkp,dvp,rot", [
+    (341, 3, 4, 2, 32, 16, 32, 16, 32),        # 1023 rows, the last of few
+    (7, 1, 16, 4, 128, 128, 128, 128, 128),    # 224 items
+    (1, 2, 32, 8, 128, 64, 128, 64, 64),       # 544 items: three work-groups a row
+    (5, 1, 6, 3, 88, 72, 96, 128, 48),         # padded heads
+    (3, 4, 8, 1, 64, 40, 64, 64, 0),           # nothing rotates
+    (2, 1, 2, 1, 512, 8, 512, 8, 512),         # a sine and a cosine per thread
+])
+def test_rotation_of_few_rows(gpu, dtype, split, B, T, H, G, dk, dv, dkp, dvp, rot):
+  """Calls of fewer than 1024 rows against the same rows in a call of more, bit for bit, from finished rows and from planes; a slot past the cache is not written."""
+  many, col = max(B + 1, -(-1024 // T)), 2
+  S = col + max(1, T - 1)
+  ko, vo = H * dk, H * dk + G * dk
+  ld = vo + G * dv
+  g = torch.Generator(device=gpu).manual_seed(split + ld)
+  y = torch.randn(split, many, T, ld, generator=g, device=gpu)
+  freq = torch.tensor([1e4 ** (-2.0 * i / max(rot, 1)) for i in range(rot // 2)] or [0.0], dtype=F32, device=gpu)
+  starts, cp = i32([b % 4 for b in range(many)], gpu), i32([col], gpu)
+
+  def run(rows):
+    keep = y[:, :rows].contiguous() if split > 1 else y[0, :rows].to(dtype)
+    out = [torch.full((rows, *shape), float("nan"), dtype=dtype, device=gpu) for shape in ((T, H, dkp), (G, S, dkp), (G, S, dvp))]
+    d = L.PartRopeDesc()
+    d.B, d.T, d.S, d.H, d.G, d.dk, d.dv, d.dkp, d.dvp, d.rot_dims, d.dtype = rows, T, S, H, G, dk, dv, dkp, dvp, rot, ops.DTYPES[dtype]
+    d.y = ops.rows_src(ws=keep, split_k=split, plane=rows * T * ld, ld=ld) if split > 1 else ops.rows_src(y=keep, ld=ld)
+    d.inv_freq, d.k_off, d.v_off, d.starts, d.col_ptr = freq.data_ptr(), ko, vo, starts.data_ptr(), cp.data_ptr()
+    d.q_out, d.kcache, d.vcache = (t.data_ptr() for t in out)
+    ops.part_rope_kvwrite(d)
+    torch.cuda.synchronize()
+    return out
+
+  for few, all_ in zip(run(B), run(many)):
+    torch.testing.assert_close(few, all_[:B], rtol=0, atol=0, equal_nan=True)
+  q, k, v = run(B)
+  n = min(T, S - col)
+  assert q[:, :n].isfinite().all() and q[:, n:].isnan().all()
+  for c, w in ((k, dk), (v, dv)):
+    assert c[:, :, :col].isnan().all() and c[:, :, col:col + n].isfinite().all() and not c[:, :, col:col + n, w:].any()
+
+
 # ---- rotation + attention -----------------------------------------------------------------------
 class Attn:
   """One attention layer's kernels over a batch: the plain implementation's inputs and the device's cache."""
