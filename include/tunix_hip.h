@@ -144,8 +144,8 @@ int tnx_qw_expand(void* stream, const uint32_t* codes, const uint16_t* scales, i
 int tnx_qw_expand_bank(void* stream, const uint32_t* codes, const uint16_t* scales, int64_t E, int64_t K, int64_t N,
                        int group, int qtype, uint16_t* w_expanded);
 /* The same layout from a dense bf16 matrix w[N][K] (an unquantised or tied lm_head, [V][D]): a
- * log-probability pass over 512 rows or more then runs the head on the many-row kernel
- * (tnx_lmhead_desc.w_expanded next to w_bf16) instead of the 128 x 128 one. */
+ * call over more than 16 rows, or over fewer with 128 tiles of 256 columns or more (144 below a width of 2048), then runs
+ * the head on the many-row kernel (tnx_lmhead_desc.w_expanded next to w_bf16) instead of the 128 x 128 one. */
 int tnx_dense_expand(void* stream, const uint16_t* w_bf16, int64_t K, int64_t N, uint16_t* w_expanded);
 
 /* ---------------------------------------------------------------------------------------

@@ -1013,6 +1013,8 @@ bool wide_shape(const QLArgs& a, int64_t min_rows = 512, int64_t min_tiles = 256
 // (Of fewer tiles the codes stay the better ones, although tiles of 64 rows from the copy take less where the weight is in cache, gemma's o
 // 14.4 | 11.7 us: in a model, whose copies no cache holds, log-probabilities over 320 rows took 5.03 | 5.45 ms, 1500 rows 6.67 | 7.32,
 // Llama-3.1-8B's eight layers over 500 rows 3.94 | 4.11.)
+// A linear that leaves the next adapter's partial sums (next_tpart) stays with qgemm128_kernel whatever its size: the runner's gate|up up to 1024 rows where down
+// has an adapter, so that the figures of gate|up above are those of models without one there.
 bool many_rows(const QLArgs& a) {
   return cdiv(a.M, 128) * cdiv(a.N, 128) > 256 && wide_shape(a, copy_fits(a) ? kWideRows + 1 : 512, 1);
 }
